@@ -11,7 +11,8 @@
 //   md_latent_append     query latent -> weighted RMS norm; latent -> weighted RMS norm, key part -> rotation, both -> cache
 //   md_head_linear       y[row][h] = W_h x[row][h]: the absorbed queries (+ their rotated part) and the way out of the latent
 //                        (* sigmoid of the head's gate)
-//   md_latent_attn       the absorbed form over the cache; 32-bit and unusual sizes run the plain attention kernel of xattn.hip
+//   md_latent_attn       the absorbed form over the cache; 32-bit and unusual sizes run the fp32 attention kernels of xattn_f32.hip or,
+//                        beyond their sizes, the plain one of xattn.hip
 //   md_latent_gather     latents of a paged context as dense rows
 //   md_latent_prefill    the expanded form
 // Positions, angles, norms, scores, softmax weights and gates are fp32.
@@ -316,6 +317,32 @@ int check_args(const char* who, const md_latent_args* a) {
     return MD_OK;
 }
 
+long keys_of(const md_latent_args* a) { return (long)a->max_pages * a->page_size; }
+
+// the absorbed form as a one-kv-head attention whose values are the first kv_rank elements of its keys
+XattnParams general_params(const md_latent_args* a) {
+    XattnParams x = {};
+    x.q = a->q;
+    x.k_cache = a->cache;
+    x.v_cache = a->cache;
+    x.out = a->out;
+    x.qo_indptr = a->qo_indptr;
+    x.pos0 = a->pos0;
+    x.page_indices = a->page_indices;
+    x.page_indptr = a->page_indptr;
+    x.B = a->B;
+    x.n_max = a->n_max;
+    x.H = x.g = a->H;
+    x.KH = 1;
+    x.D = x.DKp = x.ldk = x.ldv = row_width(a->kv_rank, a->rot_dim);
+    x.DV = x.DVp = a->kv_rank;
+    x.page_size = a->page_size;
+    x.chunk = 0x7fffffff;
+    x.scale = a->scale;
+    x.scale_log2 = a->scale * 1.4426950408889634f;
+    return x;
+}
+
 LatentParams make_params(const md_latent_args* a) {
     LatentParams p = {};
     p.z = a->z;
@@ -447,7 +474,8 @@ extern "C" int md_head_linear(const md_head_linear_args* a, md_stream_t stream) 
 }
 
 extern "C" size_t md_latent_workspace_bytes(const md_latent_args* a) {
-    if (!a || !mfma_ok(a)) return 0;
+    if (!a) return 0;
+    if (!mfma_ok(a)) return a->force_plain ? 0 : md_internal_xattn_f32_workspace(general_params(a), keys_of(a));
     const int ns = kv_splits(a);
     if (ns == 1) return 0;
     const size_t Rp = (a->kv_rank + 15) / 16 * 16;
@@ -461,26 +489,11 @@ extern "C" int md_latent_attn(const md_latent_args* a, md_stream_t stream) {
     hipStream_t st = (hipStream_t)stream;
     LatentParams p = make_params(a);
     if (!mfma_ok(a)) {
-        // the same sums as a one-kv-head attention whose values are the first kv_rank elements of its keys
-        XattnParams x = {};
-        x.q = a->q;
-        x.k_cache = a->cache;
-        x.v_cache = a->cache;
-        x.out = a->out;
-        x.qo_indptr = a->qo_indptr;
-        x.pos0 = a->pos0;
-        x.page_indices = a->page_indices;
-        x.page_indptr = a->page_indptr;
-        x.B = a->B;
-        x.n_max = a->n_max;
-        x.H = x.g = a->H;
-        x.KH = 1;
-        x.D = x.DKp = x.ldk = x.ldv = p.W;
-        x.DV = x.DVp = a->kv_rank;
-        x.page_size = a->page_size;
-        x.chunk = 0x7fffffff;
-        x.scale = a->scale;
-        return md_internal_xattn_plain(x, a->dtype, st);
+        XattnParams x = general_params(a);
+        if (a->force_plain || !md_internal_xattn_f32_ok(x)) return md_internal_xattn_plain(x, a->dtype, st);
+        const size_t need = md_latent_workspace_bytes(a);
+        if (need && a->workspace && a->workspace_bytes >= need && aligned(a->workspace, 16)) x.ws = (float*)a->workspace;
+        return md_internal_xattn_f32(x, a->dtype, keys_of(a), st);
     }
     const int qt = row_tiles(a);
     p.n_groups = row_groups(a);

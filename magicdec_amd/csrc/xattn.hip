@@ -11,7 +11,8 @@
 //   md_qk_norm_append   q -> normalised padded rows; k -> normalised, v -> the cache
 //   md_xattn            attention over the cache.  bf16 with a bounded score: the matrix-core kernels of xattn_mfma.hip --
 //                       given the RAW projection rows, a decode step's normalisation and append happen inside the attention
-//                       launch --; otherwise (32-bit, unusual sizes, unbounded scores) the plain kernel below.
+//                       launch --; otherwise (32-bit, unbounded scores, unusual pages) the fp32 matrix kernels of xattn_f32.hip,
+//                       and for head sizes beyond their tiles the plain kernel below.
 #include "xattn.h"
 
 unsigned int* md_page_overflow_counter_device();   // kvops.hip
@@ -254,10 +255,14 @@ int decode_rows(const md_xattn_args* a) { return a->n_max * (a->H / a->KH); }
 
 int g_target_wgs = 256;
 
+// keys one request can see in a step: its chunk (plus the step's own rows), or its whole page list
+long keys_of(const md_xattn_args* a) {
+    const long keys = (long)a->max_pages * a->page_size;
+    return a->chunk > 0 && (long)a->chunk + a->n_max < keys ? (long)a->chunk + a->n_max : keys;
+}
+
 int decode_splits(const md_xattn_args* a) {
-    // keys one request can see in a step: its chunk (plus the step's own rows), or its whole page list
-    long keys = (long)a->max_pages * a->page_size;
-    if (a->chunk > 0 && a->chunk + a->n_max < keys) keys = a->chunk + a->n_max;
+    const long keys = keys_of(a);
     const long tiles = (keys + 31) / 32 + 1, pairs = (long)a->B * a->KH;
     long want = (g_target_wgs + pairs - 1) / pairs;
     const long cap = tiles / 16 > 1 ? tiles / 16 : 1;        // >= 16 tiles (4 per wavefront) per workgroup
@@ -337,7 +342,9 @@ extern "C" int md_xattn_fused_supported(const md_xattn_args* a) {
 }
 
 extern "C" size_t md_xattn_workspace_bytes(const md_xattn_args* a) {
-    if (!a || !mfma_ok(a) || decode_rows(a) > 32) return 0;
+    if (!a) return 0;
+    if (!mfma_ok(a)) return a->force_plain || a->KH <= 0 ? 0 : md_internal_xattn_f32_workspace(make_params(a), keys_of(a));
+    if (decode_rows(a) > 32) return 0;
     const int ns = decode_splits(a);
     if (ns == 1) return 0;
     const size_t cap = decode_rows(a) <= 16 ? 16 : 32;
@@ -391,8 +398,11 @@ extern "C" int md_xattn(const md_xattn_args* a, md_stream_t stream) {
 #undef MD_XW
     }
     if (!mfma_ok(a) || a->force_plain || (rows > 32 && nw == 0)) {
-        MD_CHECK_ARG(!fused, "md_xattn: the plain kernel takes normalised queries");
-        return md_internal_xattn_plain(p, a->dtype, st);
+        MD_CHECK_ARG(!fused, "md_xattn: the general kernels take normalised queries");
+        if (a->force_plain || !md_internal_xattn_f32_ok(p)) return md_internal_xattn_plain(p, a->dtype, st);
+        const size_t need = mfma_ok(a) ? 0 : md_xattn_workspace_bytes(a);
+        if (need && a->workspace && a->workspace_bytes >= need && ((uintptr_t)a->workspace & 15) == 0) p.ws = (float*)a->workspace;
+        return md_internal_xattn_f32(p, a->dtype, keys_of(a), st);
     }
     int rc;
     if (rows <= 32) {

@@ -1,0 +1,428 @@
+// Attention in 32-bit arithmetic on the fp32 matrix instructions (v_mfma_f32_16x16x4_f32): 32-bit models, and 16-bit pages where the
+// bf16 matrix-core kernels of xattn_mfma.hip / latent_absorbed.hip do not apply (unbounded scores, unusual page sizes).  Queries, keys,
+// values, scores, weights and sums are fp32 throughout, as in the plain kernel of xattn.hip, whose semantics these are.
+//
+// A workgroup (4 wavefronts) owns R = 16 QT query rows -- (token, head of the kv head) pairs -- and a range of KT-key tiles:
+//   S^T = K.Q^T    a 16 x 16 score tile per wavefront and step; K and Q fragments are ds_read_b128 of padded LDS rows.  The four
+//                  elements of a b128 are four k-steps (both operands permute the contraction the same way).
+//   softmax        256 / R threads per row, scores through LDS; running maximum in log2 units, the distance penalty as one v_log_f32
+//   O^T = V^T.P^T  each wavefront owns every fourth 16-wide slice of the value size, so its sums stay in registers for any head size
+//                  and the weights are read back from LDS as B fragments.
+// Three barriers per tile (four where values are a prefix of the key rows: one image serves both); the next tile is in registers
+// while this one is computed.  Few rows (decode): 16-row tiles and the key range split over workgroups, merged by a second launch.
+//
+// Bound by the fp32 matrix rate (154 TFLOP/s in a large library product) for prompts, by latency for decode steps.  Six sequences of
+// 100 to 1 500 tokens, 32 query and 8 kv heads of 64, one layer: 9 930 -> 465 us (27 GFLOP, half of the tiles' work masked); one token
+// each behind them: 292 -> 16.5 + 5.9 us for the merge (first figure: the plain kernel, one workgroup per row and head).
+#include "xattn.h"
+
+namespace {
+
+template <typename T>
+struct Vec4;
+template <>
+struct Vec4<float> {
+    typedef f32x4 type;
+};
+template <>
+struct Vec4<bf16_t> {
+    typedef bf16x4 type;
+};
+
+struct F32Launch {
+    int nq, nsplit, R, dvw;      // row groups, kv splits, rows per group, elements per partial row
+};
+
+template <int DK, int DV, int QT, int KT, bool SHARED>
+constexpr int f32_lds_bytes() {
+    return (16 * QT * (DK + 4) + KT * (DK + 4) + (SHARED ? 0 : KT * (DV + 4)) + 16 * QT * (KT + 4) + 16 * QT) * 4 + 16;
+}
+
+template <int DK, int DV, int QT, int KT, bool SHARED>
+constexpr int f32_waves_per_simd() {
+    return f32_lds_bytes<DK, DV, QT, KT, SHARED>() <= 80 * 1024 ? 2 : 1;
+}
+
+template <typename T, int DK, int DV, int QT, int KT, bool SHARED>
+__global__ __launch_bounds__(256, (f32_waves_per_simd<DK, DV, QT, KT, SHARED>())) void xattn_f32_kernel(const XattnParams p, const F32Launch L) {
+    typedef typename Vec4<T>::type vec4;
+    constexpr int R = 16 * QT, KP = DK + 4, VP = SHARED ? KP : DV + 4, PP = KT + 4;
+    constexpr int KB = KT / 16, NS = (KB * QT + 3) / 4, NV = DV / 64;
+    constexpr int TPR = 256 / R, KPT = KT / TPR;                 // softmax: threads per row, keys per thread
+    constexpr int LK = KT * DK / 1024, LV = SHARED ? 1 : KT * DV / 1024;   // 4-element pieces of a tile per thread
+    static_assert(KT * DK % 1024 == 0 && KT * DV % 1024 == 0 && DK % 16 == 0 && DV % 64 == 0 && KT % 32 == 0, "tile shapes");
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    float* sq = lds;
+    float* sk = sq + R * KP;
+    float* sv = SHARED ? sk : sk + KT * KP;
+    float* sp = (SHARED ? sk + KT * KP : sv + KT * VP);
+    float* sa = sp + R * PP;                                     // per row: rescaling factor of a tile, final factor at the end
+    int* sbad = reinterpret_cast<int*>(sa + R);                  // [2]: the tile's values hold an infinity or a NaN
+
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lq = lane & 15, lc = lane >> 4;
+    const int b = blockIdx.z, kvh = blockIdx.y, g = p.g;
+    const int qg = L.nq - 1 - (int)blockIdx.x / L.nsplit, split = (int)blockIdx.x % L.nsplit;    // longest key ranges first
+    const int q0 = p.qo_indptr[b], nrows = (p.qo_indptr[b + 1] - q0) * g, R0 = qg * R;
+    if (R0 >= nrows) return;
+    const int pos0 = p.pos0[b], pg0 = p.page_indptr[b], cap = (p.page_indptr[b + 1] - pg0) * p.page_size;
+    const int hi_wg = min(pos0 + (min(R0 + R, nrows) - 1) / g, cap - 1), lo_wg = ((pos0 + R0 / g) / p.chunk) * p.chunk;
+    int t0 = 0, t1 = 0;
+    if (hi_wg >= lo_wg) {
+        const int first = lo_wg / KT, n = hi_wg / KT - first + 1, per = (n + L.nsplit - 1) / L.nsplit;
+        t0 = first + min(split * per, n);
+        t1 = first + min((split + 1) * per, n);
+    }
+
+    // queries: R rows, zeros beyond the rows and the head size
+    for (int i = tid; i < R * (DK / 4); i += 256) {
+        const int r = i / (DK / 4), d = (i % (DK / 4)) * 4, row = R0 + r;
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        if (row < nrows && d < p.DKp)
+            v = __builtin_convertvector(*reinterpret_cast<const vec4*>(reinterpret_cast<const T*>(p.q) +
+                                        ((int64_t)(q0 + row / g) * p.H + kvh * g + row % g) * p.DKp + d), f32x4);
+        *reinterpret_cast<f32x4*>(sq + r * KP + d) = v;
+    }
+    if (tid < 2) sbad[tid] = 0;
+
+    // the row this thread does the softmax of
+    const int r = tid / TPR, u = tid % TPR;
+    int hi = -1, lo = 0;
+    float r1 = 0.f, r2 = 0.f, m = -1e30f, l = 0.f;
+    const int pos = pos0 + (R0 + r) / g;
+    if (R0 + r < nrows) {
+        hi = min(pos, cap - 1);
+        lo = (pos / p.chunk) * p.chunk;
+        if (p.r1) {
+            r1 = p.r1[kvh * g + (R0 + r) % g];
+            r2 = p.r2[kvh * g + (R0 + r) % g];
+        }
+    }
+    const bool bias = p.r1 != nullptr;
+
+    f32x4 o[QT][NV];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) o[qt][v] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    vec4 kr[LK], vr[LV];
+    auto request = [&](int t) {              // a tile's pieces into registers; its 32-key halves lie in one page each
+        const T* kb[KT / 32];
+        const T* vb[KT / 32];
+#pragma unroll
+        for (int h = 0; h < KT / 32; ++h) {
+            const int at = min(t * KT + h * 32, cap - 32), page = at / p.page_size;
+            const int64_t row = ((int64_t)p.page_indices[pg0 + page] * p.KH + kvh) * p.page_size + (at - page * p.page_size);
+            kb[h] = reinterpret_cast<const T*>(p.k_cache) + row * p.ldk;
+            vb[h] = reinterpret_cast<const T*>(p.v_cache) + row * p.ldv;
+        }
+#pragma unroll
+        for (int i = 0; i < LK; ++i) {
+            const int e = tid + 256 * i, row = e / (DK / 4), d = (e % (DK / 4)) * 4;
+            const T* base = KT == 64 && row >= 32 ? kb[KT / 32 - 1] : kb[0];
+            kr[i] = vec4{};
+            if (d < p.DKp) kr[i] = *reinterpret_cast<const vec4*>(base + (int64_t)(row % 32) * p.ldk + d);
+        }
+        if constexpr (!SHARED) {
+#pragma unroll
+            for (int i = 0; i < LV; ++i) {
+                const int e = tid + 256 * i, row = e / (DV / 4), d = (e % (DV / 4)) * 4;
+                const T* base = KT == 64 && row >= 32 ? vb[KT / 32 - 1] : vb[0];
+                vr[i] = vec4{};
+                if (d < p.DVp) vr[i] = *reinterpret_cast<const vec4*>(base + (int64_t)(row % 32) * p.ldv + d);
+            }
+        }
+    };
+    auto odd = [](f32x4 v) {                 // an infinity or a NaN among the four
+        return !(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))) <= 3.402823466e38f) || v[0] != v[0] ||
+               v[1] != v[1] || v[2] != v[2] || v[3] != v[3];
+    };
+    auto stage_k = [&](int t) {              // rows past the workgroup's last key are zeros: they may hold anything
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < LK; ++i) {
+            const int e = tid + 256 * i, row = e / (DK / 4), d = (e % (DK / 4)) * 4;
+            f32x4 v = __builtin_convertvector(kr[i], f32x4);
+            if (t * KT + row > hi_wg) v = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (SHARED) bad |= odd(v);
+            *reinterpret_cast<f32x4*>(sk + row * KP + d) = v;
+        }
+        if (SHARED && __builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) sbad[t & 1] = 1;
+    };
+    auto stage_v = [&](int t) {
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < LV; ++i) {
+            const int e = tid + 256 * i, row = e / (DV / 4), d = (e % (DV / 4)) * 4;
+            f32x4 v = __builtin_convertvector(vr[i], f32x4);
+            if (t * KT + row > hi_wg) v = f32x4{0.f, 0.f, 0.f, 0.f};
+            bad |= odd(v);
+            *reinterpret_cast<f32x4*>(sv + row * VP + d) = v;
+        }
+        if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) sbad[t & 1] = 1;
+    };
+
+    __syncthreads();                         // sbad is clear, the queries are there
+    if (t0 < t1) {
+        request(t0);
+        stage_k(t0);
+        if constexpr (!SHARED) stage_v(t0);
+        if (t0 + 1 < t1) request(t0 + 1);
+    }
+    __syncthreads();
+    const int kt = wave % KB;                // this wavefront's 16 keys of a tile ...
+    for (int t = t0; t < t1; ++t) {
+        // ---- scores
+        {
+            f32x4 s[NS];
+            const float* kp = sk + (kt * 16 + lq) * KP + lc * 4;
+#pragma unroll
+            for (int i = 0; i < NS; ++i) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+            for (int d = 0; d < DK; d += 16) {
+                const f32x4 ka = *reinterpret_cast<const f32x4*>(kp + d);
+#pragma unroll
+                for (int i = 0; i < NS; ++i) {
+                    const int qt = (wave + 4 * i) / KB;                   // ... against every (4 / KB)-th row tile
+                    const f32x4 qb = *reinterpret_cast<const f32x4*>(sq + ((qt < QT ? qt : 0) * 16 + lq) * KP + lc * 4 + d);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[e], qb[e], s[i], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < NS; ++i) {
+                const int qt = (wave + 4 * i) / KB;
+                if (qt < QT) *reinterpret_cast<f32x4*>(sp + (qt * 16 + lq) * PP + kt * 16 + lc * 4) = s[i];
+            }
+        }
+        __syncthreads();
+        // ---- softmax of row r over the tile's keys u * KPT ..
+        {
+            typedef float fvec __attribute__((ext_vector_type(KPT < 4 ? KPT : 4)));
+            constexpr int W = KPT < 4 ? KPT : 4;
+            float* row = sp + r * PP + u * KPT;
+            float s[KPT];
+            float mx = -INFINITY;
+#pragma unroll
+            for (int k = 0; k < KPT; k += W) {
+                const fvec x = *reinterpret_cast<const fvec*>(row + k);
+#pragma unroll
+                for (int e = 0; e < W; ++e) s[k + e] = x[e];
+            }
+#pragma unroll
+            for (int k = 0; k < KPT; ++k) {
+                const int kp = t * KT + u * KPT + k;
+                float v = s[k] * p.scale_log2;
+                if (bias) v -= r1 * __builtin_amdgcn_logf(1.0f + r2 * (float)(pos - kp));
+                s[k] = kp >= lo && kp <= hi ? v : -INFINITY;
+                mx = fmaxf(mx, s[k]);
+            }
+#pragma unroll
+            for (int x = 1; x < TPR; x <<= 1) mx = fmaxf(mx, __shfl_xor(mx, x));
+            const float mnew = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f(m - mnew);
+            m = mnew;
+            float ps = 0.f;
+#pragma unroll
+            for (int k = 0; k < KPT; k += W) {
+                fvec x;
+#pragma unroll
+                for (int e = 0; e < W; ++e) {
+                    x[e] = __builtin_amdgcn_exp2f(s[k + e] - mnew);
+                    ps += x[e];
+                }
+                *reinterpret_cast<fvec*>(row + k) = x;
+            }
+#pragma unroll
+            for (int x = 1; x < TPR; x <<= 1) ps += __shfl_xor(ps, x);
+            l = l * alpha + ps;
+            if (u == 0) sa[r] = alpha;
+            if (tid == 0) sbad[(t + 1) & 1] = 0;
+        }
+        if constexpr (!SHARED) {
+            if (t + 1 < t1) stage_k(t + 1);  // every wavefront has read this tile's keys
+        }
+        __syncthreads();
+        // ---- values
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+            const float a = sa[qt * 16 + lq];
+#pragma unroll
+            for (int v = 0; v < NV; ++v) o[qt][v] *= a;
+        }
+        if (sbad[t & 1] == 0) {
+#pragma unroll
+            for (int kk = 0; kk < KT; kk += 16) {
+                f32x4 pb[QT];
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) pb[qt] = *reinterpret_cast<const f32x4*>(sp + (qt * 16 + lq) * PP + kk + lc * 4);
+#pragma unroll
+                for (int v = 0; v < NV; ++v)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float va = sv[(kk + lc * 4 + e) * VP + (wave + 4 * v) * 16 + lq];
+#pragma unroll
+                        for (int qt = 0; qt < QT; ++qt) o[qt][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(va, pb[qt][e], o[qt][v], 0, 0, 0);
+                    }
+            }
+        } else {                             // a value that a row does not see must not reach it as 0 * infinity
+            for (int k = 0; k < KT; ++k)
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) {
+                    const float w = sp[(qt * 16 + lq) * PP + k];
+                    if (w != 0.f) {
+#pragma unroll
+                        for (int v = 0; v < NV; ++v)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) o[qt][v][e] = fmaf(w, sv[k * VP + (wave + 4 * v) * 16 + lc * 4 + e], o[qt][v][e]);
+                    }
+                }
+        }
+        __syncthreads();
+        if (t + 1 < t1) {
+            if constexpr (SHARED) stage_k(t + 1);
+            else stage_v(t + 1);
+            if (t + 2 < t1) request(t + 2);
+            if constexpr (SHARED) __syncthreads();
+        }
+    }
+    // ---- out: lane (lq, lc) holds elements d .. d + 3 of row qt * 16 + lq
+    const int64_t slot = (((int64_t)b * p.KH + kvh) * L.nq + qg) * L.nsplit + split;
+    float* wo = p.ws + slot * R * L.dvw;
+    if (u == 0) {
+        if (L.nsplit == 1) {
+            const float M = p.sink ? fmaxf(m, 0.f) : m, f = __builtin_amdgcn_exp2f(m - M);
+            const float Z = l * f + (p.sink ? __builtin_amdgcn_exp2f(-M) : 0.f);
+            sa[r] = Z > 0.f ? f / Z : Z != Z ? Z : 0.f;
+        } else {
+            float* ml = p.ws + (int64_t)p.B * p.KH * L.nq * L.nsplit * R * L.dvw + (slot * R + r) * 2;
+            ml[0] = m;
+            ml[1] = l;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+        const int row = R0 + qt * 16 + lq;
+        if (row >= nrows) continue;
+        const float f = L.nsplit == 1 ? sa[qt * 16 + lq] : 1.f;
+        T* out = reinterpret_cast<T*>(p.out) + ((int64_t)(q0 + row / g) * p.H + kvh * g + row % g) * p.DV;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+            const int d = (wave + 4 * v) * 16 + lc * 4;
+            if (L.nsplit > 1) {
+                *reinterpret_cast<f32x4*>(wo + (qt * 16 + lq) * L.dvw + d) = o[qt][v];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (d + e < p.DV) out[d + e] = (T)(o[qt][v][e] * f);
+            }
+        }
+    }
+}
+
+// sums the kv splits: one thread per four elements of a row
+template <typename T>
+__global__ __launch_bounds__(256) void xattn_f32_merge_kernel(const XattnParams p, const F32Launch L) {
+    const int vpr = L.dvw / 4;
+    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x, rowid = id / vpr;
+    const int d = (int)(id - rowid * vpr) * 4, r = (int)(rowid % L.R);
+    const int64_t item = rowid / L.R;                         // (b, kvh, row group)
+    const int qg = (int)(item % L.nq), pair = (int)(item / L.nq);
+    if (pair >= p.B * p.KH || d >= p.DV) return;
+    const int b = pair / p.KH, kvh = pair % p.KH, q0 = p.qo_indptr[b], row = qg * L.R + r;
+    if (row >= (p.qo_indptr[b + 1] - q0) * p.g) return;
+    const float* ml = p.ws + (int64_t)p.B * p.KH * L.nq * L.nsplit * L.R * L.dvw;
+    float M = p.sink ? 0.f : -1e30f;
+    for (int s = 0; s < L.nsplit; ++s) M = fmaxf(M, ml[((item * L.nsplit + s) * L.R + r) * 2]);
+    float Z = p.sink ? __builtin_amdgcn_exp2f(-M) : 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < L.nsplit; ++s) {
+        const int64_t at = (item * L.nsplit + s) * L.R + r;
+        const float f = __builtin_amdgcn_exp2f(ml[at * 2] - M);
+        Z += ml[at * 2 + 1] * f;
+        o += *reinterpret_cast<const f32x4*>(p.ws + at * L.dvw + d) * f;
+    }
+    const float inv = Z > 0.f ? 1.0f / Z : Z != Z ? Z : 0.f;
+    T* out = reinterpret_cast<T*>(p.out) + ((int64_t)(q0 + row / p.g) * p.H + kvh * p.g + row % p.g) * p.DV + d;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (d + e < p.DV) out[e] = (T)(o[e] * inv);
+}
+
+// The tile shapes: rows per workgroup as many as leave two workgroups per CU in 160 KB of LDS (one for the wide heads)
+enum Shape { kNone, k64, k128, k256, kShared320, kShared576 };
+
+Shape shape_of(const XattnParams& p) {
+    if (p.k_cache == p.v_cache && p.ldk == p.ldv)
+        return p.DKp <= 320 && p.DVp <= 256 ? kShared320 : p.DKp <= 576 && p.DVp <= 512 ? kShared576 : kNone;
+    const int w = p.DKp > p.DVp ? p.DKp : p.DVp;
+    return w <= 64 ? k64 : w <= 128 ? k128 : w <= 256 ? k256 : kNone;
+}
+
+F32Launch plan(const XattnParams& p, Shape s, long keys) {
+    static const int wide[] = {0, 4, 4, 2, 2, 2}, dvw[] = {0, 64, 128, 256, 256, 512}, kt[] = {0, 64, 32, 32, 32, 32};
+    const int64_t rows = (int64_t)p.n_max * p.g;
+    F32Launch L;
+    L.R = 16 * (rows <= 16 ? 1 : wide[s]);
+    L.dvw = dvw[s];
+    L.nq = (int)((rows + L.R - 1) / L.R);
+    // two workgroups per CU; a split has at least four tiles, so that its first loads and its share of the merge are a small part
+    const int64_t groups = (int64_t)L.nq * p.KH * p.B, want = (512 + groups - 1) / groups, most = keys / (4 * kt[s]);
+    L.nsplit = (int)(want < most ? want : most);
+    if (L.nsplit < 1) L.nsplit = 1;
+    if (L.nsplit > 64) L.nsplit = 64;
+    return L;
+}
+
+template <typename T, int DK, int DV, int QT, int KT, bool SHARED>
+int launch(const XattnParams& p, const F32Launch& L, hipStream_t st) {
+    constexpr int bytes = f32_lds_bytes<DK, DV, QT, KT, SHARED>();
+    static_assert(bytes <= 160 * 1024, "LDS");
+    static MdPerDeviceOnce once;
+    if (bytes > 64 * 1024 && once.first()) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&xattn_f32_kernel<T, DK, DV, QT, KT, SHARED>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
+            once.undo();
+            md_set_error("attention: cannot raise the LDS limit to %d bytes", bytes);
+            return MD_ERR_LAUNCH;
+        }
+    }
+    hipLaunchKernelGGL((xattn_f32_kernel<T, DK, DV, QT, KT, SHARED>), dim3((unsigned)(L.nq * L.nsplit), p.KH, p.B), dim3(256), bytes,
+                       st, p, L);
+    if (L.nsplit > 1) {
+        const int64_t threads = (int64_t)p.B * p.KH * L.nq * L.R * (L.dvw / 4);
+        hipLaunchKernelGGL((xattn_f32_merge_kernel<T>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, p, L);
+    }
+    MD_CHECK_LAUNCH("attention(32-bit)");
+    return MD_OK;
+}
+
+template <typename T>
+int launch_shape(const XattnParams& p, Shape s, const F32Launch& L, hipStream_t st) {
+    const bool few = L.R == 16;
+    switch (s) {
+    case k64: return few ? launch<T, 64, 64, 1, 64, false>(p, L, st) : launch<T, 64, 64, 4, 64, false>(p, L, st);
+    case k128: return few ? launch<T, 128, 128, 1, 32, false>(p, L, st) : launch<T, 128, 128, 4, 32, false>(p, L, st);
+    case k256: return few ? launch<T, 256, 256, 1, 32, false>(p, L, st) : launch<T, 256, 256, 2, 32, false>(p, L, st);
+    case kShared320: return few ? launch<T, 320, 256, 1, 32, true>(p, L, st) : launch<T, 320, 256, 2, 32, true>(p, L, st);
+    default: return few ? launch<T, 576, 512, 1, 32, true>(p, L, st) : launch<T, 576, 512, 2, 32, true>(p, L, st);
+    }
+}
+
+}  // namespace
+
+size_t md_internal_xattn_f32_workspace(const XattnParams& p, long keys) {
+    const Shape s = shape_of(p);
+    if (s == kNone) return 0;
+    const F32Launch L = plan(p, s, keys);
+    return L.nsplit == 1 ? 0 : (size_t)p.B * p.KH * L.nq * L.nsplit * L.R * (L.dvw + 2) * 4;
+}
+
+bool md_internal_xattn_f32_ok(const XattnParams& p) { return shape_of(p) != kNone && p.page_size % 32 == 0; }
+
+int md_internal_xattn_f32(const XattnParams& p, int dtype, long keys, hipStream_t st) {
+    const Shape s = shape_of(p);
+    F32Launch L = plan(p, s, keys);
+    if (!p.ws) L.nsplit = 1;
+    return dtype == MD_T_F32 ? launch_shape<float>(p, s, L, st) : launch_shape<bf16_t>(p, s, L, st);
+}
