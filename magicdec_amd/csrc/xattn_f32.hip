@@ -367,7 +367,7 @@ F32Launch plan(const XattnParams& p, Shape s, long keys) {
     L.dvw = dvw[s];
     L.nq = (int)((rows + L.R - 1) / L.R);
     // two workgroups per CU; a split has at least four tiles, so that its first loads and its share of the merge are a small part
-    const int64_t groups = (int64_t)L.nq * p.KH * p.B, want = (512 + groups - 1) / groups, most = keys / (4 * kt[s]);
+    const int64_t groups = (int64_t)L.nq * p.KH * p.B, want = groups > 0 ? (512 + groups - 1) / groups : 1, most = keys / (4 * kt[s]);
     L.nsplit = (int)(want < most ? want : most);
     if (L.nsplit < 1) L.nsplit = 1;
     if (L.nsplit > 64) L.nsplit = 64;
