@@ -579,6 +579,26 @@ int md_accept_rollback(int64_t* tokens_buffer, const int64_t* target_tokens, int
                        int64_t* cachelens_update, int32_t* flags, md_stream_t stream);
 
 /* ------------------------------------------------------------------------
+ * The integer work around a decode step (lengths moved on, token ids in and out of a captured step's buffers), up to
+ * MD_STEP_MAX_OPS pieces in one launch.  Each is rows x cols elements of a dense dst; pieces of one call must not overlap.
+ *   MD_STEP_ADD   int32 dst += a                            (src unused)
+ *   MD_STEP_SCALE int32 dst = src * a                       (src dense)
+ *   MD_STEP_COPY  int64 dst[r][c] = src[r * src_stride + c]
+ * ---------------------------------------------------------------------- */
+#define MD_STEP_ADD 0
+#define MD_STEP_SCALE 1
+#define MD_STEP_COPY 2
+#define MD_STEP_MAX_OPS 8
+typedef struct {
+    void* dst;
+    const void* src;
+    int64_t src_stride;
+    int32_t rows, cols;
+    int32_t kind, a;
+} md_step_op;
+int md_step_ops(const md_step_op* ops_host, int count, md_stream_t stream);
+
+/* ------------------------------------------------------------------------
  * C1  the per-layer sum-all-reduce of the tensor-parallel decode path over xGMI peer-mapped buffers
  *     reference: dist.all_reduce at Engine/SnapKV/model.py:334-335,453-454 (and the StreamingLLM twins), NCCL with
  *     PyTorch's intra-node one-/two-shot kernels (README.md:59 ENABLE_INTRA_NODE_COMM=1); the fused form also

@@ -188,8 +188,10 @@ class _BackendBase:
         from .model_layers import STATE_RING
         return dict(slots=self.batch_size, state_ring=max(STATE_RING, int(dec_len) + 2))
 
+    _qo_bound = None       # while a step is captured: the tensor that every replay fills with qo_indptr * n beforehand
+
     def _qo(self, n):
-        return self.qo_indptr * n
+        return self.qo_indptr * n if self._qo_bound is None else self._qo_bound
 
     def _decode_rows(self, *per_request, two_token_step=True):
         """Row counts of this engine's decode / verify steps: batch x (1, dec_len ..., and 2 -- the two-token step after an
@@ -222,11 +224,21 @@ class _BackendBase:
         for b in self.model.layers:
             b.attention.kv_cache.calibrated = False
 
-    def _run_step(self, key, fn, *tensors):
+    def _move(self, by):
+        """Length tensors moved on in place: {attribute: tokens}."""
+        for name, n in by.items():
+            if n:
+                getattr(self, name).add_(n)
+
+    def _run_step(self, key, fn, ids, lead, tail):
+        """fn(ids) between two moves of the length tensors: {attribute: tokens} before and behind it."""
         if self._use_graphs:
             from .graph import run_captured
-            return run_captured(self, key, fn, *tensors)
-        return fn(*tensors)
+            return run_captured(self, key, fn, ids, lead, tail)
+        self._move(lead)
+        out = fn(ids)
+        self._move(tail)
+        return out
 
 
 # ======================================================================================= target (+ SnapKV self-spec)
@@ -419,43 +431,28 @@ class SnapKVTargetBackend(_BackendBase):
     def inference(self, input_ids: torch.LongTensor, benchmark=False):
         """Autoregressive step / longspec verification (backend.py:129-159)."""
         n = input_ids.shape[1]
-        self.paged_kv_last_page_len += n                      # pre_decode
-        out = self._run_step(("fwd", n), lambda ids: self.model.forward(ids, self.cachelens, self._qo(n),
-                                                                          self._t.table()), input_ids)
-        self.cachelens += n
-        if benchmark:
-            self.cachelens -= n
-            self.paged_kv_last_page_len -= n
-        return out
+        return self._run_step(("fwd", n), lambda ids: self.model.forward(ids, self.cachelens, self._qo(n), self._t.table()),
+                              input_ids, {"paged_kv_last_page_len": n},                      # pre_decode
+                              {"paged_kv_last_page_len": -n} if benchmark else {"cachelens": n})
 
     @torch.no_grad()
     def verify(self, input_ids: torch.LongTensor, benchmark=False):
         """Self-spec verification: also appends the gamma+1 rows to the draft cache (backend.py:163-197)."""
         n = input_ids.shape[1]
-        self.paged_kv_last_page_len += n                      # pre_verify
-        self.draft_paged_kv_last_page_len += 1
-        self.draft_cachelens += 1
-        out = self._run_step(("verify", n), lambda ids: self.model.verify(ids, self.cachelens, self._qo(n),
-                                                                            self._t.table(), self._d.table()),
-                             input_ids)
-        self.cachelens += n
-        if benchmark:
-            self.cachelens -= n
-            self.paged_kv_last_page_len -= n
-        return out
+        return self._run_step(("verify", n), lambda ids: self.model.verify(ids, self.cachelens, self._qo(n), self._t.table(),
+                                                                           self._d.table()),
+                              input_ids, {"paged_kv_last_page_len": n, "draft_paged_kv_last_page_len": 1,      # pre_verify
+                                          "draft_cachelens": 1},
+                              {"paged_kv_last_page_len": -n} if benchmark else {"cachelens": n})
 
     @torch.no_grad()
     def speculate(self, input_ids: torch.LongTensor, benchmark=False):
         """Self-spec draft step over the SnapKV draft cache (backend.py:200-229)."""
         n = input_ids.shape[1]
-        self.draft_paged_kv_last_page_len += n                # pre_spec
-        out = self._run_step(("spec", n), lambda ids: self.model.draft_forward(ids, self.draft_cachelens, self._qo(n),
-                                                                                 self._d.table()), input_ids)
-        self.draft_cachelens += n
-        if benchmark:
-            self.draft_cachelens -= n
-            self.draft_paged_kv_last_page_len -= n
-        return out
+        return self._run_step(("spec", n), lambda ids: self.model.draft_forward(ids, self.draft_cachelens, self._qo(n),
+                                                                                self._d.table()),
+                              input_ids, {"draft_paged_kv_last_page_len": n},                # pre_spec
+                              {"draft_paged_kv_last_page_len": -n} if benchmark else {"draft_cachelens": n})
 
 
 # ======================================================================================= SnapKV stand-alone draft
@@ -539,26 +536,24 @@ class SnapKVDraftBackend(_BackendBase):
     def inference(self, input_ids: torch.LongTensor, benchmark=False, cachelen_update=None):
         """One (or, after an all-accept iteration, a two-token) draft step (backend_draft.py:113-173)."""
         n = input_ids.shape[1]
+        # (benchmark, as the reference: always the un-prefixed table, backend_draft.py:139-142)
+        tail = {} if cachelen_update is not None else {"paged_kv_last_page_len": -n} if benchmark else {"cachelens": n}
         if self.is_compress:
-            self.draft_paged_kv_last_page_len += n            # pre_decode
             out = self._run_step(("draft", n), lambda ids: self.model.draft_forward(ids, self.cachelens, self._qo(n),
-                                                                                      self._d.table()), input_ids)
+                                                                                    self._d.table()),
+                                 input_ids, {"draft_paged_kv_last_page_len": n}, tail)       # pre_decode
         else:
-            self.paged_kv_last_page_len += n
-            out = self._run_step(("fwd", n), lambda ids: self.model.forward(ids, self.cachelens, self._qo(n),
-                                                                              self._t.table()), input_ids)
-        if cachelen_update is None:
-            self.cachelens += n
-        else:
+            out = self._run_step(("fwd", n), lambda ids: self.model.forward(ids, self.cachelens, self._qo(n), self._t.table()),
+                                 input_ids, {"paged_kv_last_page_len": n}, tail)
+        if cachelen_update is not None:
             cu = cachelen_update.to(torch.int32).flatten()
             self.cachelens += cu
             if self.is_compress:
                 self.draft_paged_kv_last_page_len = self.draft_paged_kv_last_page_len - n + cu
             else:
                 self.paged_kv_last_page_len = self.paged_kv_last_page_len - n + cu
-        if benchmark:   # as the reference: always the un-prefixed table (backend_draft.py:139-142)
-            self.cachelens -= n
-            self.paged_kv_last_page_len -= n
+            if benchmark:
+                self._move({"cachelens": -n, "paged_kv_last_page_len": -n})
         return out
 
 
@@ -635,18 +630,15 @@ class StreamingDraftBackend(_BackendBase, _StreamingMixin):
     def inference(self, input_ids: torch.LongTensor, benchmark=False, cachelen_update=None):
         """StreamingLLM/backend_draft.py:89-124."""
         n = input_ids.shape[1]
-        self.paged_kv_last_page_len += n
-        out = self._run_step(("fwd", n), lambda ids: self.model.forward(ids, self.cachelens, self._qo(n),
-                                                                          self._t.table()), input_ids)
-        if cachelen_update is None:
-            self.cachelens += n
-        else:
+        tail = {} if cachelen_update is not None else {"paged_kv_last_page_len": -n} if benchmark else {"cachelens": n}
+        out = self._run_step(("fwd", n), lambda ids: self.model.forward(ids, self.cachelens, self._qo(n), self._t.table()),
+                             input_ids, {"paged_kv_last_page_len": n}, tail)
+        if cachelen_update is not None:
             cu = cachelen_update.to(torch.int32).flatten()
             self.cachelens += cu
             self.paged_kv_last_page_len = self.paged_kv_last_page_len - n + cu
-        if benchmark:
-            self.cachelens -= n
-            self.paged_kv_last_page_len -= n
+            if benchmark:
+                self._move({"cachelens": -n, "paged_kv_last_page_len": -n})
         return out
 
 
@@ -719,29 +711,22 @@ class StreamingSelfSpecBackend(_BackendBase, _StreamingMixin):
     @torch.no_grad()
     def verify(self, input_ids: torch.LongTensor, benchmark=False):
         n = input_ids.shape[1]
-        self.paged_kv_last_page_len += n
-        out = self._run_step(("verify", n), lambda ids: self.model.verify(ids, self.cachelens, self._qo(n),
-                                                                            self._t.table()), input_ids)
-        self.cachelens += n
-        if benchmark:
-            self.cachelens -= n
-            self.paged_kv_last_page_len -= n
-        return out
+        return self._run_step(("verify", n), lambda ids: self.model.verify(ids, self.cachelens, self._qo(n), self._t.table()),
+                              input_ids, {"paged_kv_last_page_len": n},
+                              {"paged_kv_last_page_len": -n} if benchmark else {"cachelens": n})
 
     @torch.no_grad()
     def speculate(self, input_ids: torch.LongTensor, benchmark=False, cachelen_update=None):
         n = input_ids.shape[1]
-        self.draft_paged_kv_last_page_len += n
-        out = self._run_step(("spec", n), lambda ids: self.model.draft_forward(ids, self.draft_cachelens,
-                                                                                 self._qo(n), self._d.table()),
-                             input_ids)
-        if cachelen_update is None:
-            self.draft_cachelens += n
-        else:
+        tail = ({} if cachelen_update is not None else {"draft_paged_kv_last_page_len": -n} if benchmark
+                else {"draft_cachelens": n})
+        out = self._run_step(("spec", n), lambda ids: self.model.draft_forward(ids, self.draft_cachelens, self._qo(n),
+                                                                               self._d.table()),
+                             input_ids, {"draft_paged_kv_last_page_len": n}, tail)
+        if cachelen_update is not None:
             cu = cachelen_update.to(torch.int32).flatten()
             self.draft_cachelens += cu
             self.draft_paged_kv_last_page_len = self.draft_paged_kv_last_page_len - n + cu
-        if benchmark:
-            self.draft_cachelens -= n
-            self.draft_paged_kv_last_page_len -= n
+            if benchmark:
+                self._move({"draft_cachelens": -n, "draft_paged_kv_last_page_len": -n})
         return out

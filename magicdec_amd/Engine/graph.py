@@ -17,6 +17,8 @@ import warnings
 
 import torch
 
+from .. import ops
+
 _STATE_BY_KIND = {
     "fwd": ("cachelens", "qo_indptr", "paged_kv_indices", "paged_kv_indptr", "paged_kv_last_page_len"),
     "draft": ("cachelens", "qo_indptr", "draft_paged_kv_indices", "draft_paged_kv_indptr",
@@ -33,6 +35,8 @@ class _Captured:
         self.graph = None
         self.static_in = None
         self.static_out = None
+        self.static_qo = None
+        self.step_ops = {}    # the launches around a replay (_prepared)
         self.names = ()       # state attributes this step reads
 
 
@@ -115,13 +119,23 @@ def _recover_from_failed_capture(g, home_stream):
             pass
 
 
-def run_captured(backend, key, fn, input_ids):
+def run_captured(backend, key, fn, input_ids, lead, tail):
+    """fn(input_ids) as a replayed graph, with the length tensors moved by `lead` before and `tail` behind it ({attribute: tokens}).
+    Once captured, a step is three launches: the lengths, the token ids and qo_indptr * n in one, the graph, the tokens out and the
+    lengths in another."""
     kind = key[0]
     full_key = (key, tuple(input_ids.shape), tuple(getattr(backend, "paged_kv_indices").shape),
                 tuple(getattr(backend, "draft_paged_kv_indices").shape) if hasattr(backend, "draft_paged_kv_indices")
                 else None)
     ent = backend._graphs.get(full_key)
-    if ent is None:
+    if ent is not None:
+        # a tensor the caller put in the place of the static one is moved itself; _bind_state then takes its values over
+        gs = _statics(backend)
+        own = {name: n for name, n in lead.items() if getattr(backend, name) is gs.get(name) and ops.step_adds(gs[name])}
+        backend._move({name: n for name, n in lead.items() if name not in own})
+    else:
+        backend._move(lead)
+        own = {}
         ent = _Captured()
         gs = _statics(backend)
         names = []
@@ -134,36 +148,41 @@ def run_captured(backend, key, fn, input_ids):
             names.append(name)
         ent.names = tuple(names)
         _bind_state(backend, ent)
-        ent.static_in = input_ids.clone()
-        # warm up on a side stream (hipBLASLt workspaces, lazy module loads, LDS attributes); a step never
-        # changes the lengths it reads, and re-running it rewrites the same KV rows with the same values
-        s = torch.cuda.Stream()
-        s.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(s):
-            for _ in range(2):
-                fn(ent.static_in)
-        torch.cuda.current_stream().wait_stream(s)
-        torch.cuda.synchronize()
-        g = torch.cuda.CUDAGraph()
-        err = None
-        home = torch.cuda.current_stream()
-        if _CAPTURE_POISONED[0] is not None:
-            # (the warm-up above and the agreement below still run: the ranks of a TP group must issue the same collectives)
-            err = RuntimeError(f"an earlier capture in this process was invalidated ({_CAPTURE_POISONED[0]}); this PyTorch "
-                               "build cannot capture again afterwards")
-        else:
-            try:
-                # thread_local: the RCCL watchdog thread of torch.distributed polls hipEventQuery concurrently; in the
-                # default "global" capture mode such a call from ANY thread invalidates the capture and kills the process
-                # ("operation not permitted when stream is capturing", seen intermittently with a TP group)
-                with torch.cuda.graph(g, capture_error_mode="thread_local"):
-                    ent.static_out = fn(ent.static_in)
-            except Exception as e:  # noqa: BLE001 -- e.g. a collective this RCCL build (or gloo) cannot capture
-                err = e
-                invalidated = "capture" in str(e).lower() and "hip error" in str(e).lower()
-                _recover_from_failed_capture(g, home)
-                if invalidated:
-                    _CAPTURE_POISONED[0] = f"step {key}: {type(e).__name__}"
+        ent.static_in = input_ids.clone(memory_format=torch.contiguous_format)
+        ent.static_qo = gs["qo_indptr"] * key[1]
+        backend._qo_bound = ent.static_qo                # what the captured step reads in place of qo_indptr * n
+        try:
+            # warm up on a side stream (hipBLASLt workspaces, lazy module loads, LDS attributes); a step never
+            # changes the lengths it reads, and re-running it rewrites the same KV rows with the same values
+            s = torch.cuda.Stream()
+            s.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(s):
+                for _ in range(2):
+                    fn(ent.static_in)
+            torch.cuda.current_stream().wait_stream(s)
+            torch.cuda.synchronize()
+            g = torch.cuda.CUDAGraph()
+            err = None
+            home = torch.cuda.current_stream()
+            if _CAPTURE_POISONED[0] is not None:
+                # (the warm-up above and the agreement below still run: the ranks of a TP group must issue the same collectives)
+                err = RuntimeError(f"an earlier capture in this process was invalidated ({_CAPTURE_POISONED[0]}); this PyTorch "
+                                   "build cannot capture again afterwards")
+            else:
+                try:
+                    # thread_local: the RCCL watchdog thread of torch.distributed polls hipEventQuery concurrently; in the
+                    # default "global" capture mode such a call from ANY thread invalidates the capture and kills the process
+                    # ("operation not permitted when stream is capturing", seen intermittently with a TP group)
+                    with torch.cuda.graph(g, capture_error_mode="thread_local"):
+                        ent.static_out = fn(ent.static_in)
+                except Exception as e:  # noqa: BLE001 -- e.g. a collective this RCCL build (or gloo) cannot capture
+                    err = e
+                    invalidated = "capture" in str(e).lower() and "hip error" in str(e).lower()
+                    _recover_from_failed_capture(g, home)
+                    if invalidated:
+                        _CAPTURE_POISONED[0] = f"step {key}: {type(e).__name__}"
+        finally:
+            backend._qo_bound = None
         # Under tensor parallelism every rank captures the same step at the same point of the same program, but a
         # capture can fail on ONE rank only (an allocation, a watchdog race): a rank replaying a graph while another
         # launches eagerly still issues the same collectives in the same order, yet the choice must not depend on
@@ -177,14 +196,45 @@ def run_captured(backend, key, fn, input_ids):
             backend._use_graphs = False
             backend._graphs.clear()
             del g
-            return fn(input_ids)
+            out = fn(input_ids)
+            backend._move(tail)
+            return out
         ent.graph = g
         backend._graphs[full_key] = ent
+        if all(name in gs for name in lead):             # what the steps from the next one on launch
+            _lead(ent, gs, lead, key[1], True)
     _bind_state(backend, ent)
-    if input_ids.data_ptr() != ent.static_in.data_ptr():
+    ids = input_ids.data_ptr() != ent.static_in.data_ptr()
+    if ids and not ops.step_copies(input_ids):
         ent.static_in.copy_(input_ids)
+        ids = False
+    _lead(ent, _statics(backend), own, key[1], ids).run(*([input_ids] if ids else []))
     ent.graph.replay()
-    return ent.static_out.clone()
+    add = []
+    for name, n in tail.items():
+        t = getattr(backend, name)
+        if ops.step_adds(t):
+            add.append((t, n))
+        else:
+            t.add_(n)
+    out = torch.empty_like(ent.static_out)
+    _prepared(ent, ("tail", tuple(tail.items())), add, [], [ent.static_out]).run(ent.static_out, into=(out,))
+    return out
+
+
+def _lead(ent, gs, own, n, ids):
+    return _prepared(ent, ("lead", ids, tuple(own.items())), [(gs[name], k) for name, k in own.items()],
+                     [(ent.static_qo, gs["qo_indptr"], n)], [ent.static_in] if ids else [])
+
+
+def _prepared(ent, key, add, scale, copies):
+    """The launch of these pieces, set up anew where a tensor lies elsewhere than last time (ops.StepOps keeps its tensors alive)."""
+    at = [(t.data_ptr(), t.numel()) for t, _ in add]
+    at += [(t.data_ptr(), t.numel()) for d in scale for t in d[:2]]
+    held = ent.step_ops.get(key)
+    if held is None or held[1] != at:
+        held = ent.step_ops[key] = (ops.StepOps(add, scale, copies), at)
+    return held[0]
 
 
 def clear_graphs(backend):

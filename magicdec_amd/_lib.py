@@ -60,6 +60,11 @@ class LatentArgs(ctypes.Structure):
                 ("force_plain", I)]
 
 
+class StepOp(ctypes.Structure):
+    """md_step_op of include/magicdec_hip.h."""
+    _fields_ = [("dst", P), ("src", P), ("src_stride", L), ("rows", I), ("cols", I), ("kind", I), ("a", I)]
+
+
 class HeadLinearArgs(ctypes.Structure):
     """md_head_linear_args of include/magicdec_hip.h."""
     _fields_ = [("x", P), ("w", P), ("out", P), ("gate", P), ("tail", P), ("cos_sin", P), ("qo_indptr", P), ("pos0", P),
@@ -141,6 +146,7 @@ _SIGNATURES = {
     "md_argmax_f32": (c_int, [P, L, I, I, P, P]),
     "md_argmax_tp_slots": (c_int, [P, L, I, I, L, I, I, P, P, P]),
     "md_tp_argmax_merge": (c_int, [P, P, I, I, P, P]),
+    "md_step_ops": (c_int, [ctypes.POINTER(StepOp), I, P]),
     "md_accept_rollback": (c_int, [P, P, P, I, P, P, P, P, P, I, I, I, I, L, L, L, P, P, P, P, P, P]),
 }
 

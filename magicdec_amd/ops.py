@@ -1238,3 +1238,60 @@ def accept_rollback(tokens_buffer, target_tokens, output, num_nodes, cachelens, 
                                  gamma, draft_rollback, draft_cap, int(eot_1), int(eot_2), int(max_nodes),
                                  _p(accept_nums), _p(bonus), _p(double_buffer), _p(cachelens_update), _p(flags),
                                  _stream()), "md_accept_rollback")
+
+
+STEP_ADD, STEP_SCALE, STEP_COPY, STEP_MAX = 0, 1, 2, 8
+
+
+class StepOps:
+    """The integer work around a decode step in one launch: add = [(int32 tensor, a)]: t += a; scale = [(dst, src, a)]: dst = src * a
+    (int32); copies = [dst]: int64 tensors that `run` fills, from sources of unit row stride.  What does not change from call to call is
+    set up once (a launch then costs the host one foreign call); the tensors are kept alive."""
+
+    def __init__(self, add=(), scale=(), copies=()):
+        self._ops, self._n, self._kept = (_lib.StepOp * STEP_MAX)(), 0, []
+        for t, a in add:
+            self._put(STEP_ADD, _i32(t), None, int(a))
+        for dst, src, a in scale:
+            if dst.shape != src.shape or not src.is_contiguous():
+                raise ValueError("step_ops: scale needs dense tensors of one shape")
+            self._put(STEP_SCALE, _i32(dst), _i32(src), int(a))
+        self._copies, self._first = list(copies), self._n
+        for dst in self._copies:
+            if dst.dtype != torch.int64:
+                raise ValueError("step_ops: copies are int64")
+            self._put(STEP_COPY, dst, None, 0)
+
+    def _put(self, kind, dst, src, a):
+        _gpu(dst, src)
+        if self._n == STEP_MAX or not dst.is_contiguous():
+            raise ValueError(f"step_ops: at most {STEP_MAX} pieces, into dense tensors")
+        self._ops[self._n] = _lib.StepOp(dst.data_ptr(), src.data_ptr() if src is not None else None, 0, 1, dst.numel(), kind, a)
+        self._kept += [dst, src]
+        self._n += 1
+
+    def run(self, *sources, into=()):
+        """One source per copy; `into` replaces the copies' destinations for this call (dense, same shapes)."""
+        n = self._n
+        for j, (dst, src) in enumerate(zip(into or self._copies, sources, strict=True)):
+            if dst.shape != src.shape or not step_copies(src) or not dst.is_contiguous():
+                raise ValueError("step_ops: copy needs int64 tensors of one shape, rows of unit stride")
+            op = self._ops[self._first + j]
+            op.dst, op.src = dst.data_ptr(), src.data_ptr()
+            if src.is_contiguous():
+                op.rows, op.cols = 1, src.numel()
+            else:
+                (op.rows, op.cols), op.src_stride = src.shape, src.stride(0)
+        if n:
+            check(_lib.load().md_step_ops(self._ops, n, _stream()), "md_step_ops")
+
+
+def step_copies(t):
+    """Can StepOps copy from this tensor?"""
+    return t.is_cuda and t.dtype == torch.int64 and t.numel() > 0 and (
+        t.is_contiguous() or (t.dim() == 2 and (t.shape[1] == 1 or t.stride(1) == 1)))
+
+
+def step_adds(t):
+    """Can StepOps add to this tensor?"""
+    return t.is_cuda and t.dtype == torch.int32 and t.numel() > 0 and t.is_contiguous()
