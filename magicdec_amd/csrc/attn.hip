@@ -104,12 +104,8 @@ __device__ __forceinline__ void cvt16_fp8_bf16(const u32x4 x, u32x4& lo, u32x4& 
     }
 }
 
-// NWV: wavefronts per workgroup, 4 or 8 (round 5).  A launch with <= 256 workgroups puts ONE on each CU; with four waves
-// that is half the loads in flight of the two-workgroups-per-CU launches (B x KH_local = 512 pairs at TP1).  Eight waves
-// share the workgroup's tile range round-robin and merge through LDS like four.  Measured (profiles/r05_attn_waves_ab.txt):
-// it is NOT what holds the bf16 TP shards at 71-82 % (KH_local = 1 / 2 / 4 and B = 32: 8 waves equal or 1-3 % slower -- the
-// deficit there is the fixed ~10 us of launch, tail and merge on an 85 us kernel), but the fp8 kernel with two M tiles
-// (cfg5's shard: Qwen g = 5, B = 128 x 64 K keys, 2 splits) gains 7 %: 0.378 -> 0.352 ms = 71 -> 76 % of the HBM peak.
+// NWV: wavefronts per workgroup, 4 or 8 (make_plan).  Eight share the workgroup's tile range round-robin and merge through LDS like four;
+// they help where fp8 tiles (a conversion per load) leave a lone workgroup's wavefronts busy and the chip has CUs to spare.
 template <int D, int QT, bool FP8, int NWV>
 __global__ __launch_bounds__(64 * NWV, NWV == 4 ? 2 : 1) void paged_attn_kernel(const AttnParams p) {
     constexpr int EB = FP8 ? 1 : 2;          // bytes per cache element
@@ -1169,10 +1165,7 @@ struct AttnPlan {
     int rows_cap;  // rows per item in the workspace (decode mode)
 };
 
-// split-KV target: one 4-wave workgroup per CU measured best on MI355X for every TP shard shape of the verify
-// step (B=64, 16K: 81 % / 80 % / 75 % / 70 % of HBM peak at KH_local = 8 / 4 / 2 / 1 vs 77 / 77 / 72 / 47 % at 1024);
-// per-workgroup prologue/epilogue and the partial-result round trip dominate once a wave owns < ~30 tiles
-int g_target_wgs = 256;  // dev knob: md_debug_set_attn_target_wgs
+int g_target_wgs = 0;    // dev knob (md_debug_set_attn_target_wgs): 0 = the rule below, n = ceil(n / pairs) splits
 int g_decode_nw = 0;     // dev knob (md_debug_set_attn_waves): 0 = the rule in make_plan, 4 / 8 = forced
 int g_prefill_nw = 0;     // dev knob (md_debug_set_prefill_kt): 0 = the measured rule below, 4 / 8 = forced
 
@@ -1193,8 +1186,15 @@ AttnPlan make_plan(int B, int n_max, int H, int KH, int max_pages, int page_size
         pl.splitq = false;
         pl.qt = rows <= 16 ? 1 : 2;
         pl.n_qgroups = 1;
-        const long max_tiles = (long)max_pages * page_size / 32;
-        long want = (g_target_wgs + (long)B * KH - 1) / ((long)B * KH);
+        const long max_tiles = (long)max_pages * page_size / 32, pairs = (long)B * KH;
+        // Splits: as many as leave at most ONE workgroup per CU.  A CU with a second workgroup finishes last, and a lone one streams
+        // faster: 12 requests of 16 000 keys (96 pairs of 8 kv heads, bf16 of 128) take 119 us in 192 workgroups, 158 in 288, 123 in
+        // 480; 20 requests (160 pairs) 192 us unsplit, 236 in 320, 203 in 480; 7 of 4 000 (56 pairs) 27 us in 224, 35 in 280.
+        // Between one and 1.25 workgroups per CU a few CUs would work twice as long as the rest: three splits level that (33 requests
+        // of 4 000 keys, 264 pairs: 118 -> 103 us; of 16 000: 438 -> 371) once a pair's stream is long (fp8, 4 000 keys: 68.5 -> 72.3,
+        // 16 000: 234 -> 214).  Beyond that splitting costs more than it levels (352 pairs 121.6 / 120.8 / 132 us, 520 pairs 190 / 193).
+        long want = pairs <= 256 ? 256 / pairs : pairs <= 320 && max_tiles * (fp8 ? 1 : 2) >= 256 ? 3 : 1;
+        if (g_target_wgs > 0) want = (g_target_wgs + pairs - 1) / pairs;
         long cap = max_tiles / 16;  // >= 16 tiles (4 per wave) per workgroup
         if (cap < 1) cap = 1;
         if (want > cap) want = cap;
@@ -1202,10 +1202,11 @@ AttnPlan make_plan(int B, int n_max, int H, int KH, int max_pages, int page_size
         if (want < 1) want = 1;
         pl.nsplit = (int)want;
         pl.rows_cap = pl.qt * 16;
-        // eight waves where measured faster: the fp8 two-M-tile kernel when the launch leaves one workgroup per CU and
-        // every wave still owns a stream of tiles (>= 8 each); see the kernel's header
-        const long wgs = (long)B * KH * pl.nsplit, tiles_per_wg = max_tiles / pl.nsplit;
-        pl.nw = (fp8 && pl.qt == 2 && wgs <= 256 && tiles_per_wg >= 64) ? 8 : 4;
+        // eight waves per workgroup for fp8 streams on a chip that is not full: 160 pairs of 8 000 keys 74 -> 61 us (two M tiles 87 ->
+        // 68), 224 of 16 000 164 -> 148; with every CU taken four are as fast or faster (256 pairs of 8 000: 91.4 / 94.9, 240: 64.5 /
+        // 65.8), and short streams gain nothing (160 of 2 000: 24.6 / 24.9).  bf16: four everywhere.
+        const long wgs = pairs * pl.nsplit, tiles_per_wg = max_tiles / pl.nsplit;
+        pl.nw = fp8 && wgs <= 224 && tiles_per_wg >= 96 ? 8 : 4;
         if (g_decode_nw == 4 || g_decode_nw == 8) pl.nw = g_decode_nw;
     } else {
         pl.splitq = true;
@@ -1348,7 +1349,7 @@ int launch_prefill(const AttnParams& p, int grid, int nw, hipStream_t st) {
 }  // namespace
 
 #ifdef MD_DEV_KNOBS   // include/magicdec_hip_dev.h: tuning knobs, not part of the drop-in boundary
-extern "C" void md_debug_set_attn_target_wgs(int n) { g_target_wgs = n > 0 ? n : 256; }
+extern "C" void md_debug_set_attn_target_wgs(int n) { g_target_wgs = n > 0 ? n : 0; }
 extern "C" void md_debug_set_attn_waves(int nw) { g_decode_nw = (nw == 4 || nw == 8) ? nw : 0; }
 extern "C" void md_debug_set_prefill_mfma32(int kt) {
     // < 0: the rule, 0: the 16x16 kernel, 32 | 64 | 128: keys per tile; 129: 128 keys with the first version's V pairing

@@ -264,7 +264,9 @@ long keys_of(const md_xattn_args* a) {
 int decode_splits(const md_xattn_args* a) {
     const long keys = keys_of(a);
     const long tiles = (keys + 31) / 32 + 1, pairs = (long)a->B * a->KH;
-    long want = (g_target_wgs + pairs - 1) / pairs;
+    // at most one workgroup per CU: a second one on some CUs makes those finish last (one step of 2 layers with heads of 64: 12
+    // requests of 1 500 keys 170.7 us in 288 workgroups, 165.5 in 192; 20 of 1 000 176.6 in 320, 170.0 in 160)
+    long want = pairs < g_target_wgs ? g_target_wgs / pairs : 1;
     const long cap = tiles / 16 > 1 ? tiles / 16 : 1;        // >= 16 tiles (4 per wavefront) per workgroup
     if (want > cap) want = cap;
     return (int)(want < 1 ? 1 : want > 64 ? 64 : want);
