@@ -243,6 +243,9 @@ int md_silu_mul(const void* a, const void* b, int64_t a_row_stride, int64_t b_ro
 #define MD_EPI_NONE 0
 #define MD_EPI_SWIGLU 1
 #define MD_EPI_GEGLU 3 /* MD_EPI_SWIGLU's layout; out = bf16(gelu_tanh(h1) * h3), fp32 up to the one rounding */
+/* md_unpack_weight: a bf16 matrix in the streaming layout (w_packed = 1) back to w[N][K]; halves: packed as 16 rows of the first N/2
+ * beside 16 of the second (SwiGLU). */
+int md_unpack_weight(const void* w_packed, void* w, int N, int K, int halves, md_stream_t stream);
 int md_linear_supported(int M, int N, int K, int epilogue);
 size_t md_linear_workspace_bytes(int M, int N, int K, int epilogue);
 int md_linear(const void* x, int64_t ldx, const void* w, int w_dtype, int w_packed, const void* scales,

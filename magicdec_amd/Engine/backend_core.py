@@ -209,14 +209,15 @@ class _BackendBase:
         return dict(head_rows=torch.arange(1, self.batch_size + 1, device=self.device) * n - 1)
 
     def _prefill_begin(self):
-        """Prefill-sized products run on the library GEMM over the row-major weights: re-materialise the ones released
-        after the previous prefill (Transformer.restore_rowmajor)."""
-        if hasattr(self.model, "restore_rowmajor"):
-            self.model.restore_rowmajor()
+        """Prefill-sized products run on the library GEMM over the row-major weights: the ones released after the previous prefill
+        come back as the portions ask for them (a head that only ever sees the last rows is not among them)."""
+        if hasattr(self.model, "restore_on_demand"):
+            self.model.restore_on_demand(True)
 
     def _prefill_end(self):
         """Decode reads most weights in the streaming layout only: free their row-major tensors (one resident copy)."""
         if hasattr(self.model, "release_rowmajor"):
+            self.model.restore_on_demand(False)
             self.model.release_rowmajor()
 
     def _reset_kv_calibration(self):

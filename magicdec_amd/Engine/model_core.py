@@ -503,25 +503,36 @@ class Transformer(nn.Module):
         return freed
 
     def restore_rowmajor(self):
-        """Before a prefill: every released row-major tensor back from its streaming-layout copy (one permute each)."""
+        """Every released row-major tensor back from its streaming-layout copy."""
         for k in list(getattr(self, "_released", ())):
-            w = self._by_id[k]
-            rows = self._packed[k].unpack().contiguous()
-            role, i = self._roles[k]
-            if role == "w13":
-                ff = self.layers[i].feed_forward
-                inter = rows.shape[0] // 2
-                w.set_(rows)
-                ff.w1.weight.data = w[:inter]
-                ff.w3.weight.data = w[inter:]
-            else:
-                w.data = rows
-            self._released.discard(k)
+            self._restore(k)
+
+    def _restore(self, k):
+        w = self._by_id[k]
+        rows = self._packed[k].unpack().contiguous()
+        role, i = self._roles[k]
+        if role == "w13":
+            ff = self.layers[i].feed_forward
+            inter = rows.shape[0] // 2
+            w.set_(rows)
+            ff.w1.weight.data = w[:inter]
+            ff.w3.weight.data = w[inter:]
+        else:
+            w.data = rows
+        self._released.discard(k)
+
+    _on_demand = False       # during a prefill: a released tensor that a library GEMM asks for comes back until release_rowmajor()
+
+    def restore_on_demand(self, on):
+        self._on_demand = on
 
     def _resident(self, w):
         """The row-major tensor of `w` for a library GEMM; a released one is unpacked for this call only (a decode step the
         policy prediction did not foresee: correct, slow, and reported once)."""
         if id(w) in getattr(self, "_released", ()):
+            if self._on_demand:
+                self._restore(id(w))
+                return w
             if not getattr(self, "_warned_transient", False):
                 self._warned_transient = True
                 print(f"[magicdec_amd] a library GEMM needs the released row-major weight {tuple(w.shape)} in a decode step "

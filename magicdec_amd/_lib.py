@@ -100,6 +100,7 @@ _SIGNATURES = {
     "md_ar_destroy": (c_int, [P]),
     "md_streaming_shift_append": (c_int, [P, P, L, L, P, I, I, I, I, I, I, I, I, P]),
     "md_streaming_rotate": (c_int, [P, P, I, I, I, I, I, I, P, I, P]),
+    "md_unpack_weight": (c_int, [P, P, I, I, I, P]),
     "md_linear_supported": (c_int, [I, I, I, I]),
     "md_linear_workspace_bytes": (c_size_t, [I, I, I, I]),
     "md_linear": (c_int, [P, L, P, I, I, P, P, P, L, I, I, I, I, P, c_size_t, P]),

@@ -645,6 +645,29 @@ int linear_impl(const void* x, int64_t ldx, const void* w, int w_dtype, int w_pa
     MD_CHECK_LAUNCH("md_linear");
     return MD_OK;
 }
+// The streaming layout back into rows, 16-byte pieces through LDS: a workgroup takes one 32-row tile and 32 of its k-steps -- 32 KB read
+// in one run, written as 1-KB runs of each row (piece pitch 33: a wavefront's transposed reads spread over all banks).  Bound by HBM,
+// 2 x 2 x N x K bytes: the gate|up matrix of an 8B layer (470 MB both ways) takes 78.8 us, 6.0 TB/s; as torch
+// permutes and copies it was three passes, about 260 us.
+constexpr int kUnpackSteps = 32;
+
+__global__ __launch_bounds__(256) void unpack_weight_kernel(const u32x4* __restrict__ packed, u32x4* __restrict__ out, int N, int K,
+                                                            int inter) {
+    __shared__ u32x4 img[2 * kUnpackSteps * 33];
+    const int tid = threadIdx.x, t = blockIdx.y, s0 = blockIdx.x * kUnpackSteps, pieces = K / 8;      // 16-byte pieces of a row
+    const int steps = min(kUnpackSteps, K / 16 - s0);
+    const u32x4* src = packed + ((int64_t)t * (K / 16) + s0) * 64;
+    for (int i = tid; i < steps * 64; i += 256) img[(i >> 5) * 33 + (i & 31)] = __builtin_nontemporal_load(src + i);
+    __syncthreads();
+    const int c = tid & 63;
+    if (c >= 2 * steps) return;
+    for (int j = tid >> 6; j < 32; j += 4) {
+        // row j of the tile: of one matrix, or 16 rows of the first half beside 16 of the second
+        const int half = inter ? j >> 4 : 0, row = inter ? t * 16 + (j & 15) : t * 32 + j;
+        if (row < (inter ? inter : N)) out[(int64_t)(half * inter + row) * pieces + 2 * s0 + c] = img[c * 33 + j];
+    }
+}
+
 }  // namespace
 
 extern "C" int md_linear(const void* x, int64_t ldx, const void* w, int w_dtype, int w_packed, const void* scales,
@@ -747,5 +770,16 @@ extern "C" int md_linear_add_rmsnorm(const void* x, int64_t ldx, const void* w, 
                                                norm_weight, h_out, y_out, eps, st);
     if (rc != MD_OK) return rc;
     MD_CHECK_LAUNCH("md_linear_add_rmsnorm");
+    return MD_OK;
+}
+
+extern "C" int md_unpack_weight(const void* w_packed, void* w, int N, int K, int halves, md_stream_t stream) {
+    MD_CHECK_ARG(w_packed && w && ((((uintptr_t)w_packed) | (uintptr_t)w) & 15) == 0, "md_unpack_weight: 16-byte aligned tensors needed");
+    MD_CHECK_ARG(N > 0 && K > 0 && K % 16 == 0 && (!halves || N % 2 == 0), "md_unpack_weight: bad shape N=%d K=%d", N, K);
+    const int tiles = halves ? (N / 2 + 15) / 16 : (N + 31) / 32;
+    MD_CHECK_ARG(tiles <= 65535, "md_unpack_weight: %d rows", N);
+    hipLaunchKernelGGL(unpack_weight_kernel, dim3((K / 16 + kUnpackSteps - 1) / kUnpackSteps, tiles), dim3(256), 0, (hipStream_t)stream,
+                       (const u32x4*)w_packed, (u32x4*)w, N, K, halves ? N / 2 : 0);
+    MD_CHECK_LAUNCH("md_unpack_weight");
     return MD_OK;
 }

@@ -302,10 +302,13 @@ class PackedWeight:
         self.data = rows.view(t, 32, K // 16, 2, 8).permute(0, 2, 3, 1, 4).contiguous()
 
     def unpack(self):
-        """The row-major [N, K] tensor this copy was built from (the inverse permute: plumbing).  Used to re-materialise
-        a row-major weight that was released after prefill (Transformer.release_rowmajor): the streaming layout is then
-        the ONE resident copy of the weight."""
+        """The row-major [N, K] tensor this copy was built from.  Used to re-materialise a row-major weight that was released after
+        prefill (Transformer.release_rowmajor): the streaming layout is then the ONE resident copy of the weight."""
         t, K = self.data.shape[0], self.K
+        if self.data.is_cuda and self.dtype == torch.bfloat16 and t <= 65535:
+            out = torch.empty((self.N, K), dtype=self.dtype, device=self.data.device)
+            check(_lib.load().md_unpack_weight(_p(self.data), _p(out), self.N, K, int(self.swiglu), _stream()), "md_unpack_weight")
+            return out
         rows = self.data.permute(0, 3, 1, 2, 4).reshape(t, 32, K)      # [t, s, kh, j, e] -> [t, j, (s, kh, e)]
         if not self.swiglu:
             return rows.view(t * 32, K)[:self.N] if t * 32 != self.N else rows.view(t * 32, K)
