@@ -12,17 +12,17 @@
 //   indices = top-(budget-W) of score, descending score, ties -> lowest index
 //   draft rows = K,V[indices] ++ K,V[S-W:S]
 //
-// Five small launches, none on the timed decode path (once per prefill per layer):
-//   stats   : row max / sum-exp partials per 2048-column chunk (kChunkCols)   (MFMA scores; float64 sums)
+// Seven small launches, none on the timed decode path (once per prefill per layer):
+//   stats   : row max / sum-exp partials per column chunk   (MFMA scores; float64 sums)
 //   finalize: per-row (max, 1 / sum) of the whole context from the chunk partials
 //   accum   : recompute scores, p, 8-row group sums, bf16 chunk accumulation
-//   select  : pool + group sum + exact radix select + bitonic sort (one WG per b,kvh)
+//   pool    : pool + group sum
+//   select  : exact radix select, ranked by counting (one WG per b,kvh)
 //   gather  : copy the selected rows into the draft pages
 #include "md_common.h"
 
 namespace {
 
-constexpr int kChunkCols = 2048;
 
 struct SnapParams {
     const bf16_t* q;      // [B*W, H, D]
@@ -30,9 +30,10 @@ struct SnapParams {
     const float* k_scale;
     const int32_t* page_indices;
     const int32_t* page_indptr;
-    double* partials;       // [B*KH][L][nch][2] = (row max, sum of exp) per 2048-column chunk (kChunkCols), float64
+    double* partials;       // [B*KH][L][nch][2] = (row max, sum of exp) per `cols` columns, float64
     unsigned short* aws;    // [B][H][S-W] bf16 bits
     int B, H, KH, g, W, S, L, nch, page_size;
+    int cols;             // columns per workgroup of the two score kernels
     int64_t page_stride;
     int slot_stride;      // elements between rows of a page: KH*D (NHD) or D (HND)
     int head_stride;      // elements between kv heads: D (NHD) or page_size*D (HND)
@@ -77,6 +78,28 @@ __device__ __forceinline__ void load_kfrag(const SnapParams& p, int b, int kvh, 
     }
 }
 
+// The fragments of 32 consecutive columns (two 16-column groups).  Pages of a multiple of 32 rows hold all of them in one page, which is
+// then looked up once per wavefront; rows past the context are not read from beyond it (zeros).
+template <int D, bool FP8>
+__device__ __forceinline__ void load_kfrag2(const SnapParams& p, int b, int kvh, int col0, bool whole, int lq, int lc,
+                                            bf16x8 (&kf)[2][D / 32]) {
+    if (!FP8 && whole && col0 + 32 <= p.S) {
+        const int page = col0 / p.page_size;
+        const int64_t pid = p.page_indices[p.page_indptr[b] + page];
+        const bf16_t* kp = reinterpret_cast<const bf16_t*>(p.cache) + pid * p.page_stride +
+                           (int64_t)(col0 - page * p.page_size) * p.slot_stride + (int64_t)kvh * p.head_stride;
+        const unsigned off = (unsigned)(lq * p.slot_stride + lc * 8);
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int ks = 0; ks < D / 32; ++ks)
+                kf[c][ks] = *reinterpret_cast<const bf16x8*>(kp + (int64_t)c * 16 * p.slot_stride + off + ks * 32);
+    } else {
+        load_kfrag<D, FP8>(p, b, kvh, col0, lq, lc, kf[0]);
+        load_kfrag<D, FP8>(p, b, kvh, col0 + 16, lq, lc, kf[1]);
+    }
+}
+
 // exp(x) for x <= 0 in float64, ~1 ulp: k = rint(x log2 e), r = x - k ln2 (two-part constant), degree-13 Taylor polynomial
 // (|r| <= 0.347: remainder 4e-18), scaled by 2^k -- 17 dependent f64 instructions instead of OCML's exp().
 __device__ __forceinline__ double exp_neg(double x) {
@@ -106,18 +129,16 @@ __device__ __forceinline__ double exp_neg(double x) {
 // probabilities must be correctly rounded bf16(exp(s - M) / Z) (see "Rounding sequence" above: an fp32 evaluation with
 // another summation order flips ~1e-4 of those roundings).  Rounds 1-3 evaluated exp() in float64 per element: a
 // billion OCML calls per layer at the BASELINE shape, 0.21 TB/s of K bytes = 2.6 % of the HBM roofline (VERDICT r3 weak
-// #3).  Now exp(v) of every bf16 value with 2^-12 <= |v| < 2^9 sits in a float64 table in LDS (filled with OCML's exp once
+// #3).  Now exp(v) of every bf16 value with 2^-14 <= |v| < 2^9 sits in a float64 table in LDS (filled with OCML's exp once
 // per call): the row sum is  sum_i T[s_i]  (reference 0: e^512 * 65 536 columns is far below the float64 range) and a
-// probability is  T[s] * (exp(-M) / Z)  -- one LDS gather and one f64 multiply.  The few scores outside the table (|s| >=
-// 512, |s| < 2^-12, masked) take the lean exp_neg() above against a running maximum, so nothing overflows whatever the raw
-// (unscaled) scores are.
-// Round 5: round 4's table ended at |v| < 16, which covered the microbenchmark's N(0, 2.4^2) scores
-// but not the engine's: the UNSCALED q.k of a seeded-random 1B layer is ~N(0, 6.5^2) (1.4 % of the scores beyond 16, i.e.
-// every 256-score wave tile on the slow path: 5.0 ms per layer in the bench trace against 1.76 on the microbenchmark), and a
-// trained checkpoint's reaches the hundreds.  21 binades x 128 mantissas x 2 signs = 5 376 entries = 42 KB, laid out
-// [magnitude][sign] so that the byte offset of a score is (magnitude index << 4) | (sign << 3) and still fits 16 bits.
-constexpr int kTabE0 = 115;                 // biased bf16 exponent of 2^-12
-constexpr int kTabBinades = 21;             // 2^-12 .. 2^9
+// probability is  T[s] * (exp(-M) / Z)  -- one LDS gather and one f64 multiply.  Of the few scores outside the table, tiny
+// ones (|s| < 2^-14) are a short polynomial, the others (|s| >= 512, masked) take the lean exp_neg() above against a running maximum, so
+// nothing overflows whatever the raw (unscaled) scores are.
+// The UNSCALED q.k of a seeded-random 1B layer is ~N(0, 6.5^2) and a trained checkpoint's reaches the hundreds: the table covers 23
+// binades x 128 mantissas x 2 signs = 5 888 entries = 46 KB (two workgroups of pass 1 per CU), laid out [magnitude][sign] so that the
+// byte offset of a score is (magnitude index << 4) | (sign << 3) and still fits 16 bits.
+constexpr int kTabE0 = 113;                 // biased bf16 exponent of 2^-14
+constexpr int kTabBinades = 23;             // 2^-14 .. 2^9
 constexpr int kTabMag = kTabBinades * 128;  // magnitude indices: (exponent - E0) * 128 + mantissa
 constexpr int kTabN = 2 * kTabMag;          // [magnitude][sign]
 __device__ double g_exp_tab[kTabN];
@@ -129,6 +150,13 @@ __global__ __launch_bounds__(256) void snapkv_tab_kernel() {
     g_exp_tab[i] = exp((double)bf16_bits_to_f32((unsigned short)bits));
 }
 
+// exp(v) for |v| < 2^-14: the next term is below 2^-60
+__device__ __forceinline__ double exp_tiny(float v) {
+    const double x = (double)v;
+    return fma(x, fma(x, fma(x, 1.0 / 6.0, 0.5), 1.0), 1.0);
+}
+__device__ __forceinline__ bool is_tiny(float v) { return fabsf(v) < 6.103515625e-05f; }
+
 // table index of a bf16 value held in a float, or -1 (outside the table: tiny, large, zero, inf)
 __device__ __forceinline__ int tab_index(float s) {
     const unsigned int bits = __float_as_uint(s) >> 16;
@@ -136,30 +164,36 @@ __device__ __forceinline__ int tab_index(float s) {
     return a < (unsigned int)kTabMag ? (int)((a << 1) | (bits >> 15)) : -1;
 }
 
-// Two scores at a time: `w` = two bf16 values in one dword (v_cvt_pk_bf16_f32).  Returns the two table BYTE offsets in the
-// halves of a dword and ORs into `bad` a non-zero pattern if either value lies outside the table.
+// Two scores at a time: `w` = two bf16 values in one dword (v_cvt_pk_bf16_f32).  With d = bits - (E0 << 7) a score in the table has
+// magnitude index d & 0x7fff < kTabMag < 4096, so that rotating d left by four gives its byte offset (magnitude x 16 + sign x 8); any
+// other d leaves an offset past the last entry or with one of its low three bits set.  `top` (maximum) and `low` (or) collect both over
+// a batch of scores: tab_outside says whether all of them lie inside.
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
     const bf16x2 pk = {f32_to_bf16(a), f32_to_bf16(b)};
     return *reinterpret_cast<const unsigned int*>(&pk);
 }
-__device__ __forceinline__ unsigned int tab_offsets2(unsigned int w, unsigned int& bad) {
-    const u16x2 base = {(unsigned short)(kTabE0 << 7), (unsigned short)(kTabE0 << 7)};
-    const u16x2 lim = {(unsigned short)(kTabMag - 1), (unsigned short)(kTabMag - 1)};
-    const u16x2 d = *reinterpret_cast<const u16x2*>(&w) - base;            // v_pk_sub_u16 (a tiny magnitude borrows from the sign bit)
-    const unsigned int u = *reinterpret_cast<const unsigned int*>(&d);
-    const unsigned int a = u & 0x7fff7fffu;                                // (exponent - E0) * 128 + mantissa per half
-    const u16x2 av = *reinterpret_cast<const u16x2*>(&a);
-    const u16x2 cl = __builtin_elementwise_min(av, lim);                   // v_pk_min_u16
-    bad |= a ^ *reinterpret_cast<const unsigned int*>(&cl);                // a half beyond the last binade (or wrapped: tiny)
-    // offsets from the CLAMPED magnitudes: an out-of-range half -- which the callers discard through `bad` --
-    // then points at the last table entry instead of carrying into its neighbour's half
-    const unsigned int c = *reinterpret_cast<const unsigned int*>(&cl);
-    return (c << 4) | ((u >> 12) & 0x00080008u);                           // magnitude x 16 bytes + sign x 8 (< 2^16 per half)
+__device__ __forceinline__ unsigned int tab_offsets2(unsigned int w, u16x2& top, unsigned int& low) {
+    const u16x2 d = *reinterpret_cast<const u16x2*>(&w) - (unsigned short)(kTabE0 << 7);
+    const u16x2 r = d * (unsigned short)16 + (d >> (unsigned short)12);
+    top = __builtin_elementwise_max(top, r);
+    const unsigned int o = *reinterpret_cast<const unsigned int*>(&r);
+    low |= o;
+    return o;
+}
+__device__ __forceinline__ bool tab_outside(u16x2 top, unsigned int low) {
+    return (low & 0x00070007u) != 0 || top[0] >= kTabN * 8 || top[1] >= kTabN * 8;
+}
+__device__ __forceinline__ double tab_at(const double* tab, unsigned int offset) {
+    return *reinterpret_cast<const double*>(reinterpret_cast<const unsigned char*>(tab) + offset);
 }
 
 // (m, Z) <- merge of two partial softmax sums  sum exp(s - m)
 __device__ __forceinline__ void merge_mz(double& m, double& Z, double m2, double Z2) {
+    if (m2 == m) {                                       // the common case: both sums with reference 0
+        Z += Z2;
+        return;
+    }
     const double mn = fmax(m, m2);
     if (!(mn > -INFINITY)) return;
     Z = (m > -INFINITY ? Z * exp_neg(m - mn) : 0.0) + (m2 > -INFINITY ? Z2 * exp_neg(m2 - mn) : 0.0);
@@ -192,15 +226,18 @@ __device__ __forceinline__ bool masked(const SnapParams& p, int rg, int col) {
 constexpr int kSnapWaves = 8;               // wavefronts per workgroup of the two score kernels (they share table + Q image)
 
 // Pass 1: per (row, column chunk) the pair (m, Z), Z = sum over the chunk's columns of exp(s - m).  A lane owns ONE row
-// of every 16-row tile (rows <-> lanes lq) and 4 of the tile's 16 columns, and keeps the table sum of each of its rows
+// of every 16-row tile (rows <-> lanes lq) and 4 of a tile's 16 columns, and keeps the table sum of each of its rows
 // (reference 0) in registers: no cross-lane traffic until the end.  Out-of-table scores (rare) go to a per-wave (m, Z)
-// pair per row in LDS.  The next 16-column K fragment is in flight while the current one is consumed.
+// pair per row in LDS.  A wavefront takes 2 x 2 tiles at a time: two column groups share the query fragments, and the 16 table
+// gathers of a lane are in flight together -- tile by tile, each waiting for its products and then for its gathers, this kernel took
+// 150 us for 16 requests of 16 000 keys (8 kv heads of 64, 128 rows each), against 120.  Bound by LDS: 4 gathers of 8 random
+// bytes per lane and tile, about 7 cycles each, beside 8 for the fragments.
 template <int D, bool FP8, int RTM>     // RTM: register-resident 16-row tiles (8 for g * W <= 128 rows, else kMaxRT)
-__global__ __launch_bounds__(64 * kSnapWaves, 4) void snapkv_stats_kernel(const SnapParams p) {
+__global__ __launch_bounds__(64 * kSnapWaves, D == 64 && RTM == 8 ? 4 : 2) void snapkv_stats_kernel(const SnapParams p) {
     __shared__ double tab[kTabN];
     extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];   // Q image, then [waves][L][2] doubles
     const int chunk = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lq = lane & 15, lc = lane >> 4;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lq = lane & 15, lc = lane >> 4;
     unsigned char* qimg = dyn;
     double* ms = reinterpret_cast<double*>(dyn + (size_t)p.L * (D * 2 + kQPad));
     double* sw = ms + (size_t)wave * p.L * 2;                 // this wave's (m, Z) of the out-of-table scores, per row
@@ -212,71 +249,109 @@ __global__ __launch_bounds__(64 * kSnapWaves, 4) void snapkv_stats_kernel(const 
     }
     __syncthreads();
     const int RT = p.L / 16;
+    const bool whole = p.page_size % 32 == 0;
     const float kscale = FP8 ? p.k_scale[kvh] : 1.0f;
     double zt[RTM];
 #pragma unroll
     for (int rt = 0; rt < RTM; ++rt) zt[rt] = 0.0;
-    const int ncg = min(kChunkCols / 16, (p.S - chunk * kChunkCols + 15) / 16);      // 16-column groups of this chunk
-    bf16x8 kf[D / 32], kn[D / 32];
-    if (wave < ncg) load_kfrag<D, FP8>(p, b, kvh, chunk * kChunkCols + wave * 16, lq, lc, kf);
+    const int ncg = (min(p.cols, p.S - chunk * p.cols) + 31) / 32;                   // 32-column groups of this chunk
+    bf16x8 kf[2][D / 32], kn[2][D / 32];
+    if (wave < ncg) load_kfrag2<D, FP8>(p, b, kvh, chunk * p.cols + wave * 32, whole, lq, lc, kf);
     for (int cg = wave; cg < ncg; cg += kSnapWaves) {
-        const int col0 = chunk * kChunkCols + cg * 16;
-        if (cg + kSnapWaves < ncg) load_kfrag<D, FP8>(p, b, kvh, col0 + kSnapWaves * 16, lq, lc, kn);
-        const bool tail = col0 + 16 > p.S - p.W;                     // wave-uniform: only these columns can be masked
+        const int col0 = chunk * p.cols + cg * 32;
+        if (cg + kSnapWaves < ncg) load_kfrag2<D, FP8>(p, b, kvh, col0 + kSnapWaves * 32, whole, lq, lc, kn);
+        const bool tail = col0 + 32 > p.S - p.W;                     // wave-uniform: only these columns can be masked
 #pragma unroll
-        for (int rt = 0; rt < RTM; ++rt) {
-            if (rt < RT) {                                           // wave-uniform
-                const unsigned char* qp = qimg + (rt * 16 + lq) * (D * 2 + kQPad) + lc * 16;
-                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int r0 = 0; r0 < RTM; r0 += 2) {
+            if (r0 < RT) {                                           // wave-uniform
+                const bool two = r0 + 1 < RT;
+                unsigned int w[2][2][2];                             // scores rounded to bf16, two per dword: [row tile][column group]
 #pragma unroll
-                for (int ks = 0; ks < D / 32; ++ks)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[ks], *reinterpret_cast<const bf16x8*>(qp + ks * 64),
-                                                                  acc, 0, 0, 0);
-                // lane (lq, lc): row rt*16 + lq, columns col0 + lc*4 + j; scores rounded to bf16 two per dword
-                const unsigned int w0 = pack_bf16(acc[0] * kscale, acc[1] * kscale);    // kscale = 1 for a bf16 cache
-                const unsigned int w1 = pack_bf16(acc[2] * kscale, acc[3] * kscale);
-                unsigned int bad = 0;
-                const unsigned int o0 = tab_offsets2(w0, bad), o1 = tab_offsets2(w1, bad);
-                const unsigned char* tb = reinterpret_cast<const unsigned char*>(tab);
-                // hot path, no divergence: every score of the wave's tile is in the table and no column can be masked
-                if (!tail && __builtin_amdgcn_ballot_w64(bad != 0) == 0) {
-                    zt[rt] += (*reinterpret_cast<const double*>(tb + (o0 & 0xffffu)) +
-                               *reinterpret_cast<const double*>(tb + (o0 >> 16))) +
-                              (*reinterpret_cast<const double*>(tb + (o1 & 0xffffu)) +
-                               *reinterpret_cast<const double*>(tb + (o1 >> 16)));
-                } else {
-                    const float v[4] = {bf16_bits_to_f32((unsigned short)(w0 & 0xffffu)), bf16_bits_to_f32((unsigned short)(w0 >> 16)),
-                                        bf16_bits_to_f32((unsigned short)(w1 & 0xffffu)), bf16_bits_to_f32((unsigned short)(w1 >> 16))};
-                    int ti[4];
+                for (int u = 0; u < 2; ++u) {
+                    const unsigned char* qp = qimg + ((two ? r0 + u : r0) * 16 + lq) * (D * 2 + kQPad) + lc * 16;
+                    f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) ti[j] = tab_index(v[j]);
-                    const int rg = rt * 16 + lq;
-                    double m2 = -INFINITY, z2 = 0.0;                 // this lane's out-of-table scores of the tile
+                    for (int ks = 0; ks < D / 32; ++ks) {
+                        const bf16x8 qf = *reinterpret_cast<const bf16x8*>(qp + ks * 64);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        if (tail && masked(p, rg, col0 + lc * 4 + j)) continue;    // (an integer modulo: off the hot path)
-                        if (ti[j] >= 0) {
-                            zt[rt] += tab[ti[j]];
-                        } else if (v[j] > -INFINITY) {
-                            merge_mz(m2, z2, (double)v[j], 1.0);
-                        }
+                        for (int c = 0; c < 2; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[c][ks], qf, acc[c], 0, 0, 0);
                     }
-                    // the four lanes of a row take turns at the wave's LDS pair
+                    // lane (lq, lc): row rt*16 + lq, columns col0 + c*16 + lc*4 + j
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        if (lc == q && m2 > -INFINITY) {
-                            double m = sw[rg * 2], Z = sw[rg * 2 + 1];
-                            merge_mz(m, Z, m2, z2);
-                            sw[rg * 2] = m;
-                            sw[rg * 2 + 1] = Z;
+                    for (int c = 0; c < 2; ++c) {
+                        if (FP8) acc[c] *= kscale;
+                        w[u][c][0] = pack_bf16(acc[c][0], acc[c][1]);
+                        w[u][c][1] = pack_bf16(acc[c][2], acc[c][3]);
+                    }
+                }
+                u16x2 top = {0, 0};
+                unsigned int low = 0, o[2][2][2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int c = 0; c < 2; ++c)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) o[u][c][h] = tab_offsets2(w[u][c][h], top, low);
+                // hot path, no divergence: every score of the batch is in the table and no column can be masked
+                if (!tail && __builtin_amdgcn_ballot_w64(tab_outside(top, low)) == 0) {
+                    double e[2][2][4];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u)
+#pragma unroll
+                        for (int c = 0; c < 2; ++c)
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                e[u][c][j] = tab_at(tab, j & 1 ? o[u][c][j >> 1] >> 16 : o[u][c][j >> 1] & 0xffffu);
+#pragma unroll
+                    for (int u = 0; u < 2; ++u)
+#pragma unroll
+                        for (int c = 0; c < 2; ++c) {
+                            const double t = (e[u][c][0] + e[u][c][1]) + (e[u][c][2] + e[u][c][3]);
+                            if (u == 0 || two) zt[r0 + u] += t;
                         }
-                        __builtin_amdgcn_wave_barrier();
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        if (u == 1 && !two) continue;
+                        const int rg = (r0 + u) * 16 + lq;
+                        double m2 = -INFINITY, z2 = 0.0, t = 0.0;    // this lane's out-of-table scores, its table sum
+#pragma unroll
+                        for (int c = 0; c < 2; ++c) {
+                            const unsigned int w0 = w[u][c][0], w1 = w[u][c][1];
+#pragma unroll 1
+                            for (int j = 0; j < 4; ++j) {
+                                const unsigned int wj = j < 2 ? w0 : w1;
+                                const float v = bf16_bits_to_f32((unsigned short)(j & 1 ? wj >> 16 : wj & 0xffffu));
+                                if (tail && masked(p, rg, col0 + c * 16 + lc * 4 + j)) continue;   // (an integer modulo: off the hot path)
+                                const int ti = tab_index(v);
+                                if (ti >= 0)
+                                    t += tab[ti];
+                                else if (is_tiny(v))
+                                    t += exp_tiny(v);
+                                else if (v > -INFINITY)
+                                    merge_mz(m2, z2, (double)v, 1.0);
+                            }
+                        }
+                        zt[r0 + u] += t;
+                        // the four lanes of a row take turns at the wave's LDS pair
+#pragma unroll 1
+                        for (int q = 0; q < 4; ++q) {
+                            if (lc == q && m2 > -INFINITY) {
+                                double m = sw[rg * 2], Z = sw[rg * 2 + 1];
+                                merge_mz(m, Z, m2, z2);
+                                sw[rg * 2] = m;
+                                sw[rg * 2 + 1] = Z;
+                            }
+                            __builtin_amdgcn_wave_barrier();
+                        }
                     }
                 }
             }
         }
 #pragma unroll
-        for (int ks = 0; ks < D / 32; ++ks) kf[ks] = kn[ks];
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int ks = 0; ks < D / 32; ++ks) kf[c][ks] = kn[c][ks];
     }
     // per-lane -> per-row of this wave (the 4 lanes lq + 16 lc of a row), then over the waves, then out
 #pragma unroll
@@ -288,7 +363,7 @@ __global__ __launch_bounds__(64 * kSnapWaves, 4) void snapkv_stats_kernel(const 
             if (lc == 0) {
                 const int rg = rt * 16 + lq;
                 double m = Z > 0.0 ? 0.0 : -INFINITY;
-                merge_mz(m, Z, sw[rg * 2], sw[rg * 2 + 1]);
+                if (sw[rg * 2] > -INFINITY) merge_mz(m, Z, sw[rg * 2], sw[rg * 2 + 1]);
                 sw[rg * 2] = m;
                 sw[rg * 2 + 1] = Z;
             }
@@ -315,20 +390,25 @@ __global__ __launch_bounds__(256) void snapkv_finalize_kernel(const SnapParams p
     pp[1] = 1.0 / Z;
 }
 
-constexpr int kAccumCols = 2048;     // columns per workgroup of the accumulate kernel (16 groups of 16 per wave)
-
 // Pass 2: p = bf16(exp(s - M) / Z), 8-row group sums in fp32 -> bf16, bf16 accumulation over the row chunks in order.
 // Rows <-> REGISTERS here (A = Q fragment, B = K fragment: lane (lq, lc) holds rows 16 rt + 4 lc + j of column lq), so an
-// 8-row group sum is three adds in a lane and one cross-lane add, in the reference's pairwise order.
-template <int D, bool FP8>
-__global__ __launch_bounds__(64 * kSnapWaves, 4) void snapkv_accum_kernel(const SnapParams p) {
+// 8-row group sum is three adds in a lane and one exchange between neighbouring groups of 16 lanes, in the reference's pairwise order.
+// Group G = 2 rt + half (lanes lc = 2 half) belongs to chunk G / g and pseudo head r' = G % g.  For even g a lane meets the same half
+// in every tile, so the accumulators r' = 2 i + half are its registers a[i] (template GH = g / 2, else 0: accumulators in LDS, updated
+// by the two halves in turn).  2 x 2 tiles at a time as in pass 1; one tile at a time and LDS accumulators for every g took 188 us
+// where this takes 150.
+template <int D, bool FP8, int GH>
+__global__ __launch_bounds__(64 * kSnapWaves, D == 64 ? 4 : 2) void snapkv_accum_kernel(const SnapParams p) {
+    constexpr int BT = GH >= 2 ? 2 : 1;                        // row tiles per batch
     __shared__ double tab[kTabN];
-    extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];   // Q image, [L][3] doubles, [waves][g][16] floats
+    // Q image, [L] exp(-M) / Z, [L][2] (M, 1 / Z), GH == 0: [waves][g][32] floats
+    extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];
     const int ctile = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lq = lane & 15, lc = lane >> 4;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lq = lane & 15, lc = lane >> 4;
     unsigned char* qimg = dyn;
-    double* rowc = reinterpret_cast<double*>(dyn + (size_t)p.L * (D * 2 + kQPad));    // (M, 1/Z, exp(-M)/Z) per row
-    float* accs = reinterpret_cast<float*>(rowc + p.L * 3) + wave * p.g * 16;
+    double* rowc = reinterpret_cast<double*>(dyn + (size_t)p.L * (D * 2 + kQPad));
+    double* rowm = rowc + p.L;
+    float* accs = reinterpret_cast<float*>(rowm + p.L * 2) + wave * p.g * 32;
     __shared__ int s_slow_rows;
     if (tid == 0) s_slow_rows = 0;
     for (int i = tid; i < kTabN; i += 64 * kSnapWaves) tab[i] = g_exp_tab[i];
@@ -337,100 +417,171 @@ __global__ __launch_bounds__(64 * kSnapWaves, 4) void snapkv_accum_kernel(const 
     for (int row = tid; row < p.L; row += 64 * kSnapWaves) {
         const double* pp = p.partials + ((int64_t)(b * p.KH + kvh) * p.L + row) * p.nch * 2;
         const double M = pp[0], rZ = pp[1];                   // left by snapkv_finalize_kernel
-        rowc[row * 3] = M;
-        rowc[row * 3 + 1] = rZ;
+        rowm[row * 2] = M;
+        rowm[row * 2 + 1] = rZ;
         double c2 = 0.0;                                      // 0: exp(-M) is not representable -> the exp_neg path
         if (M >= 0.0) c2 = exp_neg(-M) * rZ;
         else if (M > -700.0) c2 = rZ / exp_neg(M);
-        rowc[row * 3 + 2] = c2;
+        rowc[row] = c2;
         if (!(c2 > 0.0)) s_slow_rows = 1;
     }
     __syncthreads();
     const bool fast_rows = s_slow_rows == 0;                  // workgroup-uniform
     const int N = p.S - p.W;
+    const bool whole = p.page_size % 32 == 0;
     const float kscale = FP8 ? p.k_scale[kvh] : 1.0f;
-    const int RT = p.L / 16;
-    const int ncg = min(kAccumCols / 16, (N - ctile * kAccumCols + 15) / 16);    // 16-column groups of this workgroup
-    bf16x8 kf[D / 32], kn[D / 32];
-    if (wave < ncg) load_kfrag<D, FP8>(p, b, kvh, ctile * kAccumCols + wave * 16, lq, lc, kf);
+    const int ncg = (min(p.cols, N - ctile * p.cols) + 31) / 32;                     // 32-column groups of this workgroup
+    bf16x8 kf[2][D / 32], kn[2][D / 32];
+    if (wave < ncg) load_kfrag2<D, FP8>(p, b, kvh, ctile * p.cols + wave * 32, whole, lq, lc, kf);
     for (int cg = wave; cg < ncg; cg += kSnapWaves) {
-        const int col0 = ctile * kAccumCols + cg * 16;
-        if (cg + kSnapWaves < ncg) load_kfrag<D, FP8>(p, b, kvh, col0 + kSnapWaves * 16, lq, lc, kn);
-        for (int i = lane; i < p.g * 16; i += 64) accs[i] = 0.f;
-        __builtin_amdgcn_wave_barrier();
-        const int col = col0 + lq;
-        const bool tail = col0 + 16 > p.S - p.W;               // wave-uniform: only these columns can be masked
-        int rp0 = 0;                                           // (2 rt) % g, kept by increments: no modulo per tile
-        for (int rt = 0; rt < RT; ++rt) {
-            const unsigned char* qp = qimg + (rt * 16 + lq) * (D * 2 + kQPad) + lc * 16;
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        const int col0 = ctile * p.cols + cg * 32;
+        if (cg + kSnapWaves < ncg) load_kfrag2<D, FP8>(p, b, kvh, col0 + kSnapWaves * 32, whole, lq, lc, kn);
+        const bool tail = col0 + 32 > p.S - p.W;               // wave-uniform: only these columns can be masked
+        float a[2][GH > 0 ? GH : 1];                           // [column group][i], bf16 values
+        if constexpr (GH > 0) {
 #pragma unroll
-            for (int ks = 0; ks < D / 32; ++ks)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(qp + ks * 64), kf[ks], acc,
-                                                              0, 0, 0);
-            // lane (lq, lc): rows rt*16 + lc*4 + j of column col0 + lq
-            float pj[4];
-            const unsigned int w0 = pack_bf16(acc[0] * kscale, acc[1] * kscale);
-            const unsigned int w1 = pack_bf16(acc[2] * kscale, acc[3] * kscale);
-            unsigned int bad = 0;
-            const unsigned int o0 = tab_offsets2(w0, bad), o1 = tab_offsets2(w1, bad);
-            const unsigned char* tb = reinterpret_cast<const unsigned char*>(tab);
-            const double* rc = rowc + (rt * 16 + lc * 4) * 3;
-            float v[4];
-            int ti[4];
-            if (fast_rows && !tail && __builtin_amdgcn_ballot_w64(bad != 0) == 0) {
-                // hot path, no divergence: table value x the row's exp(-M) / Z
-                pj[0] = bf16_to_f32(f32_to_bf16((float)(*reinterpret_cast<const double*>(tb + (o0 & 0xffffu)) * rc[2])));
-                pj[1] = bf16_to_f32(f32_to_bf16((float)(*reinterpret_cast<const double*>(tb + (o0 >> 16)) * rc[5])));
-                pj[2] = bf16_to_f32(f32_to_bf16((float)(*reinterpret_cast<const double*>(tb + (o1 & 0xffffu)) * rc[8])));
-                pj[3] = bf16_to_f32(f32_to_bf16((float)(*reinterpret_cast<const double*>(tb + (o1 >> 16)) * rc[11])));
-            } else {
-                v[0] = bf16_bits_to_f32((unsigned short)(w0 & 0xffffu));
-                v[1] = bf16_bits_to_f32((unsigned short)(w0 >> 16));
-                v[2] = bf16_bits_to_f32((unsigned short)(w1 & 0xffffu));
-                v[3] = bf16_bits_to_f32((unsigned short)(w1 >> 16));
+            for (int i = 0; i < GH; ++i) a[0][i] = a[1][i] = 0.f;
+        } else {
+            for (int i = lane; i < p.g * 32; i += 64) accs[i] = 0.f;
+            __builtin_amdgcn_wave_barrier();
+        }
+        // group sums of the BT row tiles from rt on, both column groups: lanes lc < 2 have group 2 rt, the others 2 rt + 1
+        auto sums = [&](int rt, float (&gs)[BT][2]) {
+            unsigned int w[BT][2][2];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) ti[j] = tab_index(v[j]);
+            for (int u = 0; u < BT; ++u) {
+                const unsigned char* qp = qimg + ((rt + u) * 16 + lq) * (D * 2 + kQPad) + lc * 16;
+                f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    float pr = 0.f;
-                    if (!(tail && masked(p, rt * 16 + lc * 4 + j, col))) {
-                        const double c2 = rc[j * 3 + 2];
-                        if (ti[j] >= 0 && c2 > 0.0)
-                            pr = (float)(tab[ti[j]] * c2);
-                        else
-                            pr = (float)(exp_neg((double)v[j] - rc[j * 3]) * rc[j * 3 + 1]);
-                    }
-                    pj[j] = bf16_to_f32(f32_to_bf16(pr));      // softmax -> bf16 (model.py:416)
+                for (int ks = 0; ks < D / 32; ++ks) {
+                    const bf16x8 qf = *reinterpret_cast<const bf16x8*>(qp + ks * 64);
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf, kf[c][ks], acc[c], 0, 0, 0);
                 }
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    if (FP8) acc[c] *= kscale;
+                    w[u][c][0] = pack_bf16(acc[c][0], acc[c][1]);
+                    w[u][c][1] = pack_bf16(acc[c][2], acc[c][3]);
+                }
+            }
+            u16x2 top = {0, 0};
+            unsigned int low = 0, o[BT][2][2], pk[BT][2][2];
+#pragma unroll
+            for (int u = 0; u < BT; ++u)
+#pragma unroll
+                for (int c = 0; c < 2; ++c)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) o[u][c][h] = tab_offsets2(w[u][c][h], top, low);
+            if (fast_rows && !tail && __builtin_amdgcn_ballot_w64(tab_outside(top, low)) == 0) {
+                // hot path, no divergence: table value x the row's exp(-M) / Z, softmax -> bf16 (model.py:416)
+#pragma unroll
+                for (int u = 0; u < BT; ++u) {
+                    const double* rc = rowc + (rt + u) * 16 + lc * 4;
+                    const double c2[4] = {rc[0], rc[1], rc[2], rc[3]};
+#pragma unroll
+                    for (int c = 0; c < 2; ++c)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h)
+                            pk[u][c][h] = pack_bf16((float)(tab_at(tab, o[u][c][h] & 0xffffu) * c2[2 * h]),
+                                                    (float)(tab_at(tab, o[u][c][h] >> 16) * c2[2 * h + 1]));
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < BT; ++u)
+#pragma unroll
+                    for (int c = 0; c < 2; ++c)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            float pr[2];
+#pragma unroll
+                            for (int e = 0; e < 2; ++e) {
+                                const int row = (rt + u) * 16 + lc * 4 + 2 * h + e;
+                                const float v = bf16_bits_to_f32((unsigned short)(e ? w[u][c][h] >> 16 : w[u][c][h] & 0xffffu));
+                                pr[e] = 0.f;
+                                if (!(tail && masked(p, row, col0 + c * 16 + lq))) {
+                                    const int ti = tab_index(v);
+                                    const double c2 = rowc[row];
+                                    if ((ti >= 0 || is_tiny(v)) && c2 > 0.0)
+                                        pr[e] = (float)((ti >= 0 ? tab[ti] : exp_tiny(v)) * c2);
+                                    else
+                                        pr[e] = (float)(exp_neg((double)v - rowm[row * 2]) * rowm[row * 2 + 1]);
+                                }
+                            }
+                            pk[u][c][h] = pack_bf16(pr[0], pr[1]);
+                        }
             }
             // 8-row group sum in fp32, pairwise as a butterfly over consecutive rows, -> bf16 (:418)
-            float t = (pj[0] + pj[1]) + (pj[2] + pj[3]);
-            t += __shfl_xor(t, 16);
-            const float gs = bf16_to_f32(f32_to_bf16(t));
-            // lanes lc = 0 / lc = 2 hold the groups G = 2 rt / 2 rt + 1 (chunk = G / g, pseudo head r' = G % g): accumulate
-            // in group order (with g = 1 both land on the same accumulator)
 #pragma unroll
-            for (int half = 0; half < 2; ++half) {
-                if (lc == 2 * half) {
-                    float* a = accs + rp0 * 16 + lq;
-                    *a = bf16_to_f32(f32_to_bf16(*a + gs));
+            for (int u = 0; u < BT; ++u) {
+                float t[2];
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const unsigned int x = pk[u][c][0], y = pk[u][c][1];
+                    t[c] = (__uint_as_float(x << 16) + __uint_as_float(x & 0xffff0000u)) +
+                           (__uint_as_float(y << 16) + __uint_as_float(y & 0xffff0000u));
+                    // lanes 16 k <-> 16 (k ^ 1): both get the sum of the pair
+                    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(t[c]), __float_as_uint(t[c]), false, false);
+                    t[c] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
                 }
-                rp0 = rp0 + 1 == p.g ? 0 : rp0 + 1;
-                __builtin_amdgcn_wave_barrier();
+                const unsigned int g2 = pack_bf16(t[0], t[1]);
+                gs[u][0] = __uint_as_float(g2 << 16);
+                gs[u][1] = __uint_as_float(g2 & 0xffff0000u);
             }
-        }
-        // write bf16 accumulators: aws[b][kvh*g + r'][col]
-        for (int i = lane; i < p.g * 16; i += 64) {
-            const int rp = i / 16, c = i % 16;
-            if (col0 + c < N) {
-                const bf16_t v = f32_to_bf16(accs[i]);
-                p.aws[((int64_t)b * p.H + kvh * p.g + rp) * N + col0 + c] = *reinterpret_cast<const unsigned short*>(&v);
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
+        };
+        if constexpr (GH > 0) {
+            for (int rt = 0; rt < p.L / 16; rt += GH)          // one chunk of 8 g rows
 #pragma unroll
-        for (int ks = 0; ks < D / 32; ++ks) kf[ks] = kn[ks];
+                for (int i = 0; i < GH; i += BT) {
+                    float gs[BT][2];
+                    sums(rt + i, gs);
+#pragma unroll
+                    for (int u = 0; u < BT; ++u) {
+                        const unsigned int n2 = pack_bf16(a[0][i + u] + gs[u][0], a[1][i + u] + gs[u][1]);
+                        a[0][i + u] = __uint_as_float(n2 << 16);
+                        a[1][i + u] = __uint_as_float(n2 & 0xffff0000u);
+                    }
+                }
+            // bf16 accumulators: aws[b][kvh*g + r'][col]; lane (lq, lc): half lc / 2, column group lc & 1
+            const int col = col0 + (lc & 1) * 16 + lq;
+#pragma unroll
+            for (int i = 0; i < GH; ++i) {
+                const float v = lc & 1 ? a[1][i] : a[0][i];
+                if (col < N)
+                    p.aws[((int64_t)b * p.H + kvh * p.g + 2 * i + (lc >> 1)) * N + col] = (unsigned short)(__float_as_uint(v) >> 16);
+            }
+        } else {
+            int rp0 = 0;                                       // (2 rt) % g, kept by increments: no modulo per tile
+            for (int rt = 0; rt < p.L / 16; ++rt) {
+                float gs[BT][2];
+                sums(rt, gs);
+                // the two halves in group order (with g = 1 both land on the same accumulator)
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    if (lc == 2 * half) {
+#pragma unroll
+                        for (int c = 0; c < 2; ++c) {
+                            float* x = accs + rp0 * 32 + c * 16 + lq;
+                            *x = bf16_to_f32(f32_to_bf16(*x + gs[0][c]));
+                        }
+                    }
+                    rp0 = rp0 + 1 == p.g ? 0 : rp0 + 1;
+                    __builtin_amdgcn_wave_barrier();
+                }
+            }
+            for (int i = lane; i < p.g * 32; i += 64) {
+                const int rp = i / 32, c = i % 32;
+                if (col0 + c < N) {
+                    const bf16_t v = f32_to_bf16(accs[i]);
+                    p.aws[((int64_t)b * p.H + kvh * p.g + rp) * N + col0 + c] = *reinterpret_cast<const unsigned short*>(&v);
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int ks = 0; ks < D / 32; ++ks) kf[c][ks] = kn[c][ks];
     }
 }
 
@@ -438,125 +589,154 @@ __device__ __forceinline__ unsigned int ordered16(unsigned short bits) {
     return (bits & 0x8000u) ? (unsigned int)(~bits & 0xffffu) : (unsigned int)(bits | 0x8000u);
 }
 
-// one workgroup (1024 threads) per (kv head, request)
-__global__ __launch_bounds__(1024) void snapkv_select_kernel(const unsigned short* __restrict__ aws, int H, int KH, int g,
-                                                             int N, int ksz, int topk, int32_t* idx_out,
-                                                             unsigned short* score_out) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smraw[];
-    unsigned short* keys = reinterpret_cast<unsigned short*>(smraw);  // [N] ordered keys
-    const int npad_keys = (N + 7) / 8 * 8;
-    unsigned int* hist = reinterpret_cast<unsigned int*>(smraw + npad_keys * 2);  // [256]
-    unsigned int* sel = hist + 256;                                               // [kpad]
-    unsigned int* misc = sel + 1024;                                              // scalars / wave counts
-    const int kvh = blockIdx.x, b = blockIdx.y;
-    const int tid = threadIdx.x;
-    const int half = ksz / 2;
+// Pooled + group-summed scores of 1024 columns of one (kv head, request), as bf16 bits: a thread owns four neighbouring columns, the
+// rows' columns (and half a pool width on either side) come through LDS.  All CUs take part; inside the selection's one workgroup per
+// (kv head, request) it was most of that kernel's 135 us.
+constexpr int kPoolCols = 1024, kPoolHalf = 64;         // widest half pool that is staged
 
-    // 1. pooled + group-summed score per column -> ordered 16-bit key
-    for (int s = tid; s < N; s += 1024) {
-        float tot = 0.f;
-        for (int rp = 0; rp < g; ++rp) {
-            const unsigned short* row = aws + ((int64_t)b * H + kvh * g + rp) * N;
-            float acc = 0.f;
-            for (int k = -half; k <= half; ++k) {
-                const int c = s + k;
-                if (c >= 0 && c < N) acc += bf16_bits_to_f32(row[c]);
-            }
-            const float pooled = bf16_to_f32(f32_to_bf16(acc / (float)ksz));
-            tot += pooled;
-        }
-        const bf16_t tb = f32_to_bf16(tot);
-        const unsigned short bits = *reinterpret_cast<const unsigned short*>(&tb);
-        keys[s] = (unsigned short)ordered16(bits);
-        if (score_out) score_out[((int64_t)b * KH + kvh) * N + s] = bits;
-    }
-    // 2. exact k-th largest key by two 8-bit histogram rounds
-    unsigned int prefix_hi = 0, kth_rem = topk;
-    for (int round = 0; round < 2; ++round) {
-        for (int i = tid; i < 256; i += 1024) hist[i] = 0;
-        __syncthreads();
-        for (int s = tid; s < N; s += 1024) {
-            const unsigned int k = keys[s];
-            if (round == 0)
-                atomicAdd(&hist[k >> 8], 1u);
-            else if ((k >> 8) == prefix_hi)
-                atomicAdd(&hist[k & 0xff], 1u);
-        }
-        __syncthreads();
-        if (tid == 0) {
-            unsigned int rem = kth_rem;
-            int bin = 255;
-            for (; bin > 0; --bin) {
-                if (hist[bin] >= rem) break;
-                rem -= hist[bin];
-            }
-            misc[0] = bin;
-            misc[1] = rem;  // rank of the k-th inside this bin (1-based from the top)
-        }
-        __syncthreads();
-        if (round == 0) prefix_hi = misc[0];
-        kth_rem = misc[1];
-        __syncthreads();
-    }
-    const unsigned int T = (prefix_hi << 8) | misc[0];
-    const unsigned int need_eq = kth_rem;  // how many keys == T are selected (lowest indices first)
-    __syncthreads();
-    // 3. compaction: > T unordered (sorted later); == T in index order
-    if (tid == 0) {
-        misc[2] = 0;  // count of > T written
-        misc[3] = 0;  // running count of == T
-    }
-    for (int i = tid; i < 1024; i += 1024) sel[i] = 0;
-    __syncthreads();
-    const int lane = tid & 63, wave = tid >> 6;
-    unsigned int* wcnt = misc + 8;  // [16]
-    for (int base = 0; base < N; base += 1024) {
-        const int s = base + tid;
-        const unsigned int k = s < N ? keys[s] : 0u;
-        const bool gt = s < N && k > T;
-        const bool eq = s < N && k == T;
-        if (gt) {
-            const unsigned int slot = atomicAdd(&misc[2], 1u);
-            sel[slot] = (k << 16) | (0xffffu - (unsigned int)s);
-        }
-        const unsigned long long bal = __ballot(eq);
-        const unsigned int before = __popcll(bal & ((1ull << lane) - 1ull));
-        if (lane == 0) wcnt[wave] = __popcll(bal);
-        __syncthreads();
-        unsigned int woff = misc[3];
-        for (int w = 0; w < wave; ++w) woff += wcnt[w];
-        if (eq) {
-            const unsigned int rank = woff + before;
-            if (rank < need_eq) sel[(topk - need_eq) + rank] = (k << 16) | (0xffffu - (unsigned int)s);
-        }
-        __syncthreads();
-        if (tid == 0) {
-            unsigned int t = misc[3];
-            for (int w = 0; w < 16; ++w) t += wcnt[w];
-            misc[3] = t;
-        }
-        __syncthreads();
-    }
-    // 4. bitonic sort (descending) of the padded selection
-    int kpad = 1;
-    while (kpad < topk) kpad <<= 1;
-    for (int size = 2; size <= kpad; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int i = tid; i < kpad / 2; i += 1024) {
-                const int lo = (i / stride) * stride * 2 + (i % stride);
-                const int hi = lo + stride;
-                const bool desc = ((lo & size) == 0);
-                const unsigned int a = sel[lo], c = sel[hi];
-                if ((a < c) == desc) {
-                    sel[lo] = c;
-                    sel[hi] = a;
-                }
+template <int KS>                                       // the pool's width where it is known (taps in registers), else 0
+__global__ __launch_bounds__(256) void snapkv_pool_kernel(const unsigned short* __restrict__ aws, int H, int KH, int g, int N, int ksz_any,
+                                                          unsigned short* __restrict__ score_out) {
+    __shared__ __attribute__((aligned(16))) float img[kPoolCols + 2 * kPoolHalf];
+    const int ksz = KS ? KS : ksz_any;
+    const int c0 = blockIdx.x * kPoolCols, kvh = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, half = ksz / 2;
+    const bool staged = half <= kPoolHalf;
+    float tot[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int rp = 0; rp < g; ++rp) {
+        const unsigned short* row = aws + ((int64_t)b * H + kvh * g + rp) * N;
+        if (staged) {
+            for (int i = tid; i < kPoolCols + 2 * half; i += 256) {
+                const int c = c0 - half + i;
+                img[i] = c >= 0 && c < N ? bf16_bits_to_f32(row[c]) : 0.f;       // (adding 0 is what leaving a column out is)
             }
             __syncthreads();
         }
+        float tap[4 + (KS ? KS - 1 : 0)];
+        if constexpr (KS > 0) {
+#pragma unroll
+            for (int k = 0; k < 4 + KS - 1; ++k) tap[k] = img[tid * 4 + k];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int s = tid * 4 + j;
+            float acc = 0.f;
+            if constexpr (KS > 0) {
+#pragma unroll
+                for (int k = 0; k < KS; ++k) acc += tap[j + k];
+            } else if (staged) {
+                for (int k = 0; k < ksz; ++k) acc += img[s + k];
+            } else {
+                for (int k = -half; k <= half; ++k) {
+                    const int c = c0 + s + k;
+                    if (c >= 0 && c < N) acc += bf16_bits_to_f32(row[c]);
+                }
+            }
+            tot[j] += bf16_to_f32(f32_to_bf16(acc / (float)ksz));
+        }
+        if (staged) __syncthreads();
     }
-    for (int j = tid; j < topk; j += 1024)
-        idx_out[((int64_t)b * KH + kvh) * topk + j] = (int32_t)(0xffffu - (sel[j] & 0xffffu));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int s = c0 + tid * 4 + j;
+        const bf16_t tb = f32_to_bf16(tot[j]);
+        if (s < N) score_out[((int64_t)b * KH + kvh) * N + s] = *reinterpret_cast<const unsigned short*>(&tb);
+    }
+}
+
+// inclusive sums over the 1024 threads of a workgroup; `waves` is LDS scratch of 16 entries
+__device__ __forceinline__ unsigned int scan1024(unsigned int v, unsigned int* waves, int lane, int wave) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned int u = __shfl_up(v, o);
+        if (lane >= o) v += u;
+    }
+    if (lane == 63) waves[wave] = v;
+    __syncthreads();
+    unsigned int before = 0;
+    for (int w = 0; w < wave; ++w) before += waves[w];
+    __syncthreads();
+    return v + before;
+}
+
+// Exact top-k of N bf16 scores, one workgroup (1024 threads) per (kv head, request).  Histogram of the keys' upper 12 bits (scores of
+// one context share a few exponents: 8 bits would put nearly all of them into two counters), a workgroup scan for the bin of the k-th
+// largest, the same over its 16 low values; a thread's run of consecutive keys then knows by one scan which of the equal ones are
+// the first; the selected keys are ranked by counting (they are distinct: each carries its index).  Bound by latency: a dozen barriers
+// (the first version had 120, with single threads walking the histograms): 17.5 us for 16 000 keys.
+__global__ __launch_bounds__(1024) void snapkv_select_kernel(const unsigned short* __restrict__ scores, int KH, int N, int topk,
+                                                             int32_t* idx_out) {
+    constexpr int kBins = 4096;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smraw[];
+    unsigned short* keys = reinterpret_cast<unsigned short*>(smraw);              // [N] ordered keys
+    unsigned int* hist = reinterpret_cast<unsigned int*>(smraw + (N + 7) / 8 * 16);    // [4096]
+    unsigned int* sel = hist + kBins;                                             // [1024]
+    unsigned int* waves = sel + 1024;                                             // [16]
+    unsigned int* misc = waves + 16;                                              // bin, rank in it, number above, [16] low counts
+    const int kvh = blockIdx.x, b = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const unsigned short* src = scores + ((int64_t)b * KH + kvh) * N;
+    for (int i = tid; i < kBins; i += 1024) hist[i] = 0;
+    sel[tid] = 0;
+    if (tid < 32) misc[tid] = 0;
+    __syncthreads();
+    for (int s = tid; s < N; s += 1024) {
+        const unsigned int k = ordered16(src[s]);
+        keys[s] = (unsigned short)k;
+        atomicAdd(&hist[k >> 4], 1u);
+    }
+    __syncthreads();
+    {   // thread t looks at the four bins 4 t .. 4 t + 3 counted from the top
+        unsigned int n[4], sum = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            n[j] = hist[kBins - 1 - (tid * 4 + j)];
+            sum += n[j];
+        }
+        const unsigned int upto = scan1024(sum, waves, lane, wave);
+        unsigned int above = upto - sum;
+        if (above < (unsigned int)topk && upto >= (unsigned int)topk) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (above < (unsigned int)topk && above + n[j] >= (unsigned int)topk) {
+                    misc[0] = kBins - 1 - (tid * 4 + j);
+                    misc[1] = topk - above;
+                    break;
+                }
+                above += n[j];
+            }
+        }
+    }
+    __syncthreads();
+    const unsigned int bin = misc[0];
+    for (int s = tid; s < N; s += 1024)
+        if ((unsigned int)keys[s] >> 4 == bin) atomicAdd(&misc[16 + (keys[s] & 15)], 1u);
+    __syncthreads();
+    unsigned int need = misc[1], low = 15;                    // (every thread: 16 broadcast reads)
+    for (; low > 0 && misc[16 + low] < need; --low) need -= misc[16 + low];
+    const unsigned int T = bin << 4 | low;                    // the k-th largest key; `need` keys == T are selected, lowest indices first
+    // thread t's run of consecutive keys
+    const int run = (N + 1023) / 1024, first = min(tid * run, N), last = min(first + run, N);
+    unsigned int eq = 0;
+    for (int s = first; s < last; ++s) eq += keys[s] == T;
+    unsigned int rank = scan1024(eq, waves, lane, wave) - eq;
+    for (int s = first; s < last; ++s) {
+        const unsigned int k = keys[s];
+        if (k > T) sel[atomicAdd(&misc[2], 1u)] = k << 16 | (0xffffu - (unsigned int)s);
+        if (k == T) {
+            if (rank < need) sel[topk - need + rank] = k << 16 | (0xffffu - (unsigned int)s);
+            ++rank;
+        }
+    }
+    __syncthreads();
+    if (tid < topk) {
+        const unsigned int mine = sel[tid];
+        unsigned int place = 0;
+        for (int i = 0; i < topk; i += 4) {                   // (sel is 0 beyond topk: below every key that matters)
+            const u32x4 o = *reinterpret_cast<const u32x4*>(sel + i);
+            place += (o[0] > mine) + (o[1] > mine) + (o[2] > mine) + (o[3] > mine);
+        }
+        idx_out[((int64_t)b * KH + kvh) * topk + place] = (int32_t)(0xffffu - (mine & 0xffffu));
+    }
 }
 
 struct GatherParams {
@@ -574,9 +754,12 @@ struct GatherParams {
     int src_hnd;         // source pages are [2][KH][page_size][D] instead of [2][page_size][KH][D]
 };
 
+// a row's 16-byte pieces (k, then v) lie across 2 D / 8 lanes, several rows per wavefront
 template <bool FP8>
-__global__ __launch_bounds__(64) void snapkv_gather_kernel(const GatherParams p) {
-    const int j = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+__global__ __launch_bounds__(256) void snapkv_gather_kernel(const GatherParams p) {
+    const int nv = p.D / 8, rows = 256 / (2 * nv), i = threadIdx.x % (2 * nv);
+    const int j = blockIdx.x * rows + threadIdx.x / (2 * nv), kvh = blockIdx.y, b = blockIdx.z;
+    if (j >= p.budget) return;
     const int src = j < p.topk ? p.idx[((int64_t)b * p.KH + kvh) * p.topk + j] : p.S - p.W + (j - p.topk);
     const int row_elems = p.KH * p.D;
     const int sp = src / p.page_size, ss = src - sp * p.page_size;
@@ -592,8 +775,7 @@ __global__ __launch_bounds__(64) void snapkv_gather_kernel(const GatherParams p)
     const int64_t dpid = p.dindices[dp0 + dpg];
     const int64_t doff = (dpid * 2 * p.page_size + dsl) * row_elems + kvh * p.D;
     const int64_t half = (int64_t)p.page_size * row_elems;
-    const int nv = p.D / 8;
-    for (int i = threadIdx.x; i < 2 * nv; i += 64) {
+    {
         const int64_t h = i < nv ? 0 : half;
         const int c = i < nv ? i : i - nv;
         if constexpr (FP8) {   // dequantise into the bf16 draft cache: bf16(byte * scale)
@@ -619,13 +801,22 @@ __global__ __launch_bounds__(64) void snapkv_gather_kernel(const GatherParams p)
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+// Columns per workgroup of the two score kernels.  A table, a query image and a merge per workgroup are worth 4 096 columns and more as
+// long as two workgroups per CU are there (16 requests of 16 000 keys, 8 kv heads of 64: 2 048 -> 4 096 pass 1 139 -> 120 us, pass 2 153
+// -> 150); one request alone has too few workgroups with 2 048 (4 128 keys, heads of 128: 118 us for the whole selection, 67 with 512).
+int score_cols(int B, int KH, int ctx_len) {
+    int cols = 512;
+    while (cols < 16384 && (int64_t)B * KH * ((ctx_len + 2 * cols - 1) / (2 * cols)) >= 512) cols *= 2;
+    return cols;
+}
+
 }  // namespace
 
 extern "C" size_t md_snapkv_workspace_bytes(int B, int H, int KH, int ctx_len, int window) {
     if (B <= 0 || H <= 0 || KH <= 0 || H % KH || ctx_len <= window) return 0;
     const int g = H / KH;
     const size_t L = (size_t)g * window;
-    const size_t nch = (ctx_len + kChunkCols - 1) / kChunkCols;
+    const size_t cols = score_cols(B, KH, ctx_len), nch = (ctx_len + cols - 1) / cols;
     const size_t partials = align_up((size_t)B * KH * L * nch * 2 * 8, 256);
     const size_t aws = align_up((size_t)B * H * (ctx_len - window) * 2, 256);
     const size_t scores = align_up((size_t)B * KH * (ctx_len - window) * 2, 256);
@@ -636,7 +827,7 @@ extern "C" size_t md_snapkv_scores_offset(int B, int H, int KH, int ctx_len, int
     if (B <= 0 || H <= 0 || KH <= 0 || H % KH || ctx_len <= window) return 0;
     const int g = H / KH;
     const size_t L = (size_t)g * window;
-    const size_t nch = (ctx_len + kChunkCols - 1) / kChunkCols;
+    const size_t cols = score_cols(B, KH, ctx_len), nch = (ctx_len + cols - 1) / cols;
     return align_up((size_t)B * KH * L * nch * 2 * 8, 256) + align_up((size_t)B * H * (ctx_len - window) * 2, 256);
 }
 
@@ -689,7 +880,8 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
     p.W = window;
     p.S = ctx_len;
     p.L = L;
-    p.nch = (ctx_len + kChunkCols - 1) / kChunkCols;
+    p.cols = score_cols(B, KH, ctx_len);
+    p.nch = (ctx_len + p.cols - 1) / p.cols;
     p.page_size = page_size;
     p.slot_stride = hnd ? D : KH * D;
     p.head_stride = hnd ? page_size * D : D;
@@ -704,23 +896,37 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
     MD_CHECK_ARG(L <= 16 * kMaxRT, "md_snapkv_select: g * window = %d rows per kv head, at most %d supported", L, 16 * kMaxRT);
     const size_t qimg_b = (size_t)L * (D * 2 + kQPad);
     const size_t lds1 = qimg_b + (size_t)kSnapWaves * L * 2 * 8;
-    const size_t lds2 = qimg_b + (size_t)L * 3 * 8 + (size_t)kSnapWaves * g * 16 * 4;
+    // accumulators in registers for g = 2, 4, 8 (a chunk of 8 g rows is then g / 2 whole tiles)
+    const int gh = g == 2 || g == 4 || g == 8 ? g / 2 : 0;
+    const size_t lds2 = qimg_b + (size_t)L * 3 * 8 + (gh ? 0 : (size_t)kSnapWaves * g * 32 * 4);
     if (lds1 + sizeof(double) * kTabN > 64 * 1024 || lds2 + sizeof(double) * kTabN > 64 * 1024) {
         static MdPerDeviceOnce lds_once;
         if (lds_once.first()) {
             const int cap = 160 * 1024 - (int)sizeof(double) * kTabN - 256;
             const void* ks[] = {reinterpret_cast<const void*>(&snapkv_stats_kernel<64, false, 8>),
-                                reinterpret_cast<const void*>(&snapkv_stats_kernel<64, true, 8>),
-                                reinterpret_cast<const void*>(&snapkv_stats_kernel<128, false, 8>),
-                                reinterpret_cast<const void*>(&snapkv_stats_kernel<128, true, 8>),
                                 reinterpret_cast<const void*>(&snapkv_stats_kernel<64, false, kMaxRT>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, false, 0>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, false, 1>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, false, 2>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, false, 4>),
+                                reinterpret_cast<const void*>(&snapkv_stats_kernel<64, true, 8>),
                                 reinterpret_cast<const void*>(&snapkv_stats_kernel<64, true, kMaxRT>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, true, 0>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, true, 1>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, true, 2>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, true, 4>),
+                                reinterpret_cast<const void*>(&snapkv_stats_kernel<128, false, 8>),
                                 reinterpret_cast<const void*>(&snapkv_stats_kernel<128, false, kMaxRT>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, false, 0>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, false, 1>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, false, 2>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, false, 4>),
+                                reinterpret_cast<const void*>(&snapkv_stats_kernel<128, true, 8>),
                                 reinterpret_cast<const void*>(&snapkv_stats_kernel<128, true, kMaxRT>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, false>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, true>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, false>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, true>)};
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, true, 0>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, true, 1>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, true, 2>),
+                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, true, 4>)};
             for (const void* k : ks)
                 if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, cap) != hipSuccess) {
                     lds_once.undo();
@@ -737,8 +943,11 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
         else                                                                                                     \
             hipLaunchKernelGGL((snapkv_stats_kernel<DD, FP, kMaxRT>), dim3(p.nch, KH, B), dim3(64 * kSnapWaves), lds1, st, p); \
         hipLaunchKernelGGL(snapkv_finalize_kernel, dim3((unsigned)(((int64_t)B * KH * L + 255) / 256)), dim3(256), 0, st, p); \
-        hipLaunchKernelGGL((snapkv_accum_kernel<DD, FP>), dim3((N + kAccumCols - 1) / kAccumCols, KH, B), dim3(64 * kSnapWaves), lds2, \
-                           st, p);                                                                               \
+        const dim3 ag((N + p.cols - 1) / p.cols, KH, B);                                                 \
+        if (gh == 4) hipLaunchKernelGGL((snapkv_accum_kernel<DD, FP, 4>), ag, dim3(64 * kSnapWaves), lds2, st, p);      \
+        else if (gh == 2) hipLaunchKernelGGL((snapkv_accum_kernel<DD, FP, 2>), ag, dim3(64 * kSnapWaves), lds2, st, p); \
+        else if (gh == 1) hipLaunchKernelGGL((snapkv_accum_kernel<DD, FP, 1>), ag, dim3(64 * kSnapWaves), lds2, st, p); \
+        else hipLaunchKernelGGL((snapkv_accum_kernel<DD, FP, 0>), ag, dim3(64 * kSnapWaves), lds2, st, p);              \
     } while (0)
     if (D == 128) {
         if (fp8) MD_SNAP_LAUNCH(128, true); else MD_SNAP_LAUNCH(128, false);
@@ -748,7 +957,12 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
 #undef MD_SNAP_LAUNCH
     MD_CHECK_LAUNCH("md_snapkv_select(scores)");
 
-    const size_t lds3 = (size_t)((N + 7) / 8 * 8) * 2 + (256 + 1024 + 32) * 4;
+    const dim3 pgrid((N + kPoolCols - 1) / kPoolCols, KH, B);
+    if (pool_kernel == 5)
+        hipLaunchKernelGGL((snapkv_pool_kernel<5>), pgrid, dim3(256), 0, st, p.aws, H, KH, g, N, pool_kernel, scores);
+    else
+        hipLaunchKernelGGL((snapkv_pool_kernel<0>), pgrid, dim3(256), 0, st, p.aws, H, KH, g, N, pool_kernel, scores);
+    const size_t lds3 = (size_t)((N + 7) / 8 * 8) * 2 + (4096 + 1024 + 16 + 32) * 4;
     static MdPerDeviceOnce attr_once;
     if (attr_once.first()) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&snapkv_select_kernel),
@@ -758,8 +972,7 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
             return MD_ERR_LAUNCH;
         }
     }
-    hipLaunchKernelGGL(snapkv_select_kernel, dim3(KH, B), dim3(1024), lds3, st, p.aws, H, KH, g, N, pool_kernel, topk,
-                       idx_out, scores);
+    hipLaunchKernelGGL(snapkv_select_kernel, dim3(KH, B), dim3(1024), lds3, st, scores, KH, N, topk, idx_out);
     MD_CHECK_LAUNCH("md_snapkv_select(select)");
 
     GatherParams gp;
@@ -781,10 +994,12 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
     gp.budget = budget;
     gp.topk = topk;
     gp.src_hnd = hnd ? 1 : 0;
+    const int rows = 256 / (2 * D / 8);
+    const dim3 ggrid((budget + rows - 1) / rows, KH, B);
     if (fp8)
-        hipLaunchKernelGGL((snapkv_gather_kernel<true>), dim3(budget, KH, B), dim3(64), 0, st, gp);
+        hipLaunchKernelGGL((snapkv_gather_kernel<true>), ggrid, dim3(256), 0, st, gp);
     else
-        hipLaunchKernelGGL((snapkv_gather_kernel<false>), dim3(budget, KH, B), dim3(64), 0, st, gp);
+        hipLaunchKernelGGL((snapkv_gather_kernel<false>), ggrid, dim3(256), 0, st, gp);
     MD_CHECK_LAUNCH("md_snapkv_select(gather)");
     return MD_OK;
 }

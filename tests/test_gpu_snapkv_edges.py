@@ -1,0 +1,44 @@
+"""The SnapKV selection where its column groups, chunks, register accumulators and bins end, against the CPU restatement of the
+reference (oracle/magicdec_ref.py).  Queries and keys are small integers: the scores are exact in any order.  On the GPU (-m gpu)."""
+import pytest
+import torch
+
+from oracle import magicdec_ref as mr
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("page", [128, 48])
+@pytest.mark.parametrize("g,W,D", [(2, 16, 64), (3, 16, 128), (4, 32, 64), (4, 32, 128), (5, 32, 64), (8, 32, 128), (7, 32, 64)])
+@pytest.mark.parametrize("S,budget,pool", [(150, 129, 5), (2080, 257, 5), (2113, 64, 7), (4200, 257, 1), (1060, 1000, 131)])
+def test_select(monkeypatch, g, W, D, S, budget, pool, page):
+    """Scores against the restatement; positions and gathered rows exactly, given the scores."""
+    from magicdec_amd import ops
+    B, KH = 2, 2
+    H, ppr, dpr = KH * g, -(-S // page), budget // page + 1
+    gen = torch.Generator().manual_seed(S + g)
+    q = torch.randint(-1, 2, (B * W, H, D), generator=gen).bfloat16()
+    kv = torch.randint(-1, 2, (B * ppr, 2, KH, page, D), generator=gen).bfloat16()
+    perm = torch.randperm(B * ppr, generator=gen).int()
+    draft = torch.zeros(B * dpr, 2, page, KH, D, dtype=torch.bfloat16, device=DEV)
+    args = (torch.arange(B * dpr, dtype=torch.int32, device=DEV), torch.arange(B + 1, dtype=torch.int32, device=DEV) * dpr,
+            torch.full((B,), budget - (dpr - 1) * page, dtype=torch.int32, device=DEV))
+    idx, sc = ops.snapkv_select(q.to(DEV), kv.to(DEV), perm.to(DEV), torch.arange(B + 1, dtype=torch.int32, device=DEV) * ppr, S, W, budget, pool,
+                                draft, *args, ops.AttnWorkspace(DEV), return_scores=True, kv_layout="HND")
+    idx, sc, draft = idx.cpu().long(), sc.cpu(), draft.cpu()
+    rows = kv[perm.long()].view(B, ppr, 2, KH, page, D).permute(2, 0, 3, 1, 4, 5).reshape(2, B, KH, ppr * page, D)[:, :, :, :S]
+    monkeypatch.setattr(mr, "LINEAR_MODE", "fp64")           # correctly rounded scores and weights
+    for b in range(B):
+        want = mr.snapkv_scores(q[b * W:(b + 1) * W], rows[0, b].transpose(0, 1).contiguous(), g, W, pool)
+        # fp32 sums of eight rounded weights in another order: at most a few of the thousands of scores, by one bf16 step
+        off = (sc[b].view(torch.int16).int() - want.view(torch.int16).int()).abs()
+        assert int(off.max()) <= 1 and int((off > 0).sum()) <= 2, (b, int((off > 0).sum()))
+    for b in range(B):
+        for h in range(KH):
+            v = sc[b, h].float()
+            order = torch.sort(v, descending=True, stable=True).indices[:budget - W]          # ties: the lowest positions
+            assert torch.equal(idx[b, h], order), (b, h)
+            keep = torch.cat([order, torch.arange(S - W, S)])
+            got = draft[b * dpr:(b + 1) * dpr, :, :, h].transpose(0, 1).reshape(2, dpr * page, D)[:, :budget]
+            assert torch.equal(got, rows[:, b, h][:, keep])
