@@ -31,6 +31,7 @@ copy stays for the prefill-sized products.  MAGICDEC_GEMM=hip forces md_linear w
 MAGICDEC_GEMM=lib forces the library, MAGICDEC_FUSED=0/1 switches md_linear_fused off / on everywhere (the A/B
 switches)."""
 import os
+import re
 
 _MODE = os.environ.get("MAGICDEC_GEMM", "auto")
 _FUSED = os.environ.get("MAGICDEC_FUSED", "auto")     # "0": never md_linear_fused, "1": wherever it supports the shape
@@ -52,6 +53,14 @@ FUSED_DEEP_SWIGLU_T22_MAX_L2_BYTES = float(os.environ.get("MAGICDEC_DEEP_SWIGLU_
 _SHARD70B = os.environ.get("MAGICDEC_SHARD70B", "1")     # "0": without the two round-6 rules for the 70B shards (A/B switch)
 FUSED_MAX_K = 4096
 FUSED_QKV_M256_MAX_L2_BYTES = 110e6
+# the bounds of _measured(): tile traffic (M tiles x weight bytes) of a qkv projection (K <= 4096, deeper) and of a residual projection
+# of 4096 < K <= 5632, and the weight bytes up to which a one-tile step prefers the tile kernel or its K split (5120 x 27 648 at one
+# row: skinny 58.8, split 65.4; 28 672 x 4096 at 32 rows: skinny 46.0, tile 47.0)
+FUSED_QKV_MAX_L2_BYTES = 270e6
+FUSED_QKV_DEEP_MAX_L2_BYTES = 230e6
+FUSED_MAX_L2_BYTES_DEEP_RESID = 100e6
+SPLIT_ONE_TILE_MAX_BYTES = 150e6
+SWIGLU_ONE_TILE_MAX_BYTES = 210e6
 # round 5 (profiles/r05_fused_tp8_shard_tiles.txt, M = 256): two more TP8 shards of the 8B verify pass go to the fused kernel --
 # w1|w3 (29.4 MB; 2 x 2 tiles: 21.1-22.3 us against 24.1 for the library + the SiLU*mul launch) and wo (4.2 MB, K = 512:
 # 12.0 against 14.1 incl. the add + norm behind it); w2 (14.7 MB: 17.1 vs 16.9) and everything wider stay on the library
@@ -122,12 +131,106 @@ def want_packed(N: int, K: int, swiglu: bool = False, int8: bool = False, rows=N
     kinds = ("swiglu",) if swiglu else ("plain", "resid", "qkv")
     for M in ((1,) + tuple(range(32, 257, 32)) if rows is None else tuple(m for m in rows if m <= 256)):
         # (default: every 32-row tile count a rule can depend on)
-        if use_skinny(M, N, K, swiglu, False, True):
-            return True
         for kind in kinds:
+            if use_skinny(M, N, K, swiglu, False, True, kind):
+                return True
             if use_block(M, N, K, kind) or use_fused(M, N, K, kind, absorbs_norm=True) or use_split(M, N, K, kind):
                 return True
     return False
+
+
+# Shapes the library holds a measured solution for (tuned/gemm_gfx950.csv, "tn_N_M_K_...").  There the library is a good deal faster
+# than where it has to guess (8B wqkv, 6144 x 4096: 20.6 us at 64 rows and 27 at 256; at 96 and 192, which the table does not hold,
+# 28.5 and 39.0), so rules below that would take a narrow product away from it leave these alone.
+_TUNED = None
+
+
+def _tuned(M: int, N: int, K: int) -> bool:
+    global _TUNED
+    if _TUNED is None:
+        path = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tuned", "gemm_gfx950.csv")
+        rows = set()
+        if os.path.exists(path):
+            with open(path) as f:
+                for line in f:
+                    m = re.match(r"GemmTunableOp_BFloat16_TN,tn_(\d+)_(\d+)_(\d+)_", line)
+                    if m:
+                        rows.add((int(m.group(2)), int(m.group(1)), int(m.group(3))))
+        _TUNED = rows
+    return (M, N, K) in _TUNED
+
+
+def _measured(M: int, N: int, K: int, kind: str, absorbs_norm: bool):
+    """The kernel for the shapes where the general rules below (drawn for the 1B and 8B models at 32, 64, 128 and 256 rows) were
+    measured to pick a slower one of the framework's own kernels, or the library where one of them is faster: "fused" | "block" |
+    "skinny" | "split", None: the general rules.  Times in us, the whole sub-step (with the add + norm, the rope or the SiLU*mul
+    behind it), graph-captured, weights cycled.  `kind` "planes": an output projection whose combine is the residual add + norm
+    launch of a model that keeps its residual in float32 (the tile kernel's residual epilogue is no choice there)."""
+    if M > 256 or K % 128 or N % 32:
+        return None
+    nbytes, m_tiles, tiles = N * K * 2, (M + 31) // 32, N // 128
+    # the block kernel takes 128 columns a workgroup: 160..256 of them are one nearly full round of the 256 CUs
+    one_round = N % 128 == 0 and BLOCK_MIN_TILES <= tiles <= 256
+    if kind == "plain":
+        # 33..128 rows of a 32 000-entry head in one round of block workgroups, against the skinny kernel's K slices and their
+        # combine: K = 2048 36.3 -> 30.3 (64 rows), 42.9 -> 32.6 (128); K = 4096 56.2 -> 50.8, 63.3 -> 53.4; K = 768, on the
+        # tile kernel, 19.4 / 30.9 -> 15.3 / 16.4.  More than one round is worse (128 256 entries: stays)
+        if 32 < M <= 128 and one_round:
+            return "block"
+        # one M tile over a long stream of columns: the tile kernel's workgroups each finish their columns, nothing to combine.
+        # 128 256 x 4096 at one row 172 -> 158, x 2048 92 -> 81; 32 000 x 4096 47.9 -> 44.6.  At 32 rows only in one round:
+        # 32 000 x 2048 31.7 -> 26.9, x 4096 51.5 -> 49.3, 14 336 x 4096 27.0 -> 25.2, but x 5120 60.0 against 61.2 and
+        # 128 256 x 2048 93.8 against 101
+        if M <= (32 if tiles <= 256 and K <= FUSED_MAX_K else 16) and N >= 14336 and nbytes >= MIN_STREAM_BYTES:
+            return "fused"
+    if kind == "swiglu":
+        if M <= 32 and N >= 14336 and not absorbs_norm and MIN_STREAM_BYTES <= nbytes <= SWIGLU_ONE_TILE_MAX_BYTES:
+            return "fused"            # 24 576 x 4096: 38.4 -> 35.5 (one row), 41.0 -> 38.3 (32); with a norm to absorb skinny is faster
+        # 65..128 rows, more than one round of block workgroups (296 or 432: the last round nearly empty): 37 888 x 3584
+        # 84.6 -> 81.0 on the skinny kernel, 55 296 x 5120 133 -> 122 (128 rows), 124 -> 115 (96)
+        if 64 < M <= 128 and N % 128 == 0 and tiles > 256:
+            return "skinny"
+    if kind in ("resid", "planes") and N <= 8192:
+        if K >= 8192 and nbytes >= MIN_STREAM_BYTES:
+            # the deep projections.  The skinny kernel cuts K into slices that divide K / 128: with K = 14 336 = 128 * 112 its
+            # grid is full, with 18 944 = 128 * 148 or 27 648 = 128 * 216 it is not, and the block kernel (64-wide slices, any
+            # remainder) is level or ahead from 33 rows on: 3584 x 18 944 47.9 / 58.1 / 63.2 -> 37.5 / 38.5 / 41.0 at 64 / 96 / 128,
+            # 5120 x 27 648 72 / 79 / 85 -> 65 / 64 / 66; 4096 columns over 14 336 stay (32.2 / 36.2 / 37.8 against
+            # 34.0 / 36.5 / 39.1)
+            if M <= 32 and kind == "resid" and nbytes <= SPLIT_ONE_TILE_MAX_BYTES:
+                return "split"        # 3584 x 18 944 37.1 / 43.7 -> 30.5 / 31.7 at 1 / 32 rows, 4096 x 14 336 28.2 -> 27.2
+            if 32 < M <= 128 and N % 128 == 0 and N % 4096:
+                return "block"
+        if FUSED_MAX_K < K < 8192:
+            if kind == "planes":
+                # 2048 x 7680: 16.0 / 16.2 / 20.3 / 26.5 on the tile kernel's K split -> 13.2 / 13.6 / 15.9 / 19.2 (1 / 8 / 32 / 64)
+                return "skinny" if M <= 64 else "split" if M <= 128 else None
+            if K <= 5632 and M <= 128:
+                if M <= 32 and nbytes < 30e6:
+                    return "skinny"   # 2048 x 5632: 14.3 / 13.4 / 18.4 in the library -> 12.1 / 12.5 / 14.8 (1 / 8 / 32 rows)
+                if m_tiles * nbytes <= FUSED_MAX_L2_BYTES_DEEP_RESID:
+                    return "fused"    # 2048 x 5632 21.1 / 19.4 -> 15.2 / 14.5 (64 / 128), 5120 x 5120 22.8 -> 16.5 (32)
+        # 3584..5632 deep and wide, more rows than the tile kernel's budget: the library, untuned, 23.8 / 26.5 / 33.8 ->
+        # 21.9 / 23.6 / 25.5 (3584 x 3584 at 96 / 128 / 192) and 26.1 / 36.6 / 54.8 -> 24.8 / 28.7 / 32.6 (5120 x 5120 at 64 / 128 /
+        # 256), 25.9 -> 22.7 (4096 x 4096 at 96)
+        if (kind == "resid" and 3584 <= K <= 5632 and N >= 3584 and N % 128 == 0 and M > (32 if K > FUSED_MAX_K else 64)
+                and not (M > 128 and _WO256 != "0" and K <= FUSED_MAX_K and nbytes <= FUSED_M256_RESID_T22_MAX_BYTES
+                         and (N // 64) * ((m_tiles + 1) // 2) >= 192) and not _tuned(M, N, K)):
+            return "block"
+    if kind == "planes" and K <= FUSED_MAX_K and M > 128 and use_fused(M, N, K, "resid"):
+        return "skinny"               # 4096 x 4096 on the tile kernel's K split 36.3 / 33.8 -> 27.5 / 28.8 (192 / 256 rows)
+    if kind == "qkv" and not _tuned(M, N, K):
+        # the tile kernel ends in rope + append; the library needs a launch for that, and has no measured solution here: 4608 x 3584
+        # 25.0 / 27.8 / 35.2 / 40.5 -> 18.0 / 22.8 / 27.3 / 32.0 (96 / 128 / 192 / 256 rows), 6144 x 4096 28.5 -> 25.0 (96),
+        # 7168 x 5120 31.5 / 34.7 -> 26.0 / 32.2 (64 / 96)
+        lim = FUSED_QKV_MAX_L2_BYTES if K <= FUSED_MAX_K else FUSED_QKV_DEEP_MAX_L2_BYTES
+        if K <= 5632 and N >= 4096 and m_tiles * nbytes <= lim and (N // 32) * m_tiles >= 100:
+            return "fused"
+    # ... and where its budget ends, the block kernel ahead of the rope launch: 7168 x 5120 39.3 / 48.5 / 57.4 -> 36.6 / 40.3 / 43.8
+    # (128 / 192 / 256), 6144 x 4096 39.0 -> 35.6 (192)
+    if kind == "plain" and 96 < M and 4096 <= K <= 5632 and N % 128 == 0 and 40 <= tiles <= 64 and not _tuned(M, N, K):
+        return "block"
+    return None
 
 
 def use_fused(M: int, N: int, K: int, kind: str = "plain", absorbs_norm: bool = False) -> bool:
@@ -137,6 +240,10 @@ def use_fused(M: int, N: int, K: int, kind: str = "plain", absorbs_norm: bool = 
         return False
     if _FUSED == "1":
         return True
+    own = _measured(M, N, K, kind, absorbs_norm)
+    if own is not None:
+        return own == "fused"
+    kind = "resid" if kind == "planes" else kind
     m_tiles = (M + 31) // 32
     # a product the kernel runs with 2 x 2 tiles (csrc/tilegemm.hip launch_tile_pro: two M tiles, an even number of column
     # tiles, >= 192 tile groups; with the deferred-norm prologue since round 6, K <= 4096) re-reads the weights once per
@@ -179,13 +286,15 @@ def use_fused(M: int, N: int, K: int, kind: str = "plain", absorbs_norm: bool = 
     return kind == "qkv" and l2_bytes <= FUSED_QKV_M256_MAX_L2_BYTES and K <= FUSED_MAX_K
 
 
-def use_skinny(M: int, N: int, K: int, swiglu: bool, int8: bool, packed: bool) -> bool:
+def use_skinny(M: int, N: int, K: int, swiglu: bool, int8: bool, packed: bool, kind: str = None, absorbs_norm: bool = False) -> bool:
     if _MODE == "lib" or M > 256:
         return False
     if _MODE == "hip" or int8:          # int8 rows are only streamed by md_linear (the library path dequantises)
         return True
     if not packed:
         return False
+    if _measured(M, N, K, kind or ("swiglu" if swiglu else "plain"), absorbs_norm) == "skinny":
+        return True
     nbytes = N * K * 2
     if M <= 64:
         return nbytes >= MIN_STREAM_BYTES
@@ -212,10 +321,13 @@ def set_split(mode: str):
 
 def use_split(M: int, N: int, K: int, kind: str) -> bool:
     """md_linear_fused_split_add_rmsnorm for this output projection (kind "resid")?"""
-    if _MODE == "lib" or _SPLIT == "0" or kind != "resid" or M > 256 or K % 128 or N % 32 or N > 8192:
+    if _MODE == "lib" or _SPLIT == "0" or kind not in ("resid", "planes") or M > 256 or K % 128 or N % 32 or N > 8192:
         return False
     if _SPLIT == "1":
         return True
+    own = _measured(M, N, K, kind, False)
+    if own is not None:
+        return own == "split"
     return M <= SPLIT_MAX_M and K >= SPLIT_MIN_K and N * K * 2 < MIN_STREAM_BYTES
 
 
@@ -233,13 +345,17 @@ def block_mode() -> str:
     return _BLOCK
 
 
-def use_block(M: int, N: int, K: int, kind: str) -> bool:
+def use_block(M: int, N: int, K: int, kind: str, absorbs_norm: bool = False) -> bool:
     """md_linear_block for this linear?  kind: "swiglu", "resid" (output projection + residual add + RMSNorm: the split-K
     combine launch does both) or "plain"."""
     if _MODE == "lib" or _BLOCK == "0" or M > 256 or N % 128 or K % 64:
         return False
     if _BLOCK == "1":
         return True
+    own = _measured(M, N, K, kind, absorbs_norm)
+    if own is not None:
+        return own == "block"
+    kind = "resid" if kind == "planes" else kind
     tiles = N // 128
     if M > 128:
         if kind == "resid":
@@ -254,10 +370,10 @@ def choose(M: int, N: int, K: int, swiglu: bool, int8: bool, packed: bool, kind:
     """"fused" (md_linear_fused), "block" (md_linear_block), "skinny" (md_linear) or "lib" (hipBLASLt) for one linear
     of a step."""
     kind = kind or ("swiglu" if swiglu else "plain")
-    if packed and not int8 and _BLOCK == "1" and use_block(M, N, K, kind):
+    if packed and not int8 and _BLOCK == "1" and use_block(M, N, K, kind, absorbs_norm):
         return "block"
     if packed and not int8 and use_fused(M, N, K, kind, absorbs_norm):
         return "fused"
-    if packed and not int8 and use_block(M, N, K, kind):
+    if packed and not int8 and use_block(M, N, K, kind, absorbs_norm):
         return "block"
-    return "skinny" if use_skinny(M, N, K, swiglu, int8, packed) else "lib"
+    return "skinny" if use_skinny(M, N, K, swiglu, int8, packed, kind, absorbs_norm) else "lib"

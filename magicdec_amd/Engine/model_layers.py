@@ -322,8 +322,8 @@ class LayeredTransformer(Transformer):
     def _project_how(self, M, N, K, packed):
         """Where an output projection runs: a split-K GEMM up to its float32 planes ("skinny" | "tile" | "block"; the residual
         add + norm launch that follows is its combine), the skinny GEMM with 16-bit rows ("rows"), or the library."""
-        how = choose(M, N, K, False, False, packed, "resid") if packed else "lib"
-        if packed and how != "block" and (how == "fused" or use_split(M, N, K, "resid")):
+        how = choose(M, N, K, False, False, packed, "planes") if packed else "lib"
+        if packed and how != "block" and (how == "fused" or use_split(M, N, K, "planes")):
             how = "tile"                     # the tile kernel's residual epilogue is 16-bit: take its K-split form instead
         if how in ("tile", "block", "skinny") and ops.linear_planes_count(how, M, N, K):
             return how
