@@ -25,6 +25,11 @@ from .model_core import PageTable
 PAGE_SIZE = 128    # Engine/SnapKV/backend.py:31
 CHUNK = 128        # Engine/SnapKV/backend.py:236
 PREFILL_ROWS = 16384   # rows of one prefill step where the portion is free to choose (models addressed by position, `step`)
+# ... and of a prompt's portion in the fixed-batch engines.  What a 16-bit product reaches on an 8B layer at 128 rows: 450 TFLOP/s (the
+# weight stream), at 512: 590..1240, at 4096 and more about 1300.  Two layers, us, against portions of 128 tokens a request: one request
+# of 8 000 tokens 34 485 -> 7 765 at 4096 rows, 7 661 at 8192; four of 1 500 (7B) 12 664 -> 7 040, 5 927; four of 2 081 12 200 -> 6 641,
+# 6 496; one of 600 2 969 -> 1 572.  8192 is what 64 requests had already; a layer's activations take 1.4 GB there on a 32B model.
+PROMPT_ROWS = 8192
 
 
 def default_kv_layout():
@@ -145,6 +150,9 @@ class _PagedState:
 
 
 class _BackendBase:
+    mapped = False         # models addressed by position (_geometry)
+    prefill_chunk = CHUNK
+
     def __init__(self, dtype=torch.bfloat16, device="cuda:0"):
         self.dtype, self.device = dtype, device
         self.model = None
@@ -200,6 +208,30 @@ class _BackendBase:
         releases weight copies for exactly these (Transformer.setup_caches(decode_rows=...))."""
         B = self.batch_size
         return sorted({B * int(n) for n in (1,) + ((2,) if two_token_step else ()) + tuple(per_request) if n})
+
+    def _portions(self, seq_len):
+        """The portions [(first token, tokens)] of a prompt whose keys all stay in the cache: any division gives every token the same
+        keys, so portions are as long as the matrix products want them.  Two stay as they are: the last CHUNK's tokens (their logits and
+        tokens are what encode returns, and the SnapKV select's window) and, for an fp8 cache, the first CHUNK, which sets its scales."""
+        if self.mapped or torch.device(self.device).type == "cpu":       # (the CPU's products round by their row counts)
+            chunk = self.prefill_chunk
+            return [(a, min(chunk, seq_len - a)) for a in range(0, seq_len, chunk)]
+        chunks = max(0, seq_len - 1) // CHUNK                    # ahead of the last one
+        out, at = [], 0
+        if chunks and self.model.layers[0].attention.kv_cache.scales("kv_cache") is not None:
+            out, at, chunks = [(0, CHUNK)], CHUNK, chunks - 1
+        if chunks:
+            most = max(1, PROMPT_ROWS // (self.batch_size * CHUNK))
+            parts = -(-chunks // most)
+            for i in range(parts):
+                n = (chunks * (i + 1) // parts - chunks * i // parts) * CHUNK
+                out.append((at, n))
+                at += n
+        return out + [(at, seq_len - at)] if seq_len > at else out
+
+    def _map_portion(self, end):
+        """Pages for a prompt's first `end` tokens."""
+        self._t.map_pages(-(-end // PAGE_SIZE), (end - 1) % PAGE_SIZE + 1)
 
     def _last_rows(self, n):
         """Extra prefill arguments of models addressed by position: logits for the last of every request's n rows only (their
@@ -318,22 +350,16 @@ class SnapKVTargetBackend(_BackendBase):
         self._prefill_begin()
         seq_len = input_ids.shape[1]
         tokens = None
-        chunk = self.prefill_chunk
-        num_chunks = (seq_len + chunk - 1) // chunk
         is_last = False
-        done = 0
-        for i in range(num_chunks):
-            ids = input_ids[:, i * chunk:min((i + 1) * chunk, seq_len)]
-            n = ids.shape[1]
-            if n != chunk:
-                is_last = True
-            self._t.map_pages(i + 1, n)                       # pre_encode
-            self.model.skip_head = i != num_chunks - 1
+        for done, n in self._portions(seq_len):
+            ids = input_ids[:, done:done + n]
+            is_last = done + n == seq_len and n % self.prefill_chunk != 0
+            self._map_portion(done + n)                       # pre_encode
+            self.model.skip_head = done + n != seq_len
             tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table((n, done + n)), is_last=is_last,
                                         draft_tab=self._d.table() if (self.is_spec and is_last) else None,
                                         ctx_len=done + n, **self._last_rows(n))
             self.cachelens += n
-            done += n
         self.model.skip_head = False
         if self.mapped:
             tokens = tokens.view(-1, 1)
@@ -508,22 +534,16 @@ class SnapKVDraftBackend(_BackendBase):
         self._prefill_begin()
         seq_len = input_ids.shape[1]
         tokens = None
-        chunk = self.prefill_chunk
-        num_chunks = (seq_len + chunk - 1) // chunk
         is_last = False
-        done = 0
-        for i in range(num_chunks):
-            ids = input_ids[:, i * chunk:min((i + 1) * chunk, seq_len)]
-            n = ids.shape[1]
-            if n != chunk:
-                is_last = True
-            self._t.map_pages(i + 1, n)
-            self.model.skip_head = i != num_chunks - 1
+        for done, n in self._portions(seq_len):
+            ids = input_ids[:, done:done + n]
+            is_last = done + n == seq_len and n % self.prefill_chunk != 0
+            self._map_portion(done + n)                       # pre_encode
+            self.model.skip_head = done + n != seq_len
             tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table((n, done + n)), is_last=is_last,
                                         draft_tab=self._d.table() if (self.is_compress and is_last) else None,
                                         ctx_len=done + n, **self._last_rows(n))
             self.cachelens += n
-            done += n
         self.model.skip_head = False
         if self.mapped:
             tokens = tokens.view(-1, 1)
@@ -692,12 +712,10 @@ class StreamingSelfSpecBackend(_BackendBase, _StreamingMixin):
         self._prefill_begin()
         seq_len = input_ids.shape[1]
         tokens = None
-        num_chunks = (seq_len + CHUNK - 1) // CHUNK
-        for i in range(num_chunks):
-            ids = input_ids[:, i * CHUNK:min((i + 1) * CHUNK, seq_len)]
-            n = ids.shape[1]
-            self._t.map_pages(i + 1, n)
-            self.model.skip_head = i != num_chunks - 1
+        for done, n in self._portions(seq_len):
+            ids = input_ids[:, done:done + n]
+            self._map_portion(done + n)
+            self.model.skip_head = done + n != seq_len
             tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table())
             self.cachelens += n
         self.model.skip_head = False

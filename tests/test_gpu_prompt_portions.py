@@ -1,0 +1,59 @@
+"""A prompt in longer portions against portions of 128 tokens: the same tables, lengths and fp8 scales, the rows and logits of 16-bit
+arithmetic.  On the GPU (-m gpu)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def engine(which, kv, batch, limit):
+    from magicdec_amd.Engine.model_core import transformer_configs
+    transformer_configs["portions-test"] = dict(block_size=4096, n_layer=2, n_head=8, n_local_heads=2, dim=512, intermediate_size=1024,
+                                                vocab_size=512)
+    if which == "draft":
+        from magicdec_amd.Engine.SnapKV.backend_draft import LMBackend_Draft
+        e, kw = LMBackend_Draft(dtype=torch.bfloat16, device=DEV, draft_budget=129), dict(draft_budget=129, window_size=32)
+    elif which == "spec":
+        from magicdec_amd.Engine.SnapKV.backend import LMBackend
+        e, kw = LMBackend(dtype=torch.bfloat16, device=DEV, dec_len=4, draft_dec_len=1), dict(draft_budget=129, window_size=32, kv_dtype=kv)
+    elif which == "stream":
+        from magicdec_amd.Engine.StreamingLLM.backend import LMBackend
+        e, kw = LMBackend(dtype=torch.bfloat16, device=DEV, dec_len=4), dict(draft_budget=129, kv_dtype=kv)
+    else:
+        from magicdec_amd.Engine.SnapKV.backend import LMBackend
+        e, kw = LMBackend(dtype=torch.bfloat16, device=DEV, dec_len=4), dict(kv_dtype=kv)
+    e.load_model("none/portions-test/model.pth", use_tp=False)
+    e.setup_caches(max_batch_size=batch, max_seq_length=limit, **kw)
+    return e
+
+
+@pytest.mark.parametrize("which,kv,batch,prompt", [
+    ("plain", "bf16", 3, 1), ("plain", "bf16", 1, 128), ("plain", "bf16", 2, 129), ("plain", "bf16", 3, 256), ("plain", "bf16", 5, 1337),
+    ("plain", "bf16", 33, 700), ("plain", "bf16", 65, 300), ("plain", "fp8", 2, 128), ("plain", "fp8", 2, 200), ("plain", "fp8", 3, 1500),
+    ("spec", "bf16", 2, 1056), ("spec", "fp8", 3, 416), ("draft", "bf16", 4, 800), ("stream", "bf16", 2, 555), ("stream", "fp8", 2, 1024)])
+def test_longer_portions(which, kv, batch, prompt, monkeypatch):
+    import magicdec_amd.Engine.backend_core as core
+    ids = torch.randint(4, 512, (batch, prompt), generator=torch.Generator().manual_seed(prompt)).to(DEV)
+    seen = []
+    for rows in (core.PROMPT_ROWS, 0):
+        monkeypatch.setattr(core, "PROMPT_ROWS", rows)
+        e = engine(which, kv, batch, 2048)
+        parts = e._portions(prompt)
+        # in order and whole, each at a page's start, the last CHUNK's tokens by themselves
+        assert [a for a, _ in parts] == [0] + [a + n for a, n in parts[:-1]] and sum(parts[-1]) == prompt
+        assert all(a % 128 == 0 for a, _ in parts) and parts[-1][1] == (prompt - 1) % 128 + 1
+        assert all(n == 128 for _, n in parts[:-1]) if rows == 0 else all(n * batch <= max(rows, 128 * batch) for _, n in parts)
+        for _ in range(2):                                           # (a second prompt over the first one's state)
+            tokens = e.encode(ids)
+        kvs = [b.attention.kv_cache for b in e.model.layers]
+        seen.append(dict(tokens=tokens, logits=e.model._last_logits.float(), lens=e.cachelens, pages=e._t.table(),
+                         scales=[s for c in kvs for s in (c.scales() or ())], rows=[c.kv_cache.float() for c in kvs]))
+    a, b = seen
+    assert a["tokens"].shape == b["tokens"].shape == (batch, parts[-1][1])
+    assert torch.equal(a["lens"], b["lens"]) and a["pages"].max_pages == b["pages"].max_pages
+    assert all(torch.equal(getattr(a["pages"], k), getattr(b["pages"], k)) for k in ("indices", "indptr", "last_page_len"))
+    assert all(torch.equal(x, y) for x, y in zip(a["scales"], b["scales"]))
+    # each within 0.8 % of exact arithmetic; an fp8 row rounds to 2^-4 of itself, so a moved rounding shows as far as that in few places
+    for x, y in zip([a["logits"]] + a["rows"], [b["logits"]] + b["rows"]):
+        assert (x - y).norm() <= (0.016 if kv == "bf16" else 0.03) * y.norm()
