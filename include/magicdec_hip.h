@@ -205,6 +205,13 @@ int md_streaming_rotate(const void* cache, void* rot_cache, int B, int valid_len
                         int pages_per_req, int KH, int D, int page_size, const float* cos_sin,
                         int max_pos, md_stream_t stream);
 
+/* Both steps above for ceil(tokens / portion) portions of a prompt at once.  k_new / v_new: rows b * tokens + t.  windows: portion c of
+ * request b sees pages (b * portions + c) * pages_per_req ..., keys rotated by slot, rows past its length unwritten.  next: every slot
+ * of the cache behind the last portion, its keys rotated (by slot, up to its length) if rotate_next.  ctx: tokens in the cache. */
+int md_streaming_windows(const void* k_new, const void* v_new, int64_t k_row_stride, int64_t v_row_stride, const void* cache,
+                         void* windows, void* next, int B, int tokens, int portion, int ctx, int kv_len, int sink, int pages_per_req,
+                         int KH, int D, int page_size, int rotate_next, const float* cos_sin, int max_pos, md_stream_t stream);
+
 /* ------------------------------------------------------------------------
  * K9  RMSNorm / SiLU*mul / residual   reference: Engine/SnapKV/model.py:451-469
  * rmsnorm: y = bf16( x_f32 * rsqrt(mean(x^2)+eps) ) * w   (weight multiply in

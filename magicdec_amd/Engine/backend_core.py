@@ -30,6 +30,7 @@ PREFILL_ROWS = 16384   # rows of one prefill step where the portion is free to c
 # of 8 000 tokens 34 485 -> 7 765 at 4096 rows, 7 661 at 8192; four of 1 500 (7B) 12 664 -> 7 040, 5 927; four of 2 081 12 200 -> 6 641,
 # 6 496; one of 600 2 969 -> 1 572.  8192 is what 64 requests had already; a layer's activations take 1.4 GB there on a 32B model.
 PROMPT_ROWS = 8192
+PROMPT_WINDOWS = 512 << 20     # bytes of one pass's StreamingLLM windows: 64 portions at a budget of 1024 rows of 8 heads of 128
 
 
 def default_kv_layout():
@@ -584,27 +585,33 @@ class _StreamingMixin:
 
     def _stream_encode(self, input_ids, state: _PagedState, lens_attr, which):
         self._prefill_begin()
-        seq_len = input_ids.shape[1]
+        seq_len, B = input_ids.shape[1], self.batch_size
         tokens = None
         num_chunks = (seq_len + CHUNK - 1) // CHUNK
-        is_last = False
+        # chunks to a pass (md_streaming_windows): PROMPT_ROWS rows and PROMPT_WINDOWS bytes of them (one where the CPU's products round by their row counts)
+        cache = getattr(self.model.layers[0].attention.kv_cache, which)
+        most = 1 if cache.device.type == "cpu" else min(PROMPT_ROWS // (B * CHUNK),
+                                                        PROMPT_WINDOWS // (cache.numel() * cache.element_size()))
+        passes = -(-num_chunks // max(1, most))
         ctx = 0                                       # host mirror of the (capped) cache length
-        for i in range(num_chunks):
-            ids = input_ids[:, i * CHUNK:min((i + 1) * CHUNK, seq_len)]
-            n = ids.shape[1]
-            if n != CHUNK:
-                is_last = True
-            if ctx + n <= self.draft_budget:          # pre_encode (StreamingLLM/backend_draft.py:155-192)
-                state.map_pages(state.host_pages + 1, n)
+        for i in range(passes):
+            first, end = num_chunks * i // passes, num_chunks * (i + 1) // passes
+            ids = input_ids[:, first * CHUNK:min(end * CHUNK, seq_len)]
+            is_last = end * CHUNK > seq_len
+            start, pages = ctx, state.host_pages
+            for c in range(first, end):               # pre_encode (StreamingLLM/backend_draft.py:155-192)
+                n = min(CHUNK, seq_len - c * CHUNK)
+                pages, last = (pages + 1, n) if ctx + n <= self.draft_budget else (state.ppr, self.draft_budget % PAGE_SIZE)
+                ctx = min(ctx + n, self.draft_budget)
+            state.map_pages(pages, last)
+            self.model.skip_head = i != passes - 1
+            if end - first > 1:
+                tokens = self.model.stream_portions(ids, start, CHUNK, is_last, which, B)
             else:
-                state.map_pages(state.ppr, self.draft_budget % PAGE_SIZE)
-            self.model.skip_head = i != num_chunks - 1
-            tokens = self.model.stream_prefill(ids, ctx, self._qo(n), state.table(), is_last, which, self.batch_size)
-            ctx += n
+                tokens = self.model.stream_prefill(ids, start, self._qo(n), state.table(), is_last, which, B)
             lens = getattr(self, lens_attr)
-            lens += n
+            lens += ids.shape[1]
             if ctx >= self.draft_budget:
-                ctx = self.draft_budget
                 lens.fill_(self.draft_budget)
         self.model.skip_head = False
         self._prefill_end()

@@ -815,7 +815,8 @@ class Transformer(nn.Module):
         Engine/StreamingLLM/model_draft.py:102-143,309-326; draft_prefill / prefill_draft of StreamingLLM/model.py).
         ctx = tokens already in the (capped) cache, host int."""
         kv_len = self.draft_budget
-        dev = idx.device
+        overflow = ctx + idx.shape[1] > kv_len
+        off = torch.full((B,), (kv_len - idx.shape[1]) if overflow else ctx, dtype=torch.int32, device=idx.device)
 
         def fn(i, layer, y, n):
             if isinstance(y, ops.DeferredNorm):
@@ -823,8 +824,6 @@ class Transformer(nn.Module):
             q, k, v, _ = self._qkv(layer, y)
             cache = getattr(layer.attention.kv_cache, which)
             ppr = cache.shape[0] // B
-            overflow = ctx + n > kv_len
-            off = torch.full((B,), (kv_len - n) if overflow else ctx, dtype=torch.int32, device=dev)
             q_rot, _ = ops.rope(q, None, kv_append_indptr, off, self.rope_table, n_max=n)
             if not overflow:
                 ops.update_kv(k, v, kv_append_indptr, cache, tab.indices, tab.indptr, tab.last_page_len, n_max=n)
@@ -841,3 +840,41 @@ class Transformer(nn.Module):
             ops.streaming_rotate(cache, rot, B, valid, ppr, self.rope_table)
             return self._attend(q_rot, rot, kv_append_indptr, tab, n)
         return self._run(idx, fn)
+
+    def stream_portions(self, idx, ctx, portion, is_last, which, B):
+        """stream_prefill of several portions in one pass over the layers: what a portion sees of a layer's cache depends on that
+        layer's rows alone, so all of them are attended at once, each over pages of its own.  Tokens and logits of the last one."""
+        kv_len, tokens, dev = self.draft_budget, idx.shape[1], idx.device
+        cache0 = getattr(self.layers[0].attention.kv_cache, which)
+        ppr, page = cache0.shape[0] // B, cache0.shape[2]
+        starts = list(range(0, tokens, portion))
+        new = [min(portion, tokens - a) for a in starts]
+        valid = [min(min(ctx + a, kv_len) + n, kv_len) for a, n in zip(starts, new)]
+        pages = [-(-v // page) for v in valid]
+        each = [(b, c) for b in range(B) for c in range(len(starts))]
+        qo = [b * tokens + starts[c] for b, c in each] + [B * tokens]
+        indptr, indices = [0], []
+        for r, (_, c) in enumerate(each):
+            indices += range(r * ppr, r * ppr + pages[c])
+            indptr.append(len(indices))
+        # one upload for all the integers of the pass
+        cut = [qo, [valid[c] - new[c] for _, c in each], indices, indptr, [(valid[c] - 1) % page + 1 for _, c in each]]
+        flat = torch.tensor([v for part in cut for v in part], dtype=torch.int32).to(dev)
+        qo, off, indices, indptr, last = torch.split(flat, [len(part) for part in cut])
+        tab = PageTable(indices, indptr, last, max(pages))
+        windows = torch.empty((len(each) * ppr, *cache0.shape[1:]), dtype=cache0.dtype, device=dev)
+        following = torch.empty_like(cache0)
+        rotated = is_last and min(ctx + starts[-1], kv_len) + new[-1] > kv_len         # (as in stream_prefill)
+
+        def fn(i, layer, y, n):
+            if isinstance(y, ops.DeferredNorm):
+                y = y.materialize()
+            q, k, v, _ = self._qkv(layer, y)
+            cache = getattr(layer.attention.kv_cache, which)
+            q_rot, _ = ops.rope(q, None, qo, off, self.rope_table, n_max=portion)
+            ops.streaming_windows(k, v, cache, windows, following, portion, ctx, kv_len, SINK, ppr, self.rope_table, rotated)
+            cache.copy_(following)
+            return self._attend(q_rot, windows, qo, tab, portion)
+        rows = (torch.arange(B, device=dev).view(B, 1) * tokens + torch.arange(starts[-1], tokens, device=dev)).flatten()
+        out = self._run(idx, fn, head_rows=rows)
+        return None if out is None else out.view(B, -1)

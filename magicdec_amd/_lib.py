@@ -99,6 +99,7 @@ _SIGNATURES = {
     "md_ar_status_async": (c_int, [P, P, P]),
     "md_ar_destroy": (c_int, [P]),
     "md_streaming_shift_append": (c_int, [P, P, L, L, P, I, I, I, I, I, I, I, I, P]),
+    "md_streaming_windows": (c_int, [P, P, L, L, P, P, P, I, I, I, I, I, I, I, I, I, I, I, P, I, P]),
     "md_streaming_rotate": (c_int, [P, P, I, I, I, I, I, I, P, I, P]),
     "md_unpack_weight": (c_int, [P, P, I, I, I, P]),
     "md_linear_supported": (c_int, [I, I, I, I]),

@@ -12,7 +12,9 @@
 //       ascending groups, a group read before any of it is overwritten);
 //   md_streaming_rotate       : rows [0,valid_len) of every request, K rotated
 //       by position = slot index, V copied, into a scratch cache (or in place
-//       on the last chunk == the reference's kv_cache.copy_(rotated_kv)).
+//       on the last chunk == the reference's kv_cache.copy_(rotated_kv));
+//   md_streaming_windows      : both for several chunks at once, where they are
+//       too small to be passed one by one (few requests).
 // Bug-for-bug: the shift covers the whole [sink,kv_len) slot range even while
 // the tail slot has never been written (the zero row of the 2nd->3rd chunk
 // transition travels exactly as in the reference).
@@ -70,7 +72,26 @@ __global__ __launch_bounds__(256) void shift_append_kernel(const bf16_t* __restr
     }
 }
 
-// grid (valid_len, B); K rotated by pos = slot (same arithmetic as kvops.hip rope8), V copied
+// eight rotated elements (same arithmetic as kvops.hip rope8); c: their cos / sin pairs
+__device__ __forceinline__ u32x4 rotate8(const u32x4 x, const float* __restrict__ c) {
+    const f32x4 c0 = *reinterpret_cast<const f32x4*>(c);
+    const f32x4 c1 = *reinterpret_cast<const f32x4*>(c + 4);
+    u32x4 r;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const float xe = __uint_as_float(x[w] << 16);
+        const float xo = __uint_as_float(x[w] & 0xffff0000u);
+        const float co = w < 2 ? c0[(w & 1) * 2] : c1[(w & 1) * 2];
+        const float si = w < 2 ? c0[(w & 1) * 2 + 1] : c1[(w & 1) * 2 + 1];
+        const float ye = __fsub_rn(__fmul_rn(xe, co), __fmul_rn(xo, si));
+        const float yo = __fadd_rn(__fmul_rn(xo, co), __fmul_rn(xe, si));
+        const bf16x2 pk = {f32_to_bf16(ye), f32_to_bf16(yo)};
+        r[w] = *reinterpret_cast<const unsigned int*>(&pk);
+    }
+    return r;
+}
+
+// grid (valid_len, B); K rotated by pos = slot, V copied
 __global__ __launch_bounds__(256) void rotate_kernel(const bf16_t* __restrict__ cache, bf16_t* rot, int ppr, int KH, int D,
                                                      int page_size, const float* __restrict__ cos_sin, int max_pos) {
     const int b = blockIdx.y, s = blockIdx.x;
@@ -85,21 +106,7 @@ __global__ __launch_bounds__(256) void rotate_kernel(const bf16_t* __restrict__ 
     for (int i = threadIdx.x; i < 2 * cols; i += blockDim.x) {
         if (i < cols) {
             const u32x4 x = *reinterpret_cast<const u32x4*>(cache + off + i * 8);
-            const float* c = cs + (i % cpr) * 8;
-            const f32x4 c0 = *reinterpret_cast<const f32x4*>(c);
-            const f32x4 c1 = *reinterpret_cast<const f32x4*>(c + 4);
-            u32x4 r;
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                const float xe = __uint_as_float(x[w] << 16);
-                const float xo = __uint_as_float(x[w] & 0xffff0000u);
-                const float co = w < 2 ? c0[(w & 1) * 2] : c1[(w & 1) * 2];
-                const float si = w < 2 ? c0[(w & 1) * 2 + 1] : c1[(w & 1) * 2 + 1];
-                const float ye = __fsub_rn(__fmul_rn(xe, co), __fmul_rn(xo, si));
-                const float yo = __fadd_rn(__fmul_rn(xo, co), __fmul_rn(xe, si));
-                const bf16x2 pk = {f32_to_bf16(ye), f32_to_bf16(yo)};
-                r[w] = *reinterpret_cast<const unsigned int*>(&pk);
-            }
+            const u32x4 r = rotate8(x, cs + (i % cpr) * 8);
             *reinterpret_cast<u32x4*>(rot + off + i * 8) = r;
         } else if (!inplace) {
             const int ii = i - cols;
@@ -109,7 +116,82 @@ __global__ __launch_bounds__(256) void rotate_kernel(const bf16_t* __restrict__ 
     }
 }
 
+// The caches that C portions of a prompt see, all at once.  What a slot holds after portion c follows from the cache before the first of
+// them and from their new rows alone, so no portion waits for the one ahead of it:
+//   while a portion fits, slot s < ctx is the old row and slot ctx + j new row j;
+//   from portion f on, the first that does not, every slot >= sink moves up by the m tokens since then: slot s is slot s + m of
+//   that moment, or new row s + m - kv_len of those m (the moment's slots past its tokens are what the cache holds there).
+// blockIdx.y = c < C writes portion c's rows, keys rotated by their slot, as pages of their own; c = C writes the cache as the last
+// portion leaves it (all slots) to `next`: the cache itself is still being read.  Bound by the traffic, 2 x 2 x (C + 1) x kv_len rows a
+// request.
+constexpr int kWindowRows = 4;
+
+struct WindowParams {
+    const bf16_t *k, *v, *cache;
+    bf16_t *windows, *next;
+    const float* cos_sin;
+    int64_t ks, vs;
+    int tokens, portion, portions, ctx, kv_len, sink, ppr, KH, D, page_size, max_pos, rotate_next;
+};
+
+__global__ __launch_bounds__(256) void windows_kernel(const WindowParams p) {
+    const int b = blockIdx.z, c = min((int)blockIdx.y, p.portions - 1);
+    const bool last = (int)blockIdx.y == p.portions;
+    const int begin = c * p.portion, n = min(p.portion, p.tokens - begin);
+    const int before = min(p.ctx + begin, p.kv_len);
+    const int pre = (p.kv_len - p.ctx) / p.portion * p.portion;      // tokens ahead of portion f
+    const bool over = before + n > p.kv_len;
+    const int valid = over ? p.kv_len : before + n, m = over ? begin + n - pre : 0;
+    const int slots = last ? p.ppr * p.page_size : valid;
+    const int row = p.KH * p.D, cols = row / 8, cpr = p.D / 8;
+    for (int i = threadIdx.x; i < kWindowRows * 2 * cols; i += 256) {
+        const int s = blockIdx.x * kWindowRows + i / (2 * cols), t = i % (2 * cols);
+        if (s >= slots) break;
+        const bool isv = t >= cols;
+        const int col = isv ? t - cols : t;
+        const int at = over && s >= p.sink && s < valid ? s + m : s;
+        int token = -1;
+        if (at >= p.kv_len && s < valid)
+            token = pre + at - p.kv_len;
+        else if (s < valid && at >= p.ctx && at < (over ? p.ctx + pre : valid))
+            token = at - p.ctx;
+        const int64_t half = isv ? (int64_t)p.page_size * row : 0;
+        const bf16_t* src = token >= 0 ? (isv ? p.v : p.k) + ((int64_t)b * p.tokens + token) * (isv ? p.vs : p.ks)
+                                       : p.cache + slot_offset(b, at, p.ppr, p.page_size, row) + half;
+        u32x4 x = *reinterpret_cast<const u32x4*>(src + col * 8);
+        if (!isv && s < valid && (!last || p.rotate_next))
+            x = rotate8(x, p.cos_sin + (int64_t)min(s, p.max_pos - 1) * p.D + col % cpr * 8);
+        bf16_t* dst = last ? p.next + slot_offset(b, s, p.ppr, p.page_size, row)
+                           : p.windows + slot_offset(b * p.portions + c, s, p.ppr, p.page_size, row);
+        *reinterpret_cast<u32x4*>(dst + half + col * 8) = x;
+    }
+}
+
 }  // namespace
+
+extern "C" int md_streaming_windows(const void* k_new, const void* v_new, int64_t k_row_stride, int64_t v_row_stride, const void* cache,
+                                    void* windows, void* next, int B, int tokens, int portion, int ctx, int kv_len, int sink,
+                                    int pages_per_req, int KH, int D, int page_size, int rotate_next, const float* cos_sin, int max_pos,
+                                    md_stream_t stream) {
+    MD_CHECK_ARG(k_new && v_new && cache && windows && next && cos_sin, "md_streaming_windows: null pointer argument");
+    MD_CHECK_ARG(next != cache && windows != cache && windows != next, "md_streaming_windows: the cache is read while the others are written");
+    MD_CHECK_ARG(B > 0 && B <= 65535 && tokens > 0 && portion > 0 && ctx >= 0 && ctx <= kv_len && kv_len > sink && sink >= 0 && KH > 0 &&
+                     D > 0 && D % 8 == 0 && page_size > 0 && (int64_t)pages_per_req * page_size >= kv_len && max_pos > 0,
+                 "md_streaming_windows: bad shape tokens=%d portion=%d ctx=%d kv_len=%d sink=%d pages_per_req=%d", tokens, portion, ctx,
+                 kv_len, sink, pages_per_req);
+    MD_CHECK_ARG((((uintptr_t)k_new | (uintptr_t)v_new | (uintptr_t)cache | (uintptr_t)windows | (uintptr_t)next | (uintptr_t)cos_sin) & 15) == 0 &&
+                     k_row_stride % 8 == 0 && v_row_stride % 8 == 0,
+                 "md_streaming_windows: 16-byte alignment / stride multiple of 8 required");
+    const int portions = (int)(((int64_t)tokens + portion - 1) / portion);
+    MD_CHECK_ARG(portions < 65535, "md_streaming_windows: %d portions", portions);
+    const WindowParams p = {(const bf16_t*)k_new, (const bf16_t*)v_new, (const bf16_t*)cache, (bf16_t*)windows, (bf16_t*)next, cos_sin,
+                            k_row_stride, v_row_stride, tokens, portion, portions, ctx, kv_len, sink, pages_per_req, KH, D, page_size,
+                            max_pos, rotate_next};
+    const int slots = pages_per_req * page_size;
+    hipLaunchKernelGGL(windows_kernel, dim3((slots + kWindowRows - 1) / kWindowRows, portions + 1, B), dim3(256), 0, (hipStream_t)stream, p);
+    MD_CHECK_LAUNCH("md_streaming_windows");
+    return MD_OK;
+}
 
 extern "C" int md_streaming_shift_append(const void* k_new, const void* v_new, int64_t k_row_stride,
                                          int64_t v_row_stride, void* cache, int B, int n_new, int kv_len, int sink,

@@ -265,6 +265,26 @@ def streaming_rotate(kv_cache, rot_cache, B, valid_len, pages_per_req, table: Ro
                                   _p(table.table), table.max_pos, _stream()), "md_streaming_rotate")
 
 
+def streaming_windows(k_new, v_new, kv_cache, windows, following, portion, ctx, kv_len, sink, pages_per_req, table: RopeTable,
+                      rotate_following):
+    """What portions of `portion` tokens see of the draft cache, for all of k_new / v_new [B * tokens, KH, D] at once: windows
+    [B * portions * pages_per_req, 2, page, KH, D] (request-major) with the keys rotated by slot, and `following` (shaped like
+    kv_cache): the cache behind the last one, its keys rotated too if asked for.  ctx: tokens in the cache before."""
+    _gpu(k_new, v_new, kv_cache, windows, following)
+    KH, D = kv_cache.shape[3], kv_cache.shape[4]
+    B = kv_cache.shape[0] // pages_per_req
+    tokens = k_new.shape[0] // B
+    if (k_new.shape != v_new.shape or k_new.shape != (B * tokens, KH, D) or following.shape != kv_cache.shape
+            or windows.shape != (kv_cache.shape[0] * (-(-tokens // portion)), *kv_cache.shape[1:])
+            or any(t.dtype != torch.bfloat16 for t in (k_new, v_new, kv_cache, windows, following))
+            or not (kv_cache.is_contiguous() and windows.is_contiguous() and following.is_contiguous())
+            or table.head_dim != D):
+        raise ValueError("streaming_windows: 16-bit rows [B * tokens, KH, D] and contiguous caches of the draft cache's pages expected")
+    check(_lib.load().md_streaming_windows(_p(k_new), _p(v_new), _row_stride(k_new), _row_stride(v_new), _p(kv_cache), _p(windows),
+                                           _p(following), B, tokens, portion, ctx, kv_len, sink, pages_per_req, KH, D, kv_cache.shape[2],
+                                           int(rotate_following), _p(table.table), table.max_pos, _stream()), "md_streaming_windows")
+
+
 # ----------------------------------------------------------------------------- K8
 MD_W_BF16, MD_W_INT8 = 0, 1
 EPI_NONE, EPI_SWIGLU, EPI_GEGLU = 0, 1, 3
