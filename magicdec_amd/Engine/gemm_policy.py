@@ -187,36 +187,31 @@ def _measured(M: int, N: int, K: int, kind: str, absorbs_norm: bool):
         if M <= 32 and N >= 14336 and not absorbs_norm and MIN_STREAM_BYTES <= nbytes <= SWIGLU_ONE_TILE_MAX_BYTES:
             return "fused"            # 24 576 x 4096: 38.4 -> 35.5 (one row), 41.0 -> 38.3 (32); with a norm to absorb skinny is faster
         # 65..128 rows, more than one round of block workgroups (296 or 432: the last round nearly empty): 37 888 x 3584
-        # 84.6 -> 81.0 on the skinny kernel, 55 296 x 5120 133 -> 122 (128 rows), 124 -> 115 (96)
+        # 84.6 -> 63.2 on the skinny kernel, 55 296 x 5120 133 -> 102 (128 rows), 124 -> 99 (96)
         if 64 < M <= 128 and N % 128 == 0 and tiles > 256:
             return "skinny"
     if kind in ("resid", "planes") and N <= 8192:
         if K >= 8192 and nbytes >= MIN_STREAM_BYTES:
-            # the deep projections.  The skinny kernel cuts K into slices that divide K / 128: with K = 14 336 = 128 * 112 its
-            # grid is full, with 18 944 = 128 * 148 or 27 648 = 128 * 216 it is not, and the block kernel (64-wide slices, any
-            # remainder) is level or ahead from 33 rows on: 3584 x 18 944 47.9 / 58.1 / 63.2 -> 37.5 / 38.5 / 41.0 at 64 / 96 / 128,
-            # 5120 x 27 648 72 / 79 / 85 -> 65 / 64 / 66; 4096 columns over 14 336 stay (32.2 / 36.2 / 37.8 against
-            # 34.0 / 36.5 / 39.1)
+            # the deep projections: 3584 x 18 944 at 1 / 32 rows 32.2 / 33.1 on the skinny kernel, 30.5 / 31.7 with the tile
+            # kernel's K split, 4096 x 14 336 28.2 -> 27.2.  (At 96 / 128 rows skinny, 40.7 / 42.9, and block, 38.5..47.5, are level.)
             if M <= 32 and kind == "resid" and nbytes <= SPLIT_ONE_TILE_MAX_BYTES:
-                return "split"        # 3584 x 18 944 37.1 / 43.7 -> 30.5 / 31.7 at 1 / 32 rows, 4096 x 14 336 28.2 -> 27.2
-            if 32 < M <= 128 and N % 128 == 0 and N % 4096:
-                return "block"
+                return "split"
         if FUSED_MAX_K < K < 8192:
             if kind == "planes":
-                # 2048 x 7680: 16.0 / 16.2 / 20.3 / 26.5 on the tile kernel's K split -> 13.2 / 13.6 / 15.9 / 19.2 (1 / 8 / 32 / 64)
-                return "skinny" if M <= 64 else "split" if M <= 128 else None
+                return "skinny"       # 2048 x 7680: 16.0 / 20.3 / 26.5 / 24.6 / 32.2 in the library -> 12.9 / 14.5 / 16.9 / 21.4 / 28.3
+                                      # (1 / 32 / 64 / 128 / 256 rows); the tile kernel's K split 14.8 / 17.1 / 24.2 / 22.8 / 35.0
             if K <= 5632 and M <= 128:
                 if M <= 32 and nbytes < 30e6:
-                    return "skinny"   # 2048 x 5632: 14.3 / 13.4 / 18.4 in the library -> 12.1 / 12.5 / 14.8 (1 / 8 / 32 rows)
+                    return "skinny"   # 2048 x 5632: 14.3 / 13.4 / 18.4 in the library -> 11.4 / 11.7 / 13.2 (1 / 8 / 32 rows)
                 if m_tiles * nbytes <= FUSED_MAX_L2_BYTES_DEEP_RESID:
                     return "fused"    # 2048 x 5632 21.1 / 19.4 -> 15.2 / 14.5 (64 / 128), 5120 x 5120 22.8 -> 16.5 (32)
-        # 3584..5632 deep and wide, more rows than the tile kernel's budget: the library, untuned, 23.8 / 26.5 / 33.8 ->
-        # 21.9 / 23.6 / 25.5 (3584 x 3584 at 96 / 128 / 192) and 26.1 / 36.6 / 54.8 -> 24.8 / 28.7 / 32.6 (5120 x 5120 at 64 / 128 /
-        # 256), 25.9 -> 22.7 (4096 x 4096 at 96)
+        # 3584..5632 deep and wide, more rows than the tile kernel's budget: the library, untuned, against the skinny kernel (up to 128
+        # rows) or the block kernel: 3584 x 3584 23.8 / 26.5 / 33.8 -> 22.4 / 23.3 / 25.5 (96 / 128 / 192), 5120 x 5120 26.1 / 36.6 /
+        # 54.8 -> 22.8 / 27.9 / 32.6 (64 / 128 / 256), 4096 x 4096 25.9 -> 21.9 (96)
         if (kind == "resid" and 3584 <= K <= 5632 and N >= 3584 and N % 128 == 0 and M > (32 if K > FUSED_MAX_K else 64)
                 and not (M > 128 and _WO256 != "0" and K <= FUSED_MAX_K and nbytes <= FUSED_M256_RESID_T22_MAX_BYTES
                          and (N // 64) * ((m_tiles + 1) // 2) >= 192) and not _tuned(M, N, K)):
-            return "block"
+            return "skinny" if M <= 128 else "block"
     if kind == "planes" and K <= FUSED_MAX_K and M > 128 and use_fused(M, N, K, "resid"):
         return "skinny"               # 4096 x 4096 on the tile kernel's K split 36.3 / 33.8 -> 27.5 / 28.8 (192 / 256 rows)
     if kind == "qkv" and not _tuned(M, N, K):

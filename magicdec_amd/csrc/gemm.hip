@@ -28,6 +28,8 @@
 // silu -> bf16, product -> bf16), weight-only int8 (Engine/quantize.py:72-86: bf16(acc) * bf16 scale -> bf16).
 #include "md_common.h"
 
+#include <algorithm>
+
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -97,7 +99,7 @@ __device__ __forceinline__ float silu_bf16(float h1) {
 }
 
 // One workgroup: NW wavefronts x 32 GEMM columns, rows [0, M), k in [blockIdx.y*kblk, +kblk).
-// NW (round 5): 4 by default; 6 or 7 where that makes the grid a whole number of workgroups per CU.  A CU ingests ~24 GB/s
+// NW: 4 by default; 5 to 7 where that loads the CUs more evenly (plan_of).  A CU ingests ~24 GB/s
 // of HBM whatever is resident on it (profiles/r04_ingest_probe.txt), so a launch ends when the most loaded CU does: the
 // 8B w1|w3 (896 wave tiles, two K slices) ran as 448 four-wave workgroups = 192 CUs with two and 64 with one (1 048 KB
 // against a mean of 918 KB); as 256 seven-wave workgroups every CU streams 917 KB.  Bits do not change: a wave's tile,
@@ -114,7 +116,7 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm_kernel(const GemmParams p
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];   // 2 x [MP][kPitch] (+ MP floats rstd when PRO)
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 31, kh = lane >> 5;
     const int k_beg = blockIdx.y * p.kblk;
-    const int nslab = p.kblk / kSlabK;
+    const int nslab = min(p.kblk, p.K - k_beg) / kSlabK;       // (the last K slice may be the shorter one)
 
     // ---- this lane's W row (GEMM column).  SwiGLU: the wave's 32 columns are 16 rows of w1 and the same 16 of w3.
     int col;            // GEMM column index in [0, N)
@@ -415,16 +417,37 @@ int pick_splits(int n_blocks, int K) {
     return best;
 }
 
-// (waves per workgroup, K slices) of a product with `ntiles` wave tiles (32 GEMM columns each; SwiGLU: 16 + 16).
-// Four waves and the split of pick_splits unless that leaves the most loaded CU with > 8 % more bytes than the mean AND
-// six or seven waves per workgroup with the SAME split (same partial planes, same bits) bring it within 2 %.
-struct SkinnyPlan { int nw, S; };
+// (waves per workgroup, K slices, their depth) of a product with `ntiles` wave tiles (32 GEMM columns each; SwiGLU: 16 + 16).  A launch
+// ends when the most loaded CU does; its load over the mean decides:
+//   * slices: the even split that gives every CU a workgroup (pick_splits), unless that is a few workgroups more than there are CUs,
+//     whatever their waves, and slices of whole slabs, the last one shorter and at least a quarter fewer, keep to one each: K = 18 944 =
+//     148 slabs over 28 column blocks is 37 x 28 = 1 036 workgroups (load 1.24) or 9 x 28 = 252 (1.05).  It depends on N and K only, as
+//     the workspace does.  3584 x 18 944 37.1 -> 32.2 us at one row, 47.9 -> 35.8 at 64, 63.2 -> 42.9 at 128; 2048 x 5632 14.8 -> 13.2
+//     at 32; 2048 x 7680 19.2 -> 16.9 at 64, 39.0 -> 28.3 at 256;
+//   * waves: four, unless that leaves the most loaded CU more than 8 % above the mean and five to seven are better by 8 % (the split and
+//     the bits stay): 432 workgroups of four (two on 176 CUs, one on 80: load 1.19) are 247 of seven (1.04), 296 are 237 of five
+//     (1.73 -> 1.08).  With six and seven only, and only where they came within 2 % of the mean:
+//     55 296 x 5120 SwiGLU 122 -> 104 us at 128 rows, 97 -> 91 at 64; 37 888 x 3584 SwiGLU 81 -> 64, 64 -> 51; 5120 x 27 648 85 -> 67,
+//     72 -> 60; 7168 x 5120 34 -> 29, 26 -> 23.
+struct SkinnyPlan { int nw, S, kblk; };
+double cu_load(int ntiles, int nslab, int nw, int S, int cus) {       // slabs of the most loaded CU over the mean (round-robin placement)
+    const long wgs = (long)((ntiles + nw - 1) / nw) * S, per_cu = (wgs + cus - 1) / cus;
+    return (double)per_cu * nw * ((nslab + S - 1) / S) * cus / ((double)ntiles * nslab);
+}
+
 SkinnyPlan plan_of(int ntiles, int K, bool allow_nw) {
+    const int nslab = K / kSlabK, n_blocks = (ntiles + 3) / 4;
     SkinnyPlan pl;
     pl.nw = 4;
-    pl.S = pick_splits((ntiles + 3) / 4, K);
+    pl.S = pick_splits(n_blocks, K);
+    const int most = std::min(std::max(g_target_blocks / n_blocks, 1), std::min(nslab, 64));
+    const int fewer = (nslab + (nslab + most - 1) / most - 1) / ((nslab + most - 1) / most);
+    double even = 1e30;
+    for (int nw : {4, 5, 6, 7}) even = std::min(even, cu_load(ntiles, nslab, nw, pl.S, g_target_blocks));
+    if (4 * fewer <= 3 * pl.S && cu_load(ntiles, nslab, 4, fewer, g_target_blocks) <= even) pl.S = fewer;
+    pl.kblk = (nslab + pl.S - 1) / pl.S * kSlabK;
     if (g_force_nw == 4 || !allow_nw) return pl;
-    // compute units of the current device, queried once per device (ADVICE r5: a partitioned or smaller part must not be
+    // compute units of the current device, queried once per device (a partitioned or smaller part must not be
     // planned as 256 CUs); unknown -> keep the four-wave shape (results are bit-identical either way)
     static int cus_of[16] = {0};
     int devid = 0;
@@ -436,21 +459,20 @@ SkinnyPlan plan_of(int ntiles, int K, bool allow_nw) {
     }
     const int kCUs = cus_of[devid];
     if (kCUs <= 0) return pl;
-    auto load = [&](int nw) {                       // bytes of the most loaded CU over the mean (round-robin placement)
-        const long wgs = (long)((ntiles + nw - 1) / nw) * pl.S;
-        const long per_cu = (wgs + kCUs - 1) / kCUs;
-        return (double)per_cu * nw * kCUs / ((double)ntiles * pl.S);
-    };
     if (g_force_nw == 6 || g_force_nw == 7) {
         pl.nw = g_force_nw;
         return pl;
     }
-    if (load(4) <= 1.08) return pl;
-    for (int nw : {7, 6})
-        if (load(nw) <= 1.02) {
+    double best = cu_load(ntiles, nslab, 4, pl.S, kCUs);
+    if (best <= 1.08) return pl;
+    best -= 0.08;
+    for (int nw : {7, 6, 5}) {
+        const double load = cu_load(ntiles, nslab, nw, pl.S, kCUs);
+        if (load < best) {
+            best = load;
             pl.nw = nw;
-            break;
         }
+    }
     return pl;
 }
 
@@ -507,12 +529,13 @@ int launch_rd(const GemmParams& p, int n_blocks, hipStream_t st) {
     return MD_OK;
 }
 
-// the 6- / 7-wave forms exist for bf16 weights at M <= 128 (nw_allowed below); everything else runs four waves
+// the 5- to 7-wave forms exist for bf16 weights at M <= 128 (nw_allowed below); everything else runs four waves
 template <int MT, int EPI, bool W8, bool PRO>
 int launch_nw(const GemmParams& p, int nw, int n_blocks, hipStream_t st) {
     if constexpr (!W8 && MT <= 4) {
         if (nw == 7) return launch<MT, EPI, W8, PRO, 7>(p, n_blocks, st);
         if (nw == 6) return launch<MT, EPI, W8, PRO, 6>(p, n_blocks, st);
+        if (nw == 5) return launch<MT, EPI, W8, PRO, 5>(p, n_blocks, st);
     }
     return launch<MT, EPI, W8, PRO, 4>(p, n_blocks, st);
 }
@@ -624,7 +647,7 @@ int linear_impl(const void* x, int64_t ldx, const void* w, int w_dtype, int w_pa
     const SkinnyPlan pl = plan_of(ntiles, K, nw_allowed(M, w8));
     const int n_blocks = (ntiles + pl.nw - 1) / pl.nw;
     p.S = pl.S;
-    p.kblk = K / p.S;
+    p.kblk = pl.kblk;
     p.partial = (float*)workspace;
     if (p.S > 1) {
         MD_CHECK_ARG(workspace && workspace_bytes >= (size_t)p.S * M * N * 4 && (((uintptr_t)workspace) & 15) == 0,
@@ -707,7 +730,7 @@ int md_internal_planes_skinny(const void* x, int64_t ldx, const void* w, int M, 
     const int ntiles = wave_tiles(N, EPI_NONE);
     const SkinnyPlan pl = plan_of(ntiles, K, nw_allowed(M, false));
     p.S = *S = pl.S;
-    p.kblk = K / p.S;
+    p.kblk = pl.kblk;
     p.partial = (float*)ws;
     MD_CHECK_ARG(ws && ws_bytes >= (size_t)p.S * M * N * 4 && ((uintptr_t)ws & 15) == 0, "md_linear_planes: workspace too small");
     return launch_mt<EPI_NONE, false>(p, pl.nw, (ntiles + pl.nw - 1) / pl.nw, st);
@@ -758,7 +781,7 @@ extern "C" int md_linear_add_rmsnorm(const void* x, int64_t ldx, const void* w, 
     const SkinnyPlan pl = plan_of(ntiles, K, nw_allowed(M, w8));
     const int n_blocks = (ntiles + pl.nw - 1) / pl.nw;
     p.S = pl.S;
-    p.kblk = K / p.S;
+    p.kblk = pl.kblk;
     p.partial = (float*)workspace;
     MD_CHECK_ARG(workspace && workspace_bytes >= (size_t)p.S * M * N * 4 && (((uintptr_t)workspace) & 15) == 0,
                  "md_linear_add_rmsnorm: workspace too small (need %zu bytes) or not 16-byte aligned",
