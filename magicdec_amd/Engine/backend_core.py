@@ -27,8 +27,8 @@ CHUNK = 128        # Engine/SnapKV/backend.py:236
 PREFILL_ROWS = 16384   # rows of one prefill step where the portion is free to choose (models addressed by position, `step`)
 # ... and of a prompt's portion in the fixed-batch engines.  What a 16-bit product reaches on an 8B layer at 128 rows: 450 TFLOP/s (the
 # weight stream), at 512: 590..1240, at 4096 and more about 1300.  Two layers, us, against portions of 128 tokens a request: one request
-# of 8 000 tokens 34 485 -> 7 765 at 4096 rows, 7 661 at 8192; four of 1 500 (7B) 12 664 -> 7 040, 5 927; four of 2 081 12 200 -> 6 641,
-# 6 496; one of 600 2 969 -> 1 572.  8192 is what 64 requests had already; a layer's activations take 1.4 GB there on a 32B model.
+# of 8 000 tokens 34 485 -> 6 955 (7 765 at 4096 rows), four of 1 500 (7B) 12 664 -> 6 157, four of 2 081 12 200 -> 6 540, one of 600
+# 2 969 -> 1 170.  8192 is what 64 requests had already; a layer's activations take 1.4 GB there on a 32B model.
 PROMPT_ROWS = 8192
 PROMPT_WINDOWS = 512 << 20     # bytes of one pass's StreamingLLM windows: 64 portions at a budget of 1024 rows of 8 heads of 128
 
@@ -212,33 +212,35 @@ class _BackendBase:
 
     def _portions(self, seq_len):
         """The portions [(first token, tokens)] of a prompt whose keys all stay in the cache: any division gives every token the same
-        keys, so portions are as long as the matrix products want them.  Two stay as they are: the last CHUNK's tokens (their logits and
-        tokens are what encode returns, and the SnapKV select's window) and, for an fp8 cache, the first CHUNK, which sets its scales."""
+        keys, so portions are as long as the matrix products want them.  An fp8 cache's first CHUNK, which sets its scales, stays one."""
         if self.mapped or torch.device(self.device).type == "cpu":       # (the CPU's products round by their row counts)
             chunk = self.prefill_chunk
             return [(a, min(chunk, seq_len - a)) for a in range(0, seq_len, chunk)]
-        chunks = max(0, seq_len - 1) // CHUNK                    # ahead of the last one
-        out, at = [], 0
-        if chunks and self.model.layers[0].attention.kv_cache.scales("kv_cache") is not None:
+        chunks, at = -(-seq_len // CHUNK), 0
+        out = []
+        if chunks > 1 and self.model.layers[0].attention.kv_cache.scales("kv_cache") is not None:
             out, at, chunks = [(0, CHUNK)], CHUNK, chunks - 1
-        if chunks:
-            most = max(1, PROMPT_ROWS // (self.batch_size * CHUNK))
-            parts = -(-chunks // most)
-            for i in range(parts):
-                n = (chunks * (i + 1) // parts - chunks * i // parts) * CHUNK
-                out.append((at, n))
-                at += n
-        return out + [(at, seq_len - at)] if seq_len > at else out
+        # the last chunk rides along unless that takes a portion more: 8192 rows are whole rounds of the library's tiles, 8324 are not
+        first, most = at, max(1, PROMPT_ROWS // (self.batch_size * CHUNK))
+        parts = max(min(1, chunks), -(-(chunks - 1) // most))
+        if chunks > parts * most:
+            chunks -= 1
+        for i in range(parts):
+            end = min(first + chunks * (i + 1) // parts * CHUNK, seq_len)
+            out.append((at, end - at))
+            at = end
+        return out + [(at, seq_len - at)] if at < seq_len else out
 
     def _map_portion(self, end):
         """Pages for a prompt's first `end` tokens."""
         self._t.map_pages(-(-end // PAGE_SIZE), (end - 1) % PAGE_SIZE + 1)
 
-    def _last_rows(self, n):
-        """Extra prefill arguments of models addressed by position: logits for the last of every request's n rows only (their
-        portions are long; encode then returns [B, 1])."""
+    def _last_rows(self, n, seq_len):
+        """Extra prefill arguments: of models addressed by position, logits for the last of every request's n rows only (their portions
+        are long; encode then returns [B, 1]); otherwise for those of the prompt's last CHUNK, as when it ran by itself."""
         if not self.mapped:
-            return {}
+            tail = (seq_len - 1) % CHUNK + 1
+            return dict(tail=tail) if n > tail else {}
         return dict(head_rows=torch.arange(1, self.batch_size + 1, device=self.device) * n - 1)
 
     def _prefill_begin(self):
@@ -359,7 +361,7 @@ class SnapKVTargetBackend(_BackendBase):
             self.model.skip_head = done + n != seq_len
             tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table((n, done + n)), is_last=is_last,
                                         draft_tab=self._d.table() if (self.is_spec and is_last) else None,
-                                        ctx_len=done + n, **self._last_rows(n))
+                                        ctx_len=done + n, **self._last_rows(n, seq_len))
             self.cachelens += n
         self.model.skip_head = False
         if self.mapped:
@@ -543,7 +545,7 @@ class SnapKVDraftBackend(_BackendBase):
             self.model.skip_head = done + n != seq_len
             tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table((n, done + n)), is_last=is_last,
                                         draft_tab=self._d.table() if (self.is_compress and is_last) else None,
-                                        ctx_len=done + n, **self._last_rows(n))
+                                        ctx_len=done + n, **self._last_rows(n, seq_len))
             self.cachelens += n
         self.model.skip_head = False
         if self.mapped:
@@ -723,7 +725,7 @@ class StreamingSelfSpecBackend(_BackendBase, _StreamingMixin):
             ids = input_ids[:, done:done + n]
             self._map_portion(done + n)
             self.model.skip_head = done + n != seq_len
-            tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table())
+            tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table(), **self._last_rows(n, seq_len))
             self.cachelens += n
         self.model.skip_head = False
         self._prefill_end()

@@ -781,6 +781,8 @@ class Transformer(nn.Module):
                                         kv_scales=scales, kv_layout=layout)
             o = self._attend(q_rot, cache, qo_indptr, tab, n, scales, layout)
             if snap_tab is not None:
+                if head_rows is not None:                 # the observation window is the prompt's last chunk
+                    q_rot = q_rot.index_select(0, head_rows)
                 ops.snapkv_select(q_rot, cache, tab.indices, tab.indptr, self._snap_ctx_len, self.window_size,
                                   self.draft_budget, POOL_KERNEL, kvc.draft_cache, snap_tab.indices, snap_tab.indptr,
                                   snap_tab.last_page_len, self.workspace, kv_scales=scales, kv_layout=layout)
@@ -798,17 +800,23 @@ class Transformer(nn.Module):
         return self._std_step(idx, input_pos, kv_append_indptr, draft_tab, which="draft_cache")
 
     def prefill(self, idx, input_pos, kv_append_indptr, tab: PageTable, is_last=False, draft_tab: PageTable = None,
-                ctx_len=None):
+                ctx_len=None, tail=None):
         """Chunked prefill; on the last chunk of a SnapKV engine also runs the select (model.py:371-387).
-        ctx_len = offsets[0]+seqlen is passed by the back-end (host-known, no device read)."""
+        ctx_len = offsets[0]+seqlen is passed by the back-end (host-known, no device read).  tail: the last rows of every request that
+        are the prompt's last chunk (the select's window; tokens and logits are theirs), None: all."""
         snap = draft_tab if (is_last and self.spec and not self.streaming and draft_tab is not None) else None
-        if snap is not None and idx.shape[1] != self.window_size:
+        B, n = idx.shape
+        if snap is not None and (tail or n) != self.window_size:
             # the reference takes the whole last chunk as the observation window (Engine/SnapKV/model.py:389-395),
             # which is `window_size` rows only under its CLI assert (prefix_len - window_size) % 128 == 0
             raise ValueError(f"SnapKV select needs the last prefill chunk to be exactly window_size="
-                             f"{self.window_size} tokens, got {idx.shape[1]} ((prefix_len - window_size) % 128 != 0)")
+                             f"{self.window_size} tokens, got {tail or n} ((prefix_len - window_size) % 128 != 0)")
         self._snap_ctx_len = ctx_len
-        return self._std_step(idx, input_pos, kv_append_indptr, tab, snap_tab=snap, calibrate=True)
+        rows = None
+        if tail is not None and not self.skip_head:
+            rows = (torch.arange(B, device=idx.device).view(B, 1) * n + torch.arange(n - tail, n, device=idx.device)).flatten()
+        out = self._std_step(idx, input_pos, kv_append_indptr, tab, snap_tab=snap, calibrate=True, n_max=n, head_rows=rows)
+        return out if out is None or tail is None else out.view(B, tail)
 
     def stream_prefill(self, idx, ctx, kv_append_indptr, tab: PageTable, is_last, which, B):
         """StreamingLLM draft prefill of one chunk (Attention.prefill + KVCache.prefill,

@@ -40,20 +40,25 @@ def test_longer_portions(which, kv, batch, prompt, monkeypatch):
         monkeypatch.setattr(core, "PROMPT_ROWS", rows)
         e = engine(which, kv, batch, 2048)
         parts = e._portions(prompt)
-        # in order and whole, each at a page's start, the last CHUNK's tokens by themselves
+        # in order and whole, each at a page's start
         assert [a for a, _ in parts] == [0] + [a + n for a, n in parts[:-1]] and sum(parts[-1]) == prompt
-        assert all(a % 128 == 0 for a, _ in parts) and parts[-1][1] == (prompt - 1) % 128 + 1
-        assert all(n == 128 for _, n in parts[:-1]) if rows == 0 else all(n * batch <= max(rows, 128 * batch) for _, n in parts)
+        assert all(a % 128 == 0 for a, _ in parts) and all(n * batch <= max(rows, 128 * batch) for _, n in parts)
+        assert rows == 0 or kv != "fp8" or parts[0][1] <= 128
         for _ in range(2):                                           # (a second prompt over the first one's state)
             tokens = e.encode(ids)
         kvs = [b.attention.kv_cache for b in e.model.layers]
         seen.append(dict(tokens=tokens, logits=e.model._last_logits.float(), lens=e.cachelens, pages=e._t.table(),
-                         scales=[s for c in kvs for s in (c.scales() or ())], rows=[c.kv_cache.float() for c in kvs]))
+                         scales=[s for c in kvs for s in (c.scales() or ())],
+                         kept=[c.draft_cache.float() for c in kvs] if which in ("spec", "draft") else [], rows=[c.kv_cache.float() for c in kvs]))
     a, b = seen
-    assert a["tokens"].shape == b["tokens"].shape == (batch, parts[-1][1])
+    assert a["tokens"].shape == b["tokens"].shape == (batch, (prompt - 1) % 128 + 1)
     assert torch.equal(a["lens"], b["lens"]) and a["pages"].max_pages == b["pages"].max_pages
     assert all(torch.equal(getattr(a["pages"], k), getattr(b["pages"], k)) for k in ("indices", "indptr", "last_page_len"))
     assert all(torch.equal(x, y) for x, y in zip(a["scales"], b["scales"]))
     # each within 0.8 % of exact arithmetic; an fp8 row rounds to 2^-4 of itself, so a moved rounding shows as far as that in few places
     for x, y in zip([a["logits"]] + a["rows"], [b["logits"]] + b["rows"]):
         assert (x - y).norm() <= (0.016 if kv == "bf16" else 0.03) * y.norm()
+    # the select over the same window: but for scores on the edge, the same rows
+    for x, y in zip(a["kept"], b["kept"]):
+        near = (x - y).norm(dim=-1) <= 0.05 * y.norm(dim=-1)
+        assert near.double().mean() > 0.8
