@@ -184,6 +184,10 @@ def _measured(M: int, N: int, K: int, kind: str, absorbs_norm: bool):
         if M <= (32 if tiles <= 256 and K <= FUSED_MAX_K else 16) and N >= 14336 and nbytes >= MIN_STREAM_BYTES:
             return "fused"
     if kind == "swiglu":
+        # up to four rows the tile kernel stages four, also with a norm to absorb: 28 672 x 4096 43.9 -> 42.2, 37 888 x 3584 52.0 ->
+        # 47.4, 55 296 x 5120 92.6 -> 88.0; at 16 rows 44.9 / 51.7 / 92.0 on the skinny kernel against 44.7 / 52.4 / 95.6
+        if M <= 4 and N >= 14336 and nbytes >= MIN_STREAM_BYTES:
+            return "fused"
         if M <= 32 and N >= 14336 and not absorbs_norm and MIN_STREAM_BYTES <= nbytes <= SWIGLU_ONE_TILE_MAX_BYTES:
             return "fused"            # 24 576 x 4096: 38.4 -> 35.5 (one row), 41.0 -> 38.3 (32); with a norm to absorb skinny is faster
         # 65..128 rows, more than one round of block workgroups (296 or 432: the last round nearly empty): 37 888 x 3584

@@ -181,9 +181,12 @@ __device__ __forceinline__ int64_t kv_elem_offset(const KvTable& t, int b, int r
 // workgroup per CU) halves both.  Each K-slice wave then owns 2 x 2 accumulators, two W fragment streams and a 64-row
 // activation image; the summation order over the K slices (wave order) and every epilogue are unchanged, so the bits
 // are those of the 1 x 1 form.
-template <int EPI, bool FP8, int NW, bool WNT, bool PRO, int MT, int NT>
+// AI = staging instructions of 32 rows, four rows each: 8, or what M <= 4 / 16 rows need (one M tile).  The rows a smaller AI leaves
+// out are rows >= M: their image, and with it their accumulators, hold anything, and are never stored.
+template <int EPI, bool FP8, int NW, bool WNT, bool PRO, int MT, int NT, int AI>
 __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel(const TileParams p) {
     constexpr int kNW = NW;
+    static_assert(AI == 8 || MT == 1, "fewer rows than a tile: one M tile");
     // Round 6, the deferred-norm prologue on 2 x 2 tiles (the 1B w1|w3 at 64 rows).  Phase timestamps of the 1 x 1 form
     // (tools/tile_timing.py, profiles/r06_tile_phase_timing.txt) show where its 6 us go: ~1 us of prologue in front of the
     // first load, +2.4 us per activation chunk between "landed" and "staged" (four wavefronts per SIMD normalising at
@@ -235,16 +238,16 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
     // activation staging: instruction i covers rows 4i + (lane >> 4), 16 lanes read one 256-B row segment
     const int ar = lane >> 4, c16 = lane & 15;
     const unsigned char* xbase = reinterpret_cast<const unsigned char*>(p.x + ks0 * 16);   // wave-uniform
-    unsigned int xrow[8];                            // byte offsets of the lane's rows (M * ldx * 2 < 2^32); MT == 1
+    unsigned int xrow[AI];                           // byte offsets of the lane's rows (M * ldx * 2 < 2^32); MT == 1
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < AI; ++i) {
         const int r = m0 + 4 * i + ar;
         xrow[i] = (unsigned int)(r < p.M ? r : p.M - 1) * (unsigned int)p.ldx * 2u;   // rows >= M re-read row M-1
     }
     const int nchunk = (ksteps_w + 7) >> 3;
-    u32x4 xa[8 * MT];
+    u32x4 xa[AI * MT];
     u32x4 nwv = {0u, 0u, 0u, 0u};                   // PRO: the norm weights of this lane's 8 columns of the chunk
-    float rs8[8];                                   // PRO, MT == 1: rstd of this lane's staging rows (MT > 1: re-read
+    float rs8[AI];                                  // PRO, MT == 1: rstd of this lane's staging rows (MT > 1: re-read
                                                     // from LDS per chunk -- 16 more registers would spill)
     // (the row scales are formed BEFORE the first loads are issued: with the loads in flight first, the barrier below
     // drains them -- 1B w1|w3 at 64 rows 29.2 us against 25.8, profiles/r04_fused_pro_prologue_ab.txt.  What the
@@ -285,7 +288,7 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
         __syncthreads();
         if constexpr (MT == 1) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) rs8[i] = rstd_lds[4 * i + ar];
+            for (int i = 0; i < AI; ++i) rs8[i] = rstd_lds[4 * i + ar];
         }
     }
     auto a_load = [&](int c) {
@@ -295,7 +298,7 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
         if constexpr (kNewPro)        // the chunk's norm weights FIRST: a_store unpacks them before it touches a row
             nwv = *reinterpret_cast<const u32x4*>(reinterpret_cast<const unsigned char*>(p.pro_w + ks0 * 16) + cc);
 #pragma unroll
-        for (int i = 0; i < 8 * MT; ++i) {
+        for (int i = 0; i < AI * MT; ++i) {
             unsigned int ro;
             if constexpr (MT == 1) {
                 ro = xrow[i];
@@ -315,7 +318,7 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
             for (int w = 0; w < 4; ++w) nwf[w] = unpack2(nwv[w]);
         }
 #pragma unroll
-        for (int i = 0; i < 8 * MT; ++i) {
+        for (int i = 0; i < AI * MT; ++i) {
             u32x4 v = xa[i];
             if constexpr (kNewPro) {
                 // rows 0..31 of the tile from the 16 instructions i = 0..15?  no: instruction i covers rows 4 i + ar of
@@ -569,10 +572,10 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
 #endif
 }
 
-template <int EPI, bool FP8, int NW, bool WNT, bool PRO, int MT = 1, int NT = 1>
+template <int EPI, bool FP8, int NW, bool WNT, bool PRO, int MT = 1, int NT = 1, int AI = 8>
 int launch_tile_cfg(const TileParams& p, hipStream_t st) {
     constexpr int lds = NW * MT * kWaveLds + (PRO ? 128 * MT : 0);
-    auto k = tile_gemm_kernel<EPI, FP8, NW, WNT, PRO, MT, NT>;
+    auto k = tile_gemm_kernel<EPI, FP8, NW, WNT, PRO, MT, NT, AI>;
     static MdPerDeviceOnce once;
     if (once.first()) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds) !=
@@ -619,6 +622,13 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
     if (g_force_nw == 8) nw16 = false;
     if (g_force_nw == 16) nw16 = p.K % 256 == 0;
     const bool wnt = p.m_tiles == 1;
+    // few rows: the 32-row form requests (M - 1 again and again) as many bytes of x as of W, and those loads stand in W's way.  At one row
+    // 4096 x 4096 + residual 11.1 -> 9.5 us, 768 x 3072 9.0 -> 7.4, 6144 x 4096 + rope 12.8 -> 11.3, 2048 x 2048 6.0 -> 5.4; with
+    // four staging instructions at 8 rows 10.6 -> 9.7, 9.2 -> 8.3, 6.1 -> 5.8
+    if (wnt && p.M <= 4)
+        return nw16 ? launch_tile_cfg<EPI, FP8, 16, true, PRO, 1, 1, 1>(p, st) : launch_tile_cfg<EPI, FP8, 8, true, PRO, 1, 1, 1>(p, st);
+    if (wnt && p.M <= 16)
+        return nw16 ? launch_tile_cfg<EPI, FP8, 16, true, PRO, 1, 1, 4>(p, st) : launch_tile_cfg<EPI, FP8, 8, true, PRO, 1, 1, 4>(p, st);
     if (nw16)
         return wnt ? launch_tile_cfg<EPI, FP8, 16, true, PRO>(p, st) : launch_tile_cfg<EPI, FP8, 16, false, PRO>(p, st);
     return wnt ? launch_tile_cfg<EPI, FP8, 8, true, PRO>(p, st) : launch_tile_cfg<EPI, FP8, 8, false, PRO>(p, st);
@@ -664,10 +674,10 @@ SplitPlan split_plan(int M, int N, int K) {
     return pl;
 }
 
-template <int MT, int NT>
+template <int MT, int NT, int AI = 8>
 int launch_split_cfg(const TileParams& p, hipStream_t st) {
     constexpr int lds = 8 * MT * kWaveLds;
-    auto k = tile_gemm_kernel<FL_PARTIAL, false, 8, true, false, MT, NT>;
+    auto k = tile_gemm_kernel<FL_PARTIAL, false, 8, true, false, MT, NT, AI>;
     static MdPerDeviceOnce once;
     if (once.first()) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds) !=
@@ -684,6 +694,8 @@ int launch_split_cfg(const TileParams& p, hipStream_t st) {
 
 int launch_split(const TileParams& p, const SplitPlan& pl, hipStream_t st) {
     if (pl.mt == 2) return pl.nt == 2 ? launch_split_cfg<2, 2>(p, st) : launch_split_cfg<2, 1>(p, st);
+    if (p.M <= 4) return pl.nt == 2 ? launch_split_cfg<1, 2, 1>(p, st) : launch_split_cfg<1, 1, 1>(p, st);
+    if (p.M <= 16) return pl.nt == 2 ? launch_split_cfg<1, 2, 4>(p, st) : launch_split_cfg<1, 1, 4>(p, st);
     return pl.nt == 2 ? launch_split_cfg<1, 2>(p, st) : launch_split_cfg<1, 1>(p, st);
 }
 
