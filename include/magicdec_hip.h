@@ -212,6 +212,10 @@ int md_streaming_windows(const void* k_new, const void* v_new, int64_t k_row_str
                          void* windows, void* next, int B, int tokens, int portion, int ctx, int kv_len, int sink, int pages_per_req,
                          int KH, int D, int page_size, int rotate_next, const float* cos_sin, int max_pos, md_stream_t stream);
 
+/* h_out = rows ids[] of the bf16 table [table_rows][dim], y = rmsnorm(h_out) * weight (md_rmsnorm's); an id outside the table: NaN. */
+int md_embed_rmsnorm(const void* table, int64_t table_rows, const int64_t* ids, const void* weight, void* h_out, void* y, int rows, int dim,
+                     float eps, md_stream_t stream);
+
 /* ------------------------------------------------------------------------
  * K9  RMSNorm / SiLU*mul / residual   reference: Engine/SnapKV/model.py:451-469
  * rmsnorm: y = bf16( x_f32 * rsqrt(mean(x^2)+eps) ) * w   (weight multiply in

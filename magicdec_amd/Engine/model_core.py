@@ -700,9 +700,12 @@ class Transformer(nn.Module):
         logits and tokens are wanted."""
         assert self._ready, "call setup_caches first"
         n = idx.shape[1] if idx.dim() == 2 else n_max
-        x = self.tok_embeddings(idx).view(idx.numel(), -1)
-        layers = self.layers
-        y = ops.rmsnorm(x, layers[0].attention_norm.weight, layers[0].attention_norm.eps)
+        layers, emb, norm = self.layers, self.tok_embeddings, self.layers[0].attention_norm
+        if type(emb) is nn.Embedding and emb.max_norm is None and idx.is_cuda and ops.embed_rmsnorm_supported(idx, emb.weight, norm.weight):
+            x, y = ops.embed_rmsnorm(idx, emb.weight, norm.weight, norm.eps)
+        else:
+            x = emb(idx).view(idx.numel(), -1)
+            y = ops.rmsnorm(x, norm.weight, norm.eps)
         for i, layer in enumerate(layers):
             o = attn_fn(i, layer, y, n)
             x, y = self._proj_add_norm(o.view(o.shape[0], -1), layer.attention.wo, x, layer.ffn_norm,

@@ -118,6 +118,7 @@ _SIGNATURES = {
     "md_linear_fused_split": (c_int, [P, L, P, P, P, L, I, I, I, P, c_size_t, P]),
     "md_linear_fused_split_add_rmsnorm": (c_int, [P, L, P, P, P, L, P, c_float, P, P, I, I, I, P, c_size_t, P]),
     "md_rmsnorm": (c_int, [P, P, P, I, I, c_float, P]),
+    "md_embed_rmsnorm": (c_int, [P, L, P, P, P, P, I, I, c_float, P]),
     "md_add_rmsnorm": (c_int, [P, P, P, P, P, I, I, c_float, P]),
     "md_silu_mul": (c_int, [P, P, L, L, P, I, I, P]),
     "md_embed_pos": (c_int, [P, P, P, I, P, P, I, I, I, I, I, c_float, P, P]),

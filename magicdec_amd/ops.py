@@ -731,6 +731,27 @@ def rmsnorm(x, weight, eps):
     return y.view(x.shape)
 
 
+def embed_rmsnorm_supported(ids, table, weight):
+    """True when embed_rmsnorm takes these tensors."""
+    return (ids.is_cuda and ids.dtype == torch.int64 and ids.numel() > 0 and ids.device == table.device == weight.device
+            and table.dtype == weight.dtype == torch.bfloat16 and table.dim() == 2 and table.is_contiguous() and weight.is_contiguous()
+            and weight.shape == table.shape[1:] and table.shape[1] % 8 == 0 and table.shape[1] <= 8192
+            and table.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+
+def embed_rmsnorm(ids, table, weight, eps):
+    """(table[ids], rmsnorm of it) as rows [ids.numel(), dim]."""
+    if not embed_rmsnorm_supported(ids, table, weight):
+        raise ValueError("embed_rmsnorm: int64 ids and a contiguous bf16 table [rows, dim <= 8192] on one GPU expected")
+    flat = ids.reshape(-1)
+    flat = flat if flat.is_contiguous() else flat.contiguous()
+    h = torch.empty(flat.numel(), table.shape[1], dtype=table.dtype, device=table.device)
+    y = torch.empty_like(h)
+    check(_lib.load().md_embed_rmsnorm(_p(table), table.shape[0], _p(flat), _p(weight), _p(h), _p(y), h.shape[0], h.shape[1], float(eps),
+                                       _stream()), "md_embed_rmsnorm")
+    return h, y
+
+
 def add_rmsnorm(x, r, weight, eps):
     """h = x + r ; y = rmsnorm(h).  Returns (h, y)."""
     _gpu(x, r, weight)
