@@ -19,6 +19,8 @@
 #include "latent.h"
 #include "xattn.h"
 
+#include <algorithm>
+
 unsigned int* md_page_overflow_counter_device();   // kvops.hip
 
 namespace {
@@ -298,7 +300,12 @@ int kv_splits(const md_latent_args* a) {
     const long tiles = ((long)a->max_pages * a->page_size + 31) / 32, groups = (long)a->B * row_groups(a);
     const long target = kTargetWgs / row_tiles(a);
     long want = (target + groups - 1) / groups;
-    const long cap = tiles / 8 > 1 ? tiles / 8 : 1;                  // >= 256 keys per workgroup
+    // >= 256 keys per workgroup; a tile is a chain of two barriers, 2 us where nothing else runs on the CU, so while one workgroup per CU
+    // is not reached 128 keys, and 64 up to one on every other.  Four layers, us: one request of 8 000 keys 316 -> 300, four of 1 000
+    // 319 -> 295, twelve of 1 500 333 -> 319 (64 keys: 325); beyond, shorter chains lose to the merge: 32 of 2 049 at 128 keys 391 against
+    // 380, 48 of 1 200 430 against 415
+    const long few = std::max(std::min(tiles / 4, target / 2 / groups), std::min(tiles / 2, target / 4 / groups));
+    const long cap = std::max(std::max(tiles / 8, few), 1L);
     if (want > cap) want = cap;
     return (int)(want < 1 ? 1 : want > 64 ? 64 : want);            // (the merge holds a split per lane)
 }
