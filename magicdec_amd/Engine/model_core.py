@@ -701,7 +701,8 @@ class Transformer(nn.Module):
         assert self._ready, "call setup_caches first"
         n = idx.shape[1] if idx.dim() == 2 else n_max
         layers, emb, norm = self.layers, self.tok_embeddings, self.layers[0].attention_norm
-        if type(emb) is nn.Embedding and emb.max_norm is None and idx.is_cuda and ops.embed_rmsnorm_supported(idx, emb.weight, norm.weight):
+        plain = type(emb) is nn.Embedding and emb.max_norm is None and not emb._forward_hooks and not emb._forward_pre_hooks
+        if plain and idx.is_cuda and ops.embed_rmsnorm_supported(idx, emb.weight, norm.weight):
             x, y = ops.embed_rmsnorm(idx, emb.weight, norm.weight, norm.eps)
         else:
             x = emb(idx).view(idx.numel(), -1)

@@ -81,75 +81,91 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const bf16_t* __restrict__
 // the thread -> column mapping, the order of every sum and every rounding point are those of skinny_reduce_kernel
 // (csrc/gemm.hip) followed by rmsnorm_kernel<true> above, so (h, y) are bit-identical to md_linear -> md_add_rmsnorm.
 //   o = bf16(sum_s partial[s] + bias)   [int8 weights: bf16(bf16(sum) * scale)];  h = bf16(x + o);  y = rmsnorm(h) * w
-template <bool W8>
-__global__ __launch_bounds__(256) void reduce_add_rmsnorm_kernel(const float* __restrict__ partial, int S, int M, int N,
-                                                                 const bf16_t* __restrict__ bias,
-                                                                 const bf16_t* __restrict__ scales,
-                                                                 const bf16_t* __restrict__ x, int64_t ldx,
-                                                                 const bf16_t* __restrict__ w, bf16_t* h_out,
-                                                                 bf16_t* y, float eps) {
-    __shared__ float red[8];
+// G groups of 256 threads, a vector of eight columns each: one group holding two to four vectors made that many round trips to the slices,
+// one after the other, and asked for the norm's weights behind the sum.  The sum of squares stays the first group's, over vectors
+// t, t + 256, ... in that order.  128 rows of 5120 columns, eight slices: 10.4 -> 8.1 us; steps 429.5 -> 422.4 (32B), 317 -> 311 (1B draft), 300 -> 295 (8B)
+template <bool W8, int G>
+__global__ __launch_bounds__(256 * G) void reduce_add_rmsnorm_kernel(const float* __restrict__ partial, int S, int M, int N,
+                                                                     const bf16_t* __restrict__ bias,
+                                                                     const bf16_t* __restrict__ scales,
+                                                                     const bf16_t* __restrict__ x, int64_t ldx,
+                                                                     const bf16_t* __restrict__ w, bf16_t* h_out,
+                                                                     bf16_t* y, float eps) {
+    __shared__ float red[4 * G];
+    __shared__ bf16x8 hs[G > 1 ? 256 * G : 1];
     const int64_t row = blockIdx.x;
-    const int nvec = N / 8;
+    const int nvec = N / 8, i = threadIdx.x;
     const int64_t plane = (int64_t)M * N;
-    constexpr int MAXV = 4;
-    f32x8 vals[MAXV];
+    f32x8 val = f32x8(0.f);
+    bf16x8 wv = {};
     float ss = 0.f;
+    if (i < nvec) {
+        const bf16x8 xv = reinterpret_cast<const bf16x8*>(x + row * ldx)[i];
+        wv = reinterpret_cast<const bf16x8*>(w)[i];
+        f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
+        // eight slices per trip, requested together and added in slice order: a load + add per loop trip was one
+        // memory round trip per slice (8.3 us for 32 rows x 8 slices; skinny_reduce_kernel does the same)
+        for (int s0 = 0; s0 < S; s0 += 8) {
+            f32x4 v0[8], v1[8];
 #pragma unroll
-    for (int it = 0; it < MAXV; ++it) {
-        const int i = threadIdx.x + it * 256;
-        if (i < nvec) {
-            f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = {0.f, 0.f, 0.f, 0.f};
-            // eight slices per trip, requested together and added in slice order: a load + add per loop trip was one
-            // memory round trip per slice (8.3 us for 32 rows x 8 slices; skinny_reduce_kernel does the same)
-            for (int s0 = 0; s0 < S; s0 += 8) {
-                f32x4 v0[8], v1[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    if (s0 + u < S) {                               // uniform: no load for a slice that does not exist
-                        const float* pp = partial + (s0 + u) * plane + row * N + i * 8;
-                        v0[u] = *reinterpret_cast<const f32x4*>(pp);
-                        v1[u] = *reinterpret_cast<const f32x4*>(pp + 4);
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    if (s0 + u < S) {                               // uniform
-                        a0 += v0[u];
-                        a1 += v1[u];
-                    }
+            for (int u = 0; u < 8; ++u) {
+                if (s0 + u < S) {                               // uniform: no load for a slice that does not exist
+                    const float* pp = partial + (s0 + u) * plane + row * N + i * 8;
+                    v0[u] = *reinterpret_cast<const f32x4*>(pp);
+                    v1[u] = *reinterpret_cast<const f32x4*>(pp + 4);
                 }
             }
-            f32x8 o;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                float v = e < 4 ? a0[e] : a1[e - 4];
-                if (bias) v += bf16_to_f32(bias[i * 8 + e]);
-                if (W8) v = bf16_to_f32(f32_to_bf16(v)) * bf16_to_f32(scales[i * 8 + e]);
-                o[e] = bf16_to_f32(f32_to_bf16(v));
+            for (int u = 0; u < 8; ++u) {
+                if (s0 + u < S) {                               // uniform
+                    a0 += v0[u];
+                    a1 += v1[u];
+                }
             }
-            const f32x8 xf = __builtin_convertvector(reinterpret_cast<const bf16x8*>(x + row * ldx)[i], f32x8);
-            const bf16x8 hb = __builtin_convertvector(xf + o, bf16x8);      // bf16 add
-            reinterpret_cast<bf16x8*>(h_out + row * N)[i] = hb;
-            const f32x8 f = __builtin_convertvector(hb, f32x8);
-            vals[it] = f;
+        }
+        f32x8 o;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
+        for (int e = 0; e < 8; ++e) {
+            float v = e < 4 ? a0[e] : a1[e - 4];
+            if (bias) v += bf16_to_f32(bias[i * 8 + e]);
+            if (W8) v = bf16_to_f32(f32_to_bf16(v)) * bf16_to_f32(scales[i * 8 + e]);
+            o[e] = bf16_to_f32(f32_to_bf16(v));
+        }
+        const bf16x8 hb = __builtin_convertvector(__builtin_convertvector(xv, f32x8) + o, bf16x8);      // bf16 add
+        reinterpret_cast<bf16x8*>(h_out + row * N)[i] = hb;
+        val = __builtin_convertvector(hb, f32x8);
+        if constexpr (G > 1) hs[i] = hb;
+        if constexpr (G == 1) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += val[e] * val[e];
         }
     }
-    const float tot = block_reduce_sum(ss, red);
+    if constexpr (G > 1) {
+        __syncthreads();
+        if (i < 256) {
+#pragma unroll
+            for (int it = 0; it < G; ++it)
+                if (i + it * 256 < nvec) {
+                    const f32x8 f = __builtin_convertvector(hs[i + it * 256], f32x8);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) ss += f[e] * f[e];
+                }
+        }
+    }
+    const float tot = block_reduce_sum(ss, red);                // (the other groups' waves add 0)
     const float rs = rsqrtf(tot / (float)N + eps);
-    const bf16x8* wv = reinterpret_cast<const bf16x8*>(w);
-#pragma unroll
-    for (int it = 0; it < MAXV; ++it) {
-        const int i = threadIdx.x + it * 256;
-        if (i < nvec) {
-            const bf16x8 nb = __builtin_convertvector(vals[it] * rs, bf16x8);
-            const f32x8 nf = __builtin_convertvector(nb, f32x8);
-            const f32x8 wf = __builtin_convertvector(wv[i], f32x8);
-            reinterpret_cast<bf16x8*>(y + row * N)[i] = __builtin_convertvector(nf * wf, bf16x8);
-        }
+    if (i < nvec) {
+        const bf16x8 nb = __builtin_convertvector(val * rs, bf16x8);
+        const f32x8 nf = __builtin_convertvector(nb, f32x8);
+        reinterpret_cast<bf16x8*>(y + row * N)[i] = __builtin_convertvector(nf * __builtin_convertvector(wv, f32x8), bf16x8);
     }
+}
+
+template <bool W8, int G>
+void launch_reduce_add_rmsnorm(const float* partial, int S, int M, int N, const void* bias, const void* scales, const void* x, int64_t ldx,
+                               const void* w, void* h_out, void* y, float eps, hipStream_t st) {
+    hipLaunchKernelGGL((reduce_add_rmsnorm_kernel<W8, G>), dim3(M), dim3(256 * G), 0, st, partial, S, M, N, (const bf16_t*)bias,
+                       (const bf16_t*)scales, (const bf16_t*)x, ldx, (const bf16_t*)w, (bf16_t*)h_out, (bf16_t*)y, eps);
 }
 
 __global__ __launch_bounds__(256) void silu_mul_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ b,
@@ -373,14 +389,10 @@ __global__ void tp_merge_kernel(const bf16_t* __restrict__ vals, const int64_t* 
 int md_internal_launch_reduce_add_rmsnorm(const float* partial, int S, int M, int N, const void* bias, const void* scales,
                                           const void* x, int64_t ldx, const void* w, void* h_out, void* y, float eps,
                                           hipStream_t st) {
-    if (scales)
-        hipLaunchKernelGGL((reduce_add_rmsnorm_kernel<true>), dim3(M), dim3(256), 0, st, partial, S, M, N,
-                           (const bf16_t*)bias, (const bf16_t*)scales, (const bf16_t*)x, ldx, (const bf16_t*)w,
-                           (bf16_t*)h_out, (bf16_t*)y, eps);
-    else
-        hipLaunchKernelGGL((reduce_add_rmsnorm_kernel<false>), dim3(M), dim3(256), 0, st, partial, S, M, N,
-                           (const bf16_t*)bias, (const bf16_t*)scales, (const bf16_t*)x, ldx, (const bf16_t*)w,
-                           (bf16_t*)h_out, (bf16_t*)y, eps);
+    const auto launch = N <= 2048 ? (scales ? launch_reduce_add_rmsnorm<true, 1> : launch_reduce_add_rmsnorm<false, 1>)
+                        : N <= 4096 ? (scales ? launch_reduce_add_rmsnorm<true, 2> : launch_reduce_add_rmsnorm<false, 2>)
+                                    : (scales ? launch_reduce_add_rmsnorm<true, 4> : launch_reduce_add_rmsnorm<false, 4>);
+    launch(partial, S, M, N, bias, scales, x, ldx, w, h_out, y, eps, st);
     return MD_OK;
 }
 
