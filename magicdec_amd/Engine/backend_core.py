@@ -30,7 +30,7 @@ PREFILL_ROWS = 16384   # rows of one prefill step where the portion is free to c
 # of 8 000 tokens 34 485 -> 6 955 (7 765 at 4096 rows), four of 1 500 (7B) 12 664 -> 6 157, four of 2 081 12 200 -> 6 540, one of 600
 # 2 969 -> 1 170.  8192 is what 64 requests had already; a layer's activations take 1.4 GB there on a 32B model.
 PROMPT_ROWS = 8192
-PROMPT_WINDOWS = 512 << 20     # bytes of one pass's StreamingLLM windows: 64 portions at a budget of 1024 rows of 8 heads of 128
+PROMPT_WINDOWS = 512 << 20     # bytes of one pass's StreamingLLM windows: 64 portions at a budget of 1 900 rows of 8 heads of 128
 
 
 def default_kv_layout():
