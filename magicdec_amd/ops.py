@@ -274,7 +274,7 @@ def streaming_windows(k_new, v_new, kv_cache, windows, following, portion, ctx, 
     KH, D = kv_cache.shape[3], kv_cache.shape[4]
     B = kv_cache.shape[0] // pages_per_req
     tokens = k_new.shape[0] // B
-    if (k_new.shape != v_new.shape or k_new.shape != (B * tokens, KH, D) or following.shape != kv_cache.shape
+    if (portion < 1 or k_new.shape != v_new.shape or k_new.shape != (B * tokens, KH, D) or following.shape != kv_cache.shape
             or windows.shape != (kv_cache.shape[0] * (-(-tokens // portion)), *kv_cache.shape[1:])
             or any(t.dtype != torch.bfloat16 for t in (k_new, v_new, kv_cache, windows, following))
             or not (kv_cache.is_contiguous() and windows.is_contiguous() and following.is_contiguous())

@@ -61,7 +61,7 @@ def test_what_it_does_not_take():
                     (7, 300), (7, 16)):
         args = list(good)
         args[at] = bad
-        with pytest.raises((ValueError, ZeroDivisionError, RuntimeError)):
+        with pytest.raises((ValueError, RuntimeError)):
             ops.streaming_windows(*args)
 
 
