@@ -200,12 +200,12 @@ def run_captured(backend, key, fn, input_ids, lead, tail):
             backend._move(tail)
             return out
         ent.graph = g
-        backend._graphs[full_key] = ent
         if all(name in gs for name in lead):             # what the steps from the next one on launch
-            _lead(ent, gs, lead, key[1], True)
+            _lead(ent, gs, lead, key[1], ops.step_copies(ent.static_in))
+        backend._graphs[full_key] = ent
     _bind_state(backend, ent)
     ids = input_ids.data_ptr() != ent.static_in.data_ptr()
-    if ids and not ops.step_copies(input_ids):
+    if ids and not (ops.step_copies(input_ids) and ops.step_copies(ent.static_in)):     # (either may hold 32-bit ids)
         ent.static_in.copy_(input_ids)
         ids = False
     _lead(ent, _statics(backend), own, key[1], ids).run(*([input_ids] if ids else []))

@@ -64,3 +64,27 @@ def test_lengths_of_a_captured_step():
             got += [e.inference(ids, benchmark=k == 5).cpu(), e.cachelens.cpu().clone(), e.paged_kv_last_page_len.cpu().clone()]
         made.append(got)
     assert all(torch.equal(a, b) for a, b in zip(*made))
+
+
+@pytest.mark.parametrize("kinds", [(torch.int32,) * 3, (torch.int32, torch.int64, torch.int32), (torch.int64, torch.int32, torch.int64)])
+def test_token_ids_of_either_width(kinds):
+    """A step captured on 32-bit ids, and one that meets the other width later: tokens and lengths of the eager engine."""
+    from magicdec_amd.Engine.model_core import transformer_configs
+    from magicdec_amd.Engine.SnapKV.backend import LMBackend
+    transformer_configs["step-ops-test"] = dict(block_size=512, n_layer=1, n_head=2, n_local_heads=1, dim=128, intermediate_size=256, vocab_size=64)
+    made = []
+    for graphs in (False, True):
+        e = LMBackend(dtype=torch.bfloat16, device=DEV)
+        e.load_model("none/step-ops-test/model.pth", use_tp=False)
+        if graphs:
+            e.compile()
+        e.setup_caches(max_batch_size=3, max_seq_length=256)
+        g = torch.Generator().manual_seed(1)
+        e.encode(torch.randint(4, 64, (3, 40), generator=g).to(DEV))
+        got = []
+        for kind in kinds:
+            got += [e.inference(torch.randint(4, 64, (3, 1), generator=g).to(kind).to(DEV)).cpu(), e.cachelens.cpu().clone(),
+                    e.paged_kv_last_page_len.cpu().clone()]
+        made.append(got)
+        assert e._use_graphs == graphs                       # (no fall-back to eager steps)
+    assert all(torch.equal(a, b) for a, b in zip(*made))
