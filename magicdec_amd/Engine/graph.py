@@ -131,7 +131,7 @@ def run_captured(backend, key, fn, input_ids, lead, tail):
     if ent is not None:
         # a tensor the caller put in the place of the static one is moved itself; _bind_state then takes its values over
         gs = _statics(backend)
-        own = {name: n for name, n in lead.items() if getattr(backend, name) is gs.get(name) and ops.step_adds(gs[name])}
+        own = {name: n for name, n in lead.items() if getattr(backend, name) is gs.get(name) and ops.step_adds(gs[name], ent.static_qo)}
         backend._move({name: n for name, n in lead.items() if name not in own})
     else:
         backend._move(lead)
@@ -205,7 +205,7 @@ def run_captured(backend, key, fn, input_ids, lead, tail):
         backend._graphs[full_key] = ent
     _bind_state(backend, ent)
     ids = input_ids.data_ptr() != ent.static_in.data_ptr()
-    if ids and not (ops.step_copies(input_ids) and ops.step_copies(ent.static_in)):     # (either may hold 32-bit ids)
+    if ids and not ops.step_copies(input_ids, ent.static_in):      # (32-bit ids, or another device's: torch copies them)
         ent.static_in.copy_(input_ids)
         ids = False
     _lead(ent, _statics(backend), own, key[1], ids).run(*([input_ids] if ids else []))
@@ -213,7 +213,7 @@ def run_captured(backend, key, fn, input_ids, lead, tail):
     add = []
     for name, n in tail.items():
         t = getattr(backend, name)
-        if ops.step_adds(t):
+        if ops.step_adds(t, ent.static_out):
             add.append((t, n))
         else:
             t.add_(n)

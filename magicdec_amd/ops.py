@@ -1289,7 +1289,8 @@ STEP_ADD, STEP_SCALE, STEP_COPY, STEP_MAX = 0, 1, 2, 8
 
 class StepOps:
     """The integer work around a decode step in one launch: add = [(int32 tensor, a)]: t += a; scale = [(dst, src, a)]: dst = src * a
-    (int32); copies = [dst]: int64 tensors that `run` fills, from sources of unit row stride.  What does not change from call to call is
+    (int32); copies = [dst]: int64 tensors that `run` fills, from sources of unit row stride.  All on one device: a kernel reads its
+    pieces' memory directly.  What does not change from call to call is
     set up once (a launch then costs the host one foreign call); the tensors are kept alive."""
 
     def __init__(self, add=(), scale=(), copies=()):
@@ -1310,6 +1311,8 @@ class StepOps:
         _gpu(dst, src)
         if self._n == STEP_MAX or not dst.is_contiguous():
             raise ValueError(f"step_ops: at most {STEP_MAX} pieces, into dense tensors")
+        if any(t is not None and t.device != dst.device for t in [src] + self._kept):
+            raise ValueError("step_ops: every piece lies on one device")
         self._ops[self._n] = _lib.StepOp(dst.data_ptr(), src.data_ptr() if src is not None else None, 0, 1, dst.numel(), kind, a)
         self._kept += [dst, src]
         self._n += 1
@@ -1318,8 +1321,8 @@ class StepOps:
         """One source per copy; `into` replaces the copies' destinations for this call (dense, same shapes)."""
         n = self._n
         for j, (dst, src) in enumerate(zip(into or self._copies, sources, strict=True)):
-            if dst.shape != src.shape or not step_copies(src) or not dst.is_contiguous():
-                raise ValueError("step_ops: copy needs int64 tensors of one shape, rows of unit stride")
+            if dst.shape != src.shape or not step_copies(src, dst) or not dst.is_contiguous():
+                raise ValueError("step_ops: copy needs int64 tensors of one shape on one device, rows of unit stride")
             op = self._ops[self._first + j]
             op.dst, op.src = dst.data_ptr(), src.data_ptr()
             if src.is_contiguous():
@@ -1330,12 +1333,12 @@ class StepOps:
             check(_lib.load().md_step_ops(self._ops, n, _stream()), "md_step_ops")
 
 
-def step_copies(t):
-    """Can StepOps copy from this tensor?"""
-    return t.is_cuda and t.dtype == torch.int64 and t.numel() > 0 and (
+def step_copies(t, dst=None):
+    """Can StepOps copy from this tensor (into `dst`)?"""
+    return t.is_cuda and t.dtype == torch.int64 and t.numel() > 0 and (dst is None or (dst.device == t.device and dst.dtype == t.dtype)) and (
         t.is_contiguous() or (t.dim() == 2 and (t.shape[1] == 1 or t.stride(1) == 1)))
 
 
-def step_adds(t):
-    """Can StepOps add to this tensor?"""
-    return t.is_cuda and t.dtype == torch.int32 and t.numel() > 0 and t.is_contiguous()
+def step_adds(t, beside=None):
+    """Can StepOps add to this tensor (in a launch that works on `beside`)?"""
+    return t.is_cuda and t.dtype == torch.int32 and t.numel() > 0 and t.is_contiguous() and (beside is None or t.device == beside.device)

@@ -1430,3 +1430,17 @@ def test_one_resident_copy_per_weight_release_and_restore():
     # without announced row counts nothing is released (any row count may come)
     m2 = build("dedupe_any", None, n_head=32, n_local_heads=8, dim=2048, intermediate_size=8192)
     assert m2.release_rowmajor() == 0 and m2.packed_bytes > 0
+
+
+def test_step_launch_takes_tensors_of_one_device():
+    """The launch around a captured step reads its tensors' memory directly: ids or lengths on another GPU are left to torch (no memory
+    is touched here: fake tensors)."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from magicdec_amd import ops
+    with FakeTensorMode():
+        ids, i32 = ({d: torch.empty(3, 2, dtype=t, device=d) for d in ("cuda:0", "cuda:1")} for t in (torch.int64, torch.int32))
+    assert ops.step_copies(ids["cuda:0"], ids["cuda:0"]) and not ops.step_copies(ids["cuda:1"], ids["cuda:0"])
+    assert not ops.step_copies(ids["cuda:0"], i32["cuda:0"])
+    assert ops.step_adds(i32["cuda:0"], ids["cuda:0"]) and not ops.step_adds(i32["cuda:1"], ids["cuda:0"])
+    with pytest.raises(ValueError, match="one device"):
+        ops.StepOps(add=[(i32["cuda:0"], 1), (i32["cuda:1"], 1)])
