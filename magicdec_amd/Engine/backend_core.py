@@ -18,6 +18,8 @@ What is different underneath:
 """
 from __future__ import annotations
 
+import contextlib
+
 import torch
 
 from .model_core import PageTable
@@ -243,17 +245,21 @@ class _BackendBase:
             return dict(tail=tail) if n > tail else {}
         return dict(head_rows=torch.arange(1, self.batch_size + 1, device=self.device) * n - 1)
 
-    def _prefill_begin(self):
-        """Prefill-sized products run on the library GEMM over the row-major weights: the ones released after the previous prefill
-        come back as the portions ask for them (a head that only ever sees the last rows is not among them)."""
+    @contextlib.contextmanager
+    def _prefilling(self):
+        """Around the portions of a prompt.  Their products run on the library GEMM over the row-major weights: the ones released after
+        the previous prompt come back as the portions ask for them (a head that only ever sees the last rows is not among them).  Behind
+        it, also where the prompt is refused: decode reads most weights in the streaming layout only, their row-major tensors are freed
+        (one resident copy), and the next step has its head."""
         if hasattr(self.model, "restore_on_demand"):
             self.model.restore_on_demand(True)
-
-    def _prefill_end(self):
-        """Decode reads most weights in the streaming layout only: free their row-major tensors (one resident copy)."""
-        if hasattr(self.model, "release_rowmajor"):
-            self.model.restore_on_demand(False)
-            self.model.release_rowmajor()
+        try:
+            yield
+        finally:
+            self.model.skip_head = False
+            if hasattr(self.model, "release_rowmajor"):
+                self.model.restore_on_demand(False)
+                self.model.release_rowmajor()
 
     def _reset_kv_calibration(self):
         """fp8 caches re-calibrate their static scales on the first prefill chunk of every encode()."""
@@ -350,20 +356,19 @@ class SnapKVTargetBackend(_BackendBase):
         if self.pool_only or self.pool.seqs:
             raise RuntimeError("encode: the pages belong to the sequences of step()")
         self.clear_kv()
-        self._prefill_begin()
         seq_len = input_ids.shape[1]
         tokens = None
         is_last = False
-        for done, n in self._portions(seq_len):
-            ids = input_ids[:, done:done + n]
-            is_last = done + n == seq_len and n % self.prefill_chunk != 0
-            self._map_portion(done + n)                       # pre_encode
-            self.model.skip_head = done + n != seq_len
-            tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table((n, done + n)), is_last=is_last,
-                                        draft_tab=self._d.table() if (self.is_spec and is_last) else None,
-                                        ctx_len=done + n, **self._last_rows(n, seq_len))
-            self.cachelens += n
-        self.model.skip_head = False
+        with self._prefilling():
+            for done, n in self._portions(seq_len):
+                ids = input_ids[:, done:done + n]
+                is_last = done + n == seq_len and n % self.prefill_chunk != 0
+                self._map_portion(done + n)                   # pre_encode
+                self.model.skip_head = done + n != seq_len
+                tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table((n, done + n)), is_last=is_last,
+                                            draft_tab=self._d.table() if (self.is_spec and is_last) else None,
+                                            ctx_len=done + n, **self._last_rows(n, seq_len))
+                self.cachelens += n
         if self.mapped:
             tokens = tokens.view(-1, 1)
         if self.is_spec:
@@ -371,7 +376,6 @@ class SnapKVTargetBackend(_BackendBase):
                 raise ValueError("SnapKV self-speculation: prefix_len is a multiple of 128, so no last chunk ran the "
                                  "select and the draft cache is empty (need (prefix_len - window_size) % 128 == 0)")
             self.draft_cachelens.copy_(self.cachelens)
-        self._prefill_end()
         return tokens
 
     # ------------------------------------------------------------------ sequences of unequal lengths
@@ -397,31 +401,28 @@ class SnapKVTargetBackend(_BackendBase):
         got = [{} for _ in entries]                        # per entry: place -> logits row
         last = [None] * len(entries)
         prefill = any(t.numel() > 1 for t in ids)
-        if prefill:
-            self._prefill_begin()
-        while any(d < t.numel() for d, t in zip(done, ids)):
-            live = [k for k, t in enumerate(ids) if done[k] < t.numel()]
-            portion = max(1, max(PREFILL_ROWS, getattr(self.model, "prefill_rows", 0)) // len(live))
-            take = {k: min(portion, ids[k].numel() - done[k]) for k in live}
-            rows, row0 = [], 0                             # (entry, place | None = sampled only, flat row)
-            for k in live:
-                lo, hi = done[k], done[k] + take[k]
-                places = set(w for w in want[k] if lo <= w < hi)
-                if sample and hi == ids[k].numel():
-                    places.add(hi - 1)
-                rows += [(k, w, row0 + w - lo) for w in sorted(places)]
-                row0 += take[k]
-            tokens, logits = self._ragged_step([(entries[k][0], ids[k][done[k]:done[k] + take[k]]) for k in live],
-                                               [r for _, _, r in rows])
-            for j, (k, w, _) in enumerate(rows):
-                if w in want[k]:
-                    got[k][w] = logits[j]
-                if sample and w == ids[k].numel() - 1:
-                    last[k] = tokens[j]
-            for k in live:
-                done[k] += take[k]
-        if prefill:
-            self._prefill_end()
+        with self._prefilling() if prefill else contextlib.nullcontext():
+            while any(d < t.numel() for d, t in zip(done, ids)):
+                live = [k for k, t in enumerate(ids) if done[k] < t.numel()]
+                portion = max(1, max(PREFILL_ROWS, getattr(self.model, "prefill_rows", 0)) // len(live))
+                take = {k: min(portion, ids[k].numel() - done[k]) for k in live}
+                rows, row0 = [], 0                             # (entry, place | None = sampled only, flat row)
+                for k in live:
+                    lo, hi = done[k], done[k] + take[k]
+                    places = set(w for w in want[k] if lo <= w < hi)
+                    if sample and hi == ids[k].numel():
+                        places.add(hi - 1)
+                    rows += [(k, w, row0 + w - lo) for w in sorted(places)]
+                    row0 += take[k]
+                tokens, logits = self._ragged_step([(entries[k][0], ids[k][done[k]:done[k] + take[k]]) for k in live],
+                                                   [r for _, _, r in rows])
+                for j, (k, w, _) in enumerate(rows):
+                    if w in want[k]:
+                        got[k][w] = logits[j]
+                    if sample and w == ids[k].numel() - 1:
+                        last[k] = tokens[j]
+                for k in live:
+                    done[k] += take[k]
         out = [got[k][w] for k in range(len(entries)) for w in want[k]]
         return (torch.stack(last) if sample else None), (torch.stack(out) if out else None)
 
@@ -534,26 +535,24 @@ class SnapKVDraftBackend(_BackendBase):
     def encode(self, input_ids: torch.LongTensor, benchmark=False):
         """backend_draft.py:176-209."""
         self.clear_kv()
-        self._prefill_begin()
         seq_len = input_ids.shape[1]
         tokens = None
         is_last = False
-        for done, n in self._portions(seq_len):
-            ids = input_ids[:, done:done + n]
-            is_last = done + n == seq_len and n % self.prefill_chunk != 0
-            self._map_portion(done + n)                       # pre_encode
-            self.model.skip_head = done + n != seq_len
-            tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table((n, done + n)), is_last=is_last,
-                                        draft_tab=self._d.table() if (self.is_compress and is_last) else None,
-                                        ctx_len=done + n, **self._last_rows(n, seq_len))
-            self.cachelens += n
-        self.model.skip_head = False
+        with self._prefilling():
+            for done, n in self._portions(seq_len):
+                ids = input_ids[:, done:done + n]
+                is_last = done + n == seq_len and n % self.prefill_chunk != 0
+                self._map_portion(done + n)                   # pre_encode
+                self.model.skip_head = done + n != seq_len
+                tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table((n, done + n)), is_last=is_last,
+                                            draft_tab=self._d.table() if (self.is_compress and is_last) else None,
+                                            ctx_len=done + n, **self._last_rows(n, seq_len))
+                self.cachelens += n
         if self.mapped:
             tokens = tokens.view(-1, 1)
         if self.is_compress and not is_last:
             raise ValueError("SnapKV draft: prefix_len is a multiple of 128, so no last chunk ran the select and the "
                              "draft cache is empty (need (prefix_len - window_size) % 128 == 0)")
-        self._prefill_end()
         return tokens
 
     @torch.no_grad()
@@ -586,7 +585,6 @@ class _StreamingMixin:
     """Sink(16)+window prefill shared by the stand-alone StreamingLLM draft and the self-spec engine."""
 
     def _stream_encode(self, input_ids, state: _PagedState, lens_attr, which):
-        self._prefill_begin()
         seq_len, B = input_ids.shape[1], self.batch_size
         tokens = None
         num_chunks = (seq_len + CHUNK - 1) // CHUNK
@@ -596,27 +594,26 @@ class _StreamingMixin:
                                                         PROMPT_WINDOWS // (cache.numel() * cache.element_size()))
         passes = -(-num_chunks // max(1, most))
         ctx = 0                                       # host mirror of the (capped) cache length
-        for i in range(passes):
-            first, end = num_chunks * i // passes, num_chunks * (i + 1) // passes
-            ids = input_ids[:, first * CHUNK:min(end * CHUNK, seq_len)]
-            is_last = end * CHUNK > seq_len
-            start, pages = ctx, state.host_pages
-            for c in range(first, end):               # pre_encode (StreamingLLM/backend_draft.py:155-192)
-                n = min(CHUNK, seq_len - c * CHUNK)
-                pages, last = (pages + 1, n) if ctx + n <= self.draft_budget else (state.ppr, self.draft_budget % PAGE_SIZE)
-                ctx = min(ctx + n, self.draft_budget)
-            state.map_pages(pages, last)
-            self.model.skip_head = i != passes - 1
-            if end - first > 1:
-                tokens = self.model.stream_portions(ids, start, CHUNK, is_last, which, B)
-            else:
-                tokens = self.model.stream_prefill(ids, start, self._qo(n), state.table(), is_last, which, B)
-            lens = getattr(self, lens_attr)
-            lens += ids.shape[1]
-            if ctx >= self.draft_budget:
-                lens.fill_(self.draft_budget)
-        self.model.skip_head = False
-        self._prefill_end()
+        with self._prefilling():
+            for i in range(passes):
+                first, end = num_chunks * i // passes, num_chunks * (i + 1) // passes
+                ids = input_ids[:, first * CHUNK:min(end * CHUNK, seq_len)]
+                is_last = end * CHUNK > seq_len
+                start, pages = ctx, state.host_pages
+                for c in range(first, end):               # pre_encode (StreamingLLM/backend_draft.py:155-192)
+                    n = min(CHUNK, seq_len - c * CHUNK)
+                    pages, last = (pages + 1, n) if ctx + n <= self.draft_budget else (state.ppr, self.draft_budget % PAGE_SIZE)
+                    ctx = min(ctx + n, self.draft_budget)
+                state.map_pages(pages, last)
+                self.model.skip_head = i != passes - 1
+                if end - first > 1:
+                    tokens = self.model.stream_portions(ids, start, CHUNK, is_last, which, B)
+                else:
+                    tokens = self.model.stream_prefill(ids, start, self._qo(n), state.table(), is_last, which, B)
+                lens = getattr(self, lens_attr)
+                lens += ids.shape[1]
+                if ctx >= self.draft_budget:
+                    lens.fill_(self.draft_budget)
         return tokens
 
 
@@ -718,17 +715,15 @@ class StreamingSelfSpecBackend(_BackendBase, _StreamingMixin):
     def encode(self, input_ids: torch.LongTensor, benchmark=False):
         """Target prefill (StreamingLLM/backend.py:190-211)."""
         self.clear_kv()
-        self._prefill_begin()
         seq_len = input_ids.shape[1]
         tokens = None
-        for done, n in self._portions(seq_len):
-            ids = input_ids[:, done:done + n]
-            self._map_portion(done + n)
-            self.model.skip_head = done + n != seq_len
-            tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table(), **self._last_rows(n, seq_len))
-            self.cachelens += n
-        self.model.skip_head = False
-        self._prefill_end()
+        with self._prefilling():
+            for done, n in self._portions(seq_len):
+                ids = input_ids[:, done:done + n]
+                self._map_portion(done + n)
+                self.model.skip_head = done + n != seq_len
+                tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table(), **self._last_rows(n, seq_len))
+                self.cachelens += n
         return tokens
 
     @torch.no_grad()

@@ -1444,3 +1444,34 @@ def test_step_launch_takes_tensors_of_one_device():
     assert ops.step_adds(i32["cuda:0"], ids["cuda:0"]) and not ops.step_adds(i32["cuda:1"], ids["cuda:0"])
     with pytest.raises(ValueError, match="one device"):
         ops.StepOps(add=[(i32["cuda:0"], 1), (i32["cuda:1"], 1)])
+
+
+@pytest.mark.parametrize("prompt", ["refused", "failing"])
+def test_a_refused_prompt_leaves_the_weights_released(cpu_ops_patched, prompt):
+    """A prompt that raises (the SnapKV engine's refusal of its length, or an error inside a portion) ends like one that does not: no
+    weight is restored on demand any more, those that were are released again, and the next step has its head."""
+    from magicdec_amd.Engine import model_core
+    from magicdec_amd.Engine.SnapKV.backend import LMBackend
+    model_core.transformer_configs["refused-prompt"] = dict(block_size=1024, n_layer=1, n_head=4, n_local_heads=2, dim=256,
+                                                            intermediate_size=512, vocab_size=128)
+    try:
+        e = LMBackend(dtype=torch.bfloat16, device="cpu", dec_len=3, draft_dec_len=1)
+        e.load_model("none/refused-prompt/model.pth", use_tp=False)
+        e.setup_caches(max_batch_size=2, max_seq_length=512, draft_budget=65, window_size=32)
+    finally:
+        model_core.transformer_configs.pop("refused-prompt", None)
+    m = e.model
+    m._pack_weights(force=True)
+    assert m.release_rowmajor() > 0
+    released, plain = set(m._released), m.prefill
+
+    def prefill(*args, **kw):                      # (a library product of the portion asks for a released weight)
+        m._resident(m.layers[0].attention.wqkv.weight)
+        assert m._on_demand and released - m._released == {id(m.layers[0].attention.wqkv.weight)}
+        if prompt == "failing" and not m.skip_head:
+            raise RuntimeError("inside a portion")
+        return plain(*args, **kw)
+    m.prefill = prefill
+    with pytest.raises((ValueError, RuntimeError)):
+        e.encode(torch.randint(4, 128, (2, 256 if prompt == "refused" else 160)))
+    assert not m._on_demand and m._released == released and not m.skip_head
