@@ -30,6 +30,7 @@ A weight a hand-written kernel will serve is re-packed once at setup_caches (Tra
 copy stays for the prefill-sized products.  MAGICDEC_GEMM=hip forces md_linear wherever it supports the shape,
 MAGICDEC_GEMM=lib forces the library, MAGICDEC_FUSED=0/1 switches md_linear_fused off / on everywhere (the A/B
 switches)."""
+import functools
 import os
 import re
 
@@ -53,13 +54,10 @@ FUSED_DEEP_SWIGLU_T22_MAX_L2_BYTES = float(os.environ.get("MAGICDEC_DEEP_SWIGLU_
 _SHARD70B = os.environ.get("MAGICDEC_SHARD70B", "1")     # "0": without the two round-6 rules for the 70B shards (A/B switch)
 FUSED_MAX_K = 4096
 FUSED_QKV_M256_MAX_L2_BYTES = 110e6
-# the bounds of _measured(): tile traffic (M tiles x weight bytes) of a qkv projection (K <= 4096, deeper) and of a residual projection
-# of 4096 < K <= 5632, and the weight bytes up to which a one-tile step prefers the tile kernel or its K split (5120 x 27 648 at one
-# row: skinny 58.8, split 65.4; 28 672 x 4096 at 32 rows: skinny 46.0, tile 47.0)
+# the bounds of _measured(): tile traffic (M tiles x weight bytes) of a qkv projection (K <= 4096, deeper), and the weight bytes up to
+# which 5..32 rows of a gated projection prefer the tile kernel
 FUSED_QKV_MAX_L2_BYTES = 270e6
 FUSED_QKV_DEEP_MAX_L2_BYTES = 230e6
-FUSED_MAX_L2_BYTES_DEEP_RESID = 100e6
-SPLIT_ONE_TILE_MAX_BYTES = 150e6
 SWIGLU_ONE_TILE_MAX_BYTES = 210e6
 # round 5 (profiles/r05_fused_tp8_shard_tiles.txt, M = 256): two more TP8 shards of the 8B verify pass go to the fused kernel --
 # w1|w3 (29.4 MB; 2 x 2 tiles: 21.1-22.3 us against 24.1 for the library + the SiLU*mul launch) and wo (4.2 MB, K = 512:
@@ -139,96 +137,174 @@ def want_packed(N: int, K: int, swiglu: bool = False, int8: bool = False, rows=N
     return False
 
 
-# Shapes the library holds a measured solution for (tuned/gemm_gfx950.csv, "tn_N_M_K_...").  There the library is a good deal faster
-# than where it has to guess (8B wqkv, 6144 x 4096: 20.6 us at 64 rows and 27 at 256; at 96 and 192, which the table does not hold,
-# 28.5 and 39.0), so rules below that would take a narrow product away from it leave these alone.
+# Shapes the library holds a tuned solution for (tuned/gemm_gfx950.csv, "tn_N_M_K_...": lines that name one; "Default" says that the
+# tuning found none better than the library's own choice).  Some rules below leave these alone: 8B wqkv (6144 x 4096) at 256 rows 32.1 us
+# with it, 37.5 on the block kernel; 4096 x 3584 + residual at 128 rows 19.8 against 21.6.
+_TABLE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tuned", "gemm_gfx950.csv")
 _TUNED = None
+
+
+def tuned_table(path):
+    """The table of tuned solutions that PyTorch took (Engine.utils.enable_tuned_gemms), None: it refused it (other library versions),
+    so that none of its solutions is in use."""
+    global _TABLE, _TUNED
+    _TABLE, _TUNED = path, None
 
 
 def _tuned(M: int, N: int, K: int) -> bool:
     global _TUNED
     if _TUNED is None:
-        path = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tuned", "gemm_gfx950.csv")
         rows = set()
-        if os.path.exists(path):
-            with open(path) as f:
+        if _TABLE is not None and os.path.exists(_TABLE):
+            with open(_TABLE) as f:
                 for line in f:
-                    m = re.match(r"GemmTunableOp_BFloat16_TN,tn_(\d+)_(\d+)_(\d+)_", line)
+                    m = re.match(r"GemmTunableOp_BFloat16_TN,tn_(\d+)_(\d+)_(\d+)_[^,]*,(?!Default,)", line)
                     if m:
                         rows.add((int(m.group(2)), int(m.group(1)), int(m.group(3))))
         _TUNED = rows
     return (M, N, K) in _TUNED
 
 
-def _measured(M: int, N: int, K: int, kind: str, absorbs_norm: bool):
+CUS = 256
+
+
+def _last_round(workgroups: int) -> float:
+    """Rounds of the chip that so many workgroups take, over the rounds they fill: 1.0 = the last one is full."""
+    return -(-workgroups // CUS) * CUS / workgroups
+
+
+def _last_chunk(K: int) -> float:
+    """The same of the tile kernel's eight waves, which stage K in chunks of 128 each: 1.0 = the last chunk is whole."""
+    return -(-K // 1024) * 1024 / K
+
+
+@functools.lru_cache(maxsize=4096)
+def _slices(kind: str, N: int, K: int) -> int:
+    """K slices of md_linear ("skinny") or md_linear_fused_split ("tile") at up to 32 rows; 0: not this shape."""
+    from .. import ops
+    return ops.linear_planes_count(kind, 1, N, K)
+
+
+def _skinny_one_round(N: int, K: int) -> bool:
+    """Are md_linear's workgroups (128 columns of one K slice) one nearly full round of the chip?"""
+    return 0.8 * CUS < -(-N // 128) * _slices("skinny", N, K) <= CUS
+
+
+def _measured(M, N, K, kind, absorbs_norm):
     """The kernel for the shapes where the general rules below (drawn for the 1B and 8B models at 32, 64, 128 and 256 rows) were
     measured to pick a slower one of the framework's own kernels, or the library where one of them is faster: "fused" | "block" |
     "skinny" | "split", None: the general rules.  Times in us, the whole sub-step (with the add + norm, the rope or the SiLU*mul
-    behind it), graph-captured, weights cycled.  `kind` "planes": an output projection whose combine is the residual add + norm
-    launch of a model that keeps its residual in float32 (the tile kernel's residual epilogue is no choice there)."""
+    behind it), graph-captured, weights cycled; every kernel at 13 row counts of 180 shapes a kind, the zoo's among them.  `kind`
+    "planes": an output projection whose combine is the residual add + norm launch of a model that keeps its residual in float32 (the
+    tile kernel's residual epilogue is no choice there).
+    The library's own choice above 128 rows is even but for exact multiples of 32, where it takes a slow kernel (6144 x 4096: 25.7..26.6
+    at 161..255 rows, but 33.3 at 192 and 36.8 at 224; 5120 x 5120: 29.7 at 193, 41.5 at 192, 49.6 at 256): `nice` below."""
     if M > 256 or K % 128 or N % 32:
         return None
-    nbytes, m_tiles, tiles = N * K * 2, (M + 31) // 32, N // 128
-    # the block kernel takes 128 columns a workgroup: 160..256 of them are one nearly full round of the 256 CUs
-    one_round = N % 128 == 0 and BLOCK_MIN_TILES <= tiles <= 256
+    nbytes, m_tiles, n_tiles, tiles = N * K * 2, (M + 31) // 32, N // 32, N // 128
+    nice = M % 32 == 0
     if kind == "plain":
-        # 33..128 rows of a 32 000-entry head in one round of block workgroups, against the skinny kernel's K slices and their
-        # combine: K = 2048 36.3 -> 30.3 (64 rows), 42.9 -> 32.6 (128); K = 4096 56.2 -> 50.8, 63.3 -> 53.4; K = 768, on the
-        # tile kernel, 19.4 / 30.9 -> 15.3 / 16.4.  More than one round is worse (128 256 entries: stays)
-        if 32 < M <= 128 and one_round:
+        # a head in one round of block workgroups (128 columns each: 160..256), 33..128 rows.  Below the streaming kernel's sizes K = 768
+        # x 32 000 19.4 / 30.9 on the tile kernel -> 15.3 / 16.4 (64 / 128 rows); against the library above 64 rows from 200 workgroups
+        # on (29 952 x 1280 23.8 -> 22.8, but 21 504 x 2048 26.5 against 29.1), against the streaming kernel above 64 rows if the round
+        # is full (32 000 x 4096 56.6 -> 52.5, 30 208 x 4096 53.1 against 57.9).  Up to 64 rows that one stays ahead: 32 000 x 2048 27.0 /
+        # 30.6, x 4096 49.2 / 52.1 (if K does not fall into many slices: 30 848 x 2944, 23 of them, 67.8 -> 41.6 at 39 rows)
+        least = BLOCK_MIN_TILES if nbytes < MIN_STREAM_BYTES or M <= 64 else 200 if nbytes < MIN_STREAM_BYTES_M128 else 240
+        if (32 < M <= 128 and N % 128 == 0 and least <= tiles <= CUS
+                and (M > 64 or nbytes < MIN_STREAM_BYTES or _slices("skinny", N, K) > 8)):
             return "block"
-        # one M tile over a long stream of columns: the tile kernel's workgroups each finish their columns, nothing to combine.
-        # 128 256 x 4096 at one row 172 -> 158, x 2048 92 -> 81; 32 000 x 4096 47.9 -> 44.6.  At 32 rows only in one round:
-        # 32 000 x 2048 31.7 -> 26.9, x 4096 51.5 -> 49.3, 14 336 x 4096 27.0 -> 25.2, but x 5120 60.0 against 61.2 and
-        # 128 256 x 2048 93.8 against 101
-        if M <= (32 if tiles <= 256 and K <= FUSED_MAX_K else 16) and N >= 14336 and nbytes >= MIN_STREAM_BYTES:
+        # one M tile over a long stream of columns: the tile kernel's workgroups each finish their columns, nothing to combine -- in
+        # fewer than two rounds, or where the last round and the last chunk of K are nearly full.  128 256 x 4096 at one row 172 -> 158,
+        # x 2048 92 -> 81; 32 000 x 4096 47.6 -> 45.5; but 16 896 x 4224 (2.06 rounds, 4.1 chunks) 27.5 against 32.4, 37 120 x 3200 (4.5,
+        # 3.1) 39.5 against 42.4 and 115 328 x 1280 (14.1, 1.25) 49.8 against 56.6.  To 32 rows only within four rounds (32 000 x 4096
+        # 49.9 -> 49.4 at 26 rows, 14 336 x 4096 26.2 -> 24.8; 54 912 x 2560 17 % slower); deep and wide to 8 (73 472 x 4736 at 16: 109
+        # against 115)
+        if (N >= 14336 and nbytes >= MIN_STREAM_BYTES and K >= 1024
+                and (n_tiles < 2 * CUS or (_last_round(n_tiles) <= 1.09 and _last_chunk(K) <= 1.15))
+                and M <= (8 if K > FUSED_MAX_K and n_tiles > 4 * CUS else 16 if K > FUSED_MAX_K or n_tiles > 4 * CUS else 32)):
             return "fused"
     if kind == "swiglu":
         # up to four rows the tile kernel stages four, also with a norm to absorb: 28 672 x 4096 43.9 -> 42.2, 37 888 x 3584 52.0 ->
         # 47.4, 55 296 x 5120 92.6 -> 88.0; at 16 rows 44.9 / 51.7 / 92.0 on the skinny kernel against 44.7 / 52.4 / 95.6
-        if M <= 4 and N >= 14336 and nbytes >= MIN_STREAM_BYTES:
+        # (not 61 312 x 1152, its second chunk of K nearly empty: 28.3 against 34.2)
+        whole = n_tiles < 2 * CUS or _last_chunk(K) <= 1.15
+        if M <= 4 and N >= 14336 and nbytes >= MIN_STREAM_BYTES and whole:
             return "fused"
-        if M <= 32 and N >= 14336 and not absorbs_norm and MIN_STREAM_BYTES <= nbytes <= SWIGLU_ONE_TILE_MAX_BYTES:
-            return "fused"            # 24 576 x 4096: 38.4 -> 35.5 (one row), 41.0 -> 38.3 (32); with a norm to absorb skinny is faster
+        # without a norm: to 16 rows 24 576 x 4096 38.4 -> 35.5, 22 016 x 4096 34.5 -> 31.8 (26 624 x 4864, 259 MB: 5 % slower); to 32
+        # rows within three rounds, the last one nearly full: 24 576 x 4096 41.3 -> 38.6, 22 016 x 4096 36.5 -> 35.8, but 18 432 x 5120
+        # (2.25 rounds) 35.5 against 39.6 and 27 648 x 3584 (3.4) 40.4 against 42.5
+        if (not absorbs_norm and N >= 14336 and MIN_STREAM_BYTES <= nbytes <= SWIGLU_ONE_TILE_MAX_BYTES and whole
+                and (M <= 16 or (M <= 32 and n_tiles <= 3 * CUS and _last_round(n_tiles) <= 1.19))):
+            return "fused"
         # 65..128 rows, more than one round of block workgroups (296 or 432: the last round nearly empty): 37 888 x 3584
         # 84.6 -> 63.2 on the skinny kernel, 55 296 x 5120 133 -> 102 (128 rows), 124 -> 99 (96)
-        if 64 < M <= 128 and N % 128 == 0 and tiles > 256:
+        if 64 < M <= 128 and N % 128 == 0 and tiles > CUS:
             return "skinny"
     if kind in ("resid", "planes") and N <= 8192:
-        if K >= 8192 and nbytes >= MIN_STREAM_BYTES:
-            # the deep projections: 3584 x 18 944 at 1 / 32 rows 32.2 / 33.1 on the skinny kernel, 30.5 / 31.7 with the tile
-            # kernel's K split, 4096 x 14 336 28.2 -> 27.2.  (At 96 / 128 rows skinny, 40.7 / 42.9, and block, 38.5..47.5, are level.)
-            if M <= 32 and kind == "resid" and nbytes <= SPLIT_ONE_TILE_MAX_BYTES:
-                return "split"
+        # the deep projections at one M tile: the tile kernel's K split where its workgroups (64 columns of one slice) are one nearly
+        # full round.  3584 x 18 944 30.8 / 32.5 -> 28.5 / 31.9 (1 / 31 rows), 4096 x 14 336 27.1 -> 25.7, 4096 x 18 432 32.4 -> 30.3;
+        # with half a round (4096 x 11 008) 23.1 against 26.8, with a second (5120 x 13 824) 32.3 against 36.7
+        if (kind == "resid" and K >= 8192 and nbytes >= MIN_STREAM_BYTES and M <= 32 and N % 64 == 0
+                and 0.8 * CUS < N // 64 * _slices("tile", N, K) <= CUS):
+            return "split"
         if FUSED_MAX_K < K < 8192:
             if kind == "planes":
-                return "skinny"       # 2048 x 7680: 16.0 / 20.3 / 26.5 / 24.6 / 32.2 in the library -> 12.9 / 14.5 / 16.9 / 21.4 / 28.3
-                                      # (1 / 32 / 64 / 128 / 256 rows); the tile kernel's K split 14.8 / 17.1 / 24.2 / 22.8 / 35.0
+                # 2048 x 7680: 16.0 / 20.3 / 26.5 / 24.6 / 32.2 in the library -> 12.9 / 14.5 / 16.9 / 21.4 / 28.3 (1 / 32 / 64 / 128 / 256
+                # rows); the tile kernel's K split 14.8 / 17.1 / 24.2 / 22.8 / 35.0.  More slices are more planes to write and add, the
+                # more so the more rows: 896 x 7680 (60) 15.5 against 19.8 at 41 rows, 2048 x 4864 (19) 18.2 against 20.7 at 101,
+                # 2176 x 5120 (14) 24.4 against 27.8 at 144 but 30.4 -> 25.8 at 256; and a second round costs (6784 x 4992, 689
+                # workgroups, 34.0 against 38.3 at 75; 3072 x 7040, 264, 40.1 against 48.7 at 256)
+                slices, one = _slices("skinny", N, K), _skinny_one_round(N, K)
+                workgroups = -(-N // 128) * slices
+                if M <= 64:
+                    return "skinny" if slices <= 50 else None
+                if M <= 128:
+                    return "skinny" if (one and slices <= 30) or (slices <= 15 and workgroups <= 1.7 * CUS) else None
+                return "skinny" if (one and K >= 6000) or (nice and slices <= 15 and workgroups <= CUS) else None
             if K <= 5632 and M <= 128:
                 if M <= 32 and nbytes < 30e6:
                     return "skinny"   # 2048 x 5632: 14.3 / 13.4 / 18.4 in the library -> 11.4 / 11.7 / 13.2 (1 / 8 / 32 rows)
-                if m_tiles * nbytes <= FUSED_MAX_L2_BYTES_DEEP_RESID:
-                    return "fused"    # 2048 x 5632 21.1 / 19.4 -> 15.2 / 14.5 (64 / 128), 5120 x 5120 22.8 -> 16.5 (32)
-        # 3584..5632 deep and wide, more rows than the tile kernel's budget: the library, untuned, against the skinny kernel (up to 128
-        # rows) or the block kernel: 3584 x 3584 23.8 / 26.5 / 33.8 -> 22.4 / 23.3 / 25.5 (96 / 128 / 192), 5120 x 5120 26.1 / 36.6 /
-        # 54.8 -> 22.8 / 27.9 / 32.6 (64 / 128 / 256), 4096 x 4096 25.9 -> 21.9 (96)
+                # one round of the tile kernel: 2048 x 5632 21.1 / 19.4 -> 15.2 / 14.5 (64 / 128), 5120 x 5120 22.8 -> 16.5 (32);
+                # 4608 x 4352 at 64 (288 workgroups) 23.6 against 30.8
+                if n_tiles * m_tiles <= CUS:
+                    return "fused"
+        # 3584..5632 deep and wide, more than one round of tile workgroups: the library against the skinny kernel (up to 128 rows):
+        # 3584 x 3584 23.8 / 26.5 -> 22.4 / 23.3 (96 / 128), 5120 x 5120 26.1 / 36.6 -> 22.8 / 27.9 (64 / 128), 4096 x 4096 25.9 -> 21.9
+        # (96); or the block kernel, at multiples of 32 rows and for the deeper ones: 3584 x 3584 33.8 -> 25.5 (192; at 170 24.3 against
+        # 27.1), 5120 x 5120 54.8 -> 32.6 (256), 38.6 -> 33.0 (247)
         if (kind == "resid" and 3584 <= K <= 5632 and N >= 3584 and N % 128 == 0 and M > (32 if K > FUSED_MAX_K else 64)
                 and not (M > 128 and _WO256 != "0" and K <= FUSED_MAX_K and nbytes <= FUSED_M256_RESID_T22_MAX_BYTES
                          and (N // 64) * ((m_tiles + 1) // 2) >= 192) and not _tuned(M, N, K)):
-            return "skinny" if M <= 128 else "block"
-    if kind == "planes" and K <= FUSED_MAX_K and M > 128 and use_fused(M, N, K, "resid"):
-        return "skinny"               # 4096 x 4096 on the tile kernel's K split 36.3 / 33.8 -> 27.5 / 28.8 (192 / 256 rows)
-    if kind == "qkv" and not _tuned(M, N, K):
-        # the tile kernel ends in rope + append; the library needs a launch for that, and has no measured solution here: 4608 x 3584
-        # 25.0 / 27.8 / 35.2 / 40.5 -> 18.0 / 22.8 / 27.3 / 32.0 (96 / 128 / 192 / 256 rows), 6144 x 4096 28.5 -> 25.0 (96),
-        # 7168 x 5120 31.5 / 34.7 -> 26.0 / 32.2 (64 / 96)
+            # (6912 x 3968, 31 slices: 28.6 against 47.6; 6784 x 4992, 689 workgroups, 32.5 against 37.9)
+            if M <= 128 and _slices("skinny", N, K) <= 15 and -(-N // 128) * _slices("skinny", N, K) <= 1.6 * CUS:
+                return "skinny"
+            if M > 128 and (nice or (K >= 5120 and N >= 4608)):
+                return "block"
+    # 4096 x 4096 on the tile kernel's K split 36.3 / 33.8 -> 27.5 / 28.8 (192 / 256 rows), 3456 x 1664 94 -> 32 (213); the wide ones
+    # only in one round (5632 x 768, 264 workgroups, 22.7 against 30.8)
+    if (kind == "planes" and K <= FUSED_MAX_K and M > 128 and use_fused(M, N, K, "resid")
+            and (N <= 4608 or -(-N // 128) * _slices("skinny", N, K) <= CUS)):
+        return "skinny"
+    if kind == "qkv" and K <= 5632 and N >= 4096 and n_tiles * m_tiles >= 100:
+        # the tile kernel ends in rope + append; the library needs a launch for that: 4608 x 3584 25.0 / 27.8 -> 18.0 / 22.8 (96 / 128
+        # rows), 6144 x 4096 28.5 -> 25.0 (96), 26.4 -> 25.0 (128), 7168 x 5120 31.5 / 34.7 -> 26.0 / 32.2 (64 / 96).  The 8B one is
+        # level at exactly 64 rows (22.8 / 22.2; 23.1 / 21.1 at 47): the library, so that 64- and 256-row steps need no second copy
         lim = FUSED_QKV_MAX_L2_BYTES if K <= FUSED_MAX_K else FUSED_QKV_DEEP_MAX_L2_BYTES
-        if K <= 5632 and N >= 4096 and m_tiles * nbytes <= lim and (N // 32) * m_tiles >= 100:
-            return "fused"
+        level = M == 64 and 3584 < K <= FUSED_MAX_K and 1.25 < _last_round(n_tiles * m_tiles) < 1.5
+        if M <= 128 and m_tiles * nbytes <= lim:
+            return None if level else "fused"
+        # above 128 rows where the library is slow: multiples of 32 (4608 x 3584 35.2 / 40.5 -> 27.3 / 32.0 at 192 / 256), 129..159
+        # (6144 x 4096 44.8 -> 29.5; not the wide ones: 8192 x 3200 28.1 against 36.2) and 193..223 narrow (4608 x 3584 38.0 -> 28.1,
+        # 4224 x 4224 40.2 -> 33.7; 5504 x 3584 29.7 against 33.2)
+        if M > 128 and m_tiles * nbytes <= lim and not _tuned(M, N, K):
+            if n_tiles * m_tiles <= (6.5 if nice else 4.5 if M < 160 else 4.05 if m_tiles == 7 else 0) * CUS:
+                return "fused"
     # ... and where its budget ends, the block kernel ahead of the rope launch: 7168 x 5120 39.3 / 48.5 / 57.4 -> 36.6 / 40.3 / 43.8
-    # (128 / 192 / 256), 6144 x 4096 39.0 -> 35.6 (192)
+    # (128 / 192 / 256), 6144 x 4096 39.0 -> 35.6 (192), 36.8 -> 33.7 (224)
     if kind == "plain" and 96 < M and 4096 <= K <= 5632 and N % 128 == 0 and 40 <= tiles <= 64 and not _tuned(M, N, K):
-        return "block"
+        # (other row counts than multiples of 32 where it is deep, 7168 x 5120 38.5 -> 36.5 at 103; 5120 x 4096 is level, 22.9 at 97)
+        if (K >= 4608 or M >= 192) if nice else tiles <= 56 and (K >= 5120 or (tiles == 40 and M <= 128)):
+            return "block"
     return None
 
 

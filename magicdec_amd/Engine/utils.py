@@ -29,7 +29,10 @@ def enable_tuned_gemms(path=None):
     tunable.enable(True)
     tunable.tuning_enable(False)
     tunable.set_filename(str(Path(tempfile.gettempdir()) / "magicdec_tunableop_unused.csv"))   # never rewrite the table
-    return bool(tunable.read_file(str(path)))
+    accepted = bool(tunable.read_file(str(path)))
+    from .gemm_policy import tuned_table
+    tuned_table(str(path) if accepted else None)         # (the dispatch counts on the solutions that are in use)
+    return accepted
 
 
 def setup_seed(seed):

@@ -12,10 +12,10 @@ SHAPES = [(33, 20480, 256, "plain", "block"), (128, 32768, 768, "plain", "block"
           (97, 5120, 4096, "plain", "block"), (256, 8192, 5632, "plain", "block"),
           (3, 14336, 2304, "swiglu", "fused"), (32, 15040, 4096, "swiglu", "fused"),
           (65, 32896, 256, "swiglu", "skinny"), (128, 37888, 512, "swiglu", "skinny"),
-          (1, 3584, 8448, "resid", "split"), (32, 4096, 14336, "resid", "split"), (33, 3584, 18944, "resid", "skinny"), (1, 2048, 4224, "resid", "skinny"), (32, 2048, 5632, "resid", "skinny"),
+          (1, 4096, 8192, "resid", "split"), (32, 4096, 14336, "resid", "split"), (33, 3584, 18944, "resid", "skinny"), (1, 2048, 4224, "resid", "skinny"), (32, 2048, 5632, "resid", "skinny"),
           (33, 2048, 5632, "resid", "fused"), (128, 2048, 4224, "resid", "fused"), (31, 5120, 5120, "resid", "fused"),
           (65, 3584, 3584, "resid", "skinny"), (33, 5120, 5120, "resid", "skinny"), (128, 5120, 4096, "resid", "skinny"), (129, 5120, 5120, "resid", "block"), (255, 5120, 5120, "resid", "block"),
-          (1, 2048, 7680, "planes", "skinny"), (64, 1056, 4224, "planes", "skinny"), (65, 2048, 7680, "planes", "skinny"), (256, 2048, 4224, "planes", "skinny"),
+          (1, 2048, 7680, "planes", "skinny"), (64, 1056, 4224, "planes", "skinny"), (65, 2048, 7680, "planes", "skinny"), (256, 2176, 5120, "planes", "skinny"),
           (129, 4096, 4096, "planes", "skinny"), (256, 4096, 4096, "planes", "skinny")]
 
 

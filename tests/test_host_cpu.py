@@ -1475,3 +1475,48 @@ def test_a_refused_prompt_leaves_the_weights_released(cpu_ops_patched, prompt):
     with pytest.raises((ValueError, RuntimeError)):
         e.encode(torch.randint(4, 128, (2, 256 if prompt == "refused" else 160)))
     assert not m._on_demand and m._released == released and not m.skip_head
+
+
+# dispatch of linears where a rule drawn from the shapes beside it picked the slower kernel: (rows, N, K, kind, kernel; us of it / of
+# the other one)
+MEASURED = [(2, 4096, 11008, "resid", "skinny"),        # 23.1 / 26.8 K split (half a round of workgroups)
+            (30, 5120, 13824, "resid", "skinny"),       # 33.3 / 42.2 K split (a round and a quarter)
+            (22, 2048, 14720, "resid", "skinny"), (1, 3584, 8448, "resid", "skinny"),     # 19.6 / 25.4, 17.1 / 21.2
+            (31, 4096, 14336, "resid", "split"), (1, 4096, 18432, "resid", "split"),      # 27.2 / 28.4, 30.3 / 32.4
+            (57, 32000, 2048, "plain", "skinny"), (64, 32000, 4096, "plain", "skinny"),   # 27.0 / 30.6, 51.2 / 53.4 block
+            (79, 32000, 4096, "plain", "block"), (109, 30208, 4096, "plain", "skinny"),   # 52.5 / 56.6, 52.4 / 56.4
+            (64, 32000, 768, "plain", "block"), (80, 21504, 2048, "plain", "lib"),        # 15.3 / 19.4, 26.5 / 29.1
+            (13, 16896, 4224, "plain", "skinny"), (13, 115328, 1280, "plain", "skinny"),  # 27.5 / 32.4, 49.8 / 56.6 tile
+            (26, 128256, 2048, "plain", "skinny"), (5, 128256, 2048, "plain", "fused"),   # 99.2 / 101, 81.2 / 91.1
+            (237, 6144, 4096, "qkv", "lib"), (192, 6144, 4096, "plain", "block"),         # 33.1 / 37.6 block, 34.7 / 40.1
+            (234, 4608, 3584, "qkv", "lib"), (192, 4608, 3584, "qkv", "fused"),           # 28.5 / 32.4, 27.3 / 35.2
+            (143, 6144, 4096, "qkv", "fused"), (156, 8192, 3200, "qkv", "lib"),           # 29.5 / 44.8, 28.1 / 36.2
+            (128, 6144, 4096, "qkv", "fused"), (256, 6144, 4096, "qkv", "lib"),           # 25.0 / 26.4, 32.1 / 37.5
+            (170, 3584, 3584, "resid", "lib"), (192, 3584, 3584, "resid", "block"),       # 24.3 / 27.1, 25.5 / 33.8
+            (64, 4608, 4352, "resid", "skinny"), (106, 6912, 3968, "resid", "fused"),     # 18.9 / 30.8 tile, 28.6 / 47.6 skinny
+            (256, 2048, 4224, "planes", "lib"), (41, 896, 7680, "planes", "lib"),         # 24.3 / 44.9, 15.5 / 19.8
+            (229, 2048, 7680, "planes", "skinny"), (20, 18432, 5120, "swiglu", "skinny"), # 28.0 / 31.0, 35.5 / 39.6
+            (25, 24576, 4096, "swiglu", "fused"), (2, 61312, 1152, "swiglu", "skinny")]   # 37.2 / 40.4, 26.9 / 28.6
+
+
+@pytest.mark.parametrize("M,N,K,kind,kernel", MEASURED)
+def test_dispatch_between_the_tuned_shapes(M, N, K, kind, kernel):
+    from magicdec_amd.Engine import gemm_policy as g
+    if g.mode() != "auto" or g.fused_mode() != "auto" or g.block_mode() != "auto" or os.environ.get("MAGICDEC_SPLIT", "auto") != "auto":
+        pytest.skip("policy overridden by the environment")
+    how = g.choose(M, N, K, kind == "swiglu", False, True, kind)
+    assert kernel == ("split" if how != "fused" and g.use_split(M, N, K, kind) else how)
+
+
+def test_tuned_solutions_count_where_they_are_in_use(tmp_path, monkeypatch):
+    """Only lines that name a solution, and only of a table that PyTorch took."""
+    from magicdec_amd.Engine import gemm_policy as g
+    monkeypatch.setattr(g, "_TABLE", g._TABLE)
+    monkeypatch.setattr(g, "_TUNED", None)
+    table = tmp_path / "t.csv"
+    table.write_text("Validator,PT_VERSION,0\nGemmTunableOp_BFloat16_TN,tn_6144_256_4096_ld_4096_4096_6144,Gemm_Rocblas_1,0.02\n"
+                     "GemmTunableOp_BFloat16_TN,tn_6144_192_4096_ld_4096_4096_6144,Default,0.02\n")
+    g.tuned_table(str(table))
+    assert g._tuned(256, 6144, 4096) and not g._tuned(192, 6144, 4096) and not g._tuned(128, 6144, 4096)
+    g.tuned_table(None)
+    assert not g._tuned(256, 6144, 4096) and g.choose(256, 6144, 4096, False, False, True, "plain") == "block"
