@@ -84,16 +84,23 @@ def skinny_absorbs_norm(M: int) -> bool:
     return _SKINNY_NORM != "0" and M <= SKINNY_NORM_MAX_M
 
 
+def _changed():
+    """A switch or the table of tuned solutions is another one."""
+    _measured.cache_clear()
+
+
 def set_mode(mode: str):
     global _MODE
     assert mode in ("auto", "hip", "lib")
     _MODE = mode
+    _changed()
 
 
 def set_fused(mode: str):
     global _FUSED
     assert mode in ("auto", "0", "1")
     _FUSED = mode
+    _changed()
 
 
 def mode() -> str:
@@ -149,6 +156,7 @@ def tuned_table(path):
     so that none of its solutions is in use."""
     global _TABLE, _TUNED
     _TABLE, _TUNED = path, None
+    _changed()
 
 
 def _tuned(M: int, N: int, K: int) -> bool:
@@ -190,6 +198,7 @@ def _skinny_one_round(N: int, K: int) -> bool:
     return 0.8 * CUS < -(-N // 128) * _slices("skinny", N, K) <= CUS
 
 
+@functools.lru_cache(maxsize=16384)      # (asked three times for every linear of a step that is not captured; _changed clears it)
 def _measured(M, N, K, kind, absorbs_norm):
     """The kernel for the shapes where the general rules below (drawn for the 1B and 8B models at 32, 64, 128 and 256 rows) were
     measured to pick a slower one of the framework's own kernels, or the library where one of them is faster: "fused" | "block" |

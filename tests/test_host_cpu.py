@@ -1508,9 +1508,10 @@ def test_dispatch_between_the_tuned_shapes(M, N, K, kind, kernel):
     assert kernel == ("split" if how != "fused" and g.use_split(M, N, K, kind) else how)
 
 
-def test_tuned_solutions_count_where_they_are_in_use(tmp_path, monkeypatch):
+def test_tuned_solutions_count_where_they_are_in_use(tmp_path, monkeypatch, request):
     """Only lines that name a solution, and only of a table that PyTorch took."""
     from magicdec_amd.Engine import gemm_policy as g
+    request.addfinalizer(g._changed)
     monkeypatch.setattr(g, "_TABLE", g._TABLE)
     monkeypatch.setattr(g, "_TUNED", None)
     table = tmp_path / "t.csv"
@@ -1520,3 +1521,22 @@ def test_tuned_solutions_count_where_they_are_in_use(tmp_path, monkeypatch):
     assert g._tuned(256, 6144, 4096) and not g._tuned(192, 6144, 4096) and not g._tuned(128, 6144, 4096)
     g.tuned_table(None)
     assert not g._tuned(256, 6144, 4096) and g.choose(256, 6144, 4096, False, False, True, "plain") == "block"
+
+
+def test_the_dispatch_is_remembered_until_a_switch_changes():
+    """A rule is worked out once per shape (a linear of a step asks three times), and anew behind a switch."""
+    from magicdec_amd.Engine import gemm_policy as g
+    if g.mode() != "auto" or g.fused_mode() != "auto":
+        pytest.skip("policy overridden by the environment")
+    ask = lambda: g.choose(160, 4096, 4096, False, False, True, "planes")
+    g._changed()
+    first = ask()
+    worked = g._measured.cache_info().misses
+    assert worked and ask() == first and g._measured.cache_info().misses == worked
+    try:
+        g.set_fused("0")
+        assert g._measured.cache_info().currsize == 0
+        assert ask() != first
+    finally:
+        g.set_fused("auto")
+    assert ask() == first
