@@ -33,6 +33,7 @@ PREFILL_ROWS = 16384   # rows of one prefill step where the portion is free to c
 # 2 969 -> 1 170.  8192 is what 64 requests had already; a layer's activations take 1.4 GB there on a 32B model.
 PROMPT_ROWS = 8192
 PROMPT_WINDOWS = 512 << 20     # bytes of one pass's StreamingLLM windows: 64 portions at a budget of 1 900 rows of 8 heads of 128
+PROMPT_MEMORY = 0.8            # share of the free device memory that a portion's activations may take; beyond it portions get shorter
 
 
 def default_kv_layout():
@@ -212,18 +213,46 @@ class _BackendBase:
         B = self.batch_size
         return sorted({B * int(n) for n in (1,) + ((2,) if two_token_step else ()) + tuple(per_request) if n})
 
+    def _rows_that_fit(self, rows, row_bytes=0, fixed=0):
+        """`rows` of a prompt, or as many as the device's free memory holds: their activations in a layer (and row_bytes each, and `fixed`)
+        beside the row-major weights that the prompt brings back.  The same on every rank of a tensor-parallel group."""
+        dev, m = torch.device(self.device), self.model
+        if dev.type != "cuda":
+            return rows
+        taken, each = getattr(m, "released_bytes", 0) + fixed, m.prompt_row_bytes() + row_bytes
+        free = torch.cuda.mem_get_info(dev)[0]
+        if PROMPT_MEMORY * (free - taken) < rows * each:         # (what the allocator holds unused: its statistics take 50 us and more)
+            free += torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
+        rows = min(rows, max(0, int(PROMPT_MEMORY * (free - taken) // each)))
+        group = getattr(m, "process_group", None)
+        if group is not None:
+            import torch.distributed as dist
+            least = torch.tensor([rows], dtype=torch.int32, device="cuda" if dist.get_backend(group) == "nccl" else "cpu")
+            dist.all_reduce(least, op=dist.ReduceOp.MIN, group=group)
+            rows = int(least.item())
+        return rows
+
     def _portions(self, seq_len):
         """The portions [(first token, tokens)] of a prompt whose keys all stay in the cache: any division gives every token the same
-        keys, so portions are as long as the matrix products want them.  An fp8 cache's first CHUNK, which sets its scales, stays one."""
+        keys, so portions are as long as the matrix products want them, and the memory holds.  An fp8 cache's first CHUNK, which sets its
+        scales, stays one."""
         if self.mapped or torch.device(self.device).type == "cpu":       # (the CPU's products round by their row counts)
             chunk = self.prefill_chunk
             return [(a, min(chunk, seq_len - a)) for a in range(0, seq_len, chunk)]
+        rows = self._rows_that_fit(PROMPT_ROWS) if seq_len > CHUNK and PROMPT_ROWS > self.batch_size * CHUNK else 0
+        return self._divide(seq_len, rows // (self.batch_size * CHUNK),
+                            self.model.layers[0].attention.kv_cache.scales("kv_cache") is not None)
+
+    @staticmethod
+    def _divide(seq_len, most, alone):
+        """Portions of a prompt: whole CHUNKs, `most` (at least one) to a portion, as even as they go, and what is left; `alone`: the
+        first CHUNK is a portion of its own."""
         chunks, at = -(-seq_len // CHUNK), 0
         out = []
-        if chunks > 1 and self.model.layers[0].attention.kv_cache.scales("kv_cache") is not None:
+        if chunks > 1 and alone:
             out, at, chunks = [(0, CHUNK)], CHUNK, chunks - 1
         # the last chunk rides along unless that takes a portion more: 8192 rows are whole rounds of the library's tiles, 8324 are not
-        first, most = at, max(1, PROMPT_ROWS // (self.batch_size * CHUNK))
+        first, most = at, max(1, most)
         parts = max(min(1, chunks), -(-(chunks - 1) // most))
         if chunks > parts * most:
             chunks -= 1
@@ -590,8 +619,10 @@ class _StreamingMixin:
         num_chunks = (seq_len + CHUNK - 1) // CHUNK
         # chunks to a pass (md_streaming_windows): PROMPT_ROWS rows and PROMPT_WINDOWS bytes of them (one where the CPU's products round by their row counts)
         cache = getattr(self.model.layers[0].attention.kv_cache, which)
-        most = 1 if cache.device.type == "cpu" else min(PROMPT_ROWS // (B * CHUNK),
-                                                        PROMPT_WINDOWS // (cache.numel() * cache.element_size()))
+        nbytes = cache.numel() * cache.element_size()
+        most = 1 if cache.device.type == "cpu" else min(PROMPT_ROWS // (B * CHUNK), PROMPT_WINDOWS // nbytes)
+        if most > 1 and num_chunks > 1:               # (a chunk's window, and the cache behind the pass, are copies of the cache)
+            most = self._rows_that_fit(most * B * CHUNK, nbytes / (B * CHUNK), nbytes) // (B * CHUNK)
         passes = -(-num_chunks // max(1, most))
         ctx = 0                                       # host mirror of the (capped) cache length
         with self._prefilling():

@@ -521,6 +521,14 @@ class Transformer(nn.Module):
             w.data = rows
         self._released.discard(k)
 
+    def prompt_row_bytes(self):
+        """Bytes of one row of a prompt in a layer: the residual stream and its norm, in and out, beside the widest stage -- gate | up and
+        their product, or the projections, the rotated queries and the attention's rows."""
+        c, layer = self.config, self.layers[0]
+        gated = 2 * layer.feed_forward.w1.weight.shape[0]
+        return self.tok_embeddings.weight.element_size() * (
+            4 * c.dim + max(3 * gated // 2, layer.attention.wqkv.weight.shape[0] + 2 * c.n_head * c.head_dim))
+
     _on_demand = False       # during a prefill: a released tensor that a library GEMM asks for comes back until release_rowmajor()
 
     def restore_on_demand(self, on):

@@ -62,3 +62,31 @@ def test_longer_portions(which, kv, batch, prompt, monkeypatch):
     for x, y in zip(a["kept"], b["kept"]):
         near = (x - y).norm(dim=-1) <= 0.05 * y.norm(dim=-1)
         assert near.double().mean() > 0.8
+
+
+@pytest.mark.parametrize("which", ["plain", "draft", "stream_draft"])
+def test_portions_where_memory_is_short(which, monkeypatch):
+    """With little free memory a prompt runs in single chunks, as it would without longer portions: the same bits."""
+    import magicdec_amd.Engine.backend_core as core
+    from magicdec_amd.Engine.model_core import transformer_configs
+    ids = torch.randint(4, 512, (2, 800), generator=torch.Generator().manual_seed(5)).to(DEV)
+    seen = []
+    for short in (True, False):
+        if which == "stream_draft":
+            from magicdec_amd.Engine.StreamingLLM.backend_draft import LMBackend_Draft
+            engine("plain", "bf16", 1, 256)                            # (registers the configuration)
+            e = LMBackend_Draft(dtype=torch.bfloat16, device=DEV)
+            e.load_model("none/portions-test/model.pth", use_tp=False)
+            e.setup_caches(max_batch_size=2, draft_budget=257)
+        else:
+            e = engine(which, "bf16", 2, 1024)
+        with monkeypatch.context() as m:
+            if short:
+                m.setattr(torch.cuda, "mem_get_info", lambda dev=None: (0, 1 << 38))
+                m.setattr(torch.cuda, "memory_reserved", lambda dev=None: torch.cuda.memory_allocated(dev) + 3 * 128 * e.model.prompt_row_bytes())
+            else:
+                m.setattr(core, "PROMPT_ROWS", 0)
+            tokens = e.encode(ids)
+        kvs = [b.attention.kv_cache for b in e.model.layers]
+        seen.append([tokens, e.model._last_logits] + [c.kv_cache for c in kvs] + ([c.draft_cache for c in kvs] if which == "draft" else []))
+    assert all(torch.equal(x, y) for x, y in zip(*seen))

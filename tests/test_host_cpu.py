@@ -1540,3 +1540,48 @@ def test_the_dispatch_is_remembered_until_a_switch_changes():
     finally:
         g.set_fused("auto")
     assert ask() == first
+
+
+def test_portions_of_a_prompt():
+    """Every division: in order and whole, each portion from a page's start, no longer than asked (one chunk at least), as few as that
+    allows, and an fp8 cache's first chunk by itself."""
+    from magicdec_amd.Engine.backend_core import CHUNK, _BackendBase
+    for most in (0, 1, 2, 3, 7, 64):
+        for seq in [1, 127, 128, 129, 255, 256, 257, 384, 1000, 1024, 1025, 8191, 8192, 8193, 8320, 8321] + list(range(1, 1500, 37)):
+            for alone in (False, True):
+                parts = _BackendBase._divide(seq, most, alone)
+                assert [a for a, _ in parts] == [0] + [a + n for a, n in parts[:-1]] and sum(parts[-1]) == seq
+                assert all(a % CHUNK == 0 and 0 < n <= max(1, most) * CHUNK for a, n in parts), (seq, most, parts)
+                chunks = -(-seq // CHUNK)
+                if alone and chunks > 1:
+                    assert parts[0] == (0, CHUNK)
+                    parts, chunks = parts[1:], chunks - 1
+                # the last chunk may be by itself, the others take no portion more than they need
+                assert len(parts) <= -(-(chunks - 1) // max(1, most)) + 1
+                if most <= 1:
+                    assert len(parts) == chunks
+
+
+def test_portions_shrink_with_the_free_memory(monkeypatch):
+    """The rows of a prompt's portion: what 8192 rows want where there is room, what fits where there is not, none beside weights that
+    have to come back first."""
+    from types import SimpleNamespace
+    from magicdec_amd.Engine import backend_core as core
+    e = core._BackendBase(device="cuda:0")
+    e.batch_size = 2
+    e.model = SimpleNamespace(prompt_row_bytes=lambda: 1000, released_bytes=0, process_group=None,
+                              layers=[SimpleNamespace(attention=SimpleNamespace(kv_cache=SimpleNamespace(scales=lambda which: None)))])
+    free = [0]
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda dev=None: (free[0] - 3_000, 1 << 30))      # (and 3 000 in the allocator)
+    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda dev=None: 5_000)
+    monkeypatch.setattr(torch.cuda, "memory_allocated", lambda dev=None: 2_000)
+    longest = lambda: max(n for _, n in e._portions(20_000))
+    free[0] = 1 << 30
+    assert e._rows_that_fit(8192) == 8192 and longest() == 32 * 128
+    free[0] = 1_000_000 / core.PROMPT_MEMORY
+    assert e._rows_that_fit(8192) == 1000 and longest() == 3 * 128
+    assert e._rows_that_fit(8192, row_bytes=1000, fixed=500_000 / core.PROMPT_MEMORY) == 250
+    e.model.released_bytes = 900_000 / core.PROMPT_MEMORY
+    assert e._rows_that_fit(8192) == 100 and longest() == 128
+    e.model.released_bytes = 1 << 30
+    assert e._rows_that_fit(8192) == 0 and longest() == 128
