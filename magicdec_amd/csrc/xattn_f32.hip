@@ -264,12 +264,14 @@ __global__ __launch_bounds__(256, (f32_waves_per_simd<DK, DV, QT, KT, SHARED>())
                         for (int qt = 0; qt < QT; ++qt) o[qt][v] = __builtin_amdgcn_mfma_f32_16x16x4f32(va, pb[qt][e], o[qt][v], 0, 0, 0);
                     }
             }
-        } else {                             // a value that a row does not see must not reach it as 0 * infinity
+        } else {
+            // a value that a row does not see must not reach it as 0 * infinity; one that it sees does, also with a weight that underflowed
             for (int k = 0; k < KT; ++k)
 #pragma unroll
                 for (int qt = 0; qt < QT; ++qt) {
                     const float w = sp[(qt * 16 + lq) * PP + k];
-                    if (w != 0.f) {
+                    const int at = pos0 + (R0 + qt * 16 + lq) / g, kp = t * KT + k;
+                    if (kp >= (at / p.chunk) * p.chunk && kp <= min(at, cap - 1)) {
 #pragma unroll
                         for (int v = 0; v < NV; ++v)
 #pragma unroll

@@ -53,6 +53,22 @@ def test_a_value_that_is_no_number_reaches_only_rows_that_see_it(ops):  # noqa: 
         assert float((got[:70].double() - want[:70]).abs().max()) <= TOL * float(want.abs().max())
 
 
+@pytest.mark.parametrize("chunk", [0, 65])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_a_value_with_a_weight_of_zero(ops, bad, chunk):  # noqa: F811
+    """Scores of up to 200 leave most weights at 0 in fp32: 0 times an infinity that a row sees is no number, as in the plain kernel --
+    the same elements of both are numbers, over whole prompts and for a few rows (kv splits)."""
+    for KH, D, n in ((2, 64, 300), (2, 64, 3), (1, 256, 300), (1, 128, 1)):
+        spec, rows, _ = attention_case(ops, 4, KH, D, 64, chunk, 3, F32, [300], score=200.0)
+        v0 = (spec.H + spec.KH) * spec.D
+        rows[0][270, v0 + 5], rows[0][70, v0 + 9] = bad, -bad
+        s = Seqs(ops, spec, F32, [300])
+        s.attend(rows[0][:300 - n], [0], [0], [300 - n]) if n < 300 else None
+        got, plain = (s.attend(rows[0][300 - n:], [0], [300 - n], [n], plain=x) for x in (False, True))
+        assert torch.equal(torch.isfinite(got), torch.isfinite(plain)) and not torch.isfinite(plain).all()
+        assert torch.allclose(got[torch.isfinite(plain)], plain[torch.isfinite(plain)], rtol=0, atol=TOL * 10)
+
+
 def test_16_bit_pages_with_an_unknown_bound(ops):  # noqa: F811
     """Without a bound on the scores the bf16 kernels do not apply: same sums as the plain kernel, rounded once."""
     for H, KH, D, n in ((8, 2, 64, 100), (4, 4, 96, 5)):
