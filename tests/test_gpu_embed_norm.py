@@ -30,3 +30,34 @@ def test_outside():
         assert not ops.embed_rmsnorm_supported(*bad)
         with pytest.raises(ValueError):
             ops.embed_rmsnorm(*bad, 1e-5)
+
+
+@pytest.mark.parametrize("graphs", [False, True])
+def test_an_id_outside_the_table_stays_in_its_request(graphs):
+    """The fixed-batch engines look no ids up on the host: one outside the table leaves its own request without numbers (token 0) and
+    the others as they are, in a prompt and in a step."""
+    from magicdec_amd.Engine.model_core import transformer_configs
+    from magicdec_amd.Engine.SnapKV.backend import LMBackend
+    transformer_configs["embed-test"] = dict(block_size=512, n_layer=2, n_head=2, n_local_heads=1, dim=128, intermediate_size=256, vocab_size=64)
+    g = torch.Generator().manual_seed(0)
+    ids, step = torch.randint(4, 64, (3, 150), generator=g), torch.randint(4, 64, (3, 1), generator=g)
+    seen = []
+    for bad in (None, 64, -3):
+        e = LMBackend(dtype=BF, device=DEV)
+        e.load_model("none/embed-test/model.pth", use_tp=False)
+        if graphs:
+            e.compile()
+        e.setup_caches(max_batch_size=3, max_seq_length=256)
+        prompt, one = ids.clone(), step.clone()
+        if bad is not None:
+            prompt[1, 70] = bad
+        tokens, logits = e.encode(prompt.to(DEV)), e.model._last_logits.view(3, 22, -1).clone()
+        if bad is not None:
+            one[1] = bad
+        for _ in range(2):
+            nxt = e.inference(one.to(DEV), benchmark=True)
+        seen.append((tokens, logits, nxt))
+    for tokens, logits, nxt in seen[1:]:
+        assert logits[1].isnan().all() and not tokens[1].any() and int(nxt[1]) == 0
+        for b in (0, 2):
+            assert torch.equal(logits[b], seen[0][1][b]) and torch.equal(tokens[b], seen[0][0][b]) and torch.equal(nxt[b], seen[0][2][b])
