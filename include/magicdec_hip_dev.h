@@ -25,7 +25,7 @@ void md_debug_set_prefill_mfma32(int kt);
 void md_debug_set_prefill_kt(int kt, int nw);
 /* md_linear: split-K policy (workgroups to aim for) */
 void md_debug_set_gemm_target_blocks(int n);
-/* md_linear: wavefronts per workgroup, 4 | 6 | 7 forced (bit-identical results); 0 = the balance rule (plan_of) */
+/* md_linear: wavefronts per workgroup, 4..7 forced (bit-identical results); 0 = the balance rule (plan_of) */
 void md_debug_set_gemm_waves(int nw);
 /* md_linear: W prefetch ring depth of the four-wave, <= 64-row, bf16 form: 16 = the deep ring (bit-identical results, measured
  * equal or 1-3 % slower: profiles/r06_ring_depth_ab.txt); 0 / 8 = the rule (8) */

@@ -475,11 +475,10 @@ class Transformer(nn.Module):
         return any(M > 256 or "lib" in self._decode_hows(role, N, K, False, M) for M in self.decode_rows)
 
     def release_rowmajor(self):
-        """After prefill: free the row-major tensor of every weight that decode only ever reads in the streaming layout
-        (every packed weight used to be held twice, 16.9 GB at configs[2]).  The Parameter objects stay
-        (same id, shape and dtype: a zero-stride view of one element) so that every look-up keyed on them keeps working;
-        restore_rowmajor() re-materialises them from the streaming copy before the next prefill.  MAGICDEC_KEEP_ROWMAJOR=1
-        switches this off."""
+        """After prefill: free the row-major tensor of every weight that decode only ever reads in the streaming layout (16.9 GB of an
+        8B target and a 1B draft).  The Parameter objects stay (same id, shape and dtype: a zero-stride view of one element) so that
+        every look-up keyed on them keeps working; a prompt's products bring back those that they ask for (restore_on_demand,
+        _resident), each from its streaming copy.  MAGICDEC_KEEP_ROWMAJOR=1 switches this off."""
         import os
         if not getattr(self, "_packed", None) or os.environ.get("MAGICDEC_KEEP_ROWMAJOR", "0") == "1":
             return 0
@@ -503,7 +502,7 @@ class Transformer(nn.Module):
         return freed
 
     def restore_rowmajor(self):
-        """Every released row-major tensor back from its streaming-layout copy."""
+        """Every released row-major tensor back from its streaming-layout copy, at once (the engines restore on demand)."""
         for k in list(getattr(self, "_released", ())):
             self._restore(k)
 

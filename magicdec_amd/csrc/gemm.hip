@@ -404,7 +404,7 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const GemmParams p) 
 }
 
 int g_target_blocks = 256;   // split-K is chosen so that about this many workgroups exist (1 per CU: measured best)
-int g_force_nw = 0;          // dev knob (md_debug_set_gemm_waves): 0 = the rule below, 4 / 6 / 7 = forced
+int g_force_nw = 0;          // dev knob (md_debug_set_gemm_waves): 0 = the rule below, 4..7 = forced
 
 int pick_splits(int n_blocks, int K) {
     const int nslab = K / kSlabK;
@@ -459,7 +459,7 @@ SkinnyPlan plan_of(int ntiles, int K, bool allow_nw) {
     }
     const int kCUs = cus_of[devid];
     if (kCUs <= 0) return pl;
-    if (g_force_nw == 6 || g_force_nw == 7) {
+    if (g_force_nw >= 5) {
         pl.nw = g_force_nw;
         return pl;
     }
@@ -582,7 +582,7 @@ int md_internal_launch_skinny_reduce(const float* partial, int S, int M, int N, 
 
 #ifdef MD_DEV_KNOBS
 extern "C" void md_debug_set_gemm_target_blocks(int n) { g_target_blocks = n > 0 ? n : 256; }
-extern "C" void md_debug_set_gemm_waves(int nw) { g_force_nw = (nw == 4 || nw == 6 || nw == 7) ? nw : 0; }
+extern "C" void md_debug_set_gemm_waves(int nw) { g_force_nw = nw >= 4 && nw <= 7 ? nw : 0; }
 extern "C" void md_debug_set_gemm_ring(int rd) { g_force_rd = (rd == 8 || rd == 16) ? rd : 0; }
 #endif
 

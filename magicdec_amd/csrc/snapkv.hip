@@ -1,4 +1,4 @@
-// SnapKV select (K6, row a8 of SURVEY.md section 8) for gfx950.
+// SnapKV select for gfx950.
 //
 // reference: Attention.gen_draft_kv  Engine/SnapKV/model.py:389-439
 // restated (bit-exact vs the reference on CPU) in oracle/magicdec_ref.py:snapkv_scores.
@@ -13,6 +13,7 @@
 //   draft rows = K,V[indices] ++ K,V[S-W:S]
 //
 // Seven small launches, none on the timed decode path (once per prefill per layer):
+//   tab     : the table of exponentials (below)
 //   stats   : row max / sum-exp partials per column chunk   (MFMA scores; float64 sums)
 //   finalize: per-row (max, 1 / sum) of the whole context from the chunk partials
 //   accum   : recompute scores, p, 8-row group sums, bf16 chunk accumulation
@@ -124,12 +125,11 @@ __device__ __forceinline__ double exp_neg(double x) {
     return ldexp(q, (int)k);
 }
 
-// ---- round 4: the softmax of the select without a float64 exponential per element.
+// ---- the softmax of the select without a float64 exponential per element.
 // The reference's scores are bf16 VALUES (model.py:411: a bf16 einsum), i.e. one of 65 536 numbers, and the
 // probabilities must be correctly rounded bf16(exp(s - M) / Z) (see "Rounding sequence" above: an fp32 evaluation with
-// another summation order flips ~1e-4 of those roundings).  Rounds 1-3 evaluated exp() in float64 per element: a
-// billion OCML calls per layer at the BASELINE shape, 0.21 TB/s of K bytes = 2.6 % of the HBM roofline (VERDICT r3 weak
-// #3).  Now exp(v) of every bf16 value with 2^-14 <= |v| < 2^9 sits in a float64 table in LDS (filled with OCML's exp once
+// another summation order flips ~1e-4 of those roundings).  exp() in float64 per element is a billion OCML calls per
+// layer for 64 requests of 16 000 tokens, 0.21 TB/s of K bytes = 2.6 % of the HBM peak.  So exp(v) of every bf16 value with 2^-14 <= |v| < 2^9 sits in a float64 table in LDS (filled with OCML's exp once
 // per call): the row sum is  sum_i T[s_i]  (reference 0: e^512 * 65 536 columns is far below the float64 range) and a
 // probability is  T[s] * (exp(-M) / Z)  -- one LDS gather and one f64 multiply.  Of the few scores outside the table, tiny
 // ones (|s| < 2^-14) are a short polynomial, the others (|s| >= 512, masked) take the lean exp_neg() above against a running maximum, so

@@ -1585,3 +1585,32 @@ def test_portions_shrink_with_the_free_memory(monkeypatch):
     assert e._rows_that_fit(8192) == 100 and longest() == 128
     e.model.released_bytes = 1 << 30
     assert e._rows_that_fit(8192) == 0 and longest() == 128
+
+
+def test_weights_come_back_on_demand():
+    """Between restore_on_demand(True) and the next release, a released weight that is asked for stays: the bits it had, w1 and w3 views
+    of w13 again; without it a product gets a tensor of its own and the weight stays released."""
+    from magicdec_amd.Engine import model_core
+    model_core.transformer_configs["on-demand"] = dict(block_size=256, n_layer=1, vocab_size=128, n_head=4, n_local_heads=2, dim=256, intermediate_size=512)
+    try:
+        m = model_core.Transformer.from_name("on-demand").to(torch.bfloat16)
+    finally:
+        model_core.transformer_configs.pop("on-demand", None)
+    for p in m.parameters():
+        p.data.normal_(0, 0.02)
+    m.setup_caches(num_pages=2, decode_rows=(4,))
+    m._pack_weights(force=True)
+    ff, w13, wo = m.layers[0].feed_forward, m._w13[0], m.layers[0].attention.wo.weight
+    was = [t.detach().clone() for t in (w13, ff.w1.weight, ff.w3.weight, wo)]
+    m.release_rowmajor()
+    released = set(m._released)
+    assert {id(w13), id(wo)} <= released
+    assert torch.equal(m._resident(w13), was[0]) and m._released == released and w13.stride() == (0, 0)
+    m.restore_on_demand(True)
+    assert m._resident(w13) is w13 and m._released == released - {id(w13)}
+    assert all(torch.equal(t, x) for t, x in zip((w13, ff.w1.weight, ff.w3.weight), was))
+    assert ff.w1.weight.data_ptr() == w13.data_ptr() and ff.w3.weight.data_ptr() == w13[512:].data_ptr()
+    assert torch.equal(m._resident(wo), was[3])
+    m.restore_on_demand(False)
+    m.release_rowmajor()
+    assert m._released == released
