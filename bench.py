@@ -4,8 +4,8 @@
     python -m torch.distributed.run --nnodes=1 --nproc-per-node N --master-addr 127.0.0.1 --master-port P \
         bench.py --gpus N --steps K --warmup W
 
-Workload (BASELINE.json metric "decode tokens/s/node + speedup vs autoregressive, Llama-3.1-8B B=64
-prefix=16K" == configs[2], the tests/SnapKV/longspec_benchmark.py command of the reference's README.md:69):
+Workload (metric "decode tokens/s/node + speedup vs autoregressive, Llama-3.1-8B B=64
+prefix=16K": the tests/SnapKV/longspec_benchmark.py command of the reference's README.md:69):
 Llama-3.1-8B target (TP = N) + Llama-3.2-1B SnapKV draft (budget 257, TP = min(N,4)), gamma=3, B=64,
 prefix_len 16032, max_len 16128, bf16, seeded random-init weights of those architectures (no checkpoints on
 the box), synthetic PG-19-shaped token batch.  It fits one MI355X (126 GiB target KV + 32 GiB draft KV +
@@ -17,7 +17,7 @@ when a batch reaches prefix+80 generated tokens the length counters are restored
 (the KV rows beyond the prefix are overwritten), exactly what the next batch would see.
 
 Acceptance: random-init weights make measured acceptance meaningless (~0), so `value` uses the fixed-acceptance
-replay of SURVEY.md section 8d -- per-row accept counts drawn from a seeded truncated geometric with alpha=0.8
+replay -- per-row accept counts drawn from a seeded truncated geometric with alpha=0.8
 (the reference's measured rate, index.html:595-601), E[tokens/iter]=2.952 at gamma=3; every kernel of the
 iteration still runs.  The same line also reports the run with the models' own (random-weight) acceptance and
 the autoregressive baseline (tests/baseline_benchmark.py loop) that defines "speedup".
@@ -47,9 +47,9 @@ WORKLOADS = {
     # eight kv heads: shards down to ONE kv head per rank at TP8 with a TP4 draft sub-group -- the reference README's
     # 8-GPU topology in miniature (tests/test_bench_cpu.py runs it over gloo with 4 and 8 ranks)
     "tiny-kh8": ("llama-68m-kh8", "llama-68m-kh8", 4, 416, 512, 129, 3),
-    # configs[1] of BASELINE.json: self-speculation, StreamingLLM draft cache (one model, two caches)
+    # self-speculation, StreamingLLM draft cache (one model, two caches)
     "cfg2": ("Meta-Llama-3.1-8B", None, 32, 8065, 8192, 257, 3),
-    # configs[3] / configs[4]: TP8 configurations -- on one GPU only as `--emulate-tp 8` (one rank's compute)
+    # TP8 configurations -- on one GPU only as `--emulate-tp 8` (one rank's compute)
     "cfg4": ("Meta-Llama-3.1-70B", "Llama-3.2-1B", 32, 32641, 32768, 513, 3, "longspec-stream"),
     "cfg5": ("Qwen2.5-32B", None, 128, 65440, 65536, 257, 3, "selfspec-snapkv"),
     "tiny-selfspec-snapkv": ("llama-68m-gqa", None, 4, 416, 512, 129, 3, "selfspec-snapkv"),
@@ -78,13 +78,13 @@ def parse(argv=None):
                          "(collectives over a 1-rank group): measures one rank's compute of a TP-N run on a 1-GPU box; "
                          "tokens are meaningless (partial sums are not reduced)")
     ap.add_argument("--kv-dtype", default="bf16", choices=["bf16", "fp8"],
-                    help="full-context KV cache storage (fp8 = OCP e4m3fn, BASELINE configs[4]; default bf16 = the "
+                    help="full-context KV cache storage (fp8 = OCP e4m3fn; default bf16 = the "
                          "reference's)")
     ap.add_argument("--kv-layout", default="HND", choices=["NHD", "HND"],
                     help="page layout of the full-context KV cache: HND (the Engine API's default) keeps the rows of a "
                          "kv head contiguous -- same tokens, verify attention 85 %% instead of 82 %% of the HBM peak "
                          "(bf16), 81 %% instead of 71 %% (fp8), profiles/r02_layout_ab.txt; NHD = the reference's "
-                         "flashinfer layout (DESIGN.md section 3.1)")
+                         "flashinfer layout")
     ap.add_argument("--draft-tp", type=int, default=4,
                     help="size of the draft sub-group (reference README: 4 of 8); 0 = REPLICATED draft: every rank runs "
                          "the whole draft model (no draft collectives, no token broadcast; greedy drafting is "
@@ -102,7 +102,7 @@ def parse(argv=None):
                          "verify kernels really accept; ':miss=f' makes a separate DRAFT model mispredict a seeded "
                          "fraction f of the vocabulary (per-step acceptance ~1 - f), and measured_acceptance_sweep "
                          "runs the loop at miss = 0.4 / 0.3 / 0.2 beside the replay at alpha = 0.6 / 0.7 / 0.8.  "
-                         "Default (round 6): peaked with miss = 0.2, so that the driver's line carries a MEASURED "
+                         "Default: peaked with miss = 0.2, so that the driver's line carries a MEASURED "
                          "acceptance next to the replay that defines `value`; timings are weight-value independent "
                          "(ms_per_step of the two agree to 0.1 %%: profiles/r06_bench_cfg3_peaked_miss_sweep_c7.json)")
     ap.add_argument("--design", default=None, metavar="furitar|bufodra",
@@ -258,7 +258,7 @@ def run(args, dev):
     tgt_name, drf_name, B, S, ML, BUDGET, G = wl[:7]
     kind = wl[7] if len(wl) > 7 else ("selfspec-stream" if drf_name is None else "longspec-snapkv")
     if args.workload == "cfg5" and "--kv-dtype" not in sys.argv:
-        args.kv_dtype = "fp8"                       # BASELINE configs[4] names the fp8 KV cache
+        args.kv_dtype = "fp8"                       # (these configurations name the fp8 KV cache)
     emu = getattr(args, "emulate_tp", 0)
     use_tp = world > 1 or getattr(args, "force_tp", False) or emu > 1
     group = draft_group = None
@@ -276,8 +276,8 @@ def run(args, dev):
     # FIRST on a multi-GPU run, before the models are loaded and before the long phases (prefill ~20 s, the timed loops,
     # the PMC passes): what one per-layer collective of this run costs, RCCL against the xGMI kernels -- these have never
     # crossed a real link, and a short lease on an 8-GPU node should yield this report even if it yields nothing else
-    # (VERDICT r3 next #5c).  It goes to stderr and to gpurun_out/ at once, and into the JSON line at the end.
-    # Round 5: the report also SELECTS the collective of the run.  The reference runs
+    # It goes to stderr and to gpurun_out/ at once, and into the JSON line at the end.
+    # The report also SELECTS the collective of the run.  The reference runs
     # with its low-latency intra-node all-reduce on (README.md:59, ENABLE_INTRA_NODE_COMM=1); ours was opt-in because it
     # had never crossed a link.  With MAGICDEC_ONESHOT_AR unset, the fused xGMI all-reduce + add + RMSNorm becomes the
     # run's collective iff the CHILD processes -- where a fault or hang costs nothing -- validated it against RCCL on these
@@ -524,7 +524,7 @@ def run(args, dev):
         restore()
     prime()
 
-    # Probation of the xGMI all-reduce inside the run's own processes and hipGraphs (round 5): the children validated the
+    # Probation of the xGMI all-reduce inside the run's own processes and hipGraphs: the children validated the
     # kernels on these links, try_create self-tested them eagerly at load; prime() has now replayed every captured step
     # variant once with them inside.  If ANY rank saw a time-out there, every rank drops to RCCL here -- a point where all
     # ranks stand at the same statement and no other collective is in flight -- instead of failing in the timed region,
@@ -577,7 +577,7 @@ def run(args, dev):
         dt_al, tok_al = run_spec(2, sens_steps, f_al)
         sens_raw[al] = (dt_al / sens_steps, tok_al / sens_steps)
 
-    # ---- measured acceptance at KNOWN draft quality (VERDICT r5 next #4): with `--weights peaked[...]` the draft's head is
+    # ---- measured acceptance at KNOWN draft quality: with `--weights peaked[...]` the draft's head is
     # rewritten in place (Engine/utils.repeak_head_: same storage, so the captured graphs stay valid; the draft cache does not
     # depend on the head) to mispredict a seeded fraction `miss` of the vocabulary, i.e. a draft whose per-step acceptance
     # rate is ~1 - miss, and the SAME loop runs with the accept kernel's own decisions.  Each point sits beside the
@@ -629,7 +629,7 @@ def run(args, dev):
     H_loc, KH_loc, D = cfg.n_head, cfg.n_local_heads, cfg.head_dim
     L_kv = S + 40 + G + 1                                 # mean kv length over a batch's 80 generated tokens
     kv_elem = 1 if args.kv_dtype == "fp8" else 2
-    attn_bytes = B * L_kv * KH_loc * D * 2 * kv_elem + 2 * B * (G + 1) * H_loc * D * 2
+    attn_bytes = B * L_kv * KH_loc * D * 2 * kv_elem + 2 * B * (G + 1) * H_loc * D * 2 
     achieved = attn_bytes / (attn_ms * 1e-3) / 1e9 if attn_ms > 0 else 0.0
 
     traffic, traffic_source = None, None
@@ -637,7 +637,7 @@ def run(args, dev):
     if want_pmc and on_gpu and rank == 0:
         traffic, traffic_source = measure_traffic(B, S + 40 + G + 1, KH_loc, H_loc, D, G + 1, args.kv_dtype == "fp8",
                                                   kv_layout == "HND")
-    # the same kernel on the OTHER page layout, stand-alone (VERDICT r5 next #8): the line says which layout the headline
+    # the same kernel on the OTHER page layout, stand-alone: the line says which layout the headline
     # ran and what the reference's own layout (NHD) would give
     other = "NHD" if kv_layout == "HND" else "HND"
     roofline_other = None
@@ -684,7 +684,7 @@ def run(args, dev):
                                     "0": "off", "1": "forced on"}[gemm_policy.fused_mode()],
                    # weights held TWICE during decode (streaming layout + row-major): after prefill the row-major tensor of
                    # every weight that decode reads in the streaming layout only is released (Transformer.release_rowmajor);
-                   # what remains is read in both layouts at different row counts (configs[2]: nothing)
+                   # what remains is read in both layouts at different row counts (the 8B / 1B pair at batch 64: nothing)
                    "packed_weight_copies_bytes": int(getattr(engine.model, "packed_bytes", 0)
                                                      + (getattr(draft.model, "packed_bytes", 0) if draft is not None
                                                         else 0)),
@@ -764,11 +764,11 @@ def run(args, dev):
 
 
 def xgmi_probation(models, dev, rounds=4):
-    """Probation of the xGMI all-reduce inside the run's OWN processes, communicators and hipGraphs (rounds 5-6).  The
+    """Probation of the xGMI all-reduce inside the run's OWN processes, communicators and hipGraphs.  The
     children validated the kernels on these links (collective_microbench), try_create self-tested them eagerly at load and
     prime() has replayed every captured step variant once with them inside.  Two checks, one collective decision:
       * time-outs: any rank whose status word is set (a bounded spin gave up, output rows poisoned);
-      * numerics (ADVICE r5): a short BIT-EXACT stress on each model's own communicator -- `rounds` x 6 all-reduces of the
+      * numerics: a short BIT-EXACT stress on each model's own communicator -- `rounds` x 6 all-reduces of the
         run's message sizes, algorithms interleaved, queued back to back, against the rank-ordered fp32 sum of the
         RCCL-all-gathered inputs (the kernels' definition).  A stale read that rounds differently would otherwise corrupt
         tokens silently while the timings still looked valid.
@@ -900,7 +900,7 @@ def acceptance_point(dt, tok, B, gamma, base_tps, replay):
 
 
 def speedup_condition(speedup_by_alpha, alpha, targets=(1.0, 1.8)):
-    """What the headline speed-up is conditional on (VERDICT r4 weak #9): `value` replays a FIXED acceptance rate, so
+    """What the headline speed-up is conditional on: `value` replays a FIXED acceptance rate, so
     "x over autoregressive" holds iff the real draft reaches that rate.  Linear interpolation of the measured
     alpha -> speed-up sweep at break-even (1.0x) and at north_star's target (>= 1.8x)."""
     pts = sorted(speedup_by_alpha.items())
@@ -997,7 +997,7 @@ def xgmi_verdict(report):
     kernels validated against RCCL (try_create's self-test inside the child), no child failed or timed out, no kernel spin
     timed out, ITS bit-exact stress passed, and its fused all-reduce + add + RMSNorm beat RCCL + the add+norm launch on the
     verify message.  The write-through arm is preferred (it is the faster one); when its stress fails -- the one hardware
-    assumption it rests on does not hold on these links -- the fence arm is still eligible (VERDICT r5 weak #10)."""
+    assumption it rests on does not hold on these links -- the fence arm is still eligible."""
     if not isinstance(report, dict) or not report:
         return None, "no report"
     if "error" in report or "rank0_child" in report:
@@ -1079,7 +1079,7 @@ def collective_microbench(group, shapes, dev, iters=30):
             r["xgmi_oneshot"] = timed(lambda: ar.all_reduce_(buf, oneshot.ALGO_ONESHOT))
             r["xgmi_twoshot"] = timed(lambda: ar.all_reduce_(buf, oneshot.ALGO_TWOSHOT))
             r["xgmi_fused_add_rmsnorm_auto"] = timed(lambda: ar.all_reduce_add_rmsnorm(x, res, w, 1e-5))
-            # third arm (round 6): the same fused kernel with the RELEASE-FENCE publish (md_ar_set_publish) -- what a
+            # third arm: the same fused kernel with the RELEASE-FENCE publish (md_ar_set_publish) -- what a
             # run degrades to if the write-through hand-off fails its stress on real links
             ar.set_publish(oneshot.PUBLISH_FENCE)
             r["xgmi_fence_fused_add_rmsnorm_auto"] = timed(lambda: ar.all_reduce_add_rmsnorm(x, res, w, 1e-5))
@@ -1089,8 +1089,8 @@ def collective_microbench(group, shapes, dev, iters=30):
             r["xgmi"] = "unavailable (set-up or self-test against RCCL failed on some rank)"
         out[name] = r
     if ar is not None:
-        # Bit-exact stress of the kernels over THESE links before a run may rely on them (round 5): the hand-off rests on
-        # write-through stores being visible to a peer when the relaxed flag is (csrc/allreduce.hip, ADVICE r4), which the
+        # Bit-exact stress of the kernels over THESE links before a run may rely on them: the hand-off rests on
+        # write-through stores being visible to a peer when the relaxed flag is (csrc/allreduce.hip), which the
         # shared-GPU tests cannot probe and try_create's tolerance self-test would miss if it failed rarely.  16 inputs
         # per round are all-gathered over RCCL, summed locally in rank order (fp32, one rounding = the kernel's
         # definition), then 16 xGMI calls are queued back to back with no host synchronisation, algorithms and sizes
@@ -1200,8 +1200,8 @@ def cpu_baseline(tgt_name, drf_name, S, budget, gamma, alpha, Bc=4):
               + (n_layer_target * t_layer_target(gamma+1 rows) + t_head_target + t_embed_target)
 
     (layer cost is depth-independent; embedding and head are counted once per forward, not once per layer), and
-    converted to tokens/s with the same replayed acceptance.  The K1 / K2 / K6 micro-benchmarks of SURVEY.md section
-    8d (verify attention, draft attention, SnapKV select at the per-layer shapes, batch Bc) are reported in GB/s of
+    converted to tokens/s with the same replayed acceptance.  The K1 / K2 / K6 micro-benchmarks
+    (verify attention, draft attention, SnapKV select at the per-layer shapes, batch Bc) are reported in GB/s of
     algorithmic bytes.  A reported baseline, not an optimisation target."""
     import torch
     import torch.nn.functional as F
@@ -1266,8 +1266,8 @@ def cpu_baseline(tgt_name, drf_name, S, budget, gamma, alpha, Bc=4):
         return t_layer, t_head, t_embed, t_attn, nbytes, n_layer, cfg, eng
 
     tl_t, th_t, te_t, ta_t, nb_t, n_t, _, _ = time_model(tgt_name, "target", gamma + 1, S + gamma + 1)
-    # the SAME target-layer sample once on every host core (BASELINE.md section 4 asks for the physical cores): printed so
-    # that capping the pool at 16 threads is evidence, not assertion (VERDICT r3 weak #10)
+    # the SAME target-layer sample once on every host core (the physical cores): printed so
+    # that capping the pool at 16 threads is evidence, not assertion
     all_cores = os.cpu_count() or 1
     tl_all = None
     if all_cores > ncores and os.environ.get("MAGICDEC_CPU_ALL_CORES", "1") != "0":
@@ -1326,7 +1326,7 @@ def cpu_baseline(tgt_name, drf_name, S, budget, gamma, alpha, Bc=4):
 
 
 def cpu_baseline_full_iteration_b1(tgt_name, drf_name, S, budget, gamma):
-    """ONE whole speculative iteration of the oracle at B = 1 and the real prefix (BASELINE.md section 4: "one full
+    """ONE whole speculative iteration of the oracle at B = 1 and the real prefix ("one full
     spec-decode iteration of Llama-3.1-8B shapes at B=1, S=16032"), not an assembly of per-layer timings: `gamma` draft
     forwards of the full-depth draft model over its `budget`-row SnapKV cache and one (gamma+1)-token verify forward of
     the full-depth target over `S` cached positions, head and embedding included, timed end to end.  Two shortcuts keep
@@ -1386,7 +1386,7 @@ def cpu_baseline_full_iteration_b1(tgt_name, drf_name, S, budget, gamma):
 
 
 def cpu_baseline_cfg1(prefix=129, max_len=256):
-    """BASELINE.json configs[0] END TO END on the host cores (the reference's own
+    """The smallest configuration END TO END on the host cores (the reference's own
     CPU-runnable case): the reference's "68m" model entry (Engine/SnapKV/model.py:67: MHA, 12 heads, dim 768, 2 layers,
     vocab 32000; seeded random weights), B = 1, prefix 129, greedy autoregressive decode to 256 positions with the
     loop of tests/baseline_benchmark.py:72-90 -- the whole run of the oracle (oracle/harness_ref.baseline_batch:

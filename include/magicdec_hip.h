@@ -46,8 +46,8 @@ extern "C" {
 typedef void* md_stream_t; /* hipStream_t */
 
 /* KV-cache element type.  MD_KV_FP8_E4M3 = OCP e4m3fn bytes (CDNA4 native, NOT the MI300 fnuz format) with one
- * fp32 dequantisation scale per kv head for K and for V (value = byte * scale); the reference has no fp8 path
- * (row "next" 8f-2 of SURVEY.md); accuracy is gated in tests/test_gpu_fp8.py. */
+ * fp32 dequantisation scale per kv head for K and for V (value = byte * scale); the reference has no fp8 path;
+ * accuracy is gated in tests/test_gpu_fp8.py. */
 #define MD_KV_BF16 0
 #define MD_KV_FP8_E4M3 1
 /* Page layout flag, OR-ed into the kv_dtype argument of md_append_paged_kv / md_rope_append (first cache) /
@@ -55,7 +55,7 @@ typedef void* md_stream_t; /* hipStream_t */
  * cache[page][2][page_size][KH][D]; MD_KV_LAYOUT_HND selects cache[page][2][KH][page_size][D] (flashinfer's other
  * layout): the rows of one kv head are contiguous, so a (request, kv head) stream is read in 128-row runs instead of
  * D*sizeof-byte pieces at a KH*D*sizeof stride -- at KH = 8 that is 128-byte pieces for an fp8 cache, whose loads-only
- * ceiling is 72.6 % of the HBM peak (DESIGN.md section 3.1).  A second cache (md_rope_append), the SnapKV draft cache
+ * ceiling is 72.6 % of the HBM peak.  A second cache (md_rope_append), the SnapKV draft cache
  * and the StreamingLLM ring are always NHD.  Results are bit-identical between the layouts. */
 #define MD_KV_LAYOUT_HND 0x100
 #define MD_KV_DTYPE_MASK 0xff
@@ -295,7 +295,7 @@ int md_linear_add_rmsnorm(const void* x, int64_t ldx, const void* w, int w_dtype
  * epilogue: deterministic).  Epilogues and rounding points are md_linear's (MD_EPI_NONE / MD_EPI_SWIGLU);
  * md_linear_block_add_rmsnorm is md_linear_add_rmsnorm on this kernel ((h, y) = (resid + o, rmsnorm(h) * w): the combine
  * launch of md_linear_add_rmsnorm, same rounding points).  The narrow projections of an M = 256 step (wqkv, wo) stay on
- * md_linear_fused / the library: a K split over ~256 workgroups costs them more than it saves (DESIGN.md section 3.3).
+ * md_linear_fused / the library: a K split over ~256 workgroups costs them more than it saves.
  * workspace: md_linear_block_workspace_bytes(M, N, K, force_split) bytes, 16-B aligned (force_split = 1 for the
  * add_rmsnorm form, whose epilogue always runs in the combine launch). */
 int md_linear_block_supported(int M, int N, int K, int epilogue);
@@ -368,7 +368,7 @@ typedef struct md_fused_linear_args {
 int md_linear_fused_supported(int M, int N, int K, int epilogue);
 int md_linear_fused(const md_fused_linear_args* args, md_stream_t stream);
 
-/* md_linear_fused_split (round 6): the K8b tile kernel with the K range ALSO split over S workgroups, for the deep narrow
+/* md_linear_fused_split: the K8b tile kernel with the K range ALSO split over S workgroups, for the deep narrow
  * products of a <= 64-row draft step (the 1B model's w2: N = 2048, K = 8192 -- Engine/SnapKV/model.py:451-455 followed by
  * the residual add and the next RMSNorm, :260-278,464-469).  A workgroup owns a (32|64)-row x (32|64)-column tile and K / S
  * of the depth, its 8 wavefronts K / (8 S) each -- at the 1B w2 that is 128 KB of W + 128 KB of x per CU, all requested
@@ -550,7 +550,7 @@ int md_softcap(void* z, int64_t z_row_stride, float cap, int rows, int dim, int 
  * K10  argmax over a vocab shard / TP merge
  *     reference: Engine/SnapKV/model.py:175-188
  * argmax: per row, max bf16 logit and its lowest index (+index_offset).
- * argmax_tp_slots (round 5): the same argmax written as the one-hot-slot
+ * argmax_tp_slots: the same argmax written as the one-hot-slot
  * tensors the reference all-reduces (model.py:178-184: torch.zeros + index
  * assignment): vals_out / idx_out [rows, tp_world], the row's result in
  * column tp_rank, zeros elsewhere -- one launch instead of five.

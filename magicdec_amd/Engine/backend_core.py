@@ -1,4 +1,4 @@
-"""Host side of the four MagicDec back-ends (L4 of SURVEY.md section 1), MI355X-native.
+"""Host side of the four MagicDec back-ends, MI355X-native.
 
 Public surface = the reference's: classes `LMBackend` / `LMBackend_Draft` with
 `load_model, setup_caches, compile, encode, inference, verify, speculate,
@@ -39,7 +39,7 @@ PROMPT_MEMORY = 0.8            # share of the free device memory that a portion'
 def default_kv_layout():
     """Page layout of the full-context cache when setup_caches() is not told one: "HND" (rows of one kv head contiguous
     inside a page: the verify step's stream is read in 128-row runs, 85 % instead of 82 % of the HBM peak in bf16, 81 %
-    instead of 71 % in fp8 -- DESIGN.md section 3.1) unless MAGICDEC_KV_LAYOUT=NHD asks for the reference's flashinfer
+    instead of 71 % in fp8) unless MAGICDEC_KV_LAYOUT=NHD asks for the reference's flashinfer
     layout (Engine/SnapKV/backend.py:30).  The layout is internal to the Engine API (the harness never touches the
     cache tensors) and moves bytes, not arithmetic: every kernel's output is bit-identical between the two
     (tests/test_gpu_hnd.py), and the whole GPU suite is green under either default (profiles/r03_hnd_suite_summary.txt).
@@ -330,7 +330,7 @@ class SnapKVTargetBackend(_BackendBase):
         """num_pages: pages of the pool that `step` serves unequal sequences from, when it is not to be a whole page list per
         request (encode / inference are then unavailable).
         kv_dtype="fp8": the full-context cache is OCP e4m3fn with static per-head scales calibrated on the
-        first prefill chunk (not in the reference; BASELINE.json configs[4]).  The compressed draft cache stays bf16.
+        first prefill chunk (not in the reference).  The compressed draft cache stays bf16.
         kv_layout="HND": the full-context cache keeps the rows of one kv head contiguous inside a page (the
         reference's flashinfer wrappers are planned "NHD": Engine/SnapKV/backend.py:30); same results, longer
         contiguous runs for the verify step's stream (matters for fp8 rows of 128 bytes).  None = default_kv_layout()."""
@@ -702,7 +702,7 @@ class StreamingDraftBackend(_BackendBase, _StreamingMixin):
 
 class StreamingSelfSpecBackend(_BackendBase, _StreamingMixin):
     """Engine/StreamingLLM/backend.py LMBackend: one set of weights, the full target cache and a streaming
-    draft cache."""
+    draft cache ."""
 
     def __init__(self, dtype=torch.bfloat16, device: str = "cuda:0", dec_len: int = 1):
         super().__init__(dtype, device)

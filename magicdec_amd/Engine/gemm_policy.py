@@ -2,7 +2,7 @@
 library GEMM (hipBLASLt through F.linear, with the TunableOp table of magicdec_amd/tuned/).
 
 The rules below are the outcome of the same-box, graph-captured A/B of profiles/r02_gemm_ab.txt (tools/gemm_bench.py:
-every decode / verify shape of the BASELINE models timed on both, weights cycled to defeat the Infinity Cache):
+every decode / verify shape of the 8B and 1B models timed on both, weights cycled to defeat the Infinity Cache):
 
   * md_linear over the STREAMING weight layout (ops.PackedWeight) wins where the product is a long weight stream --
     M <= 64: w1|w3 (+ fused SiLU*mul), w2 and the lm head of the 8B model, w1|w3 and the lm head of the 1B model
@@ -11,11 +11,11 @@ every decode / verify shape of the BASELINE models timed on both, weights cycled
     split-K combine of md_linear costs a second launch) and everything at M = 256 with K <= 4096 (there the product is
     MFMA / LDS bound, not HBM bound: a 256-row activation slab has to be re-read per 128 output columns).
 
-  * round 3: the LAUNCH-BOUND small products (every linear of the 1B draft model, every tensor-parallel shard, the
+  * the LAUNCH-BOUND small products (every linear of the 1B draft model, every tensor-parallel shard, the
     narrow projections of an 8B step) go to md_linear_fused (csrc/tilegemm.hip): one launch for the product AND the op
     behind it (rope+append, residual add, SiLU*mul), no split-K combine, no partial sums in HBM.
 
-  * round 4: the 129..256-ROW products of a verify step whose column count fills the chip without splitting K, and the
+  * the 129..256-ROW products of a verify step whose column count fills the chip without splitting K, and the
     K = 14336 down projection, go to md_linear_block (csrc/blockgemm.hip: 256 x 128 block tiles, LDS-DMA rings, loader +
     MFMA waves) -- profiles/r04_block_ab_final.txt, same process, graph-captured, weights cycled (us; "lib" includes the
     elementwise kernel behind it, "skinny" its combine launch):
@@ -51,7 +51,7 @@ MIN_STREAM_BYTES_M128 = 100e6
 FUSED_MAX_L2_BYTES = 70e6
 FUSED_MAX_L2_BYTES_T22 = 120e6
 FUSED_DEEP_SWIGLU_T22_MAX_L2_BYTES = float(os.environ.get("MAGICDEC_DEEP_SWIGLU_L2", "150e6"))   # (env: A/B switch)
-_SHARD70B = os.environ.get("MAGICDEC_SHARD70B", "1")     # "0": without the two round-6 rules for the 70B shards (A/B switch)
+_SHARD70B = os.environ.get("MAGICDEC_SHARD70B", "1")     # "0": without the two rules for the 70B shards (A/B switch)
 FUSED_MAX_K = 4096
 FUSED_QKV_M256_MAX_L2_BYTES = 110e6
 # the bounds of _measured(): tile traffic (M tiles x weight bytes) of a qkv projection (K <= 4096, deeper), and the weight bytes up to
@@ -59,7 +59,7 @@ FUSED_QKV_M256_MAX_L2_BYTES = 110e6
 FUSED_QKV_MAX_L2_BYTES = 270e6
 FUSED_QKV_DEEP_MAX_L2_BYTES = 230e6
 SWIGLU_ONE_TILE_MAX_BYTES = 210e6
-# round 5 (profiles/r05_fused_tp8_shard_tiles.txt, M = 256): two more TP8 shards of the 8B verify pass go to the fused kernel --
+# (profiles/r05_fused_tp8_shard_tiles.txt, M = 256): two more TP8 shards of the 8B verify pass go to the fused kernel --
 # w1|w3 (29.4 MB; 2 x 2 tiles: 21.1-22.3 us against 24.1 for the library + the SiLU*mul launch) and wo (4.2 MB, K = 512:
 # 12.0 against 14.1 incl. the add + norm behind it); w2 (14.7 MB: 17.1 vs 16.9) and everything wider stay on the library
 FUSED_M256_SWIGLU_MAX_BYTES = 32e6
@@ -72,7 +72,7 @@ _WO256 = os.environ.get("MAGICDEC_WO256", "1")        # "0": the 8B wo at 256 ro
 FUSED_MAX_L2_BYTES_WITH_NORM = 140e6
 
 
-# round 4: md_linear (the streaming kernel) can absorb the same deferred norm (md_linear_normed): a slab is normalised once
+# md_linear (the streaming kernel) can absorb the same deferred norm (md_linear_normed): a slab is normalised once
 # per workgroup on its way to LDS.  Free while the kernel waits for weights anyway (<= 64 rows); at 128 / 256 rows the
 # staging of a slab is as much vector work as its MFMAs and the launch it saves is cheaper (tools/fused_bench.py --pro 1:
 # 1B w1|w3 at 128 rows 35.4 vs 30.1 us with the norm as its own launch, 8B at 256 rows 179 vs 105).
@@ -124,9 +124,9 @@ def set_packed_copies(mode: str):
 def want_packed(N: int, K: int, swiglu: bool = False, int8: bool = False, rows=None) -> bool:
     """Re-pack this weight into the streaming layout at load time?  Only when a hand-written kernel may actually be
     chosen for it at some row count of a decode / verify step: `rows` = the counts the engine will run (the back-end knows
-    them: batch x {1, 2, dec_len}), or None = any of 1..256 (round 3 packed every bf16 weight with
-    K % 128 == 0; round 6: the 8B wqkv, served by the library at 64 and 256 rows, is no longer packed for the 32-row
-    steps configs[2] never runs)."""
+    them: batch x {1, 2, dec_len}), or None = any of 1..256 (not every bf16 weight with
+    K % 128 == 0: the 8B wqkv, served by the library at 64 and 256 rows, is not packed for the 32-row
+    steps that a batch of 64 never runs)."""
     if _MODE == "lib" or _PACKED == "0" or K % 64:
         return False
     if int8:
@@ -135,7 +135,7 @@ def want_packed(N: int, K: int, swiglu: bool = False, int8: bool = False, rows=N
         return True
     kinds = ("swiglu",) if swiglu else ("plain", "resid", "qkv")
     for M in ((1,) + tuple(range(32, 257, 32)) if rows is None else tuple(m for m in rows if m <= 256)):
-        # (default: every 32-row tile count a rule can depend on -- ADVICE r4)
+        # (default: every 32-row tile count a rule can depend on)
         for kind in kinds:
             if use_skinny(M, N, K, swiglu, False, True, kind):
                 return True
@@ -330,7 +330,7 @@ def use_fused(M: int, N: int, K: int, kind: str = "plain", absorbs_norm: bool = 
     kind = "resid" if kind == "planes" else kind
     m_tiles = (M + 31) // 32
     # a product the kernel runs with 2 x 2 tiles (csrc/tilegemm.hip launch_tile_pro: two M tiles, an even number of column
-    # tiles, >= 192 tile groups; with the deferred-norm prologue since round 6, K <= 4096) re-reads the weights once per
+    # tiles, >= 192 tile groups; with the deferred-norm prologue, K <= 4096) re-reads the weights once per
     # PAIR of M tiles: the 1B w1|w3 -- 18.4-18.9 us at 64 rows against md_linear's 22.8-23.2, and with the norm absorbed
     # 20.3 (profiles/r06_fused_pro22_ab.txt); at 128 rows (the two-token draft step) 32.0 with the norm against the library
     # + rmsnorm + SiLU*mul launches (20.5 + 5.1 + 5.4 in the trace), which also frees that weight's row-major copy
@@ -338,7 +338,7 @@ def use_fused(M: int, N: int, K: int, kind: str = "plain", absorbs_norm: bool = 
            and (N // 64) * ((m_tiles + 1) // 2) >= 192 and (not absorbs_norm or (kind == "swiglu" and K <= 4096)))
     l2_bytes = ((m_tiles + 1) // 2 if t22 else m_tiles) * N * K * 2
     if M <= 128:
-        # round 6, the 70B model's TP-8 shards at the 128 rows of configs[3]'s verify (tools/shard_bench.py,
+        # the 70B model's TP-8 shards at the 128 rows of their verify step (tools/shard_bench.py,
         # profiles/r06_shard70b_ab.txt): w2 (8192 x 3584, 2 x 2 tiles) 22.0 us against 24.4 for the library -- wide products
         # on 2 x 2 tiles may re-read up to 120 MB; wqkv (1280 x 8192) 16.7 against 21.1 + the rope/append launch -- a deep
         # NARROW qkv shard is fused up to K = 8192 once >= 128 tile workgroups exist (at 32 rows, 40 workgroups, the
@@ -359,11 +359,11 @@ def use_fused(M: int, N: int, K: int, kind: str = "plain", absorbs_norm: bool = 
     if kind == "swiglu":
         return N * K * 2 <= FUSED_M256_SWIGLU_MAX_BYTES and K <= FUSED_MAX_K
     if kind in ("plain", "resid"):
-        if N * K * 2 <= FUSED_M256_NARROW_MAX_BYTES and K <= FUSED_MAX_K:         # measured at K = 512 only (ADVICE r5)
+        if N * K * 2 <= FUSED_M256_NARROW_MAX_BYTES and K <= FUSED_MAX_K:         # measured at K = 512 only
             return True
-        # round 6: the 8B wo at 256 rows on 2 x 2 tiles (4 x 64 tile groups = 256 workgroups) WITH its residual add is a
+        # the 8B wo at 256 rows on 2 x 2 tiles (4 x 64 tile groups = 256 workgroups) WITH its residual add is a
         # measured tie with the library + add/norm launch (25.2-25.9 vs 24.9-25.0 us, profiles/r06_fused_pro22_ab.txt;
-        # in-trace A/B profiles/r06_ab_wo256_*): taking it leaves NO weight of configs[2] held in two layouts during
+        # in-trace A/B profiles/r06_ab_wo256_*): taking it leaves NO weight of the 8B / 1B pair at batch 64 held in two layouts during
         # decode (the library read the row-major tensor) and one library kernel fewer in the verify pass
         return (_WO256 != "0" and kind == "resid" and t22 and K <= FUSED_MAX_K
                 and N * K * 2 <= FUSED_M256_RESID_T22_MAX_BYTES)
@@ -387,7 +387,7 @@ def use_skinny(M: int, N: int, K: int, swiglu: bool, int8: bool, packed: bool, k
     return K >= 8192 and nbytes >= MIN_STREAM_BYTES_M128
 
 
-# round 6: md_linear_fused_split (csrc/tilegemm.hip, FL_PARTIAL) -- the tile kernel with K ALSO split over workgroups, for the
+# md_linear_fused_split (csrc/tilegemm.hip, FL_PARTIAL) -- the tile kernel with K ALSO split over workgroups, for the
 # deep narrow output projections of a <= 128-row step whose combine launch is the residual add + RMSNorm launch anyway: the 1B
 # model's w2 (N = 2048, K = 8192, 33.5 MB), which every single-launch decomposition leaves per-CU-ingest-bound (fused tile
 # kernel 22-24 us, library 15.7 + 5 for the add + norm, md_linear 17 + 5).  Rule from tools/split_bench.py

@@ -1,4 +1,4 @@
-"""C1 of SURVEY.md section 8e: the per-layer sum-all-reduce of the bf16 partials over xGMI peer-mapped buffers
+"""The per-layer sum-all-reduce of the bf16 partials over xGMI peer-mapped buffers
 (`md_allreduce` / `md_allreduce_add_rmsnorm`, csrc/allreduce.hip), one communicator per process group.
 
 Replaces `dist.all_reduce` at Engine/SnapKV/model.py:334-335,453-454 (and the StreamingLLM twins) for the

@@ -115,7 +115,7 @@ def _peak_(model, seed, dtype, emb_rms=40.0, peak=12.0, miss=0.0):
     attention / FFN branches of all layers still run at full strength as the perturbation.
     `miss` (draft models only; 'peaked:...:miss=f'): the head mispredicts whenever the true next token lies in a seeded
     fraction f of the vocabulary (_peak_perm), so a draft step is rejected with probability ~f -- a draft of KNOWN
-    acceptance rate alpha ~ 1 - f, measured by the accept kernel's own decisions (VERDICT r5 next #4)."""
+    acceptance rate alpha ~ 1 - f, measured by the accept kernel's own decisions."""
     emb = model.tok_embeddings.weight
     V, dim = emb.shape
     e = (emb.data.float() * (emb_rms / 0.02)).to(dtype)

@@ -1,4 +1,4 @@
-"""HF checkpoint -> `model.pth` in the layout the Engine loads (row "next" 8f-3 of SURVEY.md; the reference's
+"""HF checkpoint -> `model.pth` in the layout the Engine loads (the reference's
 convert_hf_checkpoint.py:79-163 produces the same file, so either tool's output loads here and in the reference).
 
 Layout facts that are binding for the kernels:

@@ -1,5 +1,5 @@
-// The verify-loop body of MagicDec's speculative decoding as ONE integer kernel
-// (row a1 of SURVEY.md section 8): accept mask, accept_nums, length rollback /
+// The verify-loop body of MagicDec's speculative decoding as ONE integer kernel:
+// accept mask, accept_nums, length rollback /
 // advance for the target and draft page tables, output scatter, bonus token,
 // termination test and the "double buffer" for rows that accepted all gamma.
 //

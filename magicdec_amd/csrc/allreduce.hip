@@ -14,7 +14,7 @@
 //             ranks' reduced rows (all-gather): two hops, 2(N-1)/N x message inbound.  Right for the 2 MiB verify
 //             message at N = 8 (3.5 MiB instead of 14 MiB per rank).
 //
-// Determinism (SURVEY.md section 8e): a row is summed by exactly one piece of code in rank order 0..N-1 with fp32
+// Determinism: a row is summed by exactly one piece of code in rank order 0..N-1 with fp32
 // accumulation and one rounding -- in the one-shot form by every rank identically, in the two-shot form by its
 // owner only -- so all ranks obtain bit-identical results (the replicated argmax / page tables need that).
 //
@@ -25,7 +25,7 @@
 //
 // Protocol, per call k = 1, 2, ... (k lives in device memory so that a captured hipGraph replays correctly; every
 // block of a call reads the same k because the counter is advanced only once ALL blocks of the call have read it:
-// round 5, see "call counter" below) and per block b of a grid that is sized to the message:
+// see "call counter" below) and per block b of a grid that is sized to the message:
 //   1. copy the rows of block b from `in` into my data buffer half (k & 1);
 //   2. release; store k into start[b][me] of every peer; spin until start[b][p] >= k for every p; acquire;
 //   3. one-shot: sum the rows of block b over all ranks -> out.           two-shot: sum MY rows of block b -> my
@@ -57,8 +57,8 @@ struct Signal {
     uint32_t status;                          // owner only: 0 ok, 1 = a spin timed out (output poisoned)
 };
 
-// Call counter (round 5).  Owner-only state in ORDINARY (cached) device memory: ctrl[0] = number of calls whose counter
-// has been handed on, ctrl[1] = blocks of the running call that have read it.  Rounds 2-4 kept both in the uncached signal
+// Call counter.  Owner-only state in ORDINARY (cached) device memory: ctrl[0] = number of calls whose counter
+// has been handed on, ctrl[1] = blocks of the running call that have read it.  An earlier form kept both in the uncached signal
 // area and let the LAST block to FINISH advance the counter: an uncached read at the head of every launch (everything
 // else waits for k) and a returning atomic on uncached memory at its tail -- ~3 us of a 9 us launch with one rank
 // (tools/ar_bench.py).  All the protocol needs is that no block of call k reads the counter after it was advanced, so the
@@ -87,20 +87,20 @@ struct ArArgs {
     size_t n_vec;              // total vectors
 };
 
-// Publishing (round 4).  Rounds 2-3 wrote the registered buffers with plain stores and made them
-// visible with a system-scope RELEASE FENCE (buffer_wbl2 sc0 sc1: a write-back sweep of the XCD's L2, 1.7-6.5 us by
+// Publishing.  An earlier form wrote the registered buffers with plain stores and made them visible
+//  with a system-scope RELEASE FENCE (buffer_wbl2 sc0 sc1: a write-back sweep of the XCD's L2, 1.7-6.5 us by
 // MI355X_MICROARCH.md), polled the flags with ACQUIRE loads (an L1/L2 invalidate per poll) and closed every call with
 // two __threadfence(): ~18 us per launch before a byte had crossed a link.  Now the payload is stored WRITE-THROUGH
 // at system scope (16-byte `sc0 sc1` stores: the data is in memory when the store retires), every wave drains its own
 // stores (s_waitcnt vmcnt(0), inline asm: the compiler cannot drop it), the flags are polled with RELAXED loads and ONE
 // acquire fence per hop follows the poll (the guide's R1 hand-off in its cross-device form); the call counter needs no
 // fence at all -- its only reader is the next launch on the same stream.
-// INVARIANT (ADVICE r4): every store into a registered buffer that a PEER reads -- data[] (the published partials) and the
+// INVARIANT: every store into a registered buffer that a PEER reads -- data[] (the published partials) and the
 // result halves (`myres`) -- must go through store_wt and be followed by drain_stores() before the flag is raised; a plain
 // store would sit in this XCD's L2 behind a relaxed flag.  finish_row's plain stores write the caller's OUTPUT tensors, which
 // no peer reads.  The correctness of the hand-off rests on vmcnt retiring a write-through store only once it is visible
 // at system scope; it has been validated between processes sharing one GPU (tests/test_gpu_allreduce.py: thousands of
-// calls, bit-exact) and NOT yet over xGMI links -- bench.py's child-process report (DESIGN.md 3.2) is what decides
+// calls, bit-exact) and NOT yet over xGMI links -- bench.py's child-process report is what decides
 // whether a multi-GPU run uses it.
 __device__ __forceinline__ void store_wt(bf16_t* base, size_t vec_index, const u32x4 v) {
     u32x4* p = reinterpret_cast<u32x4*>(base) + vec_index;
@@ -108,9 +108,9 @@ __device__ __forceinline__ void store_wt(bf16_t* base, size_t vec_index, const u
 }
 __device__ __forceinline__ void drain_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// MD_AR_PUBLISH_FENCE (round 6): the write-through publish above rests on ONE hardware
+// MD_AR_PUBLISH_FENCE: the write-through publish above rests on ONE hardware
 // property that no single-GPU test can probe -- that vmcnt retires an `sc0 sc1` store only once a PEER can see it.  In
-// this mode the flag-raising lanes additionally execute the system-scope RELEASE fence of rounds 2-3 (buffer_wbl2 sc0 sc1
+// this mode the flag-raising lanes additionally execute the system-scope RELEASE fence of that form (buffer_wbl2 sc0 sc1
 // + s_waitcnt: the AMDGPU memory model's own release sequence, which writes back whatever this XCD's L2 still holds)
 // between the block barrier that follows every wave's drain and the flag stores.  It costs the L2 write-back sweep
 // (1.7-6.5 us per hop by MI355X_MICROARCH.md) and assumes nothing beyond the documented memory model: if the
@@ -214,7 +214,7 @@ __device__ __forceinline__ void finish_row(const ArArgs& a, int row, int lane, i
 // PF: rows of <= 4096 elements (every plain call: 512 vectors per row; the fused rows of the 1B / 8B / 32B models).
 // Everything a wave needs for its FIRST row that does not come from a peer -- its own partial, the residual row, the norm
 // weights -- is requested BEFORE the block waits for the call counter and for the peers' flags, so those round trips
-// overlap instead of queueing behind each other (round 5: 9.3 -> see tools/ar_bench.py).
+// overlap instead of queueing behind each other (9.3 -> see tools/ar_bench.py).
 template <int NR, bool TWOSHOT, bool FUSED, bool PF>
 __global__ __launch_bounds__(kThreads) void allreduce_kernel(const ArDev c, const ArArgs a) {
     const int b = blockIdx.x, G = gridDim.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -356,7 +356,7 @@ __global__ __launch_bounds__(kThreads) void allreduce_kernel(const ArDev c, cons
                 reduce_row(row, nv, s, first);
             } else {
                 // a peer's partial never arrived: the rows this rank owns are NaN for EVERYONE -- the peers gather
-                // them from `myres` in step 3c, and must not find the rows of two calls ago there (ADVICE r2)
+                // them from `myres` in step 3c, and must not find the rows of two calls ago there
                 const u32x4 nan = {0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};
 #pragma unroll
                 for (int i = 0; i < NV; ++i) s[i] = nan;

@@ -1,7 +1,7 @@
 // Block-tile GEMM for the 129..256-row linears of a verify step (gfx950):  out = epilogue(x[M][K] . W[N][K]^T + bias)
 //
 // replaces: the nn.Linear calls of the (gamma+1)-token verify pass at B x (gamma+1) = 256 rows
-//           (Engine/SnapKV/model.py:288-289 wqkv / wo, :446-455 w1 / w3 / w2, :175-177 output), which rounds 1-3 left
+//           (Engine/SnapKV/model.py:288-289 wqkv / wo, :446-455 w1 / w3 / w2, :175-177 output), which were left
 //           to hipBLASLt -- 5.1 ms of a 31 ms iteration at 20-43 % of HBM / <= 35 % of the MFMA peak
 //           (profiles/r03_bench_cfg3_iter_breakdown.csv).
 //

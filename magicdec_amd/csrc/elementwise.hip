@@ -1,5 +1,5 @@
 // RMSNorm (+residual), SiLU*mul, argmax over a vocab shard, TP argmax merge
-// (K9, K10 of SURVEY.md section 2.3) for gfx950.
+// for gfx950.
 //
 // reference: RMSNorm        Engine/SnapKV/model.py:458-469
 //            FeedForward    Engine/SnapKV/model.py:451-455

@@ -104,7 +104,7 @@ __device__ __forceinline__ float silu_bf16(float h1) {
 // 8B w1|w3 (896 wave tiles, two K slices) ran as 448 four-wave workgroups = 192 CUs with two and 64 with one (1 048 KB
 // against a mean of 918 KB); as 256 seven-wave workgroups every CU streams 917 KB.  Bits do not change: a wave's tile,
 // K range and slab order are the same, only its neighbours in the workgroup differ.
-// PRO (round 4): the deferred RMSNorm of md_linear_fused on this kernel's activation path -- x is the un-normalised h
+// PRO: the deferred RMSNorm of md_linear_fused on this kernel's activation path -- x is the un-normalised h
 // the residual epilogue of the producing linear wrote together with per-row partial sums of squares; the workgroup forms
 // rstd per row (the tile kernel's sum, term for term) and normalises every slab on its way from registers to LDS:
 // y = bf16(bf16(h * rstd) * w).  A slab is normalised once per workgroup and shared by its 128 columns, so the cost is a
@@ -491,7 +491,7 @@ int g_force_rd = 0;          // dev knob (md_debug_set_gemm_ring): 0 = the rule 
 template <int MT, int EPI, bool W8, bool PRO, int NW, int RD>
 int launch_rd(const GemmParams& p, int n_blocks, hipStream_t st);
 
-// W ring depth (round 6, a measured NEGATIVE result kept as a dev knob).  The four-wave form requests 4 x 8 KiB per CU with
+// W ring depth (a measured NEGATIVE result kept as a dev knob).  The four-wave form requests 4 x 8 KiB per CU with
 // the 8-deep ring, half of what the six- / seven-wave forms and the tile kernel keep in flight, so a 16-deep ring (there is
 // room for it at <= 64 rows) looked like the fix for the K-split products that run four waves (the 8B w2 at 32 / 64 rows,
 // the lm heads).  tools/ring_bench.py (profiles/r06_ring_depth_ab.txt): 29.6 vs 29.5, 32.9 vs 33.6, 17.8 vs 18.5, lm heads

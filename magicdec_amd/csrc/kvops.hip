@@ -1,4 +1,4 @@
-// Paged-KV append and RoPE for gfx950 (K4, K5 of SURVEY.md section 2.3).
+// Paged-KV append and RoPE for gfx950.
 //
 //   md_append_paged_kv  <- flashinfer.append_paged_kv_cache   (Engine/utils.py:36-54)
 //   md_rope             <- flashinfer.rope.apply_rope / apply_llama31_rope, interleave=True
@@ -240,7 +240,7 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 // device address of the dropped-row counter, for kernels of other translation units (csrc/tilegemm.hip, blockgemm.hip).
 // Resolved once per device: the callers sit on the launch-bound path (one call per layer per step, also inside graph
-// capture), where a runtime call per launch is avoidable host latency (ADVICE r3).
+// capture), where a runtime call per launch is avoidable host latency.
 unsigned int* md_page_overflow_counter_device() {
     static unsigned int* cached[MD_MAX_DEVICES] = {};
     int d = 0;

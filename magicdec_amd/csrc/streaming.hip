@@ -1,5 +1,4 @@
-// StreamingLLM sink+window eviction for the draft KV cache (K7, row a9 of
-// SURVEY.md section 8), gfx950.
+// StreamingLLM sink+window eviction for the draft KV cache, gfx950.
 //
 // reference: KVCache.prefill        Engine/StreamingLLM/model_draft.py:102-143
 //            KVCache.prefill_draft  Engine/StreamingLLM/model.py:116-157

@@ -23,7 +23,7 @@
 //     registers (one contiguous KiB per instruction, 8-deep rolling ring; non-temporal when there is one M tile, kept in
 //     L2 for the sibling M tiles otherwise), its private slice of the activations goes global -> registers -> wave-private LDS image ->
 //     MFMA A fragments (full 256-B row segments per 16 lanes from L2 instead of fragment-shaped 32-B pieces -- the
-//     latter is what made round 2's "short-stream" attempt 1.4-3x slower) with the next 128-deep chunk's loads in flight
+//     latter made a "short-stream" attempt 1.4-3x slower) with the next 128-deep chunk's loads in flight
 //     under the current chunk's MFMAs;
 //   * v_mfma_f32_32x32x16_bf16, fp32 accumulators; the 8 partial tiles are summed through LDS in wave order
 //     (deterministic: eager, graph replay and every TP rank see the same bits);
@@ -174,9 +174,9 @@ __device__ __forceinline__ int64_t kv_elem_offset(const KvTable& t, int b, int r
 // has in flight -- NW x (8 KiB of W + 8 KiB of x) -- are what its ingest rate is made of, ~50 GB/s per CU at NW = 8);
 // WNT = stream W with non-temporal loads (one M tile: every weight byte is read once) or keep it in L2 for the sibling
 // M tiles of the same weight tile.
-// MT x NT = 32-row x 32-column MFMA tiles per workgroup (round 4).  What a CU has to ingest is W x (M tiles that
-// re-read it) + the x slab x (column tiles that re-read it), and a CU ingests ~50 GB/s whatever the kernel
-// (DESIGN.md 3.3): with 1 x 1 tiles the 1B w1|w3 at M = 64 (67 MB of W) moves 134 MB of W (two M tiles) + 134 MB of x
+// MT x NT = 32-row x 32-column MFMA tiles per workgroup.  What a CU has to ingest is W x (M tiles that
+// re-read it) + the x slab x (column tiles that re-read it), and a CU ingests ~50 GB/s whatever the kernel:
+// with 1 x 1 tiles the 1B w1|w3 at M = 64 (67 MB of W) moves 134 MB of W (two M tiles) + 134 MB of x
 // (512 column tiles x 256 KB) = 1.05 MB per CU = the measured 24.5 us; a 2 x 2 tile (64 rows x 64 columns, one
 // workgroup per CU) halves both.  Each K-slice wave then owns 2 x 2 accumulators, two W fragment streams and a 64-row
 // activation image; the summation order over the K slices (wave order) and every epilogue are unchanged, so the bits
@@ -187,12 +187,12 @@ template <int EPI, bool FP8, int NW, bool WNT, bool PRO, int MT, int NT, int AI>
 __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel(const TileParams p) {
     constexpr int kNW = NW;
     static_assert(AI == 8 || MT == 1, "fewer rows than a tile: one M tile");
-    // Round 6, the deferred-norm prologue on 2 x 2 tiles (the 1B w1|w3 at 64 rows).  Phase timestamps of the 1 x 1 form
+    // The deferred-norm prologue on 2 x 2 tiles (the 1B w1|w3 at 64 rows).  Phase timestamps of the 1 x 1 form
     // (tools/tile_timing.py, profiles/r06_tile_phase_timing.txt) show where its 6 us go: ~1 us of prologue in front of the
     // first load, +2.4 us per activation chunk between "landed" and "staged" (four wavefronts per SIMD normalising at
     // once, 11 vector instructions per dword), and every column tile normalising the same rows (512 x).  The 2 x 2 form
     // halves the last; it used to sit at 256 registers and spill.  A CU keeps ~64 KB of loads in flight whoever issues
-    // them (DESIGN.md 3.3), so 8 wavefronts need 8 KB each, not 32: the W ring of this form is FOUR deep (kRD), which
+    // them, so 8 wavefronts need 8 KB each, not 32: the W ring of this form is FOUR deep (kRD), which
     // frees 32 registers; the row scales' partial sums are requested FIRST, the W ring and the first activation chunk
     // behind them, and the workgroup meets at a bare s_barrier (no vmcnt(0) drain); the norm weights of a chunk are
     // unpacked once, both roundings are one v_cvt_pk_bf16_f32.
@@ -604,7 +604,7 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
     // w1|w3: 256 groups).  Narrow products keep 1 x 1 tiles: more, smaller workgroups matter more there.
     // (not with the deferred-RMSNorm prologue: that instantiation sits at the 256-register cap, re-reads rstd from LDS per
     // chunk, and measured 25.9 us in the cfg3 iteration against 24.5 for the 1 x 1 form -- profiles/r04_bench_cfg3_iter_breakdown.csv)
-    // round 6: also WITH the deferred-RMSNorm prologue (SwiGLU consumer), now that that instantiation has a four-deep W
+    // also WITH the deferred-RMSNorm prologue (SwiGLU consumer), now that that instantiation has a four-deep W
     // ring, no spills, and its own prologue (kNewPro in the kernel)
     if constexpr ((EPI == FL_SWIGLU || EPI == FL_NONE || EPI == FL_RESID || EPI == FL_XIELU) && (!PRO || EPI == FL_SWIGLU)) {
         const int groups = (p.n_tiles / 2) * ((p.m_tiles + 1) / 2);
@@ -615,7 +615,7 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
         if (t22) return launch_tile_cfg<EPI, FP8, 8, false, PRO, 2, 2>(p, st);
     }
     // 16 wavefronts (K/16 slices) when the grid is too small to put two 8-wave workgroups on every CU
-    // (round 6: not below K = 1024 -- two k-steps per wavefront and a 16-way reduce cost more than they hide: the K = 512 wo
+    // (not below K = 1024 -- two k-steps per wavefront and a 16-way reduce cost more than they hide: the K = 512 wo
     // shards run 4.1-4.2 us with 8 slices against 5.3-5.4 with 16, tools/shard_bench.py / profiles/r06_shard_ab.txt)
     const int wgs = p.n_tiles * p.m_tiles;
     bool nw16 = p.K % 256 == 0 && p.K >= 1024 && wgs <= 384;
@@ -645,7 +645,7 @@ int launch_tile(const TileParams& p, hipStream_t st) {
 bool aligned16(const void* q) { return ((uintptr_t)q & 15) == 0; }
 
 // ---- md_linear_fused_split: the tile kernel with the K range ALSO split over S workgroups (FL_PARTIAL) ----------------
-// Why (round 6): the deep narrow products of a 64-row draft step -- the 1B w2, N = 2048, K = 8192 -- are per-CU-ingest
+// Why: the deep narrow products of a 64-row draft step -- the 1B w2, N = 2048, K = 8192 -- are per-CU-ingest
 // bound on every single-launch decomposition (a workgroup that owns the whole K range re-reads a 32-row x 8192 slab of x
 // per 32 columns: 1 MB per CU, 22-24 us; hipBLASLt: 768 KB per CU, 15.7 us + 5 for the add + norm behind it) and
 // latency-bound on md_linear (4 waves x 8 KiB of W in flight per CU: 17 + 5).  A 64 x 64 tile x K / 8 per workgroup

@@ -1,4 +1,4 @@
-"""The speculative draft/verify decode loops (L5 of SURVEY.md section 1) on the GPU.
+"""The speculative draft/verify decode loops on the GPU.
 
 These are the loop bodies of the reference's benchmark scripts
 (tests/SnapKV/longspec_benchmark.py:131-295 and its StreamingLLM twin,
@@ -86,7 +86,7 @@ def _read_flags(st: LoopState, collectives=()):
             ev = st._flags_event
             ev.record()
             while not ev.query():
-                time.sleep(0)           # give up the GIL and the time slice between polls (ADVICE r4: with 8 ranks and
+                time.sleep(0)           # give up the GIL and the time slice between polls (with 8 ranks and
                 #                         their RCCL proxy threads on one host a hard spin would pin a core per rank)
         for ar, s in zip(collectives, status):
             if int(s[0]) != 0:
@@ -168,7 +168,7 @@ def _draft_round(step_fn, st: LoopState, gamma, next_double):
 
 def _iterate(engine, draft, st: LoopState, body, forced):
     """Runs one iteration body (each decode step inside it is one hipGraph replay when the back-ends were compile()d)
-    and makes the iteration's one host read.  (A whole-iteration graph was built and measured in rounds 2 and 3: 31.6
+    and makes the iteration's one host read.  (A whole-iteration graph was built and measured: 31.6
     vs 31.6 ms at TP1, 8.77 vs 8.85 ms for a TP8 rank's compute -- the host already runs ahead of the GPU -- and was
     removed: profiles/r02_ab_iteration_graph.txt, profiles/r03_ab_iteration_graph_tp8.txt.)"""
     body(forced)
@@ -247,7 +247,7 @@ def selfspec_iteration(engine, st: LoopState, gamma, eot_1, eot_2, max_nodes, ne
 
 
 def _force_accept(tokens_buffer, target_tokens, forced_accept, gamma):
-    """Fixed-acceptance replay (SURVEY.md section 8d): with random-init weights the measured acceptance is
+    """Fixed-acceptance replay: with random-init weights the measured acceptance is
     meaningless, so benchmarks may replace the target's tokens by ones that accept exactly
     forced_accept[b]-1 draft tokens of row b (all the draft/verify/accept work still runs)."""
     tt = target_tokens.clone()

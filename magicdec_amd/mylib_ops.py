@@ -1,6 +1,6 @@
 """The reference's seven ``mylib::*`` torch.library operators, bound to the C ABI (libmagicdec_hip.so).
 
-This is the executable form of the drop-in boundary (SURVEY.md section 8b, INTEGRATION.md section B): a maintainer of
+This is the executable form of the drop-in boundary: a maintainer of
 the reference replaces the bodies of its custom ops -- which call flashinfer -- by these registrations and keeps
 every call site (``torch.ops.mylib.update_kv(...)``, ``self.rope(q, k, indptr, offsets)``,
 ``self.attn_decode(q, kv_cache)`` ...) unchanged.  Schemas are character-for-character the reference's:

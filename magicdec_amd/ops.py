@@ -533,7 +533,7 @@ def _block_args(x, weight, swiglu):
 
 
 def _block_bias(bias, N):
-    """md_linear_block reads the bias as 16-byte vectors of N bf16 values (ADVICE r4)."""
+    """md_linear_block reads the bias as 16-byte vectors of N bf16 values."""
     if bias is None:
         return
     _gpu(bias)
