@@ -11,6 +11,8 @@
 //   silu:  y = bf16( silu(float(a)) ) * b                             (product rounded to bf16)
 #include "md_common.h"
 
+#include <type_traits>
+
 namespace {
 
 __device__ __forceinline__ float block_reduce_sum(float v, float* red) {
@@ -275,7 +277,7 @@ __global__ __launch_bounds__(256) void softcap_kernel(T* z, int64_t zs, float ca
 // all-reduces (Engine/SnapKV/model.py:178-184), in the argmax launch itself
 // A row is a handful of loads per thread, so its time is memory round trips and the reduction: all of a thread's loads go out together
 // (a loop that compares before it loads again made one trip each), and the first wave folds the waves' results: 64 rows over 32 000
-// tokens 7.9 -> 5.6 us, over 128 256 14.5 -> 13.1.
+// tokens 7.9 -> 5.6 us, over 128 256 14.5 -> 13.1.  As many loads as the row still has: four for a row of one cost 0.9 of 4 us.
 constexpr int kArgmaxLoads = 4;
 
 template <int NT, typename T = bf16_t>
@@ -292,12 +294,13 @@ __global__ __launch_bounds__(NT) void argmax_kernel(const T* __restrict__ logits
     const int nvec = vocab / 8;
     const bool vec_ok = (((uintptr_t)p) & (8 * sizeof(T) - 1)) == 0;
     if (vec_ok) {
-        for (int i0 = threadIdx.x; i0 < nvec; i0 += NT * kArgmaxLoads) {
-            vec8 r[kArgmaxLoads];
+        auto take = [&](auto loads, int i0) {
+            constexpr int U = decltype(loads)::value;
+            vec8 r[U];
 #pragma unroll
-            for (int u = 0; u < kArgmaxLoads; ++u) r[u] = reinterpret_cast<const vec8*>(p)[min(i0 + u * NT, nvec - 1)];
+            for (int u = 0; u < U; ++u) r[u] = reinterpret_cast<const vec8*>(p)[min(i0 + u * NT, nvec - 1)];
 #pragma unroll
-            for (int u = 0; u < kArgmaxLoads; ++u) {
+            for (int u = 0; u < U; ++u) {
                 const f32x8 f = __builtin_convertvector(r[u], f32x8);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
@@ -309,6 +312,13 @@ __global__ __launch_bounds__(NT) void argmax_kernel(const T* __restrict__ logits
                     }
                 }
             }
+        };
+        for (int base = 0; base < nvec; base += NT * kArgmaxLoads) {      // (uniform: as many loads as the row still has)
+            const int i0 = base + threadIdx.x, left = nvec - base;
+            if (left > 3 * NT) take(std::integral_constant<int, 4>(), i0);
+            else if (left > 2 * NT) take(std::integral_constant<int, 3>(), i0);
+            else if (left > NT) take(std::integral_constant<int, 2>(), i0);
+            else take(std::integral_constant<int, 1>(), i0);
         }
         for (int id = nvec * 8 + threadIdx.x; id < vocab; id += NT) {
             const float v = (float)p[id];

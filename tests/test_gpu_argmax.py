@@ -6,7 +6,7 @@ pytestmark = pytest.mark.gpu
 DEV, BF = "cuda:0", torch.bfloat16
 
 
-@pytest.mark.parametrize("rows,vocab", [(1, 1), (3, 7), (2, 1000), (1, 8192), (2, 8193), (1, 16384), (2, 32767), (3, 32768), (1, 32776), (2, 128256),
+@pytest.mark.parametrize("rows,vocab", [(1, 1), (3, 7), (2, 1000), (1, 8192), (2, 8193), (1, 16384), (2, 32767), (3, 32768), (1, 32776), (2, 128256), (1, 16392), (2, 24576), (2, 24584),
                                         (513, 16384)])
 @pytest.mark.parametrize("dtype", [BF, torch.float32])
 def test_argmax(rows, vocab, dtype):
