@@ -304,7 +304,10 @@ int kv_splits(const md_latent_args* a) {
     // is not reached 128 keys, and 64 up to one on every other.  Four layers, us: one request of 8 000 keys 316 -> 300, four of 1 000
     // 319 -> 295, twelve of 1 500 333 -> 319 (64 keys: 325); beyond, shorter chains lose to the merge: 32 of 2 049 at 128 keys 391 against
     // 380, 48 of 1 200 430 against 415
-    const long few = std::max(std::min(tiles / 4, target / 2 / groups), std::min(tiles / 2, target / 4 / groups));
+    // (not within a page, and within two only where the merge has little to do: one request of 75 keys 18.3 against 19.8, 31 of 137 with
+    // a 512-wide latent 19.9 against 21.8, but 19 of 160 with a 256-wide one 23.5 -> 18.4)
+    const bool worth = tiles > 8 || (tiles > 4 && (groups <= 16 || a->kv_rank <= 256));
+    const long few = worth ? std::max(std::min(tiles / 4, target / 2 / groups), std::min(tiles / 2, target / 4 / groups)) : 0;
     const long cap = std::max(std::max(tiles / 8, few), 1L);
     if (want > cap) want = cap;
     return (int)(want < 1 ? 1 : want > 64 ? 64 : want);            // (the merge holds a split per lane)
