@@ -804,10 +804,14 @@ size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 // Columns per workgroup of the two score kernels.  A table, a query image and a merge per workgroup are worth 4 096 columns and more as
 // long as two workgroups per CU are there (16 requests of 16 000 keys, 8 kv heads of 64: 2 048 -> 4 096 pass 1 139 -> 120 us, pass 2 153
 // -> 150); one request alone has too few workgroups with 2 048 (4 128 keys, heads of 128: 118 us for the whole selection, 67 with 512).
+// One chunk is enough for a short context already below two workgroups per CU (61 requests of 767 keys, 8 kv heads of 128: 216 us in
+// 512 + 255 columns, 198 in one).  The chunks of a context are even, whole rounds of a workgroup's wavefronts: 16 384 + 4 112 columns of
+// 296 pairs (37 requests of 20 496 keys, 8 kv heads of 128) take 1 098 us for the whole selection, twice 10 496 912 and less.
 int score_cols(int B, int KH, int ctx_len) {
     int cols = 512;
-    while (cols < 16384 && (int64_t)B * KH * ((ctx_len + 2 * cols - 1) / (2 * cols)) >= 512) cols *= 2;
-    return cols;
+    while (cols < 16384 && (int64_t)B * KH * ((ctx_len + 2 * cols - 1) / (2 * cols)) >= (cols < 1024 ? 400 : 512)) cols *= 2;
+    const int n = std::max((ctx_len + cols - 1) / cols, 1);          // (a size may be asked for any length)
+    return std::max(((ctx_len + n - 1) / n + 255) / 256 * 256, 256);
 }
 
 }  // namespace
