@@ -265,8 +265,11 @@ int decode_splits(const md_xattn_args* a) {
     const long keys = keys_of(a);
     const long tiles = (keys + 31) / 32 + 1, pairs = (long)a->B * a->KH;
     // at most one workgroup per CU: a second one on some CUs makes those finish last (one step of 2 layers with heads of 64: 12
-    // requests of 1 500 keys 170.7 us in 288 workgroups, 165.5 in 192; 20 of 1 000 176.6 in 320, 170.0 in 160)
+    // requests of 1 500 keys 170.7 us in 288 workgroups, 165.5 in 192; 20 of 1 000 176.6 in 320, 170.0 in 160) -- unless that leaves a
+    // third of them idle over long ranges (160 pairs of 8 673 keys and heads of 88: 209 us in 160, 151 in 320; 146 of 13 821 and 64: 127,
+    // 106; of 1 100 keys one is ahead, 21.9 / 23.4)
     long want = pairs < g_target_wgs ? g_target_wgs / pairs : 1;
+    if (want == 1 && 10 * pairs < 7 * g_target_wgs && keys >= 3072) want = 2;
     const long cap = tiles / 16 > 1 ? tiles / 16 : 1;        // >= 16 tiles (4 per wavefront) per workgroup
     if (want > cap) want = cap;
     return (int)(want < 1 ? 1 : want > 64 ? 64 : want);

@@ -286,6 +286,18 @@ def test_attention_splits_agree(ops):
         assert float((got.double() - ref[0][at:at + 1]).abs().max()) < 1.5e-2 * float(ref[0].abs().max()), at
 
 
+def test_two_splits_beside_short_sequences(ops):
+    """One long sequence and many short ones: half the keys of every one in a workgroup of its own."""
+    lens = [3100, 1700] + [150, 40] * 16
+    spec, rows, ref = attention_case(ops, 8, 4, 64, 64, 0, 4, BF, lens)
+    s, who, start = Seqs(ops, spec, BF, lens, seed=6), list(range(len(lens))), [n - 3 for n in lens]
+    s.attend(torch.cat([r[:n] for r, n in zip(rows, start)]), who, [0] * len(lens), start)
+    for width, at in ((1, 0), (2, 1)):
+        got = s.attend(torch.cat([r[n + at:n + at + width] for r, n in zip(rows, start)]), who, [n + at for n in start], [width] * len(lens))
+        want = torch.cat([r[n + at:n + at + width] for r, n in zip(ref, start)])
+        assert float((got.double() - want).abs().max()) < 1.5e-2 * max(1.0, float(want.abs().max())), width
+
+
 def test_sink_takes_the_weight_of_low_scores(ops):
     """Queries opposite to every key: the sink holds nearly all the weight, the output is nearly 0 (and not the mean of v)."""
     g = torch.Generator().manual_seed(0)
