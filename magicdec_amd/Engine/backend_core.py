@@ -215,7 +215,8 @@ class _BackendBase:
 
     def _rows_that_fit(self, rows, row_bytes=0, fixed=0):
         """`rows` of a prompt, or as many as the device's free memory holds: their activations in a layer (and row_bytes each, and `fixed`)
-        beside the row-major weights that the prompt brings back.  The same on every rank of a tensor-parallel group."""
+        beside the row-major weights that the prompt brings back.  The same on every rank of a tensor-parallel group, and where a whole
+        draft runs on each rank: other portions round otherwise, and the ranks' tokens have to be the same."""
         dev, m = torch.device(self.device), self.model
         if dev.type != "cuda":
             return rows
@@ -224,7 +225,7 @@ class _BackendBase:
         if PROMPT_MEMORY * (free - taken) < rows * each:         # (what the allocator holds unused: its statistics take 50 us and more)
             free += torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
         rows = min(rows, max(0, int(PROMPT_MEMORY * (free - taken) // each)))
-        group = getattr(m, "process_group", None)
+        group = getattr(m, "process_group", None) or getattr(m, "replica_group", None)
         if group is not None:
             import torch.distributed as dist
             least = torch.tensor([rows], dtype=torch.int32, device="cuda" if dist.get_backend(group) == "nccl" else "cpu")

@@ -1587,6 +1587,29 @@ def test_portions_shrink_with_the_free_memory(monkeypatch):
     assert e._rows_that_fit(8192) == 0 and longest() == 128
 
 
+@pytest.mark.parametrize("kind", ["process_group", "replica_group"])
+def test_portions_are_the_same_on_every_rank(monkeypatch, kind):
+    """The ranks of a tensor-parallel model, and those that each run the whole draft, take the portions of the one with the least memory."""
+    from types import SimpleNamespace
+    import torch.distributed as dist
+    from magicdec_amd.Engine import backend_core as core
+    e = core._BackendBase(device="cuda:0")
+    e.batch_size = 2
+    group, asked = object(), []
+    e.model = SimpleNamespace(prompt_row_bytes=lambda: 1000, released_bytes=0, process_group=None,
+                              layers=[SimpleNamespace(attention=SimpleNamespace(kv_cache=SimpleNamespace(scales=lambda which: None)))])
+    setattr(e.model, kind, group)
+
+    def all_reduce(t, op, group):
+        asked.append(group)
+        assert op == dist.ReduceOp.MIN
+        t.clamp_(max=1000)                                  # the other rank has room for as many
+    monkeypatch.setattr(dist, "get_backend", lambda group: "gloo")
+    monkeypatch.setattr(dist, "all_reduce", all_reduce)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda dev=None: (1 << 30, 1 << 30))
+    assert e._rows_that_fit(8192) == 1000 and max(n for _, n in e._portions(20_000)) == 3 * 128 and asked == [group, group]
+
+
 def test_weights_come_back_on_demand():
     """Between restore_on_demand(True) and the next release, a released weight that is asked for stays: the bits it had, w1 and w3 views
     of w13 again; without it a product gets a tensor of its own and the weight stays released."""
