@@ -614,17 +614,23 @@ class SnapKVDraftBackend(_BackendBase):
 class _StreamingMixin:
     """Sink(16)+window prefill shared by the stand-alone StreamingLLM draft and the self-spec engine."""
 
+    def _stream_chunks(self, num_chunks, cache):
+        """Chunks to a pass (md_streaming_windows): PROMPT_ROWS rows, PROMPT_WINDOWS bytes of windows, and what fits the memory; one where
+        the CPU's products round by their row counts.  Whether the ranks ask one another follows from what they all have: the windows
+        of a rank with fewer kv heads are smaller."""
+        most = PROMPT_ROWS // (self.batch_size * CHUNK)
+        if cache.device.type == "cpu" or num_chunks == 1 or most <= 1:
+            return 1
+        nbytes, rows = cache.numel() * cache.element_size(), self.batch_size * CHUNK
+        most = min(most, PROMPT_WINDOWS // nbytes)    # (a chunk's window, and the cache behind the pass, are copies of the cache)
+        return max(1, self._rows_that_fit(most * rows, nbytes / rows, nbytes) // rows)
+
     def _stream_encode(self, input_ids, state: _PagedState, lens_attr, which):
         seq_len, B = input_ids.shape[1], self.batch_size
         tokens = None
         num_chunks = (seq_len + CHUNK - 1) // CHUNK
-        # chunks to a pass (md_streaming_windows): PROMPT_ROWS rows and PROMPT_WINDOWS bytes of them (one where the CPU's products round by their row counts)
         cache = getattr(self.model.layers[0].attention.kv_cache, which)
-        nbytes = cache.numel() * cache.element_size()
-        most = 1 if cache.device.type == "cpu" else min(PROMPT_ROWS // (B * CHUNK), PROMPT_WINDOWS // nbytes)
-        if most > 1 and num_chunks > 1:               # (a chunk's window, and the cache behind the pass, are copies of the cache)
-            most = self._rows_that_fit(most * B * CHUNK, nbytes / (B * CHUNK), nbytes) // (B * CHUNK)
-        passes = -(-num_chunks // max(1, most))
+        passes = -(-num_chunks // self._stream_chunks(num_chunks, cache))
         ctx = 0                                       # host mirror of the (capped) cache length
         with self._prefilling():
             for i in range(passes):

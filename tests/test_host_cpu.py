@@ -1610,6 +1610,37 @@ def test_portions_are_the_same_on_every_rank(monkeypatch, kind):
     assert e._rows_that_fit(8192) == 1000 and max(n for _, n in e._portions(20_000)) == 3 * 128 and asked == [group, group]
 
 
+def test_windows_are_the_same_on_every_rank(monkeypatch):
+    """Three ranks of eight kv heads hold 3, 3 and 2 of them: a pass takes the chunks that the most heads allow, also where that is one."""
+    from types import SimpleNamespace
+    import torch.distributed as dist
+    from magicdec_amd.Engine import backend_core as core
+    sizes = []
+
+    def engine(budget, heads):
+        class Engine(core._BackendBase, core._StreamingMixin):
+            pass
+        e = Engine(device="cuda:0")
+        e.batch_size = 2
+        e.model = SimpleNamespace(prompt_row_bytes=lambda: heads, released_bytes=0, process_group=object())
+        cache = SimpleNamespace(device=torch.device("cuda:0"), numel=lambda: 2 * budget * heads * 128, element_size=lambda: 2)
+        return e, cache
+    monkeypatch.setattr(dist, "get_backend", lambda group: "gloo")
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda dev=None: (1 << 40, 1 << 40))
+    for budget in (1_000, 30_000, 65_000, 100_000, 150_000, 200_000, 300_000, 500_000):
+        own = []
+        for heads in (3, 2):
+            monkeypatch.setattr(dist, "all_reduce", lambda t, op, group: own.append(int(t)))      # what this rank brings
+            engine(budget, heads)[0]._stream_chunks(20, engine(budget, heads)[1])
+        assert len(own) == 2, budget                                                              # every rank asked
+        monkeypatch.setattr(dist, "all_reduce", lambda t, op, group: t.clamp_(max=min(own)))
+        both = [engine(budget, heads)[0]._stream_chunks(20, engine(budget, heads)[1]) for heads in (3, 2)]
+        assert both[0] == both[1]
+        sizes.append(both[0])
+    assert sizes[0] == 32 and sizes[-1] == 1 and len(set(sizes)) > 3
+    assert engine(1_000, 3)[0]._stream_chunks(1, engine(1_000, 3)[1]) == 1
+
+
 def test_weights_come_back_on_demand():
     """Between restore_on_demand(True) and the next release, a released weight that is asked for stays: the bits it had, w1 and w3 views
     of w13 again; without it a product gets a tensor of its own and the weight stays released."""
