@@ -1335,10 +1335,10 @@ class StepOps:
 
 def step_copies(t, dst=None):
     """Can StepOps copy from this tensor (into `dst`)?"""
-    return t.is_cuda and t.dtype == torch.int64 and t.numel() > 0 and (dst is None or (dst.device == t.device and dst.dtype == t.dtype)) and (
+    return t.is_cuda and t.dtype == torch.int64 and t.numel() > 0 and (dst is None or (dst.get_device() == t.get_device() and dst.dtype == t.dtype)) and (
         t.is_contiguous() or (t.dim() == 2 and (t.shape[1] == 1 or t.stride(1) == 1)))
 
 
 def step_adds(t, beside=None):
     """Can StepOps add to this tensor (in a launch that works on `beside`)?"""
-    return t.is_cuda and t.dtype == torch.int32 and t.numel() > 0 and t.is_contiguous() and (beside is None or t.device == beside.device)
+    return t.is_cuda and t.dtype == torch.int32 and t.numel() > 0 and t.is_contiguous() and (beside is None or t.get_device() == beside.get_device())
