@@ -709,7 +709,7 @@ class StreamingDraftBackend(_BackendBase, _StreamingMixin):
 
 class StreamingSelfSpecBackend(_BackendBase, _StreamingMixin):
     """Engine/StreamingLLM/backend.py LMBackend: one set of weights, the full target cache and a streaming
-    draft cache ."""
+    draft cache."""
 
     def __init__(self, dtype=torch.bfloat16, device: str = "cuda:0", dec_len: int = 1):
         super().__init__(dtype, device)
