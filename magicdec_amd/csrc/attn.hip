@@ -1187,13 +1187,17 @@ AttnPlan make_plan(int B, int n_max, int H, int KH, int max_pages, int page_size
         pl.qt = rows <= 16 ? 1 : 2;
         pl.n_qgroups = 1;
         const long max_tiles = (long)max_pages * page_size / 32, pairs = (long)B * KH;
-        // Splits: as many as leave at most ONE workgroup per CU.  A CU with a second workgroup finishes last, and a lone one streams
-        // faster: 12 requests of 16 000 keys (96 pairs of 8 kv heads, bf16 of 128) take 119 us in 192 workgroups, 158 in 288, 123 in
-        // 480; 20 requests (160 pairs) 192 us unsplit, 236 in 320, 203 in 480; 7 of 4 000 (56 pairs) 27 us in 224, 35 in 280.
+        // Splits: as many as leave at most ONE workgroup per CU of an XCD, where a pair's workgroups lie together (32 CUs).  A CU with a
+        // second workgroup finishes last, and a lone one streams faster: 12 requests of 16 000 keys (96 pairs of 8 kv heads, bf16 of 128)
+        // take 119 us in 192 workgroups, 158 in 288, 123 in 480; 20 requests (160 pairs) 192 us unsplit, 236 in 320, 203 in 480; 7 of 4 000
+        // (56 pairs) 27 us in 224, 35 in 280; 21 of 14 000, 4 kv heads, 102 in 168, 138 in 252 (33 on each of four XCDs).
         // Between one and 1.25 workgroups per CU a few CUs would work twice as long as the rest: three splits level that (33 requests
         // of 4 000 keys, 264 pairs: 118 -> 103 us; of 16 000: 438 -> 371) once a pair's stream is long (fp8, 4 000 keys: 68.5 -> 72.3,
-        // 16 000: 234 -> 214).  Beyond that splitting costs more than it levels (352 pairs 121.6 / 120.8 / 132 us, 520 pairs 190 / 193).
-        long want = pairs <= 256 ? 256 / pairs : pairs <= 320 && max_tiles * (fp8 ? 1 : 2) >= 256 ? 3 : 1;
+        // 6 000: 109 -> 86, 16 000: 234 -> 214), and two up to 1.5 (352 pairs of 14 000: 441 -> 394; 6 000 keys of 64: 98 -> 91).  Beyond
+        // that splitting costs more than it levels (400 pairs of 14 000: 459 / 478, 520 pairs 190 / 193).
+        const long on_xcd = (pairs + 7) / 8;
+        const bool level = max_tiles >= (fp8 ? 160 : 128);
+        long want = pairs < 8 ? 256 / pairs : on_xcd <= 32 ? 32 / on_xcd : !level || on_xcd > 48 ? 1 : on_xcd <= 40 ? 3 : 2;
         if (g_target_wgs > 0) want = (g_target_wgs + pairs - 1) / pairs;
         long cap = max_tiles / 16;  // >= 16 tiles (4 per wave) per workgroup
         if (cap < 1) cap = 1;

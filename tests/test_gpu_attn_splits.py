@@ -11,6 +11,17 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("B,KH,ctx,n", [(1, 1, 4161, 1), (5, 4, 4161, 4), (7, 8, 1500, 2), (28, 8, 3300, 1), (32, 8, 700, 4), (33, 8, 4161, 1),
                                         (40, 8, 4161, 2), (41, 8, 4161, 1), (33, 8, 8300, 1)])
 def test_splits(B, KH, ctx, n, fp8):
+    check(B, KH, ctx, n, fp8)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("B,KH,ctx,n", [(21, 4, 2100, 4), (44, 8, 8300, 1), (48, 8, 8300, 2), (49, 8, 8300, 1)])
+def test_splits_of_an_xcd(B, KH, ctx, n, fp8):
+    """A pair's workgroups lie on one XCD: 11 pairs on some of them take two splits, 44 and 48 two, 49 none."""
+    check(B, KH, ctx, n, fp8)
+
+
+def check(B, KH, ctx, n, fp8):
     """bf16 weights of the values: |error| <= 2^-8 of the weighted |v|, plus the output's own rounding; fp32 sums elsewhere."""
     from magicdec_amd import ops
     D, g, pp = 64, 4, -(-ctx // 128)
