@@ -253,26 +253,36 @@ bool mfma_ok(const md_xattn_args* a) {
 
 int decode_rows(const md_xattn_args* a) { return a->n_max * (a->H / a->KH); }
 
-int g_target_wgs = 256;
-
 // keys one request can see in a step: its chunk (plus the step's own rows), or its whole page list
 long keys_of(const md_xattn_args* a) {
     const long keys = (long)a->max_pages * a->page_size;
     return a->chunk > 0 && (long)a->chunk + a->n_max < keys ? (long)a->chunk + a->n_max : keys;
 }
 
+// Splits of a pair (request, kv head) over workgroups, in 32-key tiles: a workgroup costs its tiles and 15 more, a pair's workgroups lie on
+// one XCD of 32 CUs, two on a CU take 1.43 times as long as one (three and four, 2.4 and 3: two are resident), and an XCD's workgroups
+// together take no less than 0.75 of their sum -- 0.9 where heads wider than 64 and one 16-row tile leave HBM the bound --; the merge
+// costs 11 tiles.  Over 924 sizes (24..400 pairs, 600..12 000 keys, heads of 64, 88 and 128, several layers' pages in turn) the least of
+// that is 0.4 % above the best of 1..12.  At most one workgroup per CU of 256 lost up to half where the last CUs of an XCD got a second
+// one (84 pairs of 6 000 keys: 252 are 33 on four XCDs, 49.5 -> 38.6 us) and where 140..250 pairs stayed unsplit (92 x 2 of 6 000 keys,
+// 20 rows: 154 -> 115); at least one per CU, 160 pairs of 2 744 keys 30.0 against 25.8.
 int decode_splits(const md_xattn_args* a) {
-    const long keys = keys_of(a);
-    const long tiles = (keys + 31) / 32 + 1, pairs = (long)a->B * a->KH;
-    // at most one workgroup per CU: a second one on some CUs makes those finish last (one step of 2 layers with heads of 64: 12
-    // requests of 1 500 keys 170.7 us in 288 workgroups, 165.5 in 192; 20 of 1 000 176.6 in 320, 170.0 in 160) -- unless that leaves a
-    // third of them idle over long ranges (160 pairs of 8 673 keys and heads of 88: 209 us in 160, 151 in 320; 146 of 13 821 and 64: 127,
-    // 106; of 1 100 keys one is ahead, 21.9 / 23.4)
-    long want = pairs < g_target_wgs ? g_target_wgs / pairs : 1;
-    if (want == 1 && 10 * pairs < 7 * g_target_wgs && keys >= 3072) want = 2;
-    const long cap = tiles / 16 > 1 ? tiles / 16 : 1;        // >= 16 tiles (4 per wavefront) per workgroup
-    if (want > cap) want = cap;
-    return (int)(want < 1 ? 1 : want > 64 ? 64 : want);
+    const long tiles = (keys_of(a) + 31) / 32 + 1, on_xcd = ((long)a->B * a->KH + 7) / 8;
+    const long cap = tiles / 16 > 1 ? tiles / 16 < 64 ? tiles / 16 : 64 : 1;        // >= 16 tiles (4 per wavefront) per workgroup
+    const double together = a->D <= 64 || decode_rows(a) > 16 ? 0.75 : 0.9;
+    double least = 1e300;
+    int best = 1;
+    for (long n = 1; n <= cap; ++n) {
+        const long wgs = on_xcd * n, deep = (wgs + 31) / 32;
+        const double one = 15 + (double)tiles / n;
+        const double last = one * (deep == 1 ? 1 : deep == 2 ? 1.43 : deep == 3 ? 2.4 : 0.75 * deep), sum = one * together * wgs / 32;
+        const double cost = (last > sum ? last : sum) + (n > 1 ? 11 : 0);
+        if (cost < least) {
+            least = cost;
+            best = (int)n;
+        }
+    }
+    return best;
 }
 
 XattnParams make_params(const md_xattn_args* a) {

@@ -298,6 +298,19 @@ def test_two_splits_beside_short_sequences(ops):
         assert float((got.double() - want).abs().max()) < 1.5e-2 * max(1.0, float(want.abs().max())), width
 
 
+@pytest.mark.parametrize("H,KH,D,count", [(8, 4, 64, 21), (8, 4, 64, 46), (5, 1, 88, 100), (8, 4, 128, 64)])
+def test_splits_of_an_xcd(ops, H, KH, D, count):
+    """84 pairs (11 on some XCDs), 184, 100 and 256 of them: from one split to several on a CU, ranges that end in all of them."""
+    lens = [[2700, 1500][b] if b < 2 else (40, 600, 33, 130)[b % 4] for b in range(count)]
+    spec, rows, ref = attention_case(ops, H, KH, D, D, 0, 4, BF, lens)
+    s, who, start = Seqs(ops, spec, BF, lens, seed=6), list(range(count)), [n - 5 for n in lens]
+    s.attend(torch.cat([r[:n] for r, n in zip(rows, start)]), who, [0] * count, start)
+    for width, at in ((1, 0), (4, 1)):
+        got = s.attend(torch.cat([r[n + at:n + at + width] for r, n in zip(rows, start)]), who, [n + at for n in start], [width] * count)
+        want = torch.cat([r[n + at:n + at + width] for r, n in zip(ref, start)])
+        assert float((got.double() - want).abs().max()) < 1.5e-2 * max(1.0, float(want.abs().max())), width
+
+
 def test_sink_takes_the_weight_of_low_scores(ops):
     """Queries opposite to every key: the sink holds nearly all the weight, the output is nearly 0 (and not the mean of v)."""
     g = torch.Generator().manual_seed(0)
