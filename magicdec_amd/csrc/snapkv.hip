@@ -801,17 +801,40 @@ __global__ __launch_bounds__(256) void snapkv_gather_kernel(const GatherParams p
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
-// Columns per workgroup of the two score kernels.  A table, a query image and a merge per workgroup are worth 4 096 columns and more as
-// long as two workgroups per CU are there (16 requests of 16 000 keys, 8 kv heads of 64: 2 048 -> 4 096 pass 1 139 -> 120 us, pass 2 153
-// -> 150); one request alone has too few workgroups with 2 048 (4 128 keys, heads of 128: 118 us for the whole selection, 67 with 512).
-// One chunk is enough for a short context already below two workgroups per CU (61 requests of 767 keys, 8 kv heads of 128: 216 us in
-// 512 + 255 columns, 198 in one).  The chunks of a context are even, whole rounds of a workgroup's wavefronts: 16 384 + 4 112 columns of
-// 296 pairs (37 requests of 20 496 keys, 8 kv heads of 128) take 1 098 us for the whole selection, twice 10 496 912 and less.
-int score_cols(int B, int KH, int ctx_len) {
-    int cols = 512;
-    while (cols < 16384 && (int64_t)B * KH * ((ctx_len + 2 * cols - 1) / (2 * cols)) >= (cols < 1024 ? 400 : 512)) cols *= 2;
-    const int n = std::max((ctx_len + cols - 1) / cols, 1);          // (a size may be asked for any length)
-    return std::max(((ctx_len + n - 1) / n + 255) / 256 * 256, 256);
+// Columns per workgroup of the two score kernels, in rounds of the eight wavefronts' 32 columns each.  A workgroup costs its rounds and two
+// more for the table, the query image and the merge; a CU holds one workgroup at a time, or two that together take 1.4 times as long as
+// one (128 rows of 64); the launch ends with the CU that has the most.  The even division with the least of that is within 0.6 % of
+// the best of 1..32 chunks over 320 sizes (4..512 pairs of request and head, 521..16 032 keys) and nowhere slower than whole chunks of
+// 2 048 columns, which lost to chunks sized for two workgroups per CU where only one fits: 52 requests of 700 keys, 8 queries a kv head
+// of 64, 162 us in one chunk, 188 in two rounds of 512 columns; 19 of 521, heads of 128, 165 and 187.  Whole selections, the two
+// workgroups' rule -> this one: 32 requests of 1 100 keys, 4 kv heads of 64, 160 -> 128 us; 4 of 16 000, 8 of 128, 169 -> 146; 25 of
+// 2 100, 8 of 64, 142 -> 121.
+int score_cols(int B, int KH, int L, int D, int ctx_len) {
+    const int64_t pairs = (int64_t)B * KH;
+    const int all = std::max((ctx_len + 255) / 256, 1);              // (a size may be asked for any length)
+    const bool two = D == 64 && L <= 128;
+    double least = 1e300;
+    int best = all;
+    for (int r = 1; r <= all; ++r) {
+        const int64_t on_cu = (pairs * ((all + r - 1) / r) + 255) / 256;
+        const double cost = (2 + r) * (two ? 1.4 * (double)(on_cu / 2) + (double)(on_cu % 2) : (double)on_cu);
+        if (cost < least) {
+            least = cost;
+            best = r;
+        }
+    }
+    const int n = (all + best - 1) / best;                           // ... and as even as whole rounds go
+    return (all + n - 1) / n * 256;
+}
+
+// bytes of the partial sums: either head size (it is not among the sizes the workspace is asked for by)
+size_t partial_bytes(int B, int KH, size_t L, int ctx_len) {
+    size_t nch = 1;
+    for (int D : {64, 128}) {
+        const size_t cols = score_cols(B, KH, (int)L, D, ctx_len);
+        nch = std::max(nch, (ctx_len + cols - 1) / cols);
+    }
+    return align_up((size_t)B * KH * L * nch * 2 * 8, 256);
 }
 
 }  // namespace
@@ -820,8 +843,7 @@ extern "C" size_t md_snapkv_workspace_bytes(int B, int H, int KH, int ctx_len, i
     if (B <= 0 || H <= 0 || KH <= 0 || H % KH || ctx_len <= window) return 0;
     const int g = H / KH;
     const size_t L = (size_t)g * window;
-    const size_t cols = score_cols(B, KH, ctx_len), nch = (ctx_len + cols - 1) / cols;
-    const size_t partials = align_up((size_t)B * KH * L * nch * 2 * 8, 256);
+    const size_t partials = partial_bytes(B, KH, L, ctx_len);
     const size_t aws = align_up((size_t)B * H * (ctx_len - window) * 2, 256);
     const size_t scores = align_up((size_t)B * KH * (ctx_len - window) * 2, 256);
     return partials + aws + scores + 256;
@@ -831,8 +853,7 @@ extern "C" size_t md_snapkv_scores_offset(int B, int H, int KH, int ctx_len, int
     if (B <= 0 || H <= 0 || KH <= 0 || H % KH || ctx_len <= window) return 0;
     const int g = H / KH;
     const size_t L = (size_t)g * window;
-    const size_t cols = score_cols(B, KH, ctx_len), nch = (ctx_len + cols - 1) / cols;
-    return align_up((size_t)B * KH * L * nch * 2 * 8, 256) + align_up((size_t)B * H * (ctx_len - window) * 2, 256);
+    return partial_bytes(B, KH, L, ctx_len) + align_up((size_t)B * H * (ctx_len - window) * 2, 256);
 }
 
 extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int32_t* page_indices,
@@ -884,7 +905,7 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
     p.W = window;
     p.S = ctx_len;
     p.L = L;
-    p.cols = score_cols(B, KH, ctx_len);
+    p.cols = score_cols(B, KH, L, D, ctx_len);
     p.nch = (ctx_len + p.cols - 1) / p.cols;
     p.page_size = page_size;
     p.slot_stride = hnd ? D : KH * D;
@@ -892,7 +913,7 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
     p.page_stride = 2 * (int64_t)page_size * KH * D;
     unsigned char* ws = (unsigned char*)workspace;
     p.partials = (double*)ws;
-    const size_t partials_b = align_up((size_t)B * KH * L * p.nch * 2 * 8, 256);
+    const size_t partials_b = partial_bytes(B, KH, L, ctx_len);
     p.aws = (unsigned short*)(ws + partials_b);
     const size_t aws_b = align_up((size_t)B * H * N * 2, 256);
     unsigned short* scores = (unsigned short*)(ws + partials_b + aws_b);

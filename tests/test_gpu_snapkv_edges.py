@@ -23,6 +23,13 @@ def test_select_of_many_requests(monkeypatch, B, KH, S):
     check_select(monkeypatch, B, KH, 2, 16, 64, S, 129, 5, 128, (0, B // 2, B - 1))
 
 
+@pytest.mark.parametrize("B,KH,g,W,D,S", [(52, 4, 8, 32, 64, 700), (19, 8, 8, 32, 128, 521), (12, 8, 4, 32, 128, 1100), (3, 2, 4, 32, 128, 4150)])
+def test_select_with_one_workgroup_per_cu(monkeypatch, B, KH, g, W, D, S):
+    """Query images that leave room for one workgroup: one chunk of 768 columns, two of 768, many of 256 (over no more columns than the
+    bound on differing scores stands for, one in 4 200: over 8 200 it is 5 of 16 336 in whatever chunks)."""
+    check_select(monkeypatch, B, KH, g, W, D, S, 129, 5, 128, (0, B - 1))
+
+
 def check_select(monkeypatch, B, KH, g, W, D, S, budget, pool, page, requests):
     from magicdec_amd import ops
     H, ppr, dpr = KH * g, -(-S // page), budget // page + 1
