@@ -16,6 +16,8 @@
 // each behind them: 292 -> 16.5 + 5.9 us for the merge (first figure: the plain kernel, one workgroup per row and head).
 #include "xattn.h"
 
+#include <algorithm>
+
 namespace {
 
 template <typename T>
@@ -106,6 +108,8 @@ __global__ __launch_bounds__(256, (f32_waves_per_simd<DK, DV, QT, KT, SHARED>())
         for (int v = 0; v < NV; ++v) o[qt][v] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     vec4 kr[LK], vr[LV];
+    // A tile's last keys may be past the workgroup's last one: their rows are not read, and beyond the 16-key group that holds it neither
+    // staged nor multiplied (a sequence of a few keys costs what it has).
     auto request = [&](int t) {              // a tile's pieces into registers; its 32-key halves lie in one page each
         const T* kb[KT / 32];
         const T* vb[KT / 32];
@@ -121,7 +125,7 @@ __global__ __launch_bounds__(256, (f32_waves_per_simd<DK, DV, QT, KT, SHARED>())
             const int e = tid + 256 * i, row = e / (DK / 4), d = (e % (DK / 4)) * 4;
             const T* base = KT == 64 && row >= 32 ? kb[KT / 32 - 1] : kb[0];
             kr[i] = vec4{};
-            if (d < p.DKp) kr[i] = *reinterpret_cast<const vec4*>(base + (int64_t)(row % 32) * p.ldk + d);
+            if (d < p.DKp && t * KT + row <= hi_wg) kr[i] = *reinterpret_cast<const vec4*>(base + (int64_t)(row % 32) * p.ldk + d);
         }
         if constexpr (!SHARED) {
 #pragma unroll
@@ -129,7 +133,7 @@ __global__ __launch_bounds__(256, (f32_waves_per_simd<DK, DV, QT, KT, SHARED>())
                 const int e = tid + 256 * i, row = e / (DV / 4), d = (e % (DV / 4)) * 4;
                 const T* base = KT == 64 && row >= 32 ? vb[KT / 32 - 1] : vb[0];
                 vr[i] = vec4{};
-                if (d < p.DVp) vr[i] = *reinterpret_cast<const vec4*>(base + (int64_t)(row % 32) * p.ldv + d);
+                if (d < p.DVp && t * KT + row <= hi_wg) vr[i] = *reinterpret_cast<const vec4*>(base + (int64_t)(row % 32) * p.ldv + d);
             }
         }
     };
@@ -145,7 +149,7 @@ __global__ __launch_bounds__(256, (f32_waves_per_simd<DK, DV, QT, KT, SHARED>())
             f32x4 v = __builtin_convertvector(kr[i], f32x4);
             if (t * KT + row > hi_wg) v = f32x4{0.f, 0.f, 0.f, 0.f};
             if (SHARED) bad |= odd(v);
-            *reinterpret_cast<f32x4*>(sk + row * KP + d) = v;
+            if (t * KT + row <= (hi_wg | 15)) *reinterpret_cast<f32x4*>(sk + row * KP + d) = v;
         }
         if (SHARED && __builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) sbad[t & 1] = 1;
     };
@@ -157,7 +161,7 @@ __global__ __launch_bounds__(256, (f32_waves_per_simd<DK, DV, QT, KT, SHARED>())
             f32x4 v = __builtin_convertvector(vr[i], f32x4);
             if (t * KT + row > hi_wg) v = f32x4{0.f, 0.f, 0.f, 0.f};
             bad |= odd(v);
-            *reinterpret_cast<f32x4*>(sv + row * VP + d) = v;
+            if (t * KT + row <= (hi_wg | 15)) *reinterpret_cast<f32x4*>(sv + row * VP + d) = v;
         }
         if (__builtin_amdgcn_ballot_w64(bad) != 0 && lane == 0) sbad[t & 1] = 1;
     };
@@ -178,8 +182,9 @@ __global__ __launch_bounds__(256, (f32_waves_per_simd<DK, DV, QT, KT, SHARED>())
             const float* kp = sk + (kt * 16 + lq) * KP + lc * 4;
 #pragma unroll
             for (int i = 0; i < NS; ++i) s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const int dk = t * KT + kt * 16 <= hi_wg ? DK : 0;
 #pragma unroll 4
-            for (int d = 0; d < DK; d += 16) {
+            for (int d = 0; d < dk; d += 16) {
                 const f32x4 ka = *reinterpret_cast<const f32x4*>(kp + d);
 #pragma unroll
                 for (int i = 0; i < NS; ++i) {
@@ -252,6 +257,7 @@ __global__ __launch_bounds__(256, (f32_waves_per_simd<DK, DV, QT, KT, SHARED>())
         if (sbad[t & 1] == 0) {
 #pragma unroll
             for (int kk = 0; kk < KT; kk += 16) {
+                if (t * KT + kk > hi_wg) break;
                 f32x4 pb[QT];
 #pragma unroll
                 for (int qt = 0; qt < QT; ++qt) pb[qt] = *reinterpret_cast<const f32x4*>(sp + (qt * 16 + lq) * PP + kk + lc * 4);
@@ -363,16 +369,21 @@ Shape shape_of(const XattnParams& p) {
 
 F32Launch plan(const XattnParams& p, Shape s, long keys) {
     static const int wide[] = {0, 4, 4, 2, 2, 2}, dvw[] = {0, 64, 128, 256, 256, 512}, kt[] = {0, 64, 32, 32, 32, 32};
-    const int64_t rows = (int64_t)p.n_max * p.g;
+    const int64_t rows = (int64_t)p.n_max * p.g, items = (int64_t)p.KH * p.B, most = keys / (4 * kt[s]);
     F32Launch L;
-    L.R = 16 * (rows <= 16 ? 1 : wide[s]);
     L.dvw = dvw[s];
-    L.nq = (int)((rows + L.R - 1) / L.R);
-    // two workgroups per CU; a split has at least four tiles, so that its first loads and its share of the merge are a small part
-    const int64_t groups = (int64_t)L.nq * p.KH * p.B, want = groups > 0 ? (512 + groups - 1) / groups : 1, most = keys / (4 * kt[s]);
-    L.nsplit = (int)(want < most ? want : most);
-    if (L.nsplit < 1) L.nsplit = 1;
-    if (L.nsplit > 64) L.nsplit = 64;
+    auto with_rows = [&](int R) {
+        L.R = R;
+        L.nq = (int)((rows + R - 1) / R);
+        // two workgroups per CU; a split has at least four tiles, so that its first loads and its share of the merge are a small part
+        const int64_t groups = L.nq * items, want = groups > 0 ? (512 + groups - 1) / groups : 1;
+        L.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>({want, most, 64}));
+        return groups * L.nsplit;
+    };
+    // Wide row groups reuse a tile's keys, 16 rows are the shorter chain: ahead by a fifth to a third while the wide ones are not half as
+    // many workgroups as there are CUs (32 query heads of 64, 20 rows over 20 keys: 16.2 -> 11.6 us with the keys of a tile that are not
+    // there left out; 16 rows over 1 500: x 0.7), behind by as much from about 200 on (heads of 256: 150).
+    if (rows <= 16 || with_rows(16 * wide[s]) < 144) with_rows(16);
     return L;
 }
 

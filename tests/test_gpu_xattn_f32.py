@@ -29,6 +29,25 @@ def test_row_and_key_edges(ops, H, KH, D, DV, chunk, page):  # noqa: F811
         assert float((got.double() - want).abs().max()) <= lim and float((got - plain).abs().max()) <= lim, (n0, n1)
 
 
+@pytest.mark.parametrize("H,KH,D,DV,count", [(20, 4, 64, 64, 38), (20, 4, 128, 100, 38), (12, 4, 256, 256, 38), (20, 4, 64, 64, 35)])
+def test_wide_row_groups(ops, H, KH, D, DV, count):  # noqa: F811
+    """Many sequences of several rows: wide row groups from 144 of them on (the last case: 140), the last group and key tile of
+    each sequence partly filled, a sequence of one key among them."""
+    lens = [(17, 40, 64, 65, 90)[b % 5] for b in range(count)]
+    spec, rows, ref = attention_case(ops, H, KH, D, DV, 0, D, F32, lens)
+    s, who = Seqs(ops, spec, F32, lens, page=96, seed=2), list(range(count))
+    at = [n - min(n, 1 + 4 * (b % 4)) for b, n in enumerate(lens)]
+    at[3] = 0
+    s.attend(torch.cat([r[:n] for r, n in zip(rows, at)]), who, [0] * count, at)
+    part, new = torch.cat([r[n:] for r, n in zip(rows, at)]), [n - a for n, a in zip(lens, at)]
+    want = torch.cat([r[n:] for r, n in zip(ref, at)])
+    got, plain = (s.attend(part, who, at, new, plain=x) for x in (False, True))
+    lim = TOL * max(1.0, float(want.abs().max()))
+    assert float((got.double() - want).abs().max()) <= lim and float((got - plain).abs().max()) <= lim
+    one = Seqs(ops, spec, F32, [1] * count, page=96, seed=3).attend(torch.cat([r[:1] for r in rows]), who, [0] * count, [1] * count)
+    assert float((one.double() - torch.cat([r[:1] for r in ref])).abs().max()) <= lim
+
+
 @pytest.mark.parametrize("H,KH,D", [(4, 1, 64), (32, 1, 128), (2, 2, 256)])
 def test_kv_splits(ops, H, KH, D):  # noqa: F811
     """Few rows over many keys: the range is split over workgroups and merged, with and without a chunk that ends inside a split."""
