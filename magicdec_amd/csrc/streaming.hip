@@ -27,31 +27,34 @@ __device__ __forceinline__ int64_t slot_offset(int b, int s, int ppr, int page_s
     return ((int64_t)page * 2 * page_size + slot) * row_elems;
 }
 
-// A workgroup moves 8 adjacent 16-B columns (one 128-B line per row) of a request's k or v rows: 32 rows at a time, 8 such strips in
-// registers, i.e. 256 rows are requested at once, then -- when every wavefront has them -- written n_new rows further up.  Rows move
-// towards lower slots only, so a strip group never overwrites a row that a later one reads.  Bound by the latency of one round trip
-// per 256 rows (and HBM, 2 x 2 x budget rows, for large batches).  One thread per column walking the rows in eights (one workgroup per
-// request at 8 kv heads of 64) took 46.8 us for 16 requests of 257 rows, 15.8 MB moved; this takes 6.7.
-constexpr int kShiftCols = 8, kShiftRows = 256 / kShiftCols, kShiftStrips = 8;
+// A workgroup moves COLS adjacent 16-B columns (8: one 128-B line per row) of a request's k or v rows: 256 / COLS rows at a time, 8 such
+// strips in registers, requested at once, then -- when every wavefront has them -- written n_new rows further up.  Rows move towards
+// lower slots only, so a strip group never overwrites a row that a later one reads.  Bound by the latency of one round trip
+// per strip group while the rows fit the last-level cache: 8 columns, 256 rows a trip.  One thread per column walking the rows in eights
+// (one workgroup per request at 8 kv heads of 64) took 46.8 us for 16 requests of 257 rows, 15.8 MB moved; this takes 6.7.  Beyond it
+// bound by HBM, 2 x 2 x budget rows, which single lines reach less well than 512-B runs: 32 columns.
+constexpr int kShiftStrips = 8;
 
+template <int COLS>
 __global__ __launch_bounds__(256) void shift_append_kernel(const bf16_t* __restrict__ k_new,
                                                            const bf16_t* __restrict__ v_new, int64_t ks, int64_t vs,
                                                            bf16_t* cache, int n_new, int kv_len, int sink, int ppr,
                                                            int KH, int D, int page_size) {
+    constexpr int ROWS = 256 / COLS;
     const int b = blockIdx.y;
     const int row_elems = KH * D;
     const int cols = row_elems / 8;
-    const int t = blockIdx.x * kShiftCols + threadIdx.x % kShiftCols, strip = threadIdx.x / kShiftCols;
+    const int t = blockIdx.x * COLS + threadIdx.x % COLS, strip = threadIdx.x / COLS;
     const bool live = t < 2 * cols, isv = t >= cols;
     const int c = isv ? t - cols : t;
     const int64_t half = isv ? (int64_t)page_size * row_elems : 0;
     const bf16_t* nw = isv ? v_new : k_new;
     const int64_t ns = isv ? vs : ks;
-    for (int s0 = sink; s0 < kv_len; s0 += kShiftRows * kShiftStrips) {
+    for (int s0 = sink; s0 < kv_len; s0 += ROWS * kShiftStrips) {
         u32x4 buf[kShiftStrips];
 #pragma unroll
         for (int u = 0; u < kShiftStrips; ++u) {
-            const int s = s0 + u * kShiftRows + strip;
+            const int s = s0 + u * ROWS + strip;
             if (live && s < kv_len) {
                 const int src = s + n_new;
                 if (src < kv_len)
@@ -64,7 +67,7 @@ __global__ __launch_bounds__(256) void shift_append_kernel(const bf16_t* __restr
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < kShiftStrips; ++u) {
-            const int s = s0 + u * kShiftRows + strip;
+            const int s = s0 + u * ROWS + strip;
             if (live && s < kv_len)
                 *reinterpret_cast<u32x4*>(cache + slot_offset(b, s, ppr, page_size, row_elems) + half + c * 8) = buf[u];
         }
@@ -204,8 +207,14 @@ extern "C" int md_streaming_shift_append(const void* k_new, const void* v_new, i
                      v_row_stride % 8 == 0,
                  "md_streaming_shift_append: 16-byte alignment / stride multiple of 8 required");
     const int cols2 = 2 * KH * D / 8;
-    hipLaunchKernelGGL(shift_append_kernel, dim3((cols2 + kShiftCols - 1) / kShiftCols, B), dim3(256), 0, (hipStream_t)stream,
-                       (const bf16_t*)k_new, (const bf16_t*)v_new, k_row_stride, v_row_stride, (bf16_t*)cache, n_new,
+    // 512-B runs from two workgroups of them per CU and rows beyond the 256 MB of the last-level cache on: 64 requests of 1 025 rows, 32
+    // kv heads of 128, 482 us in 128-B lines, 411 (one thread per column: 409); 128 of 257, 32 of 128, 230, 203 (207).  Below, the long
+    // trips win: 128 requests of 257 rows, 8 kv heads of 64, 22 us, 26 in 512-B runs.
+    const int64_t wide = (int64_t)((cols2 + 31) / 32) * B;
+    const bool runs = wide >= 600 && wide * 512 * kv_len >= 266000000;
+    const int cols = runs ? 32 : 8;
+    hipLaunchKernelGGL(runs ? shift_append_kernel<32> : shift_append_kernel<8>, dim3((cols2 + cols - 1) / cols, B), dim3(256), 0,
+                       (hipStream_t)stream, (const bf16_t*)k_new, (const bf16_t*)v_new, k_row_stride, v_row_stride, (bf16_t*)cache, n_new,
                        kv_len, sink, pages_per_req, KH, D, page_size);
     MD_CHECK_LAUNCH("md_streaming_shift_append");
     return MD_OK;
