@@ -422,7 +422,7 @@ int pick_splits(int n_blocks, int K) {
 //   * slices: the even split that gives every CU a workgroup (pick_splits), unless that is a few workgroups more than there are CUs,
 //     whatever their waves, and slices of whole slabs, the last one shorter and at least a quarter fewer, keep to one each: K = 18 944 =
 //     148 slabs over 28 column blocks is 37 x 28 = 1 036 workgroups (load 1.24) or 9 x 28 = 252 (1.05).  It depends on N and K only, as
-//     the workspace does.  3584 x 18 944 37.1 -> 32.2 us at one row, 47.9 -> 35.8 at 64, 63.2 -> 42.9 at 128; 2048 x 5632 14.8 -> 13.2
+//     the planes' count does.  3584 x 18 944 37.1 -> 32.2 us at one row, 47.9 -> 35.8 at 64, 63.2 -> 42.9 at 128; 2048 x 5632 14.8 -> 13.2
 //     at 32; 2048 x 7680 19.2 -> 16.9 at 64, 39.0 -> 28.3 at 256;
 //   * waves: four, unless that leaves the most loaded CU more than 8 % above the mean and five to seven are better by 8 % (the split and
 //     the bits stay): 432 workgroups of four (two on 176 CUs, one on 80: load 1.19) are 247 of seven (1.04), 296 are 237 of five
@@ -435,7 +435,10 @@ double cu_load(int ntiles, int nslab, int nw, int S, int cus) {       // slabs o
     return (double)per_cu * nw * ((nslab + S - 1) / S) * cus / ((double)ntiles * nslab);
 }
 
-SkinnyPlan plan_of(int ntiles, int K, bool allow_nw) {
+// int8 weights (`rows8` = M, else 0) are half the loads in flight, and one four-wave workgroup per CU streams them slower than two: fewer
+// slices only where the planes they save are 0.3 of the weight's bytes or a slice is six slabs at most.  16 256 x 12 800 at 16 rows
+// 43.5 us in four slices, 64.6 in two; 3 072 x 7 552 at 16 rows 1.58 times faster in fewer.  Over 240 shapes 1.19 times faster than even slices.
+SkinnyPlan plan_of(int ntiles, int K, bool allow_nw, int rows8 = 0) {
     const int nslab = K / kSlabK, n_blocks = (ntiles + 3) / 4;
     SkinnyPlan pl;
     pl.nw = 4;
@@ -444,7 +447,8 @@ SkinnyPlan plan_of(int ntiles, int K, bool allow_nw) {
     const int fewer = (nslab + (nslab + most - 1) / most - 1) / ((nslab + most - 1) / most);
     double even = 1e30;
     for (int nw : {4, 5, 6, 7}) even = std::min(even, cu_load(ntiles, nslab, nw, pl.S, g_target_blocks));
-    if (4 * fewer <= 3 * pl.S && cu_load(ntiles, nslab, 4, fewer, g_target_blocks) <= even) pl.S = fewer;
+    const bool few_loads = rows8 && nslab > 6 * fewer && 80L * (pl.S - fewer) * rows8 < 3L * K;
+    if (4 * fewer <= 3 * pl.S && !few_loads && cu_load(ntiles, nslab, 4, fewer, g_target_blocks) <= even) pl.S = fewer;
     pl.kblk = (nslab + pl.S - 1) / pl.S * kSlabK;
     if (g_force_nw == 4 || !allow_nw) return pl;
     // compute units of the current device, queried once per device (a partitioned or smaller part must not be
@@ -588,7 +592,8 @@ extern "C" void md_debug_set_gemm_ring(int rd) { g_force_rd = (rd == 8 || rd == 
 
 extern "C" size_t md_linear_workspace_bytes(int M, int N, int K, int epilogue) {
     if (M <= 0 || N <= 0 || K <= 0 || K % kSlabK) return 0;
-    const int S = plan_of(wave_tiles(N, epilogue), K, false).S;     // the split does not depend on the waves per workgroup
+    // the split does not depend on the waves per workgroup; the weight's type is not among the arguments
+    const int tiles = wave_tiles(N, epilogue), S = std::max(plan_of(tiles, K, false).S, plan_of(tiles, K, false, M).S);
     return S > 1 ? (size_t)S * M * N * 4 : 0;     // fp32 partial sums of the K slices
 }
 
@@ -644,7 +649,7 @@ int linear_impl(const void* x, int64_t ldx, const void* w, int w_dtype, int w_pa
     }
     const bool w8 = w_dtype == MD_W_INT8;
     const int ntiles = wave_tiles(N, epilogue);
-    const SkinnyPlan pl = plan_of(ntiles, K, nw_allowed(M, w8));
+    const SkinnyPlan pl = plan_of(ntiles, K, nw_allowed(M, w8), w8 ? M : 0);
     const int n_blocks = (ntiles + pl.nw - 1) / pl.nw;
     p.S = pl.S;
     p.kblk = pl.kblk;
@@ -778,7 +783,7 @@ extern "C" int md_linear_add_rmsnorm(const void* x, int64_t ldx, const void* w, 
     p.skip_reduce = 1;
     const bool w8 = w_dtype == MD_W_INT8;
     const int ntiles = wave_tiles(N, EPI_NONE);
-    const SkinnyPlan pl = plan_of(ntiles, K, nw_allowed(M, w8));
+    const SkinnyPlan pl = plan_of(ntiles, K, nw_allowed(M, w8), w8 ? M : 0);
     const int n_blocks = (ntiles + pl.nw - 1) / pl.nw;
     p.S = pl.S;
     p.kblk = pl.kblk;

@@ -190,6 +190,20 @@ def test_linear_rejects_bad_arguments(ops):
         ops.linear(torch.zeros(4, 128, dtype=BF, device=DEV), torch.zeros(64, 128, dtype=torch.int8, device=DEV))
 
 
+@pytest.mark.parametrize("M,N,K", [(4, 2528, 21888), (256, 2528, 21888), (16, 3072, 7552), (7, 10400, 8960), (33, 2048, 5632)])
+def test_linear_int8_slices(ops, M, N, K):
+    """Even K slices or fewer, uneven ones, by rows and depth: float64 within fp32 sums (2^-24 a term, any order) and the two bf16
+    roundings of the result."""
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    wq = torch.randint(-128, 128, (N, K), generator=g, device=DEV, dtype=torch.int8)
+    sc = (torch.rand(N, generator=g, device=DEV) * 0.02 + 0.001).bfloat16()
+    got = ops.linear(x, ops.PackedWeight(wq), scales=sc, workspace=ops.AttnWorkspace(DEV)).double()
+    y, terms = (a.double() @ wq.double().abs().t() if i else x.double() @ wq.double().t() for i, a in enumerate((x, x.abs())))
+    want = y * sc.double()
+    assert bool(((got - want).abs() <= 2.0 ** -7 * want.abs() + K ** 0.5 * 2.0 ** -22 * terms * sc.double()).all())
+
+
 @pytest.mark.parametrize("M,N,K,int8", [(64, 2048, 8192, False), (256, 4096, 14336, False), (32, 1024, 2048, False),
                                         (100, 512, 1024, False), (64, 1024, 2048, True)])
 @pytest.mark.parametrize("packed", [False, True], ids=["rowmajor", "packed"])
