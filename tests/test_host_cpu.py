@@ -1665,6 +1665,10 @@ def test_weights_come_back_on_demand():
     assert all(torch.equal(t, x) for t, x in zip((w13, ff.w1.weight, ff.w3.weight), was))
     assert ff.w1.weight.data_ptr() == w13.data_ptr() and ff.w3.weight.data_ptr() == w13[512:].data_ptr()
     assert torch.equal(m._resident(wo), was[3])
+    size = lambda: sum(m._by_id[k].numel() * m._by_id[k].element_size() for k in m._released)
+    assert m.released_bytes == size() < m.packed_bytes + m.released_bytes
     m.restore_on_demand(False)
     m.release_rowmajor()
-    assert m._released == released
+    assert m._released == released and m.released_bytes == size() > 0
+    m.restore_rowmajor()
+    assert m.released_bytes == 0
