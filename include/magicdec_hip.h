@@ -307,6 +307,23 @@ int md_linear_block_add_rmsnorm(const void* x, int64_t ldx, const void* w_packed
                                 int K, void* workspace, size_t workspace_bytes, md_stream_t stream);
 
 /* ------------------------------------------------------------------------
+ * K8d  GEMM of a prompt's rows (csrc/promptgemm.hip)
+ *     reference: the nn.Linear calls of Transformer.prefill (Engine/SnapKV/model.py:288-289,446-455) over more rows than a step has
+ * out = epilogue(x[M][K] . W[N][K]^T + bias), W bf16 in the STREAMING layout of md_linear (packed for MD_EPI_SWIGLU where that or
+ * MD_EPI_GEGLU is the epilogue), K % 128 == 0, K >= 256, output columns a multiple of 8; rows of x and out 16-byte aligned, of less
+ * than 2^20 elements.  fp32 sums over k in one order, whatever the tile: the same bits from every tile.
+ *   MD_EPI_NONE    bf16(acc + bias)
+ *   MD_EPI_SWIGLU  bf16(bf16(silu(bf16(h1))) * bf16(h3))
+ *   2 (xIELU)      bf16(xielu(acc)): act = its two numbers, no bias
+ *   MD_EPI_GEGLU   bf16(gelu_tanh(h1) * h3)
+ * md_linear_prompt_supported: 1 if it takes the shape and is expected to be faster than a library GEMM (negative: no shape).  tile: 0, or 1000 * rows + columns
+ * of a tile (256 x 256, 192 x 256, 128 x 256, 256 x 128, 192 x 128, 128 x 128) instead of the one that the shape asks for.
+ * ---------------------------------------------------------------------- */
+int md_linear_prompt_supported(int M, int N, int K, int epilogue);
+int md_linear_prompt(const void* x, int64_t ldx, const void* w_packed, const void* bias, const float* act, void* out, int64_t ldo, int M,
+                     int N, int K, int epilogue, int tile, md_stream_t stream);
+
+/* ------------------------------------------------------------------------
  * K8b  fused small-problem linear: a linear of a decode / verify step TOGETHER with the op that consumes its output,
  *      one launch (csrc/tilegemm.hip; no split-K across workgroups, no workspace, deterministic)
  *     reference: Engine/SnapKV/model.py:322-336 (wqkv -> apply_rope -> update_kv), :260-278 (h = x + attention(...),

@@ -277,10 +277,10 @@ class _BackendBase:
 
     @contextlib.contextmanager
     def _prefilling(self):
-        """Around the portions of a prompt.  Their products run on the library GEMM over the row-major weights: the ones released after
-        the previous prompt come back as the portions ask for them (a head that only ever sees the last rows is not among them).  Behind
-        it, also where the prompt is refused: decode reads most weights in the streaming layout only, their row-major tensors are freed
-        (one resident copy), and the next step has its head."""
+        """Around the portions of a prompt.  Their products read the streaming layout (md_linear_prompt); for those that the library is left
+        with, the row-major weights released after the previous prompt come back as the portions ask for them.  Behind it, also where the
+        prompt is refused: decode reads most weights in the streaming layout only, their row-major tensors are freed (one resident copy),
+        and the next step has its head."""
         if hasattr(self.model, "restore_on_demand"):
             self.model.restore_on_demand(True)
         try:

@@ -26,8 +26,10 @@ every decode / verify shape of the 8B and 1B models timed on both, weights cycle
     and NOT the narrow projections, where splitting K over ~256 workgroups costs a partial-sum round trip the product is
     too small to pay for (wqkv 30-32 vs lib 27 + 6.3 for rope/append: a wash; wo 34-35 vs 25; every TP8 shard slower).
 
+  * the rows of a PROMPT (more than 256) go to md_linear_prompt (csrc/promptgemm.hip), which reads the streaming layout too: use_prompt.
+
 A weight a hand-written kernel will serve is re-packed once at setup_caches (Transformer._pack_weights); the row-major
-copy stays for the prefill-sized products.  MAGICDEC_GEMM=hip forces md_linear wherever it supports the shape,
+copy stays for the products that are left to the library.  MAGICDEC_GEMM=hip forces md_linear wherever it supports the shape,
 MAGICDEC_GEMM=lib forces the library, MAGICDEC_FUSED=0/1 switches md_linear_fused off / on everywhere (the A/B
 switches)."""
 import functools
@@ -87,6 +89,7 @@ def skinny_absorbs_norm(M: int) -> bool:
 def _changed():
     """A switch or the table of tuned solutions is another one."""
     _measured.cache_clear()
+    use_prompt.cache_clear()
 
 
 def set_mode(mode: str):
@@ -461,3 +464,13 @@ def choose(M: int, N: int, K: int, swiglu: bool, int8: bool, packed: bool, kind:
     if packed and not int8 and use_block(M, N, K, kind, absorbs_norm):
         return "block"
     return "skinny" if use_skinny(M, N, K, swiglu, int8, packed, kind, absorbs_norm) else "lib"
+
+
+@functools.lru_cache(maxsize=4096)
+def use_prompt(M: int, N: int, K: int, swiglu: bool = False) -> bool:
+    """md_linear_prompt for this linear (weight in the streaming layout) of more rows than a step has?  Where it takes the shape, but for a
+    few hundred rows of narrow and deep products (csrc/promptgemm.hip).  Against the library, 580 random products of 257 to 16 384 rows:
+    0.83 of its time with the activation behind it, 0.67 with the weight's rows brought back in front; 1.12 at the worst (12 800 x 2 048 x
+    5 632, 234 us)."""
+    from .. import ops
+    return _MODE != "lib" and M > 256 and ops.linear_prompt_supported(M, N, K, swiglu)

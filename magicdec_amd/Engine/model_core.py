@@ -14,8 +14,9 @@ token ids [B, n].  What differs from the reference is everything underneath:
   measured policy of Engine/gemm_policy.py picks: md_linear_fused (launch-bound small
   products: the product AND its consumer -- rope+append, residual add, SiLU*mul, the
   RMSNorm in front -- in one launch: a 1B draft layer is 5-7 launches), md_linear (long
-  weight streams; its split-K combine also adds the residual and normalises) or
-  hipBLASLt via F.linear (prefill-sized M, the M = 256 verify GEMMs) -- plus the
+  weight streams; its split-K combine also adds the residual and normalises),
+  md_linear_prompt (a prompt's rows, with the gated activation) or
+  hipBLASLt via F.linear (some M = 128..256 products, weights without a streaming copy) -- plus the
   attention and whatever the chosen linears did not absorb (rope+append, add+rmsnorm,
   silu*mul kernels);
 * the page table is read on the device by the attention kernel -- there is no
@@ -39,6 +40,7 @@ import torch.nn as nn
 from torch.nn import functional as F
 
 from .. import ops
+from .gemm_policy import use_prompt
 
 
 def find_multiple(n: int, k: int) -> int:
@@ -567,11 +569,12 @@ class Transformer(nn.Module):
         return y
 
     def _linear(self, x2d, lin, swiglu_w13=None, resid=None, want_ssq=False):
-        """One linear of a step.  Four implementations, chosen per shape by the measured rules of
+        """One linear of a step.  Five implementations, chosen per shape by the measured rules of
         Engine/gemm_policy.py: md_linear_fused (csrc/tilegemm.hip: the launch-bound small products -- draft-model
         linears, tensor-parallel shards -- in one launch together with their epilogue), md_linear_block
         (csrc/blockgemm.hip: the wide 129..256-row products of a verify step), md_linear (csrc/gemm.hip: the long weight
-        streams at <= 128 rows, split-K + combine) or the library GEMM (prefill-sized M, and whatever the A/B gave it).
+        streams at <= 128 rows, split-K + combine), md_linear_prompt (csrc/promptgemm.hip: more rows than a step has) or the
+        library GEMM (whatever the A/B gave it, weights without a streaming copy).
         `swiglu_w13 = (w13, s13)`: the fused w1|w3 product with the SiLU*mul epilogue.
         `resid`: return bf16(resid + linear) instead (the residual add of the block; only honoured by the fused
         kernel -- callers check `_fused_here` first); with `want_ssq` also the per-row partial sums of squares of the
@@ -593,6 +596,10 @@ class Transformer(nn.Module):
         kind = "swiglu" if swiglu else ("resid" if resid is not None else "plain")
         how = (choose(M, N, K, swiglu, w.dtype == torch.int8, pk is not None, kind, pro is not None and swiglu)
                if x2d.is_cuda else "lib")
+        if how == "lib" and x2d.is_cuda and self._on_prompt_gemm(x2d, w, pk, swiglu):
+            how = "prompt"
+        if how == "prompt":
+            return ops.linear_prompt(x2d if pro is None else pro.materialize(), pk, bias, swiglu)
         if how == "fused" and ops.fused_linear_supported(M, N, K):
             if pro is not None and not swiglu:
                 x2d, pro = pro.materialize(), None
@@ -618,6 +625,15 @@ class Transformer(nn.Module):
             inter = N // 2
             return ops.silu_mul(h[:, :inter], h[:, inter:])
         return h
+
+    @staticmethod
+    def _on_prompt_gemm(x2d, w, pk, swiglu=False):
+        """Do these rows (more than a step has) run on md_linear_prompt?  It reads the streaming layout: no row-major weight has to come
+        back.  The shapes alone decide, so that the ranks of a group agree."""
+        M, K = x2d.shape
+        return (M > 256 and pk is not None and w.dtype == torch.bfloat16 and x2d.dtype == torch.bfloat16 and x2d.stride(1) == 1
+                and x2d.stride(0) % 8 == 0 and x2d.stride(0) < 1 << 20 and x2d.data_ptr() % 16 == 0
+                and use_prompt(M, w.shape[0], K, swiglu))
 
     def _linear_how(self, M, N, K, swiglu, int8, pk, kind, has_pro):
         """Which implementation `_linear` ends up on for this shape: "fused" | "block" | "skinny" | "lib" -- the same

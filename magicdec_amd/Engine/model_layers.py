@@ -338,6 +338,8 @@ class LayeredTransformer(Transformer):
             return ops.linear_planes(inp, pk, how, self.workspace)
         if how == "rows":
             return ops.linear(inp, pk, workspace=self.workspace)
+        if inp.is_cuda and self._on_prompt_gemm(inp, lin.weight, pk):
+            return ops.linear_prompt(inp, pk)
         self._last_M = M
         return F.linear(inp, self._resident(lin.weight))
 
@@ -352,6 +354,8 @@ class LayeredTransformer(Transformer):
             return ops.linear_block(y, pk, workspace=self.workspace, xielu=act)
         if how == "skinny":
             return ops.linear(y, pk, workspace=self.workspace, xielu=act)
+        if y.is_cuda and self._on_prompt_gemm(y, lin.weight, pk):
+            return ops.linear_prompt(y, pk, xielu=act)
         self._last_M = M
         z = F.linear(y, self._resident(lin.weight))
         return ops.xielu(z, act, out=z)
@@ -361,7 +365,8 @@ class LayeredTransformer(Transformer):
         pk = self._packed.get(id(lin.weight))
         (M, K), N = y.shape, lin.weight.shape[0]
         how = self._linear_how(M, N, K, True, False, pk, "swiglu", False) if pk is not None and M <= 256 else "lib"
-        if out.stride(0) % 8 or out.data_ptr() % 16:
+        aligned = out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0
+        if not aligned:
             how = "lib"
         if how == "fused":
             return ops.fused_linear(y, pk, swiglu=True, gelu=True, out=out)
@@ -369,6 +374,8 @@ class LayeredTransformer(Transformer):
             return ops.linear_block(y, pk, swiglu=True, gelu=True, workspace=self.workspace, out=out)
         if how == "skinny":
             return ops.linear(y, pk, swiglu=True, gelu=True, workspace=self.workspace, out=out)
+        if aligned and y.is_cuda and out.stride(0) < 1 << 20 and self._on_prompt_gemm(y, lin.weight, pk, True):
+            return ops.linear_prompt(y, pk, swiglu=True, gelu=True, out=out)
         self._last_M = M
         z = F.linear(y, self._resident(lin.weight))
         return ops.gelu_mul(z[:, :N // 2], z[:, N // 2:], out=out)

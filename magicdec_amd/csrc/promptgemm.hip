@@ -1,0 +1,425 @@
+// GEMM of a prompt's rows (gfx950):  out = epilogue(x[M][K] . W[N][K]^T + bias), W in the streaming layout of md_linear
+//
+// replaces: the nn.Linear calls of a prompt (Engine/SnapKV/model.py:288-289 wqkv / wo, :446-455 w1 / w3 / w2), M of several hundred to
+//           16 384 rows, which ran on the library: over row-major weights that every prompt had to bring back from the streaming layout
+//           first (unpack_weight: 320 of 6 500 us of a two-layer 8B prompt), and with the gated activation as a pass of its own (260 us).
+//
+// What bounds it.  A full chip of matrix instructions is bound by power: the clock falls to about 1.75 of 2.4 GHz, and time is energy as much
+// as it is stalls.  v_mfma_f32_16x16x32 moves half the accumulator bytes per flop of 32x32x16 and is the faster one by clock, although its
+// 16 cycles hide less behind each (8192^3: 88 % of the cycles with the large one took as long as 82 % with the small one).  Measured, us:
+// (8192, 4096, 4096) 180, library 184; (8192, 4096, 14336) 612 / 604; (8192, 28672, 4096) with SiLU * mul 1 291 / 1 402;
+// (8196, 4096, 18432) 1 031 / 1 303; (6144, 2048, 8192) 135 / 152; (2081, 37888, 3584) 432 / 556.
+//   * four wavefronts of 256 rows x 64 columns, one per SIMD with 256 accumulators: each reads all of A from LDS and its own columns of W
+//     straight from memory, already in the instruction's order (W through LDS as well would need 2 048 of the 2 048 cycles that a step of
+//     64 takes there; 128 x 128 tiles per wavefront load W twice, which the address unit does not keep up with);
+//   * A by DMA through three buffers: by way of registers its LDS writes alone cost 12 % of the cycles;
+//   * W two steps of 64 ahead in registers, A two to three; one barrier a step, where the last LDS instruction lies some products back;
+//   * one instruction beside each product, in an order that the compiler has to keep (spread): in bunches the four wavefronts queue at the
+//     address unit and at LDS, and the matrix cores wait (1 195 -> 1 390 TFLOP/s at 8192 x 28 672 x 4 096);
+//   * workgroups stay and take tile after tile; the loads of the next tile are in flight behind the last steps of one;
+//   * an XCD's 32 workgroups take 8 row tiles x 4 column tiles, whose operands its L2 holds (4 or 16 row tiles: 1.5 / 4 % slower).
+#include "md_common.h"
+
+#include <algorithm>
+#include <type_traits>
+#include <utility>
+
+namespace {
+
+enum { PE_NONE = 0, PE_SWIGLU = 1, PE_XIELU = 2, PE_GEGLU = 3, PE_BIAS = 4 };
+
+struct PromptParams {
+    const bf16_t* x;
+    const bf16_t* w;        // [tiles of 32 columns][K/16][64 lanes][8]
+    const bf16_t* bias;     // [N] or null (PE_NONE)
+    const float* act;       // PE_XIELU
+    bf16_t* out;
+    int64_t ldx, ldo;
+    int M, K, Nout;         // output columns
+    unsigned w_bytes;
+    int wtiles;             // 32-column tiles of the weight
+    int mt, nt, total, per; // tiles of the launch, workgroups per XCD
+    int group;              // row tiles whose column tiles are walked together
+};
+
+constexpr int kBK = 64;
+constexpr int kGroup = 8;   // most row tiles in a group
+
+__device__ __forceinline__ unsigned int pack2(float a, float b) {
+    const bf16x2 v = {f32_to_bf16(a), f32_to_bf16(b)};
+    return *reinterpret_cast<const unsigned int*>(&v);
+}
+__device__ __forceinline__ float round_bf16(float a) { return bf16_to_f32(f32_to_bf16(a)); }
+// 1 / (1 + e^-z) on the transcendental unit (1 ulp each; the results are rounded to 16 bits)
+__device__ __forceinline__ float sigmoid_fast(float z) {
+    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.4426950408889634f));
+}
+
+// gelu_tanh on the transcendental unit
+__device__ __forceinline__ float gelu_fast(float z) { return z * sigmoid_fast(1.5957691216057308f * fmaf(0.044715f * z * z, z, z)); }
+// Xielu on it: e^z - 1 - z by its series near 0, where the difference would cancel
+__device__ __forceinline__ float xielu_fast(float ap, float an, float z) {
+    const float n = fminf(z, 0.f), n2 = n * n;
+    const float series = n2 * fmaf(n, fmaf(n, 1.0f / 24.0f, 1.0f / 6.0f), 0.5f);
+    const float e = n > -0.06f ? series : __builtin_amdgcn_exp2f(n * 1.4426950408889634f) - 1.0f - n;
+    return (z > 0.f ? ap * z * z : an * e) + 0.5f * z;
+}
+// f(0), f(1), ...: what a loop of this length is not always unrolled to
+template <int... I, class F>
+__device__ __forceinline__ void unrolled(std::integer_sequence<int, I...>, F f) {
+    (f(I), ...);
+}
+// f(k) for those of n things that lie behind place i of p, spread evenly; shift: 0 even places first, else odd ones
+template <class F>
+__device__ __forceinline__ void spread(int i, int p, int n, int shift, F f) {
+#pragma unroll
+    for (int k = 0; k < n; ++k)
+        if (min(k * p / n | shift, p - 1) == i) f(k);
+}
+__device__ __forceinline__ void wait_lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+template <int MT, int NT, int EPI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void prompt_gemm_kernel(const PromptParams p) {
+    constexpr int BM = 16 * MT, AL = BM / 32, AH = AL / 2;       // AL: 16-byte pieces of A per thread and step
+    constexpr int kBuf = BM * kBK * 2;
+    constexpr bool GATED = EPI == PE_SWIGLU || EPI == PE_GEGLU;
+    constexpr int CW = NT * (GATED ? 8 : 16), CH = CW / 8;       // columns of a wavefront's output, in 16-byte pieces
+    constexpr int P = MT * NT;                                   // products of half a step
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];      // 3 x [BM rows][8 chunks of 16 B], chunk ^ (row >> 1 & 7)
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, j = lane & 15, kq = lane >> 4;
+    const int grid = gridDim.x, first = (blockIdx.x & 7) * p.per + (blockIdx.x >> 3);
+    if (first >= p.total) return;
+    const int steps = p.K / kBK;
+    unsigned char* image = lds + 3 * kBuf + wave * (2 * 32 * CW * 2);
+
+    auto place = [&](int v, int& m, int& n) {
+        const int g = v / (p.group * p.nt), r = v - g * p.group * p.nt, rows = min(p.group, p.mt - g * p.group);
+        m = g * p.group + r % rows;
+        n = r / rows;
+    };
+
+    // ---- the two load streams.  A's descriptor ends with the rows (those behind them read as zeros), W's tiles behind the last are the last
+    const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(p.w), (short)0, (int)p.w_bytes, 0x00020000);
+    u32x4 ra;                                                    // A's descriptor: base, bytes, flags
+    unsigned ka, bbase[NT / 2], bnext[NT / 2];
+    const unsigned boff = (unsigned)((kq >> 1) * 1024 + (kq & 1) * 512 + j * 16);
+    unsigned aoff[AL];
+#pragma unroll
+    for (int i = 0; i < AL; ++i) aoff[i] = (unsigned)(((tid >> 3) + i * 32) * (int)p.ldx * 2 + (((tid & 7) ^ ((tid >> 4) & 7)) * 16));
+    auto seek_a = [&](int v) {
+        int m, n;
+        place(v, m, n);
+        const uint64_t base = (uint64_t)(p.x + (int64_t)m * BM * p.ldx);
+        ra = u32x4{(unsigned)base, (unsigned)(base >> 32) & 0xffffu, (unsigned)(min(p.M - m * BM, BM) * (int)p.ldx * 2), 0x00020000u};
+        ka = 0;
+    };
+    auto seek_b = [&](int v) {
+        int m, n;
+        place(v, m, n);
+#pragma unroll
+        for (int t = 0; t < NT / 2; ++t) bnext[t] = (unsigned)min((n * 4 + wave) * (NT / 2) + t, p.wtiles - 1) * (unsigned)(p.K * 64);
+    };
+    bf16x8 b[2][2][NT], a[MT];
+    // rows tid / 8 + 32 i to LDS, without a register between.  The DMA writes lane after lane: a lane fetches the piece that belongs at
+    // its place.  In assembly, since the compiler would have every LDS read wait for it; the waits are counted by hand (wait_a)
+    auto load_a = [&](unsigned buf, int i) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                     : : "s"(buf + (unsigned)(i * 4096 + wave * 1024)), "v"(aoff[i]), "s"(ra), "s"(ka) : "memory");
+    };
+    auto load_b = [&](int e, int h, const unsigned (&base)[NT / 2], int n) {
+        const u32x4 q = __builtin_amdgcn_raw_buffer_load_b128(rw, boff + h * 2048 + (n & 1) * 256, base[n >> 1], 0);
+        b[e][h][n] = *reinterpret_cast<const bf16x8*>(&q);
+    };
+    // ---- LDS addresses
+    unsigned raddr[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) raddr[h] = (unsigned)(j * 128 + (((4 * h + kq) ^ ((j >> 1) & 7)) * 16));
+    auto read_a = [&](unsigned buf, int h, int t) { a[t] = *reinterpret_cast<const bf16x8*>(lds + (raddr[h] + buf) + t * 2048); };
+    f32x4 acc[NT][MT];
+    // the products of half h of a step of parity e, each followed by what `beside` issues there: an order that the compiler keeps
+    auto half = [&](int e, int h, auto beside) {
+        unrolled(std::make_integer_sequence<int, P>(), [&](int i) __attribute__((always_inline)) {
+            const int t = i / NT, n = t & 1 ? NT - 1 - i % NT : i % NT;
+            // (in assembly: left to the compiler, accumulators of four registers wander, by 200 moves a step)
+            asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[n][t]) : "v"(b[e][h][n]), "v"(a[t]));
+            beside(i);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    // A of this step, of the next and of the one after it: places in LDS
+    unsigned buf0 = 0, buf1 = kBuf, buf2 = 2 * kBuf;
+    // step e of a pair: its products, A of the second and third step ahead, W of the second
+    auto step = [&](auto parity, auto turn) {
+        constexpr int e = decltype(parity)::value, o = 1 - e;
+        half(e, 0, [&](int i) {
+            if (i % NT == NT - 1) read_a(buf0, 1, i / NT);
+            spread(i, P, AL - AH + NT, 1, [&](int x) { if (x < NT) load_b(o, 1, bbase, x); else load_a(buf2, AH + x - NT); });
+        });
+        turn();
+        half(e, 1, [&](int i) {
+            // Behind the barrier no wavefront reads A of this step any more, and A of the next is there: of the loads in flight at most
+            // those of two halves are younger.  It stands where the last LDS instruction lies a few products back
+            if (i == 2 * NT - 1) {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NT + AL) : "memory");
+                wait_lds_barrier();
+            }
+            if (i == 2 * NT || i == 2 * NT + 1) read_a(buf1, 0, i - 2 * NT);
+            if (i >= 2 * NT && i % NT == NT - 1) read_a(buf1, 0, i / NT);
+            spread(i - 2 * NT, P - 2 * NT, AH + NT, 1, [&](int x) { if (x < NT) load_b(e, 0, bnext, x); else load_a(buf0, x - NT); });
+        });
+        const unsigned done = buf0;
+        buf0 = buf1;
+        buf1 = buf2;
+        buf2 = done;
+        asm volatile("" ::: "memory");
+    };
+    auto advance_b = [&]() {
+#pragma unroll
+        for (int t = 0; t < NT / 2; ++t) {
+            bbase[t] = bnext[t];
+            bnext[t] += 4096;
+        }
+    };
+    // ---- what is in flight when the first step begins, in the loop's order: the waits there count the loads behind what they wait for
+    auto ask = [&](auto f, int from, int to) {
+#pragma unroll
+        for (int i = from; i < to; ++i) {
+            f(i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    seek_a(first);
+    seek_b(first);
+    ask([&](int i) { load_a(buf0, i); }, 0, AL);
+    ka += kBK * 2;
+    ask([&](int i) { load_a(buf1, i); }, 0, AL);
+    ask([&](int i) { load_b(0, 0, bnext, i); }, 0, NT);
+    ka += kBK * 2;
+    ask([&](int i) { load_b(0, 1, bnext, i); }, 0, NT);
+    ask([&](int i) { load_a(buf2, i); }, 0, AH);
+#pragma unroll
+    for (int t = 0; t < NT / 2; ++t) bnext[t] += 4096;
+    ask([&](int i) { load_b(1, 0, bnext, i); }, 0, NT);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AL + AH + 3 * NT) : "memory");
+    wait_lds_barrier();
+    ask([&](int i) { read_a(buf0, 0, i); }, 0, MT);
+
+    float act_p = 0.f, act_n = 0.f;
+    if constexpr (EPI == PE_XIELU) {
+        const Xielu f(p.act);
+        act_p = f.ap;
+        act_n = f.an;
+    }
+    for (int v = first; v < p.total; v += grid) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[n][t][r] = 0.f;
+        asm volatile("s_nop 7" ::: "memory");
+        const int next = v + grid < p.total ? v + grid : first;       // (behind the last tile: rows that exist, and are not used)
+        for (int k = 0; k < steps; k += 2) {
+            advance_b();
+            if (__builtin_expect(k == steps - 2, 0)) seek_b(next);
+            __builtin_amdgcn_sched_barrier(0);
+            step(std::integral_constant<int, 0>(), [&]() { ka += kBK * 2; });
+            advance_b();
+            __builtin_amdgcn_sched_barrier(0);
+            step(std::integral_constant<int, 1>(), [&]() {
+                ka += kBK * 2;
+                if (__builtin_expect(k == steps - 4, 0)) seek_a(next);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        }
+        // (the products are assembly: what the compiler would wait between the last of them and reading its accumulator)
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        // ---- out.  Lane (j, kq) has row j of a row tile and columns 4 kq .. + 3 of each column tile.  The wavefront's columns of 32 rows
+        // go through LDS, so that a store writes whole lines (16 bytes of 32 rows each took 9 us a tile)
+        int m, n0;
+        place(v, m, n0);
+        const int rows_left = min(p.M - m * BM, BM);
+        const __amdgpu_buffer_rsrc_t rsrc =
+            __builtin_amdgcn_make_buffer_rsrc((void*)(p.out + (int64_t)m * BM * p.ldo), (short)0, rows_left * (int)p.ldo * 2, 0x00020000);
+        const int col = (n0 * 4 + wave) * CW + (lane % CH) * 8;
+        const unsigned at = col < p.Nout ? (unsigned)((lane / CH) * (int)p.ldo + col) * 2 : 0xc0000000u;     // (past the end: not stored)
+        auto put = [&](int t) {
+            unsigned char* slot = image + (t >> 1 & 1) * (32 * CW * 2);
+            const int row = (t & 1) * 16 + j;
+            constexpr int OT = GATED ? NT / 2 : NT;
+#pragma unroll
+            for (int n = 0; n < OT; ++n) {
+                float z[4], g[4], o[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(z[r]) : "a"(acc[GATED ? 2 * n : n][t][r]));
+                    if constexpr (GATED) asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(g[r]) : "a"(acc[2 * n + 1][t][r]));
+                }
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if constexpr (EPI == PE_SWIGLU) {
+                        const float h1 = round_bf16(z[r]), h3 = round_bf16(g[r]);
+                        o[r] = round_bf16(h1 * sigmoid_fast(h1)) * h3;
+                    } else if constexpr (EPI == PE_GEGLU) {
+                        o[r] = gelu_fast(z[r]) * g[r];
+                    } else if constexpr (EPI == PE_XIELU) {
+                        o[r] = xielu_fast(act_p, act_n, z[r]);
+                    } else if constexpr (EPI == PE_BIAS) {
+                        o[r] = z[r] + bf16_to_f32(p.bias[min((n0 * 4 + wave) * CW + n * 16 + kq * 4 + r, p.Nout - 1)]);
+                    } else {
+                        o[r] = z[r];
+                    }
+                }
+                const int chunk = 2 * n + (kq >> 1);
+                *reinterpret_cast<u32x2*>(slot + row * (CW * 2) + ((chunk ^ (row / (16 / CH) & (CH - 1))) * 16) + (kq & 1) * 8) =
+                    u32x2{pack2(o[0], o[1]), pack2(o[2], o[3])};
+            }
+        };
+        auto take = [&](int t) {
+            const unsigned char* slot = image + (t & 1) * (32 * CW * 2);
+#pragma unroll
+            for (int i = 0; i < CH / 2; ++i) {
+                const int r = lane / CH + i * (64 / CH), c = lane % CH;
+                const u32x4 q = *reinterpret_cast<const u32x4*>(slot + r * (CW * 2) + ((c ^ (r / (16 / CH) & (CH - 1))) * 16));
+                __builtin_amdgcn_raw_buffer_store_b128(q, rsrc, at + (unsigned)((t * 32 + i * (64 / CH)) * (int)p.ldo * 2), 0, 0);
+            }
+        };
+#pragma unroll
+        for (int t = 0; t < MT / 2; ++t) {
+            put(2 * t);
+            put(2 * t + 1);
+            if (t > 0) take(t - 1);
+        }
+        take(MT / 2 - 1);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // (the DMA of steps that do not come: not into another workgroup's LDS)
+}
+
+// Tiles: rows x columns, and what one takes: us before the first step of 64 and behind the last, us a step while most CUs idle, and how much
+// slower that is with all of them busy (the clock).  Drawn from 970 random products (257 to 16 384 rows, 33 weights of 768 x 768 to
+// 128 256 x 2 048); the tile that this picks is within 0.5 % of the best on average, 18 % at the worst.
+struct Tile {
+    int rows, cols;
+    double fixed, step, busy;
+};
+constexpr Tile kTiles[] = {{256, 256, 8.9, 0.908, 1.41}, {192, 256, 7.8, 0.694, 1.41}, {128, 256, 6.0, 0.500, 1.42},
+                           {256, 128, 5.1, 0.647, 1.22}, {192, 128, 4.5, 0.534, 1.17}, {128, 128, 3.0, 0.464, 1.05}};
+
+double tile_us(const Tile& t, int M, int64_t cols, int K) {
+    const int64_t total = (int64_t)((M + t.rows - 1) / t.rows) * ((cols + t.cols - 1) / t.cols), rounds = total / 256, rest = total % 256;
+    const double body = (double)(K / kBK) * t.step;
+    double us = (double)rounds * (t.fixed + body * t.busy);
+    if (rest) us += t.fixed + body * (1.0 + (t.busy - 1.0) * (double)rest / 256);
+    return us;
+}
+
+const Tile& best_tile(int M, int64_t cols, int K, double* us) {
+    const Tile* best = nullptr;
+    for (const Tile& t : kTiles) {
+        const double c = tile_us(t, M, cols, K);
+        if (!best || c < *us) {
+            best = &t;
+            *us = c;
+        }
+    }
+    return *best;
+}
+
+bool shape_ok(int M, int N, int K, bool gated) {
+    const int nout = gated ? N / 2 : N;
+    const size_t tiles = gated ? (nout + 15) / 16 : (nout + 31) / 32;
+    return M > 0 && N > 0 && (!gated || N % 2 == 0) && nout % 8 == 0 && K >= 4 * kBK && K % (2 * kBK) == 0 && K < (1 << 20) &&
+           nout < (1 << 20) && tiles * K * 64 < ((size_t)1 << 32);
+}
+
+template <int MT, int NT, int EPI>
+int launch_tile(PromptParams& p, hipStream_t st) {
+    constexpr int bm = 16 * MT, bn = 64 * NT;
+    constexpr bool gated = EPI == PE_SWIGLU || EPI == PE_GEGLU;
+    p.mt = (p.M + bm - 1) / bm;
+    p.nt = (p.wtiles * 32 + bn - 1) / bn;
+    const int groups = (p.mt + kGroup - 1) / kGroup;
+    p.group = (p.mt + groups - 1) / groups;                    // (9 row tiles: 5 and 4, not 8 and one that has W to itself)
+    p.total = p.mt * p.nt;
+    p.per = (std::min(p.total, 256) + 7) / 8;
+    constexpr int bytes = 3 * bm * kBK * 2 + 2 * 32 * (gated ? bn / 2 : bn) * 2;      // A's buffers; two images of 32 rows of each wavefront
+    static MdPerDeviceOnce once;
+    if (once.first() && hipFuncSetAttribute(reinterpret_cast<const void*>(&prompt_gemm_kernel<MT, NT, EPI>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
+        once.undo();
+        md_set_error("md_linear_prompt: hipFuncSetAttribute(%d B LDS) failed", bytes);
+        return MD_ERR_LAUNCH;
+    }
+    hipLaunchKernelGGL((prompt_gemm_kernel<MT, NT, EPI>), dim3(8 * p.per), dim3(256), bytes, st, p);
+    return MD_OK;
+}
+
+template <int EPI>
+int launch(PromptParams& p, int rows, int cols, hipStream_t st) {
+    if (rows == 256 && cols == 256) return launch_tile<16, 4, EPI>(p, st);
+    if (rows == 192 && cols == 256) return launch_tile<12, 4, EPI>(p, st);
+    if (rows == 128 && cols == 256) return launch_tile<8, 4, EPI>(p, st);
+    if (rows == 256 && cols == 128) return launch_tile<16, 2, EPI>(p, st);
+    if (rows == 192 && cols == 128) return launch_tile<12, 2, EPI>(p, st);
+    if (rows == 128 && cols == 128) return launch_tile<8, 2, EPI>(p, st);
+    md_set_error("md_linear_prompt: no tile of %d x %d", rows, cols);
+    return MD_ERR_UNSUPPORTED;
+}
+
+}  // namespace
+
+// (its workgroups take all of K: a few hundred rows of a narrow and deep product leave most CUs idle, 374 x 2 048 x 10 240 in 75 us where
+// the library's split of K takes 41, or 61 with the weight's rows to bring back.  The line is where those cross over the same products)
+extern "C" int md_linear_prompt_supported(int M, int N, int K, int epilogue) {
+    const bool gated = epilogue == PE_SWIGLU || epilogue == PE_GEGLU;
+    MD_CHECK_ARG(M > 0 && N > 0 && K > 0, "md_linear_prompt_supported: M=%d N=%d K=%d", M, N, K);
+    if (!shape_ok(M, N, K, gated)) return 0;
+    double us = 0;
+    best_tile(M, N, K, &us);
+    return us <= 2.4 * (2e-6 * M * N / 1400 * K + 12) ? 1 : 0;
+}
+
+extern "C" int md_linear_prompt(const void* x, int64_t ldx, const void* w_packed, const void* bias, const float* act, void* out, int64_t ldo,
+                                int M, int N, int K, int epilogue, int tile, md_stream_t stream) {
+    MD_CHECK_ARG(x && w_packed && out, "md_linear_prompt: null pointer argument");
+    const bool gated = epilogue == PE_SWIGLU || epilogue == PE_GEGLU;
+    MD_CHECK_ARG(shape_ok(M, N, K, gated), "md_linear_prompt: M=%d N=%d K=%d unsupported", M, N, K);
+    PromptParams p;
+    p.x = (const bf16_t*)x;
+    p.w = (const bf16_t*)w_packed;
+    p.bias = (const bf16_t*)bias;
+    p.act = act;
+    p.out = (bf16_t*)out;
+    p.ldx = ldx;
+    p.ldo = ldo;
+    p.M = M;
+    p.K = K;
+    p.Nout = gated ? N / 2 : N;
+    p.wtiles = gated ? (p.Nout + 15) / 16 : (N + 31) / 32;
+    p.w_bytes = (unsigned)((size_t)p.wtiles * K * 64);
+    // (32-bit offsets within a row tile: rows of less than 2^20 elements)
+    MD_CHECK_ARG(ldx >= K && ldx % 8 == 0 && ldx < (1 << 20) && ldo >= p.Nout && ldo % 8 == 0 && ldo < (1 << 20) &&
+                     (((uintptr_t)x | (uintptr_t)out | (uintptr_t)w_packed) & 15) == 0,
+                 "md_linear_prompt: x, out and w_packed must be 16-byte aligned, their rows a multiple of 8 and of less than 2^20 elements");
+    MD_CHECK_ARG(epilogue == PE_NONE || !bias, "md_linear_prompt: a bias goes with no epilogue only");
+    MD_CHECK_ARG((epilogue == PE_XIELU) == (act != nullptr), "md_linear_prompt: act goes with the xIELU epilogue");
+    double us = 0;
+    const Tile& t = best_tile(M, (int64_t)p.wtiles * 32, K, &us);
+    const int rows = tile ? tile / 1000 : t.rows, cols = tile ? tile % 1000 : t.cols;
+    hipStream_t st = (hipStream_t)stream;
+    int rc;
+    switch (epilogue) {
+        case PE_NONE: rc = bias ? launch<PE_BIAS>(p, rows, cols, st) : launch<PE_NONE>(p, rows, cols, st); break;
+        case PE_SWIGLU: rc = launch<PE_SWIGLU>(p, rows, cols, st); break;
+        case PE_XIELU: rc = launch<PE_XIELU>(p, rows, cols, st); break;
+        case PE_GEGLU: rc = launch<PE_GEGLU>(p, rows, cols, st); break;
+        default: md_set_error("md_linear_prompt: unknown epilogue %d", epilogue); return MD_ERR_INVALID_ARG;
+    }
+    if (rc != MD_OK) return rc;
+    MD_CHECK_LAUNCH("md_linear_prompt");
+    return MD_OK;
+}

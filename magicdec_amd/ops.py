@@ -587,6 +587,39 @@ def linear_block_add_rmsnorm(x, weight: "PackedWeight", resid, norm_weight, eps,
     return h, y
 
 
+# ----------------------------------------------------------------------------- K8d
+PE_NONE, PE_SWIGLU, PE_XIELU, PE_GEGLU = 0, 1, 2, 3
+
+
+def linear_prompt_supported(M, N, K, swiglu=False):
+    """True when md_linear_prompt (csrc/promptgemm.hip: the GEMM of a prompt's rows) takes this shape and is expected to be
+    faster than the library."""
+    return _lib.load().md_linear_prompt_supported(int(M), int(N), int(K), PE_SWIGLU if swiglu else PE_NONE) > 0
+
+
+def linear_prompt(x, weight: "PackedWeight", bias=None, swiglu=False, out=None, xielu=None, gelu=False, tile=0):
+    """F.linear(x, W, bias) -- or the activation of it, as linear() -- for the rows of a prompt on md_linear_prompt.
+    tile: 1000 * rows + columns of one of its tiles, 0: chosen by the shape."""
+    M, N, K = _block_args(x, weight, swiglu)
+    if bias is not None:
+        _gpu(bias)
+        if bias.dtype != torch.bfloat16 or bias.numel() != N or not bias.is_contiguous():
+            raise ValueError(f"linear_prompt: bias must be a contiguous bf16 vector of {N} elements")
+    n_out = N // 2 if swiglu else N
+    if out is None:
+        out = torch.empty((M, n_out), dtype=x.dtype, device=x.device)
+    else:
+        _gpu(out)
+        if out.dtype != torch.bfloat16 or out.dim() != 2 or out.shape != (M, n_out) or out.stride(1) != 1:
+            raise ValueError("linear_prompt: out must be bf16 [M, N_out] with unit inner stride")
+    if gelu and not swiglu or xielu is not None and (swiglu or bias is not None):
+        raise ValueError("linear_prompt: gelu goes with swiglu, the xIELU epilogue takes nothing beside it")
+    epi = PE_XIELU if xielu is not None else PE_NONE if not swiglu else PE_GEGLU if gelu else PE_SWIGLU
+    check(_lib.load().md_linear_prompt(_p(x), x.stride(0), _p(weight.data), _p(bias), _act_numbers(xielu) if xielu is not None else None,
+                                       _p(out), out.stride(0), M, N, K, epi, int(tile), _stream()), "md_linear_prompt")
+    return out
+
+
 # ----------------------------------------------------------------------------- K8b
 FL_NONE, FL_SWIGLU, FL_RESID, FL_ROPE_APPEND, FL_XIELU, FL_GEGLU = 0, 1, 2, 3, 4, 5
 

@@ -1,0 +1,98 @@
+"""md_linear_prompt (csrc/promptgemm.hip) against float64 products, at the edges of its tiles.  On the GPU (-m gpu)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+TILES = (0, 256256, 192256, 128256, 256128, 192128, 128128)
+
+
+def case(M, N, K, seed, ldx=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(M, K + ldx, device=DEV, generator=g).bfloat16()[:, :K]
+    return x, (torch.randn(N, K, device=DEV, generator=g) * 0.1).bfloat16(), torch.randn(N, device=DEV, generator=g).bfloat16()
+
+
+def product(x, w):
+    """(float64 product, bound on what fp32 sums of K terms are off it)"""
+    return x.double() @ w.double().t(), (x.double().abs() @ w.double().abs().t()) * (x.shape[1] * 2.0 ** -24)
+
+
+U = 2.0 ** -8            # half an ulp of bf16 relative to the value: 8 significant bits, the spacing in [1, 2) is 2^-7
+
+
+# rows and columns around a tile's and a wavefront's edge, one row, one piece of 8 columns, several tiles per workgroup, K of 4 and 6 steps
+@pytest.mark.parametrize("M,N,K,ldx", [(1, 8, 256, 0), (257, 264, 256, 8), (300, 520, 384, 0), (127, 1000, 640, 64), (769, 96, 512, 0),
+                                       (2049, 1032, 256, 0), (1000, 20000, 256, 0)])
+def test_products(M, N, K, ldx):
+    from magicdec_amd import ops
+    x, w, bias = case(M, N, K, M, ldx)
+    ref, off = product(x, w)
+    plain = ops.PackedWeight(w)
+    first = None
+    for tile in TILES:
+        wide = torch.full((M + 1, N + 16), -7.0, device=DEV, dtype=torch.bfloat16)
+        out = ops.linear_prompt(x, plain, out=wide[:M, 8:8 + N], tile=tile)
+        assert ((out.double() - ref).abs() <= ref.abs() * U + 2 * off).all()
+        assert (wide[M] == -7).all() and (wide[:, :8] == -7).all() and (wide[:, 8 + N:] == -7).all()       # nothing beside it
+        first = out.clone() if first is None else first
+        assert torch.equal(out, first)                                                                    # the same bits from every tile
+        got = ops.linear_prompt(x, plain, bias, tile=tile)
+        want = ref + bias.double()
+        assert ((got.double() - want).abs() <= want.abs() * U + 2 * off + 2.0 ** -23 * bias.double().abs()).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(257, 272, 256), (129, 2000, 384), (1025, 1040, 512), (2100, 12000, 256)])
+def test_activations(M, N, K):
+    from magicdec_amd import ops
+    x, w, _ = case(M, N, K, N)
+    ref, off = product(x, w)
+    act = torch.tensor([0.3, -0.2], device=DEV)
+    a, b = torch.nn.functional.softplus(act.double())
+    low = ref.clamp(max=0)
+    z = ref / 2 + torch.where(ref > 0, a * ref * ref, (0.5 + b) * (torch.expm1(low) - low))
+    slope = 0.5 + torch.where(ref > 0, 2 * a * ref, (0.5 + b) * (torch.exp(low) - 1).abs())
+    h1, h3, o1, o3 = ref[:, :N // 2], ref[:, N // 2:], off[:, :N // 2], off[:, N // 2:]
+    s = torch.sigmoid(h1)
+    silu, dsilu = h1 * s, (s * (1 + h1 * (1 - s))).abs()
+    gelu = torch.nn.functional.gelu(h1, approximate="tanh")
+    for tile in TILES:
+        got = ops.linear_prompt(x, ops.PackedWeight(w), xielu=act, tile=tile).double()
+        # (the exponential's argument and result: 2 ulp of float)
+        assert ((got - z).abs() <= z.abs() * U + slope * 2 * off + 2.0 ** -22 * (1 + ref.abs())).all()
+        gated = ops.PackedWeight(w, swiglu=True)
+        got = ops.linear_prompt(x, gated, swiglu=True, tile=tile).double()
+        # rounded: h1, h3, silu(h1), the product
+        bound = (dsilu * (h1.abs() * U + 2 * o1) * h3.abs() + silu.abs() * 2 * o3 + 3 * U * (silu * h3).abs()) * 1.02 + 1e-30
+        assert ((got - silu * h3).abs() <= bound).all()
+        got = ops.linear_prompt(x, gated, swiglu=True, gelu=True, tile=tile).double()
+        bound = 1.13 * 2 * o1 * h3.abs() + gelu.abs() * 2 * o3 + U * (gelu * h3).abs() + 2.0 ** -20 * (1 + h1.abs()) * h3.abs()
+        assert ((got - gelu * h3).abs() <= bound).all()
+
+
+def test_not_finite():
+    """An infinity or NaN of a row stays in it; a saturated activation is 0 or its argument."""
+    from magicdec_amd import ops
+    x, w, _ = case(300, 64, 256, 3)
+    x[7, 5], x[200, 100] = float("inf"), float("nan")
+    out = ops.linear_prompt(x, ops.PackedWeight(w))
+    bad = ~torch.isfinite(out).all(1)
+    assert bad[7] and bad[200] and bad.sum() == 2
+    big = torch.full((300, 256), 1.0, device=DEV).bfloat16()
+    w = torch.cat([torch.full((8, 256), -1.0), torch.full((8, 256), 1.0), torch.full((16, 256), 0.5)]).to(DEV).bfloat16()     # h1 = -256, 256
+    for gelu in (False, True):
+        out = ops.linear_prompt(big, ops.PackedWeight(w, swiglu=True), swiglu=True, gelu=gelu)
+        assert (out[:, :8] == 0).all() and (out[:, 8:] == 256 * 128).all()
+
+
+def test_refused():
+    from magicdec_amd import ops
+    x, w, bias = case(300, 64, 256, 5)
+    pw = ops.PackedWeight(w)
+    for call in (lambda: ops.linear_prompt(x[:, :192], ops.PackedWeight(w[:, :192].contiguous())),            # K of an odd number of steps
+                 lambda: ops.linear_prompt(x, ops.PackedWeight(w[:60].contiguous())),                       # columns: no multiple of 8
+                 lambda: ops.linear_prompt(x, pw, tile=64064),
+                 lambda: ops.linear_prompt(x, pw, bias[:32]),
+                 lambda: ops.linear_prompt(x, pw, out=torch.empty(300, 68, device=DEV, dtype=torch.bfloat16)[:, 2:66])):       # alignment
+        with pytest.raises((RuntimeError, ValueError)):
+            call()
