@@ -310,7 +310,7 @@ int md_linear_block_add_rmsnorm(const void* x, int64_t ldx, const void* w_packed
  * K8d  GEMM of a prompt's rows (csrc/promptgemm.hip)
  *     reference: the nn.Linear calls of Transformer.prefill (Engine/SnapKV/model.py:288-289,446-455) over more rows than a step has
  * out = epilogue(x[M][K] . W[N][K]^T + bias), W bf16 in the STREAMING layout of md_linear (packed for MD_EPI_SWIGLU where that or
- * MD_EPI_GEGLU is the epilogue), K % 128 == 0, K >= 256, output columns a multiple of 8; rows of x and out 16-byte aligned, of less
+ * MD_EPI_GEGLU is the epilogue), K % 256 == 0, output columns a multiple of 8; rows of x and out 16-byte aligned, of less
  * than 2^20 elements.  fp32 sums over k in one order, whatever the tile: the same bits from every tile.
  *   MD_EPI_NONE    bf16(acc + bias)
  *   MD_EPI_SWIGLU  bf16(bf16(silu(bf16(h1))) * bf16(h3))

@@ -469,8 +469,8 @@ def choose(M: int, N: int, K: int, swiglu: bool, int8: bool, packed: bool, kind:
 @functools.lru_cache(maxsize=4096)
 def use_prompt(M: int, N: int, K: int, swiglu: bool = False) -> bool:
     """md_linear_prompt for this linear (weight in the streaming layout) of more rows than a step has?  Where it takes the shape, but for a
-    few hundred rows of narrow and deep products (csrc/promptgemm.hip).  Against the library, 580 random products of 257 to 16 384 rows:
-    0.83 of its time with the activation behind it, 0.67 with the weight's rows brought back in front; 1.12 at the worst (12 800 x 2 048 x
-    5 632, 234 us)."""
+    few hundred rows of narrow and deep products (csrc/promptgemm.hip).  Against the library, 435 random products of 257 to 16 384 rows:
+    0.77 of its time with the activation behind it, 0.61 with the weight's rows brought back in front; 1.11 at the worst (12 719 x 2 048 x
+    8 192, 341 us)."""
     from .. import ops
     return _MODE != "lib" and M > 256 and ops.linear_prompt_supported(M, N, K, swiglu)

@@ -13,7 +13,9 @@
 //     straight from memory, already in the instruction's order (W through LDS as well would need 2 048 of the 2 048 cycles that a step of
 //     64 takes there; 128 x 128 tiles per wavefront load W twice, which the address unit does not keep up with);
 //   * A by DMA through three buffers: by way of registers its LDS writes alone cost 12 % of the cycles;
-//   * W two steps of 64 ahead in registers, A two to three; one barrier a step, where the last LDS instruction lies some products back;
+//   * W four steps of 64 ahead in registers (two: 1 024 x 4 096 x 4 096 in 37.6 us instead of 31.6, 6 144 x 3 072 x 2 048 in 70.2 instead of
+//     64.2, the large ones 1 % slower), A two to three in LDS and half a step in registers; one barrier a step, where the last LDS
+//     instruction lies some products back;
 //   * one instruction beside each product, in an order that the compiler has to keep (spread): in bunches the four wavefronts queue at the
 //     address unit and at LDS, and the matrix cores wait (1 195 -> 1 390 TFLOP/s at 8192 x 28 672 x 4 096);
 //   * workgroups stay and take tile after tile; the loads of the next tile are in flight behind the last steps of one;
@@ -88,6 +90,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     constexpr int kBuf = BM * kBK * 2;
     constexpr bool GATED = EPI == PE_SWIGLU || EPI == PE_GEGLU;
     constexpr int CW = NT * (GATED ? 8 : 16), CH = CW / 8;       // columns of a wavefront's output, in 16-byte pieces
+    constexpr int AR = MT > 8 ? MT / 2 : MT;                      // tiles of A in registers
     constexpr int P = MT * NT;                                   // products of half a step
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];      // 3 x [BM rows][8 chunks of 16 B], chunk ^ (row >> 1 & 7)
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, j = lane & 15, kq = lane >> 4;
@@ -123,7 +126,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
         for (int t = 0; t < NT / 2; ++t) bnext[t] = (unsigned)min((n * 4 + wave) * (NT / 2) + t, p.wtiles - 1) * (unsigned)(p.K * 64);
     };
-    bf16x8 b[2][2][NT], a[MT];
+    bf16x8 b[4][2][NT], a[AR];
     // rows tid / 8 + 32 i to LDS, without a register between.  The DMA writes lane after lane: a lane fetches the piece that belongs at
     // its place.  In assembly, since the compiler would have every LDS read wait for it; the waits are counted by hand (wait_a)
     auto load_a = [&](unsigned buf, int i) {
@@ -138,38 +141,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     unsigned raddr[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) raddr[h] = (unsigned)(j * 128 + (((4 * h + kq) ^ ((j >> 1) & 7)) * 16));
-    auto read_a = [&](unsigned buf, int h, int t) { a[t] = *reinterpret_cast<const bf16x8*>(lds + (raddr[h] + buf) + t * 2048); };
+    auto read_a = [&](unsigned buf, int h, int t) { a[t % AR] = *reinterpret_cast<const bf16x8*>(lds + (raddr[h] + buf) + t * 2048); };
     f32x4 acc[NT][MT];
-    // the products of half h of a step of parity e, each followed by what `beside` issues there: an order that the compiler keeps
+    // the products of half h of step e of four, each followed by what `beside` issues there: an order that the compiler keeps
     auto half = [&](int e, int h, auto beside) {
         unrolled(std::make_integer_sequence<int, P>(), [&](int i) __attribute__((always_inline)) {
             const int t = i / NT, n = t & 1 ? NT - 1 - i % NT : i % NT;
             // (in assembly: left to the compiler, accumulators of four registers wander, by 200 moves a step)
-            asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[n][t]) : "v"(b[e][h][n]), "v"(a[t]));
+            asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[n][t]) : "v"(b[e][h][n]), "v"(a[t % AR]));
             beside(i);
             __builtin_amdgcn_sched_barrier(0);
         });
     };
     // A of this step, of the next and of the one after it: places in LDS
     unsigned buf0 = 0, buf1 = kBuf, buf2 = 2 * kBuf;
-    // step e of a pair: its products, A of the second and third step ahead, W of the second
-    auto step = [&](auto parity, auto turn) {
-        constexpr int e = decltype(parity)::value, o = 1 - e;
+    // step e of four: its products, A of the second and third step ahead, W of the third and fourth
+    auto step = [&](auto place_of_four, auto turn) {
+        constexpr int e = decltype(place_of_four)::value, o = (e + 3) % 4;
+        constexpr int G = MT - AR + 2;                            // groups of products in front of the barrier
         half(e, 0, [&](int i) {
-            if (i % NT == NT - 1) read_a(buf0, 1, i / NT);
+            const int t = i / NT + AR;
+            if (i % NT == NT - 1) read_a(buf0, t / MT, t % MT);
             spread(i, P, AL - AH + NT, 1, [&](int x) { if (x < NT) load_b(o, 1, bbase, x); else load_a(buf2, AH + x - NT); });
         });
         turn();
         half(e, 1, [&](int i) {
+            const int t = i / NT + AR;
+            if (t < MT && i % NT == NT - 1) read_a(buf0, 1, t);
             // Behind the barrier no wavefront reads A of this step any more, and A of the next is there: of the loads in flight at most
             // those of two halves are younger.  It stands where the last LDS instruction lies a few products back
-            if (i == 2 * NT - 1) {
+            if (i == G * NT - 1) {
                 asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NT + AL) : "memory");
                 wait_lds_barrier();
             }
-            if (i == 2 * NT || i == 2 * NT + 1) read_a(buf1, 0, i - 2 * NT);
-            if (i >= 2 * NT && i % NT == NT - 1) read_a(buf1, 0, i / NT);
-            spread(i - 2 * NT, P - 2 * NT, AH + NT, 1, [&](int x) { if (x < NT) load_b(e, 0, bnext, x); else load_a(buf0, x - NT); });
+            if (i == G * NT || i == G * NT + 1) read_a(buf1, 0, i - G * NT);
+            if (i >= G * NT && i % NT == NT - 1) read_a(buf1, 0, t - MT);
+            spread(i, G * NT, NT, 1, [&](int x) { load_b(e, 0, bnext, x); });
+            spread(i - G * NT, P - G * NT, AH, 1, [&](int x) { load_a(buf0, x); });
         });
         const unsigned done = buf0;
         buf0 = buf1;
@@ -198,15 +206,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     ka += kBK * 2;
     ask([&](int i) { load_a(buf1, i); }, 0, AL);
     ask([&](int i) { load_b(0, 0, bnext, i); }, 0, NT);
-    ka += kBK * 2;
     ask([&](int i) { load_b(0, 1, bnext, i); }, 0, NT);
-    ask([&](int i) { load_a(buf2, i); }, 0, AH);
+    ka += kBK * 2;
 #pragma unroll
-    for (int t = 0; t < NT / 2; ++t) bnext[t] += 4096;
-    ask([&](int i) { load_b(1, 0, bnext, i); }, 0, NT);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AL + AH + 3 * NT) : "memory");
+    for (int e = 1; e < 4; ++e) {
+#pragma unroll
+        for (int t = 0; t < NT / 2; ++t) bnext[t] += 4096;
+        if (e == 3) ask([&](int i) { load_a(buf2, i); }, 0, AH);
+        ask([&](int i) { load_b(e, 0, bnext, i); }, 0, NT);
+        if (e < 3) ask([&](int i) { load_b(e, 1, bnext, i); }, 0, NT);
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AL + AH + 7 * NT) : "memory");
     wait_lds_barrier();
-    ask([&](int i) { read_a(buf0, 0, i); }, 0, MT);
+    ask([&](int i) { read_a(buf0, 0, i); }, 0, AR);
 
     float act_p = 0.f, act_n = 0.f;
     if constexpr (EPI == PE_XIELU) {
@@ -223,11 +235,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                 for (int r = 0; r < 4; ++r) acc[n][t][r] = 0.f;
         asm volatile("s_nop 7" ::: "memory");
         const int next = v + grid < p.total ? v + grid : first;       // (behind the last tile: rows that exist, and are not used)
-        for (int k = 0; k < steps; k += 2) {
+        for (int k = 0; k < steps; k += 4) {
+            auto turn = [&]() { ka += kBK * 2; };
             advance_b();
-            if (__builtin_expect(k == steps - 2, 0)) seek_b(next);
+            if (__builtin_expect(k == steps - 4, 0)) seek_b(next);
             __builtin_amdgcn_sched_barrier(0);
-            step(std::integral_constant<int, 0>(), [&]() { ka += kBK * 2; });
+            step(std::integral_constant<int, 0>(), turn);
             advance_b();
             __builtin_amdgcn_sched_barrier(0);
             step(std::integral_constant<int, 1>(), [&]() {
@@ -235,6 +248,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                 if (__builtin_expect(k == steps - 4, 0)) seek_a(next);
                 __builtin_amdgcn_sched_barrier(0);
             });
+            advance_b();
+            __builtin_amdgcn_sched_barrier(0);
+            step(std::integral_constant<int, 2>(), turn);
+            advance_b();
+            __builtin_amdgcn_sched_barrier(0);
+            step(std::integral_constant<int, 3>(), turn);
         }
         // (the products are assembly: what the compiler would wait between the last of them and reading its accumulator)
         asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
@@ -300,14 +319,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 }
 
 // Tiles: rows x columns, and what one takes: us before the first step of 64 and behind the last, us a step while most CUs idle, and how much
-// slower that is with all of them busy (the clock).  Drawn from 970 random products (257 to 16 384 rows, 33 weights of 768 x 768 to
+// slower that is with all of them busy (the clock).  Drawn from 435 random products (257 to 16 384 rows, 33 weights of 768 x 768 to
 // 128 256 x 2 048); the tile that this picks is within 0.5 % of the best on average, 18 % at the worst.
 struct Tile {
     int rows, cols;
     double fixed, step, busy;
 };
-constexpr Tile kTiles[] = {{256, 256, 8.9, 0.908, 1.41}, {192, 256, 7.8, 0.694, 1.41}, {128, 256, 6.0, 0.500, 1.42},
-                           {256, 128, 5.1, 0.647, 1.22}, {192, 128, 4.5, 0.534, 1.17}, {128, 128, 3.0, 0.464, 1.05}};
+constexpr Tile kTiles[] = {{256, 256, 9.5, 0.906, 1.41}, {192, 256, 8.0, 0.692, 1.41}, {128, 256, 6.4, 0.507, 1.38},
+                           {256, 128, 6.2, 0.540, 1.30}, {192, 128, 5.0, 0.434, 1.27}, {128, 128, 3.3, 0.368, 1.10}};
 
 double tile_us(const Tile& t, int M, int64_t cols, int K) {
     const int64_t total = (int64_t)((M + t.rows - 1) / t.rows) * ((cols + t.cols - 1) / t.cols), rounds = total / 256, rest = total % 256;
@@ -332,7 +351,7 @@ const Tile& best_tile(int M, int64_t cols, int K, double* us) {
 bool shape_ok(int M, int N, int K, bool gated) {
     const int nout = gated ? N / 2 : N;
     const size_t tiles = gated ? (nout + 15) / 16 : (nout + 31) / 32;
-    return M > 0 && N > 0 && (!gated || N % 2 == 0) && nout % 8 == 0 && K >= 4 * kBK && K % (2 * kBK) == 0 && K < (1 << 20) &&
+    return M > 0 && N > 0 && (!gated || N % 2 == 0) && nout % 8 == 0 && K >= 4 * kBK && K % (4 * kBK) == 0 && K < (1 << 20) &&
            nout < (1 << 20) && tiles * K * 64 < ((size_t)1 << 32);
 }
 
@@ -372,7 +391,7 @@ int launch(PromptParams& p, int rows, int cols, hipStream_t st) {
 
 }  // namespace
 
-// (its workgroups take all of K: a few hundred rows of a narrow and deep product leave most CUs idle, 374 x 2 048 x 10 240 in 75 us where
+// (its workgroups take all of K: a few hundred rows of a narrow and deep product leave most CUs idle, 374 x 2 048 x 10 240 in 58 us where
 // the library's split of K takes 41, or 61 with the weight's rows to bring back.  The line is where those cross over the same products)
 extern "C" int md_linear_prompt_supported(int M, int N, int K, int epilogue) {
     const bool gated = epilogue == PE_SWIGLU || epilogue == PE_GEGLU;
