@@ -316,10 +316,10 @@ int md_linear_block_add_rmsnorm(const void* x, int64_t ldx, const void* w_packed
  *   MD_EPI_SWIGLU  bf16(bf16(silu(bf16(h1))) * bf16(h3))
  *   2 (xIELU)      bf16(xielu(acc)): act = its two numbers, no bias
  *   MD_EPI_GEGLU   bf16(gelu_tanh(h1) * h3)
- * md_linear_prompt_supported: 1 if it takes the shape and is expected to be faster than a library GEMM (negative: no shape).  tile: 0, or 1000 * rows + columns
+ * md_linear_prompt_us: what a call is expected to take in microseconds, negative where it does not take the shape.  tile: 0, or 1000 * rows + columns
  * of a tile (256 x 256, 192 x 256, 128 x 256, 256 x 128, 192 x 128, 128 x 128) instead of the one that the shape asks for.
  * ---------------------------------------------------------------------- */
-int md_linear_prompt_supported(int M, int N, int K, int epilogue);
+double md_linear_prompt_us(int M, int N, int K, int epilogue);
 int md_linear_prompt(const void* x, int64_t ldx, const void* w_packed, const void* bias, const float* act, void* out, int64_t ldo, int M,
                      int N, int K, int epilogue, int tile, md_stream_t stream);
 

@@ -26,7 +26,7 @@ every decode / verify shape of the 8B and 1B models timed on both, weights cycle
     and NOT the narrow projections, where splitting K over ~256 workgroups costs a partial-sum round trip the product is
     too small to pay for (wqkv 30-32 vs lib 27 + 6.3 for rope/append: a wash; wo 34-35 vs 25; every TP8 shard slower).
 
-  * the rows of a PROMPT (more than 256) go to md_linear_prompt (csrc/promptgemm.hip), which reads the streaming layout too: use_prompt.
+  * the rows of a PROMPT (more than 256) go to md_linear_prompt (csrc/promptgemm.hip), which reads the streaming layout too: prompt_rows.
 
 A weight a hand-written kernel will serve is re-packed once at setup_caches (Transformer._pack_weights); the row-major
 copy stays for the products that are left to the library.  MAGICDEC_GEMM=hip forces md_linear wherever it supports the shape,
@@ -89,7 +89,7 @@ def skinny_absorbs_norm(M: int) -> bool:
 def _changed():
     """A switch or the table of tuned solutions is another one."""
     _measured.cache_clear()
-    use_prompt.cache_clear()
+    prompt_rows.cache_clear()
 
 
 def set_mode(mode: str):
@@ -467,10 +467,23 @@ def choose(M: int, N: int, K: int, swiglu: bool, int8: bool, packed: bool, kind:
 
 
 @functools.lru_cache(maxsize=4096)
-def use_prompt(M: int, N: int, K: int, swiglu: bool = False) -> bool:
-    """md_linear_prompt for this linear (weight in the streaming layout) of more rows than a step has?  Where it takes the shape, but for a
-    few hundred rows of narrow and deep products (csrc/promptgemm.hip).  Against the library, 435 random products of 257 to 16 384 rows:
-    0.77 of its time with the activation behind it, 0.61 with the weight's rows brought back in front; 1.11 at the worst (12 719 x 2 048 x
-    8 192, 341 us)."""
+def prompt_rows(M: int, N: int, K: int, swiglu: bool = False) -> int:
+    """How many of a prompt's M rows (more than a step has; weight in the streaming layout) go to md_linear_prompt in one call: none (the
+    library), all, or whole row tiles with fewer than 129 left for md_linear.
+    Against the library, 435 random products of 257 to 16 384 rows: 0.77 of its time with the activation behind it, 0.61 with the weight's
+    rows brought back in front; 1.11 at the worst (12 719 x 2 048 x 8 192, 341 us).  Its workgroups take all of K, so that a few hundred
+    rows of a narrow and deep product leave most CUs idle: 374 x 2 048 x 10 240 in 58 us where the library's split of K takes 41, or 61
+    with the rows to bring back; the line is where those cross over the same products.
+    Rows just behind whole rounds of tiles are a round more: 8 196 x 4 096 x 18 432 in 950 us, 8 192 in 760 and the other four in 40 on the
+    weight-streaming kernel, whose time the last line bounds from above (49 / 55 us for 28 672 x 4 096 at 64 / 128 rows, 16 / 21 for 4 096
+    x 4 096, 54 / 64 for 5 120 x 27 648)."""
     from .. import ops
-    return _MODE != "lib" and M > 256 and ops.linear_prompt_supported(M, N, K, swiglu)
+    us = ops.linear_prompt_us(M, N, K, swiglu) if _MODE != "lib" and M > 256 else -1.0
+    if us < 0 or us > 2.4 * (2e-6 * M * N / 1400 * K + 12):
+        return 0
+    rest = M % 256
+    if 0 < rest <= 128 and M - rest > 256 and ops.linear_supported(rest, N, K, swiglu):
+        streamed = (12 + N * K * 2 / 5.5e6) * (1.0 if rest <= 64 else 1.2)
+        if ops.linear_prompt_us(M - rest, N, K, swiglu) + streamed < 0.97 * us:
+            return M - rest
+    return M

@@ -40,7 +40,7 @@ import torch.nn as nn
 from torch.nn import functional as F
 
 from .. import ops
-from .gemm_policy import use_prompt
+from .gemm_policy import prompt_rows
 
 
 def find_multiple(n: int, k: int) -> int:
@@ -599,7 +599,7 @@ class Transformer(nn.Module):
         if how == "lib" and x2d.is_cuda and self._on_prompt_gemm(x2d, w, pk, swiglu):
             how = "prompt"
         if how == "prompt":
-            return ops.linear_prompt(x2d if pro is None else pro.materialize(), pk, bias, swiglu)
+            return self._prompt_linear(x2d if pro is None else pro.materialize(), pk, bias, swiglu)
         if how == "fused" and ops.fused_linear_supported(M, N, K):
             if pro is not None and not swiglu:
                 x2d, pro = pro.materialize(), None
@@ -633,7 +633,19 @@ class Transformer(nn.Module):
         M, K = x2d.shape
         return (M > 256 and pk is not None and w.dtype == torch.bfloat16 and x2d.dtype == torch.bfloat16 and x2d.stride(1) == 1
                 and x2d.stride(0) % 8 == 0 and x2d.stride(0) < 1 << 20 and x2d.data_ptr() % 16 == 0
-                and use_prompt(M, w.shape[0], K, swiglu))
+                and prompt_rows(M, w.shape[0], K, swiglu) > 0)
+
+    def _prompt_linear(self, x2d, pk, bias=None, swiglu=False, out=None, **act):
+        """A linear of a prompt's rows: whole row tiles on md_linear_prompt, a few rows behind them on the weight-streaming kernel."""
+        M, K = x2d.shape
+        rows = prompt_rows(M, pk.N, K, swiglu)
+        if rows == M:
+            return ops.linear_prompt(x2d, pk, bias, swiglu, out=out, **act)
+        if out is None:
+            out = torch.empty((M, pk.N // 2 if swiglu else pk.N), dtype=x2d.dtype, device=x2d.device)
+        ops.linear_prompt(x2d[:rows], pk, bias, swiglu, out=out[:rows], **act)
+        ops.linear(x2d[rows:], pk, bias, None, swiglu, self.workspace, out=out[rows:], **act)
+        return out
 
     def _linear_how(self, M, N, K, swiglu, int8, pk, kind, has_pro):
         """Which implementation `_linear` ends up on for this shape: "fused" | "block" | "skinny" | "lib" -- the same

@@ -339,7 +339,7 @@ class LayeredTransformer(Transformer):
         if how == "rows":
             return ops.linear(inp, pk, workspace=self.workspace)
         if inp.is_cuda and self._on_prompt_gemm(inp, lin.weight, pk):
-            return ops.linear_prompt(inp, pk)
+            return self._prompt_linear(inp, pk)
         self._last_M = M
         return F.linear(inp, self._resident(lin.weight))
 
@@ -355,7 +355,7 @@ class LayeredTransformer(Transformer):
         if how == "skinny":
             return ops.linear(y, pk, workspace=self.workspace, xielu=act)
         if y.is_cuda and self._on_prompt_gemm(y, lin.weight, pk):
-            return ops.linear_prompt(y, pk, xielu=act)
+            return self._prompt_linear(y, pk, xielu=act)
         self._last_M = M
         z = F.linear(y, self._resident(lin.weight))
         return ops.xielu(z, act, out=z)
@@ -375,7 +375,7 @@ class LayeredTransformer(Transformer):
         if how == "skinny":
             return ops.linear(y, pk, swiglu=True, gelu=True, workspace=self.workspace, out=out)
         if aligned and y.is_cuda and out.stride(0) < 1 << 20 and self._on_prompt_gemm(y, lin.weight, pk, True):
-            return ops.linear_prompt(y, pk, swiglu=True, gelu=True, out=out)
+            return self._prompt_linear(y, pk, swiglu=True, gelu=True, out=out)
         self._last_M = M
         z = F.linear(y, self._resident(lin.weight))
         return ops.gelu_mul(z[:, :N // 2], z[:, N // 2:], out=out)

@@ -391,15 +391,14 @@ int launch(PromptParams& p, int rows, int cols, hipStream_t st) {
 
 }  // namespace
 
-// (its workgroups take all of K: a few hundred rows of a narrow and deep product leave most CUs idle, 374 x 2 048 x 10 240 in 58 us where
-// the library's split of K takes 41, or 61 with the weight's rows to bring back.  The line is where those cross over the same products)
-extern "C" int md_linear_prompt_supported(int M, int N, int K, int epilogue) {
-    const bool gated = epilogue == PE_SWIGLU || epilogue == PE_GEGLU;
-    MD_CHECK_ARG(M > 0 && N > 0 && K > 0, "md_linear_prompt_supported: M=%d N=%d K=%d", M, N, K);
-    if (!shape_ok(M, N, K, gated)) return 0;
+extern "C" double md_linear_prompt_us(int M, int N, int K, int epilogue) {
+    if (!shape_ok(M, N, K, epilogue == PE_SWIGLU || epilogue == PE_GEGLU)) {
+        md_set_error("md_linear_prompt_us: M=%d N=%d K=%d unsupported", M, N, K);
+        return -1.0;
+    }
     double us = 0;
     best_tile(M, N, K, &us);
-    return us <= 2.4 * (2e-6 * M * N / 1400 * K + 12) ? 1 : 0;
+    return us;
 }
 
 extern "C" int md_linear_prompt(const void* x, int64_t ldx, const void* w_packed, const void* bias, const float* act, void* out, int64_t ldo,

@@ -591,10 +591,10 @@ def linear_block_add_rmsnorm(x, weight: "PackedWeight", resid, norm_weight, eps,
 PE_NONE, PE_SWIGLU, PE_XIELU, PE_GEGLU = 0, 1, 2, 3
 
 
-def linear_prompt_supported(M, N, K, swiglu=False):
-    """True when md_linear_prompt (csrc/promptgemm.hip: the GEMM of a prompt's rows) takes this shape and is expected to be
-    faster than the library."""
-    return _lib.load().md_linear_prompt_supported(int(M), int(N), int(K), PE_SWIGLU if swiglu else PE_NONE) > 0
+def linear_prompt_us(M, N, K, swiglu=False):
+    """What md_linear_prompt (csrc/promptgemm.hip: the GEMM of a prompt's rows) is expected to take for this shape, in microseconds;
+    negative: it does not take it."""
+    return _lib.load().md_linear_prompt_us(int(M), int(N), int(K), PE_SWIGLU if swiglu else PE_NONE)
 
 
 def linear_prompt(x, weight: "PackedWeight", bias=None, swiglu=False, out=None, xielu=None, gelu=False, tile=0):

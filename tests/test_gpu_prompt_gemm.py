@@ -96,3 +96,29 @@ def test_refused():
                  lambda: ops.linear_prompt(x, pw, out=torch.empty(300, 68, device=DEV, dtype=torch.bfloat16)[:, 2:66])):       # alignment
         with pytest.raises((RuntimeError, ValueError)):
             call()
+
+
+@pytest.mark.parametrize("M,N,K,swiglu", [(4112, 4096, 5120, False), (8193, 2048, 2560, False), (4224, 4096, 9216, False), (10241, 16384, 2048, True)])
+def test_rows_behind_whole_tiles(M, N, K, swiglu):
+    """A linear of a prompt whose last rows run on the weight-streaming kernel: every row against float64, in a view of a wider matrix."""
+    from types import SimpleNamespace
+    from magicdec_amd import ops
+    from magicdec_amd.Engine.gemm_policy import prompt_rows
+    from magicdec_amd.Engine.model_core import Transformer
+    assert 0 < prompt_rows(M, N, K, swiglu) < M
+    x, w, bias = case(M, N, K, M)
+    pk, n_out = ops.PackedWeight(w, swiglu=swiglu), N // 2 if swiglu else N
+    model = SimpleNamespace(workspace=ops.AttnWorkspace(DEV))
+    wide = torch.full((M, n_out + 8), -7.0, device=DEV, dtype=torch.bfloat16)
+    out = Transformer._prompt_linear(model, x, pk, None if swiglu else bias, swiglu, out=wide[:, :n_out])
+    assert (wide[:, n_out:] == -7).all() and out.data_ptr() == wide.data_ptr()
+    ref, off = product(x, w)
+    if not swiglu:
+        want = ref + bias.double()
+        assert ((out.double() - want).abs() <= want.abs() * U + 2 * off + 2.0 ** -23 * bias.double().abs()).all()
+        return
+    h1, h3 = ref[:, :n_out], ref[:, n_out:]
+    s = torch.sigmoid(h1)
+    bound = ((s * (1 + h1 * (1 - s))).abs() * (h1.abs() * U + 2 * off[:, :n_out]) * h3.abs() + (h1 * s).abs() * 2 * off[:, n_out:]
+             + 3 * U * (h1 * s * h3).abs()) * 1.02 + 1e-30
+    assert ((out.double() - h1 * s * h3).abs() <= bound).all()
