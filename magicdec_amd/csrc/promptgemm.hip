@@ -59,12 +59,12 @@ __device__ __forceinline__ float sigmoid_fast(float z) {
 
 // gelu_tanh on the transcendental unit
 __device__ __forceinline__ float gelu_fast(float z) { return z * sigmoid_fast(1.5957691216057308f * fmaf(0.044715f * z * z, z, z)); }
-// Xielu on it: e^z - 1 - z by its series near 0, where the difference would cancel
+// Xielu on it, without branches (a NaN goes through z / 2).  e^n - 1 - n is its series where the difference would cancel: |n| < 2^-8, where
+// the next term is 1e-8.  16 384 x 14 336 x 4 096: 1 433 us with a branch per value, 1 316 so
 __device__ __forceinline__ float xielu_fast(float ap, float an, float z) {
-    const float n = fminf(z, 0.f), n2 = n * n;
-    const float series = n2 * fmaf(n, fmaf(n, 1.0f / 24.0f, 1.0f / 6.0f), 0.5f);
-    const float e = n > -0.06f ? series : __builtin_amdgcn_exp2f(n * 1.4426950408889634f) - 1.0f - n;
-    return (z > 0.f ? ap * z * z : an * e) + 0.5f * z;
+    const float n = fminf(z, 0.f), p = fmaxf(z, 0.f);
+    const float far = __builtin_amdgcn_exp2f(n * 1.4426950408889634f) - 1.0f - n, near = 0.5f * n * n;
+    return fmaf(ap * p, p, fmaf(an, n > -0.00390625f ? near : far, 0.5f * z));
 }
 // f(0), f(1), ...: what a loop of this length is not always unrolled to
 template <int... I, class F>

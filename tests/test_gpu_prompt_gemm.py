@@ -75,9 +75,10 @@ def test_not_finite():
     from magicdec_amd import ops
     x, w, _ = case(300, 64, 256, 3)
     x[7, 5], x[200, 100] = float("inf"), float("nan")
-    out = ops.linear_prompt(x, ops.PackedWeight(w))
-    bad = ~torch.isfinite(out).all(1)
-    assert bad[7] and bad[200] and bad.sum() == 2
+    for kw in ({}, dict(xielu=torch.tensor([0.3, -0.2], device=DEV)), dict(swiglu=True), dict(swiglu=True, gelu=True)):
+        out = ops.linear_prompt(x, ops.PackedWeight(w, swiglu="swiglu" in kw), **kw)
+        bad = ~torch.isfinite(out).all(1)
+        assert bad[7] and bad[200] and bad.sum() == 2 and out[200].isnan().all()
     big = torch.full((300, 256), 1.0, device=DEV).bfloat16()
     w = torch.cat([torch.full((8, 256), -1.0), torch.full((8, 256), 1.0), torch.full((16, 256), 0.5)]).to(DEV).bfloat16()     # h1 = -256, 256
     for gelu in (False, True):
