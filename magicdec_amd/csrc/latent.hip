@@ -209,6 +209,50 @@ __global__ __launch_bounds__(256) void head_linear_mfma_kernel(const HeadLinearP
 }
 
 // 32-bit: a thread per output
+// 32-bit on the fp32 matrix instructions, laid out as above: a lane reads four k of a row at once, product e takes the e-th of each.  Dense
+// 16-byte pieces only; the kernel below has a thread per value, which waits for every k (2 400 rows, 16 heads, 128 -> 512: 4 470 us, here 126; 8 rows: 50 and 5.8).
+template <int RT>
+__global__ __launch_bounds__(256) void head_linear_f32_mfma_kernel(const HeadLinearParams p) {
+    const int lane = threadIdx.x & 63, lq = lane & 15, lc = lane >> 4, wave = threadIdx.x >> 6;
+    const int h = blockIdx.z, row0 = blockIdx.y * 16 * RT, n0 = blockIdx.x * 64 + wave * 16;
+    if (p.tail) head_tail<float>(p, h, row0, 16 * RT);
+    if (n0 >= p.N) return;
+    const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
+    const int n = n0 + lq;
+    const float* wp = reinterpret_cast<const float*>(p.w) + ((int64_t)h * p.N + min(n, p.N - 1)) * p.K;
+    const float* xp[RT];
+    f32x4 acc[RT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+        xp[r] = reinterpret_cast<const float*>(p.x) + (int64_t)min(row0 + r * 16 + lq, p.M - 1) * p.ldx + h * p.hx;
+        acc[r] = z4;
+    }
+    for (int kb = 0; kb < p.K; kb += 64) {                          // four portions of 16 k requested together (zeros past K)
+        f32x4 wf[4], xf[4][RT];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int k = kb + u * 16 + lc * 4;
+            wf[u] = k < p.K ? *reinterpret_cast<const f32x4*>(wp + k) : z4;
+#pragma unroll
+            for (int r = 0; r < RT; ++r) xf[u][r] = k < p.K ? *reinterpret_cast<const f32x4*>(xp[r] + k) : z4;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int r = 0; r < RT; ++r) acc[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[u][e], xf[u][r][e], acc[r], 0, 0, 0);
+    }
+    // acc[r][e] = y[row0 + r * 16 + lq][n0 + lc * 4 + e]
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+        const int row = row0 + r * 16 + lq, c = n0 + lc * 4;
+        if (row >= p.M || c >= p.N) continue;
+        const float s = p.gate ? sigmoid(reinterpret_cast<const float*>(p.gate)[row * p.ld_gate + h]) : 1.f;
+        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.out) + row * p.ldo + h * p.ho + c) = acc[r] * s;
+    }
+}
+
 __global__ __launch_bounds__(256) void head_linear_f32_kernel(const HeadLinearParams p) {
     const int h = blockIdx.z, row0 = blockIdx.y * 16, n = blockIdx.x * 16 + (threadIdx.x & 15), row = row0 + (threadIdx.x >> 4);
     if (n < p.N && row < p.M) {
@@ -424,6 +468,12 @@ extern "C" int md_latent_append(const md_latent_args* a, md_stream_t stream) {
     return MD_OK;
 }
 
+// 16-row tiles of a head_linear wavefront: as many as leave every CU a workgroup
+static int row_tiles(const md_head_linear_args* a) {
+    const long columns = (long)((a->N + 63) / 64) * a->H;
+    return columns * ((a->M + 63) / 64) >= 256 ? 4 : columns * ((a->M + 31) / 32) >= 256 ? 2 : 1;
+}
+
 extern "C" int md_head_linear(const md_head_linear_args* a, md_stream_t stream) {
     MD_CHECK_ARG(a && a->x && a->w && a->out, "md_head_linear: null pointer argument");
     MD_CHECK_ARG(a->M > 0 && a->H > 0 && a->H <= 65535 && a->N > 0 && a->K > 0, "md_head_linear: bad shape M=%d H=%d N=%d K=%d", a->M,
@@ -460,15 +510,24 @@ extern "C" int md_head_linear(const md_head_linear_args* a, md_stream_t stream) 
     hipStream_t st = (hipStream_t)stream;
     if (a->dtype == MD_T_F32) {
         MD_CHECK_ARG((a->M + 15) / 16 <= 65535, "md_head_linear: %d rows", a->M);
+        if (a->K % 4 == 0 && a->N % 4 == 0 && a->ldx % 4 == 0 && a->hx % 4 == 0 && a->ldo % 4 == 0 && a->ho % 4 == 0 && aligned(a->x, 16) &&
+            aligned(a->w, 16) && aligned(a->out, 16)) {
+            const int rt = row_tiles(a);
+            const dim3 grid((a->N + 63) / 64, (a->M + 16 * rt - 1) / (16 * rt), a->H);
+            if (rt == 4) hipLaunchKernelGGL(head_linear_f32_mfma_kernel<4>, grid, dim3(256), 0, st, p);
+            else if (rt == 2) hipLaunchKernelGGL(head_linear_f32_mfma_kernel<2>, grid, dim3(256), 0, st, p);
+            else hipLaunchKernelGGL(head_linear_f32_mfma_kernel<1>, grid, dim3(256), 0, st, p);
+            MD_CHECK_LAUNCH("md_head_linear");
+            return MD_OK;
+        }
         hipLaunchKernelGGL(head_linear_f32_kernel, dim3((a->N + 15) / 16, (a->M + 15) / 16, a->H), dim3(256), 0, st, p);
         MD_CHECK_LAUNCH("md_head_linear");
         return MD_OK;
     }
     const bool vec = a->K % 8 == 0 && a->ldx % 8 == 0 && a->hx % 8 == 0 && a->ldo % 4 == 0 && a->ho % 4 == 0 && aligned(a->x, 16) &&
                      aligned(a->w, 16) && aligned(a->out, 8);
-    const int nb = (a->N + 63) / 64;
-    const int rt = (long)nb * a->H * ((a->M + 63) / 64) >= 256 ? 4 : (long)nb * a->H * ((a->M + 31) / 32) >= 256 ? 2 : 1;
-    const dim3 grid(nb, (a->M + 16 * rt - 1) / (16 * rt), a->H);
+    const int rt = row_tiles(a);
+    const dim3 grid((a->N + 63) / 64, (a->M + 16 * rt - 1) / (16 * rt), a->H);
     MD_CHECK_ARG(grid.y <= 65535, "md_head_linear: %d rows", a->M);
 #define MD_HL(RT)                                                                                               \
     do {                                                                                                        \
