@@ -323,6 +323,12 @@ double md_linear_prompt_us(int M, int N, int K, int epilogue);
 int md_linear_prompt(const void* x, int64_t ldx, const void* w_packed, const void* bias, const float* act, void* out, int64_t ldo, int M,
                      int N, int K, int epilogue, int tile, md_stream_t stream);
 
+/* md_linear_f32 (csrc/f32gemm.hip): the same of float32 rows and a row-major float32 weight, out[M][N] = x[M][K] . w[N][K]^T on the fp32
+ * matrix instructions; K % 32 == 0, N % 4 == 0, everything 16-byte aligned.  _supported: 1 if it takes the shape and is expected to be
+ * faster than a library GEMM (negative: no shape).  tile: 0, or 1000 * rows + columns (64 x 128, 64 x 64, 32 x 64). */
+int md_linear_f32_supported(int M, int N, int K);
+int md_linear_f32(const float* x, int64_t ldx, const float* w, float* out, int64_t ldo, int M, int N, int K, int tile, md_stream_t stream);
+
 /* ------------------------------------------------------------------------
  * K8b  fused small-problem linear: a linear of a decode / verify step TOGETHER with the op that consumes its output,
  *      one launch (csrc/tilegemm.hip; no split-K across workgroups, no workspace, deterministic)

@@ -15,7 +15,8 @@ computes:
 * the last unshifted rows of every sequence live in a small float32 ring per layer, indexed by position (ops.resid_norm), so a
   step may be repeated (graph capture) or rolled back (rejected draft tokens) without saving state.
 
-With float32 weights every kernel runs in 32-bit (plain attention kernel, library GEMMs without reduced-precision modes).
+With float32 weights every kernel runs in 32-bit (attention and products on the fp32 matrix instructions, library GEMMs without
+reduced-precision modes for few rows).
 """
 from __future__ import annotations
 
@@ -27,7 +28,7 @@ from torch.nn import functional as F
 
 from .. import ops
 from .designs import DecoderSpec, LatentAttentionSpec, LayerSpec
-from .gemm_policy import choose, use_split
+from .gemm_policy import choose, mode, use_split
 from .model_core import PageTable, RMSNorm, Transformer
 
 STATE_RING = 16        # unshifted rows kept per sequence and layer: rollbacks of up to STATE_RING - 2 tokens
@@ -316,8 +317,19 @@ class LayeredTransformer(Transformer):
     # ------------------------------------------------------------------ the step
     def _linear(self, x2d, lin, **kw):
         if x2d.dtype == torch.float32:
-            return F.linear(x2d, lin.weight)
+            return self._library(x2d, lin.weight)
         return super()._linear(x2d, lin, **kw)
+
+    def _library(self, x2d, w):
+        """The product of a row-major weight: a prompt's float32 rows on md_linear_f32, others in the library."""
+        if x2d.dtype == torch.float32:
+            M = x2d.shape[0]
+            if (M >= 1200 and x2d.is_cuda and ops.linear_f32_supported(M, *w.shape) and x2d.stride(0) % 4 == 0 and x2d.data_ptr() % 16 == 0
+                    and w.data_ptr() % 16 == 0 and mode() != "lib"):
+                return ops.linear_f32(x2d, w)
+            return F.linear(x2d, w)
+        self._last_M = x2d.shape[0]
+        return F.linear(x2d, self._resident(w))
 
     def _project_how(self, M, N, K, packed):
         """Where an output projection runs: a split-K GEMM up to its float32 planes ("skinny" | "tile" | "block"; the residual
@@ -340,8 +352,7 @@ class LayeredTransformer(Transformer):
             return ops.linear(inp, pk, workspace=self.workspace)
         if inp.is_cuda and self._on_prompt_gemm(inp, lin.weight, pk):
             return self._prompt_linear(inp, pk)
-        self._last_M = M
-        return F.linear(inp, self._resident(lin.weight))
+        return self._library(inp, lin.weight)
 
     def _up_act(self, y, lin, act):
         """act(up . y): the activation is the GEMM's epilogue wherever a hand-written kernel runs it."""
@@ -356,8 +367,7 @@ class LayeredTransformer(Transformer):
             return ops.linear(y, pk, workspace=self.workspace, xielu=act)
         if y.is_cuda and self._on_prompt_gemm(y, lin.weight, pk):
             return self._prompt_linear(y, pk, xielu=act)
-        self._last_M = M
-        z = F.linear(y, self._resident(lin.weight))
+        z = self._library(y, lin.weight)
         return ops.xielu(z, act, out=z)
 
     def _gated(self, y, lin, out):
@@ -376,8 +386,7 @@ class LayeredTransformer(Transformer):
             return ops.linear(y, pk, swiglu=True, gelu=True, workspace=self.workspace, out=out)
         if aligned and y.is_cuda and out.stride(0) < 1 << 20 and self._on_prompt_gemm(y, lin.weight, pk, True):
             return self._prompt_linear(y, pk, swiglu=True, gelu=True, out=out)
-        self._last_M = M
-        z = F.linear(y, self._resident(lin.weight))
+        z = self._library(y, lin.weight)
         return ops.gelu_mul(z[:, :N // 2], z[:, N // 2:], out=out)
 
     def _parallel(self, i, layer, y, rows, tab: PageTable, ctx):

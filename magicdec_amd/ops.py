@@ -13,6 +13,7 @@ hand-written gfx950 kernels.  Differences from the reference's op boundary:
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 
 import torch
@@ -617,6 +618,25 @@ def linear_prompt(x, weight: "PackedWeight", bias=None, swiglu=False, out=None, 
     epi = PE_XIELU if xielu is not None else PE_NONE if not swiglu else PE_GEGLU if gelu else PE_SWIGLU
     check(_lib.load().md_linear_prompt(_p(x), x.stride(0), _p(weight.data), _p(bias), _act_numbers(xielu) if xielu is not None else None,
                                        _p(out), out.stride(0), M, N, K, epi, int(tile), _stream()), "md_linear_prompt")
+    return out
+
+
+@functools.lru_cache(maxsize=4096)
+def linear_f32_supported(M, N, K):
+    """True when md_linear_f32 (csrc/f32gemm.hip) takes this shape and is expected to be faster than the library."""
+    return _lib.load().md_linear_f32_supported(int(M), int(N), int(K)) > 0
+
+
+def linear_f32(x, weight, tile=0):
+    """F.linear(x, weight) of float32 rows [M, K] (row stride free) and a contiguous float32 weight [N, K] on md_linear_f32."""
+    _gpu(x, weight)
+    if x.dim() != 2 or x.stride(1) != 1 or weight.dim() != 2 or not weight.is_contiguous() or x.shape[1] != weight.shape[1]:
+        raise ValueError("linear_f32 expects x [M, K] with unit inner stride and a contiguous weight [N, K]")
+    if x.dtype != torch.float32 or weight.dtype != torch.float32:
+        raise TypeError("linear_f32 takes float32")
+    (M, K), N = x.shape, weight.shape[0]
+    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    check(_lib.load().md_linear_f32(_p(x), x.stride(0), _p(weight), _p(out), N, M, N, K, int(tile), _stream()), "md_linear_f32")
     return out
 
 
