@@ -22,6 +22,7 @@ import contextlib
 
 import torch
 
+from .. import ops
 from .model_core import PageTable
 
 PAGE_SIZE = 128    # Engine/SnapKV/backend.py:31
@@ -473,13 +474,13 @@ class SnapKVTargetBackend(_BackendBase):
         for v in n:
             qo.append(qo[-1] + v)
         # one upload for all the integers of the step
-        flat = torch.tensor(pos + slots + pages + indptr + last + qo, dtype=torch.int32).to(dev)
+        flat = ops.upload(pos + slots + pages + indptr + last + qo, torch.int32, dev)
         cut = torch.split(flat, [B, B, len(pages), B + 1, B, B + 1])
         tab = PageTable(cut[2], cut[3], cut[4], max(indptr[i + 1] - indptr[i] for i in range(B)), slots=cut[1],
                         lengths=(n, [p + k for p, k in zip(pos, n)]))
-        ids = torch.cat([t for _, t in parts]).to(dev)
+        ids = ops.upload(torch.cat([t for _, t in parts]), torch.long, dev)
         self.model.skip_head = not head_rows
-        rows = torch.tensor(head_rows, dtype=torch.long).to(dev) if head_rows else None
+        rows = ops.upload(head_rows, torch.long, dev) if head_rows else None
         tokens = self.model.forward(ids, cut[0], cut[5], tab, n_max=max(n), head_rows=rows)
         self.model.skip_head = False
         return (tokens, self.model._last_logits) if head_rows else (None, None)

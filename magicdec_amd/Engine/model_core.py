@@ -912,7 +912,7 @@ class Transformer(nn.Module):
             indptr.append(len(indices))
         # one upload for all the integers of the pass
         cut = [qo, [valid[c] - new[c] for _, c in each], indices, indptr, [(valid[c] - 1) % page + 1 for _, c in each]]
-        flat = torch.tensor([v for part in cut for v in part], dtype=torch.int32).to(dev)
+        flat = ops.upload([v for part in cut for v in part], torch.int32, dev)
         qo, off, indices, indptr, last = torch.split(flat, [len(part) for part in cut])
         tab = PageTable(indices, indptr, last, max(pages))
         windows = torch.empty((len(each) * ppr, *cache0.shape[1:]), dtype=cache0.dtype, device=dev)

@@ -1206,6 +1206,16 @@ def latent_attention(q, s: LatentSpec, cache, rows: StepRows, page_indices, page
     return out
 
 
+def upload(values, dtype, device):
+    """Host numbers (a list, or a CPU tensor of `dtype`) on the device, in the order of the current stream.  Through pinned memory: a copy from
+    pageable memory waits until the stream is done, and a program that brings a step's integers along with every step never gets ahead of
+    the GPU (a trace of a prompt and eight steps in 32-bit: 13.7 -> 11.0 ms).  The allocator keeps the pinned block until the copy is over."""
+    host = values if isinstance(values, torch.Tensor) else torch.tensor(values, dtype=dtype)
+    if torch.device(device).type != "cuda":
+        return host.to(device)
+    return host.pin_memory().to(device, non_blocking=True)
+
+
 class LatentContext:
     """What the host knows of a step's requests: `new` rows each, at the end of `ctx` positions."""
     MAX_EXPANDED_BYTES = 24 << 30
@@ -1220,7 +1230,7 @@ class LatentContext:
             at = [0]
             for c in self.ctx:
                 at.append(at[-1] + c)
-            self._indptr = torch.tensor(at, dtype=torch.int32).to(self._device)
+            self._indptr = upload(at, torch.int32, self._device)
         return self._indptr
 
     def expanded(self, s: LatentSpec):
