@@ -170,7 +170,7 @@ __device__ __forceinline__ int64_t kv_elem_offset(const KvTable& t, int b, int r
     return hnd ? base + ((int64_t)h * page_size + slot) * D + d : base + ((int64_t)slot * KH + h) * D + d;
 }
 
-// NW = wavefronts per workgroup = K slices (8, or 16 when the grid cannot give every CU two workgroups: the bytes a CU
+// NW = wavefronts per workgroup = K slices (8, or 16 when no CU gets a second workgroup: the bytes a CU
 // has in flight -- NW x (8 KiB of W + 8 KiB of x) -- are what its ingest rate is made of, ~50 GB/s per CU at NW = 8);
 // WNT = stream W with non-temporal loads (one M tile: every weight byte is read once) or keep it in L2 for the sibling
 // M tiles of the same weight tile.
@@ -614,11 +614,13 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
         if (PRO && p.pro_tiles > 128) t22 = false;       // the 2 x 2 prologue keeps <= 8 partial sums per thread in flight
         if (t22) return launch_tile_cfg<EPI, FP8, 8, false, PRO, 2, 2>(p, st);
     }
-    // 16 wavefronts (K/16 slices) when the grid is too small to put two 8-wave workgroups on every CU
-    // (not below K = 1024 -- two k-steps per wavefront and a 16-way reduce cost more than they hide: the K = 512 wo
-    // shards run 4.1-4.2 us with 8 slices against 5.3-5.4 with 16, tools/shard_bench.py / profiles/r06_shard_ab.txt)
+    // 16 wavefronts (K/16 slices) where every CU has one workgroup at most: their activation images take 136 of the 160 KB, so a second
+    // workgroup would wait for the first.  Two 8-wave workgroups share a CU: 32 rows of 11264 x 2048 (352 workgroups) 15.2 us with 16
+    // wavefronts, 13.3 with 8; 8192 x 2048 (256) 8.6 and 8.9; 64 rows of 6144 x 2048 (384) 12.2 and 11.0; one row of 9216 x 3072 16.0 and 13.6
+    // (not below K = 1024 -- two k-steps per wavefront and a 16-way reduce cost more than they hide: K = 512 shards run 4.1-4.2 us with
+    // 8 slices against 5.3-5.4 with 16)
     const int wgs = p.n_tiles * p.m_tiles;
-    bool nw16 = p.K % 256 == 0 && p.K >= 1024 && wgs <= 384;
+    bool nw16 = p.K % 256 == 0 && p.K >= 1024 && wgs <= 256;
     if (g_force_nw == 8) nw16 = false;
     if (g_force_nw == 16) nw16 = p.K % 256 == 0;
     const bool wnt = p.m_tiles == 1;

@@ -291,3 +291,15 @@ def test_fused_2x2_tiles_bit_identical_to_1x1(ops, M, N, K):
         assert torch.equal(a.view(torch.int32 if a.dtype == torch.float32 else torch.int16),
                            c.view(torch.int32 if c.dtype == torch.float32 else torch.int16)), what
     assert not torch.isnan(outs[22][4].float()).any()
+
+
+@pytest.mark.parametrize("M,N", [(1, 8192), (16, 8224), (32, 8224), (17, 12320), (33, 4128)])
+def test_one_workgroup_a_cu_or_two(ops, M, N):
+    """Either side of the line between 16-wave and 8-wave workgroups (256 of them), against the exact product."""
+    K = 1024
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K, generator=g).to(BF)
+    w = (torch.randn(N, K, generator=g) * 0.05).to(BF)
+    ref, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    y = ops.fused_linear(d(x), ops.PackedWeight(d(w)))
+    assert bool(((y.cpu().double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2 * K * 2.0 ** -24 * mag).all())
