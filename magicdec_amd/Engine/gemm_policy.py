@@ -147,6 +147,11 @@ def want_packed(N: int, K: int, swiglu: bool = False, int8: bool = False, rows=N
     return False
 
 
+def want_packed_prompt(N: int, K: int) -> bool:
+    """Re-pack a weight that only the rows of prompts are multiplied by?"""
+    return _MODE != "lib" and _PACKED != "0" and K % 64 == 0 and prompt_rows(8192, N, K) > 0
+
+
 # Shapes the library holds a tuned solution for (tuned/gemm_gfx950.csv, "tn_N_M_K_...": lines that name one; "Default" says that the
 # tuning found none better than the library's own choice).  Some rules below leave these alone: 8B wqkv (6144 x 4096) at 256 rows 32.1 us
 # with it, 37.5 on the block kernel; 4096 x 3584 + residual at 128 rows 19.8 against 21.6.

@@ -20,6 +20,7 @@ reduced-precision modes for few rows).
 """
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -28,7 +29,7 @@ from torch.nn import functional as F
 
 from .. import ops
 from .designs import DecoderSpec, LatentAttentionSpec, LayerSpec
-from .gemm_policy import choose, mode, use_split
+from .gemm_policy import choose, mode, use_split, want_packed_prompt
 from .model_core import PageTable, RMSNorm, Transformer
 
 STATE_RING = 16        # unshifted rows kept per sequence and layer: rollbacks of up to STATE_RING - 2 tokens
@@ -292,6 +293,7 @@ class LayeredTransformer(Transformer):
             if isinstance(b, ParallelLayer):
                 yield b.attention.win.weight, False, "win", i
                 yield b.attention.wuq.weight, False, "wuq", i
+                yield b.attention.wukv.weight, False, "wukv", i
                 if b.w13 is not None:
                     yield b.w13.weight, True, "gated", i
                 yield b.wout.weight, False, "wout", i
@@ -310,9 +312,15 @@ class LayeredTransformer(Transformer):
             return {self._linear_how(M, N, K, True, int8, True if packed else None, "swiglu", False)}
         return {self._linear_how(M, N, K, False, int8, True if packed else None, "plain", False)}
 
+    def _wants_packed(self, role, w):
+        # (wukv expands a prompt's latent rows; a step reads it as the heads' matrices of the absorbed form)
+        if role == "wukv":
+            return want_packed_prompt(*w.shape)
+        return super()._wants_packed(role, w)
+
     def _rowmajor_in_decode(self, w):
-        # (a tied head is the embedding table: its rows are gathered in every step)
-        return (self.spec.tied_head and w is self.output.weight) or super()._rowmajor_in_decode(w)
+        # (a tied head is the embedding table: its rows are gathered in every step; the heads' matrices are views of wukv)
+        return ((self.spec.tied_head and w is self.output.weight) or self._roles[id(w)][0] == "wukv" or super()._rowmajor_in_decode(w))
 
     # ------------------------------------------------------------------ the step
     def _linear(self, x2d, lin, **kw):
@@ -396,6 +404,8 @@ class LayeredTransformer(Transformer):
         z = self._linear(y, att.win)
         cq = ops.latent_append(z, s, cache, rows, tab.indices, tab.indptr, tab.max_pages)
         q = self._linear(cq, att.wuq)
+        if ctx is not None:
+            ctx.expand = functools.partial(self._linear, lin=att.wukv)
         side = torch.empty((y.shape[0], layer.wout.weight.shape[1]), dtype=y.dtype, device=y.device)
         heads = side[:, :layer.heads_out].unflatten(1, (s.H, s.vdim))
         ops.latent_attention(q, s, cache, rows, tab.indices, tab.indptr, tab.max_pages, self.workspace, heads,

@@ -1185,7 +1185,7 @@ def latent_attention(q, s: LatentSpec, cache, rows: StepRows, page_indices, page
         dense = torch.empty((ctx.total, s.kv_rank), dtype=q.dtype, device=q.device)
         a.ctx_indptr = ctx.indptr.data_ptr()
         check(lib.md_latent_gather(ctypes.byref(a), ctx.longest, _p(dense), _stream()), "md_latent_gather")
-        kv = torch.nn.functional.linear(dense, s.expand)
+        kv = ctx.expand(dense) if ctx.expand is not None else torch.nn.functional.linear(dense, s.expand)
         a.q, a.kv, a.out, a.ldo = q.data_ptr(), kv.data_ptr(), out.data_ptr(), out.stride(0)
         if gate is not None:
             a.gate, a.ld_gate = gate.data_ptr(), gate.stride(0)
@@ -1217,12 +1217,13 @@ def upload(values, dtype, device):
 
 
 class LatentContext:
-    """What the host knows of a step's requests: `new` rows each, at the end of `ctx` positions."""
+    """What the host knows of a step's requests: `new` rows each, at the end of `ctx` positions.  expand: dense latent rows -> the layer's
+    keys and values (rows . LatentSpec.expand^T), None: the library."""
     MAX_EXPANDED_BYTES = 24 << 30
 
     def __init__(self, new, ctx, device):
         self.new, self.ctx, self.total, self.longest = list(new), list(ctx), sum(ctx), max(ctx)
-        self._device, self._indptr, self._choice = device, None, {}
+        self._device, self._indptr, self._choice, self.expand = device, None, {}, None
 
     @property
     def indptr(self):

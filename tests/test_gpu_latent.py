@@ -359,6 +359,18 @@ def test_the_wide_model_takes_the_expanded_form(models, monkeypatch):
     assert taken == [False, False, False]
 
 
+@pytest.mark.parametrize("n", [70, 257, 300])
+def test_a_prompts_latent_rows_are_expanded_by_the_models_own_products(models, n):
+    """Rows of a step and of a prompt, latent ranks that the streaming layout takes (512) or not (480)."""
+    ids = lu.tokens(n, 512, 3)
+    e, own = serve(models["wide"][0], BF, slots=1), []
+    e.model._linear, linear = lambda x, lin, **kw: own.append(lin) or linear(x, lin, **kw), e.model._linear
+    assert [id(b.attention.wukv.weight) in e.model._packed for b in e.model.layers] == [False, True, True]
+    logits = feed(e, "a", ids, [n])
+    assert [sum(lin is b.attention.wukv for lin in own) for b in e.model.layers] == [1, 1, 1]
+    assert float(lu.row_errors(logits, models["wide"][1].logits(ids)).max()) < tol_of("wide", BF)
+
+
 @pytest.mark.parametrize("dtype", [F32, BF])
 @pytest.mark.parametrize("name", ["uneven", "wide"])
 def test_residual_after_every_layer(models, name, dtype):
