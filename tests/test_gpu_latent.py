@@ -261,6 +261,17 @@ def test_long_context_is_split_over_workgroups(ops):  # noqa: F811
             assert float((got.double() - refs[0][0][at:at + 1]).abs().max()) < 3e-2 * float(refs[0][0].abs().max()), at
 
 
+@pytest.mark.parametrize("D,VD", [(64, 64), (128, 128), (192, 256)])
+def test_prompts_of_more_than_64_pages(ops, D, VD):  # noqa: F811
+    """The expanded form keeps the numbers of 64 pages at a time; rows that fill no group of 256 are a prompt's first ones."""
+    n = 64 * 64 + 70
+    spec, zs, qs, _, refs, _ = attention_case(ops, 2, D, 32, VD, 32, 64, 17, BF, [n])
+    s = Seqs(ops, spec, BF, [n], page=64, seed=6)
+    for at, k in ((0, 4000), (4000, 65), (4065, n - 4065)):
+        got, _ = s.attend(zs[0][at:at + k], qs[0][at:at + k], [0], [at], [k], form="expanded")
+        assert float((got.double() - refs[0][0][at:at + k]).abs().max()) < 3e-2 * max(1.0, float(refs[0][0].abs().max())), at
+
+
 def test_scores_of_any_size(ops):  # noqa: F811
     """Large, tiny and negated scores: the running maximum moves by hundreds, or not at all."""
     for score in (0.01, 90.0, 400.0, -20.0):
