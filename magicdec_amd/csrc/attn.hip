@@ -33,6 +33,7 @@
 #include <type_traits>
 
 #include "attn_common.h"
+#include <algorithm>
 
 #include <hip/hip_ext.h>
 
@@ -654,7 +655,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(const AttnPara
     const int bid = blockIdx.x;
     const int xcd = bid & 7;
     const int r0 = bid >> 3;
-    const int qg = r0 % p.n_qgroups;
+    const int qg = p.n_qgroups - 1 - r0 % p.n_qgroups;     // a pair's longest groups (last rows) first: the last to start is the last to end
     const int pair = (r0 / p.n_qgroups) * 8 + xcd;
     if (pair >= p.B * p.KH) return;
     const int b = pair / p.KH, kvh = pair % p.KH;
@@ -932,7 +933,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(const AttnPara
 // TFLOP/s), the causal mask as a compile-time property of the tile body (two bodies: 480 -- the register file again), the
 // MFMAs of one accumulator issued back to back instead of alternating accumulators (795 vs 817).
 template <int D, int NW, int KT, bool VP = true>
-__global__ __launch_bounds__(64 * NW, 2) void prefill32_attn_kernel(const AttnParams p) {
+__global__ __launch_bounds__(64 * NW, D == 64 && KT == 64 ? 4 : 2) void prefill32_attn_kernel(const AttnParams p) {
     constexpr int KG = KT / 32;            // 32-key blocks per tile
     constexpr int CH = D * 2 / 16;
     constexpr int RPI = 64 / CH;
@@ -956,7 +957,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill32_attn_kernel(const AttnPa
     const int bid = blockIdx.x;
     const int xcd = bid & 7;
     const int r0 = bid >> 3;
-    const int qg = r0 % p.n_qgroups;
+    const int qg = p.n_qgroups - 1 - r0 % p.n_qgroups;     // a pair's longest groups (last rows) first: the last to start is the last to end
     const int pair = (r0 / p.n_qgroups) * 8 + xcd;
     if (pair >= p.B * p.KH) return;
     const int b = pair / p.KH, kvh = pair % p.KH;
@@ -967,8 +968,10 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill32_attn_kernel(const AttnPa
     const int npages = p.page_indptr[b + 1] - pg0;
     const int kv_len = npages > 0 ? min((npages - 1) * p.page_size + p.last_page_len[b], npages * p.page_size) : 0;
     const int nrows = n_b * g;
-    const int R = (qg * NW + wave) * 32 + j;           // this lane's query row (both kh halves hold the same query)
-    const bool valid = R < nrows;
+    // this lane's query row (both kh halves hold the same query).  Groups end with the last row: rows that fill none are the first
+    // ones, with the fewest keys
+    const int R0 = qg * NW * 32 - (NW * 32 - 1 - (nrows - 1) % (NW * 32)) / g * g, R = R0 + wave * 32 + j;
+    const bool valid = R >= 0 && R < nrows;
     const int qi = R / g, qr = R - qi * g;
     const int lim = valid ? (p.causal ? kv_len - n_b + qi : kv_len - 1) : -1;
     int hi = lim, lo = valid ? lim : 0x7fffffff;
@@ -1016,11 +1019,20 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill32_attn_kernel(const AttnPa
     }
     const unsigned goff = (unsigned)((wrow * p.slot_stride + kvh * p.head_stride) * 2 + wch * 16);
     u32x4 kreg[NLW], vreg[NLW];
+    // numbers of 64 pages, one a lane: no load in front of a tile's.  33 rows of 4 heads behind 2048 keys (64 workgroups) 77 -> 70 us; with
+    // the order of the groups, the odd rows first and whole output rows: 4 x 2048 rows, 32 heads of 128 on 8 kv heads 236 -> 199, 16
+    // portions of 512 rows, heads of 64 behind a window 42 -> 38
+    int pages = npages > 0 ? p.page_indices[pg0 + min(lane, npages - 1)] : 0;
+    asm volatile("" : "+v"(pages));
     auto issue = [&](int tt) {
         const int pos0 = tt * KT;
         const int page = pos0 / p.page_size;
         const int slot0 = pos0 - page * p.page_size;
-        const int pid = __builtin_amdgcn_readfirstlane(p.page_indices[pg0 + page]);
+        if (page % 64 == 0 && page > 0 && slot0 == 0) {
+            pages = p.page_indices[pg0 + min(page + lane, npages - 1)];
+            asm volatile("" : "+v"(pages));                // waited for here: behind the branch it would be in every tile
+        }
+        const int pid = __builtin_amdgcn_readlane(pages, page % 64);
         const unsigned char* kb_ = reinterpret_cast<const unsigned char*>(p.cache) +
                                    ((int64_t)pid * p.page_stride + (int64_t)slot0 * p.slot_stride) * 2;
         const unsigned char* vb_ = kb_ + p.kv_half * 2;
@@ -1141,18 +1153,27 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill32_attn_kernel(const AttnPa
     }
 
     l += __shfl_xor(l, 32);
-    if (valid) {
-        const float inv = l > 0.f ? 1.0f / l : 0.f;
-        bf16_t* op = p.out + ((int64_t)(q0 + qi) * p.H + kvh * g + qr) * D;
+    // output rows through LDS: a store writes whole rows
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    __syncthreads();                                       // every wave is past the last image
+    int ln = lane;
+    asm volatile("" : "+v"(ln));                           // nothing below is computed, and kept, in front of the tiles
+    const int oj = ln & 31, oR = R0 + wave * 32 + oj, oq = oR / g;
+    const int orow = oR >= 0 && oR < nrows ? (q0 + oq) * p.H + kvh * g + oR - oq * g : -1;
+    unsigned char* mine = smem + wave * 32 * D * 2;
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
-            for (int rg = 0; rg < 4; ++rg) {
-                const f32x4 ov = {o[db][rg * 4] * inv, o[db][rg * 4 + 1] * inv, o[db][rg * 4 + 2] * inv,
-                                  o[db][rg * 4 + 3] * inv};
-                const int dd = VP ? (db + (rg >> 1) * (NB / 2)) * 16 + (rg & 1) * 8 : db * 32 + rg * 8;
-                *reinterpret_cast<bf16x4*>(op + dd + kh * 4) = __builtin_convertvector(ov, bf16x4);
-            }
+        for (int rg = 0; rg < 4; ++rg) {
+            const f32x4 ov = {o[db][rg * 4] * inv, o[db][rg * 4 + 1] * inv, o[db][rg * 4 + 2] * inv, o[db][rg * 4 + 3] * inv};
+            const int ch = VP ? (db + (rg >> 1) * (NB / 2)) * 2 + (rg & 1) : db * 4 + rg;
+            *reinterpret_cast<bf16x4*>(mine + oj * D * 2 + lds_place<D / 8>(ch, oj) * 16 + (ln >> 5) * 8) = __builtin_convertvector(ov, bf16x4);
+        }
+#pragma unroll
+    for (int i = 0; i < D / 16; ++i) {
+        const int c = i * 64 + ln, r = c / (D / 8), ch = c % (D / 8), row = __shfl(orow, r);
+        const bf16x8 v = lds_read_b128(mine + r * D * 2 + lds_place<D / 8>(ch, r) * 16);
+        if (row >= 0) *reinterpret_cast<bf16x8_a8*>(p.out + (int64_t)row * D + ch * 8) = v;
     }
 }
 
@@ -1299,7 +1320,7 @@ int g_prefill_mfma32 = -1;
 
 template <int D, int NW, int KT, bool VP = true>
 int launch_prefill32_kt(const AttnParams& p, int grid, hipStream_t st) {
-    constexpr int lds = 2 * prefill_stage_bytes<D, KT>() + 32;
+    constexpr int lds = std::max(2 * prefill_stage_bytes<D, KT>() + 32, NW * 32 * D * 2);      // tile images; output rows
     auto k = prefill32_attn_kernel<D, NW, KT, VP>;
     if (lds > 64 * 1024) {
         static MdPerDeviceOnce once;

@@ -24,14 +24,10 @@
 
 namespace {
 
-typedef u32x4 u32x4_a8 __attribute__((aligned(8)));    // output rows start at 8 bytes
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int DK = MD_LATENT_DK, KT = 64, NW = kLatentPrefillRows / 32, NT = 64 * NW;
 
-// Place of 16-byte piece `ch` of a row of `n` pieces in the image.  Keys are read by 16 rows at a time, a piece each: their places differ.
-// Values are read transposed, two pieces of four rows at a time: pairs stay together.
-template <int N>
-__device__ __forceinline__ int key_place(int ch, int row) { return ch ^ (N % 16 ? (row >> 1) & 7 : row & 15); }
+// Places in the image (lds_place for keys): values are read transposed, two pieces of four rows at a time, and pairs stay together.
 template <int N>
 __device__ __forceinline__ int value_place(int ch, int row) { return ch ^ (2 * (row & (N % 16 ? 3 : 7))); }
 __device__ const u32x4 kZeros = {0u, 0u, 0u, 0u};
@@ -123,7 +119,7 @@ __global__ __launch_bounds__(NT, 2) void latent_prefill_kernel(const LatentParam
         const unsigned int to = (unsigned int)(img * STAGE + wave * 1024);
 #pragma unroll
         for (int i = 0; i < NK; ++i) {
-            const int c = i * NT + tid, r = c / CK, row = min(r, rem), d = key_place<CK>(c % CK, r) * 8;
+            const int c = i * NT + tid, r = c / CK, row = min(r, rem), d = lds_place<CK>(c % CK, r) * 8;
             const bf16_t* src = d < p.dim ? kvb + (row * ldkv + hk + d) : rpb + (row * p.W + d - p.dim);
             if (dq < DK) src = d < dq ? src : reinterpret_cast<const bf16_t*>(&kZeros);
             dma16(src, to + i * NT * 16);
@@ -135,7 +131,7 @@ __global__ __launch_bounds__(NT, 2) void latent_prefill_kernel(const LatentParam
         }
     };
     // ---- queries: each wave its own 32 rows, dense rows of a head at a time (a lane's own row piece by piece is 64 places a load)
-    const int kra0 = j * DK * 2 + key_place<CK>(kh, j) * 16;
+    const int kra0 = j * DK * 2 + lds_place<CK>(kh, j) * 16;
     auto key_at = [&](int ks) {                                     // step ks of the lane's row of 32, key or query
         constexpr int low = CK % 16 ? 127 : 255;
         return (kra0 ^ (ks * 32 & low)) + (ks * 32 & ~low);
@@ -143,7 +139,7 @@ __global__ __launch_bounds__(NT, 2) void latent_prefill_kernel(const LatentParam
     if (query_at<DV>() != 0) issue(0, 0);
 #pragma unroll
     for (int i = 0; i < CK / 2; ++i) {
-        const int c = i * 64 + lane, r = c / CK, d = key_place<CK>(c % CK, r) * 8;
+        const int c = i * 64 + lane, r = c / CK, d = lds_place<CK>(c % CK, r) * 8;
         const bf16_t* src = reinterpret_cast<const bf16_t*>(p.q) + ((int64_t)(q0 + max(w0 + r, 0)) * p.H + h) * dq + d;
         dma16(d < dq ? src : reinterpret_cast<const bf16_t*>(&kZeros), query_at<DV>() + wave * 32 * DK * 2 + i * 1024);
     }
@@ -274,14 +270,14 @@ __global__ __launch_bounds__(NT, 2) void latent_prefill_kernel(const LatentParam
         for (int rg = 0; rg < 4; ++rg) {
             const int ch = (db + (rg >> 1) * (NB / 2)) * 2 + (rg & 1);
             const f32x4 ov = {o[db][rg * 4] * inv, o[db][rg * 4 + 1] * inv, o[db][rg * 4 + 2] * inv, o[db][rg * 4 + 3] * inv};
-            *reinterpret_cast<bf16x4*>(mine + j * DV * 2 + key_place<CV>(ch, j) * 16 + kh * 8) = __builtin_convertvector(ov, bf16x4);
+            *reinterpret_cast<bf16x4*>(mine + j * DV * 2 + lds_place<CV>(ch, j) * 16 + kh * 8) = __builtin_convertvector(ov, bf16x4);
         }
 #pragma unroll
     for (int i = 0; i < CV / 2; ++i) {
         const int c = i * 64 + lane, r = c / CV, ch = c % CV;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(mine + r * DV * 2 + key_place<CV>(ch, r) * 16);
+        const bf16x8 v = lds_read_b128(mine + r * DV * 2 + lds_place<CV>(ch, r) * 16);
         if (w0 + r >= 0 && ch * 8 < p.vdim)
-            *reinterpret_cast<u32x4_a8*>(reinterpret_cast<bf16_t*>(p.out) + (q0 + w0 + r) * p.ldo + h * p.vdim + ch * 8) = v;
+            *reinterpret_cast<bf16x8_a8*>(reinterpret_cast<bf16_t*>(p.out) + (q0 + w0 + r) * p.ldo + h * p.vdim + ch * 8) = v;
     }
 }
 

@@ -19,6 +19,7 @@
 // A key tile of one head is one contiguous block of its page (rows padded to DK / DV, heads outermost inside a page), whatever
 // the row width: staging is a linear copy in 16-byte pieces.
 #include "attn_common.h"
+#include <algorithm>
 #include "xattn.h"
 
 #ifndef MD_XATTN_DK
@@ -342,8 +343,11 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? (small_heads<DV>() ? 4 : 2) : 1)
     float* s_bias = reinterpret_cast<float*>(smem + 2 * STAGE + 8 * NW);
     const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, kh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r0 = blockIdx.x >> 3;
-    const int qg = r0 % p.n_qgroups, pair = (r0 / p.n_qgroups) * 8 + (blockIdx.x & 7);
+    // the last groups of every pair first: the longest, until a chunk is full; the last one to start is the last to end
+    // 8 x 2049 rows, 32 heads of 128 on 8 kv heads: 601 us pair after pair, short groups first; 574 long ones first, 545 of every pair; 530
+    // without a load of the page number in front of a tile's, 514 with whole output rows
+    const int r0 = blockIdx.x >> 3, pairs = (p.B * p.KH + 7) / 8;
+    const int qg = p.n_qgroups - 1 - r0 / pairs, pair = (r0 % pairs) * 8 + (blockIdx.x & 7);
     if (pair >= p.B * p.KH) return;
     const int b = pair / p.KH, kvh = pair % p.KH, g = p.g;
     const int q0 = p.qo_indptr[b], n_b = p.qo_indptr[b + 1] - q0;
@@ -351,8 +355,9 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? (small_heads<DV>() ? 4 : 2) : 1)
     const int cap = (p.page_indptr[b + 1] - pg0) * p.page_size;
     const int nrows = n_b * g, last = min(pos_b + n_b - 1, cap - 1);
     if (qg * NW * 32 >= nrows || last < 0) return;                // whole workgroup
-    const int R = (qg * NW + wave) * 32 + j;
-    const bool valid = R < nrows;
+    // groups end with the last row (to a token): rows that fill none are the first ones, with the fewest keys
+    const int R0 = qg * NW * 32 - (NW * 32 - 1 - (nrows - 1) % (NW * 32)) / g * g, R = R0 + wave * 32 + j;
+    const bool valid = R >= 0 && R < nrows;
     const int qi = valid ? R / g : 0, qr = valid ? R - qi * g : 0, h = kvh * g + qr;
     const int pos = pos_b + qi;
     const int lim = valid ? min(pos, cap - 1) : -1, low = valid ? (pos / p.chunk) * p.chunk : 0x7fffffff;
@@ -390,7 +395,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? (small_heads<DV>() ? 4 : 2) : 1)
     const float sl2 = p.scale_log2, mref = -p.ref_log2;
     // bias table of one tile: entry e of head r is the distance d = (position of the workgroup's first token) - (last key of
     // the tile) + e.  A lane's entries have the same indexes in every tile.
-    const int tok0 = qg * NW * 32 / g, tsize = g * W;
+    const int tok0 = R0 / g, tsize = g * W;
     const float* my_bias = s_bias + (valid ? qr * W + qi - tok0 : 0) + 4 - 4 * kh;
     const int fill_r = tid / W, fill_e = tid - fill_r * W;
     auto fill = [&](int t, float* tab) {
@@ -415,9 +420,16 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? (small_heads<DV>() ? 4 : 2) : 1)
     float l = 0.f;
 
     u32x4 kreg[NK], vreg[NV];
+    // numbers of 64 pages, one a lane: no load in front of a tile's
+    int pages = p.page_indices[pg0 + min(t0 * KT / p.page_size / 64 * 64 + lane, last / p.page_size)];
+    asm volatile("" : "+v"(pages));
     auto issue = [&](int t) {
         const int kp0 = t * KT, page = kp0 / p.page_size, slot = kp0 - page * p.page_size;
-        const int pid = __builtin_amdgcn_readfirstlane(p.page_indices[pg0 + page]);
+        if (page % 64 == 0 && slot == 0 && t != t0) {
+            pages = p.page_indices[pg0 + min(page + lane, last / p.page_size)];
+            asm volatile("" : "+v"(pages));                         // waited for here: behind the branch it would be in every tile
+        }
+        const int pid = __builtin_amdgcn_readlane(pages, page % 64);
         const int64_t row = ((int64_t)pid * p.KH + kvh) * p.page_size + slot;
         const u32x4* kp = reinterpret_cast<const u32x4*>(reinterpret_cast<const bf16_t*>(p.k_cache) + row * DK);
         const u32x4* vp = reinterpret_cast<const u32x4*>(reinterpret_cast<const bf16_t*>(p.v_cache) + row * DV);
@@ -518,23 +530,35 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? (small_heads<DV>() ? 4 : 2) : 1)
     }
 
     l += __shfl_xor(l, 32);
-    if (valid) {
-        const float inv = 1.0f / (l + __builtin_amdgcn_exp2f(mref));
-        bf16_t* op = reinterpret_cast<bf16_t*>(p.out) + ((int64_t)(q0 + qi) * p.H + h) * p.DV;
+    // output rows through LDS: a store writes whole rows
+    const float inv = 1.0f / (l + __builtin_amdgcn_exp2f(mref));
+    __syncthreads();                                                // every wave is past the last image
+    int ln = lane;
+    asm volatile("" : "+v"(ln));                                    // nothing below is computed, and kept, in front of the tiles
+    const int oj = ln & 31, oR = R0 + wave * 32 + oj, oq = oR / g;
+    const int orow = oR >= 0 && oR < nrows ? (q0 + oq) * p.H + kvh * g + oR - oq * g : -1;
+    unsigned char* mine = smem + wave * 32 * DV * 2;
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
-            for (int rg = 0; rg < 4; ++rg) {
-                const int d = (db + (rg >> 1) * (NB / 2)) * 16 + (rg & 1) * 8 + kh * 4;
-                const f32x4 ov = {o[db][rg * 4] * inv, o[db][rg * 4 + 1] * inv, o[db][rg * 4 + 2] * inv, o[db][rg * 4 + 3] * inv};
-                if ((p.DV & 3) == 0) {
-                    if (d < p.DV) *reinterpret_cast<bf16x4*>(op + d) = __builtin_convertvector(ov, bf16x4);
-                } else {
+        for (int rg = 0; rg < 4; ++rg) {
+            const int ch = (db + (rg >> 1) * (NB / 2)) * 2 + (rg & 1);
+            const f32x4 ov = {o[db][rg * 4] * inv, o[db][rg * 4 + 1] * inv, o[db][rg * 4 + 2] * inv, o[db][rg * 4 + 3] * inv};
+            *reinterpret_cast<bf16x4*>(mine + oj * DV * 2 + lds_place<DV / 8>(ch, oj) * 16 + (ln >> 5) * 8) = __builtin_convertvector(ov, bf16x4);
+        }
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (d + e < p.DV) op[d + e] = f32_to_bf16(ov[e]);
-                }
-            }
+    for (int i = 0; i < DV / 16; ++i) {
+        const int c = i * 64 + ln, r = c / (DV / 8), d = c % (DV / 8) * 8, row = __shfl(orow, r);
+        const bf16x8 v = lds_read_b128(mine + r * DV * 2 + lds_place<DV / 8>(d / 8, r) * 16);
+        bf16_t* op = reinterpret_cast<bf16_t*>(p.out) + (int64_t)row * p.DV + d;
+        if (row < 0) continue;
+        if (p.DV % 8 == 0) {
+            if (d < p.DV) *reinterpret_cast<bf16x8_a8*>(op) = v;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (d + e < p.DV) op[e] = v[e];
+        }
     }
 }
 
@@ -580,7 +604,9 @@ int bias_width(int g) {
     return w;
 }
 template <int DV, int NW>
-int prefill_lds(int g) { return 2 * stage_bytes<DV>(prefill_kt<DV, NW>()) + 8 * NW + 8 * g * bias_width<DV, NW>(g); }
+int prefill_lds(int g) {
+    return std::max(2 * stage_bytes<DV>(prefill_kt<DV, NW>()) + 8 * NW + 8 * g * bias_width<DV, NW>(g), NW * 32 * DV * 2);    // (output rows)
+}
 
 template <int DV, int NW>
 int launch_prefill(const XattnParams& p, int grid, hipStream_t st) {

@@ -259,6 +259,17 @@ def test_attention(ops, H, KH, D, DV, chunk, dtype):
     parity_report(f"[layers-attention] H={H} KH={KH} D={D} DV={DV} chunk={chunk} {str(dtype)[6:]} max err {max(errs):.2e}")
 
 
+@pytest.mark.parametrize("D,DV", [(64, 64), (128, 100), (32, 128)])
+def test_prompt_rows_over_more_than_64_pages(ops, D, DV):
+    """A chunk that begins in page 39 and ends behind page 64, whose numbers are kept 64 at a time; rows that fill no workgroup."""
+    n = 64 * 128 + 205
+    spec, rows, ref = attention_case(ops, 1, 1, D, DV, 5000, D, BF, [n])
+    s = Seqs(ops, spec, BF, [n], seed=1)
+    for at, k in ((0, 8000), (8000, 33), (8033, n - 8033)):
+        got = s.attend(rows[0][at:at + k], [0], [at], [k])
+        assert float((got.double() - ref[0][at:at + k]).abs().max()) <= 1.5e-2 * max(1.0, float(ref[0].abs().max())), at
+
+
 def test_attention_across_every_chunk_and_page_edge(ops):
     """Decode 40 tokens across chunk borders that fall on, just before and just behind page and tile borders; every query asks
     for the last key of the previous chunk or the first of its own."""

@@ -92,6 +92,24 @@ def test_paged_attention_vs_oracle(ops, name, B, n, H, KH, D, lens, causal, scat
     check_attention(name, out, oracle, ref64, bnd)
 
 
+@pytest.mark.parametrize("H,KH,D,ns,lens", [(10, 2, 128, [110, 41], [4230, 4096]), (10, 2, 128, [40, 1], [4097, 64]), (3, 1, 64, [100], [4300]),
+                                            (4, 1, 64, [300, 33], [4200, 33])])
+def test_prompt_rows_over_more_than_64_pages(ops, H, KH, D, ns, lens):
+    """Page numbers are kept 64 at a time; query rows that fill no workgroup are a request's first ones, also where its heads per kv head
+    do not divide one."""
+    name = f"prefill-many-pages-{H}-{KH}-{D}-{ns[0]}"
+    cache, indices, indptr, last, max_pages = make_paged(len(ns), lens, KH, D, seed=case_seed(name), page_size=64, scatter=True)
+    q = torch.randn(sum(ns), H, D, generator=torch.Generator().manual_seed(3)).to(BF)
+    qo = torch.tensor([0] + list(np.cumsum(ns)), dtype=torch.int32)
+    oracle = fr.batch_prefill_paged(q, cache, qo, indices, indptr, last, H, KH, D, causal=True)
+    ref64, bnd = dense_attention_f64(q, cache, qo, indices, indptr, last, H, KH, D, causal=True)
+    out = torch.full((sum(ns) + 2, H, D), 7.0, dtype=BF, device=DEV)          # 2 guard rows
+    ops.paged_attention(q.to(DEV), cache.to(DEV), qo.to(DEV), indices.to(DEV), indptr.to(DEV), last.to(DEV), max(ns), max_pages,
+                        ops.AttnWorkspace(DEV), causal=True, out=out[:sum(ns)])
+    assert bool((out[sum(ns):] == 7).all())
+    check_attention(name, out[:sum(ns)], oracle, ref64, bnd)
+
+
 @pytest.mark.parametrize("name,H,KH,D,ns,lens,fp8", [
     ("verify-ragged-rows", 8, 2, 128, [3, 4, 1], [300, 257, 64], False),
     ("prefill-ragged-rows", 8, 2, 128, [100, 128, 0, 17], [384, 300, 50, 17], False),
