@@ -471,6 +471,19 @@ def choose(M: int, N: int, K: int, swiglu: bool, int8: bool, packed: bool, kind:
     return "skinny" if use_skinny(M, N, K, swiglu, int8, packed, kind, absorbs_norm) else "lib"
 
 
+def prompt_over_block(M: int, N: int, K: int, swiglu: bool = False) -> bool:
+    """Do 129 to 256 rows that `choose` gives to md_linear_block run on md_linear_prompt instead?  It takes 256 columns a workgroup, the block
+    kernel 128: twice the columns in one round of the chip, which takes it 1.5 to 1.6 times as long at up to 192 rows, 1.68 to 1.74 times
+    beyond.  Gate | up of 55 296 x 5 120 at 130 / 192 / 256 rows 143 / 163 / 174 -> 125 / 136 / 147 us, 37 888 x 3 584 93 / 102 / 113 -> 76 / 80
+    / 86, a head of 128 256 x 4 096 241 / 259 / 275 -> 207 / 223 / 245; in one round of both (28 672 x 4 096: 54 / 59 / 65 and 53 / 59 / 72)
+    or where its last round is the emptier one (152 064 x 3 584, 256 rows: 302 and 313) the block kernel stays."""
+    from .. import ops
+    if _MODE != "auto" or _BLOCK == "1" or not 128 < M <= 256:
+        return False
+    wide, narrow = -(-N // (256 * CUS)), -(-N // (128 * CUS))
+    return (1.6 if M <= 192 else 1.74) * wide < narrow and ops.linear_prompt_us(M, N, K, swiglu) >= 0
+
+
 @functools.lru_cache(maxsize=4096)
 def prompt_rows(M: int, N: int, K: int, swiglu: bool = False) -> int:
     """How many of a prompt's M rows (more than a step has; weight in the streaming layout) go to md_linear_prompt in one call: none (the

@@ -40,7 +40,7 @@ import torch.nn as nn
 from torch.nn import functional as F
 
 from .. import ops
-from .gemm_policy import prompt_rows
+from .gemm_policy import prompt_over_block, prompt_rows
 
 
 def find_multiple(n: int, k: int) -> int:
@@ -596,7 +596,7 @@ class Transformer(nn.Module):
         kind = "swiglu" if swiglu else ("resid" if resid is not None else "plain")
         how = (choose(M, N, K, swiglu, w.dtype == torch.int8, pk is not None, kind, pro is not None and swiglu)
                if x2d.is_cuda else "lib")
-        if how == "lib" and x2d.is_cuda and self._on_prompt_gemm(x2d, w, pk, swiglu):
+        if how in ("lib", "block") and x2d.is_cuda and self._on_prompt_gemm(x2d, w, pk, swiglu, how == "block"):
             how = "prompt"
         if how == "prompt":
             return self._prompt_linear(x2d if pro is None else pro.materialize(), pk, bias, swiglu)
@@ -627,18 +627,18 @@ class Transformer(nn.Module):
         return h
 
     @staticmethod
-    def _on_prompt_gemm(x2d, w, pk, swiglu=False):
-        """Do these rows (more than a step has) run on md_linear_prompt?  It reads the streaming layout: no row-major weight has to come
-        back.  The shapes alone decide, so that the ranks of a group agree."""
+    def _on_prompt_gemm(x2d, w, pk, swiglu=False, block=False):
+        """Do these rows run on md_linear_prompt: more than a step has, or (block) a step's in the place of md_linear_block?  It reads the
+        streaming layout: no row-major weight has to come back.  The shapes alone decide, so that the ranks of a group agree."""
         M, K = x2d.shape
-        return (M > 256 and pk is not None and w.dtype == torch.bfloat16 and x2d.dtype == torch.bfloat16 and x2d.stride(1) == 1
+        return (M > 128 and pk is not None and w.dtype == torch.bfloat16 and x2d.dtype == torch.bfloat16 and x2d.stride(1) == 1
                 and x2d.stride(0) % 8 == 0 and x2d.stride(0) < 1 << 20 and x2d.data_ptr() % 16 == 0
-                and prompt_rows(M, w.shape[0], K, swiglu) > 0)
+                and (prompt_rows(M, w.shape[0], K, swiglu) > 0 if M > 256 else block and prompt_over_block(M, w.shape[0], K, swiglu)))
 
     def _prompt_linear(self, x2d, pk, bias=None, swiglu=False, out=None, **act):
         """A linear of a prompt's rows: whole row tiles on md_linear_prompt, a few rows behind them on the weight-streaming kernel."""
         M, K = x2d.shape
-        rows = prompt_rows(M, pk.N, K, swiglu)
+        rows = prompt_rows(M, pk.N, K, swiglu) if M > 256 else M
         if rows == M:
             return ops.linear_prompt(x2d, pk, bias, swiglu, out=out, **act)
         if out is None:

@@ -123,3 +123,34 @@ def test_rows_behind_whole_tiles(M, N, K, swiglu):
     bound = ((s * (1 + h1 * (1 - s))).abs() * (h1.abs() * U + 2 * off[:, :n_out]) * h3.abs() + (h1 * s).abs() * 2 * off[:, n_out:]
              + 3 * U * (h1 * s * h3).abs()) * 1.02 + 1e-30
     assert ((out.double() - h1 * s * h3).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("M,N,K,swiglu,taken", [(129, 33024, 512, True, True), (192, 65536, 256, False, True), (256, 37888, 512, True, True),
+                                                (256, 32768, 512, True, False), (128, 37888, 512, True, False), (255, 152064, 256, False, False)])
+def test_a_steps_rows_in_the_place_of_the_block_kernel(M, N, K, swiglu, taken, monkeypatch):
+    """Both sides of the rule's lines, through the model's linear; every row against float64."""
+    from types import SimpleNamespace
+    from magicdec_amd import ops
+    from magicdec_amd.Engine import gemm_policy
+    from magicdec_amd.Engine.model_core import Transformer
+    monkeypatch.setattr(gemm_policy, "choose", lambda *a, **kw: "block")
+    x, w, bias = case(M, N, K, M)
+    assert gemm_policy.prompt_over_block(M, N, K, swiglu) == taken
+    calls, real = [], ops.linear_prompt
+    monkeypatch.setattr(ops, "linear_prompt", lambda *a, **kw: calls.append(1) or real(*a, **kw))
+    pk = ops.PackedWeight(w, swiglu=swiglu)
+    model = SimpleNamespace(workspace=ops.AttnWorkspace(DEV), _packed={id(w): pk}, _on_prompt_gemm=Transformer._on_prompt_gemm)
+    model._prompt_linear = lambda *a, **kw: Transformer._prompt_linear(model, *a, **kw)
+    out = Transformer._linear(model, x, SimpleNamespace(weight=w, bias=None if swiglu else bias), swiglu_w13=(w, None) if swiglu else None)
+    assert len(calls) == taken
+    ref, off = product(x, w)
+    if swiglu:
+        h1, h3 = ref[:, :N // 2], ref[:, N // 2:]
+        s = torch.sigmoid(h1)
+        # (the block kernel rounds both halves and the SiLU to bf16: as many half-ulps as roundings)
+        bound = ((s * (1 + h1 * (1 - s))).abs() * (h1.abs() * U + 2 * off[:, :N // 2]) * h3.abs() + (h1 * s).abs() * 2 * off[:, N // 2:]
+                 + 3 * U * (h1 * s * h3).abs()) * 1.02 + 1e-30
+        assert ((out.double() - h1 * s * h3).abs() <= bound).all()
+    else:
+        want = ref + bias.double()
+        assert ((out.double() - want).abs() <= want.abs() * U + 2 * off + 2.0 ** -23 * bias.double().abs()).all()
