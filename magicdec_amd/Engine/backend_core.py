@@ -253,7 +253,7 @@ class _BackendBase:
         out = []
         if chunks > 1 and alone:
             out, at, chunks = [(0, CHUNK)], CHUNK, chunks - 1
-        # the last chunk rides along unless that takes a portion more: 8192 rows are whole rounds of the library's tiles, 8324 are not
+        # the last chunk rides along unless that takes a portion more: 8192 rows are whole rounds of the GEMM's tiles, 8324 are not
         first, most = at, max(1, most)
         parts = max(min(1, chunks), -(-(chunks - 1) // most))
         if chunks > parts * most:

@@ -346,8 +346,9 @@ class Transformer(nn.Module):
     def _pack_weights(self, force=False):
         """Streaming-layout copies (ops.PackedWeight) of the weights the hand-written GEMMs serve in decode / verify
         steps -- md_linear for the long weight streams, md_linear_fused for the launch-bound small products
-        (Engine/gemm_policy.py); keyed by the id of the row-major tensor the step would otherwise use.  The row-major
-        tensors stay for the prefill-sized library GEMMs; the extra bytes are reported once (`packed_bytes`)."""
+        (Engine/gemm_policy.py), and the same copies for the rows of prompts (md_linear_prompt); keyed by the id of the row-major
+        tensor that would otherwise be used.  The row-major tensors stay for the products that are left to the library; the extra
+        bytes are reported once (`packed_bytes`)."""
         from .gemm_policy import want_packed
         self.__dict__.pop("_row_bytes", None)
         self._released_sum = 0

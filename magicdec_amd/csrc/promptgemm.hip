@@ -4,6 +4,8 @@
 //           16 384 rows, which ran on the library: over row-major weights that every prompt had to bring back from the streaming layout
 //           first (unpack_weight: 320 of 6 500 us of a two-layer 8B prompt), and with the gated activation as a pass of its own (260 us).
 //
+// Also a step's 129 to 256 rows where the block kernel needs a second round of the chip for its 128 columns a workgroup.
+//
 // What bounds it.  A full chip of matrix instructions is bound by power: the clock falls to about 1.75 of 2.4 GHz, and time is energy as much
 // as it is stalls.  v_mfma_f32_16x16x32 moves half the accumulator bytes per flop of 32x32x16 and is the faster one by clock, although its
 // 16 cycles hide less behind each (8192^3: 88 % of the cycles with the large one took as long as 82 % with the small one).  Measured, us:
