@@ -99,6 +99,14 @@ def test_layers_share_one_cache_and_the_head_is_the_embedding(latent_ops, model)
     assert e.model._xspec[0].rotary is e.model._xspec[2].rotary and e.model.rollback_depth() is None
 
 
+def test_the_product_in_fills_whole_tiles_of_columns(latent_ops, model):
+    """32 columns each; the rows behind the parts are zeros, the parts where the checkpoint's are."""
+    for layer in engine(model[0], slots=1).model.layers:
+        att, n = layer.attention, sum(layer.attention.cuts)
+        w = att.win.weight
+        assert w.shape[0] % 32 == 0 and n <= w.shape[0] < n + 32 and not w[n:].any() and bool(w[:n].any(1).all())
+
+
 @pytest.mark.parametrize("portion_rows", [6, 17, 1000])
 def test_ragged_steps_portions_and_reuse(latent_ops, model, monkeypatch, portion_rows):
     from magicdec_amd.Engine import backend_core
