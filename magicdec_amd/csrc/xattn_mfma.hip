@@ -329,6 +329,11 @@ __global__ __launch_bounds__(256, (decode_wgs<DV, QT>())) void xattn_decode_kern
 // heads of at most 64: 64-key tiles and 128 registers put two eight-wave workgroups on a CU
 template <int DV>
 constexpr bool small_heads() { return DK <= 64 && DV <= 64; }
+// Page numbers in lanes, so that no tile's loads wait for one, and output rows through LDS: with tiles of 128 keys (8 x 2049 rows, 32 heads
+// of 128 on 8 kv heads 545 -> 530 -> 514 us).  Tiles of 64 are those of the widest heads and the narrowest, which have no registers left for
+// it: 2 x 753 rows behind 16 000, 16 heads of 128 / 256 152 us, 191 with both; 2 x 676 behind 1000, 24 heads of 64 71 and 78
+template <int KT>
+constexpr bool wide_tiles() { return KT == 128; }
 
 // NW wavefronts of 32 query rows (token-major: row = token * g + head of the group) share KT-key tiles through two LDS
 // images, one barrier per tile.  A workgroup visits the tiles from its first row's chunk start to its last row's position.
@@ -338,14 +343,15 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? (small_heads<DV>() ? 4 : 2) : 1)
     constexpr int K_BYTES = KT * KROW, VG = NB * kVSub, STAGE = stage_bytes<DV>(KT);
     constexpr int CK = KT * DK / 8, CV = KT * DV / 8;            // 16-byte pieces of a tile
     constexpr int NK = (CK + 64 * NW - 1) / (64 * NW), NV = (CV + 64 * NW - 1) / (64 * NW);
+    constexpr bool WIDE = wide_tiles<KT>();
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // 2 x STAGE, int[2 NW], 2 x float[g W]
     int* s_rng = reinterpret_cast<int*>(smem + 2 * STAGE);
     float* s_bias = reinterpret_cast<float*>(smem + 2 * STAGE + 8 * NW);
     const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, kh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // the last groups of every pair first: the longest, until a chunk is full; the last one to start is the last to end
-    // 8 x 2049 rows, 32 heads of 128 on 8 kv heads: 601 us pair after pair, short groups first; 574 long ones first, 545 of every pair; 530
-    // without a load of the page number in front of a tile's, 514 with whole output rows
+    // 8 x 2049 rows, 32 heads of 128 on 8 kv heads: 601 us pair after pair, short groups first; 574 long ones first, 545 of every pair; 530 and 514:
+    // wide_tiles
     const int r0 = blockIdx.x >> 3, pairs = (p.B * p.KH + 7) / 8;
     const int qg = p.n_qgroups - 1 - r0 / pairs, pair = (r0 % pairs) * 8 + (blockIdx.x & 7);
     if (pair >= p.B * p.KH) return;
@@ -420,16 +426,19 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? (small_heads<DV>() ? 4 : 2) : 1)
     float l = 0.f;
 
     u32x4 kreg[NK], vreg[NV];
-    // numbers of 64 pages, one a lane: no load in front of a tile's
-    int pages = p.page_indices[pg0 + min(t0 * KT / p.page_size / 64 * 64 + lane, last / p.page_size)];
-    asm volatile("" : "+v"(pages));
+    // numbers of 64 pages, one a lane
+    int pages = 0;
+    if constexpr (WIDE) {
+        pages = p.page_indices[pg0 + min(t0 * KT / p.page_size / 64 * 64 + lane, last / p.page_size)];
+        asm volatile("" : "+v"(pages));
+    }
     auto issue = [&](int t) {
         const int kp0 = t * KT, page = kp0 / p.page_size, slot = kp0 - page * p.page_size;
-        if (page % 64 == 0 && slot == 0 && t != t0) {
+        if (WIDE && page % 64 == 0 && slot == 0 && t != t0) {
             pages = p.page_indices[pg0 + min(page + lane, last / p.page_size)];
             asm volatile("" : "+v"(pages));                         // waited for here: behind the branch it would be in every tile
         }
-        const int pid = __builtin_amdgcn_readlane(pages, page % 64);
+        const int pid = WIDE ? __builtin_amdgcn_readlane(pages, page % 64) : __builtin_amdgcn_readfirstlane(p.page_indices[pg0 + page]);
         const int64_t row = ((int64_t)pid * p.KH + kvh) * p.page_size + slot;
         const u32x4* kp = reinterpret_cast<const u32x4*>(reinterpret_cast<const bf16_t*>(p.k_cache) + row * DK);
         const u32x4* vp = reinterpret_cast<const u32x4*>(reinterpret_cast<const bf16_t*>(p.v_cache) + row * DV);
@@ -530,35 +539,44 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? (small_heads<DV>() ? 4 : 2) : 1)
     }
 
     l += __shfl_xor(l, 32);
-    // output rows through LDS: a store writes whole rows
     const float inv = 1.0f / (l + __builtin_amdgcn_exp2f(mref));
-    __syncthreads();                                                // every wave is past the last image
-    int ln = lane;
-    asm volatile("" : "+v"(ln));                                    // nothing below is computed, and kept, in front of the tiles
-    const int oj = ln & 31, oR = R0 + wave * 32 + oj, oq = oR / g;
-    const int orow = oR >= 0 && oR < nrows ? (q0 + oq) * p.H + kvh * g + oR - oq * g : -1;
-    unsigned char* mine = smem + wave * 32 * DV * 2;
+    if (WIDE && p.DV % 8 == 0) {                                    // output rows through LDS: a store writes whole rows
+        __syncthreads();                                            // every wave is past the last image
+        int ln = lane;
+        asm volatile("" : "+v"(ln));                                // nothing below is computed, and kept, in front of the tiles
+        const int oj = ln & 31, oR = R0 + wave * 32 + oj, oq = oR / g;
+        const int orow = oR >= 0 && oR < nrows ? (q0 + oq) * p.H + kvh * g + oR - oq * g : -1;
+        unsigned char* mine = smem + wave * 32 * DV * 2;
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
+        for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int rg = 0; rg < 4; ++rg) {
-            const int ch = (db + (rg >> 1) * (NB / 2)) * 2 + (rg & 1);
-            const f32x4 ov = {o[db][rg * 4] * inv, o[db][rg * 4 + 1] * inv, o[db][rg * 4 + 2] * inv, o[db][rg * 4 + 3] * inv};
-            *reinterpret_cast<bf16x4*>(mine + oj * DV * 2 + lds_place<DV / 8>(ch, oj) * 16 + (ln >> 5) * 8) = __builtin_convertvector(ov, bf16x4);
+            for (int rg = 0; rg < 4; ++rg) {
+                const int ch = (db + (rg >> 1) * (NB / 2)) * 2 + (rg & 1);
+                const f32x4 ov = {o[db][rg * 4] * inv, o[db][rg * 4 + 1] * inv, o[db][rg * 4 + 2] * inv, o[db][rg * 4 + 3] * inv};
+                *reinterpret_cast<bf16x4*>(mine + oj * DV * 2 + lds_place<DV / 8>(ch, oj) * 16 + (ln >> 5) * 8) = __builtin_convertvector(ov, bf16x4);
+            }
+#pragma unroll
+        for (int i = 0; i < DV / 16; ++i) {
+            const int c = i * 64 + ln, r = c / (DV / 8), d = c % (DV / 8) * 8, row = __shfl(orow, r);
+            const bf16x8 v = lds_read_b128(mine + r * DV * 2 + lds_place<DV / 8>(d / 8, r) * 16);
+            if (row >= 0 && d < p.DV) *reinterpret_cast<bf16x8_a8*>(reinterpret_cast<bf16_t*>(p.out) + (int64_t)row * p.DV + d) = v;
         }
+    } else if (valid) {
+        bf16_t* op = reinterpret_cast<bf16_t*>(p.out) + ((int64_t)(q0 + qi) * p.H + h) * p.DV;
 #pragma unroll
-    for (int i = 0; i < DV / 16; ++i) {
-        const int c = i * 64 + ln, r = c / (DV / 8), d = c % (DV / 8) * 8, row = __shfl(orow, r);
-        const bf16x8 v = lds_read_b128(mine + r * DV * 2 + lds_place<DV / 8>(d / 8, r) * 16);
-        bf16_t* op = reinterpret_cast<bf16_t*>(p.out) + (int64_t)row * p.DV + d;
-        if (row < 0) continue;
-        if (p.DV % 8 == 0) {
-            if (d < p.DV) *reinterpret_cast<bf16x8_a8*>(op) = v;
-        } else {
+        for (int db = 0; db < DB; ++db)
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if (d + e < p.DV) op[e] = v[e];
-        }
+            for (int rg = 0; rg < 4; ++rg) {
+                const int d = (db + (rg >> 1) * (NB / 2)) * 16 + (rg & 1) * 8 + kh * 4;
+                const f32x4 ov = {o[db][rg * 4] * inv, o[db][rg * 4 + 1] * inv, o[db][rg * 4 + 2] * inv, o[db][rg * 4 + 3] * inv};
+                if ((p.DV & 3) == 0) {
+                    if (d < p.DV) *reinterpret_cast<bf16x4*>(op + d) = __builtin_convertvector(ov, bf16x4);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (d + e < p.DV) op[d + e] = f32_to_bf16(ov[e]);
+                }
+            }
     }
 }
 
@@ -605,7 +623,8 @@ int bias_width(int g) {
 }
 template <int DV, int NW>
 int prefill_lds(int g) {
-    return std::max(2 * stage_bytes<DV>(prefill_kt<DV, NW>()) + 8 * NW + 8 * g * bias_width<DV, NW>(g), NW * 32 * DV * 2);    // (output rows)
+    const int tiles = 2 * stage_bytes<DV>(prefill_kt<DV, NW>()) + 8 * NW + 8 * g * bias_width<DV, NW>(g);
+    return wide_tiles<prefill_kt<DV, NW>()>() ? std::max(tiles, NW * 32 * DV * 2) : tiles;       // (output rows)
 }
 
 template <int DV, int NW>

@@ -270,6 +270,16 @@ def test_prompt_rows_over_more_than_64_pages(ops, D, DV):
         assert float((got.double() - ref[0][at:at + k]).abs().max()) <= 1.5e-2 * max(1.0, float(ref[0].abs().max())), at
 
 
+@pytest.mark.parametrize("D,DV", [(128, 128), (96, 104), (128, 100), (96, 102), (128, 97), (64, 60), (128, 252)])
+def test_output_rows_of_any_width(ops, D, DV):
+    """Output rows that are whole 16-byte pieces, 8-byte ones and neither; tiles of 128 keys and of 64."""
+    n = 301
+    spec, rows, ref = attention_case(ops, 4, 2, D, DV, 0, DV, BF, [n])
+    s = Seqs(ops, spec, BF, [n], seed=1)
+    got = s.attend(rows[0], [0], [0], [n])
+    assert got.shape == ref[0].shape and float((got.double() - ref[0]).abs().max()) <= 1.5e-2 * max(1.0, float(ref[0].abs().max()))
+
+
 def test_attention_across_every_chunk_and_page_edge(ops):
     """Decode 40 tokens across chunk borders that fall on, just before and just behind page and tile borders; every query asks
     for the last key of the previous chunk or the first of its own."""
