@@ -361,9 +361,10 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? (small_heads<DV>() ? 4 : 2) : 1)
     const int cap = (p.page_indptr[b + 1] - pg0) * p.page_size;
     const int nrows = n_b * g, last = min(pos_b + n_b - 1, cap - 1);
     if (qg * NW * 32 >= nrows || last < 0) return;                // whole workgroup
-    // groups end with the last row (to a token): rows that fill none are the first ones, with the fewest keys
-    const int R0 = qg * NW * 32 - (NW * 32 - 1 - (nrows - 1) % (NW * 32)) / g * g, R = R0 + wave * 32 + j;
-    const bool valid = R >= 0 && R < nrows;
+    // groups begin with the first row: those that end a prompt, behind the most keys, are the ones that may have few (2 x 220 rows, 8 heads
+    // of 256: 47 us, 51 with groups that end with the last row; 1183 rows, 32 heads of 128 on 8 kv heads 69 and 72)
+    const int R0 = qg * NW * 32, R = R0 + wave * 32 + j;
+    const bool valid = R < nrows;
     const int qi = valid ? R / g : 0, qr = valid ? R - qi * g : 0, h = kvh * g + qr;
     const int pos = pos_b + qi;
     const int lim = valid ? min(pos, cap - 1) : -1, low = valid ? (pos / p.chunk) * p.chunk : 0x7fffffff;
@@ -545,7 +546,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? (small_heads<DV>() ? 4 : 2) : 1)
         int ln = lane;
         asm volatile("" : "+v"(ln));                                // nothing below is computed, and kept, in front of the tiles
         const int oj = ln & 31, oR = R0 + wave * 32 + oj, oq = oR / g;
-        const int orow = oR >= 0 && oR < nrows ? (q0 + oq) * p.H + kvh * g + oR - oq * g : -1;
+        const int orow = oR < nrows ? (q0 + oq) * p.H + kvh * g + oR - oq * g : -1;
         unsigned char* mine = smem + wave * 32 * DV * 2;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
