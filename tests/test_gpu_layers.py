@@ -280,6 +280,20 @@ def test_output_rows_of_any_width(ops, D, DV):
     assert got.shape == ref[0].shape and float((got.double() - ref[0]).abs().max()) <= 1.5e-2 * max(1.0, float(ref[0].abs().max()))
 
 
+@pytest.mark.parametrize("first", [0, 1])
+@pytest.mark.parametrize("H,KH,D,DV", [(4, 2, 128, 128), (3, 3, 64, 64), (4, 1, 128, 256)])
+def test_prompt_rows_in_either_order_of_their_groups(ops, first, H, KH, D, DV):
+    """A few rows behind many and a whole prompt in one call, either of them first (which decides the order of the workgroups)."""
+    lens = [1500, 700]
+    spec, rows, ref = attention_case(ops, H, KH, D, DV, 1024, D + DV, BF, lens)
+    s = Seqs(ops, spec, BF, lens, seed=1)
+    s.attend(rows[0][:1170], [0], [0], [1170])
+    part = [(0, 1170, 330), (1, 0, 700)][::1 - 2 * first]
+    got = s.attend(torch.cat([rows[b][a:a + k] for b, a, k in part]), [b for b, _, _ in part], [a for _, a, _ in part], [k for _, _, k in part])
+    want = torch.cat([ref[b][a:a + k] for b, a, k in part])
+    assert float((got.double() - want).abs().max()) <= 1.5e-2 * max(1.0, float(want.abs().max()))
+
+
 def test_attention_across_every_chunk_and_page_edge(ops):
     """Decode 40 tokens across chunk borders that fall on, just before and just behind page and tile borders; every query asks
     for the last key of the previous chunk or the first of its own."""
