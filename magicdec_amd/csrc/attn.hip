@@ -968,9 +968,12 @@ __global__ __launch_bounds__(64 * NW, D == 64 && KT == 64 ? 4 : 2) void prefill3
     const int npages = p.page_indptr[b + 1] - pg0;
     const int kv_len = npages > 0 ? min((npages - 1) * p.page_size + p.last_page_len[b], npages * p.page_size) : 0;
     const int nrows = n_b * g;
-    // this lane's query row (both kh halves hold the same query).  Groups end with the last row: rows that fill none are the first
-    // ones, with the fewest keys
-    const int R0 = qg * NW * 32 - (NW * 32 - 1 - (nrows - 1) % (NW * 32)) / g * g, R = R0 + wave * 32 + j;
+    // this lane's query row (both kh halves hold the same query).  In more than two rounds of the chip groups end with the last row: rows
+    // that fill none are the first ones, with the fewest keys (8 x 700 rows behind 100, 32 heads on 8 kv heads 83 us, 87 otherwise).  In
+    // fewer, groups begin with the first row: the one with the most keys is the one that may have few (4 x 901 rows, 16 heads on 2 37 us,
+    // 39 otherwise; 4 x 846, 32 heads on 32 60 and 65)
+    constexpr unsigned kTwoRounds = D == 64 && KT == 64 ? 1024 : 512;
+    const int R0 = qg * NW * 32 - (gridDim.x > kTwoRounds ? (NW * 32 - 1 - (nrows - 1) % (NW * 32)) / g * g : 0), R = R0 + wave * 32 + j;
     const bool valid = R >= 0 && R < nrows;
     const int qi = R / g, qr = R - qi * g;
     const int lim = valid ? (p.causal ? kv_len - n_b + qi : kv_len - 1) : -1;

@@ -110,6 +110,26 @@ def test_prompt_rows_over_more_than_64_pages(ops, H, KH, D, ns, lens):
     check_attention(name, out[:sum(ns)], oracle, ref64, bnd)
 
 
+@pytest.mark.parametrize("H,KH,D,B", [(8, 8, 128, 32), (8, 8, 128, 33), (8, 8, 64, 64), (8, 8, 64, 65), (6, 2, 128, 129)])
+def test_groups_of_two_rounds_of_the_chip_and_more(ops, H, KH, D, B):
+    """512 and 528 workgroups of 256 rows (heads of 64: 1024 and 1040): which rows a group begins with changes between them.  Requests of
+    no row, one, a whole group, and a few rows more than one or two."""
+    name = f"prefill-rounds-{H}-{KH}-{D}-{B}"
+    ns = [(270 * KH // H + 7 * b) % (512 * KH // H) if b % 5 else (0, 1, 256 * KH // H, 512 * KH // H)[b // 5 % 4] for b in range(B)]
+    lens = [n + 30 * (b % 4) for b, n in enumerate(ns)]
+    lens = [max(v, 1) for v in lens]
+    cache, indices, indptr, last, max_pages = make_paged(B, lens, KH, D, seed=case_seed(name), scatter=True)
+    q = torch.randn(sum(ns), H, D, generator=torch.Generator().manual_seed(3)).to(BF)
+    qo = torch.tensor([0] + list(np.cumsum(ns)), dtype=torch.int32)
+    oracle = fr.batch_prefill_paged(q, cache, qo, indices, indptr, last, H, KH, D, causal=True)
+    ref64, bnd = dense_attention_f64(q, cache, qo, indices, indptr, last, H, KH, D, causal=True)
+    out = torch.full((sum(ns) + 2, H, D), 7.0, dtype=BF, device=DEV)          # 2 guard rows
+    ops.paged_attention(q.to(DEV), cache.to(DEV), qo.to(DEV), indices.to(DEV), indptr.to(DEV), last.to(DEV), max(ns), max_pages,
+                        ops.AttnWorkspace(DEV), causal=True, out=out[:sum(ns)])
+    assert bool((out[sum(ns):] == 7).all())
+    check_attention(name, out[:sum(ns)], oracle, ref64, bnd)
+
+
 @pytest.mark.parametrize("name,H,KH,D,ns,lens,fp8", [
     ("verify-ragged-rows", 8, 2, 128, [3, 4, 1], [300, 257, 64], False),
     ("prefill-ragged-rows", 8, 2, 128, [100, 128, 0, 17], [384, 300, 50, 17], False),
