@@ -78,16 +78,18 @@ __global__ __launch_bounds__(NT, 2) void latent_prefill_kernel(const LatentParam
     const int b = pair / p.H, h = pair % p.H;
     const int q0 = p.qo_indptr[b], n_b = p.qo_indptr[b + 1] - q0;
     if (qg * kLatentPrefillRows >= n_b) return;                   // whole workgroup
-    // groups end with the last row: rows that fill none are the first ones, with the shortest contexts
-    const int g0 = qg * kLatentPrefillRows - (kLatentPrefillRows - 1 - (n_b - 1) % kLatentPrefillRows);
+    // In more than a round of the chip groups end with the last row: rows that fill none are the first ones, with the shortest contexts (16 x
+    // 868 rows, 8 heads of 256 / 256 202 us, 234 otherwise).  One round waits for the group with the longest context, and the last one may
+    // have few rows: groups begin with the first row (872 rows behind 100, 8 heads of 96 / 64 40 us, 44 otherwise)
+    const int g0 = qg * kLatentPrefillRows - (gridDim.x > 256 ? kLatentPrefillRows - 1 - (n_b - 1) % kLatentPrefillRows : 0);
     const int pos_b = p.pos0[b], pg0 = p.page_indptr[b], cap = (p.page_indptr[b + 1] - pg0) * p.page_size;
     const int c0 = p.ctx_indptr[b], ctx = min(p.ctx_indptr[b + 1] - c0, cap);
-    const int wg_last = min(pos_b + g0 + kLatentPrefillRows - 1, ctx - 1);
+    const int wg_last = min(pos_b + min(g0 + kLatentPrefillRows, n_b) - 1, ctx - 1);
     if (wg_last < 0) return;
     const int w0 = g0 + wave * 32, qi = w0 + j;                     // the wave's first row, this lane's row
-    const bool valid = qi >= 0;
+    const bool valid = qi >= 0 && qi < n_b;
     const int pos = pos_b + qi, lim = valid ? min(pos, ctx - 1) : 0;
-    const int lim_lo = min(pos_b + max(w0, 0), ctx - 1), my_last = w0 > -32 ? min(pos_b + w0 + 31, ctx - 1) : -1;
+    const int lim_lo = min(pos_b + max(w0, 0), ctx - 1), my_last = w0 > -32 && w0 < n_b ? min(pos_b + min(w0 + 32, n_b) - 1, ctx - 1) : -1;
     const int t1 = wg_last / KT, my1 = my_last >= 0 ? my_last / KT : -1;
     const int dq = p.dim + p.rot_dim;
     const float sl2 = fabsf(p.scale_log2);
@@ -140,7 +142,7 @@ __global__ __launch_bounds__(NT, 2) void latent_prefill_kernel(const LatentParam
 #pragma unroll
     for (int i = 0; i < CK / 2; ++i) {
         const int c = i * 64 + lane, r = c / CK, d = lds_place<CK>(c % CK, r) * 8;
-        const bf16_t* src = reinterpret_cast<const bf16_t*>(p.q) + ((int64_t)(q0 + max(w0 + r, 0)) * p.H + h) * dq + d;
+        const bf16_t* src = reinterpret_cast<const bf16_t*>(p.q) + ((int64_t)(q0 + min(max(w0 + r, 0), n_b - 1)) * p.H + h) * dq + d;
         dma16(d < dq ? src : reinterpret_cast<const bf16_t*>(&kZeros), query_at<DV>() + wave * 32 * DK * 2 + i * 1024);
     }
     bf16x8 qf[KS];
@@ -276,7 +278,7 @@ __global__ __launch_bounds__(NT, 2) void latent_prefill_kernel(const LatentParam
     for (int i = 0; i < CV / 2; ++i) {
         const int c = i * 64 + lane, r = c / CV, ch = c % CV;
         const bf16x8 v = lds_read_b128(mine + r * DV * 2 + lds_place<CV>(ch, r) * 16);
-        if (w0 + r >= 0 && ch * 8 < p.vdim)
+        if (w0 + r >= 0 && w0 + r < n_b && ch * 8 < p.vdim)
             *reinterpret_cast<bf16x8_a8*>(reinterpret_cast<bf16_t*>(p.out) + (q0 + w0 + r) * p.ldo + h * p.vdim + ch * 8) = v;
     }
 }

@@ -272,6 +272,23 @@ def test_prompts_of_more_than_64_pages(ops, D, VD):  # noqa: F811
         assert float((got.double() - refs[0][0][at:at + k]).abs().max()) < 3e-2 * max(1.0, float(refs[0][0].abs().max())), at
 
 
+@pytest.mark.parametrize("H,lens", [(32, [300, 257, 256, 1]), (32, [300, 257, 256, 1, 505]), (130, [511])])
+def test_groups_of_a_round_of_the_chip_and_more(ops, H, lens):  # noqa: F811
+    """256 and 320 workgroups of 256 rows (and 272 of one request): which rows a group begins with changes between them.  Prompts, and
+    their last rows behind the others."""
+    spec, zs, qs, gates, refs, _ = attention_case(ops, H, 16, 8, 24, 32, 64, 21, BF, lens)
+    for first in ([0] * len(lens), [n // 3 for n in lens]):
+        s = Seqs(ops, spec, BF, lens, seed=2)
+        if any(first):
+            who = [b for b, k in enumerate(first) if k]
+            s.attend(torch.cat([zs[b][:first[b]] for b in who]), torch.cat([qs[b][:first[b]] for b in who]), who, [0] * len(who), [first[b] for b in who])
+        n = [v - k for v, k in zip(lens, first)]
+        got, _ = s.attend(torch.cat([z[k:] for z, k in zip(zs, first)]), torch.cat([q[k:] for q, k in zip(qs, first)]), range(len(lens)), first, n,
+                          torch.cat([t[k:] for t, k in zip(gates, first)]), "expanded")
+        want = torch.cat([r[1][k:] for r, k in zip(refs, first)])
+        assert float((got.double() - want).abs().max()) < 3e-2 * max(1.0, float(want.abs().max())), first
+
+
 def test_scores_of_any_size(ops):  # noqa: F811
     """Large, tiny and negated scores: the running maximum moves by hundreds, or not at all."""
     for score in (0.01, 90.0, 400.0, -20.0):
