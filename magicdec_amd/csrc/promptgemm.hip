@@ -9,8 +9,8 @@
 // What bounds it.  A full chip of matrix instructions is bound by power: the clock falls to about 1.75 of 2.4 GHz, and time is energy as much
 // as it is stalls.  v_mfma_f32_16x16x32 moves half the accumulator bytes per flop of 32x32x16 and is the faster one by clock, although its
 // 16 cycles hide less behind each (8192^3: 88 % of the cycles with the large one took as long as 82 % with the small one).  Measured, us:
-// (8192, 4096, 4096) 180, library 184; (8192, 4096, 14336) 612 / 604; (8192, 28672, 4096) with SiLU * mul 1 291 / 1 402;
-// (8196, 4096, 18432) 1 031 / 1 303; (6144, 2048, 8192) 135 / 152; (2081, 37888, 3584) 432 / 556.
+// (8192, 4096, 4096) 180, library 184; (8192, 4096, 14336) 612 / 604; (8192, 28672, 4096) with SiLU * mul 1 299 / 1 391;
+// (8196, 4096, 18432) 972 / 1 311; (6144, 2048, 8192) 135 / 152; (2081, 37888, 3584) 433 / 552.
 //   * four wavefronts of 256 rows x 64 columns, one per SIMD with 256 accumulators: each reads all of A from LDS and its own columns of W
 //     straight from memory, already in the instruction's order (W through LDS as well would need 2 048 of the 2 048 cycles that a step of
 //     64 takes there; 128 x 128 tiles per wavefront load W twice, which the address unit does not keep up with);
@@ -54,19 +54,40 @@ __device__ __forceinline__ unsigned int pack2(float a, float b) {
     return *reinterpret_cast<const unsigned int*>(&v);
 }
 __device__ __forceinline__ float round_bf16(float a) { return bf16_to_f32(f32_to_bf16(a)); }
-// 1 / (1 + e^-z) on the transcendental unit (1 ulp each; the results are rounded to 16 bits)
-__device__ __forceinline__ float sigmoid_fast(float z) {
-    return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z * -1.4426950408889634f));
+// Activations of a tile's values, without a branch and in few instructions, since no product runs beside them.  Against 64-bit arithmetic
+// they are as exact as what the other kernels call (expf and a division, expm1f): largest relative errors 1.3e-7 of SiLU (the same over
+// all bf16 numbers), 1.6e-7 of GELU around 0, where those have 1.6e-7, 1.0e-7 of xIELU (alpha 0.85 and 1.1) for 1.6e-7.
+// 8192 x 28 672 x 4096 with SiLU * mul 1 327 us, 1 351 with the calls; 8192 x 16 384 x 2048 388 and 406; 16 384 x 14 336 x 4096 with
+// xIELU 1 363 and 1 388.  (The hardware's exponential and reciprocal alone: 1 303, 372 and 1 310, but up to 3e-6, and 0 where a sigmoid is
+// no normal number; 2^x - 1 - n of a small negative n: 5e-5.)
+// z / (1 + e), as exact as a division: of a 16th of both, since the reciprocal of 1 + e (up to 2^128) may be no normal number
+__device__ __forceinline__ float over_one_plus(float z, float e) {
+    const float d = fmaf(e, 0.0625f, 0.0625f), n = z * 0.0625f, r = __builtin_amdgcn_rcpf(d), q = n * r;
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-q, d, n), r, q), d, n);        // (infinities, NaN)
 }
-
-// gelu_tanh on the transcendental unit
-__device__ __forceinline__ float gelu_fast(float z) { return z * sigmoid_fast(1.5957691216057308f * fmaf(0.044715f * z * z, z, z)); }
-// Xielu on it, without branches (a NaN goes through z / 2).  e^n - 1 - n is its series where the difference would cancel: |n| < 2^-8, where
-// the next term is 1e-8.  16 384 x 14 336 x 4 096: 1 433 us with a branch per value, 1 316 so
-__device__ __forceinline__ float xielu_fast(float ap, float an, float z) {
-    const float n = fminf(z, 0.f), p = fmaxf(z, 0.f);
-    const float far = __builtin_amdgcn_exp2f(n * 1.4426950408889634f) - 1.0f - n, near = 0.5f * n * n;
-    return fmaf(ap * p, p, fmaf(an, n > -0.00390625f ? near : far, 0.5f * z));
+// z / (1 + e^-z) of a bf16 number, whose product with 15 bits of log2(e) is exact
+__device__ __forceinline__ float silu_flat(float z) {
+    const float x = __builtin_amdgcn_fmed3f(z, -100.f, 100.f), t = x * -0x1.7154p+0f, k = rintf(t);
+    return over_one_plus(z, __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(fmaf(x, -7.05260771340736e-06f, t - k)), (int)k));
+}
+// gelu_tanh: e^(-2 sqrt(2/pi) u) = 2^(-K u), K in two parts, the product's rounding added behind
+__device__ __forceinline__ float gelu_flat(float z) {
+    constexpr float kHi = -0x1.26aec2p+1f, kLo = -1.2948402037571394e-08f;
+    const float u = __builtin_amdgcn_fmed3f(fmaf(0.044715f * z * z, z, z), -120.f, 120.f);
+    const float t = u * kHi, rest = fmaf(u, kLo, fmaf(u, kHi, -t)), e = __builtin_amdgcn_exp2f(t);
+    return over_one_plus(z, fmaf(fminf(e, 0x1.fffffep+127f), rest * 0.693147181f, e));
+}
+// Xielu.  e^n - 1 = 2^k (e^f - 1) + (2^k - 1) with n = k ln 2 + f, |f| < 0.35 (Cody and Waite), e^f - 1 from its series
+__device__ __forceinline__ float xielu_flat(float ap, float an, float z) {
+    const float n = fmaxf(fminf(z, 0.f), -104.f), k = rintf(n * 1.44269504f), f = fmaf(k, -1.42860682e-06f, fmaf(k, -0x1.62e4p-1f, n));
+    float s = fmaf(f, 1.f / 5040, 1.f / 720);
+    s = fmaf(s, f, 1.f / 120);
+    s = fmaf(s, f, 1.f / 24);
+    s = fmaf(s, f, 1.f / 6);
+    s = fmaf(s, f, 0.5f);
+    const float scale = __builtin_amdgcn_ldexpf(1.0f, (int)k), em1 = fmaf(scale, fmaf(f * f, s, f), scale - 1.0f);
+    const float half = 0.5f * z;
+    return z > 0.f ? fmaf(ap * z, z, half) : fmaf(an, em1 - z, half);
 }
 // f(0), f(1), ...: what a loop of this length is not always unrolled to
 template <int... I, class F>
@@ -284,11 +305,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                 for (int r = 0; r < 4; ++r) {
                     if constexpr (EPI == PE_SWIGLU) {
                         const float h1 = round_bf16(z[r]), h3 = round_bf16(g[r]);
-                        o[r] = round_bf16(h1 * sigmoid_fast(h1)) * h3;
+                        o[r] = round_bf16(silu_flat(h1)) * h3;
                     } else if constexpr (EPI == PE_GEGLU) {
-                        o[r] = gelu_fast(z[r]) * g[r];
+                        o[r] = gelu_flat(z[r]) * g[r];
                     } else if constexpr (EPI == PE_XIELU) {
-                        o[r] = xielu_fast(act_p, act_n, z[r]);
+                        o[r] = xielu_flat(act_p, act_n, z[r]);
                     } else if constexpr (EPI == PE_BIAS) {
                         o[r] = z[r] + bf16_to_f32(p.bias[min((n0 * 4 + wave) * CW + n * 16 + kq * 4 + r, p.Nout - 1)]);
                     } else {

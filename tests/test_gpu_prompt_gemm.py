@@ -1,4 +1,6 @@
 """md_linear_prompt (csrc/promptgemm.hip) against float64 products, at the edges of its tiles.  On the GPU (-m gpu)."""
+import math
+
 import pytest
 import torch
 
@@ -68,6 +70,52 @@ def test_activations(M, N, K):
         got = ops.linear_prompt(x, gated, swiglu=True, gelu=True, tile=tile).double()
         bound = 1.13 * 2 * o1 * h3.abs() + gelu.abs() * 2 * o3 + U * (gelu * h3).abs() + 2.0 ** -20 * (1 + h1.abs()) * h3.abs()
         assert ((got - gelu * h3).abs() <= bound).all()
+
+
+def test_silu_of_every_number_is_a_steps():
+    """SiLU of all finite bf16 numbers (a product with the identity) has the bits of the kernel beside the library's products."""
+    from magicdec_amd import ops
+    h1 = torch.arange(65536, dtype=torch.int32, device=DEV).to(torch.int16).view(torch.bfloat16).view(256, 256)
+    h1 = torch.where(h1.abs() < 3e38, h1, 0)
+    h1 = torch.where(h1.abs() > 1e-36, h1, 0)                                 # (no products that are not normal numbers)
+    eye = torch.eye(256, device=DEV).bfloat16()
+    for big in (1.0, 2.0 ** 100):                                             # ... of h1 from -88.5 on the SiLU is 1e-37
+        h3 = torch.full_like(h1, big)
+        want = ops.silu_mul(h1.t().contiguous(), h3)
+        got = ops.linear_prompt(eye, ops.PackedWeight(torch.cat([h1, h3]), swiglu=True), swiglu=True)
+        assert torch.equal(got, want)
+        assert (want[(h1.t() >= -88.5) & (h1.t() < -87.4)] < -1e-37).all()
+
+
+def test_activations_are_as_exact_as_a_steps():
+    """xIELU and GELU of 32-bit sums, almost all of them the float64 value rounded once: a relative error e rounds the other way in a share
+    e / 2^-9 at most.  xIELU has 1e-7 of its terms, GELU 2e-7 (behind -0.5 3e-6 and behind -2 1.3e-5, of its exponent); GELU twice that."""
+    from magicdec_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(11)
+    rows = torch.zeros(128, 256, device=DEV).bfloat16()
+    rows[torch.arange(128), torch.arange(128) * 2] = rows[torch.arange(128), torch.arange(128) * 2 + 1] = 1
+    N = 4096
+    for lo, hi in ((-0.02, -0.0039), (-0.0039, -1e-3), (-0.1, -0.02), (-2.0, -0.1), (-9.9, -2.0), (0.01, 6.0)):
+        grid = 2.0 ** (math.ceil(math.log2(max(-lo, hi))) - 16)               # of 16 bits: a sum of two numbers
+        z = ((torch.rand(N, 128, device=DEV, generator=g) * (hi - lo) + lo) / grid).round() * grid
+        top = z.bfloat16()
+        low = (z - top.float()).bfloat16()
+        w = torch.stack([top, low], 2).flatten(1)
+        assert torch.equal(top.double() + low.double(), z.double())
+        z = z.double().t()
+        for av, bv in ((0.3, -0.2), (5.0, 5.0)):
+            act = torch.tensor([av, bv], device=DEV)
+            a, b = torch.nn.functional.softplus(act.double())
+            want = z / 2 + torch.where(z > 0, a * z * z, (0.5 + b) * (torch.expm1(z.clamp(max=0)) - z))
+            # (its terms may cancel: as much more as they are larger than their sum)
+            share = 1e-7 * 512 * float((((0.5 + b) * z.clamp(max=0).abs() + z.abs() + a * z.clamp(min=0) ** 2) / want.abs().clamp(min=1e-4)).mean())
+            got = ops.linear_prompt(rows, ops.PackedWeight(w), xielu=act)
+            assert float((got != want.bfloat16()).float().mean()) <= share, (lo, av, share)
+        ones = torch.zeros(N, 256, device=DEV).bfloat16()
+        ones[:, ::2] = 1
+        got = ops.linear_prompt(rows, ops.PackedWeight(torch.cat([w, ones]), swiglu=True), swiglu=True, gelu=True)
+        want = z * torch.sigmoid(2 * math.sqrt(2 / math.pi) * (z + 0.044715 * z ** 3))
+        assert float((got != want.bfloat16()).float().mean()) <= 2 * 512 * (1.3e-5 if lo < -2 else 3e-6 if lo < -0.5 else 2e-7), lo
 
 
 def test_not_finite():
