@@ -485,19 +485,22 @@ def prompt_over_block(M: int, N: int, K: int, swiglu: bool = False) -> bool:
 
 
 @functools.lru_cache(maxsize=4096)
-def prompt_rows(M: int, N: int, K: int, swiglu: bool = False) -> int:
+def prompt_rows(M: int, N: int, K: int, swiglu: bool = False, rows_stay: bool = False) -> int:
     """How many of a prompt's M rows (more than a step has; weight in the streaming layout) go to md_linear_prompt in one call: none (the
     library), all, or whole row tiles with fewer than 129 left for md_linear.
     Against the library, 435 random products of 257 to 16 384 rows: 0.77 of its time with the activation behind it, 0.61 with the weight's
     rows brought back in front; 1.11 at the worst (12 719 x 2 048 x 8 192, 341 us).  Its workgroups take all of K, so that a few hundred
     rows of a narrow and deep product leave most CUs idle: 374 x 2 048 x 10 240 in 58 us where the library's split of K takes 41, or 61
-    with the rows to bring back; the line is where those cross over the same products.
+    with the rows to bring back; the line is where those cross over the same products.  rows_stay: the weight is one whose row-major
+    tensor is never released (a pool's, or one that steps of more than 256 rows read), so that the library has nothing to bring back; over
+    330 products of 257 to 2 600 rows the two cross at 1.45 times the ideal (1.10 of the library's time at the worst; beyond it 449 x
+    2 048 x 5 632 in 38 us for 27, 301 x 4 096 x 14 336 in 91 for 74).
     Rows just behind whole rounds of tiles are a round more: 8 196 x 4 096 x 18 432 in 950 us, 8 192 in 760 and the other four in 40 on the
     weight-streaming kernel, whose time the last line bounds from above (49 / 55 us for 28 672 x 4 096 at 64 / 128 rows, 16 / 21 for 4 096
     x 4 096, 54 / 64 for 5 120 x 27 648)."""
     from .. import ops
     us = ops.linear_prompt_us(M, N, K, swiglu) if _MODE != "lib" and M > 256 else -1.0
-    if us < 0 or us > 2.4 * (2e-6 * M * N / 1400 * K + 12):
+    if us < 0 or us > (1.45 if rows_stay else 2.4) * (2e-6 * M * N / 1400 * K + 12):
         return 0
     rest = M % 256
     if 0 < rest <= 128 and M - rest > 256 and ops.linear_supported(rest, N, K, swiglu):

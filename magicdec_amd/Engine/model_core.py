@@ -402,6 +402,8 @@ class Transformer(nn.Module):
             self._packed[id(w)] = pw
         self._released = set()          # ids of weights whose row-major tensor is currently released (release_rowmajor)
         self._by_id = {id(w): w for w, _ in todo}
+        for w in self._by_id.values():   # (by the shapes and the engine's row counts: the same on the ranks of a group, before every prompt)
+            self._packed[id(w)].rows_stay = self._rowmajor_in_decode(w)
 
     @property
     def packed_bytes(self):
@@ -630,16 +632,18 @@ class Transformer(nn.Module):
     @staticmethod
     def _on_prompt_gemm(x2d, w, pk, swiglu=False, block=False):
         """Do these rows run on md_linear_prompt: more than a step has, or (block) a step's in the place of md_linear_block?  It reads the
-        streaming layout: no row-major weight has to come back.  The shapes alone decide, so that the ranks of a group agree."""
+        streaming layout: no released row-major weight has to come back.  The shapes decide, and whether the weight is one that is released
+        at all, so that the ranks of a group agree."""
         M, K = x2d.shape
         return (M > 128 and pk is not None and w.dtype == torch.bfloat16 and x2d.dtype == torch.bfloat16 and x2d.stride(1) == 1
                 and x2d.stride(0) % 8 == 0 and x2d.stride(0) < 1 << 20 and x2d.data_ptr() % 16 == 0
-                and (prompt_rows(M, w.shape[0], K, swiglu) > 0 if M > 256 else block and prompt_over_block(M, w.shape[0], K, swiglu)))
+                and (prompt_rows(M, w.shape[0], K, swiglu, pk.rows_stay) > 0 if M > 256
+                     else block and prompt_over_block(M, w.shape[0], K, swiglu)))
 
     def _prompt_linear(self, x2d, pk, bias=None, swiglu=False, out=None, **act):
         """A linear of a prompt's rows: whole row tiles on md_linear_prompt, a few rows behind them on the weight-streaming kernel."""
         M, K = x2d.shape
-        rows = prompt_rows(M, pk.N, K, swiglu) if M > 256 else M
+        rows = prompt_rows(M, pk.N, K, swiglu, pk.rows_stay) if M > 256 else M
         if rows == M:
             return ops.linear_prompt(x2d, pk, bias, swiglu, out=out, **act)
         if out is None:

@@ -300,7 +300,9 @@ class PackedWeight:
     """A linear's weight in the streaming layout of md_linear (include/magicdec_hip.h: w_packed = 1):
     [ceil(N/32)][K/16][64 lanes][8] -- element (t, s, lane, e) = W[32t + lane%32][16s + 8*(lane/32) + e], rows past N
     zero; for swiglu=True tile t = rows 16t..16t+15 of w1 then rows 16t..16t+15 of w3 (weight = [w1; w3], N = 2I).
-    Built once at load time (a torch permute: plumbing); bf16 or int8."""
+    Built once at load time (a torch permute: plumbing); bf16 or int8.  rows_stay: the row-major tensor beside it is never released
+    (Transformer._pack_weights)."""
+    rows_stay = False
 
     def __init__(self, weight, swiglu=False):
         N, K = weight.shape

@@ -1672,3 +1672,29 @@ def test_weights_come_back_on_demand():
     assert m._released == released and m.released_bytes == size() > 0
     m.restore_rowmajor()
     assert m.released_bytes == 0
+
+
+def test_products_of_more_rows_than_a_step_has_know_whether_the_weight_is_there():
+    """A weight whose row-major tensor is never released (a pool's, or one that a step hands to the library) stays in the library where that
+    is the faster one without bringing rows back; one that is released runs on the streaming copy further down."""
+    from types import SimpleNamespace
+    from magicdec_amd import ops
+    from magicdec_amd.Engine import gemm_policy, model_core
+    for M, N, K in ((384, 4096, 14336), (449, 2048, 5632), (572, 2048, 8192)):
+        assert gemm_policy.prompt_rows(M, N, K) == M and gemm_policy.prompt_rows(M, N, K, rows_stay=True) == 0
+    for M, N, K, gated in ((384, 28672, 4096, True), (8192, 4096, 14336, False), (2048, 2048, 8192, False), (512, 6144, 4096, False)):
+        assert gemm_policy.prompt_rows(M, N, K, gated, rows_stay=True) == gemm_policy.prompt_rows(M, N, K, gated) > 0
+    name = "rows-stay"
+    model_core.transformer_configs[name] = dict(block_size=256, n_layer=1, vocab_size=512, n_head=16, n_local_heads=4, dim=2048, intermediate_size=8192)
+    try:
+        m = model_core.Transformer.from_name(name).to(torch.bfloat16)
+    finally:
+        model_core.transformer_configs.pop(name, None)
+    x = torch.zeros(572, 8192, dtype=torch.bfloat16)
+    for rows, stay in (((4,), False), (None, True)):
+        m.setup_caches(num_pages=2, decode_rows=rows)
+        m._pack_weights(force=True)
+        w2 = m.layers[0].feed_forward.w2.weight
+        pk = m._packed[id(w2)]
+        assert pk.rows_stay == m._rowmajor_in_decode(w2) == stay
+        assert m._on_prompt_gemm(x, w2, pk) == (not stay)
