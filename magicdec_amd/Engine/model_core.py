@@ -478,7 +478,8 @@ class Transformer(nn.Module):
         if self._packed.get(id(w)) is None or w.dtype == torch.int8 or self.decode_rows is None:
             return True
         N, K = w.shape
-        return any(M > 256 or "lib" in self._decode_hows(role, N, K, False, M) for M in self.decode_rows)
+        return any(prompt_rows(M, N, K, role in ("w13", "gated"), True) == 0 if M > 256 else "lib" in self._decode_hows(role, N, K, False, M)
+                   for M in self.decode_rows)
 
     def release_rowmajor(self):
         """After prefill: free the row-major tensor of every weight that decode only ever reads in the streaming layout (16.9 GB of an
@@ -653,8 +654,9 @@ class Transformer(nn.Module):
         return out
 
     def _linear_how(self, M, N, K, swiglu, int8, pk, kind, has_pro):
-        """Which implementation `_linear` ends up on for this shape: "fused" | "block" | "skinny" | "lib" -- the same
-        sequence of policy and shape-support checks, without running anything (release_rowmajor's prediction)."""
+        """Which implementation `_linear` ends up on for at most 256 rows of this shape: "fused" | "block" | "skinny" | "lib" -- the same
+        sequence of policy and shape-support checks, without running anything (release_rowmajor's prediction; "block" may be
+        md_linear_prompt in its place, which reads the same copy).  More rows: prompt_rows."""
         from .gemm_policy import choose
         how = choose(M, N, K, swiglu, int8, pk is not None, kind, has_pro and swiglu)
         if how == "fused" and ops.fused_linear_supported(M, N, K):

@@ -322,8 +322,13 @@ class LayeredTransformer(Transformer):
         return super()._wants_packed(role, w)
 
     def _rowmajor_in_decode(self, w):
-        # (a tied head is the embedding table: its rows are gathered in every step; the heads' matrices are views of wukv)
-        return ((self.spec.tied_head and w is self.output.weight) or self._roles[id(w)][0] == "wukv" or super()._rowmajor_in_decode(w))
+        # (a tied head is the embedding table: its rows are gathered in every step; the heads' matrices are views of wukv; beside heads
+        # of an odd width the gated product has nowhere aligned to write to)
+        if self.spec.tied_head and w is self.output.weight:
+            return True
+        role, i = self._roles[id(w)]
+        odd = role == "gated" and (self.layers[i].heads_out % 8 or self.layers[i].wout.weight.shape[1] % 8)
+        return role == "wukv" or bool(odd) or super()._rowmajor_in_decode(w)
 
     # ------------------------------------------------------------------ the step
     def _linear(self, x2d, lin, **kw):

@@ -202,3 +202,25 @@ def test_a_steps_rows_in_the_place_of_the_block_kernel(M, N, K, swiglu, taken, m
     else:
         want = ref + bias.double()
         assert ((out.double() - want).abs() <= want.abs() * U + 2 * off + 2.0 ** -23 * bias.double().abs()).all()
+
+
+def test_a_step_of_more_than_256_rows_reads_one_copy_of_its_weights(monkeypatch):
+    """After a prompt the weights that such steps multiply on md_linear_prompt have their streaming copy only, and the step asks for no
+    other: the logits have the bits of an engine that keeps both."""
+    from pathlib import Path
+    from magicdec_amd.Engine import model_core
+    from magicdec_amd.Engine.SnapKV.backend import LMBackend
+    monkeypatch.setitem(model_core.transformer_configs, "one-copy", dict(block_size=512, n_layer=2, vocab_size=4096, n_head=16, n_local_heads=4, dim=2048,
+                                                                         intermediate_size=8192))
+    B, n, got = 65, 6, []
+    ids = torch.randint(0, 4096, (B, 140), generator=torch.Generator().manual_seed(0)).to(DEV)
+    for keep in ("0", "1"):
+        monkeypatch.setenv("MAGICDEC_KEEP_ROWMAJOR", keep)
+        e = LMBackend(dtype=torch.bfloat16, device=DEV, dec_len=n)
+        torch.manual_seed(1)
+        e.load_model(Path("no-checkpoint/one-copy/model.pth"), use_tp=False)
+        e.setup_caches(max_batch_size=B, max_seq_length=256)
+        e.encode(ids)
+        e.inference(ids[:, :n])
+        got.append((e.model._last_logits.clone(), getattr(e.model, "_warned_transient", False), len(e.model._released)))
+    assert torch.equal(got[0][0], got[1][0]) and not got[0][1] and got[0][2] > 0 == got[1][2]

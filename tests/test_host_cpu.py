@@ -1698,3 +1698,28 @@ def test_products_of_more_rows_than_a_step_has_know_whether_the_weight_is_there(
         pk = m._packed[id(w2)]
         assert pk.rows_stay == m._rowmajor_in_decode(w2) == stay
         assert m._on_prompt_gemm(x, w2, pk) == (not stay)
+
+
+def test_steps_of_more_than_256_rows_leave_no_weight_in_two_layouts_for_nothing():
+    """Their products that run on the streaming copy need no row-major tensor: it is released after the prompt, and the step does not ask
+    for it; the deep one that such a step hands to the library stays."""
+    from magicdec_amd.Engine import gemm_policy, model_core
+    name = "wide-steps"
+    model_core.transformer_configs[name] = dict(block_size=256, n_layer=1, vocab_size=1024, n_head=16, n_local_heads=4, dim=2048, intermediate_size=8192)
+    try:
+        m = model_core.Transformer.from_name(name).to(torch.bfloat16)
+    finally:
+        model_core.transformer_configs.pop(name, None)
+    m.setup_caches(num_pages=2, decode_rows=(64, 384))
+    m._pack_weights(force=True)
+    layer = m.layers[0]
+    w13, w2 = m._w13[0], layer.feed_forward.w2.weight
+    assert gemm_policy.prompt_rows(384, *w13.shape, True, True) == 384 and gemm_policy.prompt_rows(384, *w2.shape, False, True) == 0
+    m.release_rowmajor()
+    assert id(w13) in m._released and id(w2) not in m._released and id(w2) in m._packed
+    for k, w in m._by_id.items():
+        role = m._roles[k][0]
+        x = torch.zeros(384, w.shape[1], dtype=torch.bfloat16)
+        own = m._on_prompt_gemm(x, w, m._packed[k], role == "w13")
+        assert own or k not in m._released, role                               # a released one is never asked for
+        assert not own or "lib" in m._decode_hows(role, *w.shape, False, 64) or k in m._released, role
