@@ -367,14 +367,17 @@ class Transformer(nn.Module):
         # and are made AFTER the KV slabs exist; if they do not fit beside them with a margin for the step's workspaces,
         # serve everything from the row-major tensors (library GEMMs / row-major md_linear) instead of failing later.
         # MAGICDEC_PACKED_COPIES=0 switches them off outright (Engine/gemm_policy.py).
-        need = sum(w.numel() * w.element_size() for w, _ in todo)
+        # Copies that only prompts read come second: without room for them too the steps still have theirs.
+        size = lambda what: sum(w.numel() * w.element_size() for w, _ in what)
+        steps = [t for t in todo if not self._only_for_prompts(self._roles[id(t[0])][0])]
+        need, every = size(steps), size(todo)
         try:
             torch.cuda.empty_cache()       # mem_get_info does not see blocks the caching allocator holds but no longer uses
             free = torch.cuda.mem_get_info(self.output.weight.device)[0]
         except Exception:              # not a HIP device (tests with stand-in ops): nothing to check
             free = None
         margin = 6 << 30
-        fits = free is None or need + margin <= free
+        fits = 2 if free is None else (need + margin <= free) + (every + margin <= free)
         # ONE decision for all ranks that must run the same kernels: the ranks of a TP group -- and the
         # ranks running a REPLICATED draft, which stay in lock-step only because they compute bit-identical tokens -- must
         # not choose per rank from their own free memory: a rank that falls back to the library GEMMs rounds differently,
@@ -384,19 +387,20 @@ class Transformer(nn.Module):
         if grp is not None:
             import torch.distributed as dist
             if dist.is_available() and dist.is_initialized():
-                t = torch.tensor([1 if fits else 0], dtype=torch.int32,
+                t = torch.tensor([fits], dtype=torch.int32,
                                  device=self.output.weight.device if dist.get_backend(grp) == "nccl" else "cpu")
                 dist.all_reduce(t, op=dist.ReduceOp.MIN, group=grp)
                 if fits and int(t.item()) == 0:
                     print("[magicdec_amd] streaming-layout weight copies fit on this rank but not on every rank of its "
                           "group: not made anywhere (all ranks must run the same kernels)")
-                fits = bool(int(t.item()))
+                fits = int(t.item())
         if not fits:
             if free is not None and need + margin > free:
                 print(f"[magicdec_amd] streaming-layout weight copies need {need / 2**30:.1f} GiB but only {free / 2**30:.1f} GiB "
                       f"are free beside the KV cache (margin {margin >> 30} GiB): not made -- the decode / verify linears run on "
                       f"the row-major weights (slower); shrink the cache or set MAGICDEC_PACKED_COPIES=0 to silence this")
             return
+        todo = todo if fits == 2 else steps
         for w, sw in todo:
             pw = ops.PackedWeight(w.data if isinstance(w, nn.Parameter) else w, swiglu=sw)
             self._packed[id(w)] = pw
@@ -459,6 +463,10 @@ class Transformer(nn.Module):
                 if how in ("skinny", "block") and ops.linear_add_rmsnorm_supported(M, N, K):
                     return {"skinny"}
         return {self._linear_how(M, N, K, False, int8, pk, "plain", False)}          # wo / w2 fall-through, lm head
+
+    def _only_for_prompts(self, role):
+        """Is a copy of this weight read by prompts only?"""
+        return False
 
     def _wants_packed(self, role, w):
         """A streaming-layout copy of this weight?  With known decode row counts: iff some step of this engine runs it on a

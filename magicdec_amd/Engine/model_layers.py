@@ -315,9 +315,12 @@ class LayeredTransformer(Transformer):
             return {self._linear_how(M, N, K, True, int8, True if packed else None, "swiglu", False)}
         return {self._linear_how(M, N, K, False, int8, True if packed else None, "plain", False)}
 
-    def _wants_packed(self, role, w):
+    def _only_for_prompts(self, role):
         # (wukv expands a prompt's latent rows; a step reads it as the heads' matrices of the absorbed form)
-        if role == "wukv":
+        return role == "wukv"
+
+    def _wants_packed(self, role, w):
+        if self._only_for_prompts(role):
             return want_packed_prompt(*w.shape)
         return super()._wants_packed(role, w)
 

@@ -107,6 +107,38 @@ def test_the_product_in_fills_whole_tiles_of_columns(latent_ops, model):
         assert w.shape[0] % 32 == 0 and n <= w.shape[0] < n + 32 and not w[n:].any() and bool(w[:n].any(1).all())
 
 
+def test_copies_for_prompts_come_behind_those_for_steps(latent_ops, tmp_path, monkeypatch):
+    """A card that holds the streaming copies that steps read, but not wukv's beside them, keeps the former; one rank of a group without
+    room for wukv's is enough for none to make them."""
+    from types import SimpleNamespace
+    cfg = lu.config([lu.layer(2, heads=16, dim=48, rot_dim=64, vdim=64, q_rank=384, kv_rank=512, ff=512, yarn=lu.YARN)], vocab=512, width=512)
+    lu.make(tmp_path / "m", cfg, 3)
+    from magicdec_amd.Engine.SnapKV.backend import LMBackend
+    e = LMBackend(dtype=torch.bfloat16, device="cpu")
+    e.load_model(tmp_path / "m", use_tp=False)
+    e.setup_caches(max_batch_size=1, max_seq_length=300)
+    m, free = e.model, [1 << 40]
+    monkeypatch.setattr(torch.cuda, "empty_cache", lambda: None)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda dev=None: (free[0], 1 << 40))
+
+    def packed(room):
+        free[0] = room + (6 << 30)
+        m._pack_weights(force=True)
+        return {m._roles[k][0] for k in m._packed}
+    every = packed(1 << 40)
+    size = lambda: sum(w.numel() * 2 for w in m._by_id.values())
+    total, wukv = size(), m.layers[0].attention.wukv.weight.numel() * 2
+    assert "wukv" in every and len(every) > 1
+    assert packed(total) == every and packed(total - 1) == every - {"wukv"} == packed(total - wukv) and packed(total - wukv - 1) == set()
+    dist = torch.distributed
+    for name, fn in (("is_initialized", lambda: True), ("get_backend", lambda g: "gloo")):
+        monkeypatch.setattr(dist, name, fn)
+    m.replica_group = SimpleNamespace()
+    for other, want in ((2, every), (1, every - {"wukv"}), (0, set())):
+        monkeypatch.setattr(dist, "all_reduce", lambda t, op, group: t.clamp_(max=other))
+        assert packed(total) == want
+
+
 @pytest.mark.parametrize("portion_rows", [6, 17, 1000])
 def test_ragged_steps_portions_and_reuse(latent_ops, model, monkeypatch, portion_rows):
     from magicdec_amd.Engine import backend_core
