@@ -48,11 +48,11 @@ __global__ __launch_bounds__(256, 2) void f32_gemm_kernel(const F32Params p) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                         : : "s"(buf * kBuf + i * 4096 + wave * 1024), "v"(xo + (unsigned)i * 128u * (unsigned)p.ldx), "s"(rx), "s"(k * 4) : "memory");
+                         : : "s"(buf * kBuf + i * 4096 + wave * 1024), "v"(xo + (unsigned)i * 128u * (unsigned)p.ldx), "s"(rx), "s"(k * 4) : "memory", "m0");
 #pragma unroll
         for (int i = 0; i < TN; ++i)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                         : : "s"(buf * kBuf + kA + i * 4096 + wave * 1024), "v"(wo + (unsigned)i * 128u * (unsigned)p.K), "s"(rw), "s"(k * 4) : "memory");
+                         : : "s"(buf * kBuf + kA + i * 4096 + wave * 1024), "v"(wo + (unsigned)i * 128u * (unsigned)p.K), "s"(rw), "s"(k * 4) : "memory", "m0");
     };
     unsigned ar[2], br[2];
 #pragma unroll

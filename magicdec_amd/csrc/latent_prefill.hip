@@ -34,7 +34,7 @@ __device__ const u32x4 kZeros = {0u, 0u, 0u, 0u};
 
 // 16 bytes a lane from `src` to LDS bytes `to` + lane * 16
 __device__ __forceinline__ void dma16(const bf16_t* src, unsigned int to) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(to), "v"(src) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(to), "v"(src) : "memory", "m0");
 }
 
 // weights -> upper 16 bits (truncated: bf16) and the rest rounded to bf16

@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // its place.  In assembly, since the compiler would have every LDS read wait for it; the waits are counted by hand (wait_a)
     auto load_a = [&](unsigned buf, int i) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                     : : "s"(buf + (unsigned)(i * 4096 + wave * 1024)), "v"(aoff[i]), "s"(ra), "s"(ka) : "memory");
+                     : : "s"(buf + (unsigned)(i * 4096 + wave * 1024)), "v"(aoff[i]), "s"(ra), "s"(ka) : "memory", "m0");
     };
     auto load_b = [&](int e, int h, const unsigned (&base)[NT / 2], int n) {
         const u32x4 q = __builtin_amdgcn_raw_buffer_load_b128(rw, boff + h * 2048 + (n & 1) * 256, base[n >> 1], 0);

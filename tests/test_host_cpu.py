@@ -1723,3 +1723,17 @@ def test_steps_of_more_than_256_rows_leave_no_weight_in_two_layouts_for_nothing(
         own = m._on_prompt_gemm(x, w, m._packed[k], role == "w13")
         assert own or k not in m._released, role                               # a released one is never asked for
         assert not own or "lib" in m._decode_hows(role, *w.shape, False, 64) or k in m._released, role
+
+
+def test_assembly_names_the_registers_it_writes():
+    """Every inline statement that writes M0 by itself says so to the compiler."""
+    import re
+    from pathlib import Path
+    import magicdec_amd
+    seen = 0
+    for path in sorted(Path(magicdec_amd.__file__).parent.glob("csrc/*.h*")):
+        for m in re.finditer(r"\basm\b[^;]*?\((.*?)\);", path.read_text(), re.S):
+            if re.search(r"\bs_\w+ m0,", m.group(1)):
+                seen += 1
+                assert '"m0"' in m.group(1).rsplit(":", 1)[1], (path.name, m.group(0)[:80])
+    assert seen >= 4
