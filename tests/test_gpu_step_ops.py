@@ -88,3 +88,24 @@ def test_token_ids_of_either_width(kinds):
         made.append(got)
         assert e._use_graphs == graphs                       # (no fall-back to eager steps)
     assert all(torch.equal(a, b) for a, b in zip(*made))
+
+
+def test_uploads_behind_queued_work():
+    """Many uploads back to back, while the stream still has work in front of them and their host memory is used again: every value; from
+    lists, host tensors of either type, and tensors that are on the device already."""
+    from magicdec_amd import ops
+    a = torch.randn(4096, 4096, device=DEV)
+    got = []
+    for i in range(200):
+        if i % 20 == 0:
+            a = (a @ a).clamp_(-1, 1)
+        n = 1 + 37 * i % 1000
+        v = torch.arange(i, i + n, dtype=torch.long if i % 3 else torch.int32)
+        v = v.pin_memory() if i % 4 == 3 else v
+        src = v.tolist() if i % 4 == 0 else v.to(DEV) if i % 4 == 1 else v
+        dtype = torch.int32 if i % 2 else torch.long
+        got.append((i, n, dtype, ops.upload(src, dtype, DEV)))
+        if i % 4 > 1:
+            v.fill_(-1)                                        # the caller's tensor is its own again
+    for i, n, dtype, t in got:
+        assert t.dtype == dtype and t.is_cuda and torch.equal(t.cpu(), torch.arange(i, i + n, dtype=dtype)), i

@@ -1737,3 +1737,11 @@ def test_assembly_names_the_registers_it_writes():
                 seen += 1
                 assert '"m0"' in m.group(1).rsplit(":", 1)[1], (path.name, m.group(0)[:80])
     assert seen >= 4
+
+
+def test_uploaded_numbers_have_the_type_asked_for():
+    from magicdec_amd import ops
+    for v in ([3, 1, 2], torch.tensor([3, 1, 2]), torch.tensor([3, 1, 2], dtype=torch.int32), torch.tensor([3, 1, 2], dtype=torch.int16)):
+        for dtype in (torch.int32, torch.long):
+            got = ops.upload(v, dtype, "cpu")
+            assert got.dtype == dtype and got.tolist() == [3, 1, 2]
