@@ -79,6 +79,13 @@ class LatentAttention(nn.Module):
         self.wuq = nn.Linear(spec.q_rank, spec.heads * (spec.dim + spec.rot_dim), bias=False)
         self.wukv = nn.Linear(spec.kv_rank, spec.heads * (spec.dim + spec.vdim), bias=False)
         self.kv_cache = None
+        self._register_load_state_dict_pre_hook(self._load_hook)
+
+    def _load_hook(self, state_dict, prefix, *args):
+        """A state_dict whose product in ends with the parts."""
+        w = state_dict.get(prefix + "win.weight")
+        if w is not None and w.shape[0] == sum(self.cuts):
+            state_dict[prefix + "win.weight"] = F.pad(w, (0, 0, 0, -w.shape[0] % 32))
 
     def kernel_spec(self, eps, rotary) -> ops.LatentSpec:
         s = self.spec

@@ -107,6 +107,20 @@ def test_the_product_in_fills_whole_tiles_of_columns(latent_ops, model):
         assert w.shape[0] % 32 == 0 and n <= w.shape[0] < n + 32 and not w[n:].any() and bool(w[:n].any(1).all())
 
 
+@pytest.mark.parametrize("assign", [False, True])
+def test_a_state_dict_without_the_rows_of_zeros_loads(latent_ops, model, assign):
+    """One saved where the product in ended with the parts."""
+    m = engine(model[0], slots=1).model
+    whole = {k: v.clone() for k, v in m.state_dict().items()}
+    saved = {k: v[:sum(m.layers[int(k.split(".")[1])].attention.cuts)].clone() if k.endswith("win.weight") else v.clone() for k, v in whole.items()}
+    assert any(saved[k].shape != whole[k].shape for k in whole)
+    for sd in (saved, whole):
+        for p in m.parameters():
+            p.data.fill_(7.0)
+        m.load_state_dict(dict(sd), assign=assign)
+        assert all(torch.equal(v, whole[k]) for k, v in m.state_dict().items())
+
+
 def test_copies_for_prompts_come_behind_those_for_steps(latent_ops, tmp_path, monkeypatch):
     """A card that holds the streaming copies that steps read, but not wukv's beside them, keeps the former; one rank of a group without
     room for wukv's is enough for none to make them."""
