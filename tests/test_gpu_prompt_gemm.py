@@ -173,6 +173,45 @@ def test_rows_behind_whole_tiles(M, N, K, swiglu):
     assert ((out.double() - h1 * s * h3).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("M,N,K,kind", [(4112, 4096, 5120, "xielu"), (8193, 2048, 2560, "xielu"), (10241, 16384, 2048, "gelu"), (10241, 16384, 2048, "swiglu")])
+def test_activations_of_rows_behind_whole_tiles(M, N, K, kind):
+    """The same with the activations, into columns of a wider matrix: both kernels' rows against float64, nothing beside them."""
+    from types import SimpleNamespace
+    from magicdec_amd import ops
+    from magicdec_amd.Engine.gemm_policy import prompt_rows
+    from magicdec_amd.Engine.model_core import Transformer
+    gated = kind != "xielu"
+    rows = prompt_rows(M, N, K, gated)
+    assert 0 < rows < M
+    x, w, _ = case(M, N, K, M + 1)
+    act = torch.tensor([0.3, -0.2], device=DEV)
+    n_out = N // 2 if gated else N
+    wide = torch.full((M, n_out + 24), -7.0, device=DEV, dtype=torch.bfloat16)
+    kw = dict(xielu=act) if not gated else dict(gelu=True) if kind == "gelu" else {}
+    out = Transformer._prompt_linear(SimpleNamespace(workspace=ops.AttnWorkspace(DEV)), x, ops.PackedWeight(w, swiglu=gated), None, gated,
+                                     out=wide[:, 16:16 + n_out], **kw)
+    assert (wide[:, :16] == -7).all() and (wide[:, 16 + n_out:] == -7).all() and out.data_ptr() == wide[:, 16:].data_ptr()
+    for lo in range(0, M, 2048):                                              # (in parts: float64 of all rows is much)
+        part, got = x[lo:lo + 2048], out[lo:lo + 2048].double()
+        ref, off = product(part, w)
+        if kind == "xielu":
+            a, b = torch.nn.functional.softplus(act.double())
+            low = ref.clamp(max=0)
+            z = ref / 2 + torch.where(ref > 0, a * ref * ref, (0.5 + b) * (torch.expm1(low) - low))
+            slope = 0.5 + torch.where(ref > 0, 2 * a * ref, (0.5 + b) * (torch.exp(low) - 1).abs())
+            assert ((got - z).abs() <= z.abs() * U + slope * 2 * off + 2.0 ** -22 * (1 + ref.abs())).all()
+            continue
+        h1, h3, o1, o3 = ref[:, :n_out], ref[:, n_out:], off[:, :n_out], off[:, n_out:]
+        if kind == "gelu":
+            gelu = torch.nn.functional.gelu(h1, approximate="tanh")
+            bound = 1.13 * 2 * o1 * h3.abs() + gelu.abs() * 2 * o3 + U * (gelu * h3).abs() + 2.0 ** -20 * (1 + h1.abs()) * h3.abs()
+            assert ((got - gelu * h3).abs() <= bound).all()
+        else:
+            s = torch.sigmoid(h1)
+            bound = ((s * (1 + h1 * (1 - s))).abs() * (h1.abs() * U + 2 * o1) * h3.abs() + (h1 * s).abs() * 2 * o3 + 3 * U * (h1 * s * h3).abs()) * 1.02 + 1e-30
+            assert ((got - h1 * s * h3).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("M,N,K,swiglu,taken", [(129, 33024, 512, True, True), (192, 65536, 256, False, True), (256, 37888, 512, True, True),
                                                 (256, 32768, 512, True, False), (128, 37888, 512, True, False), (255, 152064, 256, False, False)])
 def test_a_steps_rows_in_the_place_of_the_block_kernel(M, N, K, swiglu, taken, monkeypatch):
