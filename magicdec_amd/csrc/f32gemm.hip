@@ -170,13 +170,14 @@ bool shape_ok(int M, int N, int K) { return M > 0 && N > 0 && K > 0 && N % 4 == 
 
 // (Behind other launches, operands not in the caches, us, library / here: 4 803 x 3 072 x 2 048 521 / 441, x 2 048 x 8 192 1 233 / 1 206,
 // 1 400 x 8 192 x 2 048 372 / 336, but 999 x 2 048 x 8 192 244 / 259, 560 x 2 048 x 8 192 157 / 203, 130 x 8 192 x 2 048 47 / 54: few rows,
-// above all of deep products, leave CUs idle at the end, and the library splits K.)
+// above all of deep products, leave CUs idle at the end, and the library splits K: 1 582 x 1 024 x 4 096 112 / 132.  Over 260 products of 1 200 to
+// 6 000 rows 0.95 of the library's time, 1.09 at the worst; from 5 632 k on 0.85 to 1.09, level on average.)
 extern "C" int md_linear_f32_supported(int M, int N, int K) {
     MD_CHECK_ARG(M > 0 && N > 0 && K > 0, "md_linear_f32_supported: M=%d N=%d K=%d", M, N, K);
     if (!shape_ok(M, N, K) || M < (K < 8192 ? 1200 : 2000)) return 0;
     double us = 0;
     best_tile(M, N, K, &us);
-    return us <= 1.1 * (2e-6 * M * N / 130 * K + 12) ? 1 : 0;
+    return us <= 1.05 * (2e-6 * M * N / 130 * K + 8) ? 1 : 0;
 }
 
 extern "C" int md_linear_f32(const float* x, int64_t ldx, const float* w, float* out, int64_t ldo, int M, int N, int K, int tile,

@@ -1745,3 +1745,12 @@ def test_uploaded_numbers_have_the_type_asked_for():
         for dtype in (torch.int32, torch.long):
             got = ops.upload(v, dtype, "cpu")
             assert got.dtype == dtype and got.tolist() == [3, 1, 2]
+
+
+def test_32_bit_products_of_few_tiles_stay_in_the_library():
+    """Either side of the line: a last round of tiles that leaves most CUs idle, against the library's split of K."""
+    from magicdec_amd import ops
+    for M, N, K in ((1582, 1024, 4096), (1400, 512, 4096), (1519, 768, 3072), (1199, 2048, 2048), (1999, 2048, 8192), (2000, 2050, 2048), (4000, 2048, 2056)):
+        assert not ops.linear_f32_supported(M, N, K), (M, N, K)
+    for M, N, K in ((4803, 3072, 2048), (4803, 2048, 8192), (2535, 1024, 4096), (1200, 8192, 2048), (1500, 4096, 512)):
+        assert ops.linear_f32_supported(M, N, K), (M, N, K)
