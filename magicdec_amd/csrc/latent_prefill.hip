@@ -265,6 +265,11 @@ __global__ __launch_bounds__(NT, 2) void latent_prefill_kernel(const LatentParam
     if (p.gate && valid) inv /= 1.0f + expf(-(float)reinterpret_cast<const bf16_t*>(p.gate)[(q0 + qi) * p.ld_gate + h]);
     // ---- output rows: through LDS, so that a store writes whole rows of a head
     __syncthreads();                                                // every wave is past the last image
+    // With wide heads nothing below is computed, and kept, in front of the tiles: 192 / 192 has no register for it (40 spilled; 4 x 821 rows
+    // behind 100, 16 heads of 128 + 64 / 192 75 -> 62 us)
+    int ln = lane;
+    if constexpr (DK + DV >= 320) asm volatile("" : "+v"(ln));
+    const int oj = ln & 31;
     unsigned char* mine = smem + wave * 32 * DV * 2;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -272,11 +277,11 @@ __global__ __launch_bounds__(NT, 2) void latent_prefill_kernel(const LatentParam
         for (int rg = 0; rg < 4; ++rg) {
             const int ch = (db + (rg >> 1) * (NB / 2)) * 2 + (rg & 1);
             const f32x4 ov = {o[db][rg * 4] * inv, o[db][rg * 4 + 1] * inv, o[db][rg * 4 + 2] * inv, o[db][rg * 4 + 3] * inv};
-            *reinterpret_cast<bf16x4*>(mine + j * DV * 2 + lds_place<CV>(ch, j) * 16 + kh * 8) = __builtin_convertvector(ov, bf16x4);
+            *reinterpret_cast<bf16x4*>(mine + oj * DV * 2 + lds_place<CV>(ch, oj) * 16 + (ln >> 5) * 8) = __builtin_convertvector(ov, bf16x4);
         }
 #pragma unroll
     for (int i = 0; i < CV / 2; ++i) {
-        const int c = i * 64 + lane, r = c / CV, ch = c % CV;
+        const int c = i * 64 + ln, r = c / CV, ch = c % CV;
         const bf16x8 v = lds_read_b128(mine + r * DV * 2 + lds_place<CV>(ch, r) * 16);
         if (w0 + r >= 0 && w0 + r < n_b && ch * 8 < p.vdim)
             *reinterpret_cast<bf16x8_a8*>(reinterpret_cast<bf16_t*>(p.out) + (q0 + w0 + r) * p.ldo + h * p.vdim + ch * 8) = v;
