@@ -70,10 +70,13 @@ __global__ __launch_bounds__(NT, 2) void latent_prefill_kernel(const LatentParam
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];   // NI tile images; first the queries, last the output rows
     const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, kh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // blocks of one (request, head) differ by multiples of 8: same XCD; the long ones (late rows) of every pair first, since the last one to
-    // start is the last to end (pair after pair: 352 us; profiled, a CU was idle for 23 % of them)
+    // blocks of one (request, head) differ by multiples of 8: same XCD.  The long ones (late rows) first, since the last one to start is the
+    // last to end: of every pair where a prompt's rows are most of its context (pair after pair: 352 us for 332), one pair after the other
+    // behind a long one, where its groups are about as long and read its rows together (2 x 655 behind 4000, 128 heads of 128 + 64 / 128
+    // 714 us, 753 of every pair).  The first request decides: it is a matter of speed only
     const int r0 = blockIdx.x >> 3, pairs = (p.B * p.H + 7) / 8;
-    const int qg = p.n_groups - 1 - r0 / pairs, pair = (r0 % pairs) * 8 + (blockIdx.x & 7);
+    const bool all = p.qo_indptr[1] - p.qo_indptr[0] > p.pos0[0];
+    const int qg = p.n_groups - 1 - (all ? r0 / pairs : r0 % p.n_groups), pair = (all ? r0 % pairs : r0 / p.n_groups) * 8 + (blockIdx.x & 7);
     if (pair >= p.B * p.H) return;
     const int b = pair / p.H, h = pair % p.H;
     const int q0 = p.qo_indptr[b], n_b = p.qo_indptr[b + 1] - q0;

@@ -289,6 +289,21 @@ def test_groups_of_a_round_of_the_chip_and_more(ops, H, lens):  # noqa: F811
         assert float((got.double() - want).abs().max()) < 3e-2 * max(1.0, float(want.abs().max())), first
 
 
+@pytest.mark.parametrize("first", [0, 1])
+def test_prompt_rows_in_either_order_of_their_groups(ops, first):  # noqa: F811
+    """Two groups of rows behind many and two at a prompt's start in one call, either of them first (which decides the order of the
+    workgroups); a third request has one group."""
+    lens = [1100, 400, 90]
+    spec, zs, qs, _, refs, _ = attention_case(ops, 5, 32, 16, 40, 32, 64, 23, BF, lens)
+    s = Seqs(ops, spec, BF, lens, seed=3)
+    s.attend(zs[0][:700], qs[0][:700], [0], [0], [700])
+    part = [(0, 700, 400), (1, 0, 400)][::1 - 2 * first] + [(2, 0, 90)]
+    got, _ = s.attend(torch.cat([zs[b][a:a + k] for b, a, k in part]), torch.cat([qs[b][a:a + k] for b, a, k in part]), [b for b, _, _ in part],
+                      [a for _, a, _ in part], [k for _, _, k in part], form="expanded")
+    want = torch.cat([refs[b][0][a:a + k] for b, a, k in part])
+    assert float((got.double() - want).abs().max()) < 3e-2 * max(1.0, float(want.abs().max()))
+
+
 def test_scores_of_any_size(ops):  # noqa: F811
     """Large, tiny and negated scores: the running maximum moves by hundreds, or not at all."""
     for score in (0.01, 90.0, 400.0, -20.0):
