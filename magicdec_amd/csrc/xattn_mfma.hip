@@ -351,11 +351,14 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? (small_heads<DV>() ? 4 : 2) : 1)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // The last groups first: the longest, until a chunk is full; the last one to start is the last to end.  Of every pair where a prompt's
     // rows are most of its keys, one pair after the other where they are few behind many: its groups are then about as long, and read its
-    // keys together.  8 x 2049 rows, 32 heads of 128 on 8 kv heads: 574 us pair after pair, 545 the last groups of every pair first; 8 x 584
-    // rows behind 4000, 16 heads of 128 / 256: 680 and 712 (the first request decides: it is a matter of speed only)
+    // keys together.  8 x 2049 rows, 32 heads of 128 on 8 kv heads: 574 us pair after pair, 545 the last groups of every pair first; 8 x 2500
+    // behind 4000, 12 heads of 96 on 4 1 112 -> 1 030 pair after pair with the last groups first.  A pair of few groups is read once where
+    // they run side by side from the first, also in many rounds of the chip: 8 x 584 rows behind 4000, 16 heads of 128 / 256 655 us, 697 with
+    // the last ones first and 712 of every pair; 32 x 625 rows behind 100 473 and 502.  (The first request decides: it is a matter of speed only)
     const int r0 = blockIdx.x >> 3, pairs = (p.B * p.KH + 7) / 8;
-    const bool all = p.qo_indptr[1] - p.qo_indptr[0] > p.pos0[0];
-    const int qg = p.n_qgroups - 1 - (all ? r0 / pairs : r0 % p.n_qgroups), pair = (all ? r0 % pairs : r0 / p.n_qgroups) * 8 + (blockIdx.x & 7);
+    const bool few = p.n_qgroups < 8, all = p.qo_indptr[1] - p.qo_indptr[0] > p.pos0[0] && (!few || gridDim.x <= 1024);
+    const int at = all ? r0 / pairs : r0 % p.n_qgroups, pair = (all ? r0 % pairs : r0 / p.n_qgroups) * 8 + (blockIdx.x & 7);
+    const int qg = few && !all ? at : p.n_qgroups - 1 - at;
     if (pair >= p.B * p.KH) return;
     const int b = pair / p.KH, kvh = pair % p.KH, g = p.g;
     const int q0 = p.qo_indptr[b], n_b = p.qo_indptr[b + 1] - q0;

@@ -280,8 +280,20 @@ def test_output_rows_of_any_width(ops, D, DV):
     assert got.shape == ref[0].shape and float((got.double() - ref[0]).abs().max()) <= 1.5e-2 * max(1.0, float(ref[0].abs().max()))
 
 
+@pytest.mark.parametrize("B", [16, 17])
+def test_prompts_of_few_groups_in_many_rounds_of_the_chip(ops, B):
+    """1024 and 1088 workgroups, two a pair: whole prompts of the same rows, the last request one row shorter."""
+    H, n = 32, 300
+    spec, rows, ref = attention_case(ops, H, H, 32, 32, 0, 5, BF, [n])
+    lens = [n] * (B - 1) + [n - 1]
+    s = Seqs(ops, spec, BF, lens, seed=4)
+    got = s.attend(torch.cat([rows[0][:k] for k in lens]), range(B), [0] * B, lens)
+    want = torch.cat([ref[0][:k] for k in lens])
+    assert float((got.double() - want).abs().max()) <= 1.5e-2 * max(1.0, float(want.abs().max()))
+
+
 @pytest.mark.parametrize("first", [0, 1])
-@pytest.mark.parametrize("H,KH,D,DV", [(4, 2, 128, 128), (3, 3, 64, 64), (4, 1, 128, 256)])
+@pytest.mark.parametrize("H,KH,D,DV", [(4, 2, 128, 128), (3, 3, 64, 64), (4, 1, 128, 256), (16, 2, 128, 128)])       # (2 to 11 groups)
 def test_prompt_rows_in_either_order_of_their_groups(ops, first, H, KH, D, DV):
     """A few rows behind many and a whole prompt in one call, either of them first (which decides the order of the workgroups)."""
     lens = [1500, 700]
