@@ -494,13 +494,15 @@ def prompt_rows(M: int, N: int, K: int, swiglu: bool = False, rows_stay: bool = 
     with the rows to bring back; the line is where those cross over the same products.  rows_stay: the weight is one whose row-major
     tensor is never released (a pool's, or one that steps of more than 256 rows read), so that the library has nothing to bring back; over
     330 products of 257 to 2 600 rows the two cross at 1.45 times the ideal (1.10 of the library's time at the worst; beyond it 449 x
-    2 048 x 5 632 in 38 us for 27, 301 x 4 096 x 14 336 in 91 for 74).
+    2 048 x 5 632 in 38 us for 27, 301 x 4 096 x 14 336 in 91 for 74), those of less than a round of small tiles alone: 8 196 x 8 192 x 512
+    takes 74 us for the library's 137, far from an ideal that counts neither's first steps.
     Rows just behind whole rounds of tiles are a round more: 8 196 x 4 096 x 18 432 in 950 us, 8 192 in 760 and the other four in 40 on the
     weight-streaming kernel, whose time the last line bounds from above (49 / 55 us for 28 672 x 4 096 at 64 / 128 rows, 16 / 21 for 4 096
     x 4 096, 54 / 64 for 5 120 x 27 648)."""
     from .. import ops
     us = ops.linear_prompt_us(M, N, K, swiglu) if _MODE != "lib" and M > 256 else -1.0
-    if us < 0 or us > (1.45 if rows_stay else 2.4) * (2e-6 * M * N / 1400 * K + 12):
+    few = rows_stay and M * N < CUS * 128 * 128
+    if us < 0 or us > (1.45 if few else 2.4) * (2e-6 * M * N / 1400 * K + 12):
         return 0
     rest = M % 256
     if 0 < rest <= 128 and M - rest > 256 and ops.linear_supported(rest, N, K, swiglu):

@@ -1682,7 +1682,8 @@ def test_products_of_more_rows_than_a_step_has_know_whether_the_weight_is_there(
     from magicdec_amd.Engine import gemm_policy, model_core
     for M, N, K in ((384, 4096, 14336), (449, 2048, 5632), (572, 2048, 8192)):
         assert gemm_policy.prompt_rows(M, N, K) == M and gemm_policy.prompt_rows(M, N, K, rows_stay=True) == 0
-    for M, N, K, gated in ((384, 28672, 4096, True), (8192, 4096, 14336, False), (2048, 2048, 8192, False), (512, 6144, 4096, False)):
+    for M, N, K, gated in ((384, 28672, 4096, True), (8192, 4096, 14336, False), (2048, 2048, 8192, False), (512, 6144, 4096, False),
+                           (8196, 8192, 512, False), (4100, 4096, 512, False)):
         assert gemm_policy.prompt_rows(M, N, K, gated, rows_stay=True) == gemm_policy.prompt_rows(M, N, K, gated) > 0
     name = "rows-stay"
     model_core.transformer_configs[name] = dict(block_size=256, n_layer=1, vocab_size=512, n_head=16, n_local_heads=4, dim=2048, intermediate_size=8192)
