@@ -216,8 +216,9 @@ class _BackendBase:
 
     def _rows_that_fit(self, rows, row_bytes=0, fixed=0):
         """`rows` of a prompt, or as many as the device's free memory holds: their activations in a layer (and row_bytes each, and `fixed`)
-        beside the row-major weights that the prompt brings back.  The same on every rank of a tensor-parallel group, and where a whole
-        draft runs on each rank: other portions round otherwise, and the ranks' tokens have to be the same."""
+        beside the row-major weights that the prompt may bring back -- all that are released, since a last portion of few rows can be the
+        library's.  The same on every rank of a tensor-parallel group, and where a whole draft runs on each rank: other portions round
+        otherwise, and the ranks' tokens have to be the same."""
         dev, m = torch.device(self.device), self.model
         if dev.type != "cuda":
             return rows

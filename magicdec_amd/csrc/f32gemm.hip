@@ -3,8 +3,8 @@
 // replaces: the library products of the layered designs in 32-bit (prompts and the recorded traces that check a design).
 //
 // What bounds it: v_mfma_f32_16x16x4_f32, 64 flop per clock and SIMD (157 TFLOP/s; an 8192^3 library product reaches 152).  A step of 32 k
-// of a 128 x 128 tile is 4 096 clocks of it for 32 KB: both operands come by DMA in whole lines, three buffers, one barrier a step, two
-// and more workgroups of four wavefronts on a CU that cover each other's barriers.  (Straight from memory into the instruction's order -- 64 bytes of
+// of a 64 x 128 tile is 2 048 clocks of it for 24 KB (64 x 64: 1 024 for 16, 32 x 64: 512 for 12): both operands come by DMA in whole
+// lines, three buffers, one barrier a step, two and more workgroups of four wavefronts on a CU that cover each other's barriers.  (Straight from memory into the instruction's order -- 64 bytes of
 // 16 rows a load -- the address unit takes 42 clocks a load, and 64 x 64 wavefront tiles reach 124 TFLOP/s, 64 x 32 ones 83.)  A lane reads
 // four k of a row at once; product e takes the e-th of each, the same four k of either operand.  What is left to choose is the tile, whose
 // count should divide evenly among 256 CUs.

@@ -208,7 +208,6 @@ __global__ __launch_bounds__(256) void head_linear_mfma_kernel(const HeadLinearP
     }
 }
 
-// 32-bit: a thread per output
 // 32-bit on the fp32 matrix instructions, laid out as above: a lane reads four k of a row at once, product e takes the e-th of each.  Dense
 // 16-byte pieces only; the kernel below has a thread per value, which waits for every k (2 400 rows, 16 heads, 128 -> 512: 4 470 us, here 126; 8 rows: 50 and 5.8).
 template <int RT>
@@ -253,6 +252,7 @@ __global__ __launch_bounds__(256) void head_linear_f32_mfma_kernel(const HeadLin
     }
 }
 
+// 32-bit of any sizes: a thread per output
 __global__ __launch_bounds__(256) void head_linear_f32_kernel(const HeadLinearParams p) {
     const int h = blockIdx.z, row0 = blockIdx.y * 16, n = blockIdx.x * 16 + (threadIdx.x & 15), row = row0 + (threadIdx.x >> 4);
     if (n < p.N && row < p.M) {

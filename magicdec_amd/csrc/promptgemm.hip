@@ -6,9 +6,9 @@
 //
 // Also a step's 129 to 256 rows where the block kernel needs a second round of the chip for its 128 columns a workgroup.
 //
-// What bounds it.  A full chip of matrix instructions is bound by power: the clock falls to about 1.75 of 2.4 GHz, and time is energy as much
-// as it is stalls.  v_mfma_f32_16x16x32 moves half the accumulator bytes per flop of 32x32x16 and is the faster one by clock, although its
-// 16 cycles hide less behind each (8192^3: 88 % of the cycles with the large one took as long as 82 % with the small one).  Measured, us:
+// What bounds it.  The matrix cores, busy for 78 to 85 % of the cycles of the large products, at the clock that so many of them leave: 1.8 to
+// 1.9 of 2.4 GHz, as the library's (profiles/prompt_kernels.txt).  v_mfma_f32_16x16x32 moves half the accumulator bytes per flop of
+// 32x32x16, and an 8192^3 product took no longer with it, although its 16 cycles hide less behind each.  Measured, us:
 // (8192, 4096, 4096) 180, library 184; (8192, 4096, 14336) 612 / 604; (8192, 28672, 4096) with SiLU * mul 1 299 / 1 391;
 // (8196, 4096, 18432) 972 / 1 311; (6144, 2048, 8192) 135 / 152; (2081, 37888, 3584) 433 / 552.
 //   * four wavefronts of 256 rows x 64 columns, one per SIMD with 256 accumulators: each reads all of A from LDS and its own columns of W
@@ -19,7 +19,7 @@
 //     64.2, the large ones 1 % slower), A two to three in LDS and half a step in registers; one barrier a step, where the last LDS
 //     instruction lies some products back;
 //   * one instruction beside each product, in an order that the compiler has to keep (spread): in bunches the four wavefronts queue at the
-//     address unit and at LDS, and the matrix cores wait (1 195 -> 1 390 TFLOP/s at 8192 x 28 672 x 4 096);
+//     address unit and at LDS, and the matrix cores wait (8192 x 28 672 x 4 096: 1 610 us so, 1 384 spread);
 //   * workgroups stay and take tile after tile; the loads of the next tile are in flight behind the last steps of one;
 //   * an XCD's 32 workgroups take 8 row tiles x 4 column tiles, whose operands its L2 holds (4 or 16 row tiles: 1.5 / 4 % slower).
 #include "md_common.h"
