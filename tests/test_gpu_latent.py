@@ -263,7 +263,7 @@ def test_long_context_is_split_over_workgroups(ops):  # noqa: F811
 
 @pytest.mark.parametrize("D,VD", [(64, 64), (128, 128), (192, 256)])
 def test_prompts_of_more_than_64_pages(ops, D, VD):  # noqa: F811
-    """The expanded form keeps the numbers of 64 pages at a time; rows that fill no group of 256 are a prompt's first ones."""
+    """The expanded form keeps the numbers of 64 pages at a time; prompts whose rows fill no whole number of groups of 256."""
     n = 64 * 64 + 70
     spec, zs, qs, _, refs, _ = attention_case(ops, 2, D, 32, VD, 32, 64, 17, BF, [n])
     s = Seqs(ops, spec, BF, [n], page=64, seed=6)

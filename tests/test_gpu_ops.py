@@ -95,8 +95,8 @@ def test_paged_attention_vs_oracle(ops, name, B, n, H, KH, D, lens, causal, scat
 @pytest.mark.parametrize("H,KH,D,ns,lens", [(10, 2, 128, [110, 41], [4230, 4096]), (10, 2, 128, [40, 1], [4097, 64]), (3, 1, 64, [100], [4300]),
                                             (4, 1, 64, [300, 33], [4200, 33])])
 def test_prompt_rows_over_more_than_64_pages(ops, H, KH, D, ns, lens):
-    """Page numbers are kept 64 at a time; query rows that fill no workgroup are a request's first ones, also where its heads per kv head
-    do not divide one."""
+    """Page numbers are kept 64 at a time; query rows that fill no whole number of workgroups, also where the heads per kv head do not
+    divide one."""
     name = f"prefill-many-pages-{H}-{KH}-{D}-{ns[0]}"
     cache, indices, indptr, last, max_pages = make_paged(len(ns), lens, KH, D, seed=case_seed(name), page_size=64, scatter=True)
     q = torch.randn(sum(ns), H, D, generator=torch.Generator().manual_seed(3)).to(BF)
