@@ -329,6 +329,15 @@ int md_linear_prompt(const void* x, int64_t ldx, const void* w_packed, const voi
 int md_linear_f32_supported(int M, int N, int K);
 int md_linear_f32(const float* x, int64_t ldx, const float* w, float* out, int64_t ldo, int M, int N, int K, int tile, md_stream_t stream);
 
+/* md_linear_f32_thirds (csrc/f32thirds.hip): the same on the bf16 matrix instructions, every number as the sum of three bf16 numbers (six
+ * products of their parts, 32-bit sums): as exact as md_linear_f32.  K < 2^20.  ws: md_linear_f32_thirds_workspace(M, K) bytes, 16-byte
+ * aligned (x in three parts), free again behind the call on its stream.  _supported: 1 if it takes the shape and is expected to be faster than
+ * md_linear_f32 and a library GEMM.  tile: 0, or 1000 * rows + columns (256 / 192 / 160 / 128 x 256, 256 / 192 / 128 / 64 x 128). */
+int md_linear_f32_thirds_supported(int M, int N, int K);
+size_t md_linear_f32_thirds_workspace(int M, int K);
+int md_linear_f32_thirds(const float* x, int64_t ldx, const float* w, float* out, int64_t ldo, int M, int N, int K, int tile, void* ws,
+                         size_t ws_bytes, md_stream_t stream);
+
 /* ------------------------------------------------------------------------
  * K8b  fused small-problem linear: a linear of a decode / verify step TOGETHER with the op that consumes its output,
  *      one launch (csrc/tilegemm.hip; no split-K across workgroups, no workspace, deterministic)

@@ -127,6 +127,9 @@ _SIGNATURES = {
     "md_linear_xielu": (c_int, [P, L, P, I, P, P, L, I, I, I, P, c_size_t, P]),
     "md_linear_f32_supported": (c_int, [I, I, I]),
     "md_linear_f32": (c_int, [P, L, P, P, L, I, I, I, I, P]),
+    "md_linear_f32_thirds_supported": (c_int, [I, I, I]),
+    "md_linear_f32_thirds_workspace": (c_size_t, [I, I]),
+    "md_linear_f32_thirds": (c_int, [P, L, P, P, L, I, I, I, I, P, c_size_t, P]),
     "md_linear_prompt_us": (ctypes.c_double, [I, I, I, I]),
     "md_linear_prompt": (c_int, [P, L, P, P, P, P, L, I, I, I, I, I, P]),
     "md_linear_block_xielu": (c_int, [P, L, P, P, P, L, I, I, I, P, c_size_t, P]),

@@ -642,6 +642,39 @@ def linear_f32(x, weight, tile=0):
     return out
 
 
+@functools.lru_cache(maxsize=4096)
+def linear_f32_thirds_supported(M, N, K):
+    """True when md_linear_f32_thirds (csrc/f32thirds.hip) takes this shape and is expected to be the fastest."""
+    return _lib.load().md_linear_f32_thirds_supported(int(M), int(N), int(K)) > 0
+
+
+THIRDS_BYTES = 512 << 20        # of scratch at most (some rows of more columns than that take several calls)
+
+
+def linear_f32_thirds(x, weight, tile=0):
+    """linear_f32 on the bf16 matrix cores (csrc/f32thirds.hip): every number as the sum of three bf16 numbers, 32-bit sums.  Where there is
+    no memory for its scratch, linear_f32."""
+    _gpu(x, weight)
+    if x.dim() != 2 or x.stride(1) != 1 or weight.dim() != 2 or not weight.is_contiguous() or x.shape[1] != weight.shape[1]:
+        raise ValueError("linear_f32_thirds expects x [M, K] with unit inner stride and a contiguous weight [N, K]")
+    if x.dtype != torch.float32 or weight.dtype != torch.float32:
+        raise TypeError("linear_f32_thirds takes float32")
+    (M, K), N = x.shape, weight.shape[0]
+    lib = _lib.load()
+    parts = max(1, -(-6 * M * K // THIRDS_BYTES))
+    rows = -(-M // (256 * parts)) * 256
+    try:
+        ws = torch.empty(max(1, lib.md_linear_f32_thirds_workspace(min(M, rows), K)), dtype=torch.uint8, device=x.device)
+    except torch.OutOfMemoryError:
+        return linear_f32(x, weight)
+    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    for a in range(0, M, rows):
+        n = min(rows, M - a)
+        check(lib.md_linear_f32_thirds(_p(x[a:]), x.stride(0), _p(weight), _p(out[a:]), N, n, N, K, int(tile), _p(ws), ws.numel(), _stream()),
+              "md_linear_f32_thirds")
+    return out
+
+
 # ----------------------------------------------------------------------------- K8b
 FL_NONE, FL_SWIGLU, FL_RESID, FL_ROPE_APPEND, FL_XIELU, FL_GEGLU = 0, 1, 2, 3, 4, 5
 
