@@ -12,18 +12,24 @@
 //   indices = top-(budget-W) of score, descending score, ties -> lowest index
 //   draft rows = K,V[indices] ++ K,V[S-W:S]
 //
-// Seven small launches, none on the timed decode path (once per prefill per layer):
-//   tab     : the table of exponentials (below)
-//   stats   : row max / sum-exp partials per column chunk   (MFMA scores; float64 sums)
-//   finalize: per-row (max, 1 / sum) of the whole context from the chunk partials
+// Five small launches, none on the timed decode path (once per prefill per layer):
+//   stats   : the table of exponentials (below); row max / sum-exp partials per column chunk   (MFMA scores; float64 sums)
+//   finalize: per-row (max, 1 / sum) of the whole context from the chunk partials, where those are many
 //   accum   : recompute scores, p, 8-row group sums, bf16 chunk accumulation
 //   pool    : pool + group sum
 //   select  : exact radix select, ranked by counting (one WG per b,kvh)
 //   gather  : copy the selected rows into the draft pages
 #include "md_common.h"
 
+#include <type_traits>
+#include <utility>
+
 namespace {
 
+template <int... I, class F>
+__device__ __forceinline__ void unrolled(std::integer_sequence<int, I...>, F f) {
+    (f(std::integral_constant<int, I>()), ...);
+}
 
 struct SnapParams {
     const bf16_t* q;      // [B*W, H, D]
@@ -129,25 +135,44 @@ __device__ __forceinline__ double exp_neg(double x) {
 // The reference's scores are bf16 VALUES (model.py:411: a bf16 einsum), i.e. one of 65 536 numbers, and the
 // probabilities must be correctly rounded bf16(exp(s - M) / Z) (see "Rounding sequence" above: an fp32 evaluation with
 // another summation order flips ~1e-4 of those roundings).  exp() in float64 per element is a billion OCML calls per
-// layer for 64 requests of 16 000 tokens, 0.21 TB/s of K bytes = 2.6 % of the HBM peak.  So exp(v) of every bf16 value with 2^-14 <= |v| < 2^9 sits in a float64 table in LDS (filled with OCML's exp once
+// layer for 64 requests of 16 000 tokens, 0.21 TB/s of K bytes = 2.6 % of the HBM peak.  So exp(v) of every bf16 value with 2^-23 <= |v| < 2^9 sits in a float64 table in LDS (filled with OCML's exp once
 // per call): the row sum is  sum_i T[s_i]  (reference 0: e^512 * 65 536 columns is far below the float64 range) and a
 // probability is  T[s] * (exp(-M) / Z)  -- one LDS gather and one f64 multiply.  Of the few scores outside the table, tiny
-// ones (|s| < 2^-14) are a short polynomial, the others (|s| >= 512, masked) take the lean exp_neg() above against a running maximum, so
+// ones are a short polynomial, the others (|s| >= 512, masked) take the lean exp_neg() above against a running maximum, so
 // nothing overflows whatever the raw (unscaled) scores are.
-// The UNSCALED q.k of a seeded-random 1B layer is ~N(0, 6.5^2) and a trained checkpoint's reaches the hundreds: the table covers 23
-// binades x 128 mantissas x 2 signs = 5 888 entries = 46 KB (two workgroups of pass 1 per CU), laid out [magnitude][sign] so that the
-// byte offset of a score is (magnitude index << 4) | (sign << 3) and still fits 16 bits.
-constexpr int kTabE0 = 113;                 // biased bf16 exponent of 2^-14
-constexpr int kTabBinades = 23;             // 2^-14 .. 2^9
+// The UNSCALED q.k of a seeded-random 1B layer is ~N(0, 6.5^2) and a trained checkpoint's reaches the hundreds: the table covers 32
+// binades x 128 mantissas x 2 signs = 8 192 entries = 64 KB, laid out [magnitude][sign] so that the byte offset of a score is
+// (magnitude index << 4) | (sign << 3) and still fits 16 bits.  One score in 10^8 of N(0, 6.5^2) is smaller than that; with 2^-14 as the
+// smallest it was one in 10^5, and one batch of 1 024 in 130 left the hot path.  Kernels whose query image leaves no room take the
+// upper 23 binades.
+constexpr int kTabE0 = 104;                 // biased bf16 exponent of 2^-23
+constexpr int kTabBinades = 32;             // 2^-23 .. 2^9
 constexpr int kTabMag = kTabBinades * 128;  // magnitude indices: (exponent - E0) * 128 + mantissa
 constexpr int kTabN = 2 * kTabMag;          // [magnitude][sign]
-__device__ double g_exp_tab[kTabN];
+constexpr int kTabSmall = 23;               // binades of the small table
+__device__ __attribute__((aligned(16))) double g_exp_tab[kTabN];
+template <int BIN> struct Tab {             // BIN binades up to 2^9
+    static constexpr int E0 = kTabE0 + kTabBinades - BIN, N = BIN * 256;
+};
 
-__global__ __launch_bounds__(256) void snapkv_tab_kernel() {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= kTabN) return;
-    const unsigned int bits = ((unsigned int)(i & 1) << 15) | (unsigned int)((i >> 1) + (kTabE0 << 7));
-    g_exp_tab[i] = exp((double)bf16_bits_to_f32((unsigned short)bits));
+// Filled by every workgroup of the first pass for itself (8 exponentials a thread: 2 us, where a launch in front took 4.5) and left by
+// its first one for the second pass: the same bytes in every call.
+template <int BIN>
+__device__ __forceinline__ void fill_table(double* tab, int tid, int nthr, bool leave) {
+    for (int i = tid; i < kTabN; i += nthr) {
+        const int at = i - (kTabN - Tab<BIN>::N);
+        if (at < 0 && !leave) continue;
+        const unsigned int bits = ((unsigned int)(i & 1) << 15) | (unsigned int)((i >> 1) + (kTabE0 << 7));
+        const double e = exp((double)bf16_bits_to_f32((unsigned short)bits));
+        if (at >= 0) tab[at] = e;
+        if (leave) g_exp_tab[i] = e;
+    }
+}
+template <int BIN>
+__device__ __forceinline__ void load_table(double* tab, int tid, int nthr) {
+    const u32x4* from = reinterpret_cast<const u32x4*>(g_exp_tab + (kTabN - Tab<BIN>::N));
+#pragma unroll 4
+    for (int i = tid; i < Tab<BIN>::N / 2; i += nthr) reinterpret_cast<u32x4*>(tab)[i] = from[i];
 }
 
 // exp(v) for |v| < 2^-14: the next term is below 2^-60
@@ -158,31 +183,42 @@ __device__ __forceinline__ double exp_tiny(float v) {
 __device__ __forceinline__ bool is_tiny(float v) { return fabsf(v) < 6.103515625e-05f; }
 
 // table index of a bf16 value held in a float, or -1 (outside the table: tiny, large, zero, inf)
+template <int BIN>
 __device__ __forceinline__ int tab_index(float s) {
     const unsigned int bits = __float_as_uint(s) >> 16;
-    const unsigned int a = (bits & 0x7fffu) - ((unsigned int)kTabE0 << 7);
-    return a < (unsigned int)kTabMag ? (int)((a << 1) | (bits >> 15)) : -1;
+    const unsigned int a = (bits & 0x7fffu) - ((unsigned int)Tab<BIN>::E0 << 7);
+    return a < (unsigned int)(BIN * 128) ? (int)((a << 1) | (bits >> 15)) : -1;
 }
 
 // Two scores at a time: `w` = two bf16 values in one dword (v_cvt_pk_bf16_f32).  With d = bits - (E0 << 7) a score in the table has
-// magnitude index d & 0x7fff < kTabMag < 4096, so that rotating d left by four gives its byte offset (magnitude x 16 + sign x 8); any
-// other d leaves an offset past the last entry or with one of its low three bits set.  `top` (maximum) and `low` (or) collect both over
-// a batch of scores: tab_outside says whether all of them lie inside.
+// magnitude index d & 0x7fff < 4096, so that rotating d left by four gives its byte offset (magnitude x 16 + sign x 8); any
+// other d leaves one of the low three bits set, or (small table) an offset past the last entry.  `top` (maximum) and `low` (or) collect
+// both over a batch of scores: tab_outside says whether all of them lie inside.
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ unsigned int pack_bf16(float a, float b) {
-    const bf16x2 pk = {f32_to_bf16(a), f32_to_bf16(b)};
-    return *reinterpret_cast<const unsigned int*>(&pk);
+    return __builtin_bit_cast(unsigned int, __builtin_convertvector((f32x2{a, b}), bf16x2));
 }
+// The same where the halves are taken apart again, which the compiler would convert one by one.  (Not for a matrix product's result: the
+// compiler does not see the wait that assembly behind one needs)
+__device__ __forceinline__ unsigned int round_pair(float a, float b) {
+    unsigned int pk;
+    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(pk) : "v"(a), "v"(b));
+    return pk;
+}
+template <int BIN>
 __device__ __forceinline__ unsigned int tab_offsets2(unsigned int w, u16x2& top, unsigned int& low) {
-    const u16x2 d = *reinterpret_cast<const u16x2*>(&w) - (unsigned short)(kTabE0 << 7);
-    const u16x2 r = d * (unsigned short)16 + (d >> (unsigned short)12);
-    top = __builtin_elementwise_max(top, r);
+    const u16x2 d = *reinterpret_cast<const u16x2*>(&w) - (unsigned short)(Tab<BIN>::E0 << 7);
+    const u16x2 turned = d >> (unsigned short)12;
+    u16x2 r;
+    asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(r) : "v"(d), "s"(0x00100010u), "v"(turned));      // (left alone: a shift and an or)
+    if constexpr (BIN < kTabBinades) top = __builtin_elementwise_max(top, r);
     const unsigned int o = *reinterpret_cast<const unsigned int*>(&r);
     low |= o;
     return o;
 }
+template <int BIN>
 __device__ __forceinline__ bool tab_outside(u16x2 top, unsigned int low) {
-    return (low & 0x00070007u) != 0 || top[0] >= kTabN * 8 || top[1] >= kTabN * 8;
+    return (low & 0x00070007u) != 0 || (BIN < kTabBinades && (top[0] >= Tab<BIN>::N * 8 || top[1] >= Tab<BIN>::N * 8));
 }
 __device__ __forceinline__ double tab_at(const double* tab, unsigned int offset) {
     return *reinterpret_cast<const double*>(reinterpret_cast<const unsigned char*>(tab) + offset);
@@ -203,45 +239,104 @@ __device__ __forceinline__ void merge_mz(double& m, double& Z, double m2, double
 constexpr int kQPad = 16;                   // bytes of padding per row of the Q image in LDS
 constexpr int kMaxRT = 16;                  // 16-row tiles per kv head: L = g * W <= 256
 
-// Q rows of one (request, kv head), ordered (r, l), into LDS: row rg at rg * (2 D + 16) bytes
+// Q rows of one (request, kv head), ordered (r, l), into LDS: row rg at rg * (2 D + 16) bytes.  An odd number of 16-row tiles: the last one
+// twice, so that tiles come in twos
+__host__ __device__ constexpr int image_rows(int L) { return (L + 31) / 32 * 32; }
 template <int D>
 __device__ __forceinline__ void load_q_image(const SnapParams& p, int b, int kvh, unsigned char* qimg, int tid, int nthr) {
     constexpr int CH = D * 2 / 16;
-    for (int c = tid; c < p.L * CH; c += nthr) {
-        const int rg = c / CH, ch = c - rg * CH;
+    for (int c = tid; c < image_rows(p.L) * CH; c += nthr) {
+        const int at = c / CH, ch = c - at * CH, rg = at < p.L ? at : at - 16;
         const int r = rg / p.W, l = rg - r * p.W;
         const u32x4 v = *reinterpret_cast<const u32x4*>(p.q + ((int64_t)(b * p.W + l) * p.H + kvh * p.g + r) * D + ch * 8);
-        *reinterpret_cast<u32x4*>(qimg + rg * (D * 2 + kQPad) + ch * 16) = v;
+        *reinterpret_cast<u32x4*>(qimg + at * (D * 2 + kQPad) + ch * 16) = v;
     }
 }
 
 // is (row rg, column col) masked?  The last W rows of every 8g-row chunk x the last W columns carry the W x W causal mask
 // of the reference (model.py:412-415, mis-aligned on purpose: bug-for-bug)
-__device__ __forceinline__ bool masked(const SnapParams& p, int rg, int col) {
-    const int chunk_rows = 8 * p.g;
-    const int mrow = rg % chunk_rows - (chunk_rows - p.W);
-    return col >= p.S || (mrow >= 0 && col - (p.S - p.W) > mrow);
+__device__ __forceinline__ bool masked(int S, int W, int chunk_rows, int rg, int col) {
+    const int mrow = rg % chunk_rows - (chunk_rows - W);
+    return col >= S || (mrow >= 0 && col - (S - W) > mrow);
 }
 
-constexpr int kSnapWaves = 8;               // wavefronts per workgroup of the two score kernels (they share table + Q image)
+// Wavefronts of a workgroup of the two score kernels, which share the table and the Q image: what a CU can hold.
+constexpr int score_waves(int D, int rt) { return D == 64 && rt <= 8 ? 16 : 8; }
+
+constexpr int stats_binades(int D, int rt) { return D == 128 && rt > 8 ? kTabSmall : kTabBinades; }
+
+// One row's scores of a batch where some lie outside the table or may be masked: w = columns col .. + 3 and col + 16 .. + 19.  Returns the sum
+// of exponentials against 0; those outside go to the wavefront's (m, Z) pair of the row, the four lanes of a row in turns.
+// (A call: in line it costs the hot path ten registers that it spills.)
+typedef __attribute__((address_space(3))) double lds_double;
+template <int BIN>
+__device__ __noinline__ double stats_slow(const lds_double* tab, lds_double* pair, unsigned int w0, unsigned int w1, unsigned int w2, unsigned int w3, int S, int W,
+                                          int chunk_rows, int rg, int col, int lc, bool tail) {
+    double m2 = -INFINITY, z2 = 0.0, t = 0.0;
+#pragma unroll 1
+    for (int i = 0; i < 8; ++i) {
+        const unsigned int w = i < 4 ? (i < 2 ? w0 : w1) : (i < 6 ? w2 : w3);
+        const float v = bf16_bits_to_f32((unsigned short)(i & 1 ? w >> 16 : w & 0xffffu));
+        if (tail && masked(S, W, chunk_rows, rg, col + (i >> 2) * 16 + (i & 3))) continue;      // (an integer modulo: off the hot path)
+        const int ti = tab_index<BIN>(v);
+        if (ti >= 0)
+            t += tab[ti];
+        else if (is_tiny(v))
+            t += exp_tiny(v);
+        else if (v > -INFINITY)
+            merge_mz(m2, z2, (double)v, 1.0);
+    }
+#pragma unroll 1
+    for (int q = 0; q < 4; ++q) {
+        if (lc == q && m2 > -INFINITY) {
+            double m = pair[0], Z = pair[1];
+            merge_mz(m, Z, m2, z2);
+            pair[0] = m;
+            pair[1] = Z;
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    return t;
+}
+// Two rows' probabilities of one column likewise, as two bf16
+template <int BIN>
+__device__ __noinline__ unsigned int accum_slow(const lds_double* tab, const lds_double* rowc, const lds_double* rowm, unsigned int w, int S, int W, int chunk_rows,
+                                                int row, int col, bool tail) {
+    float pr[2] = {0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const float v = bf16_bits_to_f32((unsigned short)(e ? w >> 16 : w & 0xffffu));
+        if (!(tail && masked(S, W, chunk_rows, row + e, col))) {
+            const int ti = tab_index<BIN>(v);
+            const double c2 = rowc[row + e];
+            if ((ti >= 0 || is_tiny(v)) && c2 > 0.0)
+                pr[e] = (float)((ti >= 0 ? tab[ti] : exp_tiny(v)) * c2);
+            else
+                pr[e] = (float)(exp_neg((double)v - rowm[(row + e) * 2]) * rowm[(row + e) * 2 + 1]);
+        }
+    }
+    return pack_bf16(pr[0], pr[1]);
+}
 
 // Pass 1: per (row, column chunk) the pair (m, Z), Z = sum over the chunk's columns of exp(s - m).  A lane owns ONE row
 // of every 16-row tile (rows <-> lanes lq) and 4 of a tile's 16 columns, and keeps the table sum of each of its rows
 // (reference 0) in registers: no cross-lane traffic until the end.  Out-of-table scores (rare) go to a per-wave (m, Z)
 // pair per row in LDS.  A wavefront takes 2 x 2 tiles at a time: two column groups share the query fragments, and the 16 table
-// gathers of a lane are in flight together -- tile by tile, each waiting for its products and then for its gathers, this kernel took
-// 150 us for 16 requests of 16 000 keys (8 kv heads of 64, 128 rows each), against 120.  Bound by LDS: 4 gathers of 8 random
-// bytes per lane and tile, about 7 cycles each, beside 8 for the fragments.
+// gathers of a lane are in flight together.  16 requests of 16 000 keys (8 kv heads of 64, 128 rows each): 92 us; 120 in two workgroups of
+// eight wavefronts a CU, each with its own table and image (12 us to fill), with the rare scores in line (spills) and 23 binades (0.8 % of
+// the batches are rare then); 150 tile by tile.  Bound by LDS, active for 69 % of the cycles: 4 gathers of 8 random bytes per lane and
+// tile, about 7 cycles each, beside 8 for the fragments; vector instructions 49 %.
 template <int D, bool FP8, int RTM>     // RTM: register-resident 16-row tiles (8 for g * W <= 128 rows, else kMaxRT)
-__global__ __launch_bounds__(64 * kSnapWaves, D == 64 && RTM == 8 ? 4 : 2) void snapkv_stats_kernel(const SnapParams p) {
-    __shared__ double tab[kTabN];
+__global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) void snapkv_stats_kernel(const SnapParams p) {
+    constexpr int kSnapWaves = score_waves(D, RTM), BIN = stats_binades(D, RTM);
+    __shared__ __attribute__((aligned(16))) double tab[Tab<BIN>::N];
     extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];   // Q image, then [waves][L][2] doubles
     const int chunk = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lq = lane & 15, lc = lane >> 4;
     unsigned char* qimg = dyn;
-    double* ms = reinterpret_cast<double*>(dyn + (size_t)p.L * (D * 2 + kQPad));
+    double* ms = reinterpret_cast<double*>(dyn + (size_t)image_rows(p.L) * (D * 2 + kQPad));
     double* sw = ms + (size_t)wave * p.L * 2;                 // this wave's (m, Z) of the out-of-table scores, per row
-    for (int i = tid; i < kTabN; i += 64 * kSnapWaves) tab[i] = g_exp_tab[i];
+    fill_table<BIN>(tab, tid, 64 * kSnapWaves, (chunk | kvh | b) == 0);
     load_q_image<D>(p, b, kvh, qimg, tid, 64 * kSnapWaves);
     for (int i = lane; i < p.L; i += 64) {
         sw[i * 2] = -INFINITY;
@@ -268,7 +363,7 @@ __global__ __launch_bounds__(64 * kSnapWaves, D == 64 && RTM == 8 ? 4 : 2) void 
                 unsigned int w[2][2][2];                             // scores rounded to bf16, two per dword: [row tile][column group]
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-                    const unsigned char* qp = qimg + ((two ? r0 + u : r0) * 16 + lq) * (D * 2 + kQPad) + lc * 16;
+                    const unsigned char* qp = qimg + lq * (D * 2 + kQPad) + lc * 16 + (r0 + u) * 16 * (D * 2 + kQPad);
                     f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
                     for (int ks = 0; ks < D / 32; ++ks) {
@@ -291,9 +386,9 @@ __global__ __launch_bounds__(64 * kSnapWaves, D == 64 && RTM == 8 ? 4 : 2) void 
 #pragma unroll
                     for (int c = 0; c < 2; ++c)
 #pragma unroll
-                        for (int h = 0; h < 2; ++h) o[u][c][h] = tab_offsets2(w[u][c][h], top, low);
+                        for (int h = 0; h < 2; ++h) o[u][c][h] = tab_offsets2<BIN>(w[u][c][h], top, low);
                 // hot path, no divergence: every score of the batch is in the table and no column can be masked
-                if (!tail && __builtin_amdgcn_ballot_w64(tab_outside(top, low)) == 0) {
+                if (!tail && __builtin_amdgcn_ballot_w64(tab_outside<BIN>(top, low)) == 0) {
                     double e[2][2][4];
 #pragma unroll
                     for (int u = 0; u < 2; ++u)
@@ -314,36 +409,8 @@ __global__ __launch_bounds__(64 * kSnapWaves, D == 64 && RTM == 8 ? 4 : 2) void 
                     for (int u = 0; u < 2; ++u) {
                         if (u == 1 && !two) continue;
                         const int rg = (r0 + u) * 16 + lq;
-                        double m2 = -INFINITY, z2 = 0.0, t = 0.0;    // this lane's out-of-table scores, its table sum
-#pragma unroll
-                        for (int c = 0; c < 2; ++c) {
-                            const unsigned int w0 = w[u][c][0], w1 = w[u][c][1];
-#pragma unroll 1
-                            for (int j = 0; j < 4; ++j) {
-                                const unsigned int wj = j < 2 ? w0 : w1;
-                                const float v = bf16_bits_to_f32((unsigned short)(j & 1 ? wj >> 16 : wj & 0xffffu));
-                                if (tail && masked(p, rg, col0 + c * 16 + lc * 4 + j)) continue;   // (an integer modulo: off the hot path)
-                                const int ti = tab_index(v);
-                                if (ti >= 0)
-                                    t += tab[ti];
-                                else if (is_tiny(v))
-                                    t += exp_tiny(v);
-                                else if (v > -INFINITY)
-                                    merge_mz(m2, z2, (double)v, 1.0);
-                            }
-                        }
-                        zt[r0 + u] += t;
-                        // the four lanes of a row take turns at the wave's LDS pair
-#pragma unroll 1
-                        for (int q = 0; q < 4; ++q) {
-                            if (lc == q && m2 > -INFINITY) {
-                                double m = sw[rg * 2], Z = sw[rg * 2 + 1];
-                                merge_mz(m, Z, m2, z2);
-                                sw[rg * 2] = m;
-                                sw[rg * 2 + 1] = Z;
-                            }
-                            __builtin_amdgcn_wave_barrier();
-                        }
+                        zt[r0 + u] += stats_slow<BIN>((lds_double*)tab, (lds_double*)(sw + rg * 2), w[u][0][0], w[u][0][1], w[u][1][0], w[u][1][1], p.S, p.W, 8 * p.g, rg,
+                                                      col0 + lc * 4, lc, tail);
                     }
                 }
             }
@@ -379,7 +446,9 @@ __global__ __launch_bounds__(64 * kSnapWaves, D == 64 && RTM == 8 ? 4 : 2) void 
     }
 }
 
-// Row statistics of the whole context from the per-chunk partials, once per row: (M, 1 / Z) overwrite chunk 0's slot.
+// Row statistics of the whole context from the per-chunk partials, once per row: (M, 1 / Z) overwrite chunk 0's slot.  Of a few chunks
+// every workgroup of the second pass makes them for itself (a launch is 4.8 us).
+constexpr int kFewChunks = 8;
 __global__ __launch_bounds__(256) void snapkv_finalize_kernel(const SnapParams p) {
     const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (row >= (int64_t)p.B * p.KH * p.L) return;
@@ -395,28 +464,34 @@ __global__ __launch_bounds__(256) void snapkv_finalize_kernel(const SnapParams p
 // 8-row group sum is three adds in a lane and one exchange between neighbouring groups of 16 lanes, in the reference's pairwise order.
 // Group G = 2 rt + half (lanes lc = 2 half) belongs to chunk G / g and pseudo head r' = G % g.  For even g a lane meets the same half
 // in every tile, so the accumulators r' = 2 i + half are its registers a[i] (template GH = g / 2, else 0: accumulators in LDS, updated
-// by the two halves in turn).  2 x 2 tiles at a time as in pass 1; one tile at a time and LDS accumulators for every g took 188 us
-// where this takes 150.
-template <int D, bool FP8, int GH>
-__global__ __launch_bounds__(64 * kSnapWaves, D == 64 ? 4 : 2) void snapkv_accum_kernel(const SnapParams p) {
+// by the two halves in turn).  2 x 2 tiles at a time as in pass 1.  118 us where pass 1 takes 92: vector instructions for 69 % of the
+// cycles, LDS 61 %.  (147 with the accumulators in scratch memory, where an address of either column group had put them, halves of packed
+// bf16 converted one by one, and workgroups of eight wavefronts; the gathers of a batch in front of the next one's scores: spills, 177.)
+template <int D, bool FP8, int GH, int RTM>
+__global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) void snapkv_accum_kernel(const SnapParams p) {
+    constexpr int kSnapWaves = score_waves(D, RTM), BIN = kTabBinades;
     constexpr int BT = GH >= 2 ? 2 : 1;                        // row tiles per batch
-    __shared__ double tab[kTabN];
+    __shared__ __attribute__((aligned(16))) double tab[Tab<BIN>::N];
     // Q image, [L] exp(-M) / Z, [L][2] (M, 1 / Z), GH == 0: [waves][g][32] floats
     extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];
     const int ctile = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lq = lane & 15, lc = lane >> 4;
     unsigned char* qimg = dyn;
-    double* rowc = reinterpret_cast<double*>(dyn + (size_t)p.L * (D * 2 + kQPad));
+    double* rowc = reinterpret_cast<double*>(dyn + (size_t)image_rows(p.L) * (D * 2 + kQPad));
     double* rowm = rowc + p.L;
     float* accs = reinterpret_cast<float*>(rowm + p.L * 2) + wave * p.g * 32;
     __shared__ int s_slow_rows;
     if (tid == 0) s_slow_rows = 0;
-    for (int i = tid; i < kTabN; i += 64 * kSnapWaves) tab[i] = g_exp_tab[i];
+    load_table<BIN>(tab, tid, 64 * kSnapWaves);
     load_q_image<D>(p, b, kvh, qimg, tid, 64 * kSnapWaves);
     __syncthreads();
     for (int row = tid; row < p.L; row += 64 * kSnapWaves) {
         const double* pp = p.partials + ((int64_t)(b * p.KH + kvh) * p.L + row) * p.nch * 2;
-        const double M = pp[0], rZ = pp[1];                   // left by snapkv_finalize_kernel
+        double M = pp[0], rZ = pp[1];                         // left by snapkv_finalize_kernel, or still one of a few chunks'
+        if (p.nch <= kFewChunks) {
+            for (int c = 1; c < p.nch; ++c) merge_mz(M, rZ, pp[c * 2], pp[c * 2 + 1]);
+            rZ = 1.0 / rZ;
+        }
         rowm[row * 2] = M;
         rowm[row * 2 + 1] = rZ;
         double c2 = 0.0;                                      // 0: exp(-M) is not representable -> the exp_neg path
@@ -472,8 +547,8 @@ __global__ __launch_bounds__(64 * kSnapWaves, D == 64 ? 4 : 2) void snapkv_accum
 #pragma unroll
                 for (int c = 0; c < 2; ++c)
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) o[u][c][h] = tab_offsets2(w[u][c][h], top, low);
-            if (fast_rows && !tail && __builtin_amdgcn_ballot_w64(tab_outside(top, low)) == 0) {
+                    for (int h = 0; h < 2; ++h) o[u][c][h] = tab_offsets2<BIN>(w[u][c][h], top, low);
+            if (fast_rows && !tail && __builtin_amdgcn_ballot_w64(tab_outside<BIN>(top, low)) == 0) {
                 // hot path, no divergence: table value x the row's exp(-M) / Z, softmax -> bf16 (model.py:416)
 #pragma unroll
                 for (int u = 0; u < BT; ++u) {
@@ -483,7 +558,7 @@ __global__ __launch_bounds__(64 * kSnapWaves, D == 64 ? 4 : 2) void snapkv_accum
                     for (int c = 0; c < 2; ++c)
 #pragma unroll
                         for (int h = 0; h < 2; ++h)
-                            pk[u][c][h] = pack_bf16((float)(tab_at(tab, o[u][c][h] & 0xffffu) * c2[2 * h]),
+                            pk[u][c][h] = round_pair((float)(tab_at(tab, o[u][c][h] & 0xffffu) * c2[2 * h]),
                                                     (float)(tab_at(tab, o[u][c][h] >> 16) * c2[2 * h + 1]));
                 }
             } else {
@@ -492,24 +567,9 @@ __global__ __launch_bounds__(64 * kSnapWaves, D == 64 ? 4 : 2) void snapkv_accum
 #pragma unroll
                     for (int c = 0; c < 2; ++c)
 #pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            float pr[2];
-#pragma unroll
-                            for (int e = 0; e < 2; ++e) {
-                                const int row = (rt + u) * 16 + lc * 4 + 2 * h + e;
-                                const float v = bf16_bits_to_f32((unsigned short)(e ? w[u][c][h] >> 16 : w[u][c][h] & 0xffffu));
-                                pr[e] = 0.f;
-                                if (!(tail && masked(p, row, col0 + c * 16 + lq))) {
-                                    const int ti = tab_index(v);
-                                    const double c2 = rowc[row];
-                                    if ((ti >= 0 || is_tiny(v)) && c2 > 0.0)
-                                        pr[e] = (float)((ti >= 0 ? tab[ti] : exp_tiny(v)) * c2);
-                                    else
-                                        pr[e] = (float)(exp_neg((double)v - rowm[row * 2]) * rowm[row * 2 + 1]);
-                                }
-                            }
-                            pk[u][c][h] = pack_bf16(pr[0], pr[1]);
-                        }
+                        for (int h = 0; h < 2; ++h)
+                            pk[u][c][h] = accum_slow<BIN>((lds_double*)tab, (lds_double*)rowc, (lds_double*)rowm, w[u][c][h], p.S, p.W, 8 * p.g, (rt + u) * 16 + lc * 4 + 2 * h,
+                                                          col0 + c * 16 + lq, tail);
             }
             // 8-row group sum in fp32, pairwise as a butterfly over consecutive rows, -> bf16 (:418)
 #pragma unroll
@@ -524,29 +584,29 @@ __global__ __launch_bounds__(64 * kSnapWaves, D == 64 ? 4 : 2) void snapkv_accum
                     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(t[c]), __float_as_uint(t[c]), false, false);
                     t[c] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
                 }
-                const unsigned int g2 = pack_bf16(t[0], t[1]);
+                const unsigned int g2 = round_pair(t[0], t[1]);
                 gs[u][0] = __uint_as_float(g2 << 16);
                 gs[u][1] = __uint_as_float(g2 & 0xffff0000u);
             }
         };
         if constexpr (GH > 0) {
             for (int rt = 0; rt < p.L / 16; rt += GH)          // one chunk of 8 g rows
-#pragma unroll
-                for (int i = 0; i < GH; i += BT) {
+                unrolled(std::make_integer_sequence<int, GH / BT>(), [&](auto ic) {      // (accumulators in registers: not a loop)
+                    constexpr int i = decltype(ic)::value * BT;
                     float gs[BT][2];
                     sums(rt + i, gs);
-#pragma unroll
-                    for (int u = 0; u < BT; ++u) {
-                        const unsigned int n2 = pack_bf16(a[0][i + u] + gs[u][0], a[1][i + u] + gs[u][1]);
+                    unrolled(std::make_integer_sequence<int, BT>(), [&](auto uc) {
+                        constexpr int u = decltype(uc)::value;
+                        const unsigned int n2 = round_pair(a[0][i + u] + gs[u][0], a[1][i + u] + gs[u][1]);
                         a[0][i + u] = __uint_as_float(n2 << 16);
                         a[1][i + u] = __uint_as_float(n2 & 0xffff0000u);
-                    }
-                }
+                    });
+                });
             // bf16 accumulators: aws[b][kvh*g + r'][col]; lane (lq, lc): half lc / 2, column group lc & 1
             const int col = col0 + (lc & 1) * 16 + lq;
 #pragma unroll
             for (int i = 0; i < GH; ++i) {
-                const float v = lc & 1 ? a[1][i] : a[0][i];
+                const float v0 = a[0][i], v1 = a[1][i], v = lc & 1 ? v1 : v0;      // (values: choosing between places puts both in scratch memory)
                 if (col < N)
                     p.aws[((int64_t)b * p.H + kvh * p.g + 2 * i + (lc >> 1)) * N + col] = (unsigned short)(__float_as_uint(v) >> 16);
             }
@@ -679,10 +739,19 @@ __global__ __launch_bounds__(1024) void snapkv_select_kernel(const unsigned shor
     sel[tid] = 0;
     if (tid < 32) misc[tid] = 0;
     __syncthreads();
-    for (int s = tid; s < N; s += 1024) {
-        const unsigned int k = ordered16(src[s]);
-        keys[s] = (unsigned short)k;
-        atomicAdd(&hist[k >> 4], 1u);
+    for (int s0 = tid; s0 < N; s0 += 8 * 1024) {              // (eight loads on their way)
+        unsigned short v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = src[min(s0 + j * 1024, N - 1)];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int s = s0 + j * 1024;
+            if (s < N) {
+                const unsigned int k = ordered16(v[j]);
+                keys[s] = (unsigned short)k;
+                atomicAdd(&hist[k >> 4], 1u);
+            }
+        }
     }
     __syncthreads();
     {   // thread t looks at the four bins 4 t .. 4 t + 3 counted from the top
@@ -799,32 +868,40 @@ __global__ __launch_bounds__(256) void snapkv_gather_kernel(const GatherParams p
     }
 }
 
+// A score kernel, whose LDS, with the table of BIN binades, is more than 64 KB
+template <auto Kernel, int BIN>
+int score_launch(dim3 grid, int waves, size_t lds, const SnapParams& p, hipStream_t st) {
+    static MdPerDeviceOnce once;
+    const int cap = 160 * 1024 - Tab<BIN>::N * 8 - 256;
+    if (once.first() && hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, cap) != hipSuccess) {
+        once.undo();
+        md_set_error("md_snapkv_select: hipFuncSetAttribute(%d B LDS) failed", cap);
+        return MD_ERR_LAUNCH;
+    }
+    hipLaunchKernelGGL(Kernel, grid, dim3(64 * waves), lds, st, p);
+    return MD_OK;
+}
+
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
-// Columns per workgroup of the two score kernels, in rounds of the eight wavefronts' 32 columns each.  A workgroup costs its rounds and two
-// more for the table, the query image and the merge; a CU holds one workgroup at a time, or two that together take 1.4 times as long as
-// one (128 rows of 64); the launch ends with the CU that has the most.  The even division with the least of that is within 0.6 % of
-// the best of 1..32 chunks over 320 sizes (4..512 pairs of request and head, 521..16 032 keys) and nowhere slower than whole chunks of
-// 2 048 columns, which lost to chunks sized for two workgroups per CU where only one fits: 52 requests of 700 keys, 8 queries a kv head
-// of 64, 162 us in one chunk, 188 in two rounds of 512 columns; 19 of 521, heads of 128, 165 and 187.  Whole selections, the two
-// workgroups' rule -> this one: 32 requests of 1 100 keys, 4 kv heads of 64, 160 -> 128 us; 4 of 16 000, 8 of 128, 169 -> 146; 25 of
-// 2 100, 8 of 64, 142 -> 121.
+// Columns per workgroup of the two score kernels, in rounds of the wavefronts' 32 columns each.  A CU holds one workgroup at a time, which
+// costs its rounds and two more for the table, the query image and the merge; the launch ends with the CU that has the most.  (Drawn for
+// workgroups of eight wavefronts over 320 sizes, within 0.6 % of the best number of chunks: 52 requests of 700 keys, 8 queries a kv head
+// of 64, 162 us in one chunk, 188 in two; 25 requests of 2 100, 8 of 64, 121.)
 int score_cols(int B, int KH, int L, int D, int ctx_len) {
     const int64_t pairs = (int64_t)B * KH;
-    const int all = std::max((ctx_len + 255) / 256, 1);              // (a size may be asked for any length)
-    const bool two = D == 64 && L <= 128;
+    const int round = 32 * score_waves(D, (L + 15) / 16), all = std::max((ctx_len + round - 1) / round, 1);        // (a size may be asked for any length)
     double least = 1e300;
     int best = all;
     for (int r = 1; r <= all; ++r) {
-        const int64_t on_cu = (pairs * ((all + r - 1) / r) + 255) / 256;
-        const double cost = (2 + r) * (two ? 1.4 * (double)(on_cu / 2) + (double)(on_cu % 2) : (double)on_cu);
+        const double cost = (double)(2 + r) * (double)((pairs * ((all + r - 1) / r) + 255) / 256);
         if (cost < least) {
             least = cost;
             best = r;
         }
     }
     const int n = (all + best - 1) / best;                           // ... and as even as whole rounds go
-    return (all + n - 1) / n * 256;
+    return (all + n - 1) / n * round;
 }
 
 // bytes of the partial sums: either head size (it is not among the sizes the workspace is asked for by)
@@ -919,60 +996,32 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
     unsigned short* scores = (unsigned short*)(ws + partials_b + aws_b);
 
     MD_CHECK_ARG(L <= 16 * kMaxRT, "md_snapkv_select: g * window = %d rows per kv head, at most %d supported", L, 16 * kMaxRT);
-    const size_t qimg_b = (size_t)L * (D * 2 + kQPad);
-    const size_t lds1 = qimg_b + (size_t)kSnapWaves * L * 2 * 8;
+    const size_t qimg_b = (size_t)image_rows(L) * (D * 2 + kQPad);
+    const int waves = score_waves(D, L / 16);
+    const size_t lds1 = qimg_b + (size_t)waves * L * 2 * 8;
     // accumulators in registers for g = 2, 4, 8 (a chunk of 8 g rows is then g / 2 whole tiles)
     const int gh = g == 2 || g == 4 || g == 8 ? g / 2 : 0;
-    const size_t lds2 = qimg_b + (size_t)L * 3 * 8 + (gh ? 0 : (size_t)kSnapWaves * g * 32 * 4);
-    if (lds1 + sizeof(double) * kTabN > 64 * 1024 || lds2 + sizeof(double) * kTabN > 64 * 1024) {
-        static MdPerDeviceOnce lds_once;
-        if (lds_once.first()) {
-            const int cap = 160 * 1024 - (int)sizeof(double) * kTabN - 256;
-            const void* ks[] = {reinterpret_cast<const void*>(&snapkv_stats_kernel<64, false, 8>),
-                                reinterpret_cast<const void*>(&snapkv_stats_kernel<64, false, kMaxRT>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, false, 0>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, false, 1>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, false, 2>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, false, 4>),
-                                reinterpret_cast<const void*>(&snapkv_stats_kernel<64, true, 8>),
-                                reinterpret_cast<const void*>(&snapkv_stats_kernel<64, true, kMaxRT>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, true, 0>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, true, 1>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, true, 2>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<64, true, 4>),
-                                reinterpret_cast<const void*>(&snapkv_stats_kernel<128, false, 8>),
-                                reinterpret_cast<const void*>(&snapkv_stats_kernel<128, false, kMaxRT>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, false, 0>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, false, 1>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, false, 2>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, false, 4>),
-                                reinterpret_cast<const void*>(&snapkv_stats_kernel<128, true, 8>),
-                                reinterpret_cast<const void*>(&snapkv_stats_kernel<128, true, kMaxRT>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, true, 0>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, true, 1>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, true, 2>),
-                                reinterpret_cast<const void*>(&snapkv_accum_kernel<128, true, 4>)};
-            for (const void* k : ks)
-                if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, cap) != hipSuccess) {
-                    lds_once.undo();
-                    md_set_error("md_snapkv_select: hipFuncSetAttribute(%d B LDS) failed", cap);
-                    return MD_ERR_LAUNCH;
-                }
-        }
-    }
-    hipLaunchKernelGGL(snapkv_tab_kernel, dim3((kTabN + 255) / 256), dim3(256), 0, st);
-#define MD_SNAP_LAUNCH(DD, FP)                                                                                   \
-    do {                                                                                                         \
-        if (L <= 128)                                                                                            \
-            hipLaunchKernelGGL((snapkv_stats_kernel<DD, FP, 8>), dim3(p.nch, KH, B), dim3(64 * kSnapWaves), lds1, st, p); \
-        else                                                                                                     \
-            hipLaunchKernelGGL((snapkv_stats_kernel<DD, FP, kMaxRT>), dim3(p.nch, KH, B), dim3(64 * kSnapWaves), lds1, st, p); \
-        hipLaunchKernelGGL(snapkv_finalize_kernel, dim3((unsigned)(((int64_t)B * KH * L + 255) / 256)), dim3(256), 0, st, p); \
-        const dim3 ag((N + p.cols - 1) / p.cols, KH, B);                                                 \
-        if (gh == 4) hipLaunchKernelGGL((snapkv_accum_kernel<DD, FP, 4>), ag, dim3(64 * kSnapWaves), lds2, st, p);      \
-        else if (gh == 2) hipLaunchKernelGGL((snapkv_accum_kernel<DD, FP, 2>), ag, dim3(64 * kSnapWaves), lds2, st, p); \
-        else if (gh == 1) hipLaunchKernelGGL((snapkv_accum_kernel<DD, FP, 1>), ag, dim3(64 * kSnapWaves), lds2, st, p); \
-        else hipLaunchKernelGGL((snapkv_accum_kernel<DD, FP, 0>), ag, dim3(64 * kSnapWaves), lds2, st, p);              \
+    const size_t lds2 = qimg_b + (size_t)L * 3 * 8 + (gh ? 0 : (size_t)waves * g * 32 * 4);
+    const dim3 sg(p.nch, KH, B), ag((N + p.cols - 1) / p.cols, KH, B);
+    const bool small = L <= 128;
+    int rc = MD_OK;
+#define MD_SNAP_STATS(DD, FP)                                                                                                \
+    rc = small ? score_launch<&snapkv_stats_kernel<DD, FP, 8>, stats_binades(DD, 8)>(sg, waves, lds1, p, st)                 \
+               : score_launch<&snapkv_stats_kernel<DD, FP, kMaxRT>, stats_binades(DD, kMaxRT)>(sg, waves, lds1, p, st)
+#define MD_SNAP_ACCUM(DD, FP, GG)                                                                                            \
+    rc = small ? score_launch<&snapkv_accum_kernel<DD, FP, GG, 8>, kTabBinades>(ag, waves, lds2, p, st)                      \
+               : score_launch<&snapkv_accum_kernel<DD, FP, GG, kMaxRT>, kTabBinades>(ag, waves, lds2, p, st)
+#define MD_SNAP_LAUNCH(DD, FP)                                                                                               \
+    do {                                                                                                                     \
+        MD_SNAP_STATS(DD, FP);                                                                                               \
+        if (rc != MD_OK) return rc;                                                                                          \
+        if (p.nch > kFewChunks)                                                                                              \
+            hipLaunchKernelGGL(snapkv_finalize_kernel, dim3((unsigned)(((int64_t)B * KH * L + 255) / 256)), dim3(256), 0, st, p); \
+        if (gh == 4) MD_SNAP_ACCUM(DD, FP, 4);                                                                               \
+        else if (gh == 2) MD_SNAP_ACCUM(DD, FP, 2);                                                                          \
+        else if (gh == 1) MD_SNAP_ACCUM(DD, FP, 1);                                                                          \
+        else MD_SNAP_ACCUM(DD, FP, 0);                                                                                       \
+        if (rc != MD_OK) return rc;                                                                                          \
     } while (0)
     if (D == 128) {
         if (fp8) MD_SNAP_LAUNCH(128, true); else MD_SNAP_LAUNCH(128, false);
@@ -980,6 +1029,8 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
         if (fp8) MD_SNAP_LAUNCH(64, true); else MD_SNAP_LAUNCH(64, false);
     }
 #undef MD_SNAP_LAUNCH
+#undef MD_SNAP_STATS
+#undef MD_SNAP_ACCUM
     MD_CHECK_LAUNCH("md_snapkv_select(scores)");
 
     const dim3 pgrid((N + kPoolCols - 1) / kPoolCols, KH, B);

@@ -58,3 +58,35 @@ def check_select(monkeypatch, B, KH, g, W, D, S, budget, pool, page, requests):
             keep = torch.cat([order, torch.arange(S - W, S)])
             got = draft[b * dpr:(b + 1) * dpr, :, :, h].transpose(0, 1).reshape(2, dpr * page, D)[:, :budget]
             assert torch.equal(got, rows[:, b, h][:, keep])
+
+
+@pytest.mark.parametrize("g,W,D", [(4, 32, 64), (8, 32, 128), (3, 16, 64)])
+@pytest.mark.parametrize("power", [-30, -22, -18, -13, 8])
+def test_scores_at_the_ends_of_the_table_of_exponentials(g, W, D, power):
+    """Scores of one size, 2^power times up to 8 (the tables begin at 2^-23 and 2^-14 and end at 2^9): positions and gathered rows are those of
+    the scores that came out, and equal probabilities come out equal -- tiny scores all have the same."""
+    from magicdec_amd import ops
+    S, budget, KH, page = 1060, 129, 2, 128
+    H, ppr = KH * g, -(-S // page)
+    gen = torch.Generator().manual_seed(power)
+    q = torch.zeros(W, H, D)
+    q[:, :, 0] = 2.0 ** power
+    keys = torch.randint(1, 9, (ppr * page,), generator=gen).float() * torch.where(torch.rand(ppr * page, generator=gen) < 0.5, -1.0, 1.0)
+    kv = torch.randn(ppr, 2, KH, page, D, generator=gen)
+    kv[:, 0] = 0
+    kv[:, 0, :, :, 0] = keys.view(ppr, 1, page)
+    kv, draft = kv.bfloat16(), torch.zeros(2, 2, page, KH, D, dtype=torch.bfloat16, device=DEV)
+    one = torch.arange(2, dtype=torch.int32, device=DEV)
+    idx, sc = ops.snapkv_select(q.bfloat16().to(DEV), kv.to(DEV), torch.arange(ppr, dtype=torch.int32, device=DEV), one * ppr, S, W, budget, 1, draft, one, one * 2,
+                                one[1:], ops.AttnWorkspace(DEV), return_scores=True, kv_layout="HND")
+    s = (keys[:S].double() * 2.0 ** power)
+    p = torch.softmax(s, 0)[:S - W]                          # (every row has the same scores, but for W x W masked ones of the last few)
+    for h in range(KH):
+        v = sc[0, h].float().cpu().double()
+        # the share of one key: 8 g rows of each chunk, weights and sums rounded to bf16 a few times; masked rows' sums lack up to W keys;
+        # weights below 2^-126 are no normal numbers
+        assert ((v / (g * W) - p).abs() <= p * (0.04 + 2 * W * p.max()) + 2.0 ** -120).all()
+        order = torch.sort(v, descending=True, stable=True).indices[:budget - W]
+        assert torch.equal(idx[0, h].cpu().long(), order)
+        for k in keys[:S - W].unique():
+            assert v[keys[:S - W] == k].unique().numel() == 1
