@@ -400,6 +400,12 @@ typedef struct md_fused_linear_args {
 int md_linear_fused_supported(int M, int N, int K, int epilogue);
 int md_linear_fused(const md_fused_linear_args* args, md_stream_t stream);
 
+/* md_linear_few (csrc/tilegemm.hip): the same of at most 16 rows on tiles of 16 columns, K % 256 == 0, with sums of another order.  Two
+ * differences: ssq_out is [M][N/16], of 16 columns each, and pro_ssq goes with every epilogue.  _supported: negative for no shape at all.  pro_ssq of either entry, and of
+ * md_linear_normed, may hold K / 32 or K / 16 partial sums (pro_tiles). */
+int md_linear_few_supported(int M, int N, int K, int epilogue);
+int md_linear_few(const md_fused_linear_args* args, md_stream_t stream);
+
 /* md_linear_fused_split: the K8b tile kernel with the K range ALSO split over S workgroups, for the deep narrow
  * products of a <= 64-row draft step (the 1B model's w2: N = 2048, K = 8192 -- Engine/SnapKV/model.py:451-455 followed by
  * the residual add and the next RMSNorm, :260-278,464-469).  A workgroup owns a (32|64)-row x (32|64)-column tile and K / S

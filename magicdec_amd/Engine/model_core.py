@@ -40,7 +40,7 @@ import torch.nn as nn
 from torch.nn import functional as F
 
 from .. import ops
-from .gemm_policy import prompt_over_block, prompt_rows
+from .gemm_policy import fused_mode, prompt_over_block, prompt_rows, use_few
 
 
 def find_multiple(n: int, k: int) -> int:
@@ -613,9 +613,12 @@ class Transformer(nn.Module):
         if how == "prompt":
             return self._prompt_linear(x2d if pro is None else pro.materialize(), pk, bias, swiglu)
         if how == "fused" and ops.fused_linear_supported(M, N, K):
-            if pro is not None and not swiglu:
+            # few rows: on finer tiles, which also take a norm in front of a head
+            few = (not swiglu and ops.few_linear_supported(M, N, K)
+                   and (use_few(M, N, K) or (pro is not None and resid is None and fused_mode() == "auto")))
+            if pro is not None and not swiglu and not few:
                 x2d, pro = pro.materialize(), None
-            return ops.fused_linear(x2d, pk, bias, swiglu=swiglu, resid=resid, want_ssq=want_ssq, pro=pro)
+            return ops.fused_linear(x2d, pk, bias, swiglu=swiglu, resid=resid, want_ssq=want_ssq, pro=pro, few=few)
         assert resid is None, "the residual epilogue exists on the fused kernel only"
         skinny = how in ("fused", "skinny", "block") and ops.linear_supported(M, N, K, swiglu)
         if how == "block" and ops.linear_block_supported(M, N, K, swiglu):
@@ -691,11 +694,23 @@ class Transformer(nn.Module):
                 and choose(M, N, K, False, False, True, kind, absorbs_norm) == "fused"
                 and ops.fused_linear_supported(M, N, K))
 
-    def _proj_add_norm(self, inp, lin, x, norm, group):
+    def _absorbs_norm(self, M, w, kind):
+        """Does the linear of weight `w` behind a norm ("qkv" | "swiglu" | "plain") take M rows with the norm still to be applied?"""
+        from .gemm_policy import choose, skinny_absorbs_norm
+        pk = self._packed.get(id(w))
+        if pk is None or w.dtype != torch.bfloat16:
+            return False
+        N, K = w.shape
+        how = choose(M, N, K, kind == "swiglu", False, True, kind, kind != "plain")
+        if how == "fused":
+            return ops.few_linear_supported(M, N, K) if kind == "plain" else ops.fused_linear_supported(M, N, K)
+        return how == "skinny" and kind != "qkv" and ops.linear_supported(M, N, K, kind == "swiglu") and skinny_absorbs_norm(M)
+
+    def _proj_add_norm(self, inp, lin, x, norm, group, then=None):
         """Output projection of a sub-layer (wo / w2), the residual add and the RMSNorm for the next sub-layer:
         (h, y) = (x + sum_ranks(inp . W^T), rmsnorm(h) * w).  Without tensor parallelism and on a launch-bound shape the
         projection and the residual add are one launch (md_linear_fused, MD_FL_RESID) and y is returned as an
-        `ops.DeferredNorm`; otherwise the projection, then `_reduce_add_norm` (collective + fused add + norm)."""
+        `ops.DeferredNorm` (also on a deep one of few rows, if `then`, the weight that y goes to and its kind, takes such); otherwise the projection, then `_reduce_add_norm` (collective + fused add + norm)."""
         if group is None and x.is_contiguous() and self._fused_here(inp, lin.weight, "resid"):
             # the norm is DEFERRED: the residual epilogue leaves the per-row partial sums of squares, and the linear that
             # consumes the normalised rows (w1|w3, the next layer's wqkv) applies rmsnorm on the fly; a consumer that
@@ -708,6 +723,13 @@ class Transformer(nn.Module):
             w = lin.weight
             M, K = inp.shape
             pk = self._packed.get(id(w))
+            if (pk is not None and w.dtype == torch.bfloat16 and inp.stride(-1) == 1 and x.is_contiguous() and then is not None
+                    and M <= 4 and use_few(M, w.shape[0], K) and (use_split(M, w.shape[0], K, "resid") or choose(M, w.shape[0], K, False, False, True, "resid") == "skinny")
+                    and self._absorbs_norm(M, *then)):
+                # a row or a few of a deep product: one launch, its norm in the next product's.  (To four rows, which that one stages
+                # in one instruction: at 16 rows of the 7B model its norm costs more than the launch, 322 / 331 us of a two-layer step)
+                h, ssq = ops.fused_linear(inp, pk, lin.bias, resid=x, want_ssq=True, few=True)
+                return h, ops.DeferredNorm(h, ssq, norm.weight, norm.eps)
             if (pk is not None and w.dtype == torch.bfloat16 and inp.stride(-1) == 1
                     and use_split(M, w.shape[0], K, "resid") and ops.fused_split_supported(M, w.shape[0], K)):
                 # deep narrow projection of a draft step (the 1B w2): the tile kernel with K split over workgroups; its
@@ -766,10 +788,12 @@ class Transformer(nn.Module):
         for i, layer in enumerate(layers):
             o = attn_fn(i, layer, y, n)
             x, y = self._proj_add_norm(o.view(o.shape[0], -1), layer.attention.wo, x, layer.ffn_norm,
-                                       layer.attention.process_group)
+                                       layer.attention.process_group, (self._w13[i], "swiglu"))
             act = self._linear(y, None, swiglu_w13=(self._w13[i], self._s13[i]))
-            nxt = layers[i + 1].attention_norm if i + 1 < len(layers) else self.norm
-            x, y = self._proj_add_norm(act, layer.feed_forward.w2, x, nxt, layer.feed_forward.process_group)
+            last = i + 1 == len(layers)
+            nxt = self.norm if last else layers[i + 1].attention_norm
+            then = (self.output.weight, "plain") if last else (layers[i + 1].attention.wqkv.weight, "qkv")
+            x, y = self._proj_add_norm(act, layer.feed_forward.w2, x, nxt, layer.feed_forward.process_group, None if self.skip_head and last else then)
         if self.skip_head:
             return None
         if head_rows is not None:
@@ -823,7 +847,8 @@ class Transformer(nn.Module):
                     yin, self._packed[id(att.wqkv.weight)], att.wqkv.bias, c.n_head, c.n_local_heads, c.head_dim, n,
                     offsets, self.rope_table, cache, tab.indices, tab.indptr, tab.last_page_len, cache2,
                     tab2.indices if tab2 else None, tab2.indptr if tab2 else None,
-                    tab2.last_page_len if tab2 else None, kv_scales=scales, kv_layout=layout, pro=pro)
+                    tab2.last_page_len if tab2 else None, kv_scales=scales, kv_layout=layout, pro=pro,
+                    few=use_few(*yin.shape[:1], *att.wqkv.weight.shape))
             else:
                 if pro is not None:
                     y = pro.materialize()

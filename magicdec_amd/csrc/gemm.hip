@@ -640,8 +640,8 @@ int linear_impl(const void* x, int64_t ldx, const void* w, int w_dtype, int w_pa
         MD_CHECK_ARG(w_dtype == MD_W_BF16, "md_linear_normed: bf16 weights only");
         MD_CHECK_ARG(pro_w && (((uintptr_t)pro_w) & 15) == 0 && (((uintptr_t)pro_ssq) & 3) == 0,
                      "md_linear_normed: the norm weight must be 16-byte aligned");
-        MD_CHECK_ARG(pro_tiles > 0 && pro_tiles * 32 == K,
-                     "md_linear_normed: ssq must hold K / 32 = %d partial sums per row, got %d", K / 32, pro_tiles);
+        MD_CHECK_ARG(pro_tiles > 0 && (pro_tiles * 32 == K || pro_tiles * 16 == K),
+                     "md_linear_normed: ssq must hold K / 32 = %d partial sums per row (or twice as many), got %d", K / 32, pro_tiles);
         p.pro_ssq = pro_ssq;
         p.pro_w = (const bf16_t*)pro_w;
         p.pro_eps = pro_eps;

@@ -50,6 +50,8 @@
 // kernel behind it; K = 8192 or M = 256 with many column tiles: slower than the library -- those shapes stay there.
 #include "md_common.h"
 
+#include <type_traits>
+
 unsigned int* md_page_overflow_counter_device();   // kvops.hip: rows dropped beyond a request's mapped pages
 
 namespace {
@@ -170,6 +172,66 @@ __device__ __forceinline__ int64_t kv_elem_offset(const KvTable& t, int b, int r
     return hnd ? base + ((int64_t)h * page_size + slot) * D + d : base + ((int64_t)slot * KH + h) * D + d;
 }
 
+// The epilogues of columns n, n + 1 of row gm, whose finished sums (with the bias) are s; q: the sum of squares of what a residual
+// epilogue stores
+template <int EPI, bool FP8>
+__device__ __forceinline__ void finish_pair(const TileParams& p, int gm, int n, const f32x2& s, float& q) {
+    if constexpr (EPI == FL_XIELU) {                  // fp32 accumulator -> activation -> one rounding
+        const Xielu f_act(p.act);
+        *reinterpret_cast<unsigned int*>(p.out + (int64_t)gm * p.ldo + n) = pack2(f_act(s[0]), f_act(s[1]));
+        return;
+    }
+    // the linear's own output, rounded to bf16 as nn.Linear returns it
+    const float o0 = bf16_to_f32(f32_to_bf16(s[0])), o1 = bf16_to_f32(f32_to_bf16(s[1]));
+    if constexpr (EPI == FL_NONE) {
+        *reinterpret_cast<unsigned int*>(p.out + (int64_t)gm * p.ldo + n) = pack2(o0, o1);
+    } else if constexpr (EPI == FL_RESID) {
+        const unsigned int rv = *reinterpret_cast<const unsigned int*>(p.resid + (int64_t)gm * p.ldr + n);
+        const float r0 = __uint_as_float(rv << 16), r1 = __uint_as_float(rv & 0xffff0000u);
+        const float h0 = bf16_to_f32(f32_to_bf16(r0 + o0)), h1 = bf16_to_f32(f32_to_bf16(r1 + o1));
+        *reinterpret_cast<unsigned int*>(p.out + (int64_t)gm * p.ldo + n) = pack2(h0, h1);
+        q = h0 * h0 + h1 * h1;
+    } else if constexpr (EPI == FL_ROPE_APPEND) {
+        const int HD = p.H * p.D, KD = p.KH * p.D;
+        const int b = gm / p.rows_per_req, jrow = gm - b * p.rows_per_req;
+        const bool is_v = n >= HD + KD;
+        float y0 = o0, y1 = o1;
+        if (!is_v) {
+            int pos = p.offsets[b] + jrow;
+            pos = pos < 0 ? 0 : (pos >= p.max_pos ? p.max_pos - 1 : pos);
+            const int d = (n < HD ? n : n - HD) % p.D;          // even: (d, d+1) is one interleaved pair
+            const f32x2 cs = *reinterpret_cast<const f32x2*>(p.cos_sin + (int64_t)pos * p.D + d);
+            y0 = __fsub_rn(__fmul_rn(o0, cs[0]), __fmul_rn(o1, cs[1]));
+            y1 = __fadd_rn(__fmul_rn(o1, cs[0]), __fmul_rn(o0, cs[1]));
+        }
+        if (n < HD) {
+            *reinterpret_cast<unsigned int*>(p.out + (int64_t)gm * p.ldo + n) = pack2(y0, y1);
+            return;
+        }
+        const int nn = is_v ? n - HD - KD : n - HD;
+        const int h = nn / p.D, d = nn - h * p.D;
+        const int64_t half = (int64_t)p.page_size * KD;
+        bool over;
+        const int64_t d1 = kv_elem_offset(p.t1, b, p.rows_per_req, jrow, p.page_size, p.KH, p.D, h, d, p.hnd != 0, &over);
+        // one count per dropped row (as md_rope_append): the thread holding the row's first K pair reports it
+        if (over && !is_v && nn == 0) atomicAdd(p.overflow, 1u);
+        // what the cache receives is the bf16 tensor k / v of the reference (RoPE output rounded to bf16) -- an fp8
+        // page quantises THAT value, not the fp32 rotation result (md_rope_append does the same)
+        y0 = bf16_to_f32(f32_to_bf16(y0));
+        y1 = bf16_to_f32(f32_to_bf16(y1));
+        if (d1 >= 0) {
+            float inv = 1.f;
+            if constexpr (FP8) inv = 1.0f / (is_v ? p.v_scale[h] : p.k_scale[h]);
+            store_pair<FP8>(p.t1.cache, d1 + (is_v ? half : 0), y0, y1, inv);
+        }
+        if (p.t2.cache) {                                 // second cache (self-speculation draft cache): bf16, NHD
+            const int64_t d2 = kv_elem_offset(p.t2, b, p.rows_per_req, jrow, p.page_size, p.KH, p.D, h, d, false, &over);
+            if (over && !is_v && nn == 0) atomicAdd(p.overflow, 1u);
+            if (d2 >= 0) store_pair<false>(p.t2.cache, d2 + (is_v ? half : 0), y0, y1, 1.f);
+        }
+    }
+}
+
 // NW = wavefronts per workgroup = K slices (8, or 16 when no CU gets a second workgroup: the bytes a CU
 // has in flight -- NW x (8 KiB of W + 8 KiB of x) -- are what its ingest rate is made of, ~50 GB/s per CU at NW = 8);
 // WNT = stream W with non-temporal loads (one M tile: every weight byte is read once) or keep it in L2 for the sibling
@@ -197,6 +259,9 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
     // behind them, and the workgroup meets at a bare s_barrier (no vmcnt(0) drain); the norm weights of a chunk are
     // unpacked once, both roundings are one v_cvt_pk_bf16_f32.
     constexpr bool kNewPro = PRO && MT * NT > 1;
+    // The same for few rows (one row of 6144 x 4096 + rope behind 256 partial sums 15.3 us with the scales in front of the first loads)
+    constexpr bool kFewPro = PRO && AI < 8;
+    constexpr int kFewParts = 16;                         // partial sums a lane has in flight, of every 16th (more: one after the other)
     constexpr int kRD = kNewPro ? 4 : 8;                  // W fragments in flight per column tile and wavefront
     constexpr int kWaveLdsT = MT * kWaveLds;               // wave-private activation image of 32 x MT rows
     static_assert(MT * NT * 4096 <= kWaveLdsT, "the partial tiles of a wave must fit its activation image");
@@ -269,7 +334,16 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
         // them, and its wait (vmcnt(0)) drains the whole prefetch
         __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (PRO && !kNewPro) {
+    float fv[kFewParts];
+    if constexpr (kFewPro) {
+        if (tid < 64 * AI) {                              // wave-uniform: 16 lanes a row
+            const float* from = p.pro_ssq + (int64_t)min(tid >> 4, p.M - 1) * p.pro_tiles;
+#pragma unroll
+            for (int u = 0; u < kFewParts; ++u) fv[u] = from[min((tid & 15) + 16 * u, p.pro_tiles - 1)];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (PRO && !kNewPro && !kFewPro) {
         float* rstd_lds = reinterpret_cast<float*>(lds + NW * kWaveLdsT);
         if (tid < 512) {
 #pragma unroll
@@ -396,6 +470,27 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
         // read (and no lgkmcnt wait) per staged row
         my_rs = rstd_lds[4 * (lane & 15) + (lane >> 4)];
     }
+    if constexpr (kFewPro) {
+        float* rstd_lds = reinterpret_cast<float*>(lds + NW * kWaveLdsT);
+        if (tid < 64 * AI) {
+            const int part = tid & 15;
+            float t = 0.f;
+#pragma unroll
+            for (int u = 0; u < kFewParts; ++u)
+                if (part + 16 * u < p.pro_tiles) t += fv[u];
+            for (int i = part + 16 * kFewParts; i < p.pro_tiles; i += 16) t += p.pro_ssq[(int64_t)min(tid >> 4, p.M - 1) * p.pro_tiles + i];
+            t += __shfl_xor(t, 1);
+            t += __shfl_xor(t, 2);
+            t += __shfl_xor(t, 4);
+            t += __shfl_xor(t, 8);
+            if (part == 0) rstd_lds[tid >> 4] = rsqrtf(t / (float)p.K + p.pro_eps);      // md_rmsnorm's expression
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the LDS writes only: the global loads stay in flight
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < AI; ++i) rs8[i] = rstd_lds[4 * i + ar];
+    }
     const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
     const unsigned char* a_frag = my_lds + j * kPitch + kh * 16;
     MD_TS(1);                                     // every first load is issued
@@ -501,68 +596,16 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
                 s[1] += bf16_to_f32(p.bias[n + 1]);
             }
             if (gm >= p.M) continue;
-            if constexpr (EPI == FL_XIELU) {                  // fp32 accumulator -> activation -> one rounding
-                const Xielu f_act(p.act);
-                *reinterpret_cast<unsigned int*>(p.out + (int64_t)gm * p.ldo + n) = pack2(f_act(s[0]), f_act(s[1]));
-                continue;
-            }
-            // the linear's own output, rounded to bf16 as nn.Linear returns it
-            const float o0 = bf16_to_f32(f32_to_bf16(s[0])), o1 = bf16_to_f32(f32_to_bf16(s[1]));
-            if constexpr (EPI == FL_NONE) {
-                *reinterpret_cast<unsigned int*>(p.out + (int64_t)gm * p.ldo + n) = pack2(o0, o1);
-            } else if constexpr (EPI == FL_RESID) {
-                const unsigned int rv = *reinterpret_cast<const unsigned int*>(p.resid + (int64_t)gm * p.ldr + n);
-                const float r0 = __uint_as_float(rv << 16), r1 = __uint_as_float(rv & 0xffff0000u);
-                const float h0 = bf16_to_f32(f32_to_bf16(r0 + o0)), h1 = bf16_to_f32(f32_to_bf16(r1 + o1));
-                *reinterpret_cast<unsigned int*>(p.out + (int64_t)gm * p.ldo + n) = pack2(h0, h1);
+            float q = 0.f;
+            finish_pair<EPI, FP8>(p, gm, n, s, q);
+            if constexpr (EPI == FL_RESID) {
                 if (p.ssq_out) {
                     // sum of squares of this tile's 32 columns of row gm (the 16 lanes of the row, fixed butterfly order)
-                    float q = h0 * h0 + h1 * h1;
                     q += __shfl_xor(q, 1);
                     q += __shfl_xor(q, 2);
                     q += __shfl_xor(q, 4);
                     q += __shfl_xor(q, 8);
                     if (cp == 0) p.ssq_out[(int64_t)gm * p.n_tiles + tn] = q;
-                }
-            } else {                                            // FL_ROPE_APPEND
-                const int HD = p.H * p.D, KD = p.KH * p.D;
-                const int b = gm / p.rows_per_req, jrow = gm - b * p.rows_per_req;
-                const bool is_v = n >= HD + KD;
-                float y0 = o0, y1 = o1;
-                if (!is_v) {
-                    int pos = p.offsets[b] + jrow;
-                    pos = pos < 0 ? 0 : (pos >= p.max_pos ? p.max_pos - 1 : pos);
-                    const int d = (n < HD ? n : n - HD) % p.D;          // even: (d, d+1) is one interleaved pair
-                    const f32x2 cs = *reinterpret_cast<const f32x2*>(p.cos_sin + (int64_t)pos * p.D + d);
-                    y0 = __fsub_rn(__fmul_rn(o0, cs[0]), __fmul_rn(o1, cs[1]));
-                    y1 = __fadd_rn(__fmul_rn(o1, cs[0]), __fmul_rn(o0, cs[1]));
-                }
-                if (n < HD) {
-                    *reinterpret_cast<unsigned int*>(p.out + (int64_t)gm * p.ldo + n) = pack2(y0, y1);
-                    continue;
-                }
-                const int nn = is_v ? n - HD - KD : n - HD;
-                const int h = nn / p.D, d = nn - h * p.D;
-                const int64_t half = (int64_t)p.page_size * KD;
-                bool over;
-                const int64_t d1 = kv_elem_offset(p.t1, b, p.rows_per_req, jrow, p.page_size, p.KH, p.D, h, d, p.hnd != 0,
-                                                  &over);
-                // one count per dropped row (as md_rope_append): the thread holding the row's first K pair reports it
-                if (over && !is_v && nn == 0) atomicAdd(p.overflow, 1u);
-                // what the cache receives is the bf16 tensor k / v of the reference (RoPE output rounded to bf16) -- an fp8
-                // page quantises THAT value, not the fp32 rotation result (md_rope_append does the same)
-                y0 = bf16_to_f32(f32_to_bf16(y0));
-                y1 = bf16_to_f32(f32_to_bf16(y1));
-                if (d1 >= 0) {
-                    float inv = 1.f;
-                    if constexpr (FP8) inv = 1.0f / (is_v ? p.v_scale[h] : p.k_scale[h]);
-                    store_pair<FP8>(p.t1.cache, d1 + (is_v ? half : 0), y0, y1, inv);
-                }
-                if (p.t2.cache) {                                 // second cache (self-speculation draft cache): bf16, NHD
-                    const int64_t d2 = kv_elem_offset(p.t2, b, p.rows_per_req, jrow, p.page_size, p.KH, p.D, h, d, false,
-                                                      &over);
-                    if (over && !is_v && nn == 0) atomicAdd(p.overflow, 1u);
-                    if (d2 >= 0) store_pair<false>(p.t2.cache, d2 + (is_v ? half : 0), y0, y1, 1.f);
                 }
             }
         }
@@ -570,6 +613,164 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
 #ifdef MD_TILE_TIMING
     ts_flush();
 #endif
+}
+
+// ---- md_linear_few: at most 16 rows, 16 columns a workgroup ------------------------------------------------------------------
+// A column tile of 32 is coarse where a step has a row or a few: 768 x 3 072 is 24 workgroups, 4 096 columns 128 of 256 CUs, and 28 672 are 896
+// tiles, which leave half the CUs with four and half with three.  v_mfma_f32_16x16x32 takes 16 columns of the same streaming layout
+// (256-byte pieces of a fragment, whole lines), so that twice the workgroups share the weight, K is split over 8 or 16 wavefronts as in the
+// tile kernel, and no K split over workgroups is left to combine.  One row, us, the 32-column form / this one: 768 x 3 072 7.5 / 5.8,
+// 3 584 x 3 584 10.2 / 8.2, 2 048 x 5 632 11.1 / 8.6, 4 096 x 14 336 27.4 / 22.9 (5.1 TB/s); wider than a round of the chip the fixed part of
+// twice the workgroups shows: 28 672 x 4 096 43.7 / 46.3.
+// The partial sums of squares of a residual epilogue are of 16 columns each.  A gated tile is 8 columns of w1 and the same 8 of w3.
+constexpr int kFewLds = 16 * kPitch;               // a wavefront's activation image
+
+template <int EPI, bool FP8, int NW, bool PRO, int AI>
+__global__ __launch_bounds__(64 * NW, 4) void few_gemm_kernel(const TileParams p) {
+    constexpr int R = 4 * AI, kRD = 8;             // staged rows, W fragments in flight
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];       // NW x kFewLds, 16 floats
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, q = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tn = blockIdx.x, half = tn & 1;
+    const int nsteps = p.K / (32 * NW), k0 = wave * nsteps * 32;
+    // fragment s: columns 16 half + j (gated: 8 half + j of w1 and of w3) of k0 + 32 s + 8 q .. + 7
+    constexpr bool GATED = EPI == FL_SWIGLU;
+    const int col = GATED ? half * 8 + (j & 7) + (j >> 3) * 16 : half * 16 + j;
+    const bf16_t* wbase = p.w + ((int64_t)(tn >> 1) * (p.K >> 4) + (k0 >> 4)) * 512;
+    const unsigned woff = (unsigned)((q >> 1) * 512 + (col + 32 * (q & 1)) * 8);
+    unsigned char* my_lds = lds + wave * kFewLds;
+    const int ar = lane >> 4, c16 = lane & 15;
+    const unsigned char* xbase = reinterpret_cast<const unsigned char*>(p.x + k0);
+    unsigned int xrow[AI];
+#pragma unroll
+    for (int i = 0; i < AI; ++i) xrow[i] = (unsigned int)min(4 * i + ar, p.M - 1) * (unsigned int)p.ldx * 2u;   // rows >= M re-read row M - 1
+    // PRO: a row's partial sums first, four a lane on their way in front of everything else
+    constexpr int RW = (R + NW - 1) / NW;          // rows a wavefront adds up
+    float pv[RW][4];
+    if constexpr (PRO) {
+#pragma unroll
+        for (int u = 0; u < RW; ++u) {
+            const float* from = p.pro_ssq + (int64_t)min(wave + u * NW, p.M - 1) * p.pro_tiles;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pv[u][i] = from[min(lane + 64 * i, p.pro_tiles - 1)];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    u32x4 xa[AI], nwv = {0u, 0u, 0u, 0u};
+    auto a_load = [&](int c) {
+        const int klen = min(nsteps - c * 4, 4) * 32;
+        const unsigned int cc = (unsigned int)(c * kKC + (c16 * 8 < klen ? c16 : 0) * 8) * 2u;
+        if constexpr (PRO) nwv = *reinterpret_cast<const u32x4*>(reinterpret_cast<const unsigned char*>(p.pro_w + k0) + cc);
+#pragma unroll
+        for (int i = 0; i < AI; ++i) xa[i] = *reinterpret_cast<const u32x4*>(xbase + (xrow[i] + cc));
+    };
+    float rs[AI];
+    auto a_store = [&]() {
+#pragma unroll
+        for (int i = 0; i < AI; ++i) {
+            u32x4 v = xa[i];
+            if constexpr (PRO) {
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {       // y = bf16(bf16(h * rstd) * weight), as in the tile kernel
+                    const f32x2 t = unpack2(v[w]) * f32x2{rs[i], rs[i]};
+                    unsigned int pk;
+                    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(pk) : "v"(t[0]), "v"(t[1]));
+                    const f32x2 o = unpack2(pk) * unpack2(nwv[w]);
+                    v[w] = pack2(o[0], o[1]);
+                }
+            }
+            *reinterpret_cast<u32x4*>(my_lds + (4 * i + ar) * kPitch + c16 * 16) = v;
+        }
+    };
+    a_load(0);
+    bf16x8 wr[kRD];
+    auto w_load = [&](int s) {
+        const u32x4 v = ld_w<true>(wbase + min(s, nsteps - 1) * 1024 + woff);
+        return *reinterpret_cast<const bf16x8*>(&v);
+    };
+#pragma unroll
+    for (int s = 0; s < kRD; ++s) wr[s] = w_load(s);
+    if constexpr (PRO) {
+        float* rstd = reinterpret_cast<float*>(lds + NW * kFewLds);
+#pragma unroll
+        for (int u = 0; u < RW; ++u) {
+            const int r = wave + u * NW;
+            float t = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (lane + 64 * i < p.pro_tiles) t += pv[u][i];
+            for (int i = lane + 256; i < p.pro_tiles; i += 64) t += p.pro_ssq[(int64_t)min(r, p.M - 1) * p.pro_tiles + i];
+            t = wave_reduce_sum(t);
+            if (lane == 0 && r < R) rstd[r] = rsqrtf(t / (float)p.K + p.pro_eps);      // md_rmsnorm's expression
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // the LDS writes only: the global loads stay in flight
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < AI; ++i) rs[i] = rstd[4 * i + ar];
+    }
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    const unsigned char* a_frag = my_lds + j * kPitch + q * 16;
+    const int nchunk = (nsteps + 3) >> 2;
+    auto chunk = [&](int c, auto odd) {             // the ring holds two chunks: fragments 4 odd .. + 3 are this one's
+        constexpr int o = decltype(odd)::value * 4;
+        a_store();
+        asm volatile("" ::: "memory");              // (the image is written and read as different types)
+        if (c + 1 < nchunk) a_load(c + 1);
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+            const bool live = c * 4 + st < nsteps;                    // wave-uniform; only the last chunk can be short
+            bf16x8 b = wr[o + st];
+            wr[o + st] = w_load(c * 4 + st + kRD);
+            bf16x8 a = *reinterpret_cast<const bf16x8*>(a_frag + st * 64);
+            if (!live) a = b = zero8;                                 // (stale LDS may hold NaN)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a, acc, 0, 0, 0);
+        }
+        asm volatile("" ::: "memory");
+    };
+#pragma unroll 1
+    for (int c = 0; c < nchunk; c += 2) {
+        chunk(c, std::integral_constant<int, 0>());
+        if (c + 1 < nchunk) chunk(c + 1, std::integral_constant<int, 1>());
+    }
+    // acc[r] = row j, column 4 q + r: the wavefronts' tiles to LDS, added in their order
+    *reinterpret_cast<f32x4*>(my_lds + (j * 16 + q * 4) * 4) = acc;
+    __syncthreads();
+    if (tid >= 128) return;
+    const int gm = tid >> 3, cp = tid & 7;
+    auto sum1 = [&](int c) {
+        float t = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) t += *reinterpret_cast<const float*>(lds + w * kFewLds + (gm * 16 + c) * 4);
+        return t;
+    };
+    if constexpr (GATED) {
+        const int i = (tn >> 1) * 16 + half * 8 + cp;
+        const float a1 = sum1(cp), a3 = sum1(8 + cp);
+        const float v = p.gelu ? gelu_tanh(a1) * a3 : silu_bf16(bf16_to_f32(f32_to_bf16(a1))) * bf16_to_f32(f32_to_bf16(a3));
+        if (gm < p.M && i < p.N >> 1) p.out[(int64_t)gm * p.ldo + i] = f32_to_bf16(v);
+    } else {
+        const int n = tn * 16 + 2 * cp;
+        f32x2 s = {0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NW; ++w) s += *reinterpret_cast<const f32x2*>(lds + w * kFewLds + (gm * 16 + 2 * cp) * 4);
+        if (p.bias) {
+            s[0] += bf16_to_f32(p.bias[n]);
+            s[1] += bf16_to_f32(p.bias[n + 1]);
+        }
+        if (gm >= p.M) return;
+        float sq = 0.f;
+        finish_pair<EPI, FP8>(p, gm, n, s, sq);
+        if constexpr (EPI == FL_RESID) {
+            if (p.ssq_out) {
+                sq += __shfl_xor(sq, 1);
+                sq += __shfl_xor(sq, 2);
+                sq += __shfl_xor(sq, 4);
+                if (cp == 0) p.ssq_out[(int64_t)gm * (p.N >> 4) + tn] = sq;
+            }
+        }
+    }
 }
 
 template <int EPI, bool FP8, int NW, bool WNT, bool PRO, int MT = 1, int NT = 1, int AI = 8>
@@ -642,6 +843,38 @@ int launch_tile(const TileParams& p, hipStream_t st) {
         if (p.pro_ssq) return launch_tile_pro<EPI, FP8, true>(p, st);
     }
     return launch_tile_pro<EPI, FP8, false>(p, st);
+}
+
+template <int EPI, bool FP8, int NW, bool PRO, int AI>
+int launch_few_cfg(const TileParams& p, hipStream_t st) {
+    constexpr int lds = NW * kFewLds + 64;
+    auto k = few_gemm_kernel<EPI, FP8, NW, PRO, AI>;
+    static MdPerDeviceOnce once;
+    if (lds > 64 * 1024 && once.first() &&
+        hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) {
+        once.undo();
+        md_set_error("md_linear_few: hipFuncSetAttribute(%d B LDS) failed", lds);
+        return MD_ERR_LAUNCH;
+    }
+    hipLaunchKernelGGL(k, dim3(p.N / 16), dim3(64 * NW), lds, st, p);
+    return MD_OK;
+}
+
+// (Sixteen wavefronts are slower everywhere: 4 096 x 14 336 24.1 us, eight 22.9; 2 048 x 2 048 6.4, 5.3.)
+template <int EPI, bool FP8, bool PRO>
+int launch_few_pro(const TileParams& p, hipStream_t st) {
+    // a head behind a deferred norm, wide: 32-column tiles, whose fixed part is paid half as often (32 000 x 4 096 46 us, 51.6 on 16
+    // columns; x 768 11.1 and 20.5)
+    if constexpr (EPI == FL_NONE && PRO) {
+        if (p.N > 4096) return p.M <= 4 ? launch_tile_cfg<EPI, FP8, 8, true, PRO, 1, 1, 1>(p, st) : launch_tile_cfg<EPI, FP8, 8, true, PRO, 1, 1, 4>(p, st);
+    }
+    return p.M <= 4 ? launch_few_cfg<EPI, FP8, 8, PRO, 1>(p, st) : launch_few_cfg<EPI, FP8, 8, PRO, 4>(p, st);
+}
+
+template <int EPI, bool FP8>
+int launch_few(const TileParams& p, hipStream_t st) {
+    if (p.pro_ssq) return launch_few_pro<EPI, FP8, true>(p, st);
+    return launch_few_pro<EPI, FP8, false>(p, st);
 }
 
 bool aligned16(const void* q) { return ((uintptr_t)q & 15) == 0; }
@@ -813,11 +1046,18 @@ extern "C" int md_linear_fused_supported(int M, int N, int K, int epilogue) {
     return (epilogue >= FL_NONE && epilogue <= FL_GEGLU) ? 1 : 0;
 }
 
-extern "C" int md_linear_fused(const md_fused_linear_args* a, md_stream_t stream) {
-    MD_CHECK_ARG(a && a->x && a->w_packed && a->out, "md_linear_fused: null pointer argument");
-    MD_CHECK_ARG(md_linear_fused_supported(a->M, a->N, a->K, a->epilogue),
-                 "md_linear_fused: unsupported shape M=%d N=%d K=%d epilogue=%d (need 1 <= M <= 256, K %% 128 == 0, "
-                 "N %% 32 == 0)", a->M, a->N, a->K, a->epilogue);
+extern "C" int md_linear_few_supported(int M, int N, int K, int epilogue) {
+    MD_CHECK_ARG(M > 0 && N > 0 && K > 0, "md_linear_few_supported: M=%d N=%d K=%d", M, N, K);
+    return M <= 16 && K % 256 == 0 && md_linear_fused_supported(M, N, K, epilogue);
+}
+
+namespace {
+// md_linear_fused, md_linear_few: the same arguments; which kernel takes them
+int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream) {
+    MD_CHECK_ARG(a && a->x && a->w_packed && a->out, "md_linear_%s: null pointer argument", few ? "few" : "fused");
+    MD_CHECK_ARG(few ? md_linear_few_supported(a->M, a->N, a->K, a->epilogue) > 0 : md_linear_fused_supported(a->M, a->N, a->K, a->epilogue),
+                 "md_linear_%s: unsupported shape M=%d N=%d K=%d epilogue=%d (need 1 <= M <= %d, K %% %d == 0, "
+                 "N %% 32 == 0)", few ? "few" : "fused", a->M, a->N, a->K, a->epilogue, few ? 16 : 256, few ? 256 : 128);
     MD_CHECK_ARG(aligned16(a->x) && aligned16(a->w_packed) && aligned16(a->out) && a->ldx % 8 == 0 && a->ldo % 2 == 0,
                  "md_linear_fused: x / w / out must be 16-byte aligned, ldx %% 8 == 0, ldo %% 2 == 0");
     const bool gated = a->epilogue == FL_SWIGLU || a->epilogue == FL_GEGLU;
@@ -839,12 +1079,12 @@ extern "C" int md_linear_fused(const md_fused_linear_args* a, md_stream_t stream
     p.n_tiles = a->N / 32;
     p.m_tiles = (a->M + 31) / 32;
     if (a->pro_ssq) {
-        MD_CHECK_ARG(gated || a->epilogue == FL_ROPE_APPEND,
+        MD_CHECK_ARG(few || gated || a->epilogue == FL_ROPE_APPEND,
                      "md_linear_fused: the deferred-RMSNorm prologue exists for the qkv and w1|w3 linears");
         MD_CHECK_ARG(a->pro_norm_w && a->pro_tiles > 0 && aligned16(a->pro_norm_w),
                      "md_linear_fused: the deferred-RMSNorm prologue needs the norm weight (16-byte aligned) and pro_tiles");
-        MD_CHECK_ARG(a->pro_tiles * 32 == a->K, "md_linear_fused: pro_ssq must hold K / 32 = %d partial sums per row, got %d",
-                     a->K / 32, a->pro_tiles);
+        MD_CHECK_ARG(a->pro_tiles * 32 == a->K || a->pro_tiles * 16 == a->K,
+                     "md_linear_fused: pro_ssq must hold K / 32 = %d partial sums per row (or twice as many), got %d", a->K / 32, a->pro_tiles);
         p.pro_ssq = a->pro_ssq;
         p.pro_w = (const bf16_t*)a->pro_norm_w;
         p.pro_eps = a->pro_eps;
@@ -857,25 +1097,25 @@ extern "C" int md_linear_fused(const md_fused_linear_args* a, md_stream_t stream
     int rc = MD_OK;
     switch (a->epilogue) {
     case FL_NONE:
-        rc = launch_tile<FL_NONE, false>(p, st);
+        rc = few ? launch_few<FL_NONE, false>(p, st) : launch_tile<FL_NONE, false>(p, st);
         break;
     case FL_GEGLU:
         p.gelu = 1;
         [[fallthrough]];
     case FL_SWIGLU:
-        rc = launch_tile<FL_SWIGLU, false>(p, st);
+        rc = few ? launch_few<FL_SWIGLU, false>(p, st) : launch_tile<FL_SWIGLU, false>(p, st);
         break;
     case FL_XIELU:
         MD_CHECK_ARG(a->act && !a->bias, "md_linear_fused: the xIELU epilogue needs `act` and takes no bias");
         p.act = a->act;
-        rc = launch_tile<FL_XIELU, false>(p, st);
+        rc = few ? launch_few<FL_XIELU, false>(p, st) : launch_tile<FL_XIELU, false>(p, st);
         break;
     case FL_RESID:
         MD_CHECK_ARG(a->resid && ((uintptr_t)a->resid & 3) == 0 && a->ldr % 2 == 0,
                      "md_linear_fused: the residual epilogue needs `resid` (4-byte aligned, ldr %% 2 == 0)");
         p.resid = (const bf16_t*)a->resid;
         p.ldr = a->ldr;
-        rc = launch_tile<FL_RESID, false>(p, st);
+        rc = few ? launch_few<FL_RESID, false>(p, st) : launch_tile<FL_RESID, false>(p, st);
         break;
     default: {
         MD_CHECK_ARG(a->H > 0 && a->KH > 0 && (a->D == 64 || a->D == 128) && a->N == (a->H + 2 * a->KH) * a->D,
@@ -909,10 +1149,16 @@ extern "C" int md_linear_fused(const md_fused_linear_args* a, md_stream_t stream
         p.v_scale = a->v_scale;
         p.overflow = md_page_overflow_counter_device();
         MD_CHECK_ARG(p.overflow, "md_linear_fused: cannot resolve the page-overflow counter");
-        rc = kvd == MD_KV_FP8_E4M3 ? launch_tile<FL_ROPE_APPEND, true>(p, st) : launch_tile<FL_ROPE_APPEND, false>(p, st);
+        const bool fp8 = kvd == MD_KV_FP8_E4M3;
+        if (few) rc = fp8 ? launch_few<FL_ROPE_APPEND, true>(p, st) : launch_few<FL_ROPE_APPEND, false>(p, st);
+        else rc = fp8 ? launch_tile<FL_ROPE_APPEND, true>(p, st) : launch_tile<FL_ROPE_APPEND, false>(p, st);
     }
     }
     if (rc != MD_OK) return rc;
     MD_CHECK_LAUNCH("md_linear_fused");
     return MD_OK;
 }
+}  // namespace
+
+extern "C" int md_linear_fused(const md_fused_linear_args* a, md_stream_t stream) { return run_fused(a, false, stream); }
+extern "C" int md_linear_few(const md_fused_linear_args* a, md_stream_t stream) { return run_fused(a, true, stream); }

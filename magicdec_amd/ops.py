@@ -701,12 +701,20 @@ def _fused_args(x, weight: "PackedWeight", bias, epilogue):
     return a
 
 
-def _run_fused(a):
-    check(_lib.load().md_linear_fused(ctypes.byref(a), _stream()), "md_linear_fused")
+def few_linear_supported(M, N, K, epilogue=FL_NONE):
+    """True when md_linear_few (csrc/tilegemm.hip) takes this shape."""
+    return _lib.load().md_linear_few_supported(int(M), int(N), int(K), int(epilogue)) > 0
+
+
+def _run_fused(a, few=False):
+    if few:
+        check(_lib.load().md_linear_few(ctypes.byref(a), _stream()), "md_linear_few")
+    else:
+        check(_lib.load().md_linear_fused(ctypes.byref(a), _stream()), "md_linear_fused")
 
 
 class DeferredNorm:
-    """An RMSNorm that has NOT been applied yet: `h` [M, K] are the un-normalised hidden states and `ssq` [M, K/32]
+    """An RMSNorm that has NOT been applied yet: `h` [M, K] are the un-normalised hidden states and `ssq` [M, K/32] or [M, K/16]
     the per-row partial sums of squares the residual epilogue of the producing linear wrote; the consuming fused
     linear normalises on the fly (md_linear_fused, deferred RMSNorm).  `materialize()` is the stand-alone kernel."""
 
@@ -720,20 +728,21 @@ class DeferredNorm:
 def _set_pro(a, x, pro: "DeferredNorm"):
     if pro.h.data_ptr() != x.data_ptr() or pro.ssq.dtype != torch.float32 or not pro.ssq.is_contiguous():
         raise ValueError("deferred norm: x must be the un-normalised h the partial sums belong to")
-    if (pro.ssq.dim() != 2 or pro.ssq.shape[0] != x.shape[0] or pro.ssq.shape[1] * 32 != x.shape[1]
+    if (pro.ssq.dim() != 2 or pro.ssq.shape[0] != x.shape[0] or x.shape[1] not in (pro.ssq.shape[1] * 32, pro.ssq.shape[1] * 16)
             or pro.weight.numel() != x.shape[1] or pro.weight.dtype != torch.bfloat16):
-        # ssq must hold one partial per 32-column tile of the producer (a shorter one would give a silently wrong rstd)
-        raise ValueError("deferred norm: ssq [M, K / 32] float32 and a bf16 norm weight [K] expected")
+        # ssq must hold one partial per 32- or 16-column tile of the producer (a shorter one would give a silently wrong rstd)
+        raise ValueError("deferred norm: ssq [M, K / 32] or [M, K / 16] float32 and a bf16 norm weight [K] expected")
     a.pro_ssq, a.pro_tiles = pro.ssq.data_ptr(), pro.ssq.shape[1]
     a.pro_norm_w, a.pro_eps = pro.weight.data_ptr(), pro.eps
 
 
 def fused_linear(x, weight: "PackedWeight", bias=None, swiglu=False, resid=None, out=None, want_ssq=False,
-                 pro: "DeferredNorm" = None, xielu=None, gelu=False):
+                 pro: "DeferredNorm" = None, xielu=None, gelu=False, few=False):
     """One launch (md_linear_fused): F.linear(x, W, bias) for M <= 256 rows over a PackedWeight, optionally followed by
     SiLU(h1) * h3 (swiglu=True, weight = [w1; w3]) or by the bf16 residual add `resid + linear` (resid [M, N]).
     want_ssq (with resid): also return the per-row partial sums of squares [M, N/32] of the result (the producer half of
-    a deferred RMSNorm).  pro (with swiglu): x is pro.h and is normalised on the fly (the consumer half)."""
+    a deferred RMSNorm).  pro (with swiglu): x is pro.h and is normalised on the fly (the consumer half).
+    few: md_linear_few instead, M <= 16; its partial sums are [M, N/16], its sums of another order, and pro goes with everything."""
     epi = FL_RESID if resid is not None else (FL_XIELU if xielu is not None else FL_NONE)
     if swiglu:
         epi = FL_GEGLU if gelu else FL_SWIGLU
@@ -757,22 +766,22 @@ def fused_linear(x, weight: "PackedWeight", bias=None, swiglu=False, resid=None,
             raise ValueError("fused linear: resid must be bf16 [M, N] with unit inner stride")
         a.resid, a.ldr = resid.data_ptr(), resid.stride(0)
         if want_ssq:
-            ssq = torch.empty((x.shape[0], weight.N // 32), dtype=torch.float32, device=x.device)
+            ssq = torch.empty((x.shape[0], weight.N // (16 if few else 32)), dtype=torch.float32, device=x.device)
             a.ssq_out = ssq.data_ptr()
     elif want_ssq:
         raise ValueError("fused linear: want_ssq belongs to the residual epilogue")
     if pro is not None:
-        if not swiglu:
+        if not swiglu and not few:
             raise ValueError("fused linear: the deferred-norm prologue exists for the w1|w3 and qkv linears")
         _set_pro(a, x, pro)
-    _run_fused(a)
+    _run_fused(a, few)
     return (out, ssq) if want_ssq else out
 
 
 def fused_qkv_rope_append(x, weight: "PackedWeight", bias, H, KH, D, rows_per_req, offsets, table: RopeTable, kv_cache,
                           page_indices, page_indptr, last_page_len, kv_cache2=None, page_indices2=None,
                           page_indptr2=None, last_page_len2=None, kv_scales=None, kv_layout="NHD",
-                          pro: "DeferredNorm" = None):
+                          pro: "DeferredNorm" = None, few=False):
     """wqkv + RoPE + paged KV append in one launch (md_linear_fused, MD_FL_ROPE_APPEND): x [M, K] are the normalised
     hidden states of a decode / verify step in which request b owns rows [b * rows_per_req, (b+1) * rows_per_req).
     Returns the rotated q [M, H, D]; rotated k and v go to the paged cache (and to kv_cache2, bf16 NHD, when given).
@@ -802,7 +811,7 @@ def fused_qkv_rope_append(x, weight: "PackedWeight", bias, H, KH, D, rows_per_re
     a.kv_dtype, a.k_scale, a.v_scale = kvd, ks, vs
     if pro is not None:                      # x is the un-normalised h: normalise on the fly (deferred RMSNorm)
         _set_pro(a, x, pro)
-    _run_fused(a)
+    _run_fused(a, few)
     return q_out
 
 
