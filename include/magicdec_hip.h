@@ -329,6 +329,11 @@ int md_linear_prompt(const void* x, int64_t ldx, const void* w_packed, const voi
 int md_linear_f32_supported(int M, int N, int K);
 int md_linear_f32(const float* x, int64_t ldx, const float* w, float* out, int64_t ldo, int M, int N, int K, int tile, md_stream_t stream);
 
+/* md_linear_f32_few (csrc/f32few.hip): the same of at most 16 rows, a step's, over a narrow weight: N <= 4096, K % 256 == 0, N % 4 == 0, everything
+ * 16-byte aligned.  _supported: 1 if it takes the shape (negative: no shape).  tile: 0, or 8 or 16 columns a workgroup. */
+int md_linear_f32_few_supported(int M, int N, int K);
+int md_linear_f32_few(const float* x, int64_t ldx, const float* w, float* out, int64_t ldo, int M, int N, int K, int tile, md_stream_t stream);
+
 /* md_linear_f32_thirds (csrc/f32thirds.hip): the same on the bf16 matrix instructions, every number as the sum of three bf16 numbers (six
  * products of their parts, 32-bit sums): as exact as md_linear_f32.  K < 2^20.  ws: md_linear_f32_thirds_workspace(M, K) bytes, 16-byte
  * aligned (x in three parts), free again behind the call on its stream.  _supported: 1 if it takes the shape and is expected to be faster than

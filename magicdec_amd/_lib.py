@@ -129,6 +129,8 @@ _SIGNATURES = {
     "md_linear_xielu": (c_int, [P, L, P, I, P, P, L, I, I, I, P, c_size_t, P]),
     "md_linear_f32_supported": (c_int, [I, I, I]),
     "md_linear_f32": (c_int, [P, L, P, P, L, I, I, I, I, P]),
+    "md_linear_f32_few_supported": (c_int, [I, I, I]),
+    "md_linear_f32_few": (c_int, [P, L, P, P, L, I, I, I, I, P]),
     "md_linear_f32_thirds_supported": (c_int, [I, I, I]),
     "md_linear_f32_thirds_workspace": (c_size_t, [I, I]),
     "md_linear_f32_thirds": (c_int, [P, L, P, P, L, I, I, I, I, P, c_size_t, P]),

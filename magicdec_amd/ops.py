@@ -643,6 +643,25 @@ def linear_f32(x, weight, tile=0):
 
 
 @functools.lru_cache(maxsize=4096)
+def linear_f32_few_supported(M, N, K):
+    """True when md_linear_f32_few (csrc/f32few.hip) takes this shape."""
+    return _lib.load().md_linear_f32_few_supported(int(M), int(N), int(K)) > 0
+
+
+def linear_f32_few(x, weight, tile=0):
+    """linear_f32 of at most 16 rows, as a stream over a narrow weight (csrc/f32few.hip)."""
+    _gpu(x, weight)
+    if x.dim() != 2 or x.stride(1) != 1 or weight.dim() != 2 or not weight.is_contiguous() or x.shape[1] != weight.shape[1]:
+        raise ValueError("linear_f32_few expects x [M, K] with unit inner stride and a contiguous weight [N, K]")
+    if x.dtype != torch.float32 or weight.dtype != torch.float32:
+        raise TypeError("linear_f32_few takes float32")
+    (M, K), N = x.shape, weight.shape[0]
+    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    check(_lib.load().md_linear_f32_few(_p(x), x.stride(0), _p(weight), _p(out), N, M, N, K, int(tile), _stream()), "md_linear_f32_few")
+    return out
+
+
+@functools.lru_cache(maxsize=4096)
 def linear_f32_thirds_supported(M, N, K):
     """True when md_linear_f32_thirds (csrc/f32thirds.hip) takes this shape and is expected to be the fastest."""
     return _lib.load().md_linear_f32_thirds_supported(int(M), int(N), int(K)) > 0

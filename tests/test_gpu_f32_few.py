@@ -1,0 +1,36 @@
+"""md_linear_f32_few (csrc/f32few.hip) against float64 products, at the edges of its tiles, chunks and slices.  On the GPU (-m gpu)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+# one step a wavefront, steps that fill no chunk (K = 768: three of four or eight), several chunks; columns that end inside a tile
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("N,K,wider", [(4, 256, 0), (68, 768, 4), (132, 2048, 0), (12, 8192, 12), (2052, 1280, 0)])
+def test_products(M, N, K, wider):
+    from magicdec_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    big = torch.full((16 + 4, K + wider), float("nan"), device=DEV)                 # (rows past M stay out of it)
+    big[:M] = torch.randn(M, K + wider, device=DEV, generator=g)
+    x, w = big[:M, :K], torch.randn(N, K, device=DEV, generator=g)
+    ref = x.double() @ w.double().t()
+    off = (x.double().abs() @ w.double().abs().t()) * (K * 2.0 ** -24)               # fp32 sums of K terms in any order
+    for tile in (0, 8, 16):
+        out = ops.linear_f32_few(x, w, tile=tile)
+        assert out.shape == (M, N) and ((out.double() - ref).abs() <= off).all()
+        assert torch.equal(out[:1], ops.linear_f32_few(x[:1], w, tile=tile))          # a row's bits do not depend on the rows beside it
+    x[M // 2, 3] = float("inf")
+    out = ops.linear_f32_few(x, w)
+    assert out[M // 2].isinf().all() and out.isfinite().all(1).sum() == M - 1
+
+
+def test_refused():
+    from magicdec_amd import ops
+    x, w = torch.randn(4, 256, device=DEV), torch.randn(64, 256, device=DEV)
+    for call in (lambda: ops.linear_f32_few(torch.randn(17, 256, device=DEV), w), lambda: ops.linear_f32_few(x[:, :128], w[:, :128].contiguous()),
+                 lambda: ops.linear_f32_few(x, w[:62].contiguous()), lambda: ops.linear_f32_few(x, w, tile=32), lambda: ops.linear_f32_few(x.double(), w.double()),
+                 lambda: ops.linear_f32_few(torch.randn(4, 260, device=DEV)[:, 1:257], w)):
+        with pytest.raises((RuntimeError, ValueError, TypeError)):
+            call()
