@@ -2,18 +2,20 @@
 // bf16 matrix-core kernels of xattn_mfma.hip / latent_absorbed.hip do not apply (unbounded scores, unusual page sizes).  Queries, keys,
 // values, scores, weights and sums are fp32 throughout, as in the plain kernel of xattn.hip, whose semantics these are.
 //
-// A workgroup (4 wavefronts) owns R = 16 QT query rows -- (token, head of the kv head) pairs -- and a range of KT-key tiles:
+// Two kernels, both on (token, head of the kv head) rows and KT-key tiles:
+//   prompts, heads to 128   a wavefront owns 16 rows and all of a tile (xattn_f32_rows_kernel)
+//   else                    a workgroup of four wavefronts owns R = 16 QT rows together (xattn_f32_kernel):
 //   S^T = K.Q^T    a 16 x 16 score tile per wavefront and step; K and Q fragments are ds_read_b128 of padded LDS rows.  The four
 //                  elements of a b128 are four k-steps (both operands permute the contraction the same way).
 //   softmax        256 / R threads per row, scores through LDS; running maximum in log2 units, the distance penalty as one v_log_f32
 //   O^T = V^T.P^T  each wavefront owns every fourth 16-wide slice of the value size, so its sums stay in registers for any head size
 //                  and the weights are read back from LDS as B fragments.
-// Three barriers per tile (four where values are a prefix of the key rows: one image serves both); the next tile is in registers
+// There three barriers per tile (four where values are a prefix of the key rows: one image serves both); the next tile is in registers
 // while this one is computed.  Few rows (decode): 16-row tiles and the key range split over workgroups, merged by a second launch.
 //
 // Bound by the fp32 matrix rate (154 TFLOP/s in a large library product) for prompts, by latency for decode steps.  Six sequences of
-// 100 to 1 500 tokens, 32 query and 8 kv heads of 64, one layer: 9 930 -> 465 us (27 GFLOP, half of the tiles' work masked); one token
-// each behind them: 292 -> 16.5 + 5.9 us for the merge (first figure: the plain kernel, one workgroup per row and head).
+// 100 to 1 500 tokens, 32 query and 8 kv heads of 64, one layer (22 GFLOP): 9 930 -> 445 -> 277 us; one token each behind them:
+// 292 -> 16.5 + 5.9 us for the merge (first figure: the plain kernel, one workgroup per row and head).
 #include "xattn.h"
 
 #include <algorithm>
@@ -328,6 +330,289 @@ __global__ __launch_bounds__(256, (f32_waves_per_simd<DK, DV, QT, KT, SHARED>())
     }
 }
 
+// Prompts, heads to 128: a wavefront has 16 query rows to itself, NW of them share a tile of KT keys and values in two buffers, one barrier a
+// tile.  Scores come out of K.Q^T as V^T.P^T wants its weights -- lane (row, group) holds keys 16 k + 4 group + e -- and go from one product
+// to the next without LDS; queries and sums stay in registers.
+//
+// What bounds it: fp32 products and vector instructions of a SIMD exclude each other (12 of 42 million vector instructions less took as many
+// cycles off as they issue in), so everything beside the products counts: loads by descriptor, no address arithmetic; the reference of the
+// softmax moves only where it must; four columns of V a read.  The shape above: four wavefronts on 64 rows together 445 us, this 310, with
+// these 277 (80 TFLOP/s; products alone 250).  One prompt of 2 500 470 -> 268, 4 x 600 at 16 / 4 heads of 128 148 -> 97; tiles of 64 keys
+// 10 % slower, eight wavefronts 2 to 20 %.
+template <int DK, int DV, int KT, bool SHARED>
+constexpr int rows_lds_bytes() {
+    return 2 * KT * (DK + 4 + (SHARED ? 0 : DV + 4)) * 4 + 16;
+}
+
+template <typename T, int DK, int DV, int KT, int NW, int OCC, bool SHARED>
+__global__ __launch_bounds__(64 * NW, OCC) void xattn_f32_rows_kernel(const XattnParams p, const F32Launch L) {
+    typedef typename Vec4<T>::type vec4;
+    constexpr int R = 16 * NW, NT = 64 * NW, KP = DK + 4, VP = SHARED ? KP : DV + 4, KB = KT / 16, NV = DV / 16;
+    constexpr int kTile = KT * (KP + (SHARED ? 0 : VP));         // floats of one buffer
+    constexpr int LK = KT * DK / (4 * NT), LV = SHARED ? 1 : KT * DV / (4 * NT);
+    static_assert(KT * DK % (4 * NT) == 0 && KT * DV % (4 * NT) == 0 && DK % 16 == 0 && DV % 64 == 0 && KT == 32, "tile shapes");
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    int* sbad = reinterpret_cast<int*>(lds + 2 * kTile);         // [3]: the tile's values hold an infinity or a NaN
+
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, lq = lane & 15, lc = lane >> 4;
+    const int pairs = p.KH * p.B, pair = blockIdx.x % pairs, part = blockIdx.x / pairs, kvh = pair % p.KH, b = pair / p.KH, g = p.g;
+    const int qg = L.nq - 1 - part / L.nsplit, split = part % L.nsplit;                 // longest key ranges of all sequences first
+    const int q0 = p.qo_indptr[b], nrows = (p.qo_indptr[b + 1] - q0) * g, R0 = qg * R;
+    if (R0 >= nrows) return;
+    const int pos0 = p.pos0[b], pg0 = p.page_indptr[b], cap = (p.page_indptr[b + 1] - pg0) * p.page_size;
+    const int hi_wg = min(pos0 + (min(R0 + R, nrows) - 1) / g, cap - 1), lo_wg = ((pos0 + R0 / g) / p.chunk) * p.chunk;
+    int t0 = 0, t1 = 0;
+    if (hi_wg >= lo_wg) {
+        const int first = lo_wg / KT, n = hi_wg / KT - first + 1, per = (n + L.nsplit - 1) / L.nsplit;
+        t0 = first + min(split * per, n);
+        t1 = first + min((split + 1) * per, n);
+    }
+    // this lane's row, and the keys that all and that any of the wavefront's rows see
+    const int Rw = R0 + wave * 16, row = Rw + lq;
+    const int first_pos = pos0 + Rw / g, last_pos = pos0 + (min(Rw + 16, nrows) - 1) / g;
+    const int any_lo = first_pos / p.chunk * p.chunk, any_hi = Rw < nrows ? min(last_pos, cap - 1) : -1;
+    const int all_lo = last_pos / p.chunk * p.chunk, all_hi = min(first_pos, cap - 1);
+    int hi = -1, lo = 0;
+    float r1 = 0.f, r2 = 0.f, m = 0.f, l = 0.f, top = -INFINITY;
+    const int pos = pos0 + row / g;
+    if (row < nrows) {
+        hi = min(pos, cap - 1);
+        lo = (pos / p.chunk) * p.chunk;
+        if (p.r1) {
+            r1 = p.r1[kvh * g + row % g];
+            r2 = p.r2[kvh * g + row % g];
+        }
+    }
+    const bool bias = p.r1 != nullptr;
+    f32x4 q[DK / 16], o[NV];
+#pragma unroll
+    for (int i = 0; i < DK / 16; ++i) {
+        const int d = i * 16 + lc * 4;
+        q[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (row < nrows && d < p.DKp)
+            q[i] = __builtin_convertvector(*reinterpret_cast<const vec4*>(reinterpret_cast<const T*>(p.q) +
+                                           ((int64_t)(q0 + row / g) * p.H + kvh * g + row % g) * p.DKp + d), f32x4);
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) o[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // element x of o[v]: the values' column 4 j + v % 4 of 64 is row j of product v, so that a lane reads four columns at once
+    auto at = [&](int v, int x) { return v / 4 * 64 + lc * 16 + x * 4 + v % 4; };
+
+    // A tile's pieces into registers.  It lies in one page; the descriptor ends with the workgroup's last key, and what lies behind it or
+    // beyond the head size reads as zeros
+    vec4 kr[LK], vr[LV];
+    unsigned kat[LK], vat[LV];
+#pragma unroll
+    for (int i = 0; i < LK; ++i) {
+        const int e = tid + NT * i, key = e / (DK / 4), d = e % (DK / 4) * 4;
+        kat[i] = d < p.DKp ? (unsigned)((key * p.ldk + d) * sizeof(T)) : 0xc0000000u;
+    }
+#pragma unroll
+    for (int i = 0; i < LV; ++i) {
+        const int e = tid + NT * i, key = e / (DV / 4), d = e % (DV / 4) * 4;
+        vat[i] = d < p.DVp ? (unsigned)((key * p.ldv + d) * sizeof(T)) : 0xc0000000u;
+    }
+    auto fetch = [](__amdgpu_buffer_rsrc_t r, unsigned at) {
+        if constexpr (sizeof(T) == 4) {
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0);
+            return *reinterpret_cast<const vec4*>(&v);
+        } else {
+            const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, at, 0, 0);
+            return *reinterpret_cast<const vec4*>(&v);
+        }
+    };
+    auto request = [&](int t) {
+        const int key = t * KT, page = key / p.page_size, keys = min(hi_wg - key + 1, KT);
+        const int64_t line = ((int64_t)p.page_indices[pg0 + page] * p.KH + kvh) * p.page_size + (key - page * p.page_size);
+        const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<T*>(reinterpret_cast<const T*>(p.k_cache) + line * p.ldk), (short)0, keys * p.ldk * (int)sizeof(T), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < LK; ++i) kr[i] = fetch(rk, kat[i]);
+        if constexpr (!SHARED) {
+            const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<T*>(reinterpret_cast<const T*>(p.v_cache) + line * p.ldv), (short)0, keys * p.ldv * (int)sizeof(T), 0x00020000);
+#pragma unroll
+            for (int i = 0; i < LV; ++i) vr[i] = fetch(rv, vat[i]);
+        }
+    };
+    auto stage = [&](int t) {                // (keys past the workgroup's last one are zeros: their memory may hold anything)
+        float* sk = lds + ((t - t0) & 1) * kTile;
+        float worst = 0.f;                   // an infinity or a NaN times zero is a NaN
+#pragma unroll
+        for (int i = 0; i < LK; ++i) {
+            const int e = tid + NT * i, key = e / (DK / 4), d = (e % (DK / 4)) * 4;
+            const f32x4 v = __builtin_convertvector(kr[i], f32x4);
+            *reinterpret_cast<f32x4*>(sk + key * KP + d) = v;
+            if (SHARED)
+                for (int x = 0; x < 4; ++x) worst = fmaf(v[x], 0.f, worst);
+        }
+        if constexpr (!SHARED) {
+#pragma unroll
+            for (int i = 0; i < LV; ++i) {
+                const int e = tid + NT * i, key = e / (DV / 4), d = (e % (DV / 4)) * 4;
+                const f32x4 v = __builtin_convertvector(vr[i], f32x4);
+                *reinterpret_cast<f32x4*>(sk + KT * KP + key * VP + d) = v;
+                for (int x = 0; x < 4; ++x) worst = fmaf(v[x], 0.f, worst);
+            }
+        }
+        if (__builtin_amdgcn_ballot_w64(worst != 0.f) != 0 && lane == 0) sbad[t % 3] = 1;
+    };
+
+    if (tid < 3) sbad[tid] = 0;
+    if (t0 < t1) {
+        request(t0);
+        // (the queries have come: else the compiler waits in the loop for them, and for the tile requested behind)
+#pragma unroll
+        for (int i = 0; i < DK / 16; ++i) asm volatile("" : "+v"(q[i]));
+        asm volatile("" : "+v"(r1), "+v"(r2));
+        __syncthreads();
+        stage(t0);
+        if (t0 + 1 < t1) request(t0 + 1);
+    }
+    __syncthreads();
+    for (int t = t0; t < t1; ++t) {
+        // one barrier a tile: past it nobody reads the buffer of the tile before, nor its mark
+        if (tid == 0) sbad[(t + 2) % 3] = 0;
+        if (t + 1 < t1) stage(t + 1);
+        if (t + 2 < t1) request(t + 2);
+        const int base = t * KT;
+        if (base <= any_hi && base + KT > any_lo) {
+            const float* sk = lds + ((t - t0) & 1) * kTile;
+            const float* sv = SHARED ? sk : sk + KT * KP;
+            // ---- scores: lane (lq, lc) gets keys 16 k + 4 lc + e of row lq
+            f32x4 s[KB];
+#pragma unroll
+            for (int k = 0; k < KB; ++k) s[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < DK / 16; ++i) {
+                f32x4 ka[KB];
+#pragma unroll
+                for (int k = 0; k < KB; ++k) ka[k] = *reinterpret_cast<const f32x4*>(sk + (k * 16 + lq) * KP + i * 16 + lc * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int k = 0; k < KB; ++k) s[k] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[k][e], q[i][e], s[k], 0, 0, 0);
+            }
+            // ---- softmax.  The reference m of a row moves only where a score passes it by 8 (log2): a weight is at most 2^8, and what
+            // moving it costs is rarely paid.  A row that has seen no key yet takes the first tile's maximum, whatever it is
+            const float ahead = (float)(pos - base - lc * 4);
+#pragma unroll
+            for (int k = 0; k < KB; ++k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[k][e] = fmaf(s[k][e], p.scale_log2, -m);
+            if (bias) {
+                asm volatile("");                // (a branch: not computed and thrown away)
+#pragma unroll
+                for (int k = 0; k < KB; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        s[k][e] = fmaf(-r1, __builtin_amdgcn_logf(1.0f + r2 * (ahead - (float)(k * 16 + e))), s[k][e]);
+            }
+            if (!(base >= all_lo && base + KT - 1 <= all_hi && Rw + 16 <= nrows)) {
+#pragma unroll
+                for (int k = 0; k < KB; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int kp = base + k * 16 + lc * 4 + e;
+                        s[k][e] = kp >= lo && kp <= hi ? s[k][e] : -INFINITY;
+                    }
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int k = 0; k < KB; ++k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[k][e]);
+            if (__builtin_amdgcn_ballot_w64(mx > top) != 0) {
+                mx = fmaxf(mx, __shfl_xor(mx, 16));
+                mx = fmaxf(mx, __shfl_xor(mx, 32));
+                const float mnew = mx > top ? m + mx : m, up = mnew - m, alpha = top < 0.f ? 0.f : __builtin_amdgcn_exp2f(-up);
+                if (mx > top) top = 8.f;
+                m = mnew;
+                l *= alpha;
+#pragma unroll
+                for (int v = 0; v < NV; ++v) o[v] *= alpha;
+#pragma unroll
+                for (int k = 0; k < KB; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[k][e] -= up;
+            }
+#pragma unroll
+            for (int k = 0; k < KB; ++k)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    s[k][e] = __builtin_amdgcn_exp2f(s[k][e]);
+                    l += s[k][e];
+                }
+            // ---- values: the weights are where the product wants them
+            if (sbad[t % 3] == 0) {
+#pragma unroll
+                for (int k = 0; k < KB; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int v = 0; v < NV; v += 4) {
+                            const f32x4 va = *reinterpret_cast<const f32x4*>(sv + (k * 16 + lc * 4 + e) * VP + v * 16 + lq * 4);
+#pragma unroll
+                            for (int x = 0; x < 4; ++x) o[v + x] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[x], s[k][e], o[v + x], 0, 0, 0);
+                        }
+            } else {
+                // a value that a row does not see must not reach it as 0 * infinity; one that it sees does, also with a weight that underflowed
+#pragma unroll
+                for (int k = 0; k < KB; ++k)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        for (int c = 0; c < 4; ++c) {
+                            const float w = __shfl(s[k][e], c * 16 + lq);
+                            const int key = k * 16 + c * 4 + e;
+                            if (base + key >= lo && base + key <= hi) {
+#pragma unroll
+                                for (int v = 0; v < NV; ++v)
+#pragma unroll
+                                    for (int x = 0; x < 4; ++x) o[v][x] = fmaf(w, sv[key * VP + at(v, x)], o[v][x]);
+                            }
+                        }
+            }
+        }
+        __syncthreads();
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    // ---- out: lane (lq, lc) holds elements d .. d + 3 of its row
+    if (row >= nrows) return;
+    const int64_t slot = ((((int64_t)b * p.KH + kvh) * L.nq + qg) * L.nsplit + split) * R + wave * 16 + lq;
+    if (L.nsplit > 1) {
+        float* ml = p.ws + (int64_t)p.B * p.KH * L.nq * L.nsplit * R * L.dvw + slot * 2;
+        if (lc == 0) {
+            ml[0] = top < 0.f ? -1e30f : m;
+            ml[1] = l;
+        }
+#pragma unroll
+        for (int v = 0; v < NV; v += 4)
+#pragma unroll
+            for (int x = 0; x < 4; ++x)
+                *reinterpret_cast<f32x4*>(p.ws + slot * L.dvw + at(v, x)) = f32x4{o[v][x], o[v + 1][x], o[v + 2][x], o[v + 3][x]};
+        return;
+    }
+    const float M = p.sink ? fmaxf(m, 0.f) : m, f = __builtin_amdgcn_exp2f(m - M);
+    const float Z = l * f + (p.sink ? __builtin_amdgcn_exp2f(-M) : 0.f), inv = Z > 0.f ? f / Z : Z != Z ? Z : 0.f;
+    T* out = reinterpret_cast<T*>(p.out) + ((int64_t)(q0 + row / g) * p.H + kvh * g + row % g) * p.DV;
+    const bool wide = p.DV % 4 == 0 && reinterpret_cast<uintptr_t>(p.out) % sizeof(vec4) == 0;
+#pragma unroll
+    for (int v = 0; v < NV; v += 4)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const f32x4 y = f32x4{o[v][x], o[v + 1][x], o[v + 2][x], o[v + 3][x]} * inv;
+            if (wide) {
+                if (at(v, x) < p.DV) *reinterpret_cast<vec4*>(out + at(v, x)) = __builtin_convertvector(y, vec4);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (at(v + e, x) < p.DV) out[at(v + e, x)] = (T)y[e];
+            }
+        }
+}
+
 // sums the kv splits: one thread per four elements of a row
 template <typename T>
 __global__ __launch_bounds__(256) void xattn_f32_merge_kernel(const XattnParams p, const F32Launch L) {
@@ -382,8 +667,9 @@ F32Launch plan(const XattnParams& p, Shape s, long keys) {
     };
     // Wide row groups reuse a tile's keys, 16 rows are the shorter chain: ahead by a fifth to a third while the wide ones are not half as
     // many workgroups as there are CUs (32 query heads of 64, 20 rows over 20 keys: 16.2 -> 11.6 us with the keys of a tile that are not
-    // there left out; 16 rows over 1 500: x 0.7), behind by as much from about 200 on (heads of 256: 150).
-    if (rows <= 16 || with_rows(16 * wide[s]) < 144) with_rows(16);
+    // there left out; 16 rows over 1 500: x 0.7), behind by as much from about 200 on (heads of 256: 150).  A wavefront's own rows (heads to
+    // 128) are level at 100 workgroups (13 x 8: 22.1 and 23.3; 48 x 2: 28.3 and 26.0), ahead at 128 (8 x 60 rows, 16 / 4 heads of 128: 21.5 and 19.2).
+    if (rows <= 16 || with_rows(16 * wide[s]) < 128) with_rows(16);
     return L;
 }
 
@@ -410,12 +696,35 @@ int launch(const XattnParams& p, const F32Launch& L, hipStream_t st) {
     return MD_OK;
 }
 
+template <typename T, int DK, int DV, int KT, int NW, int OCC, bool SHARED>
+int launch_rows(const XattnParams& p, const F32Launch& L, hipStream_t st) {
+    constexpr int bytes = rows_lds_bytes<DK, DV, KT, SHARED>();
+    static_assert(bytes <= 160 * 1024, "LDS");
+    static MdPerDeviceOnce once;
+    if (bytes > 64 * 1024 && once.first()) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&xattn_f32_rows_kernel<T, DK, DV, KT, NW, OCC, SHARED>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
+            once.undo();
+            md_set_error("attention: cannot raise the LDS limit to %d bytes", bytes);
+            return MD_ERR_LAUNCH;
+        }
+    }
+    hipLaunchKernelGGL((xattn_f32_rows_kernel<T, DK, DV, KT, NW, OCC, SHARED>), dim3((unsigned)(p.KH * p.B * L.nq * L.nsplit)), dim3(64 * NW),
+                       bytes, st, p, L);
+    if (L.nsplit > 1) {
+        const int64_t threads = (int64_t)p.B * p.KH * L.nq * L.R * (L.dvw / 4);
+        hipLaunchKernelGGL((xattn_f32_merge_kernel<T>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, p, L);
+    }
+    MD_CHECK_LAUNCH("attention(32-bit)");
+    return MD_OK;
+}
+
 template <typename T>
 int launch_shape(const XattnParams& p, Shape s, const F32Launch& L, hipStream_t st) {
     const bool few = L.R == 16;
     switch (s) {
-    case k64: return few ? launch<T, 64, 64, 1, 64, false>(p, L, st) : launch<T, 64, 64, 4, 64, false>(p, L, st);
-    case k128: return few ? launch<T, 128, 128, 1, 32, false>(p, L, st) : launch<T, 128, 128, 4, 32, false>(p, L, st);
+    case k64: return few ? launch<T, 64, 64, 1, 64, false>(p, L, st) : launch_rows<T, 64, 64, 32, 4, 4, false>(p, L, st);
+    case k128: return few ? launch<T, 128, 128, 1, 32, false>(p, L, st) : launch_rows<T, 128, 128, 32, 4, 2, false>(p, L, st);
     case k256: return few ? launch<T, 256, 256, 1, 32, false>(p, L, st) : launch<T, 256, 256, 2, 32, false>(p, L, st);
     case kShared320: return few ? launch<T, 320, 256, 1, 32, true>(p, L, st) : launch<T, 320, 256, 2, 32, true>(p, L, st);
     default: return few ? launch<T, 576, 512, 1, 32, true>(p, L, st) : launch<T, 576, 512, 2, 32, true>(p, L, st);
