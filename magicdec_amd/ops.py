@@ -624,6 +624,7 @@ def linear_prompt(x, weight: "PackedWeight", bias=None, swiglu=False, out=None, 
 
 
 @functools.lru_cache(maxsize=4096)
+@functools.lru_cache(maxsize=1024)
 def linear_f32_supported(M, N, K):
     """True when md_linear_f32 (csrc/f32gemm.hip) takes this shape and is expected to be faster than the library."""
     return _lib.load().md_linear_f32_supported(int(M), int(N), int(K)) > 0
@@ -643,6 +644,7 @@ def linear_f32(x, weight, tile=0):
 
 
 @functools.lru_cache(maxsize=4096)
+@functools.lru_cache(maxsize=1024)
 def linear_f32_few_supported(M, N, K):
     """True when md_linear_f32_few (csrc/f32few.hip) takes this shape."""
     return _lib.load().md_linear_f32_few_supported(int(M), int(N), int(K)) > 0
@@ -662,6 +664,7 @@ def linear_f32_few(x, weight, tile=0):
 
 
 @functools.lru_cache(maxsize=4096)
+@functools.lru_cache(maxsize=1024)
 def linear_f32_thirds_supported(M, N, K):
     """True when md_linear_f32_thirds (csrc/f32thirds.hip) takes this shape and is expected to be the fastest."""
     return _lib.load().md_linear_f32_thirds_supported(int(M), int(N), int(K)) > 0
