@@ -411,6 +411,11 @@ int md_linear_fused(const md_fused_linear_args* args, md_stream_t stream);
 int md_linear_few_supported(int M, int N, int K, int epilogue);
 int md_linear_few(const md_fused_linear_args* args, md_stream_t stream);
 
+/* md_linear_fused_beside (csrc/tilegemm.hip): a gated product and out2[M][N2] = x . W2^T of the same rows in one launch.  _supported: 1 if it takes
+ * the shapes (negative: none). */
+int md_linear_fused_beside_supported(int M, int N, int K, int N2);
+int md_linear_fused_beside(const md_fused_linear_args* args, const void* w2_packed, int N2, void* out2, int64_t ldo2, md_stream_t stream);
+
 /* md_linear_fused_split: the K8b tile kernel with the K range ALSO split over S workgroups, for the deep narrow
  * products of a <= 64-row draft step (the 1B model's w2: N = 2048, K = 8192 -- Engine/SnapKV/model.py:451-455 followed by
  * the residual add and the next RMSNorm, :260-278,464-469).  A workgroup owns a (32|64)-row x (32|64)-column tile and K / S

@@ -420,20 +420,35 @@ class LayeredTransformer(Transformer):
         z = self._library(y, lin.weight)
         return ops.gelu_mul(z[:, :N // 2], z[:, N // 2:], out=out)
 
+    def _gated_beside(self, y, layer, out):
+        """_gated into `out` and the product into the latents, which is returned, in one launch where the tile kernel runs both; else None."""
+        M = y.shape[0]
+        if layer.w13 is None or M > 256 or not y.is_cuda or y.dtype != torch.bfloat16:
+            return None
+        gate, win = (self._packed.get(id(w.weight)) for w in (layer.w13, layer.attention.win))
+        if (gate is None or win is None or win.dtype != torch.bfloat16 or out.stride(0) % 8 or out.data_ptr() % 16
+                or self._linear_how(M, gate.N, gate.K, True, False, gate, "swiglu", False) != "fused"
+                or not ops.fused_linear_beside_supported(M, gate.N, gate.K, win.N)):
+            return None
+        return ops.fused_linear_beside(y, gate, out, win, gelu=True)
+
     def _parallel(self, i, layer, y, rows, tab: PageTable, ctx):
         """mixer(y) + feed_forward(y) in a form ops.resid_norm adds to the residual."""
         att, s = layer.attention, self._xspec[i]
         cache = att.kv_cache.rows
-        z = self._linear(y, att.win)
+        side = torch.empty((y.shape[0], layer.wout.weight.shape[1]), dtype=y.dtype, device=y.device)
+        z = self._gated_beside(y, layer, side[:, layer.heads_out:])
+        gated = z is not None
+        if not gated:
+            z = self._linear(y, att.win)
         cq = ops.latent_append(z, s, cache, rows, tab.indices, tab.indptr, tab.max_pages)
         q = self._linear(cq, att.wuq)
         if ctx is not None:
             ctx.expand = functools.partial(self._linear, lin=att.wukv)
-        side = torch.empty((y.shape[0], layer.wout.weight.shape[1]), dtype=y.dtype, device=y.device)
         heads = side[:, :layer.heads_out].unflatten(1, (s.H, s.vdim))
         ops.latent_attention(q, s, cache, rows, tab.indices, tab.indptr, tab.max_pages, self.workspace, heads,
                              gate=z[:, sum(att.cuts) - s.H:sum(att.cuts)] if att.spec.gate else None, ctx=ctx)
-        if layer.w13 is not None:
+        if layer.w13 is not None and not gated:
             self._gated(y, layer.w13, side[:, layer.heads_out:])
         return self._project(side, layer.wout)
 

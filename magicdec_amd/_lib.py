@@ -112,6 +112,8 @@ _SIGNATURES = {
     "md_linear_block_workspace_bytes": (c_size_t, [I, I, I, I]),
     "md_linear_block": (c_int, [P, L, P, P, P, L, I, I, I, I, P, c_size_t, P]),
     "md_linear_block_add_rmsnorm": (c_int, [P, L, P, P, P, L, P, c_float, P, P, I, I, I, P, c_size_t, P]),
+    "md_linear_fused_beside_supported": (c_int, [I, I, I, I]),
+    "md_linear_fused_beside": (c_int, [ctypes.POINTER(FusedLinearArgs), P, I, P, L, P]),
     "md_linear_few_supported": (c_int, [I, I, I, I]),
     "md_linear_few": (c_int, [ctypes.POINTER(FusedLinearArgs), P]),
     "md_linear_fused_supported": (c_int, [I, I, I, I]),

@@ -90,6 +90,11 @@ struct TileParams {
     const float* k_scale;
     const float* v_scale;
     const float* act;         // XIELU: the two numbers of the activation
+    // SWIGLU, 1 x 1 tiles: plain columns of a second weight over the same rows behind the gated ones (md_linear_fused_beside), or 0 of them
+    const bf16_t* side_w;
+    bf16_t* side_out;
+    int64_t side_ldo;
+    int side_tiles;
     int gelu;                 // SWIGLU: GELU (tanh form), fp32 up to the product's one rounding, instead of SiLU
     unsigned int* overflow;   // dropped-row counter (md_page_overflow_count)
     // deferred RMSNorm (see the kernel header): producer side (RESID) / consumer side (PRO)
@@ -274,7 +279,8 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
     MD_TS(0);
     // block id -> (weight tile group, M tile group): block b runs on XCD b % 8; the M groups of one weight tile group
     // stay on one XCD
-    const int m_groups = (p.m_tiles + MT - 1) / MT, n_groups = p.n_tiles / NT;
+    constexpr bool kBeside = EPI == FL_SWIGLU && !PRO && MT * NT == 1;
+    const int m_groups = (p.m_tiles + MT - 1) / MT, n_groups = p.n_tiles / NT + (kBeside ? p.side_tiles : 0);
     int tng, tmg, slice = 0;
     if constexpr (EPI == FL_PARTIAL) {
         // K slice in the FAST index: with S = 8 a slice -- i.e. the Kt columns of x it reads -- lives on one XCD's L2
@@ -289,7 +295,8 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
         tmg = slot % m_groups;
     }
     if (tng >= n_groups) return;
-    const int m0 = tmg * 32 * MT, tn0 = tng * NT;
+    const bool beside = kBeside && tng >= p.n_tiles;
+    const int m0 = tmg * 32 * MT, tn0 = beside ? tng - p.n_tiles : tng * NT;
 
     // 16-deep MFMA k-steps of this wavefront's slice (FL_PARTIAL: of this workgroup's K slice, then of the wavefront)
     const int ksteps_w = (p.K >> 4) / (kNW * (EPI == FL_PARTIAL ? p.S : 1));
@@ -297,7 +304,7 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
     const bf16_t* wbase[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
-        wbase[nt] = p.w + ((int64_t)(tn0 + nt) * (p.K >> 4) + ks0) * 512;    // wave-uniform; + lane * 8 per lane
+        wbase[nt] = (beside ? p.side_w : p.w) + ((int64_t)(tn0 + nt) * (p.K >> 4) + ks0) * 512;    // wave-uniform; + lane * 8 per lane
     unsigned char* my_lds = lds + wave * kWaveLdsT;
 
     // activation staging: instruction i covers rows 4i + (lane >> 4), 16 lanes read one 256-B row segment
@@ -582,6 +589,11 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
                 *reinterpret_cast<f32x2*>(p.partial + ((int64_t)slice * p.M + gm) * p.N + tn * 32 + 2 * cp) = s;
             continue;
         } else if constexpr (EPI == FL_SWIGLU) {
+            if (beside) {
+                const f32x2 s = tile_sum2(2 * cp);
+                if (gm < p.M) *reinterpret_cast<unsigned int*>(p.side_out + (int64_t)gm * p.side_ldo + tn * 32 + 2 * cp) = pack2(s[0], s[1]);
+                continue;
+            }
             const int I = p.N >> 1;
             const int i = tn * 16 + cp;
             const float a1 = tile_sum1(cp), a3 = tile_sum1(16 + cp);
@@ -786,7 +798,7 @@ int launch_tile_cfg(const TileParams& p, hipStream_t st) {
             return MD_ERR_LAUNCH;
         }
     }
-    const int m_groups = (p.m_tiles + MT - 1) / MT, n_groups = p.n_tiles / NT;
+    const int m_groups = (p.m_tiles + MT - 1) / MT, n_groups = p.n_tiles / NT + p.side_tiles;
     const int grid = ((n_groups + 7) / 8) * 8 * m_groups;
     hipLaunchKernelGGL(k, dim3(grid), dim3(64 * NW), lds, st, p);
     return MD_OK;
@@ -798,6 +810,11 @@ int g_force_nw = 0;   // dev knob (md_debug_set_fused_nw): 0 = the rule below, 8
 
 int g_force_tile = 0; // dev knob (md_debug_set_fused_nw 11 / 22): force 1 x 1 / 2 x 2 tiles where the shape allows
 
+bool two_by_two(int M, int N, int K) {
+    const int m_tiles = (M + 31) / 32, n_tiles = N / 32;
+    return m_tiles >= 2 && n_tiles % 2 == 0 && K % 128 == 0 && (n_tiles / 2) * ((m_tiles + 1) / 2) >= 192;
+}
+
 template <int EPI, bool FP8, bool PRO>
 int launch_tile_pro(const TileParams& p, hipStream_t st) {
     // 2 x 2 tiles (64 rows x 64 columns per workgroup, one per CU): when the M range has two 32-row tiles and the 64-column
@@ -808,10 +825,9 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
     // also WITH the deferred-RMSNorm prologue (SwiGLU consumer), now that that instantiation has a four-deep W
     // ring, no spills, and its own prologue (kNewPro in the kernel)
     if constexpr ((EPI == FL_SWIGLU || EPI == FL_NONE || EPI == FL_RESID || EPI == FL_XIELU) && (!PRO || EPI == FL_SWIGLU)) {
-        const int groups = (p.n_tiles / 2) * ((p.m_tiles + 1) / 2);
-        bool t22 = p.m_tiles >= 2 && p.n_tiles % 2 == 0 && p.K % 128 == 0 && groups >= 192;
-        if (g_force_tile == 11) t22 = false;
-        if (g_force_tile == 22) t22 = p.n_tiles % 2 == 0 && p.K % 128 == 0;
+        bool t22 = two_by_two(p.M, p.N, p.K);
+        if (g_force_tile == 11 || p.side_tiles) t22 = false;
+        if (g_force_tile == 22 && !p.side_tiles) t22 = p.n_tiles % 2 == 0 && p.K % 128 == 0;
         if (PRO && p.pro_tiles > 128) t22 = false;       // the 2 x 2 prologue keeps <= 8 partial sums per thread in flight
         if (t22) return launch_tile_cfg<EPI, FP8, 8, false, PRO, 2, 2>(p, st);
     }
@@ -820,7 +836,7 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
     // wavefronts, 13.3 with 8; 8192 x 2048 (256) 8.6 and 8.9; 64 rows of 6144 x 2048 (384) 12.2 and 11.0; one row of 9216 x 3072 16.0 and 13.6
     // (not below K = 1024 -- two k-steps per wavefront and a 16-way reduce cost more than they hide: K = 512 shards run 4.1-4.2 us with
     // 8 slices against 5.3-5.4 with 16)
-    const int wgs = p.n_tiles * p.m_tiles;
+    const int wgs = (p.n_tiles + p.side_tiles) * p.m_tiles;
     bool nw16 = p.K % 256 == 0 && p.K >= 1024 && wgs <= 256;
     if (g_force_nw == 8) nw16 = false;
     if (g_force_nw == 16) nw16 = p.K % 256 == 0;
@@ -1053,7 +1069,8 @@ extern "C" int md_linear_few_supported(int M, int N, int K, int epilogue) {
 
 namespace {
 // md_linear_fused, md_linear_few: the same arguments; which kernel takes them
-int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream) {
+int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream, const void* side_w = nullptr, int side_N = 0, void* side_out = nullptr,
+              int64_t side_ldo = 0) {
     MD_CHECK_ARG(a && a->x && a->w_packed && a->out, "md_linear_%s: null pointer argument", few ? "few" : "fused");
     MD_CHECK_ARG(few ? md_linear_few_supported(a->M, a->N, a->K, a->epilogue) > 0 : md_linear_fused_supported(a->M, a->N, a->K, a->epilogue),
                  "md_linear_%s: unsupported shape M=%d N=%d K=%d epilogue=%d (need 1 <= M <= %d, K %% %d == 0, "
@@ -1078,6 +1095,10 @@ int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream) {
     p.K = a->K;
     p.n_tiles = a->N / 32;
     p.m_tiles = (a->M + 31) / 32;
+    p.side_w = (const bf16_t*)side_w;
+    p.side_out = (bf16_t*)side_out;
+    p.side_ldo = side_ldo;
+    p.side_tiles = side_N / 32;
     if (a->pro_ssq) {
         MD_CHECK_ARG(few || gated || a->epilogue == FL_ROPE_APPEND,
                      "md_linear_fused: the deferred-RMSNorm prologue exists for the qkv and w1|w3 linears");
@@ -1162,3 +1183,22 @@ int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream) {
 
 extern "C" int md_linear_fused(const md_fused_linear_args* a, md_stream_t stream) { return run_fused(a, false, stream); }
 extern "C" int md_linear_few(const md_fused_linear_args* a, md_stream_t stream) { return run_fused(a, true, stream); }
+
+// Two products of the same rows in one launch: a gated one and, behind its columns, a plain one that alone would leave most CUs idle (a
+// parallel layer's 1 376 x 2 048 into its latents at 32 rows: 43 workgroups that take 7.0 us, beside 352 that take 14.1; together 15.3).
+// Not where the gated one runs 2 x 2 tiles, of which the second has an odd number.
+extern "C" int md_linear_fused_beside_supported(int M, int N, int K, int N2) {
+    MD_CHECK_ARG(M > 0 && N > 0 && K > 0 && N2 > 0, "md_linear_fused_beside_supported: M=%d N=%d K=%d N2=%d", M, N, K, N2);
+    return md_linear_fused_supported(M, N, K, FL_GEGLU) && md_linear_fused_supported(M, N2, K, FL_NONE) && !two_by_two(M, N, K);
+}
+
+extern "C" int md_linear_fused_beside(const md_fused_linear_args* a, const void* w2_packed, int N2, void* out2, int64_t ldo2, md_stream_t stream) {
+    MD_CHECK_ARG(a && w2_packed && out2, "md_linear_fused_beside: null pointer argument");
+    MD_CHECK_ARG(a->M > 0 && a->N > 0 && a->K > 0 && N2 > 0 && md_linear_fused_beside_supported(a->M, a->N, a->K, N2),
+                 "md_linear_fused_beside: unsupported shape M=%d N=%d K=%d N2=%d", a->M, a->N, a->K, N2);
+    MD_CHECK_ARG((a->epilogue == FL_SWIGLU || a->epilogue == FL_GEGLU) && !a->pro_ssq,
+                 "md_linear_fused_beside: the first product is a gated one of finished rows");
+    MD_CHECK_ARG(aligned16(w2_packed) && ((uintptr_t)out2 & 3) == 0 && ldo2 >= N2 && ldo2 % 2 == 0,
+                 "md_linear_fused_beside: the second weight must be 16-byte aligned, its rows 4-byte");
+    return run_fused(a, false, stream, w2_packed, N2, out2, ldo2);
+}

@@ -623,7 +623,6 @@ def linear_prompt(x, weight: "PackedWeight", bias=None, swiglu=False, out=None, 
     return out
 
 
-@functools.lru_cache(maxsize=4096)
 @functools.lru_cache(maxsize=1024)
 def linear_f32_supported(M, N, K):
     """True when md_linear_f32 (csrc/f32gemm.hip) takes this shape and is expected to be faster than the library."""
@@ -643,7 +642,6 @@ def linear_f32(x, weight, tile=0):
     return out
 
 
-@functools.lru_cache(maxsize=4096)
 @functools.lru_cache(maxsize=1024)
 def linear_f32_few_supported(M, N, K):
     """True when md_linear_f32_few (csrc/f32few.hip) takes this shape."""
@@ -663,7 +661,6 @@ def linear_f32_few(x, weight, tile=0):
     return out
 
 
-@functools.lru_cache(maxsize=4096)
 @functools.lru_cache(maxsize=1024)
 def linear_f32_thirds_supported(M, N, K):
     """True when md_linear_f32_thirds (csrc/f32thirds.hip) takes this shape and is expected to be the fastest."""
@@ -798,6 +795,25 @@ def fused_linear(x, weight: "PackedWeight", bias=None, swiglu=False, resid=None,
         _set_pro(a, x, pro)
     _run_fused(a, few)
     return (out, ssq) if want_ssq else out
+
+
+def fused_linear_beside_supported(M, N, K, N2):
+    """True when md_linear_fused_beside (csrc/tilegemm.hip) takes a gated product [M, N / 2] and a plain one [M, N2] together."""
+    return _lib.load().md_linear_fused_beside_supported(int(M), int(N), int(K), int(N2)) > 0
+
+
+def fused_linear_beside(x, weight: "PackedWeight", out, beside: "PackedWeight", gelu=False):
+    """fused_linear(x, weight, swiglu=True, gelu=gelu, out=out), and F.linear(x, W of `beside`), which is returned, in the same launch."""
+    a = _fused_args(x, weight, None, FL_GEGLU if gelu else FL_SWIGLU)
+    _gpu(out, beside.data)
+    if out.dtype != torch.bfloat16 or out.dim() != 2 or out.shape != (x.shape[0], weight.N // 2) or out.stride(1) != 1:
+        raise ValueError("fused linear: out must be bf16 [M, N / 2] with unit inner stride")
+    if beside.dtype != torch.bfloat16 or beside.swiglu or beside.K != weight.K:
+        raise ValueError("fused linear: the second weight must be a plain bf16 one of the same K")
+    a.out, a.ldo = out.data_ptr(), out.stride(0)
+    z = torch.empty((x.shape[0], beside.N), dtype=x.dtype, device=x.device)
+    check(_lib.load().md_linear_fused_beside(ctypes.byref(a), _p(beside.data), beside.N, _p(z), z.stride(0), _stream()), "md_linear_fused_beside")
+    return z
 
 
 def fused_qkv_rope_append(x, weight: "PackedWeight", bias, H, KH, D, rows_per_req, offsets, table: RopeTable, kv_cache,
