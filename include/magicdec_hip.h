@@ -580,6 +580,10 @@ typedef struct md_head_linear_args {
 } md_head_linear_args;
 int md_latent_row_width(int kv_rank, int rot_dim);    /* 0: unsupported */
 int md_latent_append(const md_latent_args* args, md_stream_t stream);
+/* md_latent_query: md_latent_append of a step's M <= 64 bf16 rows without cq, and q[M][N] = cq . W^T (W in md_linear's streaming layout) in the same
+ * launch; N % 32 == 0, q_rank % 256 == 0, <= 1536.  _supported: 1 if it takes the shape (negative: no shape). */
+int md_latent_query_supported(int M, int N, int q_rank);
+int md_latent_query(const md_latent_args* args, const void* w_packed, void* q, int64_t ldq, int M, int N, md_stream_t stream);
 size_t md_latent_workspace_bytes(const md_latent_args* args);
 int md_latent_attn(const md_latent_args* args, md_stream_t stream);
 int md_latent_gather(const md_latent_args* args, int ctx_max, void* dst, md_stream_t stream);

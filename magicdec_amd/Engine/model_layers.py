@@ -441,8 +441,11 @@ class LayeredTransformer(Transformer):
         gated = z is not None
         if not gated:
             z = self._linear(y, att.win)
-        cq = ops.latent_append(z, s, cache, rows, tab.indices, tab.indptr, tab.max_pages)
-        q = self._linear(cq, att.wuq)
+        wuq = self._packed.get(id(att.wuq.weight))
+        if wuq is not None and y.shape[0] <= 64 and ops.latent_query_supported(z, s, wuq, cache):
+            q = ops.latent_query(z, s, wuq, cache, rows, tab.indices, tab.indptr, tab.max_pages)
+        else:
+            q = self._linear(ops.latent_append(z, s, cache, rows, tab.indices, tab.indptr, tab.max_pages), att.wuq)
         if ctx is not None:
             ctx.expand = functools.partial(self._linear, lin=att.wukv)
         heads = side[:, :layer.heads_out].unflatten(1, (s.H, s.vdim))

@@ -148,6 +148,8 @@ _SIGNATURES = {
     "md_qk_norm_append": (c_int, [ctypes.POINTER(XattnArgs), P, P]),
     "md_xattn": (c_int, [ctypes.POINTER(XattnArgs), P]),
     "md_latent_row_width": (c_int, [I, I]),
+    "md_latent_query_supported": (c_int, [I, I, I]),
+    "md_latent_query": (c_int, [ctypes.POINTER(LatentArgs), P, P, L, I, I, P]),
     "md_latent_append": (c_int, [ctypes.POINTER(LatentArgs), P]),
     "md_latent_workspace_bytes": (c_size_t, [ctypes.POINTER(LatentArgs)]),
     "md_latent_attn": (c_int, [ctypes.POINTER(LatentArgs), P]),

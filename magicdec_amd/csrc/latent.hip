@@ -9,6 +9,7 @@
 //              head with dim + rot_dim and vdim numbers: several times fewer operations per (query, key): prompts.
 //
 //   md_latent_append     query latent -> weighted RMS norm; latent -> weighted RMS norm, key part -> rotation, both -> cache
+//   md_latent_query      both for a step's rows, and the queries of the normalised query latents, in one launch
 //   md_head_linear       y[row][h] = W_h x[row][h]: the absorbed queries (+ their rotated part) and the way out of the latent
 //                        (* sigmoid of the head's gate)
 //   md_latent_attn       the absorbed form over the cache; 32-bit and unusual sizes run the fp32 attention kernels of xattn_f32.hip or,
@@ -80,19 +81,9 @@ __device__ __forceinline__ float rotated(const T* x, int d, int pairs, const flo
     return d & 1 ? a * c + b * s : a * c - b * s;
 }
 
-// two wavefronts per row: one normalises the query latent, the other the latent and rotates the key part
+// row j of request b, a row of z: its latent, normalised, and its key part, rotated, to its position's cache row; by one wavefront
 template <typename T, int VEC>
-__global__ __launch_bounds__(256) void latent_append_kernel(const LatentParams p) {
-    const int b = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int q0 = p.qo_indptr[b], j = blockIdx.x * 2 + (wave >> 1);
-    if (j >= p.qo_indptr[b + 1] - q0) return;
-    const T* row = reinterpret_cast<const T*>(p.z) + (int64_t)(q0 + j) * p.ldz;
-    if ((wave & 1) == 0) {
-        norm_row<T, VEC>(row, reinterpret_cast<const T*>(p.dq_norm), reinterpret_cast<T*>(p.cq) + (int64_t)(q0 + j) * p.q_rank,
-                         p.q_rank, p.eps, lane);
-        return;
-    }
-    if (!p.append) return;
+__device__ __forceinline__ void append_row(const LatentParams& p, const T* row, int b, int j, int lane) {
     const int pos = p.pos0[b] + j, pg0 = p.page_indptr[b];
     if (pos < 0 || pos >= (p.page_indptr[b + 1] - pg0) * p.page_size || pos >= p.max_pos) {
         if (lane == 0) atomicAdd(p.overflow, 1u);
@@ -105,6 +96,106 @@ __global__ __launch_bounds__(256) void latent_append_kernel(const LatentParams p
     const float* cs = p.cos_sin + (int64_t)pos * p.rot_pairs * 2;
     for (int d = lane; d < p.W - p.kv_rank; d += 64)
         dst[p.kv_rank + d] = d < p.rot_dim ? (T)rotated(src + p.kv_rank, d, p.rot_pairs, cs) : (T)0.f;
+}
+
+// two wavefronts per row: one normalises the query latent, the other the latent and rotates the key part
+template <typename T, int VEC>
+__global__ __launch_bounds__(256) void latent_append_kernel(const LatentParams p) {
+    const int b = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int q0 = p.qo_indptr[b], j = blockIdx.x * 2 + (wave >> 1);
+    if (j >= p.qo_indptr[b + 1] - q0) return;
+    const T* row = reinterpret_cast<const T*>(p.z) + (int64_t)(q0 + j) * p.ldz;
+    if ((wave & 1) == 0) {
+        norm_row<T, VEC>(row, reinterpret_cast<const T*>(p.dq_norm), reinterpret_cast<T*>(p.cq) + (int64_t)(q0 + j) * p.q_rank,
+                         p.q_rank, p.eps, lane);
+        return;
+    }
+    if (p.append) append_row<T, VEC>(p, row, b, j, lane);
+}
+
+// ------------------------------------------------------------------------------------------------ queries of a step
+// q[M][N] = rms(query latent) * dq_norm . W^T with W in the streaming layout [N/32][K/16][64][8] (K = 256 STEPS), and beside it, in workgroups
+// behind the product's, the append.  A workgroup has 32 rows x 32 columns, each of its sixteen wavefronts a sixteenth of K: all that a wavefront
+// reads is requested at once, the norm is formed of what it holds while the weight is on its way, and its bits are latent_append_kernel's.
+//
+// A chain of latencies bounds a step of few rows: as launches of their own the norm and append take 4.6 us and the product 4.6 (32 rows of
+// 3 072 x 768), this 5.3.
+template <int STEPS>
+__global__ __launch_bounds__(1024, 4) void latent_query_kernel(const LatentParams p, const bf16_t* w, bf16_t* q, int64_t ldq, int M, int N) {
+    constexpr int NW = 16, K = 16 * NW * STEPS;
+    __shared__ float part[NW * 32];
+    extern __shared__ __attribute__((aligned(16))) float red[];            // [NW][32][32]
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 31, kh = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), m_tiles = (M + 31) / 32, tiles = N / 32 * m_tiles;
+    const bf16_t* z = reinterpret_cast<const bf16_t*>(p.z);
+    if ((int)blockIdx.x >= tiles) {
+        const int row = ((int)blockIdx.x - tiles) * NW + wave;
+        if (row >= M) return;
+        int b = 0;                                                          // requests that end in front of the row
+        for (int i = 0; i < p.B; i += 64) b += __popcll(__builtin_amdgcn_ballot_w64(i + lane < p.B && p.qo_indptr[i + lane + 1] <= row));
+        if (b < p.B) append_row<bf16_t, 8>(p, z + (int64_t)row * p.ldz, b, row - p.qo_indptr[b], lane);
+        return;
+    }
+    const int tn = blockIdx.x / m_tiles, m0 = (int)blockIdx.x % m_tiles * 32, k0 = wave * STEPS * 16 + kh * 8;
+    const bf16_t* xp = z + (int64_t)min(m0 + j, M - 1) * p.ldz + k0;
+    const bf16_t* gp = reinterpret_cast<const bf16_t*>(p.dq_norm) + k0;
+    const bf16_t* wp = w + ((int64_t)tn * (K / 16) + wave * STEPS) * 512 + lane * 8;
+    bf16x8 x[STEPS], g[STEPS], b[STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) x[s] = *reinterpret_cast<const bf16x8*>(xp + s * 16);
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) g[s] = *reinterpret_cast<const bf16x8*>(gp + s * 16);
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) b[s] = *reinterpret_cast<const bf16x8*>(wp + s * 512);
+    float ss = 0.f;
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += (float)x[s][e] * (float)x[s][e];
+    ss += __shfl_xor(ss, 32);
+    if (kh == 0) part[wave * 32 + j] = ss;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                      // (the weight stays on its way)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) t += part[i * 32 + j];
+    const float rs = 1.0f / sqrtf(t / (float)K + p.eps);
+    typedef float f32x16 __attribute__((ext_vector_type(16)));
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+        bf16x8 a;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a[e] = (bf16_t)(((float)x[s][e] * rs) * (float)g[s][e]);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[s], acc, 0, 0, 0);
+    }
+    // acc[r]: row (r & 3) + 8 (r >> 2) + 4 kh, column j
+#pragma unroll
+    for (int r = 0; r < 16; ++r) red[wave * 1024 + ((r & 3) + 8 * (r >> 2) + 4 * kh) * 32 + j] = acc[r];
+    __syncthreads();
+    const int row = tid >> 5, col = tid & 31;
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) sum += red[i * 1024 + tid];
+    if (m0 + row < M) q[(int64_t)(m0 + row) * ldq + tn * 32 + col] = (bf16_t)sum;
+}
+
+template <int STEPS>
+int launch_query(const LatentParams& p, const bf16_t* w, bf16_t* q, int64_t ldq, int M, int N, hipStream_t st) {
+    constexpr int bytes = 16 * 4096;
+    static MdPerDeviceOnce once;
+    if (once.first() && hipFuncSetAttribute(reinterpret_cast<const void*>(&latent_query_kernel<STEPS>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
+        once.undo();
+        md_set_error("md_latent_query: hipFuncSetAttribute(LDS) failed");
+        return MD_ERR_LAUNCH;
+    }
+    const int blocks = N / 32 * ((M + 31) / 32) + (p.append ? (M + 15) / 16 : 0);
+    hipLaunchKernelGGL((latent_query_kernel<STEPS>), dim3(blocks), dim3(1024), bytes, st, p, w, q, ldq, M, N);
+    return MD_OK;
 }
 
 // ------------------------------------------------------------------------------------------------ per-head linear
@@ -465,6 +556,41 @@ extern "C" int md_latent_append(const md_latent_args* a, md_stream_t stream) {
         else hipLaunchKernelGGL((latent_append_kernel<bf16_t, 1>), grid, dim3(256), 0, st, p);
     }
     MD_CHECK_LAUNCH("md_latent_append");
+    return MD_OK;
+}
+
+extern "C" int md_latent_query_supported(int M, int N, int q_rank) {
+    MD_CHECK_ARG(M > 0 && N > 0 && q_rank > 0, "md_latent_query_supported: M=%d N=%d q_rank=%d", M, N, q_rank);
+    // a workgroup a CU: 64 rows of 3 072 columns, not of 6 144 (384 workgroups: four layers 571 us a step as two launches, 582 as one)
+    return M <= 64 && N % 32 == 0 && N / 32 * ((M + 31) / 32) <= 256 && q_rank % 256 == 0 && q_rank <= 1536 ? 1 : 0;
+}
+
+extern "C" int md_latent_query(const md_latent_args* a, const void* w_packed, void* q, int64_t ldq, int M, int N, md_stream_t stream) {
+    const int rc = check_args("md_latent_query", a);
+    if (rc != MD_OK) return rc;
+    MD_CHECK_ARG(a->z && a->dq_norm && w_packed && q, "md_latent_query: null pointer argument");
+    MD_CHECK_ARG(M > 0 && N > 0 && a->q_rank > 0 && md_latent_query_supported(M, N, a->q_rank) && a->dtype == MD_T_BF16 && ldq >= N,
+                 "md_latent_query: M=%d N=%d q_rank=%d unsupported", M, N, a->q_rank);
+    MD_CHECK_ARG(!a->append || (a->kv_norm && a->cos_sin && a->max_pos > 0), "md_latent_query: the append needs kv_norm and the angle table");
+    MD_CHECK_ARG(a->ldz >= a->q_rank + (a->append ? a->kv_rank + a->rot_dim : 0) && a->ldz % 8 == 0 && a->kv_rank % 8 == 0 && aligned(a->z, 16) &&
+                     aligned(a->dq_norm, 16) && aligned(w_packed, 16) && aligned(a->cache, 32) && (!a->append || aligned(a->kv_norm, 16)),
+                 "md_latent_query: rows of %lld elements, or operands that are not 16-byte aligned", (long long)a->ldz);
+    const LatentParams p = make_params(a);
+    MD_CHECK_ARG(p.overflow, "md_latent_query: cannot resolve the page-overflow counter");
+    const bf16_t* w = (const bf16_t*)w_packed;
+    bf16_t* out = (bf16_t*)q;
+    hipStream_t st = (hipStream_t)stream;
+    int r = MD_OK;
+    switch (a->q_rank / 256) {
+    case 1: r = launch_query<1>(p, w, out, ldq, M, N, st); break;
+    case 2: r = launch_query<2>(p, w, out, ldq, M, N, st); break;
+    case 3: r = launch_query<3>(p, w, out, ldq, M, N, st); break;
+    case 4: r = launch_query<4>(p, w, out, ldq, M, N, st); break;
+    case 5: r = launch_query<5>(p, w, out, ldq, M, N, st); break;
+    default: r = launch_query<6>(p, w, out, ldq, M, N, st);
+    }
+    if (r != MD_OK) return r;
+    MD_CHECK_LAUNCH("md_latent_query");
     return MD_OK;
 }
 

@@ -1215,6 +1215,29 @@ def latent_append(z, s: LatentSpec, cache, rows: StepRows, page_indices, page_in
     return cq
 
 
+def latent_query_supported(z, s: LatentSpec, weight: "PackedWeight", cache):
+    """True when md_latent_query takes the rows z: a step's, bf16, dense enough for whole pieces."""
+    return (z.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and not weight.swiglu and weight.K == s.q_rank and z.stride(0) % 8 == 0
+            and s.kv_rank % 8 == 0 and not (z.data_ptr() | s.dq_norm.data_ptr() | (s.kv_norm.data_ptr() if s.kv_norm is not None else 0)) % 16
+            and cache.data_ptr() % 32 == 0 and _lib.load().md_latent_query_supported(z.shape[0], weight.N, s.q_rank) > 0)
+
+
+def latent_query(z, s: LatentSpec, weight: "PackedWeight", cache, rows: StepRows, page_indices, page_indptr, max_pages):
+    """F.linear(latent_append(z, ...), W) of a step's rows in one launch (md_latent_query); the query latents are not kept."""
+    _gpu(z, weight.data)
+    if z.dim() != 2 or z.stride(1) != 1 or z.shape[1] < s.q_rank + (s.kv_rank + s.rot_dim if s.kv_norm is not None else 0):
+        raise ValueError("latent_query: rows must hold the query latent, the latent and the key part")
+    if z.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or weight.swiglu or weight.K != s.q_rank:
+        raise ValueError("latent_query: bf16 rows and a plain bf16 weight of q_rank columns expected")
+    a = _latent_args(s, cache, rows, page_indices, page_indptr, max_pages, z.dtype)
+    a.z, a.ldz, a.dq_norm = z.data_ptr(), z.stride(0), s.dq_norm.data_ptr()
+    if s.kv_norm is not None:
+        a.kv_norm, a.append = s.kv_norm.data_ptr(), 1
+    q = torch.empty((z.shape[0], weight.N), dtype=z.dtype, device=z.device)
+    check(_lib.load().md_latent_query(ctypes.byref(a), _p(weight.data), _p(q), q.stride(0), z.shape[0], weight.N, _stream()), "md_latent_query")
+    return q
+
+
 def head_linear(x, w, out, gate=None):
     """out[:, h] = x[:, h] . w[h]^T (* sigmoid(gate[:, h])) for x [M, H, K], w [H, N, K], out [M, H, >= N] (strides free in the
     first two dimensions)."""
