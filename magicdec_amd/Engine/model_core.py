@@ -614,8 +614,8 @@ class Transformer(nn.Module):
             return self._prompt_linear(x2d if pro is None else pro.materialize(), pk, bias, swiglu)
         if how == "fused" and ops.fused_linear_supported(M, N, K):
             # few rows: on finer tiles, which also take a norm in front of a head
-            few = (not swiglu and ops.few_linear_supported(M, N, K)
-                   and (use_few(M, N, K) or (pro is not None and resid is None and fused_mode() == "auto")))
+            few = (M <= 16 and not swiglu and (use_few(M, N, K) or (pro is not None and resid is None and fused_mode() == "auto"))
+                   and ops.few_linear_supported(M, N, K))
             if pro is not None and not swiglu and not few:
                 x2d, pro = pro.materialize(), None
             return ops.fused_linear(x2d, pk, bias, swiglu=swiglu, resid=resid, want_ssq=want_ssq, pro=pro, few=few)

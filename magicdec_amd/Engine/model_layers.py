@@ -423,7 +423,7 @@ class LayeredTransformer(Transformer):
     def _gated_beside(self, y, layer, out):
         """_gated into `out` and the product into the latents, which is returned, in one launch where the tile kernel runs both; else None."""
         M = y.shape[0]
-        if layer.w13 is None or M > 256 or not y.is_cuda or y.dtype != torch.bfloat16:
+        if layer.w13 is None or not y.is_cuda or y.dtype != torch.bfloat16:
             return None
         gate, win = (self._packed.get(id(w.weight)) for w in (layer.w13, layer.attention.win))
         if (gate is None or win is None or win.dtype != torch.bfloat16 or out.stride(0) % 8 or out.data_ptr() % 16
@@ -437,12 +437,13 @@ class LayeredTransformer(Transformer):
         att, s = layer.attention, self._xspec[i]
         cache = att.kv_cache.rows
         side = torch.empty((y.shape[0], layer.wout.weight.shape[1]), dtype=y.dtype, device=y.device)
-        z = self._gated_beside(y, layer, side[:, layer.heads_out:])
+        right = side[:, layer.heads_out:] if layer.w13 is not None else None
+        z = self._gated_beside(y, layer, right) if y.shape[0] <= 64 else None                  # (a step's rows)
         gated = z is not None
         if not gated:
             z = self._linear(y, att.win)
-        wuq = self._packed.get(id(att.wuq.weight))
-        if wuq is not None and y.shape[0] <= 64 and ops.latent_query_supported(z, s, wuq, cache):
+        wuq = self._packed.get(id(att.wuq.weight)) if y.shape[0] <= 64 else None
+        if wuq is not None and ops.latent_query_supported(z, s, wuq, cache):
             q = ops.latent_query(z, s, wuq, cache, rows, tab.indices, tab.indptr, tab.max_pages)
         else:
             q = self._linear(ops.latent_append(z, s, cache, rows, tab.indices, tab.indptr, tab.max_pages), att.wuq)
@@ -452,7 +453,7 @@ class LayeredTransformer(Transformer):
         ops.latent_attention(q, s, cache, rows, tab.indices, tab.indptr, tab.max_pages, self.workspace, heads,
                              gate=z[:, sum(att.cuts) - s.H:sum(att.cuts)] if att.spec.gate else None, ctx=ctx)
         if layer.w13 is not None and not gated:
-            self._gated(y, layer.w13, side[:, layer.heads_out:])
+            self._gated(y, layer.w13, right)
         return self._project(side, layer.wout)
 
     def _embed(self, flat, rows, tab: PageTable):

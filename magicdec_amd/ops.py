@@ -291,6 +291,7 @@ MD_W_BF16, MD_W_INT8 = 0, 1
 EPI_NONE, EPI_SWIGLU, EPI_GEGLU = 0, 1, 3
 
 
+@functools.lru_cache(maxsize=1024)
 def linear_supported(M, N, K, swiglu=False):
     """True when md_linear (the weight-streaming skinny GEMM) takes this shape; otherwise use a library GEMM."""
     return bool(_lib.load().md_linear_supported(int(M), int(N), int(K), EPI_SWIGLU if swiglu else EPI_NONE))
@@ -506,6 +507,7 @@ def fused_split_linear_add_rmsnorm(x, weight: "PackedWeight", resid, norm_weight
 
 
 # ----------------------------------------------------------------------------- K8c
+@functools.lru_cache(maxsize=1024)
 def linear_block_supported(M, N, K, swiglu=False):
     """True when md_linear_block (csrc/blockgemm.hip: the block-tile GEMM of the 129..256-row verify linears) takes
     this shape (M <= 256, N % 128 == 0, K % 64 == 0)."""
@@ -698,6 +700,7 @@ def linear_f32_thirds(x, weight, tile=0):
 FL_NONE, FL_SWIGLU, FL_RESID, FL_ROPE_APPEND, FL_XIELU, FL_GEGLU = 0, 1, 2, 3, 4, 5
 
 
+@functools.lru_cache(maxsize=1024)
 def fused_linear_supported(M, N, K, epilogue=FL_NONE):
     """True when md_linear_fused (csrc/tilegemm.hip) takes this shape."""
     return bool(_lib.load().md_linear_fused_supported(int(M), int(N), int(K), int(epilogue)))
@@ -720,6 +723,7 @@ def _fused_args(x, weight: "PackedWeight", bias, epilogue):
     return a
 
 
+@functools.lru_cache(maxsize=1024)
 def few_linear_supported(M, N, K, epilogue=FL_NONE):
     """True when md_linear_few (csrc/tilegemm.hip) takes this shape."""
     return _lib.load().md_linear_few_supported(int(M), int(N), int(K), int(epilogue)) > 0
@@ -797,6 +801,7 @@ def fused_linear(x, weight: "PackedWeight", bias=None, swiglu=False, resid=None,
     return (out, ssq) if want_ssq else out
 
 
+@functools.lru_cache(maxsize=1024)
 def fused_linear_beside_supported(M, N, K, N2):
     """True when md_linear_fused_beside (csrc/tilegemm.hip) takes a gated product [M, N / 2] and a plain one [M, N2] together."""
     return _lib.load().md_linear_fused_beside_supported(int(M), int(N), int(K), int(N2)) > 0
