@@ -31,7 +31,7 @@ lowest-index tie-break.
 """
 from __future__ import annotations
 
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 from typing import Optional
 
 import torch
@@ -897,6 +897,10 @@ class Transformer(nn.Module):
             raise ValueError(f"SnapKV select needs the last prefill chunk to be exactly window_size="
                              f"{self.window_size} tokens, got {tail or n} ((prefix_len - window_size) % 128 != 0)")
         self._snap_ctx_len = ctx_len
+        if ctx_len is not None:                                  # the attention's plan: pages of this portion, not of the cache
+            kvc = self.layers[0].attention.kv_cache
+            page = kvc.kv_cache.shape[2 if kvc.layout_of("kv_cache") == "NHD" else 3]
+            tab = replace(tab, max_pages=min(tab.max_pages, -(-ctx_len // page)))
         rows = None
         if tail is not None and not self.skip_head:
             rows = (torch.arange(B, device=idx.device).view(B, 1) * n + torch.arange(n - tail, n, device=idx.device)).flatten()

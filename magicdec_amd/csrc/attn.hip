@@ -932,7 +932,7 @@ __global__ __launch_bounds__(64 * NW, 2) void prefill_attn_kernel(const AttnPara
 // Measured and NOT kept (same box, profiles/r03_prefill_mfma32_ab.txt): s_setprio(1) around the MFMA clusters (808 vs 820
 // TFLOP/s), the causal mask as a compile-time property of the tile body (two bodies: 480 -- the register file again), the
 // MFMAs of one accumulator issued back to back instead of alternating accumulators (795 vs 817).
-template <int D, int NW, int KT, bool VP = true>
+template <int D, int NW, int KT, bool VP = true, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW, D == 64 && KT == 64 ? 4 : 2) void prefill32_attn_kernel(const AttnParams p) {
     constexpr int KG = KT / 32;            // 32-key blocks per tile
     constexpr int CH = D * 2 / 16;
@@ -957,8 +957,10 @@ __global__ __launch_bounds__(64 * NW, D == 64 && KT == 64 ? 4 : 2) void prefill3
     const int bid = blockIdx.x;
     const int xcd = bid & 7;
     const int r0 = bid >> 3;
-    const int qg = p.n_qgroups - 1 - r0 % p.n_qgroups;     // a pair's longest groups (last rows) first: the last to start is the last to end
-    const int pair = (r0 / p.n_qgroups) * 8 + xcd;
+    // a pair's longest groups (last rows) first: the last to start is the last to end.  SPLIT: a group's keys over nsplit workgroups
+    const int parts = SPLIT ? p.nsplit : 1, sub = r0 % (p.n_qgroups * parts), split = SPLIT ? sub % parts : 0;
+    const int qg = p.n_qgroups - 1 - sub / parts;
+    const int pair = (r0 / (p.n_qgroups * parts)) * 8 + xcd;
     if (pair >= p.B * p.KH) return;
     const int b = pair / p.KH, kvh = pair % p.KH;
     const int g = p.g;
@@ -973,7 +975,7 @@ __global__ __launch_bounds__(64 * NW, D == 64 && KT == 64 ? 4 : 2) void prefill3
     // fewer, groups begin with the first row: the one with the most keys is the one that may have few (4 x 901 rows, 16 heads on 2 37 us,
     // 39 otherwise; 4 x 846, 32 heads on 32 60 and 65)
     constexpr unsigned kTwoRounds = D == 64 && KT == 64 ? 1024 : 512;
-    const int R0 = qg * NW * 32 - (gridDim.x > kTwoRounds ? (NW * 32 - 1 - (nrows - 1) % (NW * 32)) / g * g : 0), R = R0 + wave * 32 + j;
+    const int R0 = qg * NW * 32 - (!SPLIT && gridDim.x > kTwoRounds ? (NW * 32 - 1 - (nrows - 1) % (NW * 32)) / g * g : 0), R = R0 + wave * 32 + j;
     const bool valid = R >= 0 && R < nrows;
     const int qi = R / g, qr = R - qi * g;
     const int lim = valid ? (p.causal ? kv_len - n_b + qi : kv_len - 1) : -1;
@@ -993,6 +995,7 @@ __global__ __launch_bounds__(64 * NW, D == 64 && KT == 64 ? 4 : 2) void prefill3
     for (int w = 0; w < NW; ++w) kv_end_wg = max(kv_end_wg, s_end[w]);
     const int ntiles_wg = kv_end_wg > 0 ? (kv_end_wg + KT - 1) / KT : 0;
     const int my_ntiles = kv_end > 0 ? (kv_end + KT - 1) / KT : 0;
+    const int per = SPLIT ? (ntiles_wg + parts - 1) / parts : ntiles_wg, t0 = split * per, t1 = SPLIT ? min(ntiles_wg, t0 + per) : ntiles_wg;
 
     bf16x8 qf[KS];
     {
@@ -1025,7 +1028,7 @@ __global__ __launch_bounds__(64 * NW, D == 64 && KT == 64 ? 4 : 2) void prefill3
     // numbers of 64 pages, one a lane: no load in front of a tile's.  33 rows of 4 heads behind 2048 keys (64 workgroups) 77 -> 70 us; with
     // the order of the groups, the odd rows first and whole output rows: 4 x 2048 rows, 32 heads of 128 on 8 kv heads 236 -> 199, 16
     // portions of 512 rows, heads of 64 behind a window 42 -> 38
-    int pages = npages > 0 ? p.page_indices[pg0 + min(lane, npages - 1)] : 0;
+    int pages = npages > 0 ? p.page_indices[pg0 + min((SPLIT ? t0 * KT / p.page_size & ~63 : 0) + lane, npages - 1)] : 0;
     asm volatile("" : "+v"(pages));
     auto issue = [&](int tt) {
         const int pos0 = tt * KT;
@@ -1146,16 +1149,32 @@ __global__ __launch_bounds__(64 * NW, D == 64 && KT == 64 ? 4 : 2) void prefill3
                 for (int db = 0; db < DB; ++db) pv(db, kg, s16);
     };
 
-    if (ntiles_wg > 0) issue(0);
-    for (int t = 0; t < ntiles_wg; ++t) {
+    if (t0 < t1) issue(t0);
+    for (int t = t0; t < t1; ++t) {
         unsigned char* img = smem + (t & 1) * STAGE;
         stage(t, img);
-        if (t + 1 < ntiles_wg) issue(t + 1);
+        if (t + 1 < t1) issue(t + 1);
         __syncthreads();
         if (t < my_ntiles) compute(t, img, (t * KT + KT - 1) > lo);
     }
 
     l += __shfl_xor(l, 32);
+    if constexpr (SPLIT) {                                 // sums, reference and weight of its keys: attn_merge_kernel
+        if (!valid) return;
+        const int64_t slot = (((int64_t)pair * p.n_qgroups + qg) * parts + split) * (NW * 32) + wave * 32 + j;
+        if (kh == 0) {
+            p.ws_ml[slot * 2] = m;
+            p.ws_ml[slot * 2 + 1] = l;
+        }
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+            for (int rg = 0; rg < 4; ++rg) {
+                const int ch = VP ? (db + (rg >> 1) * (NB / 2)) * 2 + (rg & 1) : db * 4 + rg;
+                *reinterpret_cast<f32x4*>(p.ws_o + slot * D + ch * 8 + kh * 4) = f32x4{o[db][rg * 4], o[db][rg * 4 + 1], o[db][rg * 4 + 2], o[db][rg * 4 + 3]};
+            }
+        return;
+    }
     // output rows through LDS: a store writes whole rows
     const float inv = l > 0.f ? 1.0f / l : 0.f;
     __syncthreads();                                       // every wave is past the last image
@@ -1201,7 +1220,9 @@ int g_time_rows = 0;
 bool g_time_this = false;  // set by md_paged_attn for the launch it is about to make
 std::vector<TimedLaunch> g_timed;
 
-AttnPlan make_plan(int B, int n_max, int H, int KH, int max_pages, int page_size, bool fp8) {
+int g_prefill_mfma32 = -1;   // dev knob: see launch_prefill
+
+AttnPlan make_plan(int B, int n_max, int H, int KH, int D, int max_pages, int page_size, bool fp8) {
     AttnPlan pl;
     pl.nw = 4;
     const int g = H / KH;
@@ -1248,7 +1269,15 @@ AttnPlan make_plan(int B, int n_max, int H, int KH, int max_pages, int page_size
         const int wg_rows = 16 * pl.qt * pl.nw;
         pl.n_qgroups = (rows + wg_rows - 1) / wg_rows;
         pl.nsplit = 1;
-        pl.rows_cap = 0;
+        pl.rows_cap = wg_rows;
+        // Few groups behind a long context (a prompt's last portion): the keys of a group over several workgroups, up to a CU each, of six
+        // 64-key tiles of what lies in front of the portion at least.  us, whole / split: 33 rows of 4 requests behind 2 048 keys, 32 heads of
+        // 128 on 8 (64 workgroups) 60.9 / 29.5, one request of 400 73 / 41, 900 (120) 89 / 67, 128 behind 7 000 190 / 38; heads of 64 41 / 20,
+        // 56 / 31, 68 / 51, 148 / 31.  Not by the portion's own keys (1 000 from the first on 36.8 / 39.8: the merge,
+        // and most groups have few), nor for a short past (4 x 128 behind 385, four tiles: 24.9 / 33.3)
+        const long wgs = ((long)B * KH + 7) / 8 * 8 * pl.n_qgroups, past = ((long)max_pages * page_size - n_max) / 64;
+        if (!fp8 && pl.qt == 2 && g_prefill_mfma32 < 0 && page_size % (D == 128 && pl.nw == 8 ? 128 : 64) == 0 && wgs <= 128)
+            pl.nsplit = (int)std::max(1L, std::min({256 / wgs, past / 6, 16L}));
     }
     return pl;
 }
@@ -1319,12 +1348,11 @@ int launch_prefill_kt(const AttnParams& p, int grid, hipStream_t st) {
 // Dev knob (md_debug_set_prefill_mfma32 / MAGICDEC_PREFILL_MFMA32): -1 = this rule, 0 = the 16x16x32 kernel, 32 | 64 | 128 forced
 // (halved until it divides the page size), 129 = first V pairing.  (The two timing ablations of docs/DESIGN_r1_r5_lab_notes.md 3.5 -- no
 // softmax / no P.V, wrong results by construction -- were removed after the measurement.)
-int g_prefill_mfma32 = -1;
 
-template <int D, int NW, int KT, bool VP = true>
+template <int D, int NW, int KT, bool VP = true, bool SPLIT = false>
 int launch_prefill32_kt(const AttnParams& p, int grid, hipStream_t st) {
     constexpr int lds = std::max(2 * prefill_stage_bytes<D, KT>() + 32, NW * 32 * D * 2);      // tile images; output rows
-    auto k = prefill32_attn_kernel<D, NW, KT, VP>;
+    auto k = prefill32_attn_kernel<D, NW, KT, VP, SPLIT>;
     if (lds > 64 * 1024) {
         static MdPerDeviceOnce once;
         if (once.first()) {
@@ -1346,6 +1374,8 @@ int launch_prefill(const AttnParams& p, int grid, int nw, hipStream_t st) {
     // a shared tile never crosses a page: keys per tile must divide the page size (32 always does, md_paged_attn checks)
     const auto fits = [&](int kt) { return p.page_size % kt == 0; };
     if constexpr (!FP8 && QT == 2) {
+        if (p.nsplit > 1)
+            return nw == 8 ? launch_prefill32_kt<D, 8, D == 128 ? 128 : 64, true, true>(p, grid, st) : launch_prefill32_kt<D, 4, 64, true, true>(p, grid, st);
         if constexpr (D == 128)
             if (nw == 8 && fits(128)) {      // dev variants of the 128-key kernel (md_debug_set_prefill_mfma32)
                 if (g_prefill_mfma32 == 129) return launch_prefill32_kt<D, 8, 128, false>(p, grid, st);    // first V pairing
@@ -1411,9 +1441,9 @@ extern "C" int md_debug_attn_timing_read(float* ms_out, int cap) {
 extern "C" size_t md_paged_attn_workspace_bytes(int B, int n_max, int H, int KH, int D,
                                                 int max_pages_per_req, int page_size) {
     if (B <= 0 || KH <= 0 || H % KH != 0) return 0;
-    const AttnPlan pl = make_plan(B, n_max, H, KH, max_pages_per_req, page_size, false);
-    if (pl.splitq || pl.nsplit == 1) return 256;
-    const size_t slots = (size_t)B * KH * pl.nsplit * pl.rows_cap;
+    const AttnPlan pl = make_plan(B, n_max, H, KH, D, max_pages_per_req, page_size, false);
+    if (pl.nsplit == 1) return 256;
+    const size_t slots = (size_t)B * KH * pl.n_qgroups * pl.nsplit * pl.rows_cap;
     return slots * (size_t)D * 4 + slots * 8 + 256;
 }
 
@@ -1444,7 +1474,7 @@ extern "C" int md_paged_attn(const void* q, int64_t q_row_stride, const void* ca
                  "md_paged_attn: kv_dtype must be MD_KV_BF16 or MD_KV_FP8_E4M3 (with per-head scales)");
     const bool fp8 = kv_dtype == MD_KV_FP8_E4M3;
 
-    const AttnPlan pl = make_plan(B, n_max, H, KH, max_pages_per_req, page_size, fp8);
+    AttnPlan pl = make_plan(B, n_max, H, KH, D, max_pages_per_req, page_size, fp8);
     AttnParams p;
     p.q = (const bf16_t*)q;
     p.cache = cache;
@@ -1466,15 +1496,16 @@ extern "C" int md_paged_attn(const void* q, int64_t q_row_stride, const void* ca
     p.g = H / KH;
     p.page_size = page_size;
     p.causal = causal ? 1 : 0;
+    const size_t slots = (size_t)B * KH * pl.n_qgroups * pl.nsplit * pl.rows_cap, need = slots * (size_t)D * 4 + slots * 8;
+    const bool room = workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0;
+    if (pl.splitq && !room) pl.nsplit = 1;                       // (a prompt's keys are split where there is room for it)
     p.nsplit = pl.nsplit;
     p.n_qgroups = pl.n_qgroups;
     p.scale_log2 = sm_scale * 1.4426950408889634f;
     p.ws_o = nullptr;
     p.ws_ml = nullptr;
-    if (!pl.splitq && pl.nsplit > 1) {
-        const size_t slots = (size_t)B * KH * pl.nsplit * pl.rows_cap;
-        const size_t need = slots * (size_t)D * 4 + slots * 8;
-        if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15)) {
+    if (pl.nsplit > 1) {
+        if (!room) {
             md_set_error("md_paged_attn: workspace too small or misaligned (%zu < %zu)", workspace_bytes, need);
             return MD_ERR_WORKSPACE;
         }
@@ -1496,7 +1527,7 @@ extern "C" int md_paged_attn(const void* q, int64_t q_row_stride, const void* ca
         rc = fp8 ? MD_ATTN_DISPATCH(64, true) : MD_ATTN_DISPATCH(64, false);
 #undef MD_ATTN_DISPATCH
     if (rc != MD_OK) return rc;
-    if (!pl.splitq && pl.nsplit > 1) {
+    if (pl.nsplit > 1) {
         if (D == 128)
             launch_merge<128>(p, pl.rows_cap, st);
         else
