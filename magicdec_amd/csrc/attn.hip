@@ -1222,16 +1222,26 @@ std::vector<TimedLaunch> g_timed;
 
 int g_prefill_mfma32 = -1;   // dev knob: see launch_prefill
 
-AttnPlan make_plan(int B, int n_max, int H, int KH, int D, int max_pages, int page_size, bool fp8) {
+// split: with scratch for more than 32 rows, too
+AttnPlan make_plan(int B, int n_max, int H, int KH, int D, int max_pages, int page_size, bool fp8, bool split) {
     AttnPlan pl;
     pl.nw = 4;
     const int g = H / KH;
     const int rows = n_max * g;
-    if (rows <= 32) {
+    // 33 to 127 rows behind a long past (a verify step of many rows, the last few of a prompt): as one group a pair they walk the keys alone.
+    // fp8 pages, and 33 to 64 bf16 rows of 128 of more pairs than half the CUs, go in groups of 32 through the decode kernel; other bf16 rows
+    // split their keys in the prefill kernel (below).  us, before / now, 28 heads on 4, 6 rows: one request of 16 000 keys fp8 414 / 25, bf16
+    // 565 / 25; 16 474 / 98, 662 / 123; 34 of 4 000 123 / 72, 166 / 100; 64 132 / 88, 180 / 144; 32 heads on 8, 20 rows, 16 of 2 000 64 / 45,
+    // 77 / 43.  With many pairs not over a short past (320 pairs, 36 rows over 1 000 42 / 48, 48 / 57), nor for heads of 64 in bf16 (256 pairs,
+    // 48 rows over 4 000 75 / 83)
+    const long past = ((long)max_pages * page_size - n_max) / 64, all = (long)B * KH;
+    const bool few = all <= 128, far = past >= (few ? 12 : 32);
+    const bool grouped = split && rows > 32 && rows < 128 && far && (fp8 || (!few && D == 128 && rows <= 64));
+    if (rows <= 32 || grouped) {
         pl.splitq = false;
         pl.qt = rows <= 16 ? 1 : 2;
-        pl.n_qgroups = 1;
-        const long max_tiles = (long)max_pages * page_size / 32, pairs = (long)B * KH;
+        pl.n_qgroups = (rows + 31) / 32;
+        const long max_tiles = (long)max_pages * page_size / 32, pairs = all * pl.n_qgroups;
         // Splits: as many as leave at most ONE workgroup per CU of an XCD, where a pair's workgroups lie together (32 CUs).  A CU with a
         // second workgroup finishes last, and a lone one streams faster: 12 requests of 16 000 keys (96 pairs of 8 kv heads, bf16 of 128)
         // take 119 us in 192 workgroups, 158 in 288, 123 in 480; 20 requests (160 pairs) 192 us unsplit, 236 in 320, 203 in 480; 7 of 4 000
@@ -1275,9 +1285,15 @@ AttnPlan make_plan(int B, int n_max, int H, int KH, int D, int max_pages, int pa
         // 128 on 8 (64 workgroups) 60.9 / 29.5, one request of 400 73 / 41, 900 (120) 89 / 67, 128 behind 7 000 190 / 38; heads of 64 41 / 20,
         // 56 / 31, 68 / 51, 148 / 31.  Not by the portion's own keys (1 000 from the first on 36.8 / 39.8: the merge,
         // and most groups have few), nor for a short past (4 x 128 behind 385, four tiles: 24.9 / 33.3)
-        const long wgs = ((long)B * KH + 7) / 8 * 8 * pl.n_qgroups, past = ((long)max_pages * page_size - n_max) / 64;
-        if (!fp8 && pl.qt == 2 && g_prefill_mfma32 < 0 && page_size % (D == 128 && pl.nw == 8 ? 128 : 64) == 0 && wgs <= 128)
-            pl.nsplit = (int)std::max(1L, std::min({256 / wgs, past / 6, 16L}));
+        const long wgs = (all + 7) / 8 * 8 * (pl.qt == 2 ? pl.n_qgroups : 1);      // (on the 32-row tiles)
+        if (split && !fp8 && g_prefill_mfma32 < 0 && page_size % (D == 128 && pl.nw == 8 ? 128 : 64) == 0 && wgs <= 128)
+            pl.nsplit = (int)std::max(1L, std::min({256 / wgs, past / 6, 32L}));
+        if (pl.nsplit > 1 && pl.qt == 1) {
+            pl.qt = 2;
+            pl.nw = 4;
+            pl.n_qgroups = 1;
+            pl.rows_cap = 128;
+        }
     }
     return pl;
 }
@@ -1441,10 +1457,12 @@ extern "C" int md_debug_attn_timing_read(float* ms_out, int cap) {
 extern "C" size_t md_paged_attn_workspace_bytes(int B, int n_max, int H, int KH, int D,
                                                 int max_pages_per_req, int page_size) {
     if (B <= 0 || KH <= 0 || H % KH != 0) return 0;
-    const AttnPlan pl = make_plan(B, n_max, H, KH, D, max_pages_per_req, page_size, false);
-    if (pl.nsplit == 1) return 256;
-    const size_t slots = (size_t)B * KH * pl.n_qgroups * pl.nsplit * pl.rows_cap;
-    return slots * (size_t)D * 4 + slots * 8 + 256;
+    size_t need = 0;
+    for (bool fp8 : {false, true}) {
+        const AttnPlan pl = make_plan(B, n_max, H, KH, D, max_pages_per_req, page_size, fp8, true);
+        if (pl.nsplit > 1) need = std::max(need, (size_t)B * KH * pl.n_qgroups * pl.nsplit * pl.rows_cap * ((size_t)D * 4 + 8));
+    }
+    return need + 256;
 }
 
 extern "C" int md_paged_attn(const void* q, int64_t q_row_stride, const void* cache, void* out,
@@ -1474,7 +1492,11 @@ extern "C" int md_paged_attn(const void* q, int64_t q_row_stride, const void* ca
                  "md_paged_attn: kv_dtype must be MD_KV_BF16 or MD_KV_FP8_E4M3 (with per-head scales)");
     const bool fp8 = kv_dtype == MD_KV_FP8_E4M3;
 
-    AttnPlan pl = make_plan(B, n_max, H, KH, D, max_pages_per_req, page_size, fp8);
+    AttnPlan pl = make_plan(B, n_max, H, KH, D, max_pages_per_req, page_size, fp8, true);
+    const size_t slots = (size_t)B * KH * pl.n_qgroups * pl.nsplit * pl.rows_cap, need = slots * (size_t)D * 4 + slots * 8;
+    const bool room = workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0;
+    if (pl.nsplit > 1 && !room && n_max * (H / KH) > 32)           // (more rows than that need no scratch, they make use of it)
+        pl = make_plan(B, n_max, H, KH, D, max_pages_per_req, page_size, fp8, false);
     AttnParams p;
     p.q = (const bf16_t*)q;
     p.cache = cache;
@@ -1496,9 +1518,6 @@ extern "C" int md_paged_attn(const void* q, int64_t q_row_stride, const void* ca
     p.g = H / KH;
     p.page_size = page_size;
     p.causal = causal ? 1 : 0;
-    const size_t slots = (size_t)B * KH * pl.n_qgroups * pl.nsplit * pl.rows_cap, need = slots * (size_t)D * 4 + slots * 8;
-    const bool room = workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0;
-    if (pl.splitq && !room) pl.nsplit = 1;                       // (a prompt's keys are split where there is room for it)
     p.nsplit = pl.nsplit;
     p.n_qgroups = pl.n_qgroups;
     p.scale_log2 = sm_scale * 1.4426950408889634f;
