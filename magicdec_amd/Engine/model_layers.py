@@ -348,7 +348,7 @@ class LayeredTransformer(Transformer):
 
     def _library(self, x2d, w):
         """The product of a row-major weight: float32 rows of a prompt on md_linear_f32_thirds or md_linear_f32, a few of a step over a narrow
-        one on md_linear_f32_few, others in the library."""
+        or shallow one on md_linear_f32_few, others in the library."""
         if x2d.dtype == torch.float32:
             M = x2d.shape[0]
             if (x2d.is_cuda and x2d.stride(0) % 4 == 0 and x2d.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and mode() != "lib"):

@@ -1,4 +1,5 @@
-// 32-bit linear of a step's few rows (gfx950):  out[M][N] = x[M][K] . W[N][K]^T, all float32, row-major, M <= 16, N <= 4096
+// 32-bit linear of a step's few rows (gfx950):  out[M][N] = x[M][K] . W[N][K]^T, all float32, row-major, M <= 16, and
+// N <= 4096 (f32_few_kernel) or a shallow K (f32_wide_kernel)
 //
 // replaces: the library products of 32-bit steps of the layered designs (and of recorded traces) over narrow weights.
 //
@@ -7,8 +8,8 @@
 // v_mfma_f32_16x16x4, no barrier, no K split over workgroups to combine.  x goes through LDS: as fragments from memory it would be as many
 // bytes in flight as W.  The wavefronts' partial tiles are added in their order, so that a row's bits do not depend on the rows beside it.
 // Six rows, us, library / here: 3 072 x 2 048 12.6 / 9.9, 2 048 x 2 048 12.1 / 8.0, 2 048 x 8 192 23.5 / 19.4 (one row 16.9: 4.0 TB/s),
-// 2 048 x 5 632 17.9 / 15.6, 1 536 x 1 536 9.6 / 6.9; error against 64 bits half of the library's.  Wider weights are level (8 192 x 2 048
-// 17.9 / 18.2, 32 000 x 2 048 61.4 / 61.6).
+// 2 048 x 5 632 17.9 / 15.6, 1 536 x 1 536 9.6 / 6.9; error against 64 bits half of the library's.  Wider weights are level that
+// way (8 192 x 2 048 17.9 / 18.2, 32 000 x 2 048 61.4 / 61.6: each workgroup's x).
 #include "md_common.h"
 
 #include <algorithm>
@@ -119,6 +120,74 @@ __global__ __launch_bounds__(64 * kNW, COLS == 8 ? 2 : 4) void f32_few_kernel(co
     if (row < p.M && col < p.N) *reinterpret_cast<f32x4*>(p.out + (int64_t)row * p.ldo + col) = s;
 }
 
+// Wide weights, K = 256 STEPS at most 2 048: a workgroup a CU takes every 256th tile of 16 columns.  x stays in registers, as fragments of
+// the wavefront's slice of K; the loads of a tile are on their way while the one before it is multiplied, across the barrier at which the
+// slices' sums meet, which a wavefront after the other adds up.  Workgroups' wavefronts start at different slices: rows are a power of two apart.
+template <int STEPS>
+__global__ __launch_bounds__(64 * kNW, 2) void f32_wide_kernel(const FewParams p, int tiles) {
+    __shared__ f32x4 parts[2][kNW][64];
+    const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, q = lane >> 4, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int slice = (wave + blockIdx.x) % kNW, k0 = slice * STEPS * 32;
+    f32x4 a[STEPS][2], wr[STEPS][2];
+    const float* xr = p.x + (int64_t)min(j, p.M - 1) * p.ldx + k0 + q * 8;
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) a[s][h] = *reinterpret_cast<const f32x4*>(xr + s * 32 + h * 4);
+    auto row_of = [&](int t, int h) { return p.w + (int64_t)min(t * 16 + h * 8 + (j & 7), p.N - 1) * p.K + k0 + q * 8 + (j >> 3) * 4; };
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) wr[s][h] = *reinterpret_cast<const f32x4*>(row_of(blockIdx.x, h) + s * 32);
+    auto above = [](float keep, float other) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(keep), __float_as_int(other), 0x128, 0xf, 0xc, false));
+    };
+    auto below = [](float keep, float other) {
+        return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(keep), __float_as_int(other), 0x128, 0xf, 0x3, false));
+    };
+    int turn = 0;
+#pragma unroll 1
+    for (int t = blockIdx.x; t < tiles; t += gridDim.x, ++turn) {
+        const int next = t + (int)gridDim.x;
+        const float* from[2];                       // (behind the last tile: one line that is at hand)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) from[h] = next < tiles ? row_of(next, h) : p.w;
+        f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            f32x4 b[2];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                b[0][e] = above(wr[s][0][e], wr[s][1][e]);                // row j, k 8 q + e
+                b[1][e] = below(wr[s][1][e], wr[s][0][e]);                // and 8 q + 4 + e
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) wr[s][h] = *reinterpret_cast<const f32x4*>(from[h] + s * 32);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) acc[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(b[h][e], a[s][h][e], acc[h], 0, 0, 0);
+        }
+        parts[turn & 1][slice][lane] = acc[0] + acc[1];                   // row j, columns 4 q .. + 3
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                // (the loads stay on their way)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (wave != turn % kNW) continue;
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < kNW; ++i) sum += parts[turn & 1][i][lane];
+        const int col = t * 16 + q * 4;
+        if (j < p.M && col < p.N) *reinterpret_cast<f32x4*>(p.out + (int64_t)j * p.ldo + col) = sum;
+    }
+}
+
+template <int STEPS>
+void launch_wide(const FewParams& p, hipStream_t st) {
+    const int tiles = (p.N + 15) / 16;
+    hipLaunchKernelGGL((f32_wide_kernel<STEPS>), dim3(tiles < 256 ? tiles : 256), dim3(64 * kNW), 0, st, p, tiles);
+}
+
 template <int COLS, int ROWS>
 int launch_rows(const FewParams& p, hipStream_t st) {
     constexpr int bytes = kNW * 16 * (64 / COLS * 128 + 16);
@@ -142,7 +211,10 @@ int launch(const FewParams& p, hipStream_t st) {
 
 extern "C" int md_linear_f32_few_supported(int M, int N, int K) {
     MD_CHECK_ARG(M > 0 && N > 0 && K > 0, "md_linear_f32_few_supported: M=%d N=%d K=%d", M, N, K);
-    return M <= 16 && N <= 4096 && N % 4 == 0 && K % (32 * kNW) == 0 && K < (1 << 22) ? 1 : 0;
+    // wide: 6 rows, us, library / here 32 000 x 2 048 61.8 / 53.8, x 1 024 34.7 / 29.3, 8 192 x 1 024 14.6 / 10.9; level at 11 264 x 2 048 (22.6 / 22.1)
+    // and below (6 144 16.0 / 16.5), 16 rows of 128 256 199 / 205
+    const bool wide = K <= 1024 || (K <= 2048 && N >= 16384 && (M <= 8 || N <= 65536));
+    return M <= 16 && (N <= 4096 || wide) && N < (1 << 26) && N % 4 == 0 && K % (32 * kNW) == 0 && K < (1 << 22) ? 1 : 0;
 }
 
 extern "C" int md_linear_f32_few(const float* x, int64_t ldx, const float* w, float* out, int64_t ldo, int M, int N, int K, int tile, md_stream_t stream) {
@@ -152,6 +224,21 @@ extern "C" int md_linear_f32_few(const float* x, int64_t ldx, const float* w, fl
                  "md_linear_f32_few: M=%d N=%d K=%d ldx=%lld ldo=%lld unsupported", M, N, K, (long long)ldx, (long long)ldo);
     MD_CHECK_ARG(tile == 0 || tile == 8 || tile == 16, "md_linear_f32_few: tile of %d columns", tile);
     const FewParams p = {x, w, out, ldx, ldo, M, N, K};
+    if (N > 4096) {
+        hipStream_t st = (hipStream_t)stream;
+        switch (K / 256) {
+        case 1: launch_wide<1>(p, st); break;
+        case 2: launch_wide<2>(p, st); break;
+        case 3: launch_wide<3>(p, st); break;
+        case 4: launch_wide<4>(p, st); break;
+        case 5: launch_wide<5>(p, st); break;
+        case 6: launch_wide<6>(p, st); break;
+        case 7: launch_wide<7>(p, st); break;
+        default: launch_wide<8>(p, st);
+        }
+        MD_CHECK_LAUNCH("md_linear_f32_few");
+        return MD_OK;
+    }
     // eight rows a workgroup: where 16 leave half the CUs idle (2 048 x 2 048 9.2 us, 8.0; but 768 x 512 5.0 and 5.4: few steps a wavefront)
     const int rc = (tile ? tile == 8 : N <= 2048 && K >= 1024) ? launch<8>(p, (hipStream_t)stream) : launch<16>(p, (hipStream_t)stream);
     if (rc != MD_OK) return rc;

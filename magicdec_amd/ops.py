@@ -651,7 +651,7 @@ def linear_f32_few_supported(M, N, K):
 
 
 def linear_f32_few(x, weight, tile=0):
-    """linear_f32 of at most 16 rows, as a stream over a narrow weight (csrc/f32few.hip)."""
+    """linear_f32 of at most 16 rows, as a stream over a narrow or shallow weight (csrc/f32few.hip)."""
     _gpu(x, weight)
     if x.dim() != 2 or x.stride(1) != 1 or weight.dim() != 2 or not weight.is_contiguous() or x.shape[1] != weight.shape[1]:
         raise ValueError("linear_f32_few expects x [M, K] with unit inner stride and a contiguous weight [N, K]")

@@ -26,9 +26,27 @@ def test_products(M, N, K, wider):
     assert out[M // 2].isinf().all() and out.isfinite().all(1).sum() == M - 1
 
 
+# a shallow K under many columns: fewer tiles than workgroups, some workgroups with a tile more, the last one cut, every depth
+@pytest.mark.parametrize("M", [1, 7, 16])
+@pytest.mark.parametrize("N,K", [(4100, 256), (4352, 512), (12300, 768), (8200, 1024), (16388, 1280), (20000, 1536), (16384, 1792), (33000, 2048)])
+def test_wide(M, N, K):
+    from magicdec_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    big = torch.full((16 + 4, K + 4), float("nan"), device=DEV)
+    big[:M] = torch.randn(M, K + 4, device=DEV, generator=g)
+    x, w = big[:M, :K], torch.randn(N, K, device=DEV, generator=g)
+    assert ops.linear_f32_few_supported(M, N, K)
+    ref = x.double() @ w.double().t()
+    off = (x.double().abs() @ w.double().abs().t()) * (K * 2.0 ** -24)
+    out = ops.linear_f32_few(x, w)
+    assert out.shape == (M, N) and ((out.double() - ref).abs() <= off).all()
+    assert torch.equal(out[:1], ops.linear_f32_few(x[:1], w)) and torch.equal(out, ops.linear_f32_few(x, w))
+
+
 def test_refused():
     from magicdec_amd import ops
     x, w = torch.randn(4, 256, device=DEV), torch.randn(64, 256, device=DEV)
+    assert not any(ops.linear_f32_few_supported(*s) for s in ((4, 8192, 2048), (4, 16384, 2304), (16, 128256, 2048), (17, 64, 256)))
     for call in (lambda: ops.linear_f32_few(torch.randn(17, 256, device=DEV), w), lambda: ops.linear_f32_few(x[:, :128], w[:, :128].contiguous()),
                  lambda: ops.linear_f32_few(x, w[:62].contiguous()), lambda: ops.linear_f32_few(x, w, tile=32), lambda: ops.linear_f32_few(x.double(), w.double()),
                  lambda: ops.linear_f32_few(torch.randn(4, 260, device=DEV)[:, 1:257], w)):
