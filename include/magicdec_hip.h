@@ -139,7 +139,8 @@ int md_rope_append(const void* q, const void* k, const void* v, int64_t q_row_st
  * (verify / draft / chunked prefill) is chosen from (n_max, H/KH).
  * max_pages_per_req: host upper bound of pages of any request (sizes the
  * split-KV decomposition; no host read of the page table is made).
- * workspace: md_paged_attn_workspace_bytes() bytes of scratch.
+ * workspace: md_paged_attn_workspace_bytes() bytes of scratch; with less, calls of more than 32 query rows a kv head (n_max H / KH) keep
+ * every request's keys in one piece, which behind a long context is slower, and smaller ones are refused.
  * ---------------------------------------------------------------------- */
 size_t md_paged_attn_workspace_bytes(int B, int n_max, int H, int KH, int D,
                                      int max_pages_per_req, int page_size);
