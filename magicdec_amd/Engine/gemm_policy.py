@@ -114,6 +114,11 @@ def fused_mode() -> str:
     return _FUSED
 
 
+def joint_launches() -> bool:
+    """May a product share a launch with what is in front of it, or do the switches above say which kernel (or none) it runs on?"""
+    return _MODE == "auto" and _FUSED == "auto"
+
+
 _PACKED = os.environ.get("MAGICDEC_PACKED_COPIES", "auto")   # "0": no streaming-layout copies at all (every linear on the
                                                              # library / the row-major md_linear): saves their HBM
 
@@ -431,7 +436,7 @@ def use_few(M: int, N: int, K: int) -> bool:
     Deep ones (asked for with a row to four) against the K split and the weight-streaming kernel, with the norm behind them, which here
     the next product absorbs: 4 096 x 14 336 26.4 -> 22.9, 2 048 x 8 192 11.4 -> 10.4, 2 464 x 13 056 20.4 -> 17.7, but 608 x 14 592 (38
     workgroups) 10.1 / 15.3."""
-    if _MODE != "auto" or _FUSED != "auto" or not 1 <= M <= 16 or N > 16 * CUS or N % 32 or K % 256 or K < 1024:
+    if not joint_launches() or not 1 <= M <= 16 or N > 16 * CUS or N % 32 or K % 256 or K < 1024:
         return False
     return K < SPLIT_MIN_K or N >= 1024
 

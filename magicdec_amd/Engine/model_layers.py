@@ -29,7 +29,7 @@ from torch.nn import functional as F
 
 from .. import ops
 from .designs import DecoderSpec, LatentAttentionSpec, LayerSpec
-from .gemm_policy import choose, mode, use_split, want_packed_prompt
+from .gemm_policy import choose, joint_launches, mode, use_split, want_packed_prompt
 from .model_core import PageTable, RMSNorm, Transformer
 
 STATE_RING = 16        # unshifted rows kept per sequence and layer: rollbacks of up to STATE_RING - 2 tokens
@@ -442,7 +442,7 @@ class LayeredTransformer(Transformer):
         gated = z is not None
         if not gated:
             z = self._linear(y, att.win)
-        wuq = self._packed.get(id(att.wuq.weight)) if y.shape[0] <= 64 else None
+        wuq = self._packed.get(id(att.wuq.weight)) if y.shape[0] <= 64 and joint_launches() else None
         if wuq is not None and ops.latent_query_supported(z, s, wuq, cache):
             q = ops.latent_query(z, s, wuq, cache, rows, tab.indices, tab.indptr, tab.max_pages)
         else:

@@ -121,6 +121,34 @@ def test_a_state_dict_without_the_rows_of_zeros_loads(latent_ops, model, assign)
         assert all(torch.equal(v, whole[k]) for k, v in m.state_dict().items())
 
 
+@pytest.mark.parametrize("switch,value", [("set_mode", "lib"), ("set_mode", "hip"), ("set_fused", "0"), ("set_fused", "1"), (None, None)])
+def test_the_switches_decide_where_a_steps_queries_run(latent_ops, model, monkeypatch, switch, value):
+    """The query product shares a launch with the norm in front of it only where the policy is left to itself."""
+    from magicdec_amd import ops
+    from magicdec_amd.Engine import gemm_policy as g
+    if g.mode() != "auto" or g.fused_mode() != "auto":
+        pytest.skip("policy overridden by the environment")
+    e, joint = engine(model[0], slots=1), []
+    e.step([("a", [5, 6, 7])])
+
+    def query(z, s, weight, cache, *where):
+        joint.append(weight)
+        return torch.nn.functional.linear(ops.latent_append(z, s, cache, *where), weight)
+    monkeypatch.setattr(ops, "latent_query_supported", lambda *a: True)
+    monkeypatch.setattr(ops, "latent_query", query)
+    monkeypatch.setattr(e.model, "_gated_beside", lambda *a: None)
+    e.model._packed.update({id(b.attention.wuq.weight): b.attention.wuq.weight for b in e.model.layers})
+    if switch:
+        old = {"set_mode": g.mode(), "set_fused": g.fused_mode()}[switch]
+        getattr(g, switch)(value)
+    try:
+        e.step([("a", [8])])
+    finally:
+        if switch:
+            getattr(g, switch)(old)
+    assert len(joint) == (0 if switch else len(e.model.layers))
+
+
 def test_copies_for_prompts_come_behind_those_for_steps(latent_ops, tmp_path, monkeypatch):
     """A card that holds the streaming copies that steps read, but not wukv's beside them, keeps the former; one rank of a group without
     room for wukv's is enough for none to make them."""
