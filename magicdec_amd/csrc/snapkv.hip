@@ -467,9 +467,10 @@ __global__ __launch_bounds__(256) void snapkv_finalize_kernel(const SnapParams p
 // by the two halves in turn).  2 x 2 tiles at a time as in pass 1.  118 us where pass 1 takes 92: vector instructions for 69 % of the
 // cycles, LDS 61 %.  (147 with the accumulators in scratch memory, where an address of either column group had put them, halves of packed
 // bf16 converted one by one, and workgroups of eight wavefronts; the gathers of a batch in front of the next one's scores: spills, 177.)
-template <int D, bool FP8, int GH, int RTM>
+// BIN: the table's binades; all, but where the accumulators of 30 and 32 queries a kv head of 128 beside them would pass a CU's LDS.
+template <int D, bool FP8, int GH, int RTM, int BIN = kTabBinades>
 __global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) void snapkv_accum_kernel(const SnapParams p) {
-    constexpr int kSnapWaves = score_waves(D, RTM), BIN = kTabBinades;
+    constexpr int kSnapWaves = score_waves(D, RTM);
     constexpr int BT = GH >= 2 ? 2 : 1;                        // row tiles per batch
     __shared__ __attribute__((aligned(16))) double tab[Tab<BIN>::N];
     // Q image, [L] exp(-M) / Z, [L][2] (M, 1 / Z), GH == 0: [waves][g][32] floats
@@ -868,11 +869,17 @@ __global__ __launch_bounds__(256) void snapkv_gather_kernel(const GatherParams p
     }
 }
 
+// LDS that is left beside the table of BIN binades (and a few words)
+template <int BIN>
+constexpr int beside_table() {
+    return 160 * 1024 - Tab<BIN>::N * 8 - 256;
+}
+
 // A score kernel, whose LDS, with the table of BIN binades, is more than 64 KB
 template <auto Kernel, int BIN>
 int score_launch(dim3 grid, int waves, size_t lds, const SnapParams& p, hipStream_t st) {
     static MdPerDeviceOnce once;
-    const int cap = 160 * 1024 - Tab<BIN>::N * 8 - 256;
+    constexpr int cap = beside_table<BIN>();
     if (once.first() && hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, cap) != hipSuccess) {
         once.undo();
         md_set_error("md_snapkv_select: hipFuncSetAttribute(%d B LDS) failed", cap);
@@ -1004,6 +1011,11 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
     const size_t lds2 = qimg_b + (size_t)L * 3 * 8 + (gh ? 0 : (size_t)waves * g * 32 * 4);
     const dim3 sg(p.nch, KH, B), ag((N + p.cols - 1) / p.cols, KH, B);
     const bool small = L <= 128;
+    // (30 and 32 queries a kv head of 128: 171 648 and 174 080 bytes with the whole table, of 163 840)
+    const bool tight = lds2 > (size_t)beside_table<kTabBinades>();
+    MD_CHECK_ARG(lds1 <= (size_t)(D == 128 && !small ? beside_table<kTabSmall>() : beside_table<kTabBinades>()) &&
+                     (!tight || (D == 128 && !small && gh == 0 && lds2 <= (size_t)beside_table<kTabSmall>())),
+                 "md_snapkv_select: g=%d window=%d head_dim=%d need %zu / %zu bytes of LDS beside the table", g, window, D, lds1, lds2);
     int rc = MD_OK;
 #define MD_SNAP_STATS(DD, FP)                                                                                                \
     rc = small ? score_launch<&snapkv_stats_kernel<DD, FP, 8>, stats_binades(DD, 8)>(sg, waves, lds1, p, st)                 \
@@ -1020,7 +1032,10 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
         if (gh == 4) MD_SNAP_ACCUM(DD, FP, 4);                                                                               \
         else if (gh == 2) MD_SNAP_ACCUM(DD, FP, 2);                                                                          \
         else if (gh == 1) MD_SNAP_ACCUM(DD, FP, 1);                                                                          \
-        else MD_SNAP_ACCUM(DD, FP, 0);                                                                                       \
+        else if constexpr (DD == 128) {                                                                                      \
+            if (tight) rc = score_launch<&snapkv_accum_kernel<DD, FP, 0, kMaxRT, kTabSmall>, kTabSmall>(ag, waves, lds2, p, st); \
+            else MD_SNAP_ACCUM(DD, FP, 0);                                                                                   \
+        } else MD_SNAP_ACCUM(DD, FP, 0);                                                                                     \
         if (rc != MD_OK) return rc;                                                                                          \
     } while (0)
     if (D == 128) {

@@ -30,6 +30,13 @@ def test_select_with_one_workgroup_per_cu(monkeypatch, B, KH, g, W, D, S):
     check_select(monkeypatch, B, KH, g, W, D, S, 129, 5, 128, (0, B - 1))
 
 
+# accumulators, query image and table of exponentials in one CU's LDS: the most queries a kv head (with the whole table 160 to 170 KB of 160)
+@pytest.mark.parametrize("g,W,D", [(32, 8, 128), (30, 8, 128), (28, 8, 128), (16, 16, 128), (32, 8, 64)])
+@pytest.mark.parametrize("KH,S", [(1, 1060), (3, 150)])
+def test_select_of_many_queries_a_kv_head(monkeypatch, KH, S, g, W, D):
+    check_select(monkeypatch, 2, KH, g, W, D, S, 129, 5, 128, (0, 1))
+
+
 def check_select(monkeypatch, B, KH, g, W, D, S, budget, pool, page, requests):
     from magicdec_amd import ops
     H, ppr, dpr = KH * g, -(-S // page), budget // page + 1
