@@ -667,9 +667,12 @@ F32Launch plan(const XattnParams& p, Shape s, long keys) {
     };
     // Wide row groups reuse a tile's keys, 16 rows are the shorter chain: ahead by a fifth to a third while the wide ones are not half as
     // many workgroups as there are CUs (32 query heads of 64, 20 rows over 20 keys: 16.2 -> 11.6 us with the keys of a tile that are not
-    // there left out; 16 rows over 1 500: x 0.7), behind by as much from about 200 on (heads of 256: 150).  A wavefront's own rows (heads to
-    // 128) are level at 100 workgroups (13 x 8: 22.1 and 23.3; 48 x 2: 28.3 and 26.0), ahead at 128 (8 x 60 rows, 16 / 4 heads of 128: 21.5 and 19.2).
-    if (rows <= 16 || with_rows(16 * wide[s]) < 128) with_rows(16);
+    // there left out; 16 rows over 1 500: x 0.7).  A wavefront's own rows (heads to 128) are level at 100 workgroups (13 x 8: 22.1 and 23.3;
+    // 48 x 2: 28.3 and 26.0), ahead at 128 (8 x 60 rows, 16 / 4 heads of 128: 21.5 and 19.2).  Wider heads, two tiles of 16 rows together, are
+    // ahead where those tiles would be more than one a CU: 17 requests of 20 rows, heads of 256 (136) 53.4 and 34.9 us, of 32 rows 56.1 and
+    // 38.7, but 16 of 32 (128) 30.2 and 33.0, 4 of 128 26.2 and 30.1.
+    const long line = s == k64 || s == k128 ? 128 : 129;
+    if (rows <= 16 || with_rows(16 * wide[s]) < line) with_rows(16);
     return L;
 }
 
