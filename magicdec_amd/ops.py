@@ -178,10 +178,17 @@ class AttnWorkspace:
         self.buf = torch.empty(1 << 20, dtype=torch.uint8, device=device)
         self._retired = []     # outgrown buffers stay allocated: captured hipGraphs have their addresses baked in
 
-    def get(self, nbytes):
+    def get(self, nbytes, needed=True):
+        """At least nbytes of it; where there is no memory for them and they are not `needed`, what there is."""
         if self.buf.numel() < nbytes:
+            try:
+                grown = torch.empty(int(nbytes * 1.25) + 256, dtype=torch.uint8, device=self.device)
+            except torch.OutOfMemoryError:
+                if needed:
+                    raise
+                return self.buf
             self._retired.append(self.buf)
-            self.buf = torch.empty(int(nbytes * 1.25) + 256, dtype=torch.uint8, device=self.device)
+            self.buf = grown
         return self.buf
 
 
@@ -201,7 +208,7 @@ def paged_attention(q, kv_cache, qo_indptr, page_indices, page_indptr, last_page
         out = torch.empty((q.shape[0], H, D), dtype=q.dtype, device=q.device)
     lib = _lib.load()
     nbytes = lib.md_paged_attn_workspace_bytes(B, n_max, H, KH, D, max_pages_per_req, page_size)
-    ws = workspace.get(nbytes)
+    ws = workspace.get(nbytes, needed=n_max * (H // KH) <= 32)          # (more rows than that make use of it)
     check(lib.md_paged_attn(_p(q), _row_stride(q), _p(kv_cache), _p(out), _p(_i32(qo_indptr)), _p(_i32(page_indices)),
                             _p(_i32(page_indptr)), _p(_i32(last_page_len)), B, n_max, H, KH, D, page_size,
                             1 if causal else 0, float(sm_scale), max_pages_per_req,

@@ -57,3 +57,27 @@ def test_against_unsplit(H, KH, D, page, lens, past, layout, causal, dtype):
     off = 2 * 2.0 ** -9 * whole(sized) * 1.01 + 2.0 ** -8 * ref.abs() + 1e-30
     assert split.isfinite().all() and (split - ref).abs().le(off).all()
     assert lib.md_paged_attn_workspace_bytes(B, n, H, KH, D, most, page) > 256 or len(lens) > 30
+
+
+def test_memory_for_no_scratch(monkeypatch):
+    """Rows that need no scratch go without where there is no memory for it; a step's rows, which do, say so.  The workspace stays usable."""
+    from magicdec_amd import ops
+    B, n, H, KH, D, page, most = 1, 128, 32, 8, 128, 128, 40
+    q, cache = torch.randn(n, H, D, device=DEV).to(BF), torch.randn(most, 2, KH, page, D, device=DEV).to(BF)
+    table = [i32([0, n]), i32(list(range(most))), i32([0, most]), i32([page])]
+    ws, real = ops.AttnWorkspace(DEV), torch.empty
+    split = ops.paged_attention(q, cache, *table, n, most, ops.AttnWorkspace(DEV), kv_layout="HND")
+    with monkeypatch.context() as m:
+        def empty(*size, **kw):
+            if kw.get("dtype") == torch.uint8:
+                raise torch.OutOfMemoryError("no room")
+            return real(*size, **kw)
+        m.setattr(torch, "empty", empty)
+        whole = ops.paged_attention(q, cache, *table, n, most, ws, kv_layout="HND")
+        few = torch.randn(64, H, D, device=DEV).to(BF)
+        with pytest.raises(torch.OutOfMemoryError):
+            ops.paged_attention(few, cache, i32(list(range(0, 65, 8))), i32([0] * 8 * most), i32([most * b for b in range(9)]), i32([page] * 8), 8, most, ws,
+                                kv_layout="HND")
+    assert ws._retired == [] and ws.buf.numel() == 1 << 20
+    assert (whole.float() - split.float()).norm() <= 0.01 * whole.float().norm()
+    assert torch.equal(ops.paged_attention(q, cache, *table, n, most, ws, kv_layout="HND"), split)
