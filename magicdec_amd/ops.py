@@ -638,15 +638,19 @@ def linear_f32_supported(M, N, K):
     return _lib.load().md_linear_f32_supported(int(M), int(N), int(K)) > 0
 
 
-def linear_f32(x, weight, tile=0):
-    """F.linear(x, weight) of float32 rows [M, K] (row stride free) and a contiguous float32 weight [N, K] on md_linear_f32."""
+def linear_f32(x, weight, tile=0, out=None):
+    """F.linear(x, weight) of float32 rows [M, K] (row stride free) and a contiguous float32 weight [N, K] on md_linear_f32, into `out`
+    (float32, contiguous) if there is one."""
     _gpu(x, weight)
     if x.dim() != 2 or x.stride(1) != 1 or weight.dim() != 2 or not weight.is_contiguous() or x.shape[1] != weight.shape[1]:
         raise ValueError("linear_f32 expects x [M, K] with unit inner stride and a contiguous weight [N, K]")
     if x.dtype != torch.float32 or weight.dtype != torch.float32:
         raise TypeError("linear_f32 takes float32")
     (M, K), N = x.shape, weight.shape[0]
-    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    if out is None:
+        out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    elif out.shape != (M, N) or out.dtype != x.dtype or out.device != x.device or not out.is_contiguous():
+        raise ValueError("linear_f32: out must be a contiguous float32 [M, N]")
     check(_lib.load().md_linear_f32(_p(x), x.stride(0), _p(weight), _p(out), N, M, N, K, int(tile), _stream()), "md_linear_f32")
     return out
 
@@ -691,11 +695,11 @@ def linear_f32_thirds(x, weight, tile=0):
     lib = _lib.load()
     parts = max(1, -(-6 * M * K // THIRDS_BYTES))
     rows = -(-M // (256 * parts)) * 256
+    out = torch.empty((M, N), dtype=x.dtype, device=x.device)           # (in front of the scratch, which is not needed)
     try:
         ws = torch.empty(max(1, lib.md_linear_f32_thirds_workspace(min(M, rows), K)), dtype=torch.uint8, device=x.device)
     except torch.OutOfMemoryError:
-        return linear_f32(x, weight)
-    out = torch.empty((M, N), dtype=x.dtype, device=x.device)
+        return linear_f32(x, weight, out=out)
     for a in range(0, M, rows):
         n = min(rows, M - a)
         check(lib.md_linear_f32_thirds(_p(x[a:]), x.stride(0), _p(weight), _p(out[a:]), N, n, N, K, int(tile), _p(ws), ws.numel(), _stream()),

@@ -58,6 +58,30 @@ def test_rows_in_several_calls(monkeypatch):
     assert torch.equal(ops.linear_f32_thirds(x, w), whole)
 
 
+def room(monkeypatch, nbytes):
+    """torch.empty finds no memory once `nbytes` are asked for in all."""
+    real, left = torch.empty, [nbytes]
+
+    def empty(*size, **kw):
+        t = real(*size, **dict(kw, device="meta"))
+        if t.numel() * t.element_size() > left[0]:
+            raise torch.OutOfMemoryError("no room")
+        left[0] -= t.numel() * t.element_size()
+        return real(*size, **kw)
+    monkeypatch.setattr(torch, "empty", empty)
+
+
+@pytest.mark.parametrize("M,N,K", [(256, 512, 64), (256, 64, 512)])
+def test_memory_for_the_result_alone(monkeypatch, M, N, K):
+    """Scratch larger than the result or smaller: with room for either, not both, the rows are multiplied without it."""
+    from magicdec_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x, w = torch.randn(M, K, device=DEV, generator=g), torch.randn(N, K, device=DEV, generator=g)
+    want = ops.linear_f32(x, w)
+    room(monkeypatch, max(4 * M * N, 6 * M * K))
+    assert torch.equal(ops.linear_f32_thirds(x, w), want)
+
+
 def test_refused():
     from magicdec_amd import ops
     x, w = torch.randn(100, 64, device=DEV), torch.randn(64, 64, device=DEV)
