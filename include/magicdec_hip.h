@@ -331,8 +331,8 @@ int md_linear_f32_supported(int M, int N, int K);
 int md_linear_f32(const float* x, int64_t ldx, const float* w, float* out, int64_t ldo, int M, int N, int K, int tile, md_stream_t stream);
 
 /* md_linear_f32_few (csrc/f32few.hip): the same of at most 16 rows, a step's, over a narrow weight (N <= 4096) or a shallow one (K <= 1024, or 2048 from
- * 16 384 columns on); K % 256 == 0, N % 4 == 0, everything 16-byte aligned.  _supported: 1 if it takes the shape (negative: no shape).  tile: 0, or 8 or
- * 16 columns a workgroup of a narrow one. */
+ * 16 384 columns on); K % 256 == 0, N % 4 == 0, everything 16-byte aligned.  _supported: 1 if it takes the shape and is expected to be as fast as a
+ * library GEMM (negative: no shape).  tile: 0, or 8 or 16 columns a workgroup of a narrow one. */
 int md_linear_f32_few_supported(int M, int N, int K);
 int md_linear_f32_few(const float* x, int64_t ldx, const float* w, float* out, int64_t ldo, int M, int N, int K, int tile, md_stream_t stream);
 

@@ -657,7 +657,7 @@ def linear_f32(x, weight, tile=0, out=None):
 
 @functools.lru_cache(maxsize=1024)
 def linear_f32_few_supported(M, N, K):
-    """True when md_linear_f32_few (csrc/f32few.hip) takes this shape."""
+    """True when md_linear_f32_few (csrc/f32few.hip) takes this shape and is expected to be as fast as the library."""
     return _lib.load().md_linear_f32_few_supported(int(M), int(N), int(K)) > 0
 
 
