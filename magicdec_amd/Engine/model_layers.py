@@ -351,7 +351,8 @@ class LayeredTransformer(Transformer):
         or shallow one on md_linear_f32_few, others in the library."""
         if x2d.dtype == torch.float32:
             M = x2d.shape[0]
-            if (x2d.is_cuda and x2d.stride(0) % 4 == 0 and x2d.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and mode() != "lib"):
+            if (x2d.is_cuda and x2d.stride(1) == 1 and x2d.stride(0) % 4 == 0 and x2d.stride(0) >= x2d.shape[1] and x2d.data_ptr() % 16 == 0
+                    and w.is_contiguous() and w.data_ptr() % 16 == 0 and mode() != "lib"):
                 if M <= 16 and ops.linear_f32_few_supported(M, *w.shape):
                     return ops.linear_f32_few(x2d, w)
                 if ops.linear_f32_thirds_supported(M, *w.shape):

@@ -62,3 +62,16 @@ def test_shapes_that_the_library_multiplies_faster():
         assert not takes(M, N, K), (M, N, K)
     for M, N, K in ((6, 2048, 8192), (6, 2048, 2048), (16, 3072, 2048), (16, 1376, 2048), (8, 128, 1536), (4, 128, 256), (16, 3072, 768), (6, 32000, 2048)):
         assert takes(M, N, K), (M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(4, 2048, 512), (500, 4096, 1024)])
+def test_operands_as_they_lie(M, N, K):
+    """A weight in columns (as an assigned state dict may bring it) and rows that repeat go to the library, as before these kernels."""
+    from magicdec_amd import ops
+    from magicdec_amd.Engine.model_layers import LayeredTransformer
+    assert ops.linear_f32_few_supported(M, N, K) if M <= 16 else ops.linear_f32_thirds_supported(M, N, K)
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x, w = torch.randn(M, K, device=DEV, generator=g), torch.randn(N, K, device=DEV, generator=g)
+    for a, b in ((x, w.t().contiguous().t()), (x[:1].expand(M, K), w), (x.t().contiguous().t(), w)):
+        ref = a.double() @ b.double().t()
+        assert ((LayeredTransformer._library(None, a, b).double() - ref).abs() <= (a.double().abs() @ b.double().abs().t()) * (K * 2.0 ** -24)).all()
