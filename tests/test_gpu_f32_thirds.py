@@ -37,6 +37,54 @@ def test_no_further_off_than_the_fp32_instruction():
     assert (ops.linear_f32_thirds(x, w).double() - ref).norm() <= (ops.linear_f32(x, w).double() - ref).norm()
 
 
+@pytest.mark.parametrize("K", [256, 2048])
+@pytest.mark.parametrize("kind", ["normal", "positive", "shifted", "outliers", "zeros"])
+def test_error_beside_the_fp32_instruction_s(kind, K):
+    """The same over other distributions.  Zeros cost the fp32 instruction's sums no rounding, six parts of the others do."""
+    from magicdec_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(K)
+    x, w = torch.randn(512, K, device=DEV, generator=g), torch.randn(512, K, device=DEV, generator=g)
+    if kind == "positive":
+        x, w = torch.rand(512, K, device=DEV, generator=g), torch.rand(512, K, device=DEV, generator=g)
+    elif kind == "shifted":
+        x, w = x + 0.25, w + 0.25
+    elif kind == "outliers":
+        x[:, ::97] *= 100
+    elif kind == "zeros":
+        x = x.relu()
+    ref = x.double() @ w.double().t()
+    assert (ops.linear_f32_thirds(x, w).double() - ref).norm() <= (1.3 if kind == "zeros" else 1) * (ops.linear_f32(x, w).double() - ref).norm()
+
+
+@pytest.mark.parametrize("K", [32, 2048])
+@pytest.mark.parametrize("sign", [1, -1])
+def test_operands_whose_rests_are_as_large_as_they_can_be(K, sign):
+    """What the six products leave out is then 2^-24 of each term, and of one sign."""
+    from magicdec_amd import ops
+    v = 1 + 2.0 ** -8 - 2.0 ** -17 + 2.0 ** -23
+    x, w = torch.full((70, K), v, device=DEV), torch.full((132, K), sign * v, device=DEV)
+    ref = x.double() @ w.double().t()
+    assert ((ops.linear_f32_thirds(x, w).double() - ref).abs() <= ref.abs() * ((K + 1) * 2.0 ** -24)).all()
+
+
+@pytest.mark.parametrize("power", [-100, -110, -116, -122, -130, 100])
+@pytest.mark.parametrize("small", ["x", "w"])
+def test_numbers_of_any_size(power, small):
+    """Parts are multiples of 2^-133: each number is held to 2^-134, beside what 32-bit sums round (of results below 2^-126 to 2^-150)."""
+    from magicdec_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(-power)
+    K = 256
+    x, w = torch.randn(130, K, device=DEV, generator=g), torch.randn(132, K, device=DEV, generator=g)
+    if small == "x":
+        x = (x.double() * 2.0 ** power).float()
+    else:
+        w = (w.double() * 2.0 ** power).float()
+    a, b = x.double().abs(), w.double().abs()
+    held = 2.0 ** -134 * (a.sum(1)[:, None] + b.sum(1)[None]) * 1.01
+    off = (a @ b.t()) * (K * 2.0 ** -24) + held + K * 2.0 ** -149
+    assert ((ops.linear_f32_thirds(x, w).double() - x.double() @ w.double().t()).abs() <= off).all()
+
+
 def test_infinities_and_numbers_that_round_to_them():
     from magicdec_amd import ops
     x, w = torch.ones(70, 64, device=DEV), torch.ones(132, 64, device=DEV)
