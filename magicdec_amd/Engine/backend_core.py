@@ -237,8 +237,8 @@ class _BackendBase:
 
     def _portions(self, seq_len):
         """The portions [(first token, tokens)] of a prompt whose keys all stay in the cache: any division gives every token the same
-        keys, so portions are as long as the matrix products want them, and the memory holds.  An fp8 cache's first CHUNK, which sets its
-        scales, stays one."""
+        keys, so portions are as long as the matrix products want them, and the memory holds.  (The same keys, not the same roundings: a
+        SnapKV draft may keep other rows where two score alike.)  An fp8 cache's first CHUNK, which sets its scales, stays one."""
         if self.mapped or torch.device(self.device).type == "cpu":       # (the CPU's products round by their row counts)
             chunk = self.prefill_chunk
             return [(a, min(chunk, seq_len - a)) for a in range(0, seq_len, chunk)]

@@ -1284,8 +1284,9 @@ AttnPlan make_plan(int B, int n_max, int H, int KH, int D, int max_pages, int pa
         // 64-key tiles of what lies in front of the portion at least.  us, whole / split: 33 rows of 4 requests behind 2 048 keys, 32 heads of
         // 128 on 8 (64 workgroups) 60.9 / 29.5, one request of 400 73 / 41, 900 (120) 89 / 67, 128 behind 7 000 190 / 38; heads of 64 41 / 20,
         // 56 / 31, 68 / 51, 148 / 31.  Not by the portion's own keys (1 000 from the first on 36.8 / 39.8: the merge,
-        // and most groups have few), nor for a short past (4 x 128 behind 385, four tiles: 24.9 / 33.3; 4 x 64 behind
-        // 1 024 38.4 / 33.0): whole, a prompt in chunks rounds as one in portions.  33 to 127 rows from twelve tiles on (above)
+        // and most groups have few), nor for a short past (4 x 128 behind 385, four tiles: 24.9 / 33.3).  Between twelve and twenty tiles
+        // it gives little (4 x 64 behind 1 024 38.4 / 33.0) and is left, so that prompts to 1 280 tokens round nearly alike in chunks and in
+        // portions; behind more keys those are two roundings of the same sums.  33 to 127 rows from twelve tiles on (above)
         const long wgs = (all + 7) / 8 * 8 * (pl.qt == 2 ? pl.n_qgroups : 1);      // (on the 32-row tiles)
         if (split && !fp8 && g_prefill_mfma32 < 0 && page_size % (D == 128 && pl.nw == 8 ? 128 : 64) == 0 && wgs <= 128 && past >= (pl.qt == 2 ? 20 : 12))
             pl.nsplit = (int)std::min({256 / wgs, past / 6, 32L});

@@ -68,6 +68,30 @@ def test_longer_portions(which, kv, batch, prompt, monkeypatch):
         assert near.double().mean() > 0.8
 
 
+@pytest.mark.parametrize("which,batch,prompt", [("spec", 2, 1440), ("draft", 4, 2080), ("spec", 1, 3104)])
+def test_longer_portions_behind_split_keys(which, batch, prompt, monkeypatch):
+    """Where a chunk's keys are split over workgroups the chunks' roundings are independent of the portions' from the first layer's
+    attention on: the same bounds on rows and logits as above.  Of the rows kept for the draft, the first layer's are of the same scores but
+    for the products' rounding; behind it the scores, as close as random weights make them, move by 1 % (0.70 to 0.85 of the rows stay,
+    0.78 to 0.97 where two orders of whole keys round partly alike)."""
+    import magicdec_amd.Engine.backend_core as core
+    ids = torch.randint(4, 512, (batch, prompt), generator=torch.Generator().manual_seed(prompt)).to(DEV)
+    seen = []
+    for rows in (core.PROMPT_ROWS, 0):
+        monkeypatch.setattr(core, "PROMPT_ROWS", rows)
+        e = engine(which, "bf16", batch, 4096)
+        e.encode(ids)
+        kvs = [b.attention.kv_cache for b in e.model.layers]
+        seen.append(([e.model._last_logits.float()] + [c.kv_cache.float() for c in kvs], [c.draft_cache.float() for c in kvs]))
+    (a, kept_a), (b, kept_b) = seen
+    for x, y in zip(a, b):
+        assert (x - y).norm() <= 0.016 * y.norm()
+        x, y = x.double(), y.double()
+        assert abs(((x - y) * y).sum()) <= 6 * 0.016 * (y * y).sum() / y.count_nonzero() ** 0.5
+    for x, y, least in zip(kept_a, kept_b, (0.95, 0.6)):
+        assert ((x - y).norm(dim=-1) <= 0.05 * y.norm(dim=-1)).double().mean() > least
+
+
 @pytest.mark.parametrize("which", ["plain", "draft", "stream_draft"])
 def test_portions_where_memory_is_short(which, monkeypatch):
     """With little free memory a prompt runs in single chunks, as it would without longer portions: the same bits."""
