@@ -1071,17 +1071,18 @@ namespace {
 // md_linear_fused, md_linear_few: the same arguments; which kernel takes them
 int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream, const void* side_w = nullptr, int side_N = 0, void* side_out = nullptr,
               int64_t side_ldo = 0) {
-    MD_CHECK_ARG(a && a->x && a->w_packed && a->out, "md_linear_%s: null pointer argument", few ? "few" : "fused");
+    const char* who = few ? "md_linear_few" : side_w ? "md_linear_fused_beside" : "md_linear_fused";
+    MD_CHECK_ARG(a && a->x && a->w_packed && a->out, "%s: null pointer argument", who);
     MD_CHECK_ARG(few ? md_linear_few_supported(a->M, a->N, a->K, a->epilogue) > 0 : md_linear_fused_supported(a->M, a->N, a->K, a->epilogue),
-                 "md_linear_%s: unsupported shape M=%d N=%d K=%d epilogue=%d (need 1 <= M <= %d, K %% %d == 0, "
-                 "N %% 32 == 0)", few ? "few" : "fused", a->M, a->N, a->K, a->epilogue, few ? 16 : 256, few ? 256 : 128);
+                 "%s: unsupported shape M=%d N=%d K=%d epilogue=%d (need 1 <= M <= %d, K %% %d == 0, "
+                 "N %% 32 == 0)", who, a->M, a->N, a->K, a->epilogue, few ? 16 : 256, few ? 256 : 128);
     MD_CHECK_ARG(aligned16(a->x) && aligned16(a->w_packed) && aligned16(a->out) && a->ldx % 8 == 0 && a->ldo % 2 == 0,
-                 "md_linear_fused: x / w / out must be 16-byte aligned, ldx %% 8 == 0, ldo %% 2 == 0");
+                 "%s: x / w / out must be 16-byte aligned, ldx %% 8 == 0, ldo %% 2 == 0", who);
     const bool gated = a->epilogue == FL_SWIGLU || a->epilogue == FL_GEGLU;
-    MD_CHECK_ARG(!(gated && a->bias), "md_linear_fused: the gated epilogues take no bias");
+    MD_CHECK_ARG(!(gated && a->bias), "%s: the gated epilogues take no bias", who);
     // the kernel addresses x with 32-bit byte offsets from a scalar base
     MD_CHECK_ARG(a->ldx > 0 && ((int64_t)(a->M - 1) * a->ldx + a->K) * 2 < ((int64_t)1 << 32),
-                 "md_linear_fused: x spans more than 4 GiB (M=%d, ldx=%lld): pass a compact activation tensor", a->M,
+                 "%s: x spans more than 4 GiB (M=%d, ldx=%lld): pass a compact activation tensor", who, a->M,
                  (long long)a->ldx);
     TileParams p = {};
     p.x = (const bf16_t*)a->x;
@@ -1101,17 +1102,17 @@ int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream, const
     p.side_tiles = side_N / 32;
     if (a->pro_ssq) {
         MD_CHECK_ARG(few || gated || a->epilogue == FL_ROPE_APPEND,
-                     "md_linear_fused: the deferred-RMSNorm prologue exists for the qkv and w1|w3 linears");
+                     "%s: the deferred-RMSNorm prologue exists for the qkv and w1|w3 linears", who);
         MD_CHECK_ARG(a->pro_norm_w && a->pro_tiles > 0 && aligned16(a->pro_norm_w),
-                     "md_linear_fused: the deferred-RMSNorm prologue needs the norm weight (16-byte aligned) and pro_tiles");
+                     "%s: the deferred-RMSNorm prologue needs the norm weight (16-byte aligned) and pro_tiles", who);
         MD_CHECK_ARG(a->pro_tiles * 32 == a->K || a->pro_tiles * 16 == a->K,
-                     "md_linear_fused: pro_ssq must hold K / 32 = %d partial sums per row (or twice as many), got %d", a->K / 32, a->pro_tiles);
+                     "%s: pro_ssq must hold K / 32 = %d partial sums per row (or twice as many), got %d", who, a->K / 32, a->pro_tiles);
         p.pro_ssq = a->pro_ssq;
         p.pro_w = (const bf16_t*)a->pro_norm_w;
         p.pro_eps = a->pro_eps;
         p.pro_tiles = a->pro_tiles;
     }
-    MD_CHECK_ARG(!a->ssq_out || a->epilogue == FL_RESID, "md_linear_fused: ssq_out belongs to the residual epilogue");
+    MD_CHECK_ARG(!a->ssq_out || a->epilogue == FL_RESID, "%s: ssq_out belongs to the residual epilogue", who);
     p.ssq_out = a->ssq_out;
     p.dbg = g_tile_dbg;
     hipStream_t st = (hipStream_t)stream;
@@ -1127,35 +1128,35 @@ int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream, const
         rc = few ? launch_few<FL_SWIGLU, false>(p, st) : launch_tile<FL_SWIGLU, false>(p, st);
         break;
     case FL_XIELU:
-        MD_CHECK_ARG(a->act && !a->bias, "md_linear_fused: the xIELU epilogue needs `act` and takes no bias");
+        MD_CHECK_ARG(a->act && !a->bias, "%s: the xIELU epilogue needs `act` and takes no bias", who);
         p.act = a->act;
         rc = few ? launch_few<FL_XIELU, false>(p, st) : launch_tile<FL_XIELU, false>(p, st);
         break;
     case FL_RESID:
         MD_CHECK_ARG(a->resid && ((uintptr_t)a->resid & 3) == 0 && a->ldr % 2 == 0,
-                     "md_linear_fused: the residual epilogue needs `resid` (4-byte aligned, ldr %% 2 == 0)");
+                     "%s: the residual epilogue needs `resid` (4-byte aligned, ldr %% 2 == 0)", who);
         p.resid = (const bf16_t*)a->resid;
         p.ldr = a->ldr;
         rc = few ? launch_few<FL_RESID, false>(p, st) : launch_tile<FL_RESID, false>(p, st);
         break;
     default: {
         MD_CHECK_ARG(a->H > 0 && a->KH > 0 && (a->D == 64 || a->D == 128) && a->N == (a->H + 2 * a->KH) * a->D,
-                     "md_linear_fused: rope+append needs N == (H + 2 KH) * D with D in {64, 128} (H=%d KH=%d D=%d N=%d)",
+                     "%s: rope+append needs N == (H + 2 KH) * D with D in {64, 128} (H=%d KH=%d D=%d N=%d)", who,
                      a->H, a->KH, a->D, a->N);
         MD_CHECK_ARG(a->rows_per_req > 0 && a->M % a->rows_per_req == 0 && a->offsets && a->cos_sin && a->max_pos > 0 &&
                          a->page_size > 0,
-                     "md_linear_fused: rope+append needs rows_per_req | M, offsets, the RoPE table and page_size");
+                     "%s: rope+append needs rows_per_req | M, offsets, the RoPE table and page_size", who);
         MD_CHECK_ARG(a->cache && a->page_indices && a->page_indptr && a->last_page_len,
-                     "md_linear_fused: rope+append needs the paged cache and its page table");
+                     "%s: rope+append needs the paged cache and its page table", who);
         MD_CHECK_ARG(!a->cache2 || (a->page_indices2 && a->page_indptr2 && a->last_page_len2),
-                     "md_linear_fused: the second cache needs its page table");
-        MD_CHECK_ARG(a->ldo == (int64_t)a->H * a->D, "md_linear_fused: q_out must be contiguous [M][H*D]");
+                     "%s: the second cache needs its page table", who);
+        MD_CHECK_ARG(a->ldo == (int64_t)a->H * a->D, "%s: q_out must be contiguous [M][H*D]", who);
         int kvd = a->kv_dtype;
         p.hnd = (kvd & MD_KV_LAYOUT_HND) ? 1 : 0;
-        MD_CHECK_ARG((kvd & ~(MD_KV_DTYPE_MASK | MD_KV_LAYOUT_HND)) == 0, "md_linear_fused: unknown kv_dtype flags");
+        MD_CHECK_ARG((kvd & ~(MD_KV_DTYPE_MASK | MD_KV_LAYOUT_HND)) == 0, "%s: unknown kv_dtype flags", who);
         kvd &= MD_KV_DTYPE_MASK;
         MD_CHECK_ARG(kvd == MD_KV_BF16 || (kvd == MD_KV_FP8_E4M3 && a->k_scale && a->v_scale),
-                     "md_linear_fused: kv_dtype must be MD_KV_BF16 or MD_KV_FP8_E4M3 (with per-head scales)");
+                     "%s: kv_dtype must be MD_KV_BF16 or MD_KV_FP8_E4M3 (with per-head scales)", who);
         p.H = a->H;
         p.KH = a->KH;
         p.D = a->D;
@@ -1169,14 +1170,14 @@ int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream, const
         p.k_scale = a->k_scale;
         p.v_scale = a->v_scale;
         p.overflow = md_page_overflow_counter_device();
-        MD_CHECK_ARG(p.overflow, "md_linear_fused: cannot resolve the page-overflow counter");
+        MD_CHECK_ARG(p.overflow, "%s: cannot resolve the page-overflow counter", who);
         const bool fp8 = kvd == MD_KV_FP8_E4M3;
         if (few) rc = fp8 ? launch_few<FL_ROPE_APPEND, true>(p, st) : launch_few<FL_ROPE_APPEND, false>(p, st);
         else rc = fp8 ? launch_tile<FL_ROPE_APPEND, true>(p, st) : launch_tile<FL_ROPE_APPEND, false>(p, st);
     }
     }
     if (rc != MD_OK) return rc;
-    MD_CHECK_LAUNCH("md_linear_fused");
+    MD_CHECK_LAUNCH(who);
     return MD_OK;
 }
 }  // namespace

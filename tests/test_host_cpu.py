@@ -805,6 +805,19 @@ def test_hnd_page_layout_host_logic(cpu_ops_patched, ckpt_dir):
         d.model.setup_caches(num_pages=4, streaming=True, draft_budget=gc.BUDGET, kv_layout="HND")
 
 
+def test_the_tile_kernels_entries_report_errors_by_their_own_names():
+    import ctypes
+
+    from magicdec_amd import _lib
+    lib = _lib.load()
+    a = _lib.FusedLinearArgs()
+    a.x = a.w_packed = a.out = a.bias = 16
+    a.M, a.N, a.K, a.ldx, a.ldo, a.epilogue = 4, 64, 256, 256, 32, 1              # a gated product with a bias
+    for who, rest in (("md_linear_fused", ()), ("md_linear_few", ()), ("md_linear_fused_beside", (16, 32, 16, 32))):
+        assert getattr(lib, who)(ctypes.byref(a), *rest, None) < 0
+        assert lib.md_last_error_string().decode().startswith(who + ":")
+
+
 def test_c_abi_rejects_unknown_kv_dtype_flags():
     """kv_dtype carries the storage type in its low byte and MD_KV_LAYOUT_HND (0x100) as a flag; anything else is
     refused before a kernel is launched (host pointers are enough to reach the check)."""
