@@ -116,7 +116,8 @@ __global__ __launch_bounds__(256) void latent_append_kernel(const LatentParams p
 // ------------------------------------------------------------------------------------------------ queries of a step
 // q[M][N] = rms(query latent) * dq_norm . W^T with W in the streaming layout [N/32][K/16][64][8] (K = 256 STEPS), and beside it, in workgroups
 // behind the product's, the append.  A workgroup has 32 rows x 32 columns, each of its sixteen wavefronts a sixteenth of K: all that a wavefront
-// reads is requested at once, the norm is formed of what it holds while the weight is on its way, and its bits are latent_append_kernel's.
+// reads is requested at once, and the norm is formed of what it holds while the weight is on its way: rounded where latent_append_kernel
+// rounds, its sum of squares of another order, so that a latent may round the other way.  The appended row is that kernel's bit for bit.
 //
 // A chain of latencies bounds a step of few rows: as launches of their own the norm and append take 4.6 us and the product 4.6 (32 rows of
 // 3 072 x 768), this 5.3.
