@@ -628,18 +628,20 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
 }
 
 // ---- md_linear_few: at most 16 rows, 16 columns a workgroup ------------------------------------------------------------------
-// A column tile of 32 is coarse where a step has a row or a few: 768 x 3 072 is 24 workgroups, 4 096 columns 128 of 256 CUs, and 28 672 are 896
-// tiles, which leave half the CUs with four and half with three.  v_mfma_f32_16x16x32 takes 16 columns of the same streaming layout
-// (256-byte pieces of a fragment, whole lines), so that twice the workgroups share the weight, K is split over 8 or 16 wavefronts as in the
-// tile kernel, and no K split over workgroups is left to combine.  One row, us, the 32-column form / this one: 768 x 3 072 7.5 / 5.8,
+// A column tile of 32 is coarse where a step has a row or a few: 768 x 3 072 is 24 workgroups, 4 096 columns 128 of 256 CUs.
+// v_mfma_f32_16x16x32 takes 16 columns of the same streaming layout (256-byte pieces of a fragment, whole lines), so that twice the workgroups
+// share the weight; K is split over eight wavefronts (sixteen are slower everywhere: 4 096 x 14 336 24.1 us, eight 22.9; 2 048 x 2 048 6.4, 5.3),
+// and no K split over workgroups is left to combine.  One row, us, the 32-column form / this one: 768 x 3 072 7.5 / 5.8,
 // 3 584 x 3 584 10.2 / 8.2, 2 048 x 5 632 11.1 / 8.6, 4 096 x 14 336 27.4 / 22.9 (5.1 TB/s); wider than a round of the chip the fixed part of
-// twice the workgroups shows: 28 672 x 4 096 43.7 / 46.3.
+// twice the workgroups shows: 28 672 x 4 096 43.7 / 46.3, so that a step's gated product and its activations stay on the 32-column form, and
+// reach this one through the C entry alone.
 // The partial sums of squares of a residual epilogue are of 16 columns each.  A gated tile is 8 columns of w1 and the same 8 of w3.
+constexpr int kFewNW = 8;                          // wavefronts, K slices
 constexpr int kFewLds = 16 * kPitch;               // a wavefront's activation image
 
-template <int EPI, bool FP8, int NW, bool PRO, int AI>
-__global__ __launch_bounds__(64 * NW, 4) void few_gemm_kernel(const TileParams p) {
-    constexpr int R = 4 * AI, kRD = 8;             // staged rows, W fragments in flight
+template <int EPI, bool FP8, bool PRO, int AI>
+__global__ __launch_bounds__(64 * kFewNW, 4) void few_gemm_kernel(const TileParams p) {
+    constexpr int NW = kFewNW, R = 4 * AI, kRD = 8;             // staged rows, W fragments in flight
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];       // NW x kFewLds, 16 floats
     const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, q = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -861,22 +863,14 @@ int launch_tile(const TileParams& p, hipStream_t st) {
     return launch_tile_pro<EPI, FP8, false>(p, st);
 }
 
-template <int EPI, bool FP8, int NW, bool PRO, int AI>
+template <int EPI, bool FP8, bool PRO, int AI>
 int launch_few_cfg(const TileParams& p, hipStream_t st) {
-    constexpr int lds = NW * kFewLds + 64;
-    auto k = few_gemm_kernel<EPI, FP8, NW, PRO, AI>;
-    static MdPerDeviceOnce once;
-    if (lds > 64 * 1024 && once.first() &&
-        hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) {
-        once.undo();
-        md_set_error("md_linear_few: hipFuncSetAttribute(%d B LDS) failed", lds);
-        return MD_ERR_LAUNCH;
-    }
-    hipLaunchKernelGGL(k, dim3(p.N / 16), dim3(64 * NW), lds, st, p);
+    constexpr int lds = kFewNW * kFewLds + 64;
+    static_assert(lds <= 64 * 1024, "no limit to raise");
+    hipLaunchKernelGGL((few_gemm_kernel<EPI, FP8, PRO, AI>), dim3(p.N / 16), dim3(64 * kFewNW), lds, st, p);
     return MD_OK;
 }
 
-// (Sixteen wavefronts are slower everywhere: 4 096 x 14 336 24.1 us, eight 22.9; 2 048 x 2 048 6.4, 5.3.)
 template <int EPI, bool FP8, bool PRO>
 int launch_few_pro(const TileParams& p, hipStream_t st) {
     // a head behind a deferred norm, wide: 32-column tiles, whose fixed part is paid half as often (32 000 x 4 096 46 us, 51.6 on 16
@@ -884,7 +878,7 @@ int launch_few_pro(const TileParams& p, hipStream_t st) {
     if constexpr (EPI == FL_NONE && PRO) {
         if (p.N > 4096) return p.M <= 4 ? launch_tile_cfg<EPI, FP8, 8, true, PRO, 1, 1, 1>(p, st) : launch_tile_cfg<EPI, FP8, 8, true, PRO, 1, 1, 4>(p, st);
     }
-    return p.M <= 4 ? launch_few_cfg<EPI, FP8, 8, PRO, 1>(p, st) : launch_few_cfg<EPI, FP8, 8, PRO, 4>(p, st);
+    return p.M <= 4 ? launch_few_cfg<EPI, FP8, PRO, 1>(p, st) : launch_few_cfg<EPI, FP8, PRO, 4>(p, st);
 }
 
 template <int EPI, bool FP8>

@@ -339,17 +339,17 @@ __global__ __launch_bounds__(256, (f32_waves_per_simd<DK, DV, QT, KT, SHARED>())
 // softmax moves only where it must; four columns of V a read.  The shape above: four wavefronts on 64 rows together 445 us, this 310, with
 // these 277 (80 TFLOP/s; products alone 250).  One prompt of 2 500 470 -> 268, 4 x 600 at 16 / 4 heads of 128 148 -> 97; tiles of 64 keys
 // 10 % slower, eight wavefronts 2 to 20 %.
-template <int DK, int DV, int KT, bool SHARED>
+template <int DK, int DV, int KT>
 constexpr int rows_lds_bytes() {
-    return 2 * KT * (DK + 4 + (SHARED ? 0 : DV + 4)) * 4 + 16;
+    return 2 * KT * (DK + DV + 8) * 4 + 16;
 }
 
-template <typename T, int DK, int DV, int KT, int NW, int OCC, bool SHARED>
+template <typename T, int DK, int DV, int KT, int NW, int OCC>
 __global__ __launch_bounds__(64 * NW, OCC) void xattn_f32_rows_kernel(const XattnParams p, const F32Launch L) {
     typedef typename Vec4<T>::type vec4;
-    constexpr int R = 16 * NW, NT = 64 * NW, KP = DK + 4, VP = SHARED ? KP : DV + 4, KB = KT / 16, NV = DV / 16;
-    constexpr int kTile = KT * (KP + (SHARED ? 0 : VP));         // floats of one buffer
-    constexpr int LK = KT * DK / (4 * NT), LV = SHARED ? 1 : KT * DV / (4 * NT);
+    constexpr int R = 16 * NW, NT = 64 * NW, KP = DK + 4, VP = DV + 4, KB = KT / 16, NV = DV / 16;
+    constexpr int kTile = KT * (KP + VP);                        // floats of one buffer
+    constexpr int LK = KT * DK / (4 * NT), LV = KT * DV / (4 * NT);
     static_assert(KT * DK % (4 * NT) == 0 && KT * DV % (4 * NT) == 0 && DK % 16 == 0 && DV % 64 == 0 && KT == 32, "tile shapes");
     extern __shared__ __attribute__((aligned(16))) float lds[];
     int* sbad = reinterpret_cast<int*>(lds + 2 * kTile);         // [3]: the tile's values hold an infinity or a NaN
@@ -429,12 +429,10 @@ __global__ __launch_bounds__(64 * NW, OCC) void xattn_f32_rows_kernel(const Xatt
             const_cast<T*>(reinterpret_cast<const T*>(p.k_cache) + line * p.ldk), (short)0, keys * p.ldk * (int)sizeof(T), 0x00020000);
 #pragma unroll
         for (int i = 0; i < LK; ++i) kr[i] = fetch(rk, kat[i]);
-        if constexpr (!SHARED) {
-            const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<T*>(reinterpret_cast<const T*>(p.v_cache) + line * p.ldv), (short)0, keys * p.ldv * (int)sizeof(T), 0x00020000);
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<T*>(reinterpret_cast<const T*>(p.v_cache) + line * p.ldv), (short)0, keys * p.ldv * (int)sizeof(T), 0x00020000);
 #pragma unroll
-            for (int i = 0; i < LV; ++i) vr[i] = fetch(rv, vat[i]);
-        }
+        for (int i = 0; i < LV; ++i) vr[i] = fetch(rv, vat[i]);
     };
     auto stage = [&](int t) {                // (keys past the workgroup's last one are zeros: their memory may hold anything)
         float* sk = lds + ((t - t0) & 1) * kTile;
@@ -442,19 +440,14 @@ __global__ __launch_bounds__(64 * NW, OCC) void xattn_f32_rows_kernel(const Xatt
 #pragma unroll
         for (int i = 0; i < LK; ++i) {
             const int e = tid + NT * i, key = e / (DK / 4), d = (e % (DK / 4)) * 4;
-            const f32x4 v = __builtin_convertvector(kr[i], f32x4);
-            *reinterpret_cast<f32x4*>(sk + key * KP + d) = v;
-            if (SHARED)
-                for (int x = 0; x < 4; ++x) worst = fmaf(v[x], 0.f, worst);
+            *reinterpret_cast<f32x4*>(sk + key * KP + d) = __builtin_convertvector(kr[i], f32x4);
         }
-        if constexpr (!SHARED) {
 #pragma unroll
-            for (int i = 0; i < LV; ++i) {
-                const int e = tid + NT * i, key = e / (DV / 4), d = (e % (DV / 4)) * 4;
-                const f32x4 v = __builtin_convertvector(vr[i], f32x4);
-                *reinterpret_cast<f32x4*>(sk + KT * KP + key * VP + d) = v;
-                for (int x = 0; x < 4; ++x) worst = fmaf(v[x], 0.f, worst);
-            }
+        for (int i = 0; i < LV; ++i) {
+            const int e = tid + NT * i, key = e / (DV / 4), d = (e % (DV / 4)) * 4;
+            const f32x4 v = __builtin_convertvector(vr[i], f32x4);
+            *reinterpret_cast<f32x4*>(sk + KT * KP + key * VP + d) = v;
+            for (int x = 0; x < 4; ++x) worst = fmaf(v[x], 0.f, worst);
         }
         if (__builtin_amdgcn_ballot_w64(worst != 0.f) != 0 && lane == 0) sbad[t % 3] = 1;
     };
@@ -479,7 +472,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void xattn_f32_rows_kernel(const Xatt
         const int base = t * KT;
         if (base <= any_hi && base + KT > any_lo) {
             const float* sk = lds + ((t - t0) & 1) * kTile;
-            const float* sv = SHARED ? sk : sk + KT * KP;
+            const float* sv = sk + KT * KP;
             // ---- scores: lane (lq, lc) gets keys 16 k + 4 lc + e of row lq
             f32x4 s[KB];
 #pragma unroll
@@ -699,20 +692,20 @@ int launch(const XattnParams& p, const F32Launch& L, hipStream_t st) {
     return MD_OK;
 }
 
-template <typename T, int DK, int DV, int KT, int NW, int OCC, bool SHARED>
+template <typename T, int DK, int DV, int KT, int NW, int OCC>
 int launch_rows(const XattnParams& p, const F32Launch& L, hipStream_t st) {
-    constexpr int bytes = rows_lds_bytes<DK, DV, KT, SHARED>();
+    constexpr int bytes = rows_lds_bytes<DK, DV, KT>();
     static_assert(bytes <= 160 * 1024, "LDS");
     static MdPerDeviceOnce once;
     if (bytes > 64 * 1024 && once.first()) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&xattn_f32_rows_kernel<T, DK, DV, KT, NW, OCC, SHARED>),
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(&xattn_f32_rows_kernel<T, DK, DV, KT, NW, OCC>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
             once.undo();
             md_set_error("attention: cannot raise the LDS limit to %d bytes", bytes);
             return MD_ERR_LAUNCH;
         }
     }
-    hipLaunchKernelGGL((xattn_f32_rows_kernel<T, DK, DV, KT, NW, OCC, SHARED>), dim3((unsigned)(p.KH * p.B * L.nq * L.nsplit)), dim3(64 * NW),
+    hipLaunchKernelGGL((xattn_f32_rows_kernel<T, DK, DV, KT, NW, OCC>), dim3((unsigned)(p.KH * p.B * L.nq * L.nsplit)), dim3(64 * NW),
                        bytes, st, p, L);
     if (L.nsplit > 1) {
         const int64_t threads = (int64_t)p.B * p.KH * L.nq * L.R * (L.dvw / 4);
@@ -726,8 +719,8 @@ template <typename T>
 int launch_shape(const XattnParams& p, Shape s, const F32Launch& L, hipStream_t st) {
     const bool few = L.R == 16;
     switch (s) {
-    case k64: return few ? launch<T, 64, 64, 1, 64, false>(p, L, st) : launch_rows<T, 64, 64, 32, 4, 4, false>(p, L, st);
-    case k128: return few ? launch<T, 128, 128, 1, 32, false>(p, L, st) : launch_rows<T, 128, 128, 32, 4, 2, false>(p, L, st);
+    case k64: return few ? launch<T, 64, 64, 1, 64, false>(p, L, st) : launch_rows<T, 64, 64, 32, 4, 4>(p, L, st);
+    case k128: return few ? launch<T, 128, 128, 1, 32, false>(p, L, st) : launch_rows<T, 128, 128, 32, 4, 2>(p, L, st);
     case k256: return few ? launch<T, 256, 256, 1, 32, false>(p, L, st) : launch<T, 256, 256, 2, 32, false>(p, L, st);
     case kShared320: return few ? launch<T, 320, 256, 1, 32, true>(p, L, st) : launch<T, 320, 256, 2, 32, true>(p, L, st);
     default: return few ? launch<T, 576, 512, 1, 32, true>(p, L, st) : launch<T, 576, 512, 2, 32, true>(p, L, st);
