@@ -432,11 +432,12 @@ def use_few(M: int, N: int, K: int) -> bool:
     """md_linear_few in the place of what `choose` (and use_split) gives one of the framework's own kernels, for at most 16 rows?  Its tiles
     are of 16 columns: where those are one round of the chip at most, twice the CUs load the weight.  us, md_linear_fused / here, 1 and 16
     rows, 40 random products of 512 to 4 096 columns: 608 x 2 816 7.4 -> 5.6, 8.9 -> 6.5; 3 136 x 4 864 12.9 -> 9.4, 13.8 -> 11.0;
-    2 048 x 2 048 5.6 -> 5.3, 6.2 -> 5.8; level at K = 1 280 and 7 % slower below 1 024.  Wider ones lose (4 352 x 4 352 12.9 / 14.5).
+    2 048 x 2 048 5.6 -> 5.3, 6.2 -> 5.8; level at K = 1 280 and 7 % slower below 1 024.  Wider ones lose (4 352 x 4 352 12.9 / 14.5), and
+    so do 128 columns and fewer, a handful of workgroups in either form (64 x 1 536 1.11 times, 128 x 1 280 1.08; 160 to 256 level or ahead).
     Deep ones (asked for with a row to four) against the K split and the weight-streaming kernel, with the norm behind them, which here
     the next product absorbs: 4 096 x 14 336 26.4 -> 22.9, 2 048 x 8 192 11.4 -> 10.4, 2 464 x 13 056 20.4 -> 17.7, but 608 x 14 592 (38
     workgroups) 10.1 / 15.3."""
-    if not joint_launches() or not 1 <= M <= 16 or N > 16 * CUS or N % 32 or K % 256 or K < 1024:
+    if not joint_launches() or not 1 <= M <= 16 or not 128 < N <= 16 * CUS or N % 32 or K % 256 or K < 1024:
         return False
     return K < SPLIT_MIN_K or N >= 1024
 

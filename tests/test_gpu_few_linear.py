@@ -99,3 +99,8 @@ def test_rule():
     assert use_few(1, 768, 3072) and use_few(16, 4096, 4096) and use_few(4, 4096, 14336)
     for M, N, K in ((17, 768, 3072), (1, 4128, 4096), (1, 768, 768), (1, 992, 8192), (1, 2048, 1152), (0, 768, 3072)):
         assert not use_few(M, N, K)
+
+
+def test_rule_ends_where_either_form_is_a_handful_of_workgroups():
+    from magicdec_amd.Engine.gemm_policy import use_few
+    assert use_few(1, 160, 1536) and not any(use_few(M, N, 1536) for M in (1, 16) for N in (32, 128))
