@@ -43,6 +43,11 @@ from .. import ops
 from .gemm_policy import fused_mode, prompt_over_block, prompt_rows, use_few
 
 
+# A deep output projection leaves its norm to the next product up to the rows which that one stages in one instruction: at 16 rows of the
+# 7B model its norm costs more than the launch that is saved, 322 / 331 us of a two-layer step
+DEEP_FEW_ROWS = 4
+
+
 def find_multiple(n: int, k: int) -> int:
     return n if n % k == 0 else n + k - (n % k)
 
@@ -710,7 +715,8 @@ class Transformer(nn.Module):
         """Output projection of a sub-layer (wo / w2), the residual add and the RMSNorm for the next sub-layer:
         (h, y) = (x + sum_ranks(inp . W^T), rmsnorm(h) * w).  Without tensor parallelism and on a launch-bound shape the
         projection and the residual add are one launch (md_linear_fused, MD_FL_RESID) and y is returned as an
-        `ops.DeferredNorm` (also on a deep one of few rows, if `then`, the weight that y goes to and its kind, takes such); otherwise the projection, then `_reduce_add_norm` (collective + fused add + norm)."""
+        `ops.DeferredNorm` (also on a deep one of few rows, if `then`, the weight that y goes to and its kind, takes such; None: not asked);
+        otherwise the projection, then `_reduce_add_norm` (collective + fused add + norm)."""
         if group is None and x.is_contiguous() and self._fused_here(inp, lin.weight, "resid"):
             # the norm is DEFERRED: the residual epilogue leaves the per-row partial sums of squares, and the linear that
             # consumes the normalised rows (w1|w3, the next layer's wqkv) applies rmsnorm on the fly; a consumer that
@@ -723,11 +729,10 @@ class Transformer(nn.Module):
             w = lin.weight
             M, K = inp.shape
             pk = self._packed.get(id(w))
-            if (pk is not None and w.dtype == torch.bfloat16 and inp.stride(-1) == 1 and x.is_contiguous() and then is not None
-                    and M <= 4 and use_few(M, w.shape[0], K) and (use_split(M, w.shape[0], K, "resid") or choose(M, w.shape[0], K, False, False, True, "resid") == "skinny")
+            if (then is not None and pk is not None and w.dtype == torch.bfloat16 and inp.stride(-1) == 1 and x.is_contiguous()
+                    and M <= DEEP_FEW_ROWS and use_few(M, w.shape[0], K) and (use_split(M, w.shape[0], K, "resid") or choose(M, w.shape[0], K, False, False, True, "resid") == "skinny")
                     and self._absorbs_norm(M, *then)):
-                # a row or a few of a deep product: one launch, its norm in the next product's.  (To four rows, which that one stages
-                # in one instruction: at 16 rows of the 7B model its norm costs more than the launch, 322 / 331 us of a two-layer step)
+                # a row or a few of a deep product: one launch, its norm in the next product's
                 h, ssq = ops.fused_linear(inp, pk, lin.bias, resid=x, want_ssq=True, few=True)
                 return h, ops.DeferredNorm(h, ssq, norm.weight, norm.eps)
             if (pk is not None and w.dtype == torch.bfloat16 and inp.stride(-1) == 1
@@ -785,15 +790,17 @@ class Transformer(nn.Module):
         else:
             x = emb(idx).view(idx.numel(), -1)
             y = ops.rmsnorm(x, norm.weight, norm.eps)
+        few = x.shape[0] <= DEEP_FEW_ROWS
         for i, layer in enumerate(layers):
             o = attn_fn(i, layer, y, n)
             x, y = self._proj_add_norm(o.view(o.shape[0], -1), layer.attention.wo, x, layer.ffn_norm,
-                                       layer.attention.process_group, (self._w13[i], "swiglu"))
+                                       layer.attention.process_group, (self._w13[i], "swiglu") if few else None)
             act = self._linear(y, None, swiglu_w13=(self._w13[i], self._s13[i]))
             last = i + 1 == len(layers)
-            nxt = self.norm if last else layers[i + 1].attention_norm
-            then = (self.output.weight, "plain") if last else (layers[i + 1].attention.wqkv.weight, "qkv")
-            x, y = self._proj_add_norm(act, layer.feed_forward.w2, x, nxt, layer.feed_forward.process_group, None if self.skip_head and last else then)
+            nxt, then = self.norm if last else layers[i + 1].attention_norm, None
+            if few and not (self.skip_head and last):
+                then = (self.output.weight, "plain") if last else (layers[i + 1].attention.wqkv.weight, "qkv")
+            x, y = self._proj_add_norm(act, layer.feed_forward.w2, x, nxt, layer.feed_forward.process_group, then)
         if self.skip_head:
             return None
         if head_rows is not None:

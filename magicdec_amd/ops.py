@@ -1231,11 +1231,16 @@ def latent_append(z, s: LatentSpec, cache, rows: StepRows, page_indices, page_in
     return cq
 
 
+@functools.lru_cache(maxsize=1024)
+def _latent_query_shape(M, N, q_rank):
+    return _lib.load().md_latent_query_supported(int(M), int(N), int(q_rank)) > 0
+
+
 def latent_query_supported(z, s: LatentSpec, weight: "PackedWeight", cache):
     """True when md_latent_query takes the rows z: a step's, bf16, dense enough for whole pieces."""
     return (z.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and not weight.swiglu and weight.K == s.q_rank and z.stride(0) % 8 == 0
             and s.kv_rank % 8 == 0 and not (z.data_ptr() | s.dq_norm.data_ptr() | (s.kv_norm.data_ptr() if s.kv_norm is not None else 0)) % 16
-            and cache.data_ptr() % 32 == 0 and _lib.load().md_latent_query_supported(z.shape[0], weight.N, s.q_rank) > 0)
+            and cache.data_ptr() % 32 == 0 and _latent_query_shape(z.shape[0], weight.N, s.q_rank))
 
 
 def latent_query(z, s: LatentSpec, weight: "PackedWeight", cache, rows: StepRows, page_indices, page_indptr, max_pages):
