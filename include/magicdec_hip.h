@@ -338,7 +338,7 @@ int md_linear_f32_few(const float* x, int64_t ldx, const float* w, float* out, i
 
 /* md_linear_f32_thirds (csrc/f32thirds.hip): the same on the bf16 matrix instructions, every number as the sum of three bf16 numbers (six
  * products of their parts, 32-bit sums): the error against 64 bits is 0.6 to 0.9 of md_linear_f32's for dense operands, 1.1 to 1.3 of it where many
- * are zero; of a term, at most 2^-24 more, and 2^-134 of one operand's numbers below 2^-110.  K < 2^20.  ws: md_linear_f32_thirds_workspace(M, K) bytes, 16-byte
+ * are zero; of a term, at most 2^-24 more, and 2^-134 of one operand's numbers below 2^-110.  K < 2^20, M <= 16 * 65 535.  ws: md_linear_f32_thirds_workspace(M, K) bytes, 16-byte
  * aligned (x in three parts), free again behind the call on its stream.  _supported: 1 if it takes the shape and is expected to be faster than
  * md_linear_f32 and a library GEMM.  tile: 0, or 1000 * rows + columns (256 / 192 / 160 / 128 x 256, 256 / 192 / 128 / 64 x 128). */
 int md_linear_f32_thirds_supported(int M, int N, int K);

@@ -346,6 +346,7 @@ extern "C" int md_linear_f32_thirds(const float* x, int64_t ldx, const float* w,
     MD_CHECK_ARG(shape_ok(M, N, K) && ldx >= K && ldx % 4 == 0 && ldo >= N && ldo % 4 == 0 &&
                      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)ws) & 15) == 0,
                  "md_linear_f32_thirds: M=%d N=%d K=%d ldx=%lld ldo=%lld unsupported", M, N, K, (long long)ldx, (long long)ldo);
+    MD_CHECK_ARG(M <= 16 * 65535, "md_linear_f32_thirds: M=%d: the parts' grid has a row of workgroups for 16 rows, at most 65 535", M);
     MD_CHECK_ARG(ws_bytes >= md_linear_f32_thirds_workspace(M, K), "md_linear_f32_thirds: workspace of %zu bytes, %zu needed", ws_bytes,
                  md_linear_f32_thirds_workspace(M, K));
     ThirdsParams p;

@@ -694,7 +694,7 @@ def linear_f32_thirds(x, weight, tile=0):
     (M, K), N = x.shape, weight.shape[0]
     lib = _lib.load()
     parts = max(1, -(-6 * M * K // THIRDS_BYTES))
-    rows = -(-M // (256 * parts)) * 256
+    rows = min(-(-M // (256 * parts)) * 256, 4095 * 256)              # (a call takes 16 * 65 535)
     out = torch.empty((M, N), dtype=x.dtype, device=x.device)           # (in front of the scratch, which is not needed)
     try:
         ws = torch.empty(max(1, lib.md_linear_f32_thirds_workspace(min(M, rows), K)), dtype=torch.uint8, device=x.device)

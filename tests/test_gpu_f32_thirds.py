@@ -106,6 +106,15 @@ def test_rows_in_several_calls(monkeypatch):
     assert torch.equal(ops.linear_f32_thirds(x, w), whole)
 
 
+def test_more_rows_than_a_call_takes():
+    from magicdec_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(2)
+    x, w = torch.randn(16 * 65535 + 100, 32, device=DEV, generator=g), torch.randn(4, 32, device=DEV, generator=g)
+    out = ops.linear_f32_thirds(x, w)
+    for at in (0, 4095 * 256 - 64, x.shape[0] - 128):
+        assert torch.equal(out[at:at + 128], ops.linear_f32_thirds(x[at:at + 128], w))
+
+
 def room(monkeypatch, nbytes):
     """torch.empty finds no memory once `nbytes` are asked for in all."""
     real, left = torch.empty, [nbytes]

@@ -818,6 +818,14 @@ def test_the_tile_kernels_entries_report_errors_by_their_own_names():
         assert lib.md_last_error_string().decode().startswith(who + ":")
 
 
+def test_thirds_refuse_more_rows_than_a_grid_has():
+    from magicdec_amd import _lib
+    lib = _lib.load()
+    M = 16 * 65535 + 1
+    assert lib.md_linear_f32_thirds(16, 32, 16, 16, 4, M, 4, 32, 0, 16, lib.md_linear_f32_thirds_workspace(M, 32), None) < 0
+    assert "65 535" in lib.md_last_error_string().decode()
+
+
 def test_c_abi_rejects_unknown_kv_dtype_flags():
     """kv_dtype carries the storage type in its low byte and MD_KV_LAYOUT_HND (0x100) as a flag; anything else is
     refused before a kernel is launched (host pointers are enough to reach the check)."""
