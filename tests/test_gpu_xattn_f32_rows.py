@@ -77,3 +77,62 @@ def test_against_float64(H, KH, D, DV, lens, pos, chunk, kind):
         ref, off = reference(q[p:], spec, n, p, past)
         last = ref.isinf()
         assert torch.equal(o.isinf(), last) and (o[~last].double() - ref[~last]).abs().le(off[~last]).all(), (o.double() - ref)[~last].abs().max()
+
+
+def attend_alone(q, k, v, spec, page=32):
+    """One sequence from its first token: q [n, H, D], k [n, KH, D], v [n, KH, DV]"""
+    from magicdec_amd import ops
+    n, pages = q.shape[0], -(-q.shape[0] // page)
+    caches = [torch.zeros(pages, spec.KH, page, ops.head_pad(w), device=DEV) for w in (spec.D, spec.DV)]
+    return ops.extended_attention(torch.cat([x.flatten(1) for x in (q, k, v)], 1), spec, *caches, ops.StepRows(i32([0, n]), i32([0]), n), i32(list(range(pages))),
+                                  i32([0, pages]), pages, ops.AttnWorkspace(DEV)).view(n, spec.H, spec.DV)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("score", [3.0, 1e6, -1e9, -1e28])
+def test_equal_scores_weigh_the_same_whatever_their_size(D, score):
+    """Tiles of equal scores: each value of the past counts once.  (A scaled score that is part of a fused operation in one tile and rounded
+    in another is half a step of its own size off.)"""
+    from magicdec_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(D)
+    H, KH, n = 32, 16, 300
+    spec = ops.XattnSpec(H, KH, D, D, D ** -0.5, 1e-6)
+    q, k = torch.ones(n, H, D, device=DEV), torch.full((n, KH, D), score / D * D ** 0.5, device=DEV)
+    v = torch.randn(n, KH, D, device=DEV, generator=g)
+    out, count = attend_alone(q, k, v, spec).double(), torch.arange(1, n + 1, device=DEV)[:, None, None]
+    mean, size = ((x.double().cumsum(0) / count).repeat_interleave(H // KH, 1) for x in (v, v.abs()))
+    assert (out - mean).abs().le(size * (n + 16) * 2.0 ** -23).all()
+
+
+@pytest.mark.parametrize("above", [0.0, 1.9, 3.9, 30.0])
+def test_values_near_the_end_of_the_range(above):
+    """Values whose sum over the keys is a number as long as weights are at most 1, behind a tile whose scores are lower by `above` (log2)."""
+    from magicdec_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(int(above))
+    H, KH, n, D = 32, 16, 400, 64
+    spec = ops.XattnSpec(H, KH, D, D, D ** -0.5, 1e-6)
+    q, k = torch.ones(n, H, D, device=DEV), torch.zeros(n, KH, D, device=DEV)
+    k[32:] = above / 1.4426950408889634 / D * D ** 0.5
+    v = (torch.rand(n, KH, D, device=DEV, generator=g) - 0.25) * 1.5e36
+    out = attend_alone(q, k, v, spec).double()
+    s = (torch.einsum("nhd,khd->hnk", q[:, ::2].double(), k.double()) * spec.scale).masked_fill(torch.ones(n, n, dtype=torch.bool, device=DEV).triu(1), -torch.inf)
+    w = torch.softmax(s, 2)
+    ref, size = (torch.einsum("hnk,khd->nhd", w, x.double()).repeat_interleave(2, 1) for x in (v, v.abs()))
+    assert out.isfinite().all() and (out - ref).abs().le(size * (n + 64) * 2.0 ** -22).all()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_error_of_a_biased_prompt(D):
+    """Against float64 no further off, as a 2-norm, than the kernel of row groups of 16, which takes each head alone (the order in which the
+    bias and the reference come off a score is worth a fifth of the error)."""
+    from magicdec_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(D)
+    H, n = 16, 700
+    b = [torch.rand(H, device=DEV, generator=g) * 2 for _ in range(2)]
+    spec = ops.XattnSpec(H, H, D, D, D ** -0.5, 1e-6, r1=b[0], r2=b[1])
+    qkv = torch.randn(n, 3 * H * D, device=DEV, generator=g)
+    heads = [x.view(n, H, D) for x in qkv.chunk(3, 1)]
+    none = torch.zeros(0, H * D, device=DEV, dtype=torch.float64)
+    ref = reference(qkv, spec, n, 0, (none, none))[0].view(n, H, D)
+    alone = [attend_alone(*(x[:, h:h + 1].contiguous() for x in heads), ops.XattnSpec(1, 1, D, D, D ** -0.5, 1e-6, r1=b[0][h:h + 1], r2=b[1][h:h + 1])) for h in range(H)]
+    assert (attend_alone(*heads, spec).double() - ref).norm() <= 1.03 * (torch.cat(alone, 1).double() - ref).norm()
