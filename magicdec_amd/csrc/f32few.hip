@@ -221,12 +221,14 @@ bool shape_ok(int M, int N, int K) {
 // Against the library over 1 800 products of 1 to 16 rows (16 to 140 000 columns, K = 256 to 16 384; operands from memory), which is the faster
 // one, us, library / here:
 //   * above 2 048 columns behind a K of 2 048: 4 096 x 4 096 17.1 / 18.6, 2 304 x 8 192 23.8 / 27.1 (its workgroups have 16 columns and all of K);
-//   * with nine rows and more, whose x is staged twice as often, behind that K everywhere (1 024 x 3 072 9.0 / 10.6, 64 x 8 192 16.3 / 17.7) and, of
-//     few columns, in front of it (128 x 1 536 6.1 / 6.9; from 512 on and at 256 x 2 048 level or ahead);
+//   * with nine rows and more, whose x is staged twice as often, over up to 1 024 columns behind that K (1 024 x 3 072 9.0 / 10.6, 64 x 8 192
+//     16.3 / 17.7), over more of them up to a K of 4 096 (2 048 x 3 072 11.7 / 12.7), and of few columns in front of it (128 x 1 536 6.1 / 6.9;
+//     from 512 on and at 256 x 2 048 level or ahead).  Deeper ones of more than 1 024 columns are level alone (2 048 x 8 192 22.3 / 23.1), a
+//     hundredth of a step faster in one, and less far off 64 bits (0.7 of the library's error);
 //   * where either is little more than a launch: 4 096 x 256 5.0 / 5.1, 1 024 x 256 4.1 / 4.6, 16 x 256 3.9 / 4.3, 512 x 512 4.6 / 5.0,
 //     384 x 768 1.03 times, but 128 x 256 9.9 / 4.5, 256 x 512 11.4 / 4.9, 768 x 512 5.7 / 5.0, 512 x 768 6.4 / 5.3;
 //   * of a very wide weight, 65 536 x 256 18.0 / 22.3 (40 000 0.97 on average).
-// What is left is 0.81 of the library's time on average, 1.09 at the worst (16 384 x 2 048, which the library likes).
+// What is left is 0.8 of the library's time on average, 1.09 at the worst (16 384 x 2 048, which the library likes).
 extern "C" int md_linear_f32_few_supported(int M, int N, int K) {
     MD_CHECK_ARG(M > 0 && N > 0 && K > 0, "md_linear_f32_few_supported: M=%d N=%d K=%d", M, N, K);
     if (!shape_ok(M, N, K)) return 0;
@@ -234,7 +236,8 @@ extern "C" int md_linear_f32_few_supported(int M, int N, int K) {
     if (K == 256) return N > 32 && N <= 256;
     if (K <= 768) return (N > 32 && N <= 256) || N >= (K == 512 ? 768 : 512);
     if (N > 2048) return K <= 2048;
-    return M <= 8 || (K <= 2048 && (N >= 512 || (N >= 256 && K > 1536)));
+    if (M <= 8) return 1;
+    return K <= 2048 ? N >= 512 || (N >= 256 && K > 1536) : N > 1024 && K > 4096;
 }
 
 extern "C" int md_linear_f32_few(const float* x, int64_t ldx, const float* w, float* out, int64_t ldo, int M, int N, int K, int tile, md_stream_t stream) {

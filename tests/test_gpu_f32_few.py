@@ -55,12 +55,13 @@ def test_refused():
 
 
 def test_shapes_that_the_library_multiplies_faster():
-    """They stay there: deep ones of more than 2 048 columns, deep or very narrow ones of nine rows and more, little more than a launch."""
+    """They stay there: deep ones of more than 2 048 columns, deep or very narrow ones of nine rows and more over up to 1 024, little more than a
+    launch."""
     from magicdec_amd.ops import linear_f32_few_supported as takes
-    for M, N, K in ((1, 4096, 4096), (6, 2304, 8192), (9, 1024, 3072), (16, 64, 8192), (12, 128, 1536), (1, 1024, 256), (4, 16, 256), (6, 512, 512),
+    for M, N, K in ((1, 4096, 4096), (6, 2304, 8192), (9, 1024, 3072), (9, 2048, 3072), (16, 64, 8192), (12, 128, 1536), (1, 1024, 256), (4, 16, 256), (6, 512, 512),
                     (3, 65536, 256)):
         assert not takes(M, N, K), (M, N, K)
-    for M, N, K in ((6, 2048, 8192), (6, 2048, 2048), (16, 3072, 2048), (16, 1376, 2048), (8, 128, 1536), (4, 128, 256), (16, 3072, 768), (6, 32000, 2048)):
+    for M, N, K in ((6, 2048, 8192), (6, 2048, 2048), (16, 3072, 2048), (16, 1376, 2048), (16, 2048, 8192), (8, 128, 1536), (4, 128, 256), (16, 3072, 768), (6, 32000, 2048)):
         assert takes(M, N, K), (M, N, K)
 
 
