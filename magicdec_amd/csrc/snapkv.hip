@@ -85,25 +85,29 @@ __device__ __forceinline__ void load_kfrag(const SnapParams& p, int b, int kvh, 
     }
 }
 
-// The fragments of 32 consecutive columns (two 16-column groups).  Pages of a multiple of 32 rows hold all of them in one page, which is
+// The fragments of 32 or 64 consecutive columns (NC 16-column groups).  Pages of a multiple of 32 rows hold all of them in one page, which is
 // then looked up once per wavefront; rows past the context are not read from beyond it (zeros).
-template <int D, bool FP8>
-__device__ __forceinline__ void load_kfrag2(const SnapParams& p, int b, int kvh, int col0, bool whole, int lq, int lc,
-                                            bf16x8 (&kf)[2][D / 32]) {
-    if (!FP8 && whole && col0 + 32 <= p.S) {
-        const int page = col0 / p.page_size;
-        const int64_t pid = p.page_indices[p.page_indptr[b] + page];
-        const bf16_t* kp = reinterpret_cast<const bf16_t*>(p.cache) + pid * p.page_stride +
-                           (int64_t)(col0 - page * p.page_size) * p.slot_stride + (int64_t)kvh * p.head_stride;
-        const unsigned off = (unsigned)(lq * p.slot_stride + lc * 8);
+template <int D, bool FP8, int NC>
+__device__ __forceinline__ void load_kfrags(const SnapParams& p, int b, int kvh, int col0, bool whole, int lq, int lc,
+                                            bf16x8 (&kf)[NC][D / 32]) {
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+    for (int g = 0; g < NC; g += 2) {
+        const int at = col0 + g * 16;
+        if (!FP8 && whole && at + 32 <= p.S) {
+            const int page = at / p.page_size;
+            const int64_t pid = p.page_indices[p.page_indptr[b] + page];
+            const bf16_t* kp = reinterpret_cast<const bf16_t*>(p.cache) + pid * p.page_stride +
+                               (int64_t)(at - page * p.page_size) * p.slot_stride + (int64_t)kvh * p.head_stride;
+            const unsigned off = (unsigned)(lq * p.slot_stride + lc * 8);
 #pragma unroll
-            for (int ks = 0; ks < D / 32; ++ks)
-                kf[c][ks] = *reinterpret_cast<const bf16x8*>(kp + (int64_t)c * 16 * p.slot_stride + off + ks * 32);
-    } else {
-        load_kfrag<D, FP8>(p, b, kvh, col0, lq, lc, kf[0]);
-        load_kfrag<D, FP8>(p, b, kvh, col0 + 16, lq, lc, kf[1]);
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int ks = 0; ks < D / 32; ++ks)
+                    kf[g + c][ks] = *reinterpret_cast<const bf16x8*>(kp + (int64_t)c * 16 * p.slot_stride + off + ks * 32);
+        } else {
+            load_kfrag<D, FP8>(p, b, kvh, at, lq, lc, kf[g]);
+            load_kfrag<D, FP8>(p, b, kvh, at + 16, lq, lc, kf[g + 1]);
+        }
     }
 }
 
@@ -204,6 +208,12 @@ __device__ __forceinline__ unsigned int round_pair(float a, float b) {
     unsigned int pk;
     asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(pk) : "v"(a), "v"(b));
     return pk;
+}
+// both to bf16 and back (they may be one and the same)
+__device__ __forceinline__ void round2(float& a, float& b) {
+    const unsigned int pk = round_pair(a, b);
+    a = __uint_as_float(pk << 16);
+    if (&a != &b) b = __uint_as_float(pk & 0xffff0000u);
 }
 template <int BIN>
 __device__ __forceinline__ unsigned int tab_offsets2(unsigned int w, u16x2& top, unsigned int& low) {
@@ -351,10 +361,10 @@ __global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) 
     for (int rt = 0; rt < RTM; ++rt) zt[rt] = 0.0;
     const int ncg = (min(p.cols, p.S - chunk * p.cols) + 31) / 32;                   // 32-column groups of this chunk
     bf16x8 kf[2][D / 32], kn[2][D / 32];
-    if (wave < ncg) load_kfrag2<D, FP8>(p, b, kvh, chunk * p.cols + wave * 32, whole, lq, lc, kf);
+    if (wave < ncg) load_kfrags<D, FP8>(p, b, kvh, chunk * p.cols + wave * 32, whole, lq, lc, kf);
     for (int cg = wave; cg < ncg; cg += kSnapWaves) {
         const int col0 = chunk * p.cols + cg * 32;
-        if (cg + kSnapWaves < ncg) load_kfrag2<D, FP8>(p, b, kvh, col0 + kSnapWaves * 32, whole, lq, lc, kn);
+        if (cg + kSnapWaves < ncg) load_kfrags<D, FP8>(p, b, kvh, col0 + kSnapWaves * 32, whole, lq, lc, kn);
         const bool tail = col0 + 32 > p.S - p.W;                     // wave-uniform: only these columns can be masked
 #pragma unroll
         for (int r0 = 0; r0 < RTM; r0 += 2) {
@@ -463,15 +473,18 @@ __global__ __launch_bounds__(256) void snapkv_finalize_kernel(const SnapParams p
 // Rows <-> REGISTERS here (A = Q fragment, B = K fragment: lane (lq, lc) holds rows 16 rt + 4 lc + j of column lq), so an
 // 8-row group sum is three adds in a lane and one exchange between neighbouring groups of 16 lanes, in the reference's pairwise order.
 // Group G = 2 rt + half (lanes lc = 2 half) belongs to chunk G / g and pseudo head r' = G % g.  For even g a lane meets the same half
-// in every tile, so the accumulators r' = 2 i + half are its registers a[i] (template GH = g / 2, else 0: accumulators in LDS, updated
-// by the two halves in turn).  2 x 2 tiles at a time as in pass 1.  118 us where pass 1 takes 92: vector instructions for 69 % of the
-// cycles, LDS 61 %.  (147 with the accumulators in scratch memory, where an address of either column group had put them, halves of packed
-// bf16 converted one by one, and workgroups of eight wavefronts; the gathers of a batch in front of the next one's scores: spills, 177.)
+// in every tile, so the accumulators r' = 2 i + half are its registers a[x][i] (template GH = g / 2, else 0: accumulators in LDS, updated
+// by the two halves in turn).  After the exchange a lane keeps one of two column groups' sums, so that one rounding serves two sums.
+// NC column groups share a row tile's fragments and factors: four where a wavefront's 64 columns come out even (`four` below), the next
+// ones' keys then loaded behind the last row tile's products.  16 requests of 16 000 keys, as above: 109 us; 124 on the same card with two
+// row tiles of two column groups, both of whose sums every lane kept.  Bound by LDS as pass 1 is: random gathers are active for 62 % of the
+// cycles with all LDS work at 74 %, vector instructions at 67 %.  (A table of floats, and the float64 product only where rounding is in
+// doubt: 4 bytes at random cost what 8 do, 118 against 123; the scores a batch ahead of the gathers: 118 / 118.)
 // BIN: the table's binades; all, but where the accumulators of 30 and 32 queries a kv head of 128 beside them would pass a CU's LDS.
-template <int D, bool FP8, int GH, int RTM, int BIN = kTabBinades>
+template <int D, bool FP8, int GH, int RTM, int NC, int BIN = kTabBinades>
 __global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) void snapkv_accum_kernel(const SnapParams p) {
     constexpr int kSnapWaves = score_waves(D, RTM);
-    constexpr int BT = GH >= 2 ? 2 : 1;                        // row tiles per batch
+    constexpr int BT = GH >= 2 && NC == 2 ? 2 : 1, NG = NC / 2, COLS = NC * 16;      // row tiles per batch; column groups of a lane
     __shared__ __attribute__((aligned(16))) double tab[Tab<BIN>::N];
     // Q image, [L] exp(-M) / Z, [L][2] (M, 1 / Z), GH == 0: [waves][g][32] floats
     extern __shared__ __attribute__((aligned(16))) unsigned char dyn[];
@@ -506,47 +519,54 @@ __global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) 
     const int N = p.S - p.W;
     const bool whole = p.page_size % 32 == 0;
     const float kscale = FP8 ? p.k_scale[kvh] : 1.0f;
-    const int ncg = (min(p.cols, N - ctile * p.cols) + 31) / 32;                     // 32-column groups of this workgroup
-    bf16x8 kf[2][D / 32], kn[2][D / 32];
-    if (wave < ncg) load_kfrag2<D, FP8>(p, b, kvh, ctile * p.cols + wave * 32, whole, lq, lc, kf);
+    const int ncg = (min(p.cols, N - ctile * p.cols) + COLS - 1) / COLS;             // column groups of this workgroup
+    bf16x8 kf[NC][D / 32], kn[NC == 2 ? 2 : 1][D / 32];
+    if (wave < ncg) load_kfrags<D, FP8>(p, b, kvh, ctile * p.cols + wave * COLS, whole, lq, lc, kf);
     for (int cg = wave; cg < ncg; cg += kSnapWaves) {
-        const int col0 = ctile * p.cols + cg * 32;
-        if (cg + kSnapWaves < ncg) load_kfrag2<D, FP8>(p, b, kvh, col0 + kSnapWaves * 32, whole, lq, lc, kn);
-        const bool tail = col0 + 32 > p.S - p.W;               // wave-uniform: only these columns can be masked
-        float a[2][GH > 0 ? GH : 1];                           // [column group][i], bf16 values
+        const int col0 = ctile * p.cols + cg * COLS;
+        const bool more = cg + kSnapWaves < ncg;
+        if (NC == 2 && more) load_kfrags<D, FP8>(p, b, kvh, col0 + kSnapWaves * COLS, whole, lq, lc, kn);
+        const bool tail = col0 + COLS > p.S - p.W;             // wave-uniform: only these columns can be masked
+        float a[NG][GH > 0 ? GH : 1];                          // [column group 2 x + (lc & 1)][i], bf16 values
         if constexpr (GH > 0) {
 #pragma unroll
-            for (int i = 0; i < GH; ++i) a[0][i] = a[1][i] = 0.f;
+            for (int x = 0; x < NG; ++x)
+#pragma unroll
+                for (int i = 0; i < GH; ++i) a[x][i] = 0.f;
         } else {
             for (int i = lane; i < p.g * 32; i += 64) accs[i] = 0.f;
             __builtin_amdgcn_wave_barrier();
         }
-        // group sums of the BT row tiles from rt on, both column groups: lanes lc < 2 have group 2 rt, the others 2 rt + 1
-        auto sums = [&](int rt, float (&gs)[BT][2]) {
-            unsigned int w[BT][2][2];
+        // group sums of the BT row tiles from rt on: lanes lc < 2 have group 2 rt, the others 2 rt + 1, of column groups 2 x + (lc & 1)
+        auto sums = [&](int rt, float (&gs)[BT][NG]) {
+            unsigned int w[BT][NC][2];
 #pragma unroll
             for (int u = 0; u < BT; ++u) {
                 const unsigned char* qp = qimg + ((rt + u) * 16 + lq) * (D * 2 + kQPad) + lc * 16;
-                f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+                f32x4 acc[NC];
+#pragma unroll
+                for (int c = 0; c < NC; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int ks = 0; ks < D / 32; ++ks) {
                     const bf16x8 qf = *reinterpret_cast<const bf16x8*>(qp + ks * 64);
 #pragma unroll
-                    for (int c = 0; c < 2; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf, kf[c][ks], acc[c], 0, 0, 0);
+                    for (int c = 0; c < NC; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qf, kf[c][ks], acc[c], 0, 0, 0);
                 }
 #pragma unroll
-                for (int c = 0; c < 2; ++c) {
+                for (int c = 0; c < NC; ++c) {
                     if (FP8) acc[c] *= kscale;
                     w[u][c][0] = pack_bf16(acc[c][0], acc[c][1]);
                     w[u][c][1] = pack_bf16(acc[c][2], acc[c][3]);
                 }
             }
+            // the next columns' fragments in the place of these, while the last row tiles' gathers and sums go on
+            if (NC == 4 && more && rt + BT == p.L / 16) load_kfrags<D, FP8>(p, b, kvh, col0 + kSnapWaves * COLS, whole, lq, lc, kf);
             u16x2 top = {0, 0};
-            unsigned int low = 0, o[BT][2][2], pk[BT][2][2];
+            unsigned int low = 0, o[BT][NC][2], pk[BT][NC][2];
 #pragma unroll
             for (int u = 0; u < BT; ++u)
 #pragma unroll
-                for (int c = 0; c < 2; ++c)
+                for (int c = 0; c < NC; ++c)
 #pragma unroll
                     for (int h = 0; h < 2; ++h) o[u][c][h] = tab_offsets2<BIN>(w[u][c][h], top, low);
             if (fast_rows && !tail && __builtin_amdgcn_ballot_w64(tab_outside<BIN>(top, low)) == 0) {
@@ -556,7 +576,7 @@ __global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) 
                     const double* rc = rowc + (rt + u) * 16 + lc * 4;
                     const double c2[4] = {rc[0], rc[1], rc[2], rc[3]};
 #pragma unroll
-                    for (int c = 0; c < 2; ++c)
+                    for (int c = 0; c < NC; ++c)
 #pragma unroll
                         for (int h = 0; h < 2; ++h)
                             pk[u][c][h] = round_pair((float)(tab_at(tab, o[u][c][h] & 0xffffu) * c2[2 * h]),
@@ -566,7 +586,7 @@ __global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) 
 #pragma unroll
                 for (int u = 0; u < BT; ++u)
 #pragma unroll
-                    for (int c = 0; c < 2; ++c)
+                    for (int c = 0; c < NC; ++c)
 #pragma unroll
                         for (int h = 0; h < 2; ++h)
                             pk[u][c][h] = accum_slow<BIN>((lds_double*)tab, (lds_double*)rowc, (lds_double*)rowm, w[u][c][h], p.S, p.W, 8 * p.g, (rt + u) * 16 + lc * 4 + 2 * h,
@@ -574,57 +594,54 @@ __global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) 
             }
             // 8-row group sum in fp32, pairwise as a butterfly over consecutive rows, -> bf16 (:418)
 #pragma unroll
-            for (int u = 0; u < BT; ++u) {
-                float t[2];
+            for (int u = 0; u < BT; ++u)
 #pragma unroll
-                for (int c = 0; c < 2; ++c) {
-                    const unsigned int x = pk[u][c][0], y = pk[u][c][1];
-                    t[c] = (__uint_as_float(x << 16) + __uint_as_float(x & 0xffff0000u)) +
-                           (__uint_as_float(y << 16) + __uint_as_float(y & 0xffff0000u));
-                    // lanes 16 k <-> 16 (k ^ 1): both get the sum of the pair
-                    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(t[c]), __float_as_uint(t[c]), false, false);
-                    t[c] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+                for (int x = 0; x < NG; ++x) {
+                    float t[2];
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) {
+                        const unsigned int v = pk[u][2 * x + c][0], y = pk[u][2 * x + c][1];
+                        t[c] = (__uint_as_float(v << 16) + __uint_as_float(v & 0xffff0000u)) +
+                               (__uint_as_float(y << 16) + __uint_as_float(y & 0xffff0000u));
+                    }
+                    // the one column group's odd 16 lanes against the other's even ones: a lane then has both halves of one group's sum
+                    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(t[0]), __float_as_uint(t[1]), false, false);
+                    gs[u][x] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
                 }
-                const unsigned int g2 = round_pair(t[0], t[1]);
-                gs[u][0] = __uint_as_float(g2 << 16);
-                gs[u][1] = __uint_as_float(g2 & 0xffff0000u);
-            }
+            round2(gs[0][0], gs[BT - 1][NG - 1]);
         };
         if constexpr (GH > 0) {
             for (int rt = 0; rt < p.L / 16; rt += GH)          // one chunk of 8 g rows
                 unrolled(std::make_integer_sequence<int, GH / BT>(), [&](auto ic) {      // (accumulators in registers: not a loop)
                     constexpr int i = decltype(ic)::value * BT;
-                    float gs[BT][2];
+                    float gs[BT][NG];
                     sums(rt + i, gs);
-                    unrolled(std::make_integer_sequence<int, BT>(), [&](auto uc) {
-                        constexpr int u = decltype(uc)::value;
-                        const unsigned int n2 = round_pair(a[0][i + u] + gs[u][0], a[1][i + u] + gs[u][1]);
-                        a[0][i + u] = __uint_as_float(n2 << 16);
-                        a[1][i + u] = __uint_as_float(n2 & 0xffff0000u);
-                    });
-                });
-            // bf16 accumulators: aws[b][kvh*g + r'][col]; lane (lq, lc): half lc / 2, column group lc & 1
-            const int col = col0 + (lc & 1) * 16 + lq;
 #pragma unroll
-            for (int i = 0; i < GH; ++i) {
-                const float v0 = a[0][i], v1 = a[1][i], v = lc & 1 ? v1 : v0;      // (values: choosing between places puts both in scratch memory)
-                if (col < N)
-                    p.aws[((int64_t)b * p.H + kvh * p.g + 2 * i + (lc >> 1)) * N + col] = (unsigned short)(__float_as_uint(v) >> 16);
+                    for (int u = 0; u < BT; ++u)
+#pragma unroll
+                        for (int x = 0; x < NG; ++x) a[x][i + u] += gs[u][x];
+                    round2(a[0][i], a[NG - 1][i + BT - 1]);
+                });
+            // bf16 accumulators: aws[b][kvh*g + r'][col]; lane (lq, lc): half lc / 2
+#pragma unroll
+            for (int x = 0; x < NG; ++x) {
+                const int col = col0 + (2 * x + (lc & 1)) * 16 + lq;
+#pragma unroll
+                for (int i = 0; i < GH; ++i)
+                    if (col < N)
+                        p.aws[((int64_t)b * p.H + kvh * p.g + 2 * i + (lc >> 1)) * N + col] = (unsigned short)(__float_as_uint(a[x][i]) >> 16);
             }
         } else {
             int rp0 = 0;                                       // (2 rt) % g, kept by increments: no modulo per tile
             for (int rt = 0; rt < p.L / 16; ++rt) {
-                float gs[BT][2];
+                float gs[BT][NG];
                 sums(rt, gs);
                 // the two halves in group order (with g = 1 both land on the same accumulator)
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
-                    if (lc == 2 * half) {
-#pragma unroll
-                        for (int c = 0; c < 2; ++c) {
-                            float* x = accs + rp0 * 32 + c * 16 + lq;
-                            *x = bf16_to_f32(f32_to_bf16(*x + gs[0][c]));
-                        }
+                    if (lc >> 1 == half) {
+                        float* x = accs + rp0 * 32 + (lc & 1) * 16 + lq;
+                        *x = bf16_to_f32(f32_to_bf16(*x + gs[0][0]));
                     }
                     rp0 = rp0 + 1 == p.g ? 0 : rp0 + 1;
                     __builtin_amdgcn_wave_barrier();
@@ -639,10 +656,12 @@ __global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) 
             }
             __builtin_amdgcn_wave_barrier();
         }
+        if constexpr (NC == 2) {
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+            for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int ks = 0; ks < D / 32; ++ks) kf[c][ks] = kn[c][ks];
+                for (int ks = 0; ks < D / 32; ++ks) kf[c][ks] = kn[c][ks];
+        }
     }
 }
 
@@ -653,48 +672,66 @@ __device__ __forceinline__ unsigned int ordered16(unsigned short bits) {
 // Pooled + group-summed scores of 1024 columns of one (kv head, request), as bf16 bits: a thread owns four neighbouring columns, the
 // rows' columns (and half a pool width on either side) come through LDS.  All CUs take part; inside the selection's one workgroup per
 // (kv head, request) it was most of that kernel's 135 us.
+// Bound by latency: the columns of four rows are asked for together (each row behind the last one's barrier: 14 us for 16 MB, now 10.6).
 constexpr int kPoolCols = 1024, kPoolHalf = 64;         // widest half pool that is staged
+constexpr int kPoolRows = 4;                            // rows staged at a time
 
 template <int KS>                                       // the pool's width where it is known (taps in registers), else 0
 __global__ __launch_bounds__(256) void snapkv_pool_kernel(const unsigned short* __restrict__ aws, int H, int KH, int g, int N, int ksz_any,
                                                           unsigned short* __restrict__ score_out) {
-    __shared__ __attribute__((aligned(16))) float img[kPoolCols + 2 * kPoolHalf];
+    constexpr int kImg = kPoolCols + 2 * kPoolHalf, kLoads = (kPoolCols + 2 * (KS ? KS / 2 : kPoolHalf) + 255) / 256;
+    __shared__ __attribute__((aligned(16))) float img[kPoolRows][kImg];
     const int ksz = KS ? KS : ksz_any;
     const int c0 = blockIdx.x * kPoolCols, kvh = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, half = ksz / 2;
     const bool staged = half <= kPoolHalf;
+    const unsigned short* rows = aws + ((int64_t)b * H + kvh * g) * N;
     float tot[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int rp = 0; rp < g; ++rp) {
-        const unsigned short* row = aws + ((int64_t)b * H + kvh * g + rp) * N;
+    for (int r0 = 0; r0 < g; r0 += kPoolRows) {
         if (staged) {
-            for (int i = tid; i < kPoolCols + 2 * half; i += 256) {
-                const int c = c0 - half + i;
-                img[i] = c >= 0 && c < N ? bf16_bits_to_f32(row[c]) : 0.f;       // (adding 0 is what leaving a column out is)
-            }
+            unsigned short v[kPoolRows][kLoads];
+#pragma unroll
+            for (int r = 0; r < kPoolRows; ++r)
+#pragma unroll
+                for (int k = 0; k < kLoads; ++k) {
+                    v[r][k] = rows[(int64_t)min(r0 + r, g - 1) * N + min(max(c0 - half + tid + k * 256, 0), N - 1)];
+                }
+            if (r0) __syncthreads();
+#pragma unroll
+            for (int r = 0; r < kPoolRows; ++r)
+#pragma unroll
+                for (int k = 0; k < kLoads; ++k)
+                    if (tid + k * 256 < kPoolCols + 2 * half) {
+                        const int c = c0 - half + tid + k * 256;
+                        img[r][tid + k * 256] = c >= 0 && c < N ? bf16_bits_to_f32(v[r][k]) : 0.f;       // (adding 0 is what leaving a column out is)
+                    }
             __syncthreads();
         }
-        float tap[4 + (KS ? KS - 1 : 0)];
-        if constexpr (KS > 0) {
 #pragma unroll
-            for (int k = 0; k < 4 + KS - 1; ++k) tap[k] = img[tid * 4 + k];
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int s = tid * 4 + j;
-            float acc = 0.f;
+        for (int r = 0; r < kPoolRows; ++r) {
+            if (r0 + r >= g) break;
+            float tap[4 + (KS ? KS - 1 : 0)];
             if constexpr (KS > 0) {
 #pragma unroll
-                for (int k = 0; k < KS; ++k) acc += tap[j + k];
-            } else if (staged) {
-                for (int k = 0; k < ksz; ++k) acc += img[s + k];
-            } else {
-                for (int k = -half; k <= half; ++k) {
-                    const int c = c0 + s + k;
-                    if (c >= 0 && c < N) acc += bf16_bits_to_f32(row[c]);
-                }
+                for (int k = 0; k < 4 + KS - 1; ++k) tap[k] = img[r][tid * 4 + k];
             }
-            tot[j] += bf16_to_f32(f32_to_bf16(acc / (float)ksz));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int s = tid * 4 + j;
+                float acc = 0.f;
+                if constexpr (KS > 0) {
+#pragma unroll
+                    for (int k = 0; k < KS; ++k) acc += tap[j + k];
+                } else if (staged) {
+                    for (int k = 0; k < ksz; ++k) acc += img[r][s + k];
+                } else {
+                    for (int k = -half; k <= half; ++k) {
+                        const int c = c0 + s + k;
+                        if (c >= 0 && c < N) acc += bf16_bits_to_f32(rows[(int64_t)(r0 + r) * N + c]);
+                    }
+                }
+                tot[j] += bf16_to_f32(f32_to_bf16(acc / (float)ksz));
+            }
         }
-        if (staged) __syncthreads();
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -1011,6 +1048,8 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
     const size_t lds2 = qimg_b + (size_t)L * 3 * 8 + (gh ? 0 : (size_t)waves * g * 32 * 4);
     const dim3 sg(p.nch, KH, B), ag((N + p.cols - 1) / p.cols, KH, B);
     const bool small = L <= 128;
+    const int rounds = p.cols / (32 * waves);                  // (wavefronts of 64 columns: half of the rounds, one too many of few odd ones)
+    const bool four = rounds % 2 == 0 || rounds > 6;
     // (30 and 32 queries a kv head of 128: 171 648 and 174 080 bytes with the whole table, of 163 840)
     const bool tight = lds2 > (size_t)beside_table<kTabBinades>();
     MD_CHECK_ARG(lds1 <= (size_t)(D == 128 && !small ? beside_table<kTabSmall>() : beside_table<kTabBinades>()) &&
@@ -1021,8 +1060,9 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
     rc = small ? score_launch<&snapkv_stats_kernel<DD, FP, 8>, stats_binades(DD, 8)>(sg, waves, lds1, p, st)                 \
                : score_launch<&snapkv_stats_kernel<DD, FP, kMaxRT>, stats_binades(DD, kMaxRT)>(sg, waves, lds1, p, st)
 #define MD_SNAP_ACCUM(DD, FP, GG)                                                                                            \
-    rc = small ? score_launch<&snapkv_accum_kernel<DD, FP, GG, 8>, kTabBinades>(ag, waves, lds2, p, st)                      \
-               : score_launch<&snapkv_accum_kernel<DD, FP, GG, kMaxRT>, kTabBinades>(ag, waves, lds2, p, st)
+    rc = !small          ? score_launch<&snapkv_accum_kernel<DD, FP, GG, kMaxRT, 2>, kTabBinades>(ag, waves, lds2, p, st)    \
+         : four && GG > 0 ? score_launch<&snapkv_accum_kernel<DD, FP, GG, 8, GG ? 4 : 2>, kTabBinades>(ag, waves, lds2, p, st) \
+                         : score_launch<&snapkv_accum_kernel<DD, FP, GG, 8, 2>, kTabBinades>(ag, waves, lds2, p, st)
 #define MD_SNAP_LAUNCH(DD, FP)                                                                                               \
     do {                                                                                                                     \
         MD_SNAP_STATS(DD, FP);                                                                                               \
@@ -1033,7 +1073,7 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
         else if (gh == 2) MD_SNAP_ACCUM(DD, FP, 2);                                                                          \
         else if (gh == 1) MD_SNAP_ACCUM(DD, FP, 1);                                                                          \
         else if constexpr (DD == 128) {                                                                                      \
-            if (tight) rc = score_launch<&snapkv_accum_kernel<DD, FP, 0, kMaxRT, kTabSmall>, kTabSmall>(ag, waves, lds2, p, st); \
+            if (tight) rc = score_launch<&snapkv_accum_kernel<DD, FP, 0, kMaxRT, 2, kTabSmall>, kTabSmall>(ag, waves, lds2, p, st); \
             else MD_SNAP_ACCUM(DD, FP, 0);                                                                                   \
         } else MD_SNAP_ACCUM(DD, FP, 0);                                                                                     \
         if (rc != MD_OK) return rc;                                                                                          \

@@ -30,6 +30,13 @@ def test_select_with_one_workgroup_per_cu(monkeypatch, B, KH, g, W, D, S):
     check_select(monkeypatch, B, KH, g, W, D, S, 129, 5, 128, (0, B - 1))
 
 
+@pytest.mark.parametrize("g,W,D", [(2, 16, 64), (4, 32, 64), (8, 16, 64), (2, 16, 128), (4, 32, 128), (8, 16, 128)])
+@pytest.mark.parametrize("S", [1000, 897 + 64, 1024])
+def test_select_in_groups_of_64_columns(monkeypatch, g, W, D, S):
+    """256 pairs, an even number of rounds of columns: wavefronts of four column groups, the last of them partly or wholly behind the context."""
+    check_select(monkeypatch, 64, 4, g, W, D, S, 129, 5, 128, (0, 63))
+
+
 # accumulators, query image and table of exponentials in one CU's LDS: the most queries a kv head (with the whole table 160 to 170 KB of 160)
 @pytest.mark.parametrize("g,W,D", [(32, 8, 128), (30, 8, 128), (28, 8, 128), (16, 16, 128), (32, 8, 64)])
 @pytest.mark.parametrize("KH,S", [(1, 1060), (3, 150)])
