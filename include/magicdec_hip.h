@@ -653,10 +653,14 @@ int md_accept_rollback(int64_t* tokens_buffer, const int64_t* target_tokens, int
  *   MD_STEP_ADD   int32 dst += a                            (src unused)
  *   MD_STEP_SCALE int32 dst = src * a                       (src dense)
  *   MD_STEP_COPY  int64 dst[r][c] = src[r * src_stride + c]
+ *   MD_STEP_FILL  int32 dst[i] = a
+ *   MD_STEP_GRID  int32 dst[r][c] = r * a + c
  * ---------------------------------------------------------------------- */
 #define MD_STEP_ADD 0
 #define MD_STEP_SCALE 1
 #define MD_STEP_COPY 2
+#define MD_STEP_FILL 3
+#define MD_STEP_GRID 4
 #define MD_STEP_MAX_OPS 8
 typedef struct {
     void* dst;

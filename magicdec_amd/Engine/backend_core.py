@@ -105,6 +105,47 @@ class SequencePool:
         self.free_pages.extend(reversed(pages))
 
 
+class _Integers:
+    """int32 tensors to be written, all in one launch where the device and the tensors allow that: page tables and lengths of a few hundred
+    bytes, for which as many launches are 4.5 us each between the portions of a prompt.  No piece reads what another one writes."""
+
+    def __init__(self):
+        self._pieces = []
+
+    def _add(self, t, on_gpu, otherwise):
+        if t.numel():
+            self._pieces.append((t, on_gpu, otherwise))
+
+    def fill(self, t, a):
+        self._add(t, dict(fill=[(t, a)]), lambda: t.fill_(a))
+
+    def grid(self, t, rows, a):
+        """t as `rows` rows: t[r][c] = r * a + c."""
+        def torch_does():
+            r, c = (torch.arange(n, dtype=t.dtype, device=t.device) for n in (rows, t.numel() // rows))
+            t.copy_((r.view(-1, 1) * a + c).view(t.shape))
+        self._add(t, dict(grid=[(t, rows, a)]), torch_does)
+
+    def scale(self, dst, src, a):
+        self._add(dst, dict(scale=[(dst, src, a)]) if ops.step_adds(src, dst) else None, lambda: dst.copy_(src * a))
+
+    def run(self):
+        now = {}, []                                   # kinds of pieces, of one launch
+        for t, on_gpu, otherwise in self._pieces:
+            if on_gpu is None or not ops.step_adds(t, (now[1] or [t])[0]):
+                otherwise()
+                continue
+            if len(now[1]) == ops.STEP_MAX:
+                ops.StepOps(**now[0]).run()
+                now = {}, []
+            for kind, args in on_gpu.items():
+                now[0].setdefault(kind, []).extend(args)
+            now[1].append(t)
+        if now[1]:
+            ops.StepOps(**now[0]).run()
+        self._pieces = []
+
+
 class _PagedState:
     """One paged cache's bookkeeping under a name prefix ('' or 'draft_') on the owning back-end."""
 
@@ -118,32 +159,43 @@ class _PagedState:
     def _set(self, name, val):
         setattr(self.o, self.p + name, val)
 
-    def reset(self, last_page_len_init=0, full_table=False, indptr_stride=1):
+    def reset(self, last_page_len_init=0, full_table=False, indptr_stride=1, ints=None):
+        """ints: where the caller has more integers to write (and runs them)."""
         o, B, dev = self.o, self.o.batch_size, self.o.device
-        ppr = self.ppr
-        self._set("num_pages_per_request", torch.zeros(B, dtype=torch.int32, device=dev))
+        ppr, w = self.ppr, ints or _Integers()
+
+        def new(name, n):
+            self._set(name, torch.empty(n, dtype=torch.int32, device=dev))
+            return self._get(name)
+        w.fill(new("num_pages_per_request", B), 0)
         self.host_pages = 0
         if full_table or self.mapped:   # SnapKV draft cache: all pages mapped from the start (backend.py:87-90)
-            self._set("paged_kv_indptr", torch.arange(B + 1, dtype=torch.int32, device=dev) * ppr)
-            self._set("paged_kv_indices", torch.arange(B * ppr, dtype=torch.int32, device=dev))
+            w.grid(new("paged_kv_indptr", B + 1), B + 1, ppr)
+            w.grid(new("paged_kv_indices", B * ppr), 1, 0)
             self.host_pages = ppr
         else:
-            self._set("paged_kv_indptr", torch.arange(B + 1, dtype=torch.int32, device=dev) * indptr_stride)
-            self._set("paged_kv_indices", torch.zeros(B * ppr, dtype=torch.int32, device=dev))
-        self._set("paged_kv_last_page_len", torch.full((B,), last_page_len_init, dtype=torch.int32, device=dev))
+            w.grid(new("paged_kv_indptr", B + 1), B + 1, indptr_stride)
+            w.fill(new("paged_kv_indices", B * ppr), 0)
+        w.fill(new("paged_kv_last_page_len", B), last_page_len_init)
+        if ints is None:
+            w.run()
 
-    def map_pages(self, n_pages, last_page_len):
+    def map_pages(self, n_pages, last_page_len, ints=None):
         """Request b maps pages b*ppr .. b*ppr+n_pages-1; last page holds `last_page_len` rows
-        (pre_encode, Engine/SnapKV/backend.py:270-275)."""
+        (pre_encode, Engine/SnapKV/backend.py:270-275).  ints: as in reset."""
         if self.mapped:
             return
         o, B, dev = self.o, self.o.batch_size, self.o.device
+        w = ints or _Integers()
         self.host_pages = n_pages
-        self._get("num_pages_per_request").fill_(n_pages)
-        base = torch.arange(B, dtype=torch.int32, device=dev).view(-1, 1) * self.ppr
-        self._set("paged_kv_indices", (base + torch.arange(n_pages, dtype=torch.int32, device=dev).view(1, -1)).flatten())
-        self._get("paged_kv_indptr").copy_(torch.arange(B + 1, dtype=torch.int32, device=dev) * n_pages)
-        self._set("paged_kv_last_page_len", torch.full((B,), last_page_len, dtype=torch.int32, device=dev))
+        w.fill(self._get("num_pages_per_request"), n_pages)
+        self._set("paged_kv_indices", torch.empty(B * n_pages, dtype=torch.int32, device=dev))
+        w.grid(self._get("paged_kv_indices"), B, self.ppr)
+        w.grid(self._get("paged_kv_indptr"), B + 1, n_pages)
+        self._set("paged_kv_last_page_len", torch.empty(B, dtype=torch.int32, device=dev))
+        w.fill(self._get("paged_kv_last_page_len"), last_page_len)
+        if ints is None:
+            w.run()
 
     def table(self, lengths=None):
         """lengths: (new rows, positions after the step), the same for every request of the batch."""
@@ -265,9 +317,22 @@ class _BackendBase:
             at = end
         return out + [(at, seq_len - at)] if at < seq_len else out
 
-    def _map_portion(self, end):
-        """Pages for a prompt's first `end` tokens."""
-        self._t.map_pages(-(-end // PAGE_SIZE), (end - 1) % PAGE_SIZE + 1)
+    def _portion(self, end, n):
+        """Pages for a prompt's first `end` tokens, n of them new: their qo_indptr."""
+        ints, qo = _Integers(), torch.empty_like(self.qo_indptr)
+        self._t.map_pages(-(-end // PAGE_SIZE), (end - 1) % PAGE_SIZE + 1, ints)
+        ints.scale(qo, self.qo_indptr, n)
+        ints.run()
+        return qo
+
+    def _clear_lengths(self, *lens):
+        """Length tensors to zero, the plain qo_indptr: the integers of a clear_kv, beside those of its page tables (and not run yet)."""
+        ints = _Integers()
+        for name in lens:
+            ints.fill(getattr(self, name), 0)
+        self.qo_indptr = torch.empty(self.batch_size + 1, dtype=torch.int32, device=self.device)
+        ints.grid(self.qo_indptr, self.batch_size + 1, 1)
+        return ints
 
     def _last_rows(self, n, seq_len):
         """Extra prefill arguments: of models addressed by position, logits for the last of every request's n rows only (their portions
@@ -275,7 +340,7 @@ class _BackendBase:
         if not self.mapped:
             tail = (seq_len - 1) % CHUNK + 1
             return dict(tail=tail) if n > tail else {}
-        return dict(head_rows=torch.arange(1, self.batch_size + 1, device=self.device) * n - 1)
+        return dict(head_rows=torch.arange(n - 1, self.batch_size * n, n, device=self.device))
 
     @contextlib.contextmanager
     def _prefilling(self):
@@ -375,12 +440,11 @@ class SnapKVTargetBackend(_BackendBase):
         for b in self.model.layers:
             b.attention.kv_cache.clear()
         self._reset_kv_calibration()
-        self.cachelens.zero_()
-        self.qo_indptr = torch.arange(self.batch_size + 1, dtype=torch.int32, device=self.device)
-        self._t.reset()
+        ints = self._clear_lengths("cachelens", *(["draft_cachelens"] if self.is_spec else []))
+        self._t.reset(ints=ints)
         if self.is_spec:
-            self.draft_cachelens.zero_()
-            self._d.reset(last_page_len_init=1, full_table=True)
+            self._d.reset(last_page_len_init=1, full_table=True, ints=ints)
+        ints.run()
 
     @torch.no_grad()
     def encode(self, input_ids: torch.LongTensor, benchmark=False):
@@ -395,9 +459,9 @@ class SnapKVTargetBackend(_BackendBase):
             for done, n in self._portions(seq_len):
                 ids = input_ids[:, done:done + n]
                 is_last = done + n == seq_len and n % self.prefill_chunk != 0
-                self._map_portion(done + n)                   # pre_encode
+                qo = self._portion(done + n, n)               # pre_encode
                 self.model.skip_head = done + n != seq_len
-                tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table((n, done + n)), is_last=is_last,
+                tokens = self.model.prefill(ids, self.cachelens, qo, self._t.table((n, done + n)), is_last=is_last,
                                             draft_tab=self._d.table() if (self.is_spec and is_last) else None,
                                             ctx_len=done + n, **self._last_rows(n, seq_len))
                 self.cachelens += n
@@ -557,11 +621,11 @@ class SnapKVDraftBackend(_BackendBase):
         for b in self.model.layers:
             b.attention.kv_cache.clear()
         self._reset_kv_calibration()
-        self.cachelens.zero_()
-        self.qo_indptr = torch.arange(self.batch_size + 1, dtype=torch.int32, device=self.device)
-        self._t.reset()
+        ints = self._clear_lengths("cachelens")
+        self._t.reset(ints=ints)
         if self.is_compress:
-            self._d.reset(last_page_len_init=1, full_table=True)
+            self._d.reset(last_page_len_init=1, full_table=True, ints=ints)
+        ints.run()
 
     @torch.no_grad()
     def encode(self, input_ids: torch.LongTensor, benchmark=False):
@@ -574,9 +638,9 @@ class SnapKVDraftBackend(_BackendBase):
             for done, n in self._portions(seq_len):
                 ids = input_ids[:, done:done + n]
                 is_last = done + n == seq_len and n % self.prefill_chunk != 0
-                self._map_portion(done + n)                   # pre_encode
+                qo = self._portion(done + n, n)               # pre_encode
                 self.model.skip_head = done + n != seq_len
-                tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table((n, done + n)), is_last=is_last,
+                tokens = self.model.prefill(ids, self.cachelens, qo, self._t.table((n, done + n)), is_last=is_last,
                                             draft_tab=self._d.table() if (self.is_compress and is_last) else None,
                                             ctx_len=done + n, **self._last_rows(n, seq_len))
                 self.cachelens += n
@@ -651,9 +715,10 @@ class _StreamingMixin:
                 else:
                     tokens = self.model.stream_prefill(ids, start, self._qo(n), state.table(), is_last, which, B)
                 lens = getattr(self, lens_attr)
-                lens += ids.shape[1]
                 if ctx >= self.draft_budget:
                     lens.fill_(self.draft_budget)
+                else:
+                    lens += ids.shape[1]
         return tokens
 
 
@@ -684,9 +749,9 @@ class StreamingDraftBackend(_BackendBase, _StreamingMixin):
         for b in self.model.layers:
             b.attention.kv_cache.clear()
         self._reset_kv_calibration()
-        self.cachelens.zero_()
-        self.qo_indptr = torch.arange(self.batch_size + 1, dtype=torch.int32, device=self.device)
-        self._t.reset()
+        ints = self._clear_lengths("cachelens")
+        self._t.reset(ints=ints)
+        ints.run()
 
     @torch.no_grad()
     def encode(self, input_ids: torch.LongTensor, benchmark=False):
@@ -745,11 +810,10 @@ class StreamingSelfSpecBackend(_BackendBase, _StreamingMixin):
         for b in self.model.layers:
             b.attention.kv_cache.clear()
         self._reset_kv_calibration()
-        self.cachelens.zero_()
-        self.draft_cachelens.zero_()
-        self.qo_indptr = torch.arange(self.batch_size + 1, dtype=torch.int32, device=self.device)
-        self._t.reset()
-        self._d.reset(indptr_stride=self.draft_max_num_pages_per_request)   # StreamingLLM/backend.py:316
+        ints = self._clear_lengths("cachelens", "draft_cachelens")
+        self._t.reset(ints=ints)
+        self._d.reset(indptr_stride=self.draft_max_num_pages_per_request, ints=ints)   # StreamingLLM/backend.py:316
+        ints.run()
 
     @torch.no_grad()
     def encode(self, input_ids: torch.LongTensor, benchmark=False):
@@ -760,9 +824,9 @@ class StreamingSelfSpecBackend(_BackendBase, _StreamingMixin):
         with self._prefilling():
             for done, n in self._portions(seq_len):
                 ids = input_ids[:, done:done + n]
-                self._map_portion(done + n)
+                qo = self._portion(done + n, n)
                 self.model.skip_head = done + n != seq_len
-                tokens = self.model.prefill(ids, self.cachelens, self._qo(n), self._t.table(), **self._last_rows(n, seq_len))
+                tokens = self.model.prefill(ids, self.cachelens, qo, self._t.table(), **self._last_rows(n, seq_len))
                 self.cachelens += n
         return tokens
 

@@ -910,7 +910,7 @@ class Transformer(nn.Module):
             tab = replace(tab, max_pages=min(tab.max_pages, -(-ctx_len // page)))
         rows = None
         if tail is not None and not self.skip_head:
-            rows = (torch.arange(B, device=idx.device).view(B, 1) * n + torch.arange(n - tail, n, device=idx.device)).flatten()
+            rows = torch.arange(B * n, device=idx.device).view(B, n)[:, n - tail:].flatten()
         out = self._std_step(idx, input_pos, kv_append_indptr, tab, snap_tab=snap, calibrate=True, n_max=n, head_rows=rows)
         return out if out is None or tail is None else out.view(B, tail)
 
@@ -979,6 +979,6 @@ class Transformer(nn.Module):
             ops.streaming_windows(k, v, cache, windows, following, portion, ctx, kv_len, SINK, ppr, self.rope_table, rotated)
             cache.copy_(following)
             return self._attend(q_rot, windows, qo, tab, portion)
-        rows = (torch.arange(B, device=dev).view(B, 1) * tokens + torch.arange(starts[-1], tokens, device=dev)).flatten()
+        rows = None if self.skip_head else torch.arange(B * tokens, device=dev).view(B, tokens)[:, starts[-1]:].flatten()
         out = self._run(idx, fn, head_rows=rows)
         return None if out is None else out.view(B, -1)

@@ -1474,16 +1474,17 @@ def accept_rollback(tokens_buffer, target_tokens, output, num_nodes, cachelens, 
                                  _stream()), "md_accept_rollback")
 
 
-STEP_ADD, STEP_SCALE, STEP_COPY, STEP_MAX = 0, 1, 2, 8
+STEP_ADD, STEP_SCALE, STEP_COPY, STEP_FILL, STEP_GRID, STEP_MAX = 0, 1, 2, 3, 4, 8
 
 
 class StepOps:
     """The integer work around a decode step in one launch: add = [(int32 tensor, a)]: t += a; scale = [(dst, src, a)]: dst = src * a
-    (int32); copies = [dst]: int64 tensors that `run` fills, from sources of unit row stride.  All on one device: a kernel reads its
+    (int32); copies = [dst]: int64 tensors that `run` fills, from sources of unit row stride; fill = [(int32 tensor, a)]: t = a; grid = [(int32
+    tensor, rows, a)]: t[r][c] = r * a + c of the tensor as that many rows.  All on one device: a kernel reads its
     pieces' memory directly.  What does not change from call to call is
     set up once (a launch then costs the host one foreign call); the tensors are kept alive."""
 
-    def __init__(self, add=(), scale=(), copies=()):
+    def __init__(self, add=(), scale=(), copies=(), fill=(), grid=()):
         self._ops, self._n, self._kept = (_lib.StepOp * STEP_MAX)(), 0, []
         for t, a in add:
             self._put(STEP_ADD, _i32(t), None, int(a))
@@ -1491,19 +1492,25 @@ class StepOps:
             if dst.shape != src.shape or not src.is_contiguous():
                 raise ValueError("step_ops: scale needs dense tensors of one shape")
             self._put(STEP_SCALE, _i32(dst), _i32(src), int(a))
+        for t, a in fill:
+            self._put(STEP_FILL, _i32(t), None, int(a))
+        for t, rows, a in grid:
+            if rows <= 0 or t.numel() % rows:
+                raise ValueError("step_ops: a grid of whole rows")
+            self._put(STEP_GRID, _i32(t), None, int(a), rows)
         self._copies, self._first = list(copies), self._n
         for dst in self._copies:
             if dst.dtype != torch.int64:
                 raise ValueError("step_ops: copies are int64")
             self._put(STEP_COPY, dst, None, 0)
 
-    def _put(self, kind, dst, src, a):
+    def _put(self, kind, dst, src, a, rows=1):
         _gpu(dst, src)
         if self._n == STEP_MAX or not dst.is_contiguous():
             raise ValueError(f"step_ops: at most {STEP_MAX} pieces, into dense tensors")
         if any(t is not None and t.device != dst.device for t in [src] + self._kept):
             raise ValueError("step_ops: every piece lies on one device")
-        self._ops[self._n] = _lib.StepOp(dst.data_ptr(), src.data_ptr() if src is not None else None, 0, 1, dst.numel(), kind, a)
+        self._ops[self._n] = _lib.StepOp(dst.data_ptr(), src.data_ptr() if src is not None else None, 0, rows, dst.numel() // rows, kind, a)
         self._kept += [dst, src]
         self._n += 1
 

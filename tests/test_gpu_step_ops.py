@@ -22,6 +22,27 @@ def test_pieces(n):
     assert torch.equal(out.cpu(), wide[:, 3:4]) and torch.equal(pair.cpu(), wide[:, 1:3]) and torch.equal(dense.cpu(), wide)
 
 
+@pytest.mark.parametrize("rows,cols", [(1, 1), (2, 255), (64, 126), (257, 1), (1, 300)])
+def test_fills_and_grids(rows, cols):
+    """Constants and page tables: every piece of a launch of eight, and what another launch takes."""
+    from magicdec_amd import ops
+    from magicdec_amd.Engine.backend_core import _Integers
+    ints, want = _Integers(), []
+    for k in range(5):
+        t, u = (torch.full((rows * cols + 2,), -1, dtype=torch.int32, device=DEV)[1:-1] for _ in range(2))      # (views: nothing beside them)
+        ints.fill(t, 7 - k)
+        ints.grid(u, rows, cols + k)
+        want += [(t, torch.full((rows, cols), 7 - k)), (u, torch.arange(rows).view(-1, 1) * (cols + k) + torch.arange(cols))]
+    strided, src = torch.zeros(rows, 2, dtype=torch.int32, device=DEV)[:, 0], torch.arange(rows, dtype=torch.int32, device=DEV)
+    ints.scale(strided, src, 3)                              # (not dense: torch writes it)
+    ints.run()
+    for t, w in want + [(strided, src.cpu() * 3)]:
+        assert torch.equal(t.cpu(), w.int().view(t.shape))
+    assert all(t._base[0].item() == -1 and t._base[-1].item() == -1 for t, _ in want)
+    with pytest.raises(ValueError):
+        ops.StepOps(grid=[(torch.zeros(5, dtype=torch.int32, device=DEV), 2, 1)])
+
+
 def test_what_it_does_not_take():
     from magicdec_amd import ops
     t = torch.zeros(8, 2, dtype=torch.int64, device=DEV)
