@@ -532,8 +532,12 @@ extern "C" int md_argmax_f32(const float* logits, int64_t row_stride, int rows, 
                              md_stream_t stream) {
     MD_CHECK_ARG(logits && idx_out, "md_argmax_f32: null pointer argument");
     MD_CHECK_ARG(rows > 0 && vocab > 0, "md_argmax_f32: bad shape rows=%d vocab=%d", rows, vocab);
-    hipLaunchKernelGGL((argmax_kernel<256, float>), dim3(rows), dim3(256), 0, (hipStream_t)stream, logits, row_stride, vocab,
-                       (int64_t)0, (bf16_t*)nullptr, idx_out, 0, 0);
+    if (rows <= 512 && vocab >= 16384)
+        hipLaunchKernelGGL((argmax_kernel<1024, float>), dim3(rows), dim3(1024), 0, (hipStream_t)stream, logits, row_stride, vocab,
+                           (int64_t)0, (bf16_t*)nullptr, idx_out, 0, 0);
+    else
+        hipLaunchKernelGGL((argmax_kernel<256, float>), dim3(rows), dim3(256), 0, (hipStream_t)stream, logits, row_stride, vocab,
+                           (int64_t)0, (bf16_t*)nullptr, idx_out, 0, 0);
     MD_CHECK_LAUNCH("md_argmax_f32");
     return MD_OK;
 }

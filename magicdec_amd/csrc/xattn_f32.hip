@@ -15,10 +15,12 @@
 //
 // Bound by the fp32 matrix rate (154 TFLOP/s in a large library product) for prompts, by latency for decode steps.  Six sequences of
 // 100 to 1 500 tokens, 32 query and 8 kv heads of 64, one layer (22 GFLOP): 9 930 -> 445 -> 277 us; one token each behind them:
-// 292 -> 16.5 + 5.9 us for the merge (first figure: the plain kernel, one workgroup per row and head).
+// 292 -> 17.4 + 5.8 us for the merge -> 15.0 + 5.3 with splits of three tiles, all with keys, and their loads together in the merge (first
+// figure: the plain kernel, one workgroup per row and head).
 #include "xattn.h"
 
 #include <algorithm>
+#include <cstdlib>
 
 namespace {
 
@@ -625,15 +627,35 @@ __global__ __launch_bounds__(256) void xattn_f32_merge_kernel(const XattnParams 
     const int b = pair / p.KH, kvh = pair % p.KH, q0 = p.qo_indptr[b], row = qg * L.R + r;
     if (row >= (p.qo_indptr[b + 1] - q0) * p.g) return;
     const float* ml = p.ws + (int64_t)p.B * p.KH * L.nq * L.nsplit * L.R * L.dvw;
+    // (eight splits' loads together: they are all there is to wait for)
+    constexpr int U = 8;
+    const int64_t first = item * L.nsplit * L.R + r;
     float M = p.sink ? 0.f : -1e30f;
-    for (int s = 0; s < L.nsplit; ++s) M = fmaxf(M, ml[((item * L.nsplit + s) * L.R + r) * 2]);
+    for (int s0 = 0; s0 < L.nsplit; s0 += U) {
+        float m[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) m[u] = ml[(first + (int64_t)min(s0 + u, L.nsplit - 1) * L.R) * 2];
+#pragma unroll
+        for (int u = 0; u < U; ++u) M = fmaxf(M, m[u]);
+    }
     float Z = p.sink ? __builtin_amdgcn_exp2f(-M) : 0.f;
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < L.nsplit; ++s) {
-        const int64_t at = (item * L.nsplit + s) * L.R + r;
-        const float f = __builtin_amdgcn_exp2f(ml[at * 2] - M);
-        Z += ml[at * 2 + 1] * f;
-        o += *reinterpret_cast<const f32x4*>(p.ws + at * L.dvw + d) * f;
+    for (int s0 = 0; s0 < L.nsplit; s0 += U) {
+        f32x2 x[U];
+        f32x4 y[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t at = first + (int64_t)min(s0 + u, L.nsplit - 1) * L.R;
+            x[u] = *reinterpret_cast<const f32x2*>(ml + at * 2);
+            y[u] = *reinterpret_cast<const f32x4*>(p.ws + at * L.dvw + d);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (s0 + u >= L.nsplit) break;
+            const float f = __builtin_amdgcn_exp2f(x[u][0] - M);
+            Z += x[u][1] * f;
+            o += y[u] * f;
+        }
     }
     const float inv = Z > 0.f ? 1.0f / Z : Z != Z ? Z : 0.f;
     T* out = reinterpret_cast<T*>(p.out) + ((int64_t)(q0 + row / p.g) * p.H + kvh * p.g + row % p.g) * p.DV + d;
@@ -654,7 +676,7 @@ Shape shape_of(const XattnParams& p) {
 
 F32Launch plan(const XattnParams& p, Shape s, long keys) {
     static const int wide[] = {0, 4, 4, 2, 2, 2}, dvw[] = {0, 64, 128, 256, 256, 512}, kt[] = {0, 64, 32, 32, 32, 32};
-    const int64_t rows = (int64_t)p.n_max * p.g, items = (int64_t)p.KH * p.B, most = keys / (4 * kt[s]);
+    const int64_t rows = (int64_t)p.n_max * p.g, items = (int64_t)p.KH * p.B, tiles = (keys + kt[s] - 1) / kt[s];
     F32Launch L;
     L.dvw = dvw[s];
     auto with_rows = [&](int R) {
@@ -662,8 +684,23 @@ F32Launch plan(const XattnParams& p, Shape s, long keys) {
         L.nq = (int)((rows + R - 1) / R);
         // two workgroups per CU; a split has at least four tiles, so that its first loads and its share of the merge are a small part
         const int64_t groups = L.nq * items, want = groups > 0 ? (512 + groups - 1) / groups : 1;
-        L.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>({want, most, 64}));
+        L.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>({want, keys / (4 * kt[s]), 64}));
         return groups * L.nsplit;
+    };
+    // Sixteen rows a workgroup: a tile is 1.5 to 2 us of a step, one more split to merge 0.2, so splits go down to two tiles, none without
+    // a tile, and a sequence of four tiles stays whole (130 keys 13.9 us whole, 14.8 in two).  us, at least four tiles a split / now, 8 kv
+    // heads of 64: one request of 600 keys 22.8 / 15.5, of 2 000 25.0 / 20.5, 6 of 300 20.3 / 16.5, of 1 500 29.2 / 25.3, 12 of 600 25.9 /
+    // 21.5, 16 of 2 000 51.6 / 50.9.  Heads above 128, one workgroup a CU: 5 x 8 kv heads of 256, 600 keys 33.8 / 33.0, 6 of 8, 790
+    // 56.9 / 40.2, but unequal sequences of more than 32 pairs level out with more splits than one round of CUs (7 x 8, to 1 587 keys 65.5 /
+    // 73.8, 11 x 8 95.5 / 137): as above.
+    auto few_rows = [&]() {
+        with_rows(16);
+        const int64_t groups = L.nq * items;
+        const bool two = s == k64 || s == k128;
+        if (groups <= 0 || (!two && groups > 32)) return;
+        const int64_t want = two ? (512 + groups - 1) / groups : 256 / groups;
+        const int64_t n = std::max<int64_t>(1, std::min<int64_t>({want, tiles < 5 ? 1 : tiles / 2, 64})), per = (tiles + n - 1) / n;
+        L.nsplit = per > 0 ? (int)((tiles + per - 1) / per) : 1;
     };
     // Wide row groups reuse a tile's keys, 16 rows are the shorter chain: ahead by a fifth to a third while the wide ones are not half as
     // many workgroups as there are CUs (32 query heads of 64, 20 rows over 20 keys: 16.2 -> 11.6 us with the keys of a tile that are not
@@ -672,7 +709,7 @@ F32Launch plan(const XattnParams& p, Shape s, long keys) {
     // ahead where those tiles would be more than one a CU: 17 requests of 20 rows, heads of 256 (136) 53.4 and 34.9 us, of 32 rows 56.1 and
     // 38.7, but 16 of 32 (128) 30.2 and 33.0, 4 of 128 26.2 and 30.1.
     const long line = s == k64 || s == k128 ? 128 : 129;
-    if (rows <= 16 || with_rows(16 * wide[s]) < line) with_rows(16);
+    if (rows <= 16 || with_rows(16 * wide[s]) < line) few_rows();
     return L;
 }
 

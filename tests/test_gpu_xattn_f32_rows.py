@@ -79,6 +79,16 @@ def test_against_float64(H, KH, D, DV, lens, pos, chunk, kind):
         assert torch.equal(o.isinf(), last) and (o[~last].double() - ref[~last]).abs().le(off[~last]).all(), (o.double() - ref)[~last].abs().max()
 
 
+# steps of a row or a few: pasts around the first that is split, whose splits are two tiles, more than eight splits to merge, splits of
+# several tiles, wide heads, a chunk that begins inside a tile; sequences of unequal lengths, whose last splits have no key
+@pytest.mark.parametrize("H,KH,D,DV,lens,pos,chunk,kind", [
+    (32, 8, 64, 64, [1, 1, 1], [0, 255, 254], 0, "bias"), (32, 8, 64, 64, [1, 1], [319, 3], 0, "none"), (8, 2, 64, 64, [4, 1, 1], [1500, 600, 40], 0, "sink"),
+    (16, 4, 64, 48, [1], [2300], 1000, "bias"), (8, 4, 128, 128, [2, 1, 1], [127, 160, 900], 0, "bias"), (4, 1, 256, 256, [1, 1], [129, 700], 0, "sink"),
+    (16, 16, 256, 192, [1, 1, 1], [800, 60, 300], 0, "none")])
+def test_steps_against_float64(H, KH, D, DV, lens, pos, chunk, kind):
+    test_against_float64(H, KH, D, DV, lens, pos, chunk, kind)
+
+
 def attend_alone(q, k, v, spec, page=32):
     """One sequence from its first token: q [n, H, D], k [n, KH, D], v [n, KH, DV]"""
     from magicdec_amd import ops
