@@ -90,7 +90,7 @@ struct TileParams {
     const float* k_scale;
     const float* v_scale;
     const float* act;         // XIELU: the two numbers of the activation
-    // SWIGLU, 1 x 1 tiles: plain columns of a second weight over the same rows behind the gated ones (md_linear_fused_beside), or 0 of them
+    // SWIGLU, one M tile a workgroup: plain columns of a second weight over the same rows behind the gated ones (md_linear_fused_beside), or 0 of them
     const bf16_t* side_w;
     bf16_t* side_out;
     int64_t side_ldo;
@@ -279,8 +279,8 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
     MD_TS(0);
     // block id -> (weight tile group, M tile group): block b runs on XCD b % 8; the M groups of one weight tile group
     // stay on one XCD
-    constexpr bool kBeside = EPI == FL_SWIGLU && !PRO && MT * NT == 1;
-    const int m_groups = (p.m_tiles + MT - 1) / MT, n_groups = p.n_tiles / NT + (kBeside ? p.side_tiles : 0);
+    constexpr bool kBeside = EPI == FL_SWIGLU && !PRO && MT == 1;
+    const int m_groups = (p.m_tiles + MT - 1) / MT, n_groups = p.n_tiles / NT + (kBeside ? (p.side_tiles + NT - 1) / NT : 0);
     int tng, tmg, slice = 0;
     if constexpr (EPI == FL_PARTIAL) {
         // K slice in the FAST index: with S = 8 a slice -- i.e. the Kt columns of x it reads -- lives on one XCD's L2
@@ -295,8 +295,8 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
         tmg = slot % m_groups;
     }
     if (tng >= n_groups) return;
-    const bool beside = kBeside && tng >= p.n_tiles;
-    const int m0 = tmg * 32 * MT, tn0 = beside ? tng - p.n_tiles : tng * NT;
+    const bool beside = kBeside && tng >= p.n_tiles / NT;
+    const int m0 = tmg * 32 * MT, tn0 = (beside ? tng - p.n_tiles / NT : tng) * NT;
 
     // 16-deep MFMA k-steps of this wavefront's slice (FL_PARTIAL: of this workgroup's K slice, then of the wavefront)
     const int ksteps_w = (p.K >> 4) / (kNW * (EPI == FL_PARTIAL ? p.S : 1));
@@ -304,7 +304,8 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
     const bf16_t* wbase[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
-        wbase[nt] = (beside ? p.side_w : p.w) + ((int64_t)(tn0 + nt) * (p.K >> 4) + ks0) * 512;    // wave-uniform; + lane * 8 per lane
+        wbase[nt] = (beside ? p.side_w : p.w) +                // wave-uniform; + lane * 8 per lane (an odd number beside: the last tile twice)
+                    ((int64_t)(beside ? min(tn0 + nt, p.side_tiles - 1) : tn0 + nt) * (p.K >> 4) + ks0) * 512;
     unsigned char* my_lds = lds + wave * kWaveLdsT;
 
     // activation staging: instruction i covers rows 4i + (lane >> 4), 16 lanes read one 256-B row segment
@@ -591,7 +592,7 @@ __global__ __launch_bounds__(64 * NW, MT * NT > 1 ? 2 : 4) void tile_gemm_kernel
         } else if constexpr (EPI == FL_SWIGLU) {
             if (beside) {
                 const f32x2 s = tile_sum2(2 * cp);
-                if (gm < p.M) *reinterpret_cast<unsigned int*>(p.side_out + (int64_t)gm * p.side_ldo + tn * 32 + 2 * cp) = pack2(s[0], s[1]);
+                if (gm < p.M && tn < p.side_tiles) *reinterpret_cast<unsigned int*>(p.side_out + (int64_t)gm * p.side_ldo + tn * 32 + 2 * cp) = pack2(s[0], s[1]);
                 continue;
             }
             const int I = p.N >> 1;
@@ -800,7 +801,7 @@ int launch_tile_cfg(const TileParams& p, hipStream_t st) {
             return MD_ERR_LAUNCH;
         }
     }
-    const int m_groups = (p.m_tiles + MT - 1) / MT, n_groups = p.n_tiles / NT + p.side_tiles;
+    const int m_groups = (p.m_tiles + MT - 1) / MT, n_groups = p.n_tiles / NT + (p.side_tiles + NT - 1) / NT;
     const int grid = ((n_groups + 7) / 8) * 8 * m_groups;
     hipLaunchKernelGGL(k, dim3(grid), dim3(64 * NW), lds, st, p);
     return MD_OK;
@@ -840,6 +841,12 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
     // 8 slices against 5.3-5.4 with 16)
     const int wgs = (p.n_tiles + p.side_tiles) * p.m_tiles;
     bool nw16 = p.K % 256 == 0 && p.K >= 1024 && wgs <= 256;
+    // 17 to 32 rows of 257 to 512 column tiles: two of them a workgroup, one workgroup a CU, which then takes in its x once and as much of W
+    // as every other one (the same K slices and sums: the same bits).  Bufodra 1B's steps (352 gated tiles and 43 beside them, 14.5 -> 13.8
+    // us) of 24 and 32 requests 277.6 -> 273.9 and 282.1 -> 279.5 us a step of four layers, a 1B draft's (512) of 32 265.8 -> 263.6
+    if constexpr ((EPI == FL_SWIGLU || EPI == FL_NONE || EPI == FL_RESID || EPI == FL_XIELU) && !PRO)
+        if (p.m_tiles == 1 && p.M > 16 && p.n_tiles % 2 == 0 && wgs > 256 && wgs <= 512 && g_force_tile == 0 && g_force_nw == 0)
+            return launch_tile_cfg<EPI, FP8, 8, true, PRO, 1, 2>(p, st);
     if (g_force_nw == 8) nw16 = false;
     if (g_force_nw == 16) nw16 = p.K % 256 == 0;
     const bool wnt = p.m_tiles == 1;

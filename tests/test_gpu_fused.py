@@ -293,6 +293,25 @@ def test_fused_2x2_tiles_bit_identical_to_1x1(ops, M, N, K):
     assert not torch.isnan(outs[22][4].float()).any()
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 8256, 128), (32, 8256, 1024), (17, 16384, 2048), (32, 11264, 384)])
+def test_one_row_tile_of_64_columns(ops, M, N, K):
+    """17 to 32 rows of 257 to 512 column tiles, two of them a workgroup: the bits of one a workgroup."""
+    lib = ops._lib.load()
+    g = torch.Generator().manual_seed(M + N)
+    x, w, b, resid = (d(torch.randn(*n, generator=g).to(BF)) for n in ((M, K), (N, K), (N,), (M, N)))
+    act = d(torch.rand(2, generator=g) + 0.5)
+    pw, pw13 = ops.PackedWeight(w), ops.PackedWeight(w, swiglu=True)
+    outs = {}
+    try:
+        for knob in (0, 11):
+            lib.md_debug_set_fused_nw(knob)
+            outs[knob] = (ops.fused_linear(x, pw, b), *ops.fused_linear(x, pw, b, resid=resid, want_ssq=True), ops.fused_linear(x, pw13, swiglu=True),
+                          ops.fused_linear(x, pw13, swiglu=True, gelu=True), ops.fused_linear(x, pw, xielu=act))
+    finally:
+        lib.md_debug_set_fused_nw(0)
+    assert all(torch.equal(a, c) and a.isfinite().all() for a, c in zip(outs[0], outs[11]))
+
+
 @pytest.mark.parametrize("M,N", [(1, 8192), (16, 8224), (32, 8224), (17, 12320), (33, 4128)])
 def test_one_workgroup_a_cu_or_two(ops, M, N):
     """Either side of the line between 16-wave and 8-wave workgroups (256 of them), against the exact product."""
