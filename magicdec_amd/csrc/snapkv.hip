@@ -672,15 +672,15 @@ __device__ __forceinline__ unsigned int ordered16(unsigned short bits) {
 // Pooled + group-summed scores of 1024 columns of one (kv head, request), as bf16 bits: a thread owns four neighbouring columns, the
 // rows' columns (and half a pool width on either side) come through LDS.  All CUs take part; inside the selection's one workgroup per
 // (kv head, request) it was most of that kernel's 135 us.
-// Bound by latency: the columns of four rows are asked for together (each row behind the last one's barrier: 14 us for 16 MB, now 10.6).
+// Bound by latency: the columns of four rows are asked for together (each row behind the last one's barrier: 14 us for 16 MB, now 10.2; two bytes a load 10.6).
 constexpr int kPoolCols = 1024, kPoolHalf = 64;         // widest half pool that is staged
 constexpr int kPoolRows = 4;                            // rows staged at a time
 
-template <int KS>                                       // the pool's width where it is known (taps in registers), else 0
+template <int KS, bool VEC>                             // the pool's width where it is known (taps in registers), else 0; rows of whole 8-byte pieces
 __global__ __launch_bounds__(256) void snapkv_pool_kernel(const unsigned short* __restrict__ aws, int H, int KH, int g, int N, int ksz_any,
                                                           unsigned short* __restrict__ score_out) {
-    constexpr int kImg = kPoolCols + 2 * kPoolHalf, kLoads = (kPoolCols + 2 * (KS ? KS / 2 : kPoolHalf) + 255) / 256;
-    __shared__ __attribute__((aligned(16))) float img[kPoolRows][kImg];
+    constexpr int kImg = kPoolCols + 2 * kPoolHalf, kEdge = (2 * (KS ? KS / 2 : kPoolHalf) + 255) / 256;
+    __shared__ __attribute__((aligned(16))) float img[kPoolRows][kImg];      // column c0 + i at kPoolHalf + i
     const int ksz = KS ? KS : ksz_any;
     const int c0 = blockIdx.x * kPoolCols, kvh = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, half = ksz / 2;
     const bool staged = half <= kPoolHalf;
@@ -688,22 +688,39 @@ __global__ __launch_bounds__(256) void snapkv_pool_kernel(const unsigned short* 
     float tot[4] = {0.f, 0.f, 0.f, 0.f};
     for (int r0 = 0; r0 < g; r0 += kPoolRows) {
         if (staged) {
-            unsigned short v[kPoolRows][kLoads];
+            // a thread's own four columns of each row, and the first threads' half widths on either side
+            unsigned short v[kPoolRows][4], w[kPoolRows][kEdge > 0 ? kEdge : 1];
+            const int own = c0 + tid * 4;
 #pragma unroll
-            for (int r = 0; r < kPoolRows; ++r)
+            for (int r = 0; r < kPoolRows; ++r) {
+                const unsigned short* row = rows + (int64_t)min(r0 + r, g - 1) * N;
+                if constexpr (VEC) {
+                    const u32x2 x = *reinterpret_cast<const u32x2*>(row + min(own, N - 4));
 #pragma unroll
-                for (int k = 0; k < kLoads; ++k) {
-                    v[r][k] = rows[(int64_t)min(r0 + r, g - 1) * N + min(max(c0 - half + tid + k * 256, 0), N - 1)];
+                    for (int j = 0; j < 4; ++j) v[r][j] = (unsigned short)(x[j >> 1] >> (16 * (j & 1)));
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[r][j] = row[min(own + j, N - 1)];
                 }
+#pragma unroll
+                for (int k = 0; k < kEdge; ++k) {
+                    const int i = tid + k * 256, at = i < half ? c0 - half + i : c0 + kPoolCols + i - half;
+                    w[r][k] = row[min(max(at, 0), N - 1)];
+                }
+            }
             if (r0) __syncthreads();
 #pragma unroll
-            for (int r = 0; r < kPoolRows; ++r)
+            for (int r = 0; r < kPoolRows; ++r) {            // (adding 0 is what leaving a column out is)
+                f32x4 x;
 #pragma unroll
-                for (int k = 0; k < kLoads; ++k)
-                    if (tid + k * 256 < kPoolCols + 2 * half) {
-                        const int c = c0 - half + tid + k * 256;
-                        img[r][tid + k * 256] = c >= 0 && c < N ? bf16_bits_to_f32(v[r][k]) : 0.f;       // (adding 0 is what leaving a column out is)
-                    }
+                for (int j = 0; j < 4; ++j) x[j] = own + j < N ? bf16_bits_to_f32(v[r][j]) : 0.f;
+                *reinterpret_cast<f32x4*>(img[r] + kPoolHalf + tid * 4) = x;
+#pragma unroll
+                for (int k = 0; k < kEdge; ++k) {
+                    const int i = tid + k * 256, at = i < half ? c0 - half + i : c0 + kPoolCols + i - half;
+                    if (i < 2 * half) img[r][kPoolHalf + at - c0] = at >= 0 && at < N ? bf16_bits_to_f32(w[r][k]) : 0.f;
+                }
+            }
             __syncthreads();
         }
 #pragma unroll
@@ -712,7 +729,7 @@ __global__ __launch_bounds__(256) void snapkv_pool_kernel(const unsigned short* 
             float tap[4 + (KS ? KS - 1 : 0)];
             if constexpr (KS > 0) {
 #pragma unroll
-                for (int k = 0; k < 4 + KS - 1; ++k) tap[k] = img[r][tid * 4 + k];
+                for (int k = 0; k < 4 + KS - 1; ++k) tap[k] = img[r][kPoolHalf - KS / 2 + tid * 4 + k];
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -722,7 +739,7 @@ __global__ __launch_bounds__(256) void snapkv_pool_kernel(const unsigned short* 
 #pragma unroll
                     for (int k = 0; k < KS; ++k) acc += tap[j + k];
                 } else if (staged) {
-                    for (int k = 0; k < ksz; ++k) acc += img[r][s + k];
+                    for (int k = 0; k < ksz; ++k) acc += img[r][kPoolHalf - half + s + k];
                 } else {
                     for (int k = -half; k <= half; ++k) {
                         const int c = c0 + s + k;
@@ -760,7 +777,10 @@ __device__ __forceinline__ unsigned int scan1024(unsigned int v, unsigned int* w
 // one context share a few exponents: 8 bits would put nearly all of them into two counters), a workgroup scan for the bin of the k-th
 // largest, the same over its 16 low values; a thread's run of consecutive keys then knows by one scan which of the equal ones are
 // the first; the selected keys are ranked by counting (they are distinct: each carries its index).  Bound by latency: a dozen barriers
-// (the first version had 120, with single threads walking the histograms): 17.5 us for 16 000 keys.
+// (the first version had 120, with single threads walking the histograms).  Scores come and keys go eight at a time where the rows are
+// whole pieces of eight (VEC: contexts of a window and whole pages): 16 000 keys 16.7 -> 13.2 us.  (The copy of the rows by the same workgroup: 21 for 13.2 + 7.5
+here, but 7 us longer for rows of 128 or one request, where a workgroup's chain of loads is longer than the launch.)
+template <bool VEC>
 __global__ __launch_bounds__(1024) void snapkv_select_kernel(const unsigned short* __restrict__ scores, int KH, int N, int topk,
                                                              int32_t* idx_out) {
     constexpr int kBins = 4096;
@@ -773,21 +793,37 @@ __global__ __launch_bounds__(1024) void snapkv_select_kernel(const unsigned shor
     const int kvh = blockIdx.x, b = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const unsigned short* src = scores + ((int64_t)b * KH + kvh) * N;
+    constexpr int V = VEC ? 8 : 1;                            // keys at a time
+    typedef std::conditional_t<VEC, u32x4, unsigned short> piece;
+    const int np = N / V;                                     // pieces of the row
+    auto key_of = [](piece x, int e) -> unsigned int {
+        if constexpr (VEC) return e & 1 ? x[e >> 1] >> 16 : x[e >> 1] & 0xffffu;
+        else return x;
+    };
+    auto held = [&](int i) -> piece { return reinterpret_cast<const piece*>(keys)[i]; };
     for (int i = tid; i < kBins; i += 1024) hist[i] = 0;
     sel[tid] = 0;
     if (tid < 32) misc[tid] = 0;
     __syncthreads();
-    for (int s0 = tid; s0 < N; s0 += 8 * 1024) {              // (eight loads on their way)
-        unsigned short v[8];
+    constexpr int U = VEC ? 2 : 8;                            // (loads on their way)
+    for (int s0 = tid; s0 < np; s0 += U * 1024) {
+        piece v[U];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = src[min(s0 + j * 1024, N - 1)];
+        for (int j = 0; j < U; ++j) v[j] = reinterpret_cast<const piece*>(src)[min(s0 + j * 1024, np - 1)];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < U; ++j) {
             const int s = s0 + j * 1024;
-            if (s < N) {
-                const unsigned int k = ordered16(v[j]);
-                keys[s] = (unsigned short)k;
-                atomicAdd(&hist[k >> 4], 1u);
+            if (s < np) {
+                unsigned int k[V];
+#pragma unroll
+                for (int e = 0; e < V; ++e) {
+                    k[e] = ordered16((unsigned short)key_of(v[j], e));
+                    atomicAdd(&hist[k[e] >> 4], 1u);
+                }
+                if constexpr (VEC)
+                    reinterpret_cast<u32x4*>(keys)[s] = u32x4{k[0] | k[1] << 16, k[2] | k[3] << 16, k[4] | k[5] << 16, k[6] | k[7] << 16};
+                else
+                    keys[s] = (unsigned short)k[0];
             }
         }
     }
@@ -815,23 +851,35 @@ __global__ __launch_bounds__(1024) void snapkv_select_kernel(const unsigned shor
     }
     __syncthreads();
     const unsigned int bin = misc[0];
-    for (int s = tid; s < N; s += 1024)
-        if ((unsigned int)keys[s] >> 4 == bin) atomicAdd(&misc[16 + (keys[s] & 15)], 1u);
+    for (int s = tid; s < np; s += 1024) {
+        const piece x = held(s);
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+            if (key_of(x, e) >> 4 == bin) atomicAdd(&misc[16 + (key_of(x, e) & 15)], 1u);
+    }
     __syncthreads();
     unsigned int need = misc[1], low = 15;                    // (every thread: 16 broadcast reads)
     for (; low > 0 && misc[16 + low] < need; --low) need -= misc[16 + low];
     const unsigned int T = bin << 4 | low;                    // the k-th largest key; `need` keys == T are selected, lowest indices first
     // thread t's run of consecutive keys
-    const int run = (N + 1023) / 1024, first = min(tid * run, N), last = min(first + run, N);
+    const int run = (np + 1023) / 1024, first = min(tid * run, np), last = min(first + run, np);
     unsigned int eq = 0;
-    for (int s = first; s < last; ++s) eq += keys[s] == T;
+    for (int s = first; s < last; ++s) {
+        const piece x = held(s);
+#pragma unroll
+        for (int e = 0; e < V; ++e) eq += key_of(x, e) == T;
+    }
     unsigned int rank = scan1024(eq, waves, lane, wave) - eq;
     for (int s = first; s < last; ++s) {
-        const unsigned int k = keys[s];
-        if (k > T) sel[atomicAdd(&misc[2], 1u)] = k << 16 | (0xffffu - (unsigned int)s);
-        if (k == T) {
-            if (rank < need) sel[topk - need + rank] = k << 16 | (0xffffu - (unsigned int)s);
-            ++rank;
+        const piece x = held(s);
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+            const unsigned int k = key_of(x, e), tag = k << 16 | (0xffffu - (unsigned int)(s * V + e));
+            if (k > T) sel[atomicAdd(&misc[2], 1u)] = tag;
+            if (k == T) {
+                if (rank < need) sel[topk - need + rank] = tag;
+                ++rank;
+            }
         }
     }
     __syncthreads();
@@ -923,6 +971,21 @@ int score_launch(dim3 grid, int waves, size_t lds, const SnapParams& p, hipStrea
         return MD_ERR_LAUNCH;
     }
     hipLaunchKernelGGL(Kernel, grid, dim3(64 * waves), lds, st, p);
+    return MD_OK;
+}
+
+template <auto Kernel>
+int select_launch(int KH, int B, size_t lds, const unsigned short* scores, int N, int topk, int32_t* idx_out, hipStream_t st) {
+    static MdPerDeviceOnce once;
+    if (once.first()) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) {
+            once.undo();
+            md_set_error("md_snapkv_select: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
+            return MD_ERR_LAUNCH;
+        }
+    }
+    hipLaunchKernelGGL(Kernel, dim3(KH, B), dim3(1024), lds, st, scores, KH, N, topk, idx_out);
     return MD_OK;
 }
 
@@ -1089,21 +1152,13 @@ extern "C" int md_snapkv_select(const void* q_win, const void* cache, const int3
     MD_CHECK_LAUNCH("md_snapkv_select(scores)");
 
     const dim3 pgrid((N + kPoolCols - 1) / kPoolCols, KH, B);
-    if (pool_kernel == 5)
-        hipLaunchKernelGGL((snapkv_pool_kernel<5>), pgrid, dim3(256), 0, st, p.aws, H, KH, g, N, pool_kernel, scores);
-    else
-        hipLaunchKernelGGL((snapkv_pool_kernel<0>), pgrid, dim3(256), 0, st, p.aws, H, KH, g, N, pool_kernel, scores);
+    const auto pool = pool_kernel == 5 ? (N % 4 == 0 ? &snapkv_pool_kernel<5, true> : &snapkv_pool_kernel<5, false>)
+                                       : (N % 4 == 0 ? &snapkv_pool_kernel<0, true> : &snapkv_pool_kernel<0, false>);
+    hipLaunchKernelGGL(pool, pgrid, dim3(256), 0, st, p.aws, H, KH, g, N, pool_kernel, scores);
     const size_t lds3 = (size_t)((N + 7) / 8 * 8) * 2 + (4096 + 1024 + 16 + 32) * 4;
-    static MdPerDeviceOnce attr_once;
-    if (attr_once.first()) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&snapkv_select_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-        if (e != hipSuccess) {
-            md_set_error("md_snapkv_select: hipFuncSetAttribute failed: %s", hipGetErrorString(e));
-            return MD_ERR_LAUNCH;
-        }
-    }
-    hipLaunchKernelGGL(snapkv_select_kernel, dim3(KH, B), dim3(1024), lds3, st, scores, KH, N, topk, idx_out);
+    rc = N % 8 == 0 ? select_launch<&snapkv_select_kernel<true>>(KH, B, lds3, scores, N, topk, idx_out, st)
+                    : select_launch<&snapkv_select_kernel<false>>(KH, B, lds3, scores, N, topk, idx_out, st);
+    if (rc != MD_OK) return rc;
     MD_CHECK_LAUNCH("md_snapkv_select(select)");
 
     GatherParams gp;
