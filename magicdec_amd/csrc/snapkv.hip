@@ -779,7 +779,7 @@ __device__ __forceinline__ unsigned int scan1024(unsigned int v, unsigned int* w
 // the first; the selected keys are ranked by counting (they are distinct: each carries its index).  Bound by latency: a dozen barriers
 // (the first version had 120, with single threads walking the histograms).  Scores come and keys go eight at a time where the rows are
 // whole pieces of eight (VEC: contexts of a window and whole pages): 16 000 keys 16.7 -> 13.2 us.  (The copy of the rows by the same workgroup: 21 for 13.2 + 7.5
-here, but 7 us longer for rows of 128 or one request, where a workgroup's chain of loads is longer than the launch.)
+// here, but 7 us longer for rows of 128 or one request, where a workgroup's chain of loads is longer than the launch.)
 template <bool VEC>
 __global__ __launch_bounds__(1024) void snapkv_select_kernel(const unsigned short* __restrict__ scores, int KH, int N, int topk,
                                                              int32_t* idx_out) {
