@@ -544,6 +544,7 @@ int md_xattn(const md_xattn_args* args, md_stream_t stream);
  *                    with `tail` [row][h][tail_dim] also out[row][h][N ..] = rotated tail, zeros up to tail_pad.
  * md_embed_bigram    out (fp32) = rms(table[token] + pairs[(mul_before * before + mul_token * token) mod buckets]) * norm_weight;
  *                    row `buckets` of pairs for a sequence's first token; history (int32 [pages][page_size]) holds the tokens.
+ * md_embed_bigram_norm   and y (dtype) = rms(out) * next_weight, the first layer's norm, as md_resid_norm gives it, in the same launch.
  * md_gelu_mul        y = gelu_tanh(a) * b;  md_softcap  z = cap * tanh(z / cap), in place.
  * ---------------------------------------------------------------------- */
 typedef struct md_latent_args {
@@ -597,6 +598,11 @@ int md_embed_bigram(const int64_t* tokens, const void* table, const void* pairs,
                     const int32_t* qo_indptr, const int32_t* pos0, int B, int n_max, int width, int vocab, int buckets,
                     int64_t mul_before, int64_t mul_token, int32_t* history, const int32_t* page_indices,
                     const int32_t* page_indptr, int page_size, float eps, float* out, md_stream_t stream);
+int md_embed_bigram_norm(const int64_t* tokens, const void* table, const void* pairs, const void* norm_weight, int dtype,
+                         const int32_t* qo_indptr, const int32_t* pos0, int B, int n_max, int width, int vocab, int buckets,
+                         int64_t mul_before, int64_t mul_token, int32_t* history, const int32_t* page_indices,
+                         const int32_t* page_indptr, int page_size, float eps, float* out, const void* next_weight, void* y,
+                         md_stream_t stream);
 int md_gelu_mul(const void* a, const void* b, int64_t a_row_stride, int64_t b_row_stride, void* y, int64_t y_row_stride, int rows,
                 int dim, int dtype, md_stream_t stream);
 int md_softcap(void* z, int64_t z_row_stride, float cap, int rows, int dim, int dtype, md_stream_t stream);

@@ -458,12 +458,16 @@ class LayeredTransformer(Transformer):
         return self._project(side, layer.wout)
 
     def _embed(self, flat, rows, tab: PageTable):
-        c = self.spec
+        """(embedded rows, the first layer's norm of them where the same launch gives it, else None)."""
+        c, first = self.spec, self.layers[0]
         if c.bigram is not None:
-            return ops.embed_bigram(flat, self.tok_embeddings.weight, self.pair_embeddings.weight, self.embed_norm.weight, c.norm_eps,
-                                    c.bigram.mul_before, c.bigram.mul_token, self._history, rows, tab.indices, tab.indptr)
+            args = (flat, self.tok_embeddings.weight, self.pair_embeddings.weight, self.embed_norm.weight, c.norm_eps,
+                    c.bigram.mul_before, c.bigram.mul_token, self._history, rows, tab.indices, tab.indptr)
+            if flat.is_cuda and getattr(first, "shift", None) is None:
+                return ops.embed_bigram(*args, next_norm=first.attention_norm.weight)
+            return ops.embed_bigram(*args), None
         return ops.embed_pos(flat, self.tok_embeddings.weight,
-                             self.pos_embeddings.weight if self.pos_embeddings is not None else None, rows, c.embed_scale)
+                             self.pos_embeddings.weight if self.pos_embeddings is not None else None, rows, c.embed_scale), None
 
     def _step(self, idx, offsets, qo_indptr, tab: PageTable, n_max=None, head_rows=None):
         """One step over `idx` ([B, n], or flat with n_max): embed -> layers -> norm -> head -> argmax.  head_rows: the flat
@@ -472,15 +476,16 @@ class LayeredTransformer(Transformer):
         c = self.spec
         flat = idx.reshape(-1).contiguous()
         rows = ops.StepRows(qo_indptr, offsets, idx.shape[1] if idx.dim() == 2 else n_max, tab.slots)
-        x = self._embed(flat, rows, tab)
+        x, y = self._embed(flat, rows, tab)
         ctx = None
         if tab.lengths is not None and self.output.weight.dtype == torch.bfloat16:
             ctx = ops.LatentContext(*tab.lengths, x.device)
         delta = None
         for i, layer in enumerate(self.layers):
             att, kvc = layer.attention, layer.attention.kv_cache
-            x, y = ops.resid_norm(x, delta, layer.attention_norm.weight, c.norm_eps,
-                                  shift=getattr(layer, "shift", None), ring=self._rings[i], rows=rows)
+            if i > 0 or y is None:
+                x, y = ops.resid_norm(x, delta, layer.attention_norm.weight, c.norm_eps,
+                                      shift=getattr(layer, "shift", None), ring=self._rings[i], rows=rows)
             if isinstance(layer, ParallelLayer):
                 delta = self._parallel(i, layer, y, rows, tab, ctx)
                 if self._layer_hook is not None:

@@ -158,6 +158,7 @@ _SIGNATURES = {
     "md_latent_prefill": (c_int, [ctypes.POINTER(LatentArgs), P]),
     "md_head_linear": (c_int, [ctypes.POINTER(HeadLinearArgs), P]),
     "md_embed_bigram": (c_int, [P, P, P, P, I, P, P, I, I, I, I, I, L, L, P, P, P, I, c_float, P, P]),
+    "md_embed_bigram_norm": (c_int, [P, P, P, P, I, P, P, I, I, I, I, I, L, L, P, P, P, I, c_float, P, P, P, P]),
     "md_gelu_mul": (c_int, [P, P, L, L, P, L, I, I, I, P]),
     "md_softcap": (c_int, [P, L, c_float, I, I, I, P]),
     "md_argmax": (c_int, [P, L, I, I, L, P, P, P]),

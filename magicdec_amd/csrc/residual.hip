@@ -300,13 +300,17 @@ struct BigramParams {
     int64_t mul_before, mul_token;
     int width, vocab, buckets, page_size;
     float eps;
+    const void* next_w;      // NEXT: weight of the norm behind it (the same eps) ...
+    void* y;                 // ... and its rows, model dtype
 };
 
 __device__ __forceinline__ int64_t clamp_token(int64_t t, int vocab) {   // the host refuses such ids; never index past the table
     return t < 0 ? 0 : (t >= vocab ? vocab - 1 : t);
 }
 
-template <typename T, int VEC, int MAXV>
+// NEXT: also the first layer's norm of the row that is in registers, as resid_norm_kernel forms it (bit for bit): a step pays no launch for it
+// (32 rows of 2 048: 5.1 + 2.8 us, now 6.1), a prompt reads no row again (8 196 of 4 096: 58 + 60, now 68.5).
+template <typename T, int VEC, int MAXV, bool NEXT>
 __global__ __launch_bounds__(256) void embed_bigram_kernel(const BigramParams p) {
     __shared__ float red[8];
     const int b = blockIdx.y, j = blockIdx.x;
@@ -349,18 +353,39 @@ __global__ __launch_bounds__(256) void embed_bigram_kernel(const BigramParams p)
             st_vec<VEC>(p.out + (int64_t)(q0 + j) * p.width + i * VEC, h[it]);
         }
     }
+    if constexpr (NEXT) {
+        float s2 = 0.f;
+#pragma unroll
+        for (int it = 0; it < MAXV; ++it)
+            if ((int)threadIdx.x + it * 256 < nvec) {
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) s2 += h[it][e] * h[it][e];
+            }
+        const float rs2 = 1.0f / sqrtf(block_sum(s2, red) / (float)p.width + p.eps);
+#pragma unroll
+        for (int it = 0; it < MAXV; ++it) {
+            const int i = threadIdx.x + it * 256;
+            if (i < nvec) {
+                float w[VEC];
+                ld_vec<VEC>(reinterpret_cast<const T*>(p.next_w) + i * VEC, w);
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) h[it][e] = (h[it][e] * rs2) * w[e];
+                st_vec<VEC>(reinterpret_cast<T*>(p.y) + (int64_t)(q0 + j) * p.width + i * VEC, h[it]);
+            }
+        }
+    }
 }
 
-template <typename T>
+template <typename T, bool NEXT>
 void launch_bigram(const BigramParams& p, bool vec, dim3 grid, hipStream_t st) {
     const int trips = (p.width / (vec ? 8 : 1) + 255) / 256;
     if (vec) {
-        if (trips <= 1) hipLaunchKernelGGL((embed_bigram_kernel<T, 8, 1>), grid, dim3(256), 0, st, p);
-        else if (trips <= 2) hipLaunchKernelGGL((embed_bigram_kernel<T, 8, 2>), grid, dim3(256), 0, st, p);
-        else hipLaunchKernelGGL((embed_bigram_kernel<T, 8, 4>), grid, dim3(256), 0, st, p);
+        if (trips <= 1) hipLaunchKernelGGL((embed_bigram_kernel<T, 8, 1, NEXT>), grid, dim3(256), 0, st, p);
+        else if (trips <= 2) hipLaunchKernelGGL((embed_bigram_kernel<T, 8, 2, NEXT>), grid, dim3(256), 0, st, p);
+        else hipLaunchKernelGGL((embed_bigram_kernel<T, 8, 4, NEXT>), grid, dim3(256), 0, st, p);
     } else {
-        if (trips <= 4) hipLaunchKernelGGL((embed_bigram_kernel<T, 1, 4>), grid, dim3(256), 0, st, p);
-        else hipLaunchKernelGGL((embed_bigram_kernel<T, 1, 32>), grid, dim3(256), 0, st, p);
+        if (trips <= 4) hipLaunchKernelGGL((embed_bigram_kernel<T, 1, 4, NEXT>), grid, dim3(256), 0, st, p);
+        else hipLaunchKernelGGL((embed_bigram_kernel<T, 1, 32, NEXT>), grid, dim3(256), 0, st, p);
     }
 }
 
@@ -447,22 +472,42 @@ extern "C" int md_embed_pos(const int64_t* tokens, const void* table, const void
     return MD_OK;
 }
 
+static int embed_bigram(const char* who, const int64_t* tokens, const void* table, const void* pairs, const void* norm_weight, int dtype,
+                        const int32_t* qo_indptr, const int32_t* pos0, int B, int n_max, int width, int vocab, int buckets,
+                        int64_t mul_before, int64_t mul_token, int32_t* history, const int32_t* page_indices, const int32_t* page_indptr,
+                        int page_size, float eps, float* out, const void* next_weight, void* y, hipStream_t st) {
+    MD_CHECK_ARG(tokens && table && pairs && norm_weight && qo_indptr && pos0 && history && page_indices && page_indptr && out,
+                 "%s: null pointer argument", who);
+    MD_CHECK_ARG(B > 0 && B <= 65535 && n_max > 0 && width > 0 && width <= 8192 && vocab > 0 && buckets > 0 && page_size > 0,
+                 "%s: bad shape B=%d n_max=%d width=%d (<= 8192) buckets=%d", who, B, n_max, width, buckets);
+    MD_CHECK_ARG(dtype == MD_T_BF16 || dtype == MD_T_F32, "%s: dtype must be MD_T_BF16 or MD_T_F32", who);
+    BigramParams p = {tokens, table, pairs, norm_weight, qo_indptr, pos0, page_indices, page_indptr, history, out,
+                      mul_before, mul_token, width, vocab, buckets, page_size, eps, next_weight, y};
+    const bool vec = width % 8 == 0 && aligned16(table) && aligned16(pairs) && aligned16(norm_weight) && aligned16(out) &&
+                     aligned16(next_weight) && aligned16(y);
+    const dim3 grid(n_max, B);
+    if (dtype == MD_T_F32) y ? launch_bigram<float, true>(p, vec, grid, st) : launch_bigram<float, false>(p, vec, grid, st);
+    else y ? launch_bigram<bf16_t, true>(p, vec, grid, st) : launch_bigram<bf16_t, false>(p, vec, grid, st);
+    MD_CHECK_LAUNCH(who);
+    return MD_OK;
+}
+
 extern "C" int md_embed_bigram(const int64_t* tokens, const void* table, const void* pairs, const void* norm_weight, int dtype,
                                const int32_t* qo_indptr, const int32_t* pos0, int B, int n_max, int width, int vocab, int buckets,
                                int64_t mul_before, int64_t mul_token, int32_t* history, const int32_t* page_indices,
                                const int32_t* page_indptr, int page_size, float eps, float* out, md_stream_t stream) {
-    MD_CHECK_ARG(tokens && table && pairs && norm_weight && qo_indptr && pos0 && history && page_indices && page_indptr && out,
-                 "md_embed_bigram: null pointer argument");
-    MD_CHECK_ARG(B > 0 && B <= 65535 && n_max > 0 && width > 0 && width <= 8192 && vocab > 0 && buckets > 0 && page_size > 0,
-                 "md_embed_bigram: bad shape B=%d n_max=%d width=%d (<= 8192) buckets=%d", B, n_max, width, buckets);
-    MD_CHECK_ARG(dtype == MD_T_BF16 || dtype == MD_T_F32, "md_embed_bigram: dtype must be MD_T_BF16 or MD_T_F32");
-    BigramParams p = {tokens, table, pairs, norm_weight, qo_indptr, pos0, page_indices, page_indptr, history, out,
-                      mul_before, mul_token, width, vocab, buckets, page_size, eps};
-    const bool vec = width % 8 == 0 && aligned16(table) && aligned16(pairs) && aligned16(norm_weight) && aligned16(out);
-    if (dtype == MD_T_F32) launch_bigram<float>(p, vec, dim3(n_max, B), (hipStream_t)stream);
-    else launch_bigram<bf16_t>(p, vec, dim3(n_max, B), (hipStream_t)stream);
-    MD_CHECK_LAUNCH("md_embed_bigram");
-    return MD_OK;
+    return embed_bigram("md_embed_bigram", tokens, table, pairs, norm_weight, dtype, qo_indptr, pos0, B, n_max, width, vocab, buckets,
+                        mul_before, mul_token, history, page_indices, page_indptr, page_size, eps, out, nullptr, nullptr, (hipStream_t)stream);
+}
+
+extern "C" int md_embed_bigram_norm(const int64_t* tokens, const void* table, const void* pairs, const void* norm_weight, int dtype,
+                                    const int32_t* qo_indptr, const int32_t* pos0, int B, int n_max, int width, int vocab, int buckets,
+                                    int64_t mul_before, int64_t mul_token, int32_t* history, const int32_t* page_indices,
+                                    const int32_t* page_indptr, int page_size, float eps, float* out, const void* next_weight, void* y,
+                                    md_stream_t stream) {
+    MD_CHECK_ARG(next_weight && y, "md_embed_bigram_norm: null pointer argument");
+    return embed_bigram("md_embed_bigram_norm", tokens, table, pairs, norm_weight, dtype, qo_indptr, pos0, B, n_max, width, vocab, buckets,
+                        mul_before, mul_token, history, page_indices, page_indptr, page_size, eps, out, next_weight, y, (hipStream_t)stream);
 }
 
 extern "C" int md_resid_norm(const md_resid_norm_args* a, md_stream_t stream) {

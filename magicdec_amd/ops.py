@@ -1370,9 +1370,11 @@ class LatentContext:
         return self._choice[key]
 
 
-def embed_bigram(tokens, table, pairs, norm_weight, eps, mul_before, mul_token, history, rows: StepRows, page_indices, page_indptr):
+def embed_bigram(tokens, table, pairs, norm_weight, eps, mul_before, mul_token, history, rows: StepRows, page_indices, page_indptr,
+                 next_norm=None):
     """float32 rows rms(table[t] + pairs[(mul_before * before + mul_token * t) mod n]) * norm_weight; the last row of `pairs`
-    (row n) for a sequence's first token.  history: int32 [pages, page_size], the tokens of every sequence by position."""
+    (row n) for a sequence's first token.  history: int32 [pages, page_size], the tokens of every sequence by position.
+    next_norm: the weight of the norm behind them: (rows, resid_norm(rows, None, next_norm, eps)[1]) in the same launch."""
     _gpu(tokens, table, pairs, norm_weight, history)
     _dense(tokens, table, pairs, norm_weight, history)
     vocab, width = table.shape
@@ -1383,11 +1385,19 @@ def embed_bigram(tokens, table, pairs, norm_weight, eps, mul_before, mul_token, 
     if page_indptr.numel() != rows.B + 1:
         raise ValueError("embed_bigram: page table of another batch")
     out = torch.empty((tokens.numel(), width), dtype=torch.float32, device=table.device)
-    check(_lib.load().md_embed_bigram(_p(tokens), _p(table), _p(pairs), _p(norm_weight), _model_dtype(table), _p(rows.qo_indptr),
-                                      _p(rows.pos0), rows.B, rows.n_max, width, vocab, pairs.shape[0] - 1, int(mul_before),
-                                      int(mul_token), _p(history), _p(_i32(page_indices)), _p(_i32(page_indptr)), history.shape[1],
-                                      float(eps), _p(out), _stream()), "md_embed_bigram")
-    return out
+    args = (_p(tokens), _p(table), _p(pairs), _p(norm_weight), _model_dtype(table), _p(rows.qo_indptr), _p(rows.pos0), rows.B, rows.n_max,
+            width, vocab, pairs.shape[0] - 1, int(mul_before), int(mul_token), _p(history), _p(_i32(page_indices)),
+            _p(_i32(page_indptr)), history.shape[1], float(eps), _p(out))
+    if next_norm is None:
+        check(_lib.load().md_embed_bigram(*args, _stream()), "md_embed_bigram")
+        return out
+    _gpu(next_norm)
+    _dense(next_norm)
+    if next_norm.numel() != width or next_norm.dtype != table.dtype:
+        raise ValueError("embed_bigram: the next norm's weight is [width] of the tables' dtype")
+    y = torch.empty((tokens.numel(), width), dtype=table.dtype, device=table.device)
+    check(_lib.load().md_embed_bigram_norm(*args, _p(next_norm), _p(y), _stream()), "md_embed_bigram_norm")
+    return out, y
 
 
 def gelu_mul(a, b, out=None):

@@ -50,8 +50,10 @@ def test_embed_bigram_over_portions(ops, dtype, width, mul):  # noqa: F811
                 idx += own[b]
                 ptr.append(len(idx))
             rows = ops.StepRows(i32(qo), i32([at[b] for b in live]), max(n))
-            got = ops.embed_bigram(dev(torch.cat([seqs[b][at[b]:at[b] + k] for b, k in zip(live, n)])), dev(E), dev(G), dev(w), 1e-5, *mul,
-                                   history, rows, i32(idx), i32(ptr))
+            ids, held = dev(torch.cat([seqs[b][at[b]:at[b] + k] for b, k in zip(live, n)])), history.clone()
+            got = ops.embed_bigram(ids, dev(E), dev(G), dev(w), 1e-5, *mul, history, rows, i32(idx), i32(ptr))
+            both = ops.embed_bigram(ids, dev(E), dev(G), dev(w), 1e-5, *mul, held, rows, i32(idx), i32(ptr), next_norm=dev(w + 1))
+            assert torch.equal(both[0], got) and torch.equal(held, history) and torch.equal(both[1], ops.resid_norm(got, None, dev(w + 1), 1e-5)[1])
             ref = torch.cat([want[b][at[b]:at[b] + k] for b, k in zip(live, n)])
             assert got.dtype == F32 and torch.allclose(got.cpu().double(), ref, rtol=2e-6, atol=2e-6), (cuts, step)
             for b, k in zip(live, n):
