@@ -357,6 +357,7 @@ int md_linear_f32_thirds(const float* x, int64_t ldx, const float* w, float* out
  *   MD_FL_SWIGLU       out[M][N/2] = bf16(bf16(silu(bf16(h1))) * bf16(h3)); W packed for MD_EPI_SWIGLU, no bias
  *   MD_FL_RESID        out[M][N]   = bf16(resid + bf16(acc + bias))                 (the bf16 residual add)
  *   MD_FL_XIELU        out[M][N]   = bf16(xielu(acc)), no bias (md_xielu)
+ *   MD_FL_SOFTCAP      out[M][N]   = bf16(c * tanh(bf16(acc) / c)), c = act[0], no bias (md_softcap; not md_linear_few)
  *   MD_FL_ROPE_APPEND  N = (H + 2 KH) * D fused qkv rows [q; k; v]: q columns -> interleaved RoPE -> out = q_rot
  *                      [M][H*D] (contiguous); k columns -> RoPE -> paged cache; v columns -> paged cache.  Request b
  *                      owns rows [b * rows_per_req, (b+1) * rows_per_req) (uniform append, what a decode step has);
@@ -371,6 +372,7 @@ int md_linear_f32_thirds(const float* x, int64_t ldx, const float* w, float* out
 #define MD_FL_ROPE_APPEND 3
 #define MD_FL_XIELU 4
 #define MD_FL_GEGLU 5  /* MD_FL_SWIGLU's layout; out = bf16(gelu_tanh(h1) * h3), fp32 up to the one rounding */
+#define MD_FL_SOFTCAP 7
 typedef struct md_fused_linear_args {
     const void* x;            /* [M][K] bf16, row stride ldx (elements) */
     const void* w_packed;     /* streaming layout (md_linear, w_packed = 1) */
@@ -403,7 +405,7 @@ typedef struct md_fused_linear_args {
     const void* pro_norm_w;   /* bf16 [K] */
     float pro_eps;
     int pro_tiles;
-    const float* act;         /* MD_FL_XIELU: the two fp32 numbers of the activation (md_xielu) */
+    const float* act;         /* MD_FL_XIELU: the two fp32 numbers of the activation (md_xielu); MD_FL_SOFTCAP: the cap */
 } md_fused_linear_args;
 int md_linear_fused_supported(int M, int N, int K, int epilogue);
 int md_linear_fused(const md_fused_linear_args* args, md_stream_t stream);

@@ -29,7 +29,7 @@ from torch.nn import functional as F
 
 from .. import ops
 from .designs import DecoderSpec, LatentAttentionSpec, LayerSpec
-from .gemm_policy import choose, joint_launches, mode, use_split, want_packed_prompt
+from .gemm_policy import choose, joint_launches, mode, use_few, use_split, want_packed_prompt
 from .model_core import PageTable, RMSNorm, Transformer
 
 STATE_RING = 16        # unshifted rows kept per sequence and layer: rollbacks of up to STATE_RING - 2 tokens
@@ -266,6 +266,7 @@ class LayeredTransformer(Transformer):
         self.state_ring = max(int(state_ring), 2)
         longest = max_positions or num_pages * page_size
         self._xspec, self._rings, self._act = [], [], []
+        self._cap = torch.full((1,), c.logit_softcap or 0.0, dtype=torch.float32, device=dev)
         self._rotary, self._history = {}, None
         if c.bigram is not None:
             self._history = torch.zeros((num_pages, page_size), dtype=torch.int32, device=dev)
@@ -505,12 +506,20 @@ class LayeredTransformer(Transformer):
         x, y = ops.resid_norm(x, delta, self.norm.weight, c.norm_eps, out_scale=c.logit_scale)
         if head_rows is not None:
             y = y.index_select(0, head_rows)
-        logits = self._linear(y, self.output)
-        if c.logit_softcap is not None:
-            logits = ops.softcap_(logits, c.logit_softcap)
-        self._last_logits = logits
+        self._last_logits = logits = self._head(y)
         tokens = self._argmax(logits)
         return tokens.view(idx.shape) if head_rows is None else tokens
+
+    def _head(self, y):
+        cap, w = self.spec.logit_softcap, self.output.weight
+        if cap is None:
+            return self._linear(y, self.output)
+        # a step's head on the tile kernel caps its logits itself
+        if (y.dtype == torch.bfloat16 and y.is_cuda and self.output.bias is None and self._fused_here(y, w, "plain")
+                and not use_few(y.shape[0], *w.shape) and ops.fused_linear_supported(y.shape[0], *w.shape, ops.FL_SOFTCAP)):
+            self._last_M = y.shape[0]
+            return ops.fused_linear(y, self._packed[id(w)], softcap=self._cap)
+        return ops.softcap_(self._linear(y, self.output), cap)
 
     _layer_hook = None       # called as (layer index, residual, pending delta): diagnostics
 

@@ -65,6 +65,7 @@ constexpr int kWaveLds = 32 * kPitch;    // wave-private activation image (8704 
 enum { FL_NONE = 0, FL_SWIGLU = 1, FL_RESID = 2, FL_ROPE_APPEND = 3,
        FL_XIELU = 4,
        FL_GEGLU = 5,           // FL_SWIGLU's kernels with p.gelu
+       FL_SOFTCAP = 7,
        FL_PARTIAL = 6 };      // internal: the K range is ALSO split over workgroups; fp32 partial tiles -> workspace
 
 struct KvTable {
@@ -190,6 +191,9 @@ __device__ __forceinline__ void finish_pair(const TileParams& p, int gm, int n, 
     const float o0 = bf16_to_f32(f32_to_bf16(s[0])), o1 = bf16_to_f32(f32_to_bf16(s[1]));
     if constexpr (EPI == FL_NONE) {
         *reinterpret_cast<unsigned int*>(p.out + (int64_t)gm * p.ldo + n) = pack2(o0, o1);
+    } else if constexpr (EPI == FL_SOFTCAP) {         // md_softcap of the rounded product: no launch of 4.7 us behind a step's head
+        const float cap = p.act[0];
+        *reinterpret_cast<unsigned int*>(p.out + (int64_t)gm * p.ldo + n) = pack2(cap * tanhf(o0 / cap), cap * tanhf(o1 / cap));
     } else if constexpr (EPI == FL_RESID) {
         const unsigned int rv = *reinterpret_cast<const unsigned int*>(p.resid + (int64_t)gm * p.ldr + n);
         const float r0 = __uint_as_float(rv << 16), r1 = __uint_as_float(rv & 0xffff0000u);
@@ -827,7 +831,7 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
     // chunk, and measured 25.9 us in the cfg3 iteration against 24.5 for the 1 x 1 form -- profiles/r04_bench_cfg3_iter_breakdown.csv)
     // also WITH the deferred-RMSNorm prologue (SwiGLU consumer), now that that instantiation has a four-deep W
     // ring, no spills, and its own prologue (kNewPro in the kernel)
-    if constexpr ((EPI == FL_SWIGLU || EPI == FL_NONE || EPI == FL_RESID || EPI == FL_XIELU) && (!PRO || EPI == FL_SWIGLU)) {
+    if constexpr ((EPI == FL_SWIGLU || EPI == FL_NONE || EPI == FL_SOFTCAP || EPI == FL_RESID || EPI == FL_XIELU) && (!PRO || EPI == FL_SWIGLU)) {
         bool t22 = two_by_two(p.M, p.N, p.K);
         if (g_force_tile == 11 || p.side_tiles) t22 = false;
         if (g_force_tile == 22 && !p.side_tiles) t22 = p.n_tiles % 2 == 0 && p.K % 128 == 0;
@@ -844,7 +848,7 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
     // 17 to 32 rows of 257 to 512 column tiles: two of them a workgroup, one workgroup a CU, which then takes in its x once and as much of W
     // as every other one (the same K slices and sums: the same bits).  Bufodra 1B's steps (352 gated tiles and 43 beside them, 14.5 -> 13.8
     // us) of 24 and 32 requests 277.6 -> 273.9 and 282.1 -> 279.5 us a step of four layers, a 1B draft's (512) of 32 265.8 -> 263.6
-    if constexpr ((EPI == FL_SWIGLU || EPI == FL_NONE || EPI == FL_RESID || EPI == FL_XIELU) && !PRO)
+    if constexpr ((EPI == FL_SWIGLU || EPI == FL_NONE || EPI == FL_SOFTCAP || EPI == FL_RESID || EPI == FL_XIELU) && !PRO)
         if (p.m_tiles == 1 && p.M > 16 && p.n_tiles % 2 == 0 && wgs > 256 && wgs <= 512 && g_force_tile == 0 && g_force_nw == 0)
             return launch_tile_cfg<EPI, FP8, 8, true, PRO, 1, 2>(p, st);
     if (g_force_nw == 8) nw16 = false;
@@ -1060,12 +1064,12 @@ extern "C" void md_debug_set_fused_nw(int nw) {
 
 extern "C" int md_linear_fused_supported(int M, int N, int K, int epilogue) {
     if (M < 1 || M > 256 || K < 128 || K % 128 || N < 32 || N % 32) return 0;
-    return (epilogue >= FL_NONE && epilogue <= FL_GEGLU) ? 1 : 0;
+    return ((epilogue >= FL_NONE && epilogue <= FL_GEGLU) || epilogue == FL_SOFTCAP) ? 1 : 0;
 }
 
 extern "C" int md_linear_few_supported(int M, int N, int K, int epilogue) {
     MD_CHECK_ARG(M > 0 && N > 0 && K > 0, "md_linear_few_supported: M=%d N=%d K=%d", M, N, K);
-    return M <= 16 && K % 256 == 0 && md_linear_fused_supported(M, N, K, epilogue);
+    return M <= 16 && K % 256 == 0 && epilogue != FL_SOFTCAP && md_linear_fused_supported(M, N, K, epilogue);
 }
 
 namespace {
@@ -1127,6 +1131,11 @@ int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream, const
         [[fallthrough]];
     case FL_SWIGLU:
         rc = few ? launch_few<FL_SWIGLU, false>(p, st) : launch_tile<FL_SWIGLU, false>(p, st);
+        break;
+    case FL_SOFTCAP:
+        MD_CHECK_ARG(a->act && !a->bias, "%s: the soft cap needs `act` and takes no bias", who);
+        p.act = a->act;
+        rc = launch_tile<FL_SOFTCAP, false>(p, st);
         break;
     case FL_XIELU:
         MD_CHECK_ARG(a->act && !a->bias, "%s: the xIELU epilogue needs `act` and takes no bias", who);

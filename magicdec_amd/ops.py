@@ -708,7 +708,7 @@ def linear_f32_thirds(x, weight, tile=0):
 
 
 # ----------------------------------------------------------------------------- K8b
-FL_NONE, FL_SWIGLU, FL_RESID, FL_ROPE_APPEND, FL_XIELU, FL_GEGLU = 0, 1, 2, 3, 4, 5
+FL_NONE, FL_SWIGLU, FL_RESID, FL_ROPE_APPEND, FL_XIELU, FL_GEGLU, FL_SOFTCAP = 0, 1, 2, 3, 4, 5, 7
 
 
 @functools.lru_cache(maxsize=1024)
@@ -771,20 +771,30 @@ def _set_pro(a, x, pro: "DeferredNorm"):
 
 
 def fused_linear(x, weight: "PackedWeight", bias=None, swiglu=False, resid=None, out=None, want_ssq=False,
-                 pro: "DeferredNorm" = None, xielu=None, gelu=False, few=False):
+                 pro: "DeferredNorm" = None, xielu=None, gelu=False, few=False, softcap=None):
     """One launch (md_linear_fused): F.linear(x, W, bias) for M <= 256 rows over a PackedWeight, optionally followed by
     SiLU(h1) * h3 (swiglu=True, weight = [w1; w3]) or by the bf16 residual add `resid + linear` (resid [M, N]).
     want_ssq (with resid): also return the per-row partial sums of squares [M, N/32] of the result (the producer half of
     a deferred RMSNorm).  pro (with swiglu): x is pro.h and is normalised on the fly (the consumer half).
-    few: md_linear_few instead, M <= 16; its partial sums are [M, N/16], its sums of another order, and pro goes with everything."""
+    few: md_linear_few instead, M <= 16; its partial sums are [M, N/16], its sums of another order, and pro goes with everything.
+    softcap (float32 [1] on the GPU): softcap_ of the result, bit for bit."""
     epi = FL_RESID if resid is not None else (FL_XIELU if xielu is not None else FL_NONE)
     if swiglu:
         epi = FL_GEGLU if gelu else FL_SWIGLU
     if xielu is not None and epi != FL_XIELU:
         raise ValueError("fused linear: the xIELU epilogue takes nothing beside it")
+    if softcap is not None:
+        if epi != FL_NONE or few or bias is not None or pro is not None:
+            raise ValueError("fused linear: the soft cap takes nothing beside it")
+        _gpu(softcap)
+        if softcap.dtype != torch.float32 or softcap.numel() != 1:
+            raise ValueError("fused linear: float32 softcap[1] on the GPU expected")
+        epi = FL_SOFTCAP
     a = _fused_args(x, weight, bias, epi)
     if xielu is not None:
         a.act = _act_numbers(xielu).value
+    elif softcap is not None:
+        a.act = softcap.data_ptr()
     n_out = weight.N // 2 if swiglu else weight.N
     if out is None:
         out = torch.empty((x.shape[0], n_out), dtype=x.dtype, device=x.device)

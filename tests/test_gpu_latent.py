@@ -60,6 +60,19 @@ def test_embed_bigram_over_portions(ops, dtype, width, mul):  # noqa: F811
                 at[b] += k
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 64, 256), (5, 8256, 128), (17, 8256, 512), (32, 32000, 256), (64, 16384, 128), (200, 96, 384)])
+def test_softcap_behind_a_head(ops, M, N, K):  # noqa: F811
+    """The cap in the product's launch: the bits of md_softcap behind it, also of scores far beyond the cap."""
+    g = torch.Generator().manual_seed(M + N)
+    x, w = dev(torch.randn(M, K, generator=g).mul(4).to(BF)), ops.PackedWeight(dev(torch.randn(N, K, generator=g).to(BF)))
+    for cap in (30.0, 2.5):
+        assert torch.equal(ops.fused_linear(x, w, softcap=torch.tensor([cap], device=DEV)), ops.softcap_(ops.fused_linear(x, w), cap))
+    with pytest.raises(ValueError):
+        ops.fused_linear(x, w, softcap=torch.tensor([30.0], dtype=torch.float64, device=DEV))
+    with pytest.raises(ValueError):
+        ops.fused_linear(x, w, torch.zeros(N, dtype=BF, device=DEV), softcap=torch.tensor([30.0], device=DEV))
+
+
 @pytest.mark.parametrize("dtype", [BF, F32])
 @pytest.mark.parametrize("shape", [(3, 64), (65, 300), (2, 33)])
 def test_gelu_mul_and_softcap(ops, dtype, shape):  # noqa: F811
