@@ -373,6 +373,7 @@ int md_linear_f32_thirds(const float* x, int64_t ldx, const float* w, float* out
 #define MD_FL_XIELU 4
 #define MD_FL_GEGLU 5  /* MD_FL_SWIGLU's layout; out = bf16(gelu_tanh(h1) * h3), fp32 up to the one rounding */
 #define MD_FL_SOFTCAP 7
+#define MD_FL_STREAMED 0x100  /* or-ed to an epilogue: the weight is one of more than the last-level cache holds until it is read again (a hint) */
 typedef struct md_fused_linear_args {
     const void* x;            /* [M][K] bf16, row stride ldx (elements) */
     const void* w_packed;     /* streaming layout (md_linear, w_packed = 1) */

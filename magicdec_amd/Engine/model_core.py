@@ -45,6 +45,7 @@ from .gemm_policy import fused_mode, prompt_over_block, prompt_rows, use_few
 
 # A deep output projection leaves its norm to the next product up to the rows which that one stages in one instruction: at 16 rows of the
 # 7B model its norm costs more than the launch that is saved, 322 / 331 us of a two-layer step
+LAST_LEVEL_CACHE = 256 << 20     # bytes; of weights of twice as many, next to nothing is left when a step comes back to them
 DEEP_FEW_ROWS = 4
 
 
@@ -411,6 +412,8 @@ class Transformer(nn.Module):
             self._packed[id(w)] = pw
         self._released = set()          # ids of weights whose row-major tensor is currently released (release_rowmajor)
         self._by_id = {id(w): w for w, _ in todo}
+        for pw in self._packed.values():
+            pw.streamed = need > 2 * LAST_LEVEL_CACHE
         for w in self._by_id.values():   # (by the shapes and the engine's row counts: the same on the ranks of a group, before every prompt)
             self._packed[id(w)].rows_stay = self._rowmajor_in_decode(w)
 

@@ -96,6 +96,7 @@ struct TileParams {
     bf16_t* side_out;
     int64_t side_ldo;
     int side_tiles;
+    bool streamed;                   // host: W is not read again before the caches have lost it
     int gelu;                 // SWIGLU: GELU (tanh form), fp32 up to the product's one rounding, instead of SiLU
     unsigned int* overflow;   // dropped-row counter (md_page_overflow_count)
     // deferred RMSNorm (see the kernel header): producer side (RESID) / consumer side (PRO)
@@ -836,6 +837,11 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
         if (g_force_tile == 11 || p.side_tiles) t22 = false;
         if (g_force_tile == 22 && !p.side_tiles) t22 = p.n_tiles % 2 == 0 && p.K % 128 == 0;
         if (PRO && p.pro_tiles > 128) t22 = false;       // the 2 x 2 prologue keeps <= 8 partial sums per thread in flight
+        // Weights that no cache keeps until the next step: past the caches, where one group of rows reads them.  The product gains nothing
+        // by it (a 1B draft's gated one at 64 rows 20.2 / 21.1 us), but what is read again does: the other projections' weights, which stay in
+        // the last-level cache (qkv 8.0 -> 7.1, wo 7.4 -> 6.4).  A step of four layers (617 MB) 311.9 -> 301.3 us, of sixteen 1 083 -> 1 059;
+        // of two (373 MB, half of which the cache keeps) 160.2 -> 162.9, so that it is the caller who says which (MD_FL_STREAMED)
+        if (t22 && p.streamed && p.m_tiles <= 2) return launch_tile_cfg<EPI, FP8, 8, true, PRO, 2, 2>(p, st);
         if (t22) return launch_tile_cfg<EPI, FP8, 8, false, PRO, 2, 2>(p, st);
     }
     // 16 wavefronts (K/16 slices) where every CU has one workgroup at most: their activation images take 136 of the 160 KB, so a second
@@ -1074,10 +1080,13 @@ extern "C" int md_linear_few_supported(int M, int N, int K, int epilogue) {
 
 namespace {
 // md_linear_fused, md_linear_few: the same arguments; which kernel takes them
-int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream, const void* side_w = nullptr, int side_N = 0, void* side_out = nullptr,
+int run_fused(const md_fused_linear_args* given, bool few, md_stream_t stream, const void* side_w = nullptr, int side_N = 0, void* side_out = nullptr,
               int64_t side_ldo = 0) {
     const char* who = few ? "md_linear_few" : side_w ? "md_linear_fused_beside" : "md_linear_fused";
-    MD_CHECK_ARG(a && a->x && a->w_packed && a->out, "%s: null pointer argument", who);
+    MD_CHECK_ARG(given && given->x && given->w_packed && given->out, "%s: null pointer argument", who);
+    md_fused_linear_args args = *given;
+    args.epilogue &= ~MD_FL_STREAMED;
+    const md_fused_linear_args* a = &args;
     MD_CHECK_ARG(few ? md_linear_few_supported(a->M, a->N, a->K, a->epilogue) > 0 : md_linear_fused_supported(a->M, a->N, a->K, a->epilogue),
                  "%s: unsupported shape M=%d N=%d K=%d epilogue=%d (need 1 <= M <= %d, K %% %d == 0, "
                  "N %% 32 == 0)", who, a->M, a->N, a->K, a->epilogue, few ? 16 : 256, few ? 256 : 128);
@@ -1101,6 +1110,7 @@ int run_fused(const md_fused_linear_args* a, bool few, md_stream_t stream, const
     p.K = a->K;
     p.n_tiles = a->N / 32;
     p.m_tiles = (a->M + 31) / 32;
+    p.streamed = (given->epilogue & MD_FL_STREAMED) != 0;
     p.side_w = (const bf16_t*)side_w;
     p.side_out = (bf16_t*)side_out;
     p.side_ldo = side_ldo;
@@ -1207,7 +1217,8 @@ extern "C" int md_linear_fused_beside(const md_fused_linear_args* a, const void*
     MD_CHECK_ARG(a && w2_packed && out2, "md_linear_fused_beside: null pointer argument");
     MD_CHECK_ARG(a->M > 0 && a->N > 0 && a->K > 0 && N2 > 0 && md_linear_fused_beside_supported(a->M, a->N, a->K, N2),
                  "md_linear_fused_beside: unsupported shape M=%d N=%d K=%d N2=%d", a->M, a->N, a->K, N2);
-    MD_CHECK_ARG((a->epilogue == FL_SWIGLU || a->epilogue == FL_GEGLU) && !a->pro_ssq,
+    const int epilogue = a->epilogue & ~MD_FL_STREAMED;
+    MD_CHECK_ARG((epilogue == FL_SWIGLU || epilogue == FL_GEGLU) && !a->pro_ssq,
                  "md_linear_fused_beside: the first product is a gated one of finished rows");
     MD_CHECK_ARG(aligned16(w2_packed) && ((uintptr_t)out2 & 3) == 0 && ldo2 >= N2 && ldo2 % 2 == 0,
                  "md_linear_fused_beside: the second weight must be 16-byte aligned, its rows 4-byte");

@@ -308,9 +308,9 @@ class PackedWeight:
     """A linear's weight in the streaming layout of md_linear (include/magicdec_hip.h: w_packed = 1):
     [ceil(N/32)][K/16][64 lanes][8] -- element (t, s, lane, e) = W[32t + lane%32][16s + 8*(lane/32) + e], rows past N
     zero; for swiglu=True tile t = rows 16t..16t+15 of w1 then rows 16t..16t+15 of w3 (weight = [w1; w3], N = 2I).
-    Built once at load time (a torch permute: plumbing); bf16 or int8.  rows_stay: the row-major tensor beside it is never released
-    (Transformer._pack_weights)."""
-    rows_stay = False
+    Built once at load time (a torch permute: plumbing); bf16 or int8.  rows_stay: the row-major tensor beside it is never released;
+    streamed: a step's weights are more than the last-level cache keeps until the next one (Transformer._pack_weights)."""
+    rows_stay = streamed = False
 
     def __init__(self, weight, swiglu=False):
         N, K = weight.shape
@@ -708,7 +708,7 @@ def linear_f32_thirds(x, weight, tile=0):
 
 
 # ----------------------------------------------------------------------------- K8b
-FL_NONE, FL_SWIGLU, FL_RESID, FL_ROPE_APPEND, FL_XIELU, FL_GEGLU, FL_SOFTCAP = 0, 1, 2, 3, 4, 5, 7
+FL_NONE, FL_SWIGLU, FL_RESID, FL_ROPE_APPEND, FL_XIELU, FL_GEGLU, FL_SOFTCAP, FL_STREAMED = 0, 1, 2, 3, 4, 5, 7, 0x100
 
 
 @functools.lru_cache(maxsize=1024)
@@ -730,7 +730,7 @@ def _fused_args(x, weight: "PackedWeight", bias, epilogue):
         raise ValueError("PackedWeight was packed for a different epilogue")
     a = _lib.FusedLinearArgs()
     a.x, a.ldx, a.w_packed, a.bias = x.data_ptr(), x.stride(0), weight.data.data_ptr(), (bias.data_ptr() if bias is not None else None)
-    a.M, a.N, a.K, a.epilogue = M, weight.N, K, epilogue
+    a.M, a.N, a.K, a.epilogue = M, weight.N, K, epilogue | (FL_STREAMED if weight.streamed else 0)
     return a
 
 

@@ -293,6 +293,18 @@ def test_fused_2x2_tiles_bit_identical_to_1x1(ops, M, N, K):
     assert not torch.isnan(outs[22][4].float()).any()
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 16384, 2048), (64, 12288, 128), (40, 12352, 384), (128, 8192, 256)])
+def test_streamed_weights_give_the_same_bits(ops, M, N, K):
+    """2 x 2 tiles with loads past the caches and through them, and shapes that have one form."""
+    g = torch.Generator().manual_seed(M + N)
+    x, w, resid = (d(torch.randn(*n, generator=g).to(BF)) for n in ((M, K), (N, K), (M, N)))
+    pw, pw13, outs = ops.PackedWeight(w), ops.PackedWeight(w, swiglu=True), []
+    for pw.streamed in (False, True):
+        pw13.streamed = pw.streamed
+        outs.append((ops.fused_linear(x, pw), *ops.fused_linear(x, pw, resid=resid, want_ssq=True), ops.fused_linear(x, pw13, swiglu=True)))
+    assert all(torch.equal(a, c) and a.isfinite().all() for a, c in zip(*outs))
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 8256, 128), (32, 8256, 1024), (17, 16384, 2048), (32, 11264, 384)])
 def test_one_row_tile_of_64_columns(ops, M, N, K):
     """17 to 32 rows of 257 to 512 column tiles, two of them a workgroup: the bits of one a workgroup."""
