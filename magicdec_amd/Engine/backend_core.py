@@ -107,7 +107,8 @@ class SequencePool:
 
 class _Integers:
     """int32 tensors to be written, all in one launch where the device and the tensors allow that: page tables and lengths of a few hundred
-    bytes, for which as many launches are 4.5 us each between the portions of a prompt.  No piece reads what another one writes."""
+    bytes, for which as many launches are 4.5 us each between the portions of a prompt.  No piece reads what another one writes.  The
+    launch goes to the current device's stream: tensors of another device are written by torch, which finds the device from the tensor."""
 
     def __init__(self):
         self._pieces = []
@@ -132,7 +133,7 @@ class _Integers:
     def run(self):
         now = {}, []                                   # kinds of pieces, of one launch
         for t, on_gpu, otherwise in self._pieces:
-            if on_gpu is None or not ops.step_adds(t, (now[1] or [t])[0]):
+            if on_gpu is None or not ops.step_adds(t) or t.get_device() != torch.cuda.current_device():
                 otherwise()
                 continue
             if len(now[1]) == ops.STEP_MAX:

@@ -1467,6 +1467,34 @@ def test_step_launch_takes_tensors_of_one_device():
         ops.StepOps(add=[(i32["cuda:0"], 1), (i32["cuda:1"], 1)])
 
 
+def test_integers_of_another_device_are_left_to_torch(monkeypatch):
+    """Lengths and page tables of an engine whose device is not the current one: torch writes them, no launch goes to the current device's
+    stream; those of the current device are pieces of one launch (fake tensors: no memory is touched)."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from magicdec_amd import ops
+    from magicdec_amd.Engine.backend_core import _Integers
+    launched, written = [], []
+
+    class Launch:
+        def __init__(self, **pieces):
+            launched.append(sorted((kind, args[0].device.index) for kind, many in pieces.items() for args in many))
+
+        def run(self):
+            pass
+    monkeypatch.setattr(ops, "StepOps", Launch)
+    with FakeTensorMode():
+        t = {k: torch.empty(6, dtype=torch.int32, device=f"cuda:{k}") for k in (0, 1)}
+    for now in (0, 1):
+        monkeypatch.setattr(torch.cuda, "current_device", lambda: now)
+        launched.clear(), written.clear()
+        ints = _Integers()
+        for k in (1, 0):
+            ints.fill(t[k], 7), ints.grid(t[k], 2, 3), ints.scale(t[k], t[k], 2)
+        ints._pieces = [(x, on_gpu, lambda k=x.get_device(): written.append(k)) for x, on_gpu, _ in ints._pieces]
+        ints.run()
+        assert launched == [[("fill", now), ("grid", now), ("scale", now)]] and written == [1 - now] * 3
+
+
 @pytest.mark.parametrize("prompt", ["refused", "failing"])
 def test_a_refused_prompt_leaves_the_weights_released(cpu_ops_patched, prompt):
     """A prompt that raises (the SnapKV engine's refusal of its length, or an error inside a portion) ends like one that does not: no
