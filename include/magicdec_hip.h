@@ -526,6 +526,8 @@ typedef struct md_xattn_args {
 } md_xattn_args;
 int md_xattn_head_pad(int head_size);
 int md_xattn_fused_supported(const md_xattn_args* args);
+/* of attention on the fp32 matrix instructions (md_latent_workspace_bytes likewise): enough also for the same call with fewer pages; with
+ * less, or none, its keys are not split */
 size_t md_xattn_workspace_bytes(const md_xattn_args* args);
 int md_qk_norm_append(const md_xattn_args* args, void* q_out, md_stream_t stream);
 int md_xattn(const md_xattn_args* args, md_stream_t stream);

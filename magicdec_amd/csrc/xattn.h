@@ -27,7 +27,7 @@ struct XattnParams {
 // the plain kernel of xattn.hip (16- or 32-bit pages): any head sizes up to 1024, online softmax in fp32
 int md_internal_xattn_plain(const XattnParams& p, int dtype, hipStream_t st);
 // the same on the fp32 matrix instructions (xattn_f32.hip), for the head sizes its tiles fit; `keys`: the most one request can see.
-// p.ws: room for kv splits (md_internal_xattn_f32_workspace bytes), or null: no splits
+// p.ws: room for kv splits (md_internal_xattn_f32_workspace bytes: enough also for the same call with fewer keys), or null: no splits
 bool md_internal_xattn_f32_ok(const XattnParams& p);
 size_t md_internal_xattn_f32_workspace(const XattnParams& p, long keys);
 int md_internal_xattn_f32(const XattnParams& p, int dtype, long keys, hipStream_t st);

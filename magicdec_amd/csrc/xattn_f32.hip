@@ -674,7 +674,8 @@ Shape shape_of(const XattnParams& p) {
     return w <= 64 ? k64 : w <= 128 ? k128 : w <= 256 ? k256 : kNone;
 }
 
-F32Launch plan(const XattnParams& p, Shape s, long keys) {
+// room: bytes of scratch that are enough for this call and for the same one with fewer keys, whose rounded splits may be more of them
+F32Launch plan(const XattnParams& p, Shape s, long keys, size_t* room = nullptr) {
     static const int wide[] = {0, 4, 4, 2, 2, 2}, dvw[] = {0, 64, 128, 256, 256, 512}, kt[] = {0, 64, 32, 32, 32, 32};
     const int64_t rows = (int64_t)p.n_max * p.g, items = (int64_t)p.KH * p.B, tiles = (keys + kt[s] - 1) / kt[s];
     F32Launch L;
@@ -693,14 +694,16 @@ F32Launch plan(const XattnParams& p, Shape s, long keys) {
     // 21.5, 16 of 2 000 51.6 / 50.9.  Heads above 128, one workgroup a CU: 5 x 8 kv heads of 256, 600 keys 33.8 / 33.0, 6 of 8, 790
     // 56.9 / 40.2, but unequal sequences of more than 32 pairs level out with more splits than one round of CUs (7 x 8, to 1 587 keys 65.5 /
     // 73.8, 11 x 8 95.5 / 137): as above.
-    auto few_rows = [&]() {
+    // (returns the most splits of as many keys or fewer: 64 over 128 tiles, 43 of three over 129)
+    auto few_rows = [&]() -> int64_t {
         with_rows(16);
         const int64_t groups = L.nq * items;
         const bool two = s == k64 || s == k128;
-        if (groups <= 0 || (!two && groups > 32)) return;
+        if (groups <= 0 || (!two && groups > 32)) return L.nsplit;
         const int64_t want = two ? (512 + groups - 1) / groups : 256 / groups;
         const int64_t n = std::max<int64_t>(1, std::min<int64_t>({want, tiles < 5 ? 1 : tiles / 2, 64})), per = (tiles + n - 1) / n;
         L.nsplit = per > 0 ? (int)((tiles + per - 1) / per) : 1;
+        return n;
     };
     // Wide row groups reuse a tile's keys, 16 rows are the shorter chain: ahead by a fifth to a third while the wide ones are not half as
     // many workgroups as there are CUs (32 query heads of 64, 20 rows over 20 keys: 16.2 -> 11.6 us with the keys of a tile that are not
@@ -709,7 +712,17 @@ F32Launch plan(const XattnParams& p, Shape s, long keys) {
     // ahead where those tiles would be more than one a CU: 17 requests of 20 rows, heads of 256 (136) 53.4 and 34.9 us, of 32 rows 56.1 and
     // 38.7, but 16 of 32 (128) 30.2 and 33.0, 4 of 128 26.2 and 30.1.
     const long line = s == k64 || s == k128 ? 128 : 129;
-    if (rows <= 16 || with_rows(16 * wide[s]) < line) few_rows();
+    auto bytes = [&](int64_t splits) { return splits == 1 ? (size_t)0 : (size_t)(items * L.nq * splits * L.R) * (L.dvw + 2) * 4; };
+    const bool few = rows <= 16 || with_rows(16 * wide[s]) < line;
+    if (few) {
+        const int64_t most = few_rows();
+        if (room) *room = bytes(most);
+    } else if (room) {
+        const F32Launch W = L;
+        *room = bytes(L.nsplit);
+        if (W.nq * items < line) *room = std::max(*room, bytes(few_rows()));        // (behind fewer keys on 16 rows)
+        L = W;
+    }
     return L;
 }
 
@@ -776,8 +789,9 @@ int launch_shape(const XattnParams& p, Shape s, const F32Launch& L, hipStream_t 
 size_t md_internal_xattn_f32_workspace(const XattnParams& p, long keys) {
     const Shape s = shape_of(p);
     if (s == kNone) return 0;
-    const F32Launch L = plan(p, s, keys);
-    return L.nsplit == 1 ? 0 : (size_t)p.B * p.KH * L.nq * L.nsplit * L.R * (L.dvw + 2) * 4;
+    size_t room = 0;
+    plan(p, s, keys, &room);
+    return room;
 }
 
 bool md_internal_xattn_f32_ok(const XattnParams& p) { return shape_of(p) != kNone && p.page_size % 32 == 0; }

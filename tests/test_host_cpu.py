@@ -1495,6 +1495,29 @@ def test_integers_of_another_device_are_left_to_torch(monkeypatch):
         assert launched == [[("fill", now), ("grid", now), ("scale", now)]] and written == [1 - now] * 3
 
 
+@pytest.mark.parametrize("D,KH", [(64, 8), (128, 2), (192, 4), (0, 1)])
+def test_scratch_of_32_bit_attention_for_the_longest_is_enough_for_shorter_ones(D, KH):
+    """With less scratch than a call asks for, attention in 32 bits does not split its keys at all: a caller that sized it for the longest
+    context keeps the splits of every shorter one.  D = 0: latent attention."""
+    import ctypes
+    from magicdec_amd import _lib
+    lib = _lib.load()
+    split = False
+    for B in (1, 3, 8, 40, 70):
+        for n_max in (1, 5, 9, 12, 300):
+            if D:
+                a, ask = _lib.XattnArgs(dtype=1, D=D, DV=D, KH=KH, H=4 * KH), lib.md_xattn_workspace_bytes
+            else:
+                a, ask = _lib.LatentArgs(dtype=1, H=4, kv_rank=256, rot_dim=32), lib.md_latent_workspace_bytes
+            a.B, a.n_max, a.page_size, room = B, n_max, 32, 0
+            for a.max_pages in range(1, 1200):
+                need = ask(ctypes.byref(a))
+                assert need >= room, (B, n_max, a.max_pages)
+                room = need
+            split |= room > 0
+    assert split
+
+
 @pytest.mark.parametrize("prompt", ["refused", "failing"])
 def test_a_refused_prompt_leaves_the_weights_released(cpu_ops_patched, prompt):
     """A prompt that raises (the SnapKV engine's refusal of its length, or an error inside a portion) ends like one that does not: no
