@@ -1069,13 +1069,14 @@ extern "C" void md_debug_set_fused_nw(int nw) {
 #endif
 
 extern "C" int md_linear_fused_supported(int M, int N, int K, int epilogue) {
+    epilogue &= ~MD_FL_STREAMED;
     if (M < 1 || M > 256 || K < 128 || K % 128 || N < 32 || N % 32) return 0;
     return ((epilogue >= FL_NONE && epilogue <= FL_GEGLU) || epilogue == FL_SOFTCAP) ? 1 : 0;
 }
 
 extern "C" int md_linear_few_supported(int M, int N, int K, int epilogue) {
     MD_CHECK_ARG(M > 0 && N > 0 && K > 0, "md_linear_few_supported: M=%d N=%d K=%d", M, N, K);
-    return M <= 16 && K % 256 == 0 && epilogue != FL_SOFTCAP && md_linear_fused_supported(M, N, K, epilogue);
+    return M <= 16 && K % 256 == 0 && (epilogue & ~MD_FL_STREAMED) != FL_SOFTCAP && md_linear_fused_supported(M, N, K, epilogue);
 }
 
 namespace {

@@ -1518,6 +1518,16 @@ def test_scratch_of_32_bit_attention_for_the_longest_is_enough_for_shorter_ones(
     assert split
 
 
+def test_an_epilogue_is_supported_with_the_hint_as_without_it():
+    from magicdec_amd import _lib, ops
+    lib = _lib.load()
+    for ask in (lib.md_linear_fused_supported, lib.md_linear_few_supported):
+        for M, N, K in ((1, 64, 256), (16, 4096, 4096), (64, 16384, 2048), (256, 96, 128), (257, 64, 256), (4, 65, 256)):
+            for epilogue in range(-1, 10):
+                assert ask(M, N, K, epilogue | ops.FL_STREAMED) == ask(M, N, K, epilogue), (M, N, K, epilogue)
+    assert lib.md_linear_fused_supported(64, 16384, 2048, ops.FL_SOFTCAP | ops.FL_STREAMED) == 1
+
+
 @pytest.mark.parametrize("prompt", ["refused", "failing"])
 def test_a_refused_prompt_leaves_the_weights_released(cpu_ops_patched, prompt):
     """A prompt that raises (the SnapKV engine's refusal of its length, or an error inside a portion) ends like one that does not: no
