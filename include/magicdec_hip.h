@@ -549,7 +549,8 @@ int md_xattn(const md_xattn_args* args, md_stream_t stream);
  *                    with `tail` [row][h][tail_dim] also out[row][h][N ..] = rotated tail, zeros up to tail_pad.
  * md_embed_bigram    out (fp32) = rms(table[token] + pairs[(mul_before * before + mul_token * token) mod buckets]) * norm_weight;
  *                    row `buckets` of pairs for a sequence's first token; history (int32 [pages][page_size]) holds the tokens.
- * md_embed_bigram_norm   and y (dtype) = rms(out) * next_weight, the first layer's norm, as md_resid_norm gives it, in the same launch.
+ * md_embed_bigram_norm   and y (dtype) = rms(out) * next_weight, the first layer's norm, as md_resid_norm gives it, in the same launch
+ *                    (operands that are not 16-byte aligned: up to the order of a row's sums).
  * md_gelu_mul        y = gelu_tanh(a) * b;  md_softcap  z = cap * tanh(z / cap), in place.
  * ---------------------------------------------------------------------- */
 typedef struct md_latent_args {

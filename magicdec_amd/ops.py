@@ -1384,9 +1384,10 @@ def embed_bigram(tokens, table, pairs, norm_weight, eps, mul_before, mul_token, 
                  next_norm=None):
     """float32 rows rms(table[t] + pairs[(mul_before * before + mul_token * t) mod n]) * norm_weight; the last row of `pairs`
     (row n) for a sequence's first token.  history: int32 [pages, page_size], the tokens of every sequence by position.
-    next_norm: the weight of the norm behind them: (rows, resid_norm(rows, None, next_norm, eps)[1]) in the same launch."""
-    _gpu(tokens, table, pairs, norm_weight, history)
-    _dense(tokens, table, pairs, norm_weight, history)
+    next_norm: the weight of the norm behind them: (rows, resid_norm(rows, None, next_norm, eps)[1]), in the same launch unless that weight is
+    of another dtype than the tables, or one of them lies unaligned (whose rows the two launches add up in orders of their own)."""
+    _gpu(tokens, table, pairs, norm_weight, history, next_norm)
+    _dense(tokens, table, pairs, norm_weight, history, next_norm)
     vocab, width = table.shape
     if tokens.dtype != torch.int64 or history.dtype != torch.int32 or history.dim() != 2:
         raise TypeError("embed_bigram: token ids are int64, the token history int32 [pages, page_size]")
@@ -1394,17 +1395,15 @@ def embed_bigram(tokens, table, pairs, norm_weight, eps, mul_before, mul_token, 
         raise ValueError("embed_bigram: tables of different widths or dtypes")
     if page_indptr.numel() != rows.B + 1:
         raise ValueError("embed_bigram: page table of another batch")
+    if next_norm is not None and next_norm.numel() != width:
+        raise ValueError("embed_bigram: the next norm's weight is [width]")
     out = torch.empty((tokens.numel(), width), dtype=torch.float32, device=table.device)
     args = (_p(tokens), _p(table), _p(pairs), _p(norm_weight), _model_dtype(table), _p(rows.qo_indptr), _p(rows.pos0), rows.B, rows.n_max,
             width, vocab, pairs.shape[0] - 1, int(mul_before), int(mul_token), _p(history), _p(_i32(page_indices)),
             _p(_i32(page_indptr)), history.shape[1], float(eps), _p(out))
-    if next_norm is None:
+    if next_norm is None or next_norm.dtype != table.dtype or any(t.data_ptr() % 16 for t in (table, pairs, norm_weight, next_norm)):
         check(_lib.load().md_embed_bigram(*args, _stream()), "md_embed_bigram")
-        return out
-    _gpu(next_norm)
-    _dense(next_norm)
-    if next_norm.numel() != width or next_norm.dtype != table.dtype:
-        raise ValueError("embed_bigram: the next norm's weight is [width] of the tables' dtype")
+        return out if next_norm is None else (out, resid_norm(out, None, next_norm, eps)[1])
     y = torch.empty((tokens.numel(), width), dtype=table.dtype, device=table.device)
     check(_lib.load().md_embed_bigram_norm(*args, _p(next_norm), _p(y), _stream()), "md_embed_bigram_norm")
     return out, y

@@ -54,6 +54,12 @@ def test_embed_bigram_over_portions(ops, dtype, width, mul):  # noqa: F811
             got = ops.embed_bigram(ids, dev(E), dev(G), dev(w), 1e-5, *mul, history, rows, i32(idx), i32(ptr))
             both = ops.embed_bigram(ids, dev(E), dev(G), dev(w), 1e-5, *mul, held, rows, i32(idx), i32(ptr), next_norm=dev(w + 1))
             assert torch.equal(both[0], got) and torch.equal(held, history) and torch.equal(both[1], ops.resid_norm(got, None, dev(w + 1), 1e-5)[1])
+            # the norm's weight or a table unaligned; a weight of another dtype
+            shifted = lambda t: dev(torch.cat([t.reshape(-1)[:1], t.reshape(-1)]))[1:].view(t.shape)        # noqa: E731
+            for table, other in ((dev(E), shifted(w + 1)), (shifted(E), dev(w + 1)), (dev(E), dev((w + 1).to(F32 if dtype == BF else BF)))):
+                alone = ops.embed_bigram(ids, table, dev(G), dev(w), 1e-5, *mul, held, rows, i32(idx), i32(ptr))
+                both = ops.embed_bigram(ids, table, dev(G), dev(w), 1e-5, *mul, held, rows, i32(idx), i32(ptr), next_norm=other)
+                assert torch.equal(both[0], alone) and torch.equal(both[1], ops.resid_norm(alone, None, other, 1e-5)[1]) and both[1].dtype == other.dtype
             ref = torch.cat([want[b][at[b]:at[b] + k] for b, k in zip(live, n)])
             assert got.dtype == F32 and torch.allclose(got.cpu().double(), ref, rtol=2e-6, atol=2e-6), (cuts, step)
             for b, k in zip(live, n):
