@@ -823,6 +823,20 @@ bool two_by_two(int M, int N, int K) {
     return m_tiles >= 2 && n_tiles % 2 == 0 && K % 128 == 0 && (n_tiles / 2) * ((m_tiles + 1) / 2) >= 192;
 }
 
+// Two column tiles a workgroup for 17 to 32 rows of 257 to 512 of them: at most one workgroup a CU, which takes its x in once for both (the
+// same K slices and sums: the same bits).  us, one tile a workgroup / two, 17 and 32 rows: 264 x 2 048 + residual 12.1 / 10.5, 12.9 / 11.0;
+// 352 plain 12.9 / 12.6, 13.3 / 12.0; 384 x 5 120 29.9 / 26.1, 31.2 / 27.0; 512 x 2 048 level.  Steps of four layers: Bufodra 1B (352 gated
+// tiles and 43 beside them) of 24 and 32 requests 277.6 -> 273.9 and 282.1 -> 279.5, a 1B draft (512) of 32 265.8 -> 263.6.
+// Not where a workgroup's second sum and epilogue outweigh its x.  Of few K: plain, residual and capped ones gain from 896 on (258 x 896
+// 6.5 / 6.2, 7.0 / 6.6; 258 x 768 with a residual 6.3 / 6.5), gated ones beyond 1 024 (384 x 1 024, 17 rows 7.6 / 8.1; 258 x 512 5.7 / 6.5), xIELU,
+// whose epilogue is the longest, from 1 920 on and to 352 tiles (320 x 640 7.5 / 8.8; 320 x 2 048 13.0 / 12.9, 14.1 / 13.2; 448 x 2 048 14.5 / 15.4).
+// And K = 4 096, to 400 tiles: 400 23.9 / 23.1, 25.3 / 23.8, but 448 24.3 / 25.3, 26.0 / 25.5, 512 26.7 / 28.4, 28.0 / 28.8 (3 968 and 4 224 gain 4 to
+// 17 % everywhere: one tile of exactly 4 096 is a sixth faster than its neighbours, two are not).
+bool two_columns(int epi, int M, int K, int wgs) {
+    const int deep = epi == FL_XIELU ? 1920 : epi == FL_SWIGLU ? 1152 : 896, most = epi == FL_XIELU ? 352 : K == 4096 ? 400 : 512;
+    return M > 16 && M <= 32 && K >= deep && wgs > 256 && wgs <= most;
+}
+
 template <int EPI, bool FP8, bool PRO>
 int launch_tile_pro(const TileParams& p, hipStream_t st) {
     // 2 x 2 tiles (64 rows x 64 columns per workgroup, one per CU): when the M range has two 32-row tiles and the 64-column
@@ -851,11 +865,8 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
     // 8 slices against 5.3-5.4 with 16)
     const int wgs = (p.n_tiles + p.side_tiles) * p.m_tiles;
     bool nw16 = p.K % 256 == 0 && p.K >= 1024 && wgs <= 256;
-    // 17 to 32 rows of 257 to 512 column tiles: two of them a workgroup, one workgroup a CU, which then takes in its x once and as much of W
-    // as every other one (the same K slices and sums: the same bits).  Bufodra 1B's steps (352 gated tiles and 43 beside them, 14.5 -> 13.8
-    // us) of 24 and 32 requests 277.6 -> 273.9 and 282.1 -> 279.5 us a step of four layers, a 1B draft's (512) of 32 265.8 -> 263.6
     if constexpr ((EPI == FL_SWIGLU || EPI == FL_NONE || EPI == FL_SOFTCAP || EPI == FL_RESID || EPI == FL_XIELU) && !PRO)
-        if (p.m_tiles == 1 && p.M > 16 && p.n_tiles % 2 == 0 && wgs > 256 && wgs <= 512 && g_force_tile == 0 && g_force_nw == 0)
+        if (p.n_tiles % 2 == 0 && two_columns(EPI, p.M, p.K, wgs) && g_force_tile == 0 && g_force_nw == 0)
             return launch_tile_cfg<EPI, FP8, 8, true, PRO, 1, 2>(p, st);
     if (g_force_nw == 8) nw16 = false;
     if (g_force_nw == 16) nw16 = p.K % 256 == 0;
