@@ -293,15 +293,19 @@ def test_fused_2x2_tiles_bit_identical_to_1x1(ops, M, N, K):
     assert not torch.isnan(outs[22][4].float()).any()
 
 
-@pytest.mark.parametrize("M,N,K", [(33, 16384, 2048), (64, 12288, 128), (40, 12352, 384), (128, 8192, 256)])
+@pytest.mark.parametrize("M,N,K", [(33, 16384, 2048), (64, 12288, 128), (40, 12352, 384), (128, 8192, 256), (64, 16384, 2048), (48, 12288, 1024)])
 def test_streamed_weights_give_the_same_bits(ops, M, N, K):
-    """2 x 2 tiles with loads past the caches and through them, and shapes that have one form."""
+    """2 x 2 tiles with loads past the caches and through them, with and without the norm of a draft's step in front, and shapes that have
+    one form."""
     g = torch.Generator().manual_seed(M + N)
     x, w, resid = (d(torch.randn(*n, generator=g).to(BF)) for n in ((M, K), (N, K), (M, N)))
+    nw, ssq, act = d((1 + 0.1 * torch.randn(K, generator=g)).to(BF)), d(torch.rand(M, K // 32, generator=g) * 32.0), d(torch.rand(2, generator=g) + 0.5)
     pw, pw13, outs = ops.PackedWeight(w), ops.PackedWeight(w, swiglu=True), []
     for pw.streamed in (False, True):
         pw13.streamed = pw.streamed
-        outs.append((ops.fused_linear(x, pw), *ops.fused_linear(x, pw, resid=resid, want_ssq=True), ops.fused_linear(x, pw13, swiglu=True)))
+        outs.append((ops.fused_linear(x, pw), *ops.fused_linear(x, pw, resid=resid, want_ssq=True), ops.fused_linear(x, pw13, swiglu=True),
+                     ops.fused_linear(x, pw13, swiglu=True, pro=ops.DeferredNorm(x, ssq, nw, 1e-5)),
+                     ops.fused_linear(x, pw13, swiglu=True, gelu=True), ops.fused_linear(x, pw, xielu=act), ops.fused_linear(x, pw, softcap=act[:1])))
     assert all(torch.equal(a, c) and a.isfinite().all() for a, c in zip(*outs))
 
 

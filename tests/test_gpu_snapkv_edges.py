@@ -37,6 +37,33 @@ def test_select_in_groups_of_64_columns(monkeypatch, g, W, D, S):
     check_select(monkeypatch, 64, 4, g, W, D, S, 129, 5, 128, (0, 63))
 
 
+# rounds of 16 wavefronts of 32 columns (heads of 64) and of 8 (128): 4 and 8, where a wavefront loads its next 64 columns behind the last
+# products, and 7 and 9, the odd numbers from which 64 columns are taken as well; the last columns end inside a group
+@pytest.mark.parametrize("g,W,D,S", [(2, 16, 64, 2048), (4, 32, 64, 2040), (8, 16, 64, 4000), (4, 32, 64, 3584), (8, 16, 64, 3500),
+                                     (2, 16, 128, 2048), (4, 32, 128, 1792), (8, 16, 128, 2300)])
+def test_select_in_groups_of_64_columns_one_after_the_other(monkeypatch, g, W, D, S):
+    check_select(monkeypatch, 64, 4, g, W, D, S, 129, 5, 128, (0, 63))
+
+
+@pytest.mark.parametrize("g,W,D,S", [(2, 16, 64, 1000), (4, 32, 64, 2048), (8, 16, 64, 3584), (2, 16, 128, 1024), (4, 32, 128, 2048), (8, 16, 128, 1792)])
+def test_select_in_groups_of_64_columns_of_fp8_pages(g, W, D, S):
+    """fp8 pages of the same numbers, with scales that are powers of two: the bits of 16-bit pages that hold them scaled."""
+    from magicdec_amd import ops
+    B, KH, page, budget = 64, 4, 128, 129
+    H, ppr, dpr = KH * g, -(-S // page), budget // page + 1
+    gen = torch.Generator().manual_seed(S + g)
+    q = torch.randint(-1, 2, (B * W, H, D), generator=gen).bfloat16().to(DEV)
+    kv = torch.randint(-1, 2, (B * ppr, 2, KH, page, D), generator=gen).to(DEV)
+    scales = tuple(torch.tensor(s, device=DEV) for s in ([0.5, 1.0, 2.0, 0.25], [1.0, 4.0, 0.5, 2.0]))
+    table = lambda n: (torch.arange(B * n, dtype=torch.int32, device=DEV), torch.arange(B + 1, dtype=torch.int32, device=DEV) * n)      # noqa: E731
+    got = []
+    for cache, kw in ((kv.to(torch.float8_e4m3fn), dict(kv_scales=scales)), ((kv * torch.stack(scales).view(1, 2, KH, 1, 1)).bfloat16(), {})):
+        draft = torch.zeros(B * dpr, 2, page, KH, D, dtype=torch.bfloat16, device=DEV)
+        got.append((*ops.snapkv_select(q, cache, *table(ppr), S, W, budget, 5, draft, *table(dpr), torch.ones(B, dtype=torch.int32, device=DEV),
+                                       ops.AttnWorkspace(DEV), return_scores=True, kv_layout="HND", **kw), draft))
+    assert all(torch.equal(a, c) for a, c in zip(*got)) and got[0][1].float().isfinite().all() and got[0][2].any()
+
+
 # accumulators, query image and table of exponentials in one CU's LDS: the most queries a kv head (with the whole table 160 to 170 KB of 160)
 @pytest.mark.parametrize("g,W,D", [(32, 8, 128), (30, 8, 128), (28, 8, 128), (16, 16, 128), (32, 8, 64)])
 @pytest.mark.parametrize("KH,S", [(1, 1060), (3, 150)])
