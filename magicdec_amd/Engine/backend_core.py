@@ -131,9 +131,12 @@ class _Integers:
         self._add(dst, dict(scale=[(dst, src, a)]) if ops.step_adds(src, dst) else None, lambda: dst.copy_(src * a))
 
     def run(self):
-        now = {}, []                                   # kinds of pieces, of one launch
+        now, here = ({}, []), None                     # kinds of pieces, of one launch; the current device
         for t, on_gpu, otherwise in self._pieces:
-            if on_gpu is None or not ops.step_adds(t) or t.get_device() != torch.cuda.current_device():
+            ours = on_gpu is not None and ops.step_adds(t)
+            if ours and here is None:
+                here = torch.cuda.current_device()
+            if not ours or t.get_device() != here:
                 otherwise()
                 continue
             if len(now[1]) == ops.STEP_MAX:
@@ -320,6 +323,8 @@ class _BackendBase:
 
     def _portion(self, end, n):
         """Pages for a prompt's first `end` tokens, n of them new: their qo_indptr."""
+        if self._t.mapped:
+            return self._qo(n)                                # (nothing beside it to be written)
         ints, qo = _Integers(), torch.empty_like(self.qo_indptr)
         self._t.map_pages(-(-end // PAGE_SIZE), (end - 1) % PAGE_SIZE + 1, ints)
         ints.scale(qo, self.qo_indptr, n)

@@ -1518,6 +1518,17 @@ def test_scratch_of_32_bit_attention_for_the_longest_is_enough_for_shorter_ones(
     assert split
 
 
+def test_a_portion_of_a_model_addressed_by_position_writes_no_page_table(monkeypatch):
+    """Its pages are mapped from the start: qo_indptr * n is all there is to write, one torch operation and not a launch that is put together
+    for it."""
+    from types import SimpleNamespace
+    from magicdec_amd.Engine import backend_core as bc
+    monkeypatch.setattr(bc, "_Integers", None)
+    o = SimpleNamespace(qo_indptr=torch.arange(4, dtype=torch.int32), _qo_bound=None, _t=SimpleNamespace(mapped=True))
+    o._qo = lambda n: bc._BackendBase._qo(o, n)
+    assert torch.equal(bc._BackendBase._portion(o, 80, 16), torch.tensor([0, 16, 32, 48], dtype=torch.int32))
+
+
 def test_an_epilogue_is_supported_with_the_hint_as_without_it():
     from magicdec_amd import _lib, ops
     lib = _lib.load()
