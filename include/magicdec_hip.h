@@ -409,6 +409,8 @@ typedef struct md_fused_linear_args {
     const float* act;         /* MD_FL_XIELU: the two fp32 numbers of the activation (md_xielu); MD_FL_SOFTCAP: the cap */
 } md_fused_linear_args;
 int md_linear_fused_supported(int M, int N, int K, int epilogue);
+/* columns of a workgroup of md_linear_fused (N2 > 0: md_linear_fused_beside) without a deferred norm, 32 or 64; a result does not depend on them */
+int md_linear_fused_columns(int M, int N, int K, int epilogue, int N2);
 int md_linear_fused(const md_fused_linear_args* args, md_stream_t stream);
 
 /* md_linear_few (csrc/tilegemm.hip): the same of at most 16 rows on tiles of 16 columns, K % 256 == 0, with sums of another order.  Two

@@ -117,6 +117,7 @@ _SIGNATURES = {
     "md_linear_few_supported": (c_int, [I, I, I, I]),
     "md_linear_few": (c_int, [ctypes.POINTER(FusedLinearArgs), P]),
     "md_linear_fused_supported": (c_int, [I, I, I, I]),
+    "md_linear_fused_columns": (c_int, [I, I, I, I, I]),
     "md_linear_fused": (c_int, [ctypes.POINTER(FusedLinearArgs), P]),
     "md_linear_fused_split_workspace_bytes": (c_size_t, [I, I, I]),
     "md_linear_fused_split": (c_int, [P, L, P, P, P, L, I, I, I, P, c_size_t, P]),

@@ -832,9 +832,12 @@ bool two_by_two(int M, int N, int K) {
 // whose epilogue is the longest, from 1 920 on and to 352 tiles (320 x 640 7.5 / 8.8; 320 x 2 048 13.0 / 12.9, 14.1 / 13.2; 448 x 2 048 14.5 / 15.4).
 // And K = 4 096, to 400 tiles: 400 23.9 / 23.1, 25.3 / 23.8, but 448 24.3 / 25.3, 26.0 / 25.5, 512 26.7 / 28.4, 28.0 / 28.8 (3 968 and 4 224 gain 4 to
 // 17 % everywhere: one tile of exactly 4 096 is a sixth faster than its neighbours, two are not).
-bool two_columns(int epi, int M, int K, int wgs) {
+// The line at 257 tiles stands although 129 workgroups leave half of the CUs idle: 258 tiles, 17 and 32 rows, gated or not, two runs
+// each, two tiles a workgroup are ahead by 6 to 11 % at K = 1 024, 11 to 18 at 2 048, 13 to 21 at 3 072 (gated 13 to 18); 512 tiles -2 to 1 % at
+// 2 048, 0 to 4 at 3 072.
+bool two_columns(int epi, int M, int K, int n_tiles, int side_tiles) {
     const int deep = epi == FL_XIELU ? 1920 : epi == FL_SWIGLU ? 1152 : 896, most = epi == FL_XIELU ? 352 : K == 4096 ? 400 : 512;
-    return M > 16 && M <= 32 && K >= deep && wgs > 256 && wgs <= most;
+    return M > 16 && M <= 32 && K >= deep && n_tiles % 2 == 0 && n_tiles + side_tiles > 256 && n_tiles + side_tiles <= most;
 }
 
 template <int EPI, bool FP8, bool PRO>
@@ -866,7 +869,7 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
     const int wgs = (p.n_tiles + p.side_tiles) * p.m_tiles;
     bool nw16 = p.K % 256 == 0 && p.K >= 1024 && wgs <= 256;
     if constexpr ((EPI == FL_SWIGLU || EPI == FL_NONE || EPI == FL_SOFTCAP || EPI == FL_RESID || EPI == FL_XIELU) && !PRO)
-        if (p.n_tiles % 2 == 0 && two_columns(EPI, p.M, p.K, wgs) && g_force_tile == 0 && g_force_nw == 0)
+        if (two_columns(EPI, p.M, p.K, p.n_tiles, p.side_tiles) && g_force_tile == 0 && g_force_nw == 0)
             return launch_tile_cfg<EPI, FP8, 8, true, PRO, 1, 2>(p, st);
     if (g_force_nw == 8) nw16 = false;
     if (g_force_nw == 16) nw16 = p.K % 256 == 0;
@@ -1083,6 +1086,14 @@ extern "C" int md_linear_fused_supported(int M, int N, int K, int epilogue) {
     epilogue &= ~MD_FL_STREAMED;
     if (M < 1 || M > 256 || K < 128 || K % 128 || N < 32 || N % 32) return 0;
     return ((epilogue >= FL_NONE && epilogue <= FL_GEGLU) || epilogue == FL_SOFTCAP) ? 1 : 0;
+}
+
+extern "C" int md_linear_fused_columns(int M, int N, int K, int epilogue, int N2) {
+    MD_CHECK_ARG(md_linear_fused_supported(M, N, K, epilogue) && N2 >= 0 && N2 % 32 == 0,
+                 "md_linear_fused_columns: M=%d N=%d K=%d epilogue=%d N2=%d", M, N, K, epilogue, N2);
+    const int epi = (epilogue & ~MD_FL_STREAMED) == FL_GEGLU ? FL_SWIGLU : epilogue & ~MD_FL_STREAMED;
+    if (epi == FL_ROPE_APPEND) return 32;
+    return (!N2 && two_by_two(M, N, K)) || two_columns(epi, M, K, N / 32, N2 / 32) ? 64 : 32;
 }
 
 extern "C" int md_linear_few_supported(int M, int N, int K, int epilogue) {

@@ -313,6 +313,7 @@ def test_streamed_weights_give_the_same_bits(ops, M, N, K):
 def test_one_row_tile_of_64_columns(ops, M, N, K):
     """17 to 32 rows of 257 to 512 column tiles, two of them a workgroup (shallow products: one): the bits of one a workgroup."""
     lib = ops._lib.load()
+    assert lib.md_linear_fused_columns(M, N, K, ops.FL_NONE, 0) == (64 if K >= 896 else 32)
     g = torch.Generator().manual_seed(M + N)
     x, w, b, resid = (d(torch.randn(*n, generator=g).to(BF)) for n in ((M, K), (N, K), (N,), (M, N)))
     act = d(torch.rand(2, generator=g) + 0.5)
@@ -326,41 +327,6 @@ def test_one_row_tile_of_64_columns(ops, M, N, K):
     finally:
         lib.md_debug_set_fused_nw(0)
     assert all(torch.equal(a, c) and a.isfinite().all() for a, c in zip(outs[0], outs[11]))
-
-
-@pytest.mark.parametrize("M,tiles,K,kind", [(17, 258, 512, "gated"), (32, 258, 256, "gated"), (17, 320, 640, "xielu"), (24, 512, 1024, "xielu"), (17, 448, 2048, "xielu"),
-                                            (17, 512, 4096, "plain"), (17, 352, 2048, "plain"), (32, 320, 2048, "xielu"), (32, 352, 2048, "gated")])
-def test_two_column_tiles_a_workgroup_only_where_they_pay(ops, M, tiles, K, kind):
-    """The rule's choice is no slower than one column tile a workgroup: replays of the same launches over weights that no cache keeps, in turn
-    (the shapes beside the rule's range were 5 to 17 % slower with two)."""
-    lib, N = ops._lib.load(), 32 * tiles
-    x, w = (d(torch.randn(*n).to(BF)) for n in ((M, K), (N, K)))
-    act, out = d(torch.rand(2) + 0.5), d(torch.empty(M, N // 2 if kind == "gated" else N, dtype=BF))
-    packs = [ops.PackedWeight(w, swiglu=kind == "gated") for _ in range(min(64, (600 << 20) // (2 * N * K)))]
-
-    def launches():
-        for pw in packs:
-            ops.fused_linear(x, pw, swiglu=kind == "gated", xielu=act if kind == "xielu" else None, out=out)
-    graphs, best = {}, {}
-    try:
-        for knob in (0, 11):
-            lib.md_debug_set_fused_nw(knob)
-            launches()
-            torch.cuda.synchronize()
-            graphs[knob] = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graphs[knob]):
-                launches()
-    finally:
-        lib.md_debug_set_fused_nw(0)
-    for _ in range(15):
-        for knob, graph in graphs.items():
-            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-            start.record()
-            graph.replay()
-            end.record()
-            end.synchronize()
-            best[knob] = min(best.get(knob, 1e9), start.elapsed_time(end))
-    assert best[0] <= 1.04 * best[11], best
 
 
 @pytest.mark.parametrize("M,N", [(1, 8192), (16, 8224), (32, 8224), (17, 12320), (33, 4128)])

@@ -1539,6 +1539,23 @@ def test_an_epilogue_is_supported_with_the_hint_as_without_it():
     assert lib.md_linear_fused_supported(64, 16384, 2048, ops.FL_SOFTCAP | ops.FL_STREAMED) == 1
 
 
+@pytest.mark.parametrize("M,tiles,K,kind,beside,want", [
+    (17, 258, 512, "SWIGLU", 0, 32), (17, 384, 1024, "GEGLU", 0, 32), (32, 258, 1280, "SWIGLU", 0, 64), (32, 352, 2048, "GEGLU", 43, 64),
+    (17, 320, 640, "XIELU", 0, 32), (24, 512, 1024, "XIELU", 0, 32), (17, 448, 2048, "XIELU", 0, 32), (32, 320, 2048, "XIELU", 0, 64),
+    (17, 258, 768, "RESID", 0, 32), (17, 258, 896, "RESID", 0, 64), (32, 304, 1024, "SOFTCAP", 0, 64), (17, 512, 3072, "NONE", 0, 64),
+    (17, 400, 4096, "NONE", 0, 64), (17, 448, 4096, "NONE", 0, 32), (17, 512, 4096, "NONE", 0, 32), (17, 512, 4224, "NONE", 0, 64),
+    (16, 352, 2048, "NONE", 0, 32), (33, 352, 2048, "NONE", 0, 32), (64, 512, 2048, "NONE", 0, 64), (32, 256, 2048, "NONE", 0, 32),
+    (32, 257, 2048, "NONE", 0, 32), (32, 514, 2048, "NONE", 0, 32), (32, 512, 2048, "SWIGLU", 1, 32), (32, 352, 2048, "ROPE_APPEND", 0, 32)])
+def test_two_column_tiles_a_workgroup_only_where_they_pay(M, tiles, K, kind, beside, want):
+    """The rule of the tile GEMM for 17 to 32 rows at the shapes it was measured at: not for the products that two column tiles a workgroup
+    slow down by up to a fifth (shallow ones, xIELU ones, 4 096 deep ones of many tiles)."""
+    from magicdec_amd import _lib, ops
+    lib = _lib.load()
+    for hint in (0, ops.FL_STREAMED):
+        assert lib.md_linear_fused_columns(M, 32 * tiles, K, getattr(ops, "FL_" + kind) | hint, 32 * beside) == want
+    assert lib.md_linear_fused_columns(M, 32 * tiles + 1, K, ops.FL_NONE, 0) < 0
+
+
 @pytest.mark.parametrize("prompt", ["refused", "failing"])
 def test_a_refused_prompt_leaves_the_weights_released(cpu_ops_patched, prompt):
     """A prompt that raises (the SnapKV engine's refusal of its length, or an error inside a portion) ends like one that does not: no
