@@ -856,8 +856,8 @@ int launch_tile_pro(const TileParams& p, hipStream_t st) {
         if (PRO && p.pro_tiles > 128) t22 = false;       // the 2 x 2 prologue keeps <= 8 partial sums per thread in flight
         // Weights that no cache keeps until the next step: past the caches, where one group of rows reads them.  The product gains nothing
         // by it (a 1B draft's gated one at 64 rows 20.2 / 21.1 us), but what is read again does: the other projections' weights, which stay in
-        // the last-level cache (qkv 8.0 -> 7.1, wo 7.4 -> 6.4).  A step of four layers (617 MB) 311.9 -> 301.3 us, of sixteen 1 083 -> 1 059;
-        // of two (373 MB, half of which the cache keeps) 160.2 -> 162.9, so that it is the caller who says which (MD_FL_STREAMED)
+        // the last-level cache (qkv 8.0 -> 7.1, wo 7.4 -> 6.4): a step of four layers (618 MB) 310 -> 295 us, but of two (374 MB, half of
+        // which the cache keeps) 172 -> 174, so that it is the caller who says which (MD_FL_STREAMED)
         if (t22 && p.streamed && p.m_tiles <= 2) return launch_tile_cfg<EPI, FP8, 8, true, PRO, 2, 2>(p, st);
         if (t22) return launch_tile_cfg<EPI, FP8, 8, false, PRO, 2, 2>(p, st);
     }

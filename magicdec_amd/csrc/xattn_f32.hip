@@ -15,12 +15,11 @@
 //
 // Bound by the fp32 matrix rate (154 TFLOP/s in a large library product) for prompts, by latency for decode steps.  Six sequences of
 // 100 to 1 500 tokens, 32 query and 8 kv heads of 64, one layer (22 GFLOP): 9 930 -> 445 -> 277 us; one token each behind them:
-// 292 -> 17.4 + 5.8 us for the merge -> 15.0 + 5.3 with splits of three tiles, all with keys, and their loads together in the merge (first
-// figure: the plain kernel, one workgroup per row and head).
+// 292 -> 17.4 + 5.8 us for the merge -> 15.0 + 5.3 with splits of three tiles (of the longest page table's keys) and their loads together in
+// the merge (first figure: the plain kernel, one workgroup per row and head).
 #include "xattn.h"
 
 #include <algorithm>
-#include <cstdlib>
 
 namespace {
 
@@ -688,8 +687,9 @@ F32Launch plan(const XattnParams& p, Shape s, long keys, size_t* room = nullptr)
         L.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>({want, keys / (4 * kt[s]), 64}));
         return groups * L.nsplit;
     };
-    // Sixteen rows a workgroup: a tile is 1.5 to 2 us of a step, one more split to merge 0.2, so splits go down to two tiles, none without
-    // a tile, and a sequence of four tiles stays whole (130 keys 13.9 us whole, 14.8 in two).  us, at least four tiles a split / now, 8 kv
+    // Sixteen rows a workgroup: a tile is 1.5 to 2 us of a step, one more split to merge 0.2, so splits go down to two tiles of the
+    // longest page table, none of them without a tile there, and four tiles stay whole (130 keys 13.9 us whole, 14.8 in two).  A shorter
+    // sequence beside the longest has as many splits, of fewer tiles, the last ones of none.  us, at least four tiles a split / now, 8 kv
     // heads of 64: one request of 600 keys 22.8 / 15.5, of 2 000 25.0 / 20.5, 6 of 300 20.3 / 16.5, of 1 500 29.2 / 25.3, 12 of 600 25.9 /
     // 21.5, 16 of 2 000 51.6 / 50.9.  Heads above 128, one workgroup a CU: 5 x 8 kv heads of 256, 600 keys 33.8 / 33.0, 6 of 8, 790
     // 56.9 / 40.2, but unequal sequences of more than 32 pairs level out with more splits than one round of CUs (7 x 8, to 1 587 keys 65.5 /
