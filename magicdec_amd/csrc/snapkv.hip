@@ -334,8 +334,8 @@ __device__ __noinline__ unsigned int accum_slow(const lds_double* tab, const lds
 // pair per row in LDS.  A wavefront takes 2 x 2 tiles at a time: two column groups share the query fragments, and the 16 table
 // gathers of a lane are in flight together.  16 requests of 16 000 keys (8 kv heads of 64, 128 rows each): 92 us; 120 in two workgroups of
 // eight wavefronts a CU, each with its own table and image (12 us to fill), with the rare scores in line (spills) and 23 binades (0.8 % of
-// the batches are rare then); 150 tile by tile.  Bound by LDS, active for 69 % of the cycles: 4 gathers of 8 random bytes per lane and
-// tile, about 7 cycles each, beside 8 for the fragments; vector instructions 49 %.
+// the batches are rare then); 150 tile by tile.  Bound by LDS, active for 68 % of the cycles: 4 gathers of 8 random bytes per lane and
+// tile, about 7 cycles each, beside 8 for the fragments; vector instructions 47 %.
 template <int D, bool FP8, int RTM>     // RTM: register-resident 16-row tiles (8 for g * W <= 128 rows, else kMaxRT)
 __global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) void snapkv_stats_kernel(const SnapParams p) {
     constexpr int kSnapWaves = score_waves(D, RTM), BIN = stats_binades(D, RTM);
@@ -477,9 +477,10 @@ __global__ __launch_bounds__(256) void snapkv_finalize_kernel(const SnapParams p
 // by the two halves in turn).  After the exchange a lane keeps one of two column groups' sums, so that one rounding serves two sums.
 // NC column groups share a row tile's fragments and factors: four where a wavefront's 64 columns come out even (`four` below), the next
 // ones' keys then loaded behind the last row tile's products.  16 requests of 16 000 keys, as above: 109 us; 124 on the same card with two
-// row tiles of two column groups, both of whose sums every lane kept.  Bound by LDS as pass 1 is: random gathers are active for 62 % of the
-// cycles with all LDS work at 74 %, vector instructions at 67 %.  (A table of floats, and the float64 product only where rounding is in
-// doubt: 4 bytes at random cost what 8 do, 118 against 123; the scores a batch ahead of the gathers: 118 / 118.)
+// row tiles of two column groups, both of whose sums every lane kept.  Bound by vector issue and LDS in turn: vector
+// instructions for 70 % of the cycles, LDS active for 58 % (37 of them bank conflicts of the random gathers).  (A table of floats, and the
+// float64 product only where rounding is in doubt: 4 bytes at random cost what 8 do, 118 against 123; the scores a batch ahead of the
+// gathers: 118 / 118.)
 // BIN: the table's binades; all, but where the accumulators of 30 and 32 queries a kv head of 128 beside them would pass a CU's LDS.
 template <int D, bool FP8, int GH, int RTM, int NC, int BIN = kTabBinades>
 __global__ __launch_bounds__(64 * score_waves(D, RTM), score_waves(D, RTM) / 4) void snapkv_accum_kernel(const SnapParams p) {
